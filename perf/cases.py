@@ -35,23 +35,23 @@ def listed() -> list:
                 **kw}
     return [
         # one user of the small model: nothing but latency and launches
-        case("decode 1b, 1 sequence", "decode", "llama-3-1b", 1, 101),
+        case("decode 1b 1 sequence", "decode", "llama-3-1b", 1, 101),
         # one user of the flagship in a short chat
-        case("decode 8b, 1 sequence", "decode", "llama-3-8b", 1, 1000),
+        case("decode 8b 1 sequence", "decode", "llama-3-8b", 1, 1000),
         # the serving benchmark's steady state: 64 clients, 128 + 64 tokens
-        case("decode 8b, 64 sequences", "decode", "llama-3-8b", 64, 192, 0.3),
+        case("decode 8b 64 sequences", "decode", "llama-3-8b", 64, 192, 0.3),
         # long conversations, lengths as they come
-        case("decode 8b, long contexts", "decode", "llama-3-8b", 16, 4096,
+        case("decode 8b long contexts", "decode", "llama-3-8b", 16, 4096,
              0.6),
         # the 8-bit cache of config.features.yaml, a batch that is not round
-        case("decode 8b, 8-bit cache", "decode", "llama-3-8b", 37, 2000, 0.5,
+        case("decode 8b 8-bit cache", "decode", "llama-3-8b", 37, 2000, 0.5,
              kv8=True),
         # time to first token of a short question
-        case("prompt 1b, short", "prompt", "llama-3-1b", 1, 45),
+        case("prompt 1b short", "prompt", "llama-3-1b", 1, 45),
         # the serving benchmark's burst: 64 prompts arrive together
-        case("prompts 8b, burst", "prompt", "llama-3-8b", 64, 128),
+        case("prompts 8b burst", "prompt", "llama-3-8b", 64, 128),
         # a document in the prompt
-        case("prompt 8b, long", "prompt", "llama-3-8b", 1, 7901),
+        case("prompt 8b long", "prompt", "llama-3-8b", 1, 7901),
         # a worker's ordinary step under load: a 512-token chunk of a long
         # prompt beside sequences that decode
         case("chunk 8b beside decodes", "chunk", "llama-3-8b", 24, 1500, 0.5,
@@ -60,7 +60,7 @@ def listed() -> list:
         case("prompts nesizen", "prompt", NESIZEN, 4, 2048, 0.2),
         case("decode nesizen", "decode", NESIZEN, 16, 2048, 0.4),
         # the experts of the mixed designs over a prefill batch
-        case("experts, prompt rows", "experts", "moe-w2048", 1, 0, rows=6001),
+        case("experts prompt rows", "experts", "moe-w2048", 1, 0, rows=6001),
     ]
 
 

@@ -43,8 +43,7 @@ LIBRARIES = {
         "rope_kv.hip",
         "decode_attn.hip",
         "prefill_attn.hip",
-        "prefill_mfma.hip",
-        "prefill_paged.hip",
+        "prefill_flash.hip",
         "sampling.hip",
         "skinny_gemm.hip",
         "skinny2.hip",

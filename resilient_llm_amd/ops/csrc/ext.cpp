@@ -389,7 +389,8 @@ Tensor prefill_attn_qkv(const Tensor& qkv, const Tensor& cu_seqlens,
                         double scale, int64_t n_q, int64_t n_kv,
                         int64_t head_dim) {
   check_bf16_contig(qkv, "qkv");
-  TORCH_CHECK(cu_seqlens.scalar_type() == at::kInt && cu_seqlens.is_contiguous());
+  TORCH_CHECK(cu_seqlens.scalar_type() == at::kInt &&
+              cu_seqlens.is_contiguous() && cu_seqlens.numel() >= 1);
   const int T = int(qkv.size(0));
   const int D = int(head_dim);
   const int stride = int(qkv.size(1));
@@ -400,25 +401,9 @@ Tensor prefill_attn_qkv(const Tensor& qkv, const Tensor& cu_seqlens,
   const int n_seqs = int(cu_seqlens.numel()) - 1;
   Tensor out = at::empty({T, n_q * D}, qkv.options());
   c10::hip::HIPGuardMasqueradingAsCUDA guard(qkv.device());
-  // chunk tables for the MFMA kernel (host-side; prefill is not captured)
-  Tensor cu_cpu = cu_seqlens.to(at::kCPU);
-  const int32_t* cu = cu_cpu.data_ptr<int32_t>();
-  std::vector<int32_t> t0s, starts, ends;
-  for (int s = 0; s < n_seqs; ++s)
-    for (int t = cu[s]; t < cu[s + 1]; t += 32) {
-      t0s.push_back(t);
-      starts.push_back(cu[s]);
-      ends.push_back(cu[s + 1]);
-    }
-  const int n_chunks = int(t0s.size());
-  auto iopt = at::TensorOptions().dtype(at::kInt);
-  Tensor t0_d = at::tensor(t0s, iopt).to(qkv.device(), /*nb=*/true);
-  Tensor st_d = at::tensor(starts, iopt).to(qkv.device(), true);
-  Tensor en_d = at::tensor(ends, iopt).to(qkv.device(), true);
-  rlli::launch_prefill_mfma(
-      bf16_ptr(qkv), t0_d.data_ptr<int32_t>(), st_d.data_ptr<int32_t>(),
-      en_d.data_ptr<int32_t>(), bf16_ptr(out), n_chunks, int(n_kv),
-      group, D, stride, float(scale), current_stream(qkv));
+  rlli::launch_prefill_rows(
+      bf16_ptr(qkv), cu_seqlens.data_ptr<int32_t>(), bf16_ptr(out), n_seqs, T,
+      int(n_kv), group, D, stride, float(scale), current_stream(qkv));
   check_launch("prefill_attn_qkv");
   return out;
 }

@@ -83,15 +83,14 @@ void launch_prefill_attn(
     int head_dim, float scale, int q_stride, int kv_stride,
     hipStream_t stream);
 
-// MFMA varlen causal prefill attention over a fused qkv tensor.
-void launch_prefill_mfma(const uint16_t* qkv, const int32_t* chunk_t0,
-                         const int32_t* chunk_seq_start,
-                         const int32_t* chunk_seq_end, uint16_t* out,
-                         int n_chunks, int n_kv_heads, int group,
-                         int head_dim, int qkv_stride, float scale,
+// Causal attention of whole prompts over a fused qkv tensor; cu_seqlens
+// [n_seqs + 1] stays on the device.
+void launch_prefill_rows(const uint16_t* qkv, const int32_t* cu_seqlens,
+                         uint16_t* out, int n_seqs, int rows, int n_kv_heads,
+                         int group, int head_dim, int qkv_stride, float scale,
                          hipStream_t stream);
 
-// MFMA chunked-prefill attention over the paged cache (mixed batches).
+// The same over the paged cache (chunks and mixed batches).
 void launch_prefill_paged(const uint16_t* qkv, const void* k_cache,
                           const void* v_cache, const int32_t* chunk_row0,
                           const int32_t* chunk_pos0,

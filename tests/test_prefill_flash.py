@@ -1,0 +1,69 @@
+"""Causal prompt attention at the sizes where its tiles end: 32 rows, 64
+keys, sequences counted 64 at a time, pages of any size, every head group."""
+
+import pytest
+import torch
+
+from resilient_llm_amd import ops
+from resilient_llm_amd.ops import ref
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def close(got, want):
+    # weights and outputs are each rounded to bf16 (2^-9 of them), values
+    # are of size one and weights sum to one
+    torch.testing.assert_close(got.cpu().float(), want.float(), atol=2 ** -7,
+                               rtol=2 ** -7)
+
+
+@pytest.mark.parametrize("n_q,n_kv,D", [
+    (4, 1, 128), (8, 8, 64), (4, 2, 128), (8, 1, 64), (32, 8, 128)])
+@pytest.mark.parametrize("lens", [
+    [1], [31, 32, 33], [63, 64, 65], [0, 5, 0, 129], [3] * 66 + [40]],
+    ids=str)
+def test_batch_rows(n_q, n_kv, D, lens):
+    gen = torch.Generator().manual_seed(len(lens))
+    T = sum(lens)
+    qkv = torch.randn(T, (n_q + 2 * n_kv) * D, generator=gen) \
+        .to(torch.bfloat16)
+    cu = torch.tensor([0] + lens).cumsum(0).to(torch.int32)
+    # scores far apart: maxima move from tile to tile
+    for scale in (D ** -0.5, -1.5):
+        got = ops.prefill_attn_qkv(qkv.to(DEV), cu.to(DEV), scale, n_q, n_kv,
+                                   D)
+        q, k, v = (t.reshape(T, -1, D) for t in torch.split(
+            qkv, [n_q * D, n_kv * D, n_kv * D], 1))
+        close(got, ref.prefill_attn(q, k, v, cu, scale).reshape(T, -1))
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("n_q,n_kv,D,bs", [
+    (8, 2, 128, 16), (8, 1, 64, 16), (2, 1, 128, 8), (3, 3, 64, 4),
+    (4, 1, 128, 32)])
+def test_pages(n_q, n_kv, D, bs, fp8):
+    gen = torch.Generator().manual_seed(D + bs)
+    # (position of the first row, rows) of each sequence
+    seqs = [(0, 33), (63, 1), (64, 32), (97, 31)]
+    width = max(-(-(s + n) // bs) for s, n in seqs)
+    pages = len(seqs) * width
+    k, v = (torch.randn(pages, n_kv, bs, D, generator=gen) for _ in "kv")
+    k, v = (t.to(torch.float8_e4m3fn if fp8 else torch.bfloat16)
+            for t in (k, v))
+    tables = torch.randperm(pages, generator=gen).to(torch.int32) \
+        .view(len(seqs), width)
+    T = sum(n for _, n in seqs)
+    qkv = torch.randn(T, (n_q + 2 * n_kv) * D, generator=gen) \
+        .to(torch.bfloat16)
+    tiles, row = [], 0
+    for b, (start, n) in enumerate(seqs):
+        tiles += [(row + o, start + o, min(32, n - o), b)
+                  for o in range(0, n, 32)]
+        row += n
+    t = torch.tensor(tiles, dtype=torch.int32).t().contiguous()
+    got = ops.prefill_paged_attn(
+        qkv.to(DEV), k.to(DEV), v.to(DEV), *t.to(DEV), tables.to(DEV),
+        D ** -0.5, n_q)
+    k, v = (x.float().to(torch.bfloat16) for x in (k, v))
+    close(got, ref.prefill_paged_attn(qkv, k, v, *t, tables, D ** -0.5, n_q))

@@ -29,8 +29,7 @@ import torch.nn.functional as F
 from .. import ops
 from ..ops import autotune as lt_autotune
 
-# Opt-in: route decode-shaped GEMMs (M<=64) through the custom skinny-M
-# MFMA kernel instead of hipBLASLt (A/B lever; see ops/csrc/skinny_gemm.hip)
+# Opt-in: the kernel for few rows ahead of everything else (A/B lever)
 _USE_SKINNY = os.environ.get("RLLI_SKINNY") == "1"
 
 
@@ -44,8 +43,11 @@ _LT_ROWS = frozenset({1, 2, 4, 8, 12, 16, 24, 32, 48, 64, 96, 128})
 def _linear(x, w):
     if _USE_SKINNY:
         return ops.linear_auto(x, w)
-    if x.is_cuda and x.dim() == 2 and x.shape[0] in _LT_ROWS:
+    if (lt_autotune.enabled() and x.is_cuda and x.dim() == 2
+            and x.shape[0] in _LT_ROWS):
         return lt_autotune.tuned_linear(x, w)
+    if ops.rows_fit(x, w):
+        return ops.rows_linear(x, w)
     return F.linear(x, w)
 
 

@@ -45,8 +45,7 @@ LIBRARIES = {
         "prefill_attn.hip",
         "prefill_flash.hip",
         "sampling.hip",
-        "skinny_gemm.hip",
-        "skinny2.hip",
+        "rows_gemm.hip",
         "streamprobe.hip",
     ],
     "rlli_attn": [

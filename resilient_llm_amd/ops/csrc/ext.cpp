@@ -447,100 +447,94 @@ Tensor prefill_paged_attn(const Tensor& qkv, const Tensor& k_cache,
   return out;
 }
 
-// --------------------------------------------------------- skinny_linear
+// ------------------------------------------------------------ rows_gemm
+static void check_rows(const Tensor& x, const Tensor& w) {
+  check_bf16_contig(x, "x");
+  check_bf16_contig(w, "w");
+  TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && w.size(1) == x.size(1),
+              "x/W K mismatch");
+  TORCH_CHECK(x.size(0) >= 1 && x.size(0) <= 64, "1 to 64 rows, got ",
+              x.size(0));
+  TORCH_CHECK(x.size(1) % 64 == 0 && x.size(1) > 0 && w.size(0) % 4 == 0 &&
+                  w.size(0) > 0,
+              "K % 64 == 0 and N % 4 == 0, got K=", x.size(1), " N=",
+              w.size(0));
+  TORCH_CHECK(reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0 &&
+                  reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0,
+              "x and W start at multiples of 16 bytes");
+}
+
+// y = x w^T in f32 parts [splits, M, N] to be summed, or whole in bf16
+// [M, N] where K is not divided.
+Tensor rows_linear_parts(const Tensor& x, const Tensor& w) {
+  check_rows(x, w);
+  const int M = int(x.size(0)), N = int(w.size(0)), K = int(x.size(1));
+  c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
+  const int splits = rlli::rows_gemm_splits(N, K);
+  Tensor out = splits > 1
+                   ? at::empty({splits, M, N}, x.options().dtype(at::kFloat))
+                   : at::empty({M, N}, x.options());
+  rlli::launch_rows_gemm(
+      bf16_ptr(x), bf16_ptr(w), splits > 1 ? out.data_ptr<float>() : nullptr,
+      splits > 1 ? nullptr : bf16_ptr(out), M, N, K, splits,
+      current_stream(x));
+  check_launch("rows_linear");
+  return out;
+}
+
+Tensor rows_linear(const Tensor& x, const Tensor& w) {
+  Tensor parts = rows_linear_parts(x, w);
+  if (parts.dim() == 2) return parts;
+  c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
+  Tensor out = at::empty({x.size(0), w.size(0)}, x.options());
+  rlli::launch_sum_parts(parts.data_ptr<float>(), bf16_ptr(out),
+                         int(parts.size(0)), out.numel(), current_stream(x));
+  check_launch("sum_parts");
+  return out;
+}
+
+Tensor rows_linear_silu(const Tensor& x, const Tensor& w) {
+  check_rows(x, w);
+  const int inter = int(w.size(0)) / 2;
+  TORCH_CHECK(w.size(0) % 8 == 0, "gate and up rows are multiples of 4");
+  c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
+  Tensor out = at::empty({x.size(0), inter}, x.options());
+  rlli::launch_rows_gemm_silu(bf16_ptr(x), bf16_ptr(w), bf16_ptr(out),
+                              int(x.size(0)), inter, int(x.size(1)),
+                              current_stream(x));
+  check_launch("rows_linear_silu");
+  return out;
+}
+
+// The same under the names and limits of earlier kernels; ``splitk`` has no
+// effect any more.
+static void check_skinny(const char* op, const Tensor& x, const Tensor& w,
+                         int64_t K) {
+  check_bf16_contig(x, "x");
+  check_bf16_contig(w, "w");
+  const int64_t M = x.size(0), N = w.size(0);
+  TORCH_CHECK(w.size(1) == K, "x/W K mismatch");
+  TORCH_CHECK(M >= 1 && M <= 64, op, " needs 1 <= M <= 64, got ", M);
+  TORCH_CHECK(K % 256 == 0 && N % 64 == 0, op,
+              " needs K%256==0 and N%64==0, got K=", K, " N=", N);
+}
+
 Tensor skinny_linear(const Tensor& x, const Tensor& w) {
-  check_bf16_contig(x, "x");
-  check_bf16_contig(w, "w");
-  const int M = int(x.size(0));
-  const int K = int(x.size(1));
-  const int N = int(w.size(0));
-  TORCH_CHECK(w.size(1) == K, "x/W K mismatch");
-  TORCH_CHECK(M >= 1 && M <= 64, "skinny_linear needs 1 <= M <= 64, got ", M);
-  TORCH_CHECK(K % 256 == 0 && N % 64 == 0,
-              "skinny_linear needs K%256==0 and N%64==0, got K=", K, " N=", N);
-  const int n_panels = N / 64;
-  int splitk = 1;
-  if (n_panels < 256) {
-    splitk = std::min<int>(8, std::max<int>(1, 512 / n_panels));
-    splitk = std::min<int>(splitk, K / 256);
-  }
-  Tensor out = at::empty({M, N}, x.options());
-  Tensor ws;
-  float* ws_ptr = nullptr;
-  if (splitk > 1) {
-    ws = at::empty({splitk, M, N}, x.options().dtype(at::kFloat));
-    ws_ptr = ws.data_ptr<float>();
-  }
-  c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
-  rlli::launch_skinny_gemm(bf16_ptr(x), bf16_ptr(w), ws_ptr, bf16_ptr(out),
-                           M, N, K, splitk, current_stream(x));
-  check_launch("skinny_linear");
-  return out;
+  check_skinny("skinny_linear", x, w, x.size(1));
+  return rows_linear(x, w);
 }
 
-// ------------------------------------------------------------- skinny2
-// v2 zero-LDS skinny GEMM; splitk <= 0 picks the grid-fill heuristic
-// (>= ~512 workgroups).  Requirements: M <= 64, K % 256 == 0, N % 16 == 0.
-static int skinny2_auto_splitk(int N, int K) {
-  const int panels = N / 64;   // one 64-column panel per wave
-  int sk = std::max(1, (512 + panels - 1) / panels);
-  return std::min<int>(sk, std::max(1, K / 256));
+Tensor skinny2_linear(const Tensor& x, const Tensor& w, int64_t /*splitk*/) {
+  check_skinny("skinny2_linear", x, w, x.size(1));
+  return rows_linear(x, w);
 }
 
-Tensor skinny2_linear(const Tensor& x, const Tensor& w, int64_t splitk) {
-  check_bf16_contig(x, "x");
-  check_bf16_contig(w, "w");
-  const int M = int(x.size(0));
-  const int K = int(x.size(1));
-  const int N = int(w.size(0));
-  TORCH_CHECK(w.size(1) == K, "x/W K mismatch");
-  TORCH_CHECK(M >= 1 && M <= 64, "skinny2_linear needs 1 <= M <= 64, got ", M);
-  TORCH_CHECK(K % 256 == 0 && N % 64 == 0,
-              "skinny2_linear needs K%256==0 and N%64==0, got K=", K, " N=", N);
-  int sk = int(splitk) > 0 ? int(splitk) : skinny2_auto_splitk(N, K);
-  sk = std::min(sk, K / 256);
-  Tensor out = at::empty({M, N}, x.options());
-  Tensor ws;
-  float* ws_ptr = nullptr;
-  if (sk > 1) {
-    ws = at::empty({sk, M, N}, x.options().dtype(at::kFloat));
-    ws_ptr = ws.data_ptr<float>();
-  }
-  c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
-  rlli::launch_skinny2(bf16_ptr(x), bf16_ptr(w), ws_ptr, bf16_ptr(out),
-                       M, N, K, sk, current_stream(x));
-  check_launch("skinny2_linear");
-  return out;
-}
-
-// down-proj with the SwiGLU fused into the A-fragment path:
-// out = (silu(gu[:, :K]) * gu[:, K:]) @ w^T,  gu = [M, 2K].
-Tensor skinny2_silu_linear(const Tensor& gu, const Tensor& w, int64_t splitk) {
-  check_bf16_contig(gu, "gu");
-  check_bf16_contig(w, "w");
-  const int M = int(gu.size(0));
-  const int K2 = int(gu.size(1));
-  TORCH_CHECK(K2 % 2 == 0, "gu must be [M, 2K]");
-  const int K = K2 / 2;
-  const int N = int(w.size(0));
-  TORCH_CHECK(w.size(1) == K, "gu/W K mismatch");
-  TORCH_CHECK(M >= 1 && M <= 64, "skinny2_silu needs 1 <= M <= 64, got ", M);
-  TORCH_CHECK(K % 256 == 0 && N % 64 == 0,
-              "skinny2_silu needs K%256==0 and N%64==0, got K=", K, " N=", N);
-  int sk = int(splitk) > 0 ? int(splitk) : skinny2_auto_splitk(N, K);
-  sk = std::min(sk, K / 256);
-  Tensor out = at::empty({M, N}, gu.options());
-  Tensor ws;
-  float* ws_ptr = nullptr;
-  if (sk > 1) {
-    ws = at::empty({sk, M, N}, gu.options().dtype(at::kFloat));
-    ws_ptr = ws.data_ptr<float>();
-  }
-  c10::hip::HIPGuardMasqueradingAsCUDA guard(gu.device());
-  rlli::launch_skinny2_silu(bf16_ptr(gu), bf16_ptr(w), ws_ptr, bf16_ptr(out),
-                            M, N, K, sk, current_stream(gu));
-  check_launch("skinny2_silu_linear");
-  return out;
+// down-proj behind SwiGLU: (silu(gu[:, :K]) * gu[:, K:]) @ w^T, gu [M, 2K]
+Tensor skinny2_silu_linear(const Tensor& gu, const Tensor& w,
+                           int64_t /*splitk*/) {
+  TORCH_CHECK(gu.size(1) % 2 == 0, "gu must be [M, 2K]");
+  check_skinny("skinny2_silu", gu, w, gu.size(1) / 2);
+  return rows_linear(silu_mul(gu), w);
 }
 
 Tensor stream_probe(const Tensor& w, int64_t splitk) {
@@ -615,6 +609,9 @@ TORCH_LIBRARY(rlli, m) {
   m.def("prefill_attn(Tensor q, Tensor k, Tensor v, Tensor cu_seqlens, "
         "float scale) -> Tensor");
   m.def("sample(Tensor logits, Tensor temperatures, Tensor seeds, int step) -> Tensor");
+  m.def("rows_linear_parts(Tensor x, Tensor w) -> Tensor");
+  m.def("rows_linear(Tensor x, Tensor w) -> Tensor");
+  m.def("rows_linear_silu(Tensor x, Tensor w) -> Tensor");
   m.def("skinny_linear(Tensor x, Tensor w) -> Tensor");
   m.def("skinny2_linear(Tensor x, Tensor w, int splitk) -> Tensor");
   m.def("skinny2_silu_linear(Tensor gu, Tensor w, int splitk) -> Tensor");
@@ -640,6 +637,9 @@ TORCH_LIBRARY_IMPL(rlli, CUDA, m) {
   m.impl("prefill_attn_qkv", &prefill_attn_qkv);
   m.impl("prefill_attn", &prefill_attn);
   m.impl("sample", &sample);
+  m.impl("rows_linear_parts", &rows_linear_parts);
+  m.impl("rows_linear", &rows_linear);
+  m.impl("rows_linear_silu", &rows_linear_silu);
   m.impl("skinny_linear", &skinny_linear);
   m.impl("skinny2_linear", &skinny2_linear);
   m.impl("skinny2_silu_linear", &skinny2_silu_linear);

@@ -102,21 +102,21 @@ void launch_prefill_paged(const uint16_t* qkv, const void* k_cache,
                           int block_size, float scale, bool cache_fp8,
                           hipStream_t stream);
 
-// Skinny-M GEMM (decode projections): out[M,N] = x[M,K] @ W[N,K]^T.
-// ws is a [splitk, M, N] f32 workspace (unused when splitk == 1).
-// v2: zero-LDS one-wave-per-16-columns register-dataflow skinny GEMM
-// (skinny2.hip); ws is the [splitk, M, N] f32 slab when splitk > 1.
-void launch_skinny2(const uint16_t* x, const uint16_t* w, float* ws,
-                    uint16_t* out, int M, int N, int K, int splitk,
-                    hipStream_t stream);
-// silu(g)*u fused into the A-fragment path: gu is [M, 2K] (gate|up).
-void launch_skinny2_silu(const uint16_t* gu, const uint16_t* w, float* ws,
-                         uint16_t* out, int M, int N, int K, int splitk,
-                         hipStream_t stream);
-
-void launch_skinny_gemm(const uint16_t* x, const uint16_t* w, float* ws,
-                        uint16_t* out, int M, int N, int K, int splitk,
-                        hipStream_t stream);
+// Products of at most 64 rows, y[M, N] = x[M, K] w[N, K]^T (rows_gemm.hip).
+// With parts given, f32 [splits, M, N] whose sum is y; otherwise out.
+// N % 4 == 0, K % 64 == 0, 16-byte aligned rows.
+int rows_gemm_splits(int N, int K);
+void launch_rows_gemm(const uint16_t* x, const uint16_t* w, float* parts,
+                      uint16_t* out, int M, int N, int K, int splits,
+                      hipStream_t stream);
+// silu(x w[:I]^T) * (x w[I:]^T) for w [2 I, K]; false where I is so small
+// that the product in parts is faster
+bool rows_gemm_silu_ok(int inter);
+void launch_rows_gemm_silu(const uint16_t* x, const uint16_t* w,
+                           uint16_t* out, int M, int inter, int K,
+                           hipStream_t stream);
+void launch_sum_parts(const float* parts, uint16_t* out, int splits,
+                      int64_t n, hipStream_t stream);
 
 // Diagnostic: pure nt-stream of W at skinny_gemm geometry.
 void launch_stream_probe(const uint16_t* w, float* sink, int N, int K,

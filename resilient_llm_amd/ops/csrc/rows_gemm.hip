@@ -1,0 +1,320 @@
+// Products of few rows with a weight matrix, as decoding has them:
+// y[M, N] = x[M, K] w[N, K]^T, M <= 64, bf16 with f32 sums.
+//
+// What there is to do is to read w once; everything else has to stay out of
+// its way.  A workgroup has 64 (or 128) rows of w over a range of K, four
+// waves with 16 (32) of them each, and walks 64-wide steps of K through a
+// ring in LDS that direct global -> LDS loads fill R - 1 steps ahead: 32 to
+// 64 KB of w are under way per CU whatever the waves do, which is what the
+// latency of memory at its full rate asks for.  Rows of w arrive in whole
+// 128-byte lines; the 16-byte pieces of a line are swizzled by the row, so
+// that the matrix operand's reads (one piece of sixteen rows) are free of
+// bank conflicts.  x comes along in the same ring and is shared by the waves.
+// Rows are a power of two apart more often than not, so the lines of one step
+// lie on few memory channels: each workgroup starts its walk at a step of its
+// own, which spreads what is asked for at a time over all of them (28672 rows
+// of 4096: 43.7 -> 36 us).
+//
+// Where 64-row panels are fewer than the CUs, K is divided as well, and the
+// parts are written in f32, [splits, M, N], for whoever reads the product to
+// sum; in order, so a result does not depend on when workgroups run.  Nor
+// does it depend on M: the order of sums follows from N and K alone.
+
+#include "common.h"
+
+#include <algorithm>
+#include <type_traits>
+
+namespace rlli {
+
+namespace {
+
+typedef short s16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 b16x2 __attribute__((ext_vector_type(2)));
+
+constexpr int KS = 64;            // a step of K: one 128-byte line of a row
+constexpr int LINE = KS;          // elements
+
+enum { OUT_PARTS = 0, OUT_BF16 = 1, OUT_SILU = 2 };
+
+DEV_INLINE uint32_t pack2(float a, float b) {
+  const b16x2 v = __builtin_convertvector((f32x2{a, b}), b16x2);
+  return __builtin_bit_cast(uint32_t, v);
+}
+
+template <int AUX>
+DEV_INLINE void lds_load16(const void* g, void* l) {
+  __builtin_amdgcn_global_load_lds(
+      (const __attribute__((address_space(1))) void*)g,
+      (__attribute__((address_space(3))) void*)l, 16, 0, AUX);
+}
+
+template <int N>
+DEV_INLINE void wait_vm() {
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(N) : "memory");
+}
+
+// all but the newest L * left loads have landed
+template <int L, int MOST>
+DEV_INLINE void wait_steps(int left) {
+  if constexpr (MOST == 0) {
+    wait_vm<0>();
+  } else {
+    if (left >= MOST) wait_vm<L * MOST>();
+    else wait_steps<L, MOST - 1>(left);
+  }
+}
+
+// CT: 16-row tiles of w per wave; XR: rows of x that are staged; MT: 16-row
+// tiles of x; R: steps in the ring.  OUT_SILU: a wave's first tile is of the
+// gate's rows, the second the same rows of the upper half of w.
+template <int CT, int XR, int MT, int R, int OUT>
+__global__ __launch_bounds__(256)
+void rows_gemm_kernel(const uint16_t* __restrict__ x,
+                      const uint16_t* __restrict__ w, void* __restrict__ out,
+                      int M, int N, int K, int splits) {
+  constexpr int WPART = 4 * CT * 16 * LINE;          // elements of a step
+  constexpr int STEP = WPART + XR * LINE;
+  constexpr int L = CT * 2 + XR / 32;                // loads of a wave
+  extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
+
+  const int panel = blockIdx.x / splits, split = blockIdx.x % splits;
+  const int steps = K / KS;
+  const int s0 = int(int64_t(steps) * split / splits);
+  const int n = int(int64_t(steps) * (split + 1) / splits) - s0;
+  const int lane = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int half = N / 2;
+  // where this workgroup starts within its steps
+  const int rot = int(blockIdx.x / 8 % unsigned(n));
+
+  // first row of w of this wave's tile t
+  auto tile_row = [&](int t) {
+    if constexpr (OUT != OUT_SILU) return panel * 64 * CT + (wv * CT + t) * 16;
+    else if constexpr (CT == 2) return t * half + panel * 64 + wv * 16;
+    else return (wv >> 1) * half + panel * 32 + (wv & 1) * 16;
+  };
+  const int last = OUT == OUT_SILU ? half : N;       // rows end here
+  // a load takes 8 rows, a lane the piece of row lane / 8 that belongs in
+  // slot lane % 8
+  const int lr = lane >> 3;
+  const uint16_t *wp[CT * 2], *xp[XR / 32];
+#pragma unroll
+  for (int j = 0; j < CT * 2; ++j) {
+    const int r = (j & 1) * 8 + lr;
+    int row = tile_row(j >> 1) + r;
+    // rows past the end repeat the last one; nobody stores them
+    if constexpr (OUT == OUT_SILU)
+      row = min(row, (CT == 2 ? j >> 1 : wv >> 1) * half + half - 1);
+    else
+      row = min(row, N - 1);
+    wp[j] = w + int64_t(row) * K + int64_t(s0) * KS +
+            ((lane & 7) ^ ((r >> 1) & 7)) * 8;
+  }
+#pragma unroll
+  for (int j = 0; j < XR / 32; ++j) {
+    const int r = (j * 4 + wv) * 8 + lr;
+    xp[j] = x + int64_t(min(r, M - 1)) * K + int64_t(s0) * KS +
+            ((lane & 7) ^ ((r >> 1) & 7)) * 8;
+  }
+  auto issue = [&](int s, int slot) {
+    uint16_t* at = lds + slot * STEP;
+    s += rot;
+    if (s >= n) s -= n;
+#pragma unroll
+    for (int j = 0; j < CT * 2; ++j)
+      lds_load16<2>(wp[j] + s * KS, at + (wv * CT * 2 + j) * 8 * LINE);
+#pragma unroll
+    for (int j = 0; j < XR / 32; ++j)
+      lds_load16<0>(xp[j] + s * KS, at + WPART + (j * 4 + wv) * 8 * LINE);
+  };
+
+  f32x4 acc[CT][MT];
+#pragma unroll
+  for (int t = 0; t < CT; ++t)
+#pragma unroll
+    for (int m = 0; m < MT; ++m) acc[t][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  const int tr = lane & 15, oct = lane >> 4;
+  const int sw = tr >> 1;
+#pragma unroll
+  for (int s = 0; s < R - 1; ++s)
+    if (s < n) issue(s, s);
+  int slot = 0;
+  for (int s = 0; s < n; ++s) {
+    // this wave's loads of the step have landed, then everybody's; nobody
+    // reads the step before any more
+    wait_steps<L, R - 2>(n - 1 - s);
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (s + R - 1 < n) issue(s + R - 1, slot == 0 ? R - 1 : slot - 1);
+    const uint16_t* at = lds + slot * STEP;
+    slot = slot == R - 1 ? 0 : slot + 1;
+    const uint16_t* wt = at + wv * CT * 16 * LINE + tr * LINE;
+    const uint16_t* xt = at + WPART + tr * LINE;
+    s16x8 a[2][CT], b[2][MT];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      const int piece = ((k * 4 + oct) ^ sw) * 8;
+#pragma unroll
+      for (int t = 0; t < CT; ++t)
+        a[k][t] = *reinterpret_cast<const s16x8*>(wt + t * 16 * LINE + piece);
+#pragma unroll
+      for (int m = 0; m < MT; ++m)
+        b[k][m] = *reinterpret_cast<const s16x8*>(xt + m * 16 * LINE + piece);
+    }
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+#pragma unroll
+      for (int t = 0; t < CT; ++t)
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+          acc[t][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              a[k][t], b[k][m], acc[t][m], 0, 0, 0);
+    constexpr int MFMA = 0x8, DS_READ = 0x100;
+    __builtin_amdgcn_sched_group_barrier(DS_READ, 2 * (CT + MT), 0);
+    __builtin_amdgcn_sched_group_barrier(MFMA, 2 * CT * MT, 0);
+  }
+
+  if constexpr (OUT == OUT_SILU && CT == 1) {
+    // the upper waves' sums to the lower ones
+    __syncthreads();
+    f32x4* side = reinterpret_cast<f32x4*>(lds) + (wv & 1) * MT * 64 + lane;
+    if (wv >= 2)
+#pragma unroll
+      for (int m = 0; m < MT; ++m) side[m * 64] = acc[0][m];
+    __syncthreads();
+    if (wv >= 2) return;
+  }
+  // a lane has four columns of y of one row
+#pragma unroll
+  for (int m = 0; m < MT; ++m) {
+    const int row = m * 16 + tr;
+    if (row >= M) continue;
+    if constexpr (OUT == OUT_SILU) {
+      const int c = tile_row(0) + oct * 4;
+      if (c >= last) continue;
+      f32x4 up;
+      if constexpr (CT == 2) up = acc[1][m];
+      else up = reinterpret_cast<const f32x4*>(lds)[((wv & 1) * MT + m) * 64 +
+                                                    lane];
+      float v[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float g = acc[0][m][r];
+        v[r] = g / (1.f + __expf(-g)) * up[r];
+      }
+      *reinterpret_cast<uint2*>(static_cast<uint16_t*>(out) +
+                                int64_t(row) * half + c) =
+          uint2{pack2(v[0], v[1]), pack2(v[2], v[3])};
+    } else {
+#pragma unroll
+      for (int t = 0; t < CT; ++t) {
+        const int c = tile_row(t) + oct * 4;
+        if (c >= last) continue;
+        const f32x4 v = acc[t][m];
+        if constexpr (OUT == OUT_PARTS)
+          *reinterpret_cast<f32x4*>(static_cast<float*>(out) +
+                                    (int64_t(split) * M + row) * N + c) = v;
+        else
+          *reinterpret_cast<uint2*>(static_cast<uint16_t*>(out) +
+                                    int64_t(row) * N + c) =
+              uint2{pack2(v[0], v[1]), pack2(v[2], v[3])};
+      }
+    }
+  }
+}
+
+__global__ __launch_bounds__(256)
+void sum_parts_kernel(const float* __restrict__ parts,
+                      uint16_t* __restrict__ out, int splits, int64_t n) {
+  const int64_t i = (int64_t(blockIdx.x) * 256 + threadIdx.x) * 4;
+  if (i >= n) return;
+  f32x4 v = *reinterpret_cast<const f32x4*>(parts + i);
+  for (int s = 1; s < splits; ++s)
+    v += *reinterpret_cast<const f32x4*>(parts + s * n + i);
+  *reinterpret_cast<uint2*>(out + i) =
+      uint2{pack2(v[0], v[1]), pack2(v[2], v[3])};
+}
+
+// R32, R64: steps in the ring with 32 and with 64 rows of x
+template <int CT, int R32, int R64, int OUT>
+void go(const uint16_t* x, const uint16_t* w, void* out, int M, int N, int K,
+        int panels, int splits, hipStream_t st) {
+  auto run = [&](auto xr, auto mt) {
+    constexpr int XR = decltype(xr)::value, MT = decltype(mt)::value;
+    constexpr int R = XR == 32 ? R32 : R64;
+    constexpr size_t smem = size_t(R) * (4 * CT * 16 + XR) * LINE * 2;
+    auto* k = rows_gemm_kernel<CT, XR, MT, R, OUT>;
+    if (smem > 65536)
+      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(k),
+                                hipFuncAttributeMaxDynamicSharedMemorySize,
+                                int(smem));
+    hipLaunchKernelGGL(k, dim3(panels * splits), dim3(256), smem, st, x, w,
+                       out, M, N, K, splits);
+  };
+  using I1 = std::integral_constant<int, 1>;
+  using I2 = std::integral_constant<int, 2>;
+  using I3 = std::integral_constant<int, 3>;
+  using I4 = std::integral_constant<int, 4>;
+  using X32 = std::integral_constant<int, 32>;
+  using X64 = std::integral_constant<int, 64>;
+  if (M <= 16) run(X32{}, I1{});
+  else if (M <= 32) run(X32{}, I2{});
+  else if (M <= 48) run(X64{}, I3{});
+  else run(X64{}, I4{});
+}
+
+}  // namespace
+
+// As many parts as 64-row panels leave CUs for: with more workgroups than
+// CUs some CUs have twice the work (N 4096, K 14336: 256 workgroups 19.1 us,
+// 320 24.2, 512 19.5), with half of them latency shows (128: 24.4).
+int rows_gemm_splits(int N, int K) {
+  const int panels = (N + 63) / 64;
+  int n = std::max(1, 256 / panels);
+  // far from a whole round, two rounds waste less
+  if (panels * n < 180 && panels < 256) n = 512 / panels;
+  return std::min(n, K / KS);
+}
+
+// Rings of about 72 KB (whole 64-row steps of x) to 80 KB: one workgroup per
+// CU keeps enough under way, two fit where there are more.  Panels of 128
+// halve what x costs and are taken where they still cover the CUs (128256
+// rows of 4096: 155 us against 158 for one row, 177 against 207 for 64).
+void launch_rows_gemm(const uint16_t* x, const uint16_t* w, float* parts,
+                      uint16_t* out, int M, int N, int K, int splits,
+                      hipStream_t st) {
+  const int panels = (N + 63) / 64;
+  if (parts)
+    go<1, 6, 5, OUT_PARTS>(x, w, parts, M, N, K, panels, splits, st);
+  else if (panels < 400)
+    go<1, 6, 5, OUT_BF16>(x, w, out, M, N, K, panels, 1, st);
+  else
+    go<2, 3, 3, OUT_BF16>(x, w, out, M, N, K, (N + 127) / 128, 1, st);
+}
+
+// Panels of 64 pairs where they cover the CUs, of 32 otherwise (14336 pairs
+// of 4096: 35.3 us against 39.3; 8192 of 2048: 14.5 against 12.1).
+bool rows_gemm_silu_ok(int inter) { return (inter + 31) / 32 >= 160; }
+
+void launch_rows_gemm_silu(const uint16_t* x, const uint16_t* w,
+                           uint16_t* out, int M, int inter, int K,
+                           hipStream_t st) {
+  if ((inter + 63) / 64 >= 200)
+    go<2, 5, 5, OUT_SILU>(x, w, out, M, 2 * inter, K, (inter + 63) / 64, 1,
+                          st);
+  else
+    go<1, 6, 5, OUT_SILU>(x, w, out, M, 2 * inter, K, (inter + 31) / 32, 1,
+                          st);
+}
+
+void launch_sum_parts(const float* parts, uint16_t* out, int splits,
+                      int64_t n, hipStream_t st) {
+  hipLaunchKernelGGL(sum_parts_kernel, dim3(unsigned((n / 4 + 255) / 256)),
+                     dim3(256), 0, st, parts, out, splits, n);
+}
+
+}  // namespace rlli

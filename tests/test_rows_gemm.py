@@ -1,0 +1,64 @@
+"""Products of few rows: edges of row tiles, weight panels, the ring of K
+steps and the division of K; a row's result is the same in any batch."""
+
+import pytest
+import torch
+
+from resilient_llm_amd import ops
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+ROWS = [1, 15, 16, 17, 32, 33, 48, 49, 64]
+
+
+def operands(N, K, seed=0):
+    gen = torch.Generator().manual_seed(seed)
+    x = torch.randn(64, K, generator=gen).to(torch.bfloat16).to(DEV)
+    w = torch.randn(N, K, generator=gen).to(torch.bfloat16).to(DEV)
+    return x, w
+
+
+def close(got, want, size):
+    # half a step of bf16 for the result, K f32 roundings of sums of ``size``
+    torch.testing.assert_close(got.double(), want, rtol=2 ** -8,
+                               atol=float(size) * 2 ** -20)
+
+
+@pytest.mark.parametrize("N,K", [
+    (4, 64), (60, 64), (64, 128), (68, 192), (6160, 320), (8196, 448),
+    (16448, 64), (25540, 192), (25664, 704), (1536, 4096)])
+def test_rows_linear(N, K):
+    x, w = operands(N, K)
+    whole = ops.rows_linear(x, w)
+    close(whole, x.double() @ w.double().T, K ** 0.5)
+    for m in ROWS:
+        assert torch.equal(ops.rows_linear(x[:m].contiguous(), w), whole[:m])
+    parts = torch.ops.rlli.rows_linear_parts(x, w)
+    if parts.dim() == 3:
+        s = parts[0].clone()
+        for p in parts[1:]:
+            s += p
+        assert torch.equal(s.to(torch.bfloat16), whole)
+
+
+@pytest.mark.parametrize("inter,K", [(4, 64), (68, 128), (5152, 64),
+                                     (12740, 192), (12800, 448)])
+def test_rows_linear_silu(inter, K):
+    x, w = operands(2 * inter, K, 1)
+    w *= K ** -0.5
+    whole = torch.ops.rlli.rows_linear_silu(x, w)
+    g, u = (x.double() @ w.double().T).chunk(2, 1)
+    # a sum's f32 error times the other factor, both of size one
+    close(whole, torch.nn.functional.silu(g) * u, 8.0)
+    for m in ROWS:
+        assert torch.equal(
+            torch.ops.rlli.rows_linear_silu(x[:m].contiguous(), w), whole[:m])
+
+
+@pytest.mark.parametrize("M,N,K", [(65, 64, 64), (1, 64, 96), (1, 6, 64)])
+def test_what_does_not_fit(M, N, K):
+    x = torch.zeros(M, K, dtype=torch.bfloat16, device=DEV)
+    w = torch.zeros(N, K, dtype=torch.bfloat16, device=DEV)
+    assert not ops.rows_fit(x, w)
+    with pytest.raises(RuntimeError):
+        ops.rows_linear(x, w)

@@ -78,8 +78,11 @@ def rmsnorm(x: torch.Tensor, w: torch.Tensor, eps: float = 1e-5) -> torch.Tensor
 
 def rmsnorm_residual_(x: torch.Tensor, residual: torch.Tensor, w: torch.Tensor,
                       eps: float = 1e-5) -> torch.Tensor:
+    """``x`` may be the f32 parts of rows_linear_parts."""
     if x.is_cuda:
         _gpu()
+        if x.dim() == 3 and x.dtype == torch.float32:
+            return torch.ops.rlli.rmsnorm_residual_parts_(x, residual, w, eps)
         return torch.ops.rlli.rmsnorm_residual_(x, residual, w, eps)
     return ref.rmsnorm_residual_(x, residual, w, eps)
 
@@ -165,12 +168,31 @@ def decode_attn_rope_qkv(qkv, positions, cos_sin, k_cache, v_cache,
                          slot_mapping, block_table, seq_lens, scale: float,
                          n_q: int) -> torch.Tensor:
     """Fused decode step: rope(q,k) + cache append + paged attention in
-    one kernel on GPU; composed from the unfused reference ops on CPU."""
+    one kernel on GPU; composed from the unfused reference ops on CPU.
+    ``qkv`` may be the f32 parts of rows_linear_parts."""
     if qkv.is_cuda:
         _gpu()
         return torch.ops.rlli.decode_attn_rope_qkv(
             qkv, positions, cos_sin, k_cache, v_cache, slot_mapping,
             block_table, seq_lens, scale, n_q)
+    rope_kv_append_qkv_(qkv, positions, cos_sin, k_cache, v_cache,
+                        slot_mapping, n_q)
+    return decode_attn_qkv(qkv, k_cache, v_cache, block_table, seq_lens,
+                           scale, n_q)
+
+
+def decode_attn_rows_qkv(qkv, positions, cos_sin, k_cache, v_cache,
+                         slot_mapping, block_table, seq_lens, scale: float,
+                         n_q: int) -> torch.Tensor:
+    """decode_attn_rope_qkv for rows that may belong to one sequence: all
+    keys and values are appended first."""
+    if qkv.is_cuda:
+        _gpu()
+        torch.ops.rlli.kv_append_qkv_(qkv, positions, cos_sin, k_cache,
+                                      v_cache, slot_mapping, n_q)
+        return torch.ops.rlli.decode_attn_q_rope(
+            qkv, positions, cos_sin, k_cache, v_cache, block_table, seq_lens,
+            scale, n_q)
     rope_kv_append_qkv_(qkv, positions, cos_sin, k_cache, v_cache,
                         slot_mapping, n_q)
     return decode_attn_qkv(qkv, k_cache, v_cache, block_table, seq_lens,
@@ -235,9 +257,12 @@ def prefill_paged_attn(qkv, k_cache, v_cache, chunk_row0, chunk_pos0,
 
 
 def rows_fit(x: torch.Tensor, w: torch.Tensor) -> bool:
-    """Whether rows_linear takes x w^T: up to 64 rows on the GPU, where
-    reading w is what costs; more are the library's."""
-    return (x.is_cuda and x.dim() == 2 and 1 <= x.shape[0] <= 64
+    """Whether rows_linear takes x w^T: as many rows as leave reading w what
+    costs.  That is 64, or 128 where w is large (128 rows, us, the library's
+    time first: 4096 x 4096 24.4 and 18.6, 4096 x 14336 75.5 and 41.2, but
+    6144 x 2048 15.4 and 17.1, and for 129 rows 21.8 and 26.8)."""
+    return (x.is_cuda and x.dim() == 2 and 1 <= x.shape[0] <= 128
+            and (x.shape[0] <= 64 or w.numel() >= 1 << 24)
             and x.dtype == w.dtype == torch.bfloat16
             and x.shape[1] % 64 == 0 and x.shape[1] > 0
             and w.shape[0] % 4 == 0 and w.shape[0] > 0
@@ -253,6 +278,24 @@ def rows_linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
         _gpu()
         return torch.ops.rlli.rows_linear(x, w)
     return torch.nn.functional.linear(x, w)
+
+
+def rows_linear_parts(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """rows_linear for readers that sum: f32 parts [n, rows, N] of the
+    product, or all of it in bf16 [rows, N] where it was not divided."""
+    if x.is_cuda:
+        _gpu()
+        return torch.ops.rlli.rows_linear_parts(x, w)
+    return torch.nn.functional.linear(x, w)
+
+
+def rows_linear_silu(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """silu_mul(x w^T) for the rows of rows_linear, without the product in
+    between."""
+    if x.is_cuda:
+        _gpu()
+        return torch.ops.rlli.rows_linear_silu(x, w)
+    return silu_mul(torch.nn.functional.linear(x, w))
 
 
 def skinny_linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:

@@ -1,683 +1,650 @@
-// Paged GQA decode attention (one new query token per sequence).
+// Paged GQA decode attention: one new query per sequence.
 //
-// Memory-bound: the cost is streaming each sequence's K/V exactly once
-// from HBM.  Geometry per workgroup = (sequence, kv-head) — times a
-// split-K factor when batch*n_kv_heads alone cannot fill 256 CUs
-// (flash-decode: each of n_split WGs walks an interleaved share of the
-// block chain, emits an f32 partial, and decode_combine_kernel reduces;
-// 2.9-12.7x at batch<=8, bit-identical path at n_split==1).
-// Within a workgroup, 256 threads = 4 waves:
-//   - the GROUP (= n_q / n_kv, Llama-8B: 4) query heads that share this
-//     kv-head ride along in registers, so K/V bytes are read ONCE for
-//     all of them;
-//   - a wave64 splits into 64/GW lane-groups of GW = head_dim/8 lanes;
-//     each lane holds 8 dims (one bf16x8 = 16 B load — G13), each
-//     lane-group walks its share of the tokens of a cache block, each
-//     wave walks every 4th cache block (split-KV);
-//   - each lane-group keeps a private online-softmax partial
-//     (m, l, acc[GROUP][8]); the 4*(64/GW) partials merge through LDS at
-//     the end (log-sum-exp combine).
-// Lane-group token validity is group-uniform, so the tail branch never
-// diverges within a lane-group's reduction.
-// Reference parity: no kernel exists in aws-samples/sample-resilient-llm-inference
-// (model execution lived in Bedrock) — greenfield
-// against the BASELINE.json north-star kernel list.
+// What it costs is to read every key and value once, so the work is laid out
+// by tokens: a wave takes units of 32 of them for the query heads of one
+// key/value head, asks for all their keys and values at once (16 KB), and
+// needs few registers beyond, so that four waves per SIMD keep several times
+// what memory's latency asks for under way.
+//
+// Both products run on the matrix cores, 16 tokens by 16 columns.  A query
+// and a weight are 32-bit numbers: each is cut into two 16-bit ones whose
+// sum has 16 bits of it, and the two are two columns of the same product
+// (columns 0-7 the heads' upper parts, 8-15 the lower), which costs nothing
+// as no more than eight heads share a key/value head.  Scores come out as the
+// second product wants its weights: a lane holds four tokens of a column.
+// The second product is transposed; row n of its tile t is channel VT n + t,
+// so a lane loads VT neighbouring channels of each of its tokens, in whole
+// rows, and makes the operands of all tiles from them.
+//
+// Who takes what, two ways:
+//   whole sequences  a workgroup per (sequence, key/value head), for batches
+//                    that fill the chip with contexts that are not long
+//   parts            sequences are cut into parts of a size that follows
+//                    from all lengths, so that about as many workgroups as
+//                    the chip holds have about as much to do each, whatever
+//                    the lengths are; decode_combine puts the parts of a
+//                    sequence together
+// Against as many parts for each sequence as the batch had of sequences, in
+// lane groups with one accumulator each, 32/8 heads of 128, us: 64 sequences
+// of 134-192 tokens 19.6 -> 13.2 (3.2 TB/s); 16 of 1.7k-4.1k 59 -> 48
+// (4 TB/s, 5 but for what a launch, the lengths and the second kernel take);
+// 37 of 1k-2k with an 8-bit cache 59 -> 40; one of 8000 33 -> 16.
+//
+// Fused form: rotation of q and k, the append to the cache and the new
+// token's own term are part of it; that token's key and value come from LDS,
+// so nothing waits for the append.  Without slots it rotates queries only.
 
 #include "common.h"
 
+#include <algorithm>
+#include <cstdlib>
 #include <type_traits>
 
 namespace rlli {
 
 namespace {
 
+typedef short s16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
 constexpr float kNegInf = -1e30f;
+constexpr int UNIT = 32;          // tokens
+constexpr int MIN_UNITS = 8;      // of a part: two per wave
 
-// FUSED variant: rope(q,k) + cache append of the new token + its
-// self-attention term live INSIDE this kernel (decode fuses 2 kernels
-// into 1; the self token is handled in registers by partial 0, so no
-// in-kernel cache write->read ordering exists — future steps read the
-// appended k/v after the kernel boundary).
-// BS: compile-time cache block size (0 = runtime).  The engine's paged
-// cache uses 16; baking it makes tok_per_grp a constant, so the K/V
-// issue loop fully unrolls with no per-load `i < tok_per_grp` branch
-// (the runtime form emitted s_cbranch between every load pair,
-// fragmenting the batch and forcing early vmcnt waits).
-// ABL: perf-ablation variants (RLLI_ATTN_ABLATE, results intentionally
-// WRONG, never used for real inference): 1 = skip LDS publish/merge,
-// 2 = skip online softmax, 3 = loads only.  Isolates which phase owns
-// the wall time (guide pitfall 8: ablate before optimizing).
-template <int GW, int GROUP, bool FUSED, int BS = 0, int ABL = 0,
-          typename KC = CacheBF16>
-__global__ __launch_bounds__(256)
-void decode_attn_kernel(const uint16_t* __restrict__ q,
-                        const typename KC::elem* __restrict__ k_cache,
-                        const typename KC::elem* __restrict__ v_cache,
-                        const int32_t* __restrict__ block_table,
-                        const int32_t* __restrict__ seq_lens,
-                        uint16_t* __restrict__ out,
-                        int n_kv_heads, int block_size_rt, int max_blocks,
-                        float scale, int q_stride,
-                        const uint16_t* __restrict__ k_src,
-                        const uint16_t* __restrict__ v_src,
-                        const int32_t* __restrict__ positions,
-                        const float* __restrict__ cos_sin,
-                        const int32_t* __restrict__ slot_mapping,
-                        typename KC::elem* __restrict__ k_cache_w,
-                        typename KC::elem* __restrict__ v_cache_w,
-                        int n_split,
-                        float* __restrict__ part_out,
-                        float* __restrict__ part_ml) {
-  constexpr int D = GW * 8;
-  constexpr int GPW = 64 / GW;                 // lane-groups per wave
-  const int block_size = BS ? BS : block_size_rt;
-  // split-K (flash-decode): when batch*n_kv_heads can't fill the chip,
-  // n_split workgroups share one (sequence, kv-head) — each walks an
-  // interleaved subset of the cache blocks and emits an f32 partial
-  // (unnormalized acc + running max/denominator); a tiny combine
-  // kernel reduces them.  n_split==1 is the classic single-WG path.
-  const int split = blockIdx.x % n_split;
-  const int sk = blockIdx.x / n_split;
-  const int seq = sk / n_kv_heads;
-  const int kvh = sk % n_kv_heads;
-  const int len = seq_lens[seq];
-  const int lane = threadIdx.x & (kWave - 1);
-  const int wave = threadIdx.x >> 6;
-  const int n_waves = blockDim.x >> 6;
-  const int group = lane / GW;
-  const int gl = lane % GW;
-  const int d0 = gl * 8;
-  const int n_part = n_waves;    // one partial per wave (in-wave merged)
-
-  extern __shared__ __attribute__((aligned(16))) char smem_raw[];
-  float* accs = reinterpret_cast<float*>(smem_raw);       // [n_part][GROUP][D]
-  float* ml = accs + n_part * GROUP * D;                  // [n_part][GROUP][2]
-
-  // ---- load the GROUP query heads that map to this kv head ----
-  float qv[GROUP][8];
-#pragma unroll
-  for (int h = 0; h < GROUP; ++h) {
-    bf16x8 qh;
-    qh.u = *reinterpret_cast<const uint4*>(
-        q + int64_t(seq) * q_stride + (kvh * GROUP + h) * D + d0);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) qv[h][i] = bf16_to_f32(qh.s[i]);
-  }
-
-  // rope coefficients for this lane's 8 dims (pair index = d mod D/2);
-  // the rotation partner's raw value sits GW/2 lanes away in the group
-  float cs_c[FUSED ? 8 : 1], cs_s[FUSED ? 8 : 1];
-  bool first_half = true;
-  if constexpr (FUSED) {
-    constexpr int HALF = D / 2;
-    const int pos = positions[seq];
-    first_half = d0 < HALF;
-    const int pidx = d0 % HALF;
-    const float* cs = cos_sin + int64_t(pos) * D;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      cs_c[i] = cs[pidx + i];
-      cs_s[i] = cs[HALF + pidx + i];
-    }
-    // rotate every query head in place
-#pragma unroll
-    for (int h = 0; h < GROUP; ++h) {
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const float own = qv[h][i];
-        const float other = __shfl_xor(own, GW / 2, kWave);
-        qv[h][i] = first_half ? own * cs_c[i] - other * cs_s[i]
-                              : own * cs_c[i] + other * cs_s[i];
-      }
-    }
-  }
-
-  float m[GROUP], l[GROUP], acc[GROUP][8];
-#pragma unroll
-  for (int h = 0; h < GROUP; ++h) {
-    m[h] = kNegInf;
-    l[h] = 0.f;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) acc[h][i] = 0.f;
-  }
-
-  if constexpr (FUSED) {
-    // group 0 of wave 0: rope k, append k/v to the cache, and fold the
-    // NEW token's self-attention term into partial 0
-    if (wave == 0 && group == 0 && split == 0) {
-      bf16x8 kr, vr;
-      kr.u = *reinterpret_cast<const uint4*>(
-          k_src + int64_t(seq) * q_stride + kvh * D + d0);
-      vr.u = *reinterpret_cast<const uint4*>(
-          v_src + int64_t(seq) * q_stride + kvh * D + d0);
-      float kf[8], vf[8];
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const float own = bf16_to_f32(kr.s[i]);
-        const float other = __shfl_xor(own, GW / 2, kWave);
-        kf[i] = first_half ? own * cs_c[i] - other * cs_s[i]
-                           : own * cs_c[i] + other * cs_s[i];
-        vf[i] = bf16_to_f32(vr.s[i]);
-      }
-      const int32_t slot = slot_mapping[seq];
-      const int64_t cbase =
-          (int64_t(slot / block_size) * n_kv_heads + kvh) * block_size * D +
-          int64_t(slot % block_size) * D + d0;
-      // append at cache precision (bf16 identity / fp8 cvt_pk); the
-      // self-attention term below uses the STORED values so future
-      // steps reproduce this step's math exactly
-      const typename KC::vec8 kw = KC::from_f32(kf);
-      const typename KC::vec8 vw = KC::from_f32(vf);
-      *reinterpret_cast<typename KC::vec8*>(k_cache_w + cbase) = kw;
-      *reinterpret_cast<typename KC::vec8*>(v_cache_w + cbase) = vw;
-      KC::to_f32(kw, kf);
-      KC::to_f32(vw, vf);
-#pragma unroll
-      for (int h = 0; h < GROUP; ++h) {
-        float s = 0.f;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) s += qv[h][i] * kf[i];
-        s = group_sum_dpp<GW>(s) * scale;
-        m[h] = s;
-        l[h] = 1.f;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) acc[h][i] = vf[i];
-      }
-    }
-  }
-
-  // Latency discipline: batch-issue ALL of a cache block's K/V vectors
-  // for this lane-group (TPG k-loads + TPG v-loads back to back, plus
-  // the NEXT block's K prefetched) before any arithmetic touches them —
-  // one lane then has ~2*TPG+ loads in flight instead of 2, which is
-  // what moves this kernel from latency-bound to bandwidth-bound
-  // (guide Guideline 7/15: waits belong at the first consumer).
-  const int len_cache = FUSED ? len - 1 : len;   // FUSED: prefix only
-  const int n_blocks = (len_cache + block_size - 1) / block_size;
-  constexpr int TPG = 16 / GPW >= 1 ? 16 / GPW : 1;   // tokens per group @bs16
-  const int tok_per_grp = block_size / GPW;
-
-  // phys index fetched one pipeline stage AHEAD of its block's K/V
-  // issue: with the load inside issue_block the address of every K/V
-  // load depended on a just-issued block_table load and the compiler
-  // had to drain vmcnt before computing it, serializing the double
-  // buffer.
-  auto fetch_phys = [&](int b) -> int {
-    return block_table[int64_t(seq) * max_blocks + b];
-  };
-  using cvec8 = typename KC::vec8;
-  auto issue_block = [&](int phys, cvec8 (&kraw)[TPG], cvec8 (&vraw)[TPG]) {
-    const int64_t kv_base =
-        (int64_t(phys) * n_kv_heads + kvh) * block_size * D;
-#pragma unroll
-    for (int i = 0; i < TPG; ++i) {
-      if (i < tok_per_grp) {
-        const int tok = group + GPW * i;
-        kraw[i] = *reinterpret_cast<const cvec8*>(
-            k_cache + kv_base + int64_t(tok) * D + d0);
-        vraw[i] = *reinterpret_cast<const cvec8*>(
-            v_cache + kv_base + int64_t(tok) * D + d0);
-      }
-    }
-  };
-  auto consume_block = [&](int b, const cvec8 (&kraw)[TPG],
-                           const cvec8 (&vraw)[TPG]) {
-#pragma unroll
-    for (int i = 0; i < TPG; ++i) {
-      if (i >= tok_per_grp) break;
-      const int tok = group + GPW * i;         // token within the block
-      if (b * block_size + tok >= len_cache) continue;   // group-uniform tail
-      float kf[8], vf[8];
-      KC::to_f32(kraw[i], kf);
-      KC::to_f32(vraw[i], vf);
-
-      if constexpr (ABL == 3) {              // loads only
-#pragma unroll
-        for (int j = 0; j < 8; ++j) acc[0][j] += kf[j] + vf[j];
-        continue;
-      }
-#pragma unroll
-      for (int h = 0; h < GROUP; ++h) {
-        float s = 0.f;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) s += qv[h][j] * kf[j];
-        s = group_sum_dpp<GW>(s);
-        s *= scale;
-        if constexpr (ABL == 2) {            // no online softmax
-          l[h] += s;
-#pragma unroll
-          for (int j = 0; j < 8; ++j) acc[h][j] += s * vf[j];
-          continue;
-        }
-        const float m_new = fmaxf(m[h], s);
-        const float corr = __expf(m[h] - m_new);
-        const float p = __expf(s - m_new);
-        m[h] = m_new;
-        l[h] = l[h] * corr + p;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) acc[h][j] = acc[h][j] * corr + p * vf[j];
-      }
-    }
-  };
-
-  // Block-batched softmax consume: all TPG scores per head are computed
-  // before ONE running-max update for the whole block — the per-token
-  // form's serial corr/exp chain was 4.6 us of the 20.8 us kernel at
-  // batch 64 (RLLI_ATTN_ABLATE=2 vs 1); batching makes the TPG exps
-  // independent and pays one corr per (block, head).  Invalid tail
-  // tokens contribute exp(kNegInf - m_new) == 0 (kNegInf is a finite
-  // -1e30, so no -inf minus -inf NaN is reachable; every walked block
-  // holds at least one valid token, so m_new is always finite).
-  auto consume_block_batched = [&](int bb, const cvec8 (&kraw)[TPG],
-                                   const cvec8 (&vraw)[TPG]) {
-    float vfs[TPG][8];
-    float svals[GROUP][TPG];
-#pragma unroll
-    for (int i = 0; i < TPG; ++i) {
-      if (i >= tok_per_grp) break;
-      const int tok = group + GPW * i;
-      const bool valid = bb * block_size + tok < len_cache;
-      float kf[8];
-      KC::to_f32(kraw[i], kf);
-      KC::to_f32(vraw[i], vfs[i]);
-#pragma unroll
-      for (int h = 0; h < GROUP; ++h) {
-        float s = 0.f;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) s += qv[h][j] * kf[j];
-        s = group_sum_dpp<GW>(s) * scale;
-        svals[h][i] = valid ? s : kNegInf;
-      }
-    }
-#pragma unroll
-    for (int h = 0; h < GROUP; ++h) {
-      float m_new = m[h];
-#pragma unroll
-      for (int i = 0; i < TPG; ++i) {
-        if (i >= tok_per_grp) break;
-        m_new = fmaxf(m_new, svals[h][i]);
-      }
-      const float corr = __expf(m[h] - m_new);
-      float p[TPG], psum = 0.f;
-#pragma unroll
-      for (int i = 0; i < TPG; ++i) {
-        if (i >= tok_per_grp) break;
-        p[i] = __expf(svals[h][i] - m_new);
-        psum += p[i];
-      }
-      m[h] = m_new;
-      l[h] = l[h] * corr + psum;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        float t = acc[h][j] * corr;
-#pragma unroll
-        for (int i = 0; i < TPG; ++i) {
-          if (i >= tok_per_grp) break;
-          t += p[i] * vfs[i][j];
-        }
-        acc[h][j] = t;
-      }
-    }
-  };
-
-  const int bstride = n_waves * n_split;     // global block-chain count
-  if (tok_per_grp <= TPG) {
-    // depth-2 software pipeline over cache blocks: the NEXT block's
-    // K/V loads are in flight while this block computes (named A/B
-    // buffers, statically indexed — guide §5.4 rule 20)
-    cvec8 kA[TPG], vA[TPG], kB[TPG], vB[TPG];
-    int b = split * n_waves + wave;
-    int physA = 0, physB = 0;
-    if (b < n_blocks) {
-      physA = fetch_phys(b);
-      if (b + bstride < n_blocks) physB = fetch_phys(b + bstride);
-      issue_block(physA, kA, vA);
-    }
-    auto consume = [&](int bb, const cvec8 (&kraw)[TPG],
-                       const cvec8 (&vraw)[TPG]) {
-      if constexpr (ABL == 0)
-        consume_block_batched(bb, kraw, vraw);
-      else
-        consume_block(bb, kraw, vraw);
-    };
-    while (b < n_blocks) {
-      if (b + bstride < n_blocks) {
-        issue_block(physB, kB, vB);
-        if (b + 2 * bstride < n_blocks) physA = fetch_phys(b + 2 * bstride);
-      }
-      consume(b, kA, vA);
-      b += bstride;
-      if (b >= n_blocks) break;
-      if (b + bstride < n_blocks) {
-        issue_block(physA, kA, vA);
-        if (b + 2 * bstride < n_blocks) physB = fetch_phys(b + 2 * bstride);
-      }
-      consume(b, kB, vB);
-      b += bstride;
-    }
-  } else {
-    // oversized cache blocks: plain per-sub-batch loop
-    for (int b = split * n_waves + wave; b < n_blocks; b += bstride) {
-      const int phys = block_table[int64_t(seq) * max_blocks + b];
-      const int64_t kv_base =
-          (int64_t(phys) * n_kv_heads + kvh) * block_size * D;
-      for (int bi = 0; bi < tok_per_grp; ++bi) {
-        const int tok = group + GPW * bi;
-        if (b * block_size + tok >= len_cache) continue;
-        float kf[8], vf[8];
-        KC::to_f32(*reinterpret_cast<const cvec8*>(
-            k_cache + kv_base + int64_t(tok) * D + d0), kf);
-        KC::to_f32(*reinterpret_cast<const cvec8*>(
-            v_cache + kv_base + int64_t(tok) * D + d0), vf);
-#pragma unroll
-        for (int h = 0; h < GROUP; ++h) {
-          float s = 0.f;
-#pragma unroll
-          for (int j = 0; j < 8; ++j) s += qv[h][j] * kf[j];
-          s = group_sum_dpp<GW>(s);
-          s *= scale;
-          const float m_new = fmaxf(m[h], s);
-          const float corr = __expf(m[h] - m_new);
-          const float p = __expf(s - m_new);
-          m[h] = m_new;
-          l[h] = l[h] * corr + p;
-#pragma unroll
-          for (int j = 0; j < 8; ++j)
-            acc[h][j] = acc[h][j] * corr + p * vf[j];
-        }
-      }
-    }
-  }
-
-  if constexpr (ABL != 0) {
-    // ablation: no LDS publish/merge — wave 0's lane-groups dump their
-    // raw partials straight to out (wrong values, comparable traffic)
-    if (wave == 0) {
-#pragma unroll
-      for (int h = 0; h < GROUP; ++h) {
-        bf16x8 o;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) o.s[j] = f32_to_bf16(acc[h][j] + l[h]);
-        if (group == 0)
-          *reinterpret_cast<uint4*>(
-              out + (int64_t(seq) * n_kv_heads * GROUP + kvh * GROUP + h) * D +
-              d0) = o.u;
-      }
-    }
-    return;
-  }
-
-  // ---- in-wave cross-group merge (log-sum-exp): lanes off apart hold
-  // the same d0 slice for sibling lane-groups, so GPW partials combine
-  // with shuffles instead of LDS round-trips — the LDS image shrinks
-  // GPWx (16 -> 4 partials at GW=16) and the final scan with it (the
-  // full publish+merge was 4.1 us of the 20.8 us kernel at batch 64,
-  // RLLI_ATTN_ABLATE=1 vs 0).  kNegInf is finite, so idle lane-groups
-  // (m = kNegInf, l = 0) combine as weight-0 with no -inf-inf NaN.
-#pragma unroll
-  for (int off = GW; off < 64; off <<= 1) {
-#pragma unroll
-    for (int h = 0; h < GROUP; ++h) {
-      const float m_o = __shfl_xor(m[h], off, kWave);
-      const float l_o = __shfl_xor(l[h], off, kWave);
-      const float M = fmaxf(m[h], m_o);
-      const float wa = __expf(m[h] - M);
-      const float wb = __expf(m_o - M);
-      l[h] = l[h] * wa + l_o * wb;
-#pragma unroll
-      for (int j = 0; j < 8; ++j)
-        acc[h][j] = acc[h][j] * wa + __shfl_xor(acc[h][j], off, kWave) * wb;
-      m[h] = M;
-    }
-  }
-
-  // ---- publish one partial per WAVE (group 0 lanes carry the merged
-  // value for their d0 slice) ----
-  if (group == 0) {
-#pragma unroll
-    for (int h = 0; h < GROUP; ++h) {
-      float* dst = accs + ((int64_t(wave) * GROUP + h) * D) + d0;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) dst[j] = acc[h][j];
-      if (gl == 0) {
-        ml[(wave * GROUP + h) * 2 + 0] = m[h];
-        ml[(wave * GROUP + h) * 2 + 1] = l[h];
-      }
-    }
-  }
-  __syncthreads();
-
-  // ---- merge: each thread owns (head, dim) output elements ----
-  const int n_wpart = n_waves;
-  for (int idx = threadIdx.x; idx < GROUP * D; idx += blockDim.x) {
-    const int h = idx / D;
-    const int d = idx % D;
-    float M = kNegInf;
-    for (int p = 0; p < n_wpart; ++p)
-      M = fmaxf(M, ml[(p * GROUP + h) * 2 + 0]);
-    float num = 0.f, den = 0.f;
-    for (int p = 0; p < n_wpart; ++p) {
-      const float w = __expf(ml[(p * GROUP + h) * 2 + 0] - M);
-      num += w * accs[(int64_t(p) * GROUP + h) * D + d];
-      den += w * ml[(p * GROUP + h) * 2 + 1];
-    }
-    if (n_split == 1) {
-      out[(int64_t(seq) * n_kv_heads * GROUP + kvh * GROUP + h) * D + d] =
-          f32_to_bf16(den > 0.f ? num / den : 0.f);
-    } else {
-      // unnormalized partial in this split's max-frame; a split whose
-      // block range was empty publishes M=-inf/den=0 and combines to 0
-      const int64_t pb = (int64_t(sk) * n_split + split) * GROUP + h;
-      part_out[pb * D + d] = num;
-      if (d == 0) {
-        part_ml[pb * 2 + 0] = M;
-        part_ml[pb * 2 + 1] = den;
-      }
-    }
-  }
-}
-
-// Reduce n_split partials per (sequence, kv-head): one WG per (seq,
-// kv-head), threads stride over GROUP*D output elements.
-__global__ __launch_bounds__(256)
-void decode_combine_kernel(const float* __restrict__ part,
-                           const float* __restrict__ ml,
-                           uint16_t* __restrict__ out,
-                           int n_split, int group, int D) {
-  const int sk = blockIdx.x;
-  const int ghd = group * D;
-  for (int idx = threadIdx.x; idx < ghd; idx += blockDim.x) {
-    const int h = idx / D;
-    float M = kNegInf;
-    for (int s = 0; s < n_split; ++s)
-      M = fmaxf(M, ml[((int64_t(sk) * n_split + s) * group + h) * 2]);
-    float num = 0.f, den = 0.f;
-    if (M > kNegInf) {
-      for (int s = 0; s < n_split; ++s) {
-        const int64_t b = (int64_t(sk) * n_split + s) * group + h;
-        const float w = __expf(ml[b * 2] - M);
-        num += w * part[(int64_t(sk) * n_split + s) * ghd + idx];
-        den += w * ml[b * 2 + 1];
-      }
-    }
-    out[int64_t(sk) * ghd + idx] = f32_to_bf16(den > 0.f ? num / den : 0.f);
-  }
-}
-
-struct FusedArgs {
-  const uint16_t* k_src = nullptr;
-  const uint16_t* v_src = nullptr;
-  const int32_t* positions = nullptr;
-  const float* cos_sin = nullptr;
-  const int32_t* slot_mapping = nullptr;
-  void* k_cache_w = nullptr;     // cache-codec elem type
-  void* v_cache_w = nullptr;
+struct DecodeArgs {
+  const uint16_t* q;       // rows q_stride apart: q heads (| k | v: fused)
+  const float* parts;      // or n_parts f32 parts of them, to be summed
+  const void *k_cache, *v_cache;     // [blocks, n_kv, block, D]
+  void *k_cache_w, *v_cache_w;
+  const int32_t* block_table;
+  const int32_t* seq_lens;
+  const int32_t* positions;
+  const float* cos_sin;
+  const int32_t* slot_mapping;
+  uint16_t* out;
+  float* part_out;         // shares: [n_kv, shares + batch, GROUP, D]
+  float* part_ml;          //         [.., GROUP, 2]
+  int batch, n_kv, block_size, max_blocks, q_stride, n_parts, shares;
+  float scale;
 };
 
-template <int GW, int GROUP, typename KC>
-void dispatch_decode(const uint16_t* q, const void* k_cache_v,
-                     const void* v_cache_v, const int32_t* block_table,
-                     const int32_t* seq_lens, uint16_t* out, int batch,
-                     int n_kv_heads, int block_size, int max_blocks,
-                     float scale, int q_stride, const FusedArgs* fa,
-                     int n_split, float* part_out, float* part_ml,
-                     hipStream_t stream) {
-  using CElem = typename KC::elem;
-  const CElem* k_cache = static_cast<const CElem*>(k_cache_v);
-  const CElem* v_cache = static_cast<const CElem*>(v_cache_v);
-  constexpr int D = GW * 8;
-  const int n_part = 4;          // one in-wave-merged partial per wave
-  const size_t smem = size_t(n_part) * GROUP * (D + 2) * sizeof(float);
-  const dim3 grid(batch * n_kv_heads * n_split);
-  auto launch = [&](auto bs_tag, auto abl_tag) {
-    constexpr int BS = decltype(bs_tag)::value;
-    constexpr int ABL = decltype(abl_tag)::value;
-    if (fa != nullptr) {
-      hipLaunchKernelGGL((decode_attn_kernel<GW, GROUP, true, BS, ABL, KC>),
-                         grid, dim3(256), smem, stream,
-                         q, k_cache, v_cache, block_table, seq_lens, out,
-                         n_kv_heads, block_size, max_blocks, scale, q_stride,
-                         fa->k_src, fa->v_src, fa->positions, fa->cos_sin,
-                         fa->slot_mapping,
-                         static_cast<CElem*>(fa->k_cache_w),
-                         static_cast<CElem*>(fa->v_cache_w),
-                         n_split, part_out, part_ml);
+DEV_INLINE int units_of(int len) { return (len + UNIT - 1) / UNIT; }
+
+// How many units a part may have, so that ``shares`` parts cover all
+// sequences (each ends in one that is not full).
+DEV_INLINE int part_size(const DecodeArgs& a) {
+  int t = 0;
+  for (int s = threadIdx.x & 63; s < a.batch; s += 64)
+    t += units_of(a.seq_lens[s]);
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) t += __shfl_xor(t, d, kWave);
+  return max((__builtin_amdgcn_readfirstlane(t) + a.shares - 1) / a.shares,
+             MIN_UNITS);
+}
+
+DEV_INLINE int parts_of(int len, int size) {
+  return (units_of(len) + size - 1) / size;
+}
+
+// Parts of the sequences ahead of ``seq``.
+DEV_INLINE int parts_before(const DecodeArgs& a, int size, int seq) {
+  int t = 0;
+  for (int s = threadIdx.x & 63; s < seq; s += 64)
+    t += parts_of(a.seq_lens[s], size);
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) t += __shfl_xor(t, d, kWave);
+  return __builtin_amdgcn_readfirstlane(t);
+}
+
+// The sequence that part number ``part`` belongs to (a.batch: none) and
+// which of its parts it is.
+DEV_INLINE int find_part(const DecodeArgs& a, int size, int part, int& rel) {
+  const int lane = threadIdx.x & 63;
+  int before = 0;
+  for (int s0 = 0; s0 < a.batch; s0 += 64) {
+    const int mine =
+        s0 + lane < a.batch ? parts_of(a.seq_lens[s0 + lane], size) : 0;
+    int upto = mine;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int t = __shfl_up(upto, d, kWave);
+      if (lane >= d) upto += t;
+    }
+    const int at = part - before;
+    const uint64_t hit = __ballot(at < upto && at >= upto - mine);
+    if (hit) {
+      const int src = __ffsll(static_cast<unsigned long long>(hit)) - 1;
+      rel = __builtin_amdgcn_readfirstlane(
+          at - __shfl(upto - mine, src, kWave));
+      return __builtin_amdgcn_readfirstlane(s0 + src);
+    }
+    before += __shfl(upto, 63, kWave);
+  }
+  rel = 0;
+  return a.batch;
+}
+
+// for what goes through LDS; loads from memory stay under way
+DEV_INLINE void lds_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+// the column eight away has the other part
+DEV_INLINE float other_part(float v) { return dpp_mov_f32<0x128>(v); }
+
+// N bytes of cache elements, in registers
+template <int N>
+struct Words {
+  typedef uint32_t type __attribute__((ext_vector_type(N / 4)));
+};
+template <>
+struct Words<4> {
+  using type = uint32_t;
+};
+
+DEV_INLINE uint32_t word(uint32_t w, int) { return w; }
+template <typename V>
+DEV_INLINE uint32_t word(const V& w, int i) { return w[i]; }
+
+DEV_INLINE uint32_t bf16_pair(float a, float b) {
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 b16x2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint32_t,
+                            __builtin_convertvector((f32x2{a, b}), b16x2));
+}
+
+// cache elements as bf16 (8-bit ones are exact in it), two per dword
+template <typename KC, int N, typename R>
+DEV_INLINE void widen(const R& raw, uint32_t (&out)[N]) {
+  if constexpr (std::is_same<KC, CacheBF16>::value) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) out[i] = word(raw, i);
+  } else {
+#pragma unroll
+    for (int i = 0; i < N; i += 2) {
+      const int w = int(word(raw, i / 2));
+      const f32x2_cvt a = __builtin_amdgcn_cvt_pk_f32_fp8(w, false);
+      const f32x2_cvt b = __builtin_amdgcn_cvt_pk_f32_fp8(w, true);
+      out[i] = bf16_pair(a.x, a.y);
+      out[i + 1] = bf16_pair(b.x, b.y);
+    }
+  }
+}
+
+// BS: block size of the cache where it is known (0: any)
+template <int D, int GROUP, typename KC, int BS, bool FUSED, bool SHARES>
+__global__ __launch_bounds__(256, 3)
+void decode_attn_kernel(DecodeArgs a) {
+  using elem = typename KC::elem;
+  using vec8 = typename KC::vec8;
+  constexpr int KSTEPS = D / 32;
+  constexpr int VT = D / 16;               // channel tiles
+  using kraw = typename Words<sizeof(elem) * 8>::type;
+  using vraw = typename Words<sizeof(elem) * VT>::type;
+  constexpr int QROW = D + 8;
+  __shared__ __attribute__((aligned(16))) float raw[(GROUP + 2) * D];
+  __shared__ __attribute__((aligned(16))) uint16_t qs[16 * QROW];
+  __shared__ __attribute__((aligned(16))) elem self[2 * D];       // k | v
+  __shared__ __attribute__((aligned(16))) float accs[4 * GROUP * D];
+  __shared__ float ml[4 * GROUP * 2];
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int col = lane & 15, oct = lane >> 4;
+  const int head = col & 7;
+  const bool lower = col >= 8;
+  const int bs = BS ? BS : a.block_size;
+  const elem* kc = static_cast<const elem*>(a.k_cache);
+  const elem* vc = static_cast<const elem*>(a.v_cache);
+  const int n_q = a.n_kv * GROUP;
+  const float c2 = a.scale * 1.4426950408889634f;
+
+  int kvh, seq, part = 0, u0 = 0, u1, n_parts = 1;
+  if constexpr (SHARES) {
+    kvh = blockIdx.x % a.n_kv;
+    part = blockIdx.x / a.n_kv;
+    const int size = part_size(a);
+    int rel;
+    seq = find_part(a, size, part, rel);
+    if (seq >= a.batch) return;
+    const int all = units_of(a.seq_lens[seq]);
+    n_parts = parts_of(a.seq_lens[seq], size);
+    u0 = all * rel / n_parts;
+    u1 = all * (rel + 1) / n_parts;
+  } else {
+    seq = blockIdx.x / a.n_kv;
+    kvh = blockIdx.x % a.n_kv;
+    u1 = units_of(a.seq_lens[seq]);
+  }
+  const int len = a.seq_lens[seq];
+  // whether this workgroup appends the new token
+  const bool newest = FUSED && a.slot_mapping && u1 == units_of(len);
+
+  const int32_t* table = a.block_table + int64_t(seq) * a.max_blocks;
+  const int last = len - 1;
+  // Pages of a unit: of its two halves where a half lies in one page,
+  // otherwise of this lane's key and value tokens.
+  constexpr int NPG = BS == 16 ? 2 : 10;
+  int page[NPG];
+  auto key_tok = [&](int u, int t) {     // tokens past the last repeat it
+    return min(u * UNIT + t * 16 + col, last);
+  };
+  auto value_tok = [&](int u, int t, int i) {
+    return min(u * UNIT + t * 16 + oct * 4 + i, last);
+  };
+  auto look_up = [&](int u) {
+    if (u >= u1) return;
+    if constexpr (BS == 16) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t) page[t] = table[min(u * 2 + t, last / 16)];
     } else {
-      hipLaunchKernelGGL((decode_attn_kernel<GW, GROUP, false, BS, ABL, KC>),
-                         grid, dim3(256), smem, stream,
-                         q, k_cache, v_cache, block_table, seq_lens, out,
-                         n_kv_heads, block_size, max_blocks, scale, q_stride,
-                         nullptr, nullptr, nullptr, nullptr, nullptr,
-                         nullptr, nullptr, n_split, part_out, part_ml);
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        page[t * 5] = table[key_tok(u, t) / bs];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          page[t * 5 + 1 + i] = table[value_tok(u, t, i) / bs];
+      }
     }
   };
-  using I0 = std::integral_constant<int, 0>;
-  // RLLI_ATTN_ABLATE: perf-ablation kernels (WRONG results — bench
-  // only; instantiated for the bf16 cache only)
-  static const int abl = [] {
-    const char* e = std::getenv("RLLI_ATTN_ABLATE");
-    return e ? atoi(e) : 0;
-  }();
-  if (block_size == 16) {
-    using B16 = std::integral_constant<int, 16>;
-    if constexpr (std::is_same_v<KC, CacheBF16>) {
-      switch (abl) {
-        case 1: launch(B16{}, std::integral_constant<int, 1>{}); break;
-        case 2: launch(B16{}, std::integral_constant<int, 2>{}); break;
-        case 3: launch(B16{}, std::integral_constant<int, 3>{}); break;
-        default: launch(B16{}, I0{});
-      }
-    } else {
-      launch(B16{}, I0{});
+  auto row_of = [&](int u, int t, int i, int tok) -> int64_t {
+    if constexpr (BS == 16)
+      return (int64_t(page[t]) * a.n_kv + kvh) * 16 + tok -
+             min(u * 2 + t, last / 16) * 16;
+    else
+      return (int64_t(page[t * 5 + i]) * a.n_kv + kvh) * bs + tok % bs;
+  };
+  kraw kr[2][KSTEPS];
+  vraw vr[2][4];
+  auto load_keys = [&](int u) {
+    if (u >= u1) return;
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const elem* p = kc + row_of(u, t, 0, key_tok(u, t)) * D + oct * 8;
+#pragma unroll
+      for (int k = 0; k < KSTEPS; ++k)
+        kr[t][k] = *reinterpret_cast<const kraw*>(p + k * 32);
     }
-  } else {
-    launch(I0{}, I0{});
+  };
+  auto load_values = [&](int u) {
+    if (u >= u1) return;
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        vr[t][i] = *reinterpret_cast<const vraw*>(
+            vc + row_of(u, t, 1 + i, value_tok(u, t, i)) * D + col * VT);
+  };
+  look_up(u0 + wave);
+  load_keys(u0 + wave);
+  load_values(u0 + wave);
+  look_up(u0 + wave + 4);
+
+  // ---- the heads' queries (and the new key and value) -----------------
+  const int n_in = (GROUP + (newest ? 2 : 0)) * D;
+  for (int e = tid * 4; e < n_in; e += 1024) {
+    int at = kvh * GROUP * D + e;
+    if (e >= GROUP * D) {
+      const int r = e - GROUP * D;
+      at = r < D ? (n_q + kvh) * D + r : (n_q + a.n_kv + kvh) * D + r - D;
+    }
+    f32x4 v;
+    if (a.parts) {
+      const float* p = a.parts + int64_t(seq) * a.q_stride + at;
+      const int64_t step = int64_t(a.batch) * a.q_stride;
+      v = *reinterpret_cast<const f32x4*>(p);
+      for (int s = 1; s < a.n_parts; ++s)
+        v += *reinterpret_cast<const f32x4*>(p + s * step);
+      // the product is a 16-bit one
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = bf16_to_f32(f32_to_bf16(v[i]));
+    } else {
+      const uint2 w = *reinterpret_cast<const uint2*>(
+          a.q + int64_t(seq) * a.q_stride + at);
+      v = f32x4{__builtin_bit_cast(float, w.x << 16),
+                __builtin_bit_cast(float, w.x & 0xffff0000u),
+                __builtin_bit_cast(float, w.y << 16),
+                __builtin_bit_cast(float, w.y & 0xffff0000u)};
+    }
+    *reinterpret_cast<f32x4*>(raw + e) = v;
   }
-  if (n_split > 1) {
-    hipLaunchKernelGGL(decode_combine_kernel, dim3(batch * n_kv_heads),
-                       dim3(256), 0, stream, part_out, part_ml, out,
-                       n_split, GROUP, D);
+  lds_barrier();
+  {
+    constexpr int HALF = D / 2;
+    const float* cs =
+        FUSED ? a.cos_sin + int64_t(a.positions[seq]) * D : nullptr;
+    auto store = [&](int h, int d, float v) {
+      const uint16_t up = f32_to_bf16(v);
+      qs[h * QROW + d] = up;
+      qs[(8 + h) * QROW + d] = f32_to_bf16(v - bf16_to_f32(up));
+    };
+    for (int e = tid; e < (GROUP + (newest ? 1 : 0)) * HALF; e += 256) {
+      const int h = e / HALF, j = e % HALF;
+      const float u = raw[h * D + j], v = raw[h * D + HALF + j];
+      float x = u, y = v;
+      if constexpr (FUSED) {
+        const float c = cs[j], s = cs[HALF + j];
+        x = u * c - v * s;
+        y = v * c + u * s;
+      }
+      if (h < GROUP) {
+        store(h, j, x);
+        store(h, HALF + j, y);
+      } else {
+        raw[h * D + j] = x;
+        raw[h * D + HALF + j] = y;
+      }
+    }
   }
+  lds_barrier();
+  if (newest) {
+    // append at cache precision; this step sees what later ones will
+    if (tid < 2 * D / 8) {
+      const int e = tid * 8;
+      const vec8 w = KC::from_f32(raw + GROUP * D + e);
+      const int slot = a.slot_mapping[seq];
+      elem* to = static_cast<elem*>(e < D ? a.k_cache_w : a.v_cache_w);
+      *reinterpret_cast<vec8*>(
+          to + ((int64_t(slot / bs) * a.n_kv + kvh) * bs + slot % bs) * D +
+          e % D) = w;
+      *reinterpret_cast<vec8*>(self + e) = w;
+    }
+    lds_barrier();
+  }
+  s16x8 qf[KSTEPS];
+#pragma unroll
+  for (int k = 0; k < KSTEPS; ++k) {
+    uint4 w{0, 0, 0, 0};
+    if (head < GROUP)
+      w = *reinterpret_cast<const uint4*>(qs + col * QROW + k * 32 +
+                                          oct * 8);
+    qf[k] = __builtin_bit_cast(s16x8, w);
+  }
+
+  // ---- units; the next one's loads as soon as registers are free ------
+  f32x4 o[VT];
+#pragma unroll
+  for (int t = 0; t < VT; ++t) o[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float m = kNegInf, l = 0.f;
+  for (int u = u0 + wave; u < u1; u += 4) {
+    const int tok0 = u * UNIT;
+    if (newest && tok0 + UNIT > last) {
+      // the new token's key and value instead of what its slot held
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        const bool own = key_tok(u, t) == last;
+#pragma unroll
+        for (int k = 0; k < KSTEPS; ++k) {
+          const kraw w =
+              *reinterpret_cast<const kraw*>(self + k * 32 + oct * 8);
+          kr[t][k] = own ? w : kr[t][k];
+        }
+      }
+      const vraw w = *reinterpret_cast<const vraw*>(self + D + col * VT);
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          vr[t][i] = value_tok(u, t, i) == last ? w : vr[t][i];
+    }
+    f32x4 s[2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      s[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int k = 0; k < KSTEPS; ++k) {
+        uint32_t w[4];
+        widen<KC>(kr[t][k], w);
+        s[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+            __builtin_bit_cast(s16x8, (uint4{w[0], w[1], w[2], w[3]})),
+            qf[k], s[t], 0, 0, 0);
+      }
+    }
+    load_keys(u + 4);
+    float mx = kNegInf;
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int tok = tok0 + t * 16 + oct * 4 + r;
+        const float v = (s[t][r] + other_part(s[t][r])) * c2;
+        s[t][r] = tok <= last ? v : kNegInf;
+        mx = fmaxf(mx, s[t][r]);
+      }
+    mx = fmaxf(mx, __shfl_xor(mx, 16, kWave));
+    mx = fmaxf(mx, __shfl_xor(mx, 32, kWave));
+    const float mn = fmaxf(m, mx);
+    if (!__all(mn == m)) {
+      const float corr = __builtin_amdgcn_exp2f(m - mn);
+      l *= corr;
+#pragma unroll
+      for (int t = 0; t < VT; ++t) o[t] *= corr;
+      m = mn;
+    }
+    uint32_t pw[4];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      float p[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        p[r] = __builtin_amdgcn_exp2f(s[t][r] - m);
+        l += p[r];
+      }
+      const uint32_t u01 = bf16_pair(p[0], p[1]), u23 = bf16_pair(p[2], p[3]);
+      const uint32_t l01 =
+          bf16_pair(p[0] - __builtin_bit_cast(float, u01 << 16),
+                    p[1] - __builtin_bit_cast(float, u01 & 0xffff0000u));
+      const uint32_t l23 =
+          bf16_pair(p[2] - __builtin_bit_cast(float, u23 << 16),
+                    p[3] - __builtin_bit_cast(float, u23 & 0xffff0000u));
+      pw[t * 2] = lower ? l01 : u01;
+      pw[t * 2 + 1] = lower ? l23 : u23;
+    }
+    const s16x8 pf =
+        __builtin_bit_cast(s16x8, (uint4{pw[0], pw[1], pw[2], pw[3]}));
+    uint32_t vw[2][4][VT / 2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) widen<KC>(vr[t][i], vw[t][i]);
+#pragma unroll
+    for (int t = 0; t < VT; ++t) {
+      const uint32_t sel = t & 1 ? 0x07060302u : 0x05040100u;
+      const int d = t / 2;
+      const uint4 w = {
+          __builtin_amdgcn_perm(vw[0][1][d], vw[0][0][d], sel),
+          __builtin_amdgcn_perm(vw[0][3][d], vw[0][2][d], sel),
+          __builtin_amdgcn_perm(vw[1][1][d], vw[1][0][d], sel),
+          __builtin_amdgcn_perm(vw[1][3][d], vw[1][2][d], sel)};
+      o[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+          __builtin_bit_cast(s16x8, w), pf, o[t], 0, 0, 0);
+    }
+    load_values(u + 4);
+    look_up(u + 8);
+  }
+
+  // ---- the four waves' results, through LDS ---------------------------
+  l += __shfl_xor(l, 16, kWave);
+  l += __shfl_xor(l, 32, kWave);
+#pragma unroll
+  for (int t = 0; t < VT; ++t)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) o[t][r] += other_part(o[t][r]);
+  if (col < GROUP) {
+    float* to = accs + (wave * GROUP + col) * D + oct * 4 * VT;
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int t = 0; t < VT; t += 4)
+        *reinterpret_cast<f32x4*>(to + r * VT + t) =
+            f32x4{o[t][r], o[t + 1][r], o[t + 2][r], o[t + 3][r]};
+    if (oct == 0) {
+      ml[(wave * GROUP + col) * 2] = m;
+      ml[(wave * GROUP + col) * 2 + 1] = l;
+    }
+  }
+  lds_barrier();
+  const bool whole = !SHARES || n_parts == 1;
+  const int64_t slot =
+      (int64_t(kvh) * (a.shares + a.batch) + part) * GROUP;
+  for (int e = tid; e < GROUP * D; e += 256) {
+    const int h = e / D, d = e % D;
+    float M = kNegInf;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) M = fmaxf(M, ml[(w * GROUP + h) * 2]);
+    float num = 0.f, den = 0.f;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      const float c = __builtin_amdgcn_exp2f(ml[(w * GROUP + h) * 2] - M);
+      num += c * accs[(w * GROUP + h) * D + d];
+      den += c * ml[(w * GROUP + h) * 2 + 1];
+    }
+    if (whole) {
+      a.out[(int64_t(seq) * n_q + kvh * GROUP + h) * D + d] =
+          f32_to_bf16(den > 0.f ? num / den : 0.f);
+    } else {
+      a.part_out[(slot + h) * D + d] = num;
+      if (d == 0) {
+        a.part_ml[(slot + h) * 2] = M;
+        a.part_ml[(slot + h) * 2 + 1] = den;
+      }
+    }
+  }
+  }
+
+// Sequences of several parts (and those without tokens).  A
+// workgroup per (sequence, query head): D / 4 threads have a part's channels,
+// the others other parts.
+template <int D, int GROUP>
+__global__ __launch_bounds__(256)
+void decode_combine_kernel(DecodeArgs a) {
+  constexpr int TD = D / 4, NG = 256 / TD;
+  const int n_q = a.n_kv * GROUP;
+  const int seq = blockIdx.x / n_q, h = blockIdx.x % n_q;
+  const int kvh = h / GROUP;
+  const int size = part_size(a);
+  const int n = parts_of(a.seq_lens[seq], size);
+  if (n == 1) return;
+  const int first = parts_before(a, size, seq);
+  const int td = threadIdx.x % TD, tg = threadIdx.x / TD;
+  const int64_t slot0 =
+      (int64_t(kvh) * (a.shares + a.batch) + first) * GROUP + h % GROUP;
+  const float* po = a.part_out + slot0 * D + td * 4;
+  const float* pm = a.part_ml + slot0 * 2;
+  float M = kNegInf, den = 0.f;
+  f32x4 num = {0.f, 0.f, 0.f, 0.f};
+  // four parts' loads at a time
+  for (int g = tg; g < n; g += 4 * NG) {
+    f32x4 v[4];
+    float mm[4], ll[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const bool ok = g + i * NG < n;
+      const int64_t at = int64_t(ok ? g + i * NG : g) * GROUP;
+      v[i] = *reinterpret_cast<const f32x4*>(po + at * D);
+      mm[i] = ok ? pm[at * 2] : kNegInf;
+      ll[i] = ok ? pm[at * 2 + 1] : 0.f;
+    }
+    const float mn =
+        fmaxf(M, fmaxf(fmaxf(mm[0], mm[1]), fmaxf(mm[2], mm[3])));
+    const float corr = __builtin_amdgcn_exp2f(M - mn);
+    num *= corr;
+    den *= corr;
+    M = mn;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float c = g + i * NG < n ? __builtin_amdgcn_exp2f(mm[i] - mn) : 0.f;
+      num += c * v[i];
+      den += c * ll[i];
+    }
+  }
+  __shared__ f32x4 nums[NG][TD];
+  __shared__ float ms[NG], dens[NG];
+  nums[tg][td] = num;
+  if (td == 0) {
+    ms[tg] = M;
+    dens[tg] = den;
+  }
+  __syncthreads();
+  if (threadIdx.x >= D) return;
+  M = kNegInf;
+#pragma unroll
+  for (int g = 0; g < NG; ++g) M = fmaxf(M, ms[g]);
+  float x = 0.f, y = 0.f;
+#pragma unroll
+  for (int g = 0; g < NG; ++g) {
+    const float c = __builtin_amdgcn_exp2f(ms[g] - M);
+    x += c * nums[g][threadIdx.x / 4][threadIdx.x % 4];
+    y += c * dens[g];
+  }
+  a.out[(int64_t(seq) * n_q + h) * D + threadIdx.x] =
+      f32_to_bf16(y > 0.f ? x / y : 0.f);
+}
+
+template <int D, int GROUP, typename KC, bool FUSED>
+void run(const DecodeArgs& a, hipStream_t st) {
+  auto go = [&](auto bs) {
+    constexpr int BS = decltype(bs)::value;
+    if (a.shares > 0) {
+      hipLaunchKernelGGL((decode_attn_kernel<D, GROUP, KC, BS, FUSED, true>),
+                         dim3((a.shares + a.batch) * a.n_kv), dim3(256), 0, st, a);
+      hipLaunchKernelGGL((decode_combine_kernel<D, GROUP>),
+                         dim3(a.batch * a.n_kv * GROUP), dim3(256), 0, st, a);
+    } else {
+      hipLaunchKernelGGL((decode_attn_kernel<D, GROUP, KC, BS, FUSED, false>),
+                         dim3(a.batch * a.n_kv), dim3(256), 0, st, a);
+    }
+  };
+  if (a.block_size == 16) go(std::integral_constant<int, 16>{});
+  else go(std::integral_constant<int, 0>{});
+}
+
+template <bool FUSED>
+void dispatch(const DecodeArgs& a, int group, int head_dim, bool fp8,
+              hipStream_t st) {
+  if (a.batch == 0) return;
+  auto by_cache = [&](auto d, auto g) {
+    constexpr int D = decltype(d)::value, G = decltype(g)::value;
+    if (fp8) run<D, G, CacheFP8, FUSED>(a, st);
+    else run<D, G, CacheBF16, FUSED>(a, st);
+  };
+  auto by_group = [&](auto d) {
+    if (group == 1) by_cache(d, std::integral_constant<int, 1>{});
+    else if (group == 2) by_cache(d, std::integral_constant<int, 2>{});
+    else if (group == 4) by_cache(d, std::integral_constant<int, 4>{});
+    else if (group == 8) by_cache(d, std::integral_constant<int, 8>{});
+  };
+  if (head_dim == 128) by_group(std::integral_constant<int, 128>{});
+  else if (head_dim == 64) by_group(std::integral_constant<int, 64>{});
 }
 
 }  // namespace
 
-// Split factor so decode fills the chip: 256 CUs want >=512 workgroups
-// in flight; small batches (interactive / long-context) get their
-// sequences split across block-chains instead of idling CUs.
-int decode_attn_n_split(int batch, int n_kv_heads) {
-  // RLLI_ATTN_SPLIT forces the factor (A/B tuning); 0/unset = heuristic
-  static const int forced = [] {
-    const char* e = std::getenv("RLLI_ATTN_SPLIT");
-    return e ? atoi(e) : 0;
-  }();
-  if (forced > 0) return forced > 16 ? 16 : forced;
-  const int wgs = batch * n_kv_heads;
-  if (wgs >= 384) return 1;
-  int n = (512 + wgs - 1) / wgs;
-  return n > 16 ? 16 : n;
+int decode_attn_shares(int batch, int n_kv_heads, int max_tokens) {
+  static const bool off = std::getenv("RLLI_NO_SPLITK") != nullptr;
+  if (off) return 0;
+  if (batch * n_kv_heads >= 384 && max_tokens <= 1024) return 0;
+  if (max_tokens <= MIN_UNITS * UNIT) return 0;      // never cut
+  return std::max(1, 512 / n_kv_heads);
 }
 
-void launch_decode_attn_impl(const uint16_t* q, const void* k_cache,
-                             const void* v_cache,
-                             const int32_t* block_table,
-                             const int32_t* seq_lens, uint16_t* out,
-                             int batch, int n_q_heads, int n_kv_heads,
-                             int head_dim, int block_size, int max_blocks,
-                             float scale, int q_stride, const FusedArgs* fa,
-                             int n_split, float* part_out, float* part_ml,
-                             bool cache_fp8, hipStream_t stream) {
-  if (batch == 0) return;
-  if (part_out == nullptr) n_split = 1;
-  const int group = n_q_heads / n_kv_heads;
-  auto run = [&](auto gw_tag, auto group_tag) {
-    if (cache_fp8)
-      dispatch_decode<decltype(gw_tag)::value, decltype(group_tag)::value,
-                      CacheFP8>(
-          q, k_cache, v_cache, block_table, seq_lens, out, batch, n_kv_heads,
-          block_size, max_blocks, scale, q_stride, fa, n_split, part_out,
-          part_ml, stream);
-    else
-      dispatch_decode<decltype(gw_tag)::value, decltype(group_tag)::value,
-                      CacheBF16>(
-          q, k_cache, v_cache, block_table, seq_lens, out, batch, n_kv_heads,
-          block_size, max_blocks, scale, q_stride, fa, n_split, part_out,
-          part_ml, stream);
-  };
-  using I8 = std::integral_constant<int, 8>;
-  using I16 = std::integral_constant<int, 16>;
-  using G1 = std::integral_constant<int, 1>;
-  using G2 = std::integral_constant<int, 2>;
-  using G4 = std::integral_constant<int, 4>;
-  using G8 = std::integral_constant<int, 8>;
-  if (head_dim == 128) {
-    if (group == 1) run(I16{}, G1{});
-    else if (group == 2) run(I16{}, G2{});
-    else if (group == 4) run(I16{}, G4{});
-    else if (group == 8) run(I16{}, G8{});
-    else return;   // caller validates
-  } else if (head_dim == 64) {
-    if (group == 1) run(I8{}, G1{});
-    else if (group == 2) run(I8{}, G2{});
-    else if (group == 4) run(I8{}, G4{});
-    else if (group == 8) run(I8{}, G8{});
-    else return;
-  }
-}
-
-void launch_decode_attn(const uint16_t* q, const void* k_cache,
-                        const void* v_cache, const int32_t* block_table,
-                        const int32_t* seq_lens, uint16_t* out, int batch,
-                        int n_q_heads, int n_kv_heads, int head_dim,
-                        int block_size, int max_blocks, float scale,
-                        int q_stride, int n_split, float* part_out,
-                        float* part_ml, bool cache_fp8, hipStream_t stream) {
-  launch_decode_attn_impl(q, k_cache, v_cache, block_table, seq_lens, out,
-                          batch, n_q_heads, n_kv_heads, head_dim, block_size,
-                          max_blocks, scale, q_stride, nullptr,
-                          n_split, part_out, part_ml, cache_fp8, stream);
-}
-
-void launch_decode_attn_fused(
-    const uint16_t* qkv, void* k_cache, void* v_cache,
-    const int32_t* block_table, const int32_t* seq_lens,
+void launch_decode_attn(
+    const uint16_t* q, const float* parts, int n_parts, void* k_cache,
+    void* v_cache, const int32_t* block_table, const int32_t* seq_lens,
     const int32_t* positions, const float* cos_sin,
     const int32_t* slot_mapping, uint16_t* out, int batch, int n_q_heads,
-    int n_kv_heads, int head_dim, int block_size, int max_blocks,
-    float scale, int qkv_stride, int n_split, float* part_out,
-    float* part_ml, bool cache_fp8, hipStream_t stream) {
-  FusedArgs fa;
-  fa.k_src = qkv + n_q_heads * head_dim;
-  fa.v_src = qkv + (n_q_heads + n_kv_heads) * head_dim;
-  fa.positions = positions;
-  fa.cos_sin = cos_sin;
-  fa.slot_mapping = slot_mapping;
-  fa.k_cache_w = k_cache;
-  fa.v_cache_w = v_cache;
-  launch_decode_attn_impl(qkv, k_cache, v_cache, block_table, seq_lens, out,
-                          batch, n_q_heads, n_kv_heads, head_dim, block_size,
-                          max_blocks, scale, qkv_stride, &fa,
-                          n_split, part_out, part_ml, cache_fp8, stream);
+    int n_kv_heads, int head_dim, int block_size, int max_blocks, float scale,
+    int q_stride, int shares, float* part_out, float* part_ml, bool cache_fp8,
+    hipStream_t stream) {
+  const DecodeArgs a{q, parts, k_cache, v_cache, k_cache, v_cache,
+                     block_table, seq_lens, positions, cos_sin, slot_mapping,
+                     out, part_out, part_ml, batch, n_kv_heads, block_size,
+                     max_blocks, q_stride, n_parts, shares, scale};
+  const int group = n_q_heads / n_kv_heads;
+  if (positions) dispatch<true>(a, group, head_dim, cache_fp8, stream);
+  else dispatch<false>(a, group, head_dim, cache_fp8, stream);
 }
 
 }  // namespace rlli

@@ -110,6 +110,30 @@ std::tuple<Tensor, Tensor> rmsnorm_fp8(const Tensor& x, const Tensor& w,
   return {y8, scales};
 }
 
+// rmsnorm_residual_ with x = the sum of f32 parts [n, rows, dim]
+Tensor rmsnorm_residual_parts_(const Tensor& parts, Tensor residual,
+                               const Tensor& w, double eps) {
+  check_bf16_contig(residual, "residual");
+  check_bf16_contig(w, "w");
+  const int64_t dim = residual.size(-1);
+  TORCH_CHECK(parts.scalar_type() == at::kFloat && parts.is_cuda() &&
+                  parts.is_contiguous() && parts.dim() == 3 &&
+                  parts.size(2) == dim &&
+                  parts.size(1) * dim == residual.numel() &&
+                  w.numel() == dim,
+              "parts must be contiguous f32 [n, rows, dim]");
+  TORCH_CHECK(dim % 8 == 0 && dim <= 8192, "dim must be a multiple of 8, at "
+              "most 8192, got ", dim);
+  Tensor y = at::empty_like(residual);
+  c10::hip::HIPGuardMasqueradingAsCUDA guard(residual.device());
+  rlli::launch_rmsnorm_parts(parts.data_ptr<float>(), int(parts.size(0)),
+                             bf16_ptr(residual), bf16_ptr(w), bf16_ptr(y),
+                             int(parts.size(1)), int(dim), float(eps),
+                             current_stream(residual));
+  check_launch("rmsnorm_residual_parts_");
+  return y;
+}
+
 std::tuple<Tensor, Tensor> rmsnorm_residual_fp8(const Tensor& x,
                                                 Tensor residual,
                                                 const Tensor& w, double eps) {
@@ -228,64 +252,114 @@ void rope_kv_append_qkv_(Tensor qkv, const Tensor& positions,
   check_launch("rope_kv_append_qkv_");
 }
 
-
-// split-K scratch for decode attention (empty tensors when n_split==1);
-// allocation participates in hipGraph capture pools, so graphed decode
-// buckets capture their scratch once and reuse it on replay.
-struct SplitScratch {
-  int n_split = 1;
-  Tensor part, ml;
-  float* part_ptr() { return n_split > 1 ? part.data_ptr<float>() : nullptr; }
-  float* ml_ptr() { return n_split > 1 ? ml.data_ptr<float>() : nullptr; }
-};
-
-static SplitScratch make_split_scratch(const Tensor& ref, int batch,
-                                       int n_kv, int group, int D) {
-  SplitScratch s;
-  static const bool disabled = std::getenv("RLLI_NO_SPLITK") != nullptr;
-  if (disabled) return s;
-  s.n_split = rlli::decode_attn_n_split(batch, n_kv);
-  if (s.n_split > 1) {
-    auto opt = ref.options().dtype(at::kFloat);
-    s.part = at::empty({int64_t(batch) * n_kv * s.n_split * group * D}, opt);
-    s.ml = at::empty({int64_t(batch) * n_kv * s.n_split * group * 2}, opt);
-  }
-  return s;
+// The same without the queries, which stay as they are.
+void kv_append_qkv_(Tensor qkv, const Tensor& positions,
+                    const Tensor& cos_sin, Tensor k_cache, Tensor v_cache,
+                    const Tensor& slot_mapping, int64_t n_q) {
+  check_bf16_contig(qkv, "qkv");
+  const bool cache_fp8 = check_cache(k_cache, v_cache);
+  const int n_kv = int(k_cache.size(1));
+  const int D = int(k_cache.size(3));
+  const int stride = int(qkv.size(1));
+  const int tokens = int(qkv.size(0));
+  TORCH_CHECK(stride == (n_q + 2 * n_kv) * D, "qkv width mismatch");
+  TORCH_CHECK(positions.numel() == tokens && slot_mapping.numel() == tokens);
+  TORCH_CHECK(cos_sin.size(1) == D && D % 16 == 0);
+  uint16_t* base = bf16_ptr(qkv);
+  c10::hip::HIPGuardMasqueradingAsCUDA guard(qkv.device());
+  rlli::launch_rope_kv_append(
+      base, base + n_q * D, base + (n_q + n_kv) * D,
+      positions.data_ptr<int32_t>(), cos_sin.data_ptr<float>(),
+      k_cache.data_ptr(), v_cache.data_ptr(),
+      slot_mapping.data_ptr<int32_t>(), tokens, 0, n_kv, D,
+      int(k_cache.size(2)), stride, stride, cache_fp8, current_stream(qkv));
+  check_launch("kv_append_qkv_");
 }
 
 // ---------------------------------------------------------- decode_attn
+// One launch for all forms.  q: bf16 rows that start with the query heads
+// ([batch, .., stride]), or f32 parts [n, batch, stride] whose sum they are.
+// With ``positions`` queries are rotated here; with ``slot_mapping`` as well
+// the rows are q | k | v, and key and value are appended.
+static Tensor decode_attn_any(const Tensor& q, int64_t n_q,
+                              const Tensor& k_cache, const Tensor& v_cache,
+                              const Tensor& block_table,
+                              const Tensor& seq_lens, double scale,
+                              const Tensor* positions, const Tensor* cos_sin,
+                              const Tensor* slot_mapping) {
+  const bool parts = q.scalar_type() == at::kFloat;
+  if (parts) {
+    TORCH_CHECK(q.is_cuda() && q.is_contiguous() && q.dim() == 3,
+                "parts must be contiguous f32 [n, batch, width]");
+  } else {
+    check_bf16_contig(q, "q");
+  }
+  const bool cache_fp8 = check_cache(k_cache, v_cache);
+  for (const Tensor* t : {&block_table, &seq_lens})
+    TORCH_CHECK(t->scalar_type() == at::kInt && t->is_contiguous(),
+                "tables and lengths must be contiguous int32");
+  const int batch = int(q.size(parts ? 1 : 0));
+  const int stride = batch ? int(q.numel() / batch / (parts ? q.size(0) : 1))
+                           : 0;
+  const int n_kv = int(k_cache.size(1));
+  const int block_size = int(k_cache.size(2));
+  const int D = int(k_cache.size(3));
+  const int max_blocks = int(block_table.size(1));
+  const int group = int(n_q) / n_kv;
+  TORCH_CHECK(n_q % n_kv == 0 && (group == 1 || group == 2 || group == 4 ||
+                                  group == 8),
+              "GQA group must be 1/2/4/8, got ", group);
+  TORCH_CHECK(D == 64 || D == 128, "head_dim must be 64 or 128, got ", D);
+  TORCH_CHECK(block_size > 0 && v_cache.sizes() == k_cache.sizes());
+  TORCH_CHECK(block_table.size(0) == batch && seq_lens.numel() == batch);
+  Tensor out = at::empty({batch, n_q * D},
+                         q.options().dtype(at::kBFloat16));
+  if (batch == 0) return out;
+  c10::hip::HIPGuardMasqueradingAsCUDA guard(q.device());
+  // scratch of sequences that several workgroups share; allocated here, so
+  // that a captured step keeps its own
+  const int shares =
+      rlli::decode_attn_shares(batch, n_kv, max_blocks * block_size);
+  Tensor part, ml;
+  if (shares > 0) {
+    const int64_t slots = int64_t(n_kv) * (shares + batch) * group;
+    auto opt = q.options().dtype(at::kFloat);
+    part = at::empty({slots, D}, opt);
+    ml = at::empty({slots, 2}, opt);
+  }
+  rlli::launch_decode_attn(
+      parts ? nullptr : bf16_ptr(q), parts ? q.data_ptr<float>() : nullptr,
+      parts ? int(q.size(0)) : 0, k_cache.data_ptr(), v_cache.data_ptr(),
+      block_table.data_ptr<int32_t>(), seq_lens.data_ptr<int32_t>(),
+      positions ? positions->data_ptr<int32_t>() : nullptr,
+      cos_sin ? cos_sin->data_ptr<float>() : nullptr,
+      slot_mapping ? slot_mapping->data_ptr<int32_t>() : nullptr,
+      bf16_ptr(out), batch, int(n_q), n_kv, D, block_size, max_blocks,
+      float(scale), stride, shares,
+      shares > 0 ? part.data_ptr<float>() : nullptr,
+      shares > 0 ? ml.data_ptr<float>() : nullptr, cache_fp8,
+      current_stream(q));
+  check_launch("decode_attn");
+  return out;
+}
+
 Tensor decode_attn(const Tensor& q, const Tensor& k_cache,
                    const Tensor& v_cache, const Tensor& block_table,
                    const Tensor& seq_lens, double scale) {
   check_bf16_contig(q, "q");
-  const bool cache_fp8 = check_cache(k_cache, v_cache);
-  TORCH_CHECK(block_table.scalar_type() == at::kInt && block_table.is_contiguous());
-  TORCH_CHECK(seq_lens.scalar_type() == at::kInt && seq_lens.is_contiguous());
-  const int batch = int(q.size(0));
-  const int n_q = int(q.size(1));
-  const int D = int(q.size(2));
-  const int n_kv = int(k_cache.size(1));
-  const int block_size = int(k_cache.size(2));
-  const int max_blocks = int(block_table.size(1));
-  const int group = n_q / n_kv;
-  TORCH_CHECK(n_q % n_kv == 0 && (group == 1 || group == 2 || group == 4 || group == 8),
-              "GQA group must be 1/2/4/8, got ", group);
-  TORCH_CHECK(D == 64 || D == 128, "head_dim must be 64 or 128, got ", D);
-  const int gpw = 64 / (D / 8);
-  TORCH_CHECK(block_size % gpw == 0, "block_size must be a multiple of ", gpw);
-  TORCH_CHECK(k_cache.size(3) == D && v_cache.sizes() == k_cache.sizes());
-  TORCH_CHECK(block_table.size(0) == batch && seq_lens.numel() == batch);
-  Tensor out = at::empty_like(q);
-  c10::hip::HIPGuardMasqueradingAsCUDA guard(q.device());
-  SplitScratch ss = make_split_scratch(q, batch, n_kv, group, D);
-  rlli::launch_decode_attn(
-      bf16_ptr(q), k_cache.data_ptr(), v_cache.data_ptr(),
-      block_table.data_ptr<int32_t>(), seq_lens.data_ptr<int32_t>(),
-      bf16_ptr(out), batch, n_q, n_kv, D, block_size, max_blocks,
-      float(scale), n_q * D, ss.n_split, ss.part_ptr(), ss.ml_ptr(),
-      cache_fp8, current_stream(q));
-  check_launch("decode_attn");
-  return out;
+  TORCH_CHECK(q.dim() == 3 && q.size(2) == k_cache.size(3));
+  const int gpw = 64 / (int(q.size(2)) / 8);
+  TORCH_CHECK(k_cache.size(2) % gpw == 0, "block_size must be a multiple of ",
+              gpw);
+  return decode_attn_any(q, q.size(1), k_cache, v_cache, block_table,
+                         seq_lens, scale, nullptr, nullptr, nullptr)
+      .view(q.sizes());
+}
+
+static void check_qkv_width(const Tensor& qkv, const Tensor& k_cache,
+                            int64_t n_q) {
+  TORCH_CHECK(qkv.size(-1) == (n_q + 2 * k_cache.size(1)) * k_cache.size(3),
+              "qkv width mismatch");
 }
 
 // Fused-QKV decode attention: q read strided from the qkv GEMM output.
@@ -293,67 +367,42 @@ Tensor decode_attn_qkv(const Tensor& qkv, const Tensor& k_cache,
                        const Tensor& v_cache, const Tensor& block_table,
                        const Tensor& seq_lens, double scale, int64_t n_q) {
   check_bf16_contig(qkv, "qkv");
-  const bool cache_fp8 = check_cache(k_cache, v_cache);
-  const int batch = int(qkv.size(0));
-  const int n_kv = int(k_cache.size(1));
-  const int D = int(k_cache.size(3));
-  const int block_size = int(k_cache.size(2));
-  const int max_blocks = int(block_table.size(1));
-  const int stride = int(qkv.size(1));
-  TORCH_CHECK(stride == (n_q + 2 * n_kv) * D, "qkv width mismatch");
-  const int group = int(n_q) / n_kv;
-  TORCH_CHECK(group == 1 || group == 2 || group == 4 || group == 8);
-  TORCH_CHECK(D == 64 || D == 128);
-  Tensor out = at::empty({batch, n_q * D}, qkv.options());
-  c10::hip::HIPGuardMasqueradingAsCUDA guard(qkv.device());
-  SplitScratch ss = make_split_scratch(qkv, batch, n_kv, group, D);
-  rlli::launch_decode_attn(
-      bf16_ptr(qkv), k_cache.data_ptr(), v_cache.data_ptr(),
-      block_table.data_ptr<int32_t>(), seq_lens.data_ptr<int32_t>(),
-      bf16_ptr(out), batch, int(n_q), n_kv, D, block_size, max_blocks,
-      float(scale), stride, ss.n_split, ss.part_ptr(), ss.ml_ptr(),
-      cache_fp8, current_stream(qkv));
-  check_launch("decode_attn_qkv");
-  return out;
+  check_qkv_width(qkv, k_cache, n_q);
+  return decode_attn_any(qkv, n_q, k_cache, v_cache, block_table, seq_lens,
+                         scale, nullptr, nullptr, nullptr);
 }
 
-// Fused decode: rope + append + attention in one kernel.
+// Fused decode: rope + append + attention in one kernel.  qkv: bf16 rows, or
+// the f32 parts of rows_linear_parts.
 Tensor decode_attn_rope_qkv(const Tensor& qkv, const Tensor& positions,
                             const Tensor& cos_sin, Tensor k_cache,
                             Tensor v_cache, const Tensor& slot_mapping,
                             const Tensor& block_table, const Tensor& seq_lens,
                             double scale, int64_t n_q) {
-  check_bf16_contig(qkv, "qkv");
-  const bool cache_fp8 = check_cache(k_cache, v_cache);
   TORCH_CHECK(positions.scalar_type() == at::kInt && positions.is_contiguous());
   TORCH_CHECK(slot_mapping.scalar_type() == at::kInt && slot_mapping.is_contiguous());
   TORCH_CHECK(cos_sin.scalar_type() == at::kFloat && cos_sin.is_contiguous());
-  TORCH_CHECK(block_table.scalar_type() == at::kInt && block_table.is_contiguous());
-  TORCH_CHECK(seq_lens.scalar_type() == at::kInt && seq_lens.is_contiguous());
-  const int batch = int(qkv.size(0));
-  const int n_kv = int(k_cache.size(1));
-  const int block_size = int(k_cache.size(2));
-  const int D = int(k_cache.size(3));
-  const int stride = int(qkv.size(1));
-  TORCH_CHECK(stride == (n_q + 2 * n_kv) * D, "qkv width mismatch");
-  const int group = int(n_q) / n_kv;
-  TORCH_CHECK(group == 1 || group == 2 || group == 4 || group == 8);
-  TORCH_CHECK(D == 64 || D == 128);
-  TORCH_CHECK(cos_sin.size(1) == D);
-  const int max_blocks = int(block_table.size(1));
-  Tensor out = at::empty({batch, n_q * D}, qkv.options());
-  c10::hip::HIPGuardMasqueradingAsCUDA guard(qkv.device());
-  SplitScratch ss = make_split_scratch(qkv, batch, n_kv, group, D);
-  rlli::launch_decode_attn_fused(
-      bf16_ptr(qkv), k_cache.data_ptr(), v_cache.data_ptr(),
-      block_table.data_ptr<int32_t>(), seq_lens.data_ptr<int32_t>(),
-      positions.data_ptr<int32_t>(), cos_sin.data_ptr<float>(),
-      slot_mapping.data_ptr<int32_t>(), bf16_ptr(out), batch, int(n_q),
-      n_kv, D, block_size, max_blocks, float(scale), stride,
-      ss.n_split, ss.part_ptr(), ss.ml_ptr(), cache_fp8,
-      current_stream(qkv));
-  check_launch("decode_attn_rope_qkv");
-  return out;
+  TORCH_CHECK(cos_sin.size(1) == k_cache.size(3));
+  const int64_t batch = qkv.size(qkv.dim() == 3 ? 1 : 0);
+  TORCH_CHECK(positions.numel() == batch && slot_mapping.numel() == batch);
+  check_qkv_width(qkv, k_cache, n_q);
+  return decode_attn_any(qkv, n_q, k_cache, v_cache, block_table, seq_lens,
+                         scale, &positions, &cos_sin, &slot_mapping);
+}
+
+// Queries rotated here, everything they see already in the cache.
+Tensor decode_attn_q_rope(const Tensor& qkv, const Tensor& positions,
+                          const Tensor& cos_sin, const Tensor& k_cache,
+                          const Tensor& v_cache, const Tensor& block_table,
+                          const Tensor& seq_lens, double scale, int64_t n_q) {
+  check_bf16_contig(qkv, "qkv");
+  TORCH_CHECK(positions.scalar_type() == at::kInt && positions.is_contiguous());
+  TORCH_CHECK(cos_sin.scalar_type() == at::kFloat && cos_sin.is_contiguous());
+  TORCH_CHECK(cos_sin.size(1) == k_cache.size(3) &&
+              positions.numel() == qkv.size(0));
+  check_qkv_width(qkv, k_cache, n_q);
+  return decode_attn_any(qkv, n_q, k_cache, v_cache, block_table, seq_lens,
+                         scale, &positions, &cos_sin, nullptr);
 }
 
 // --------------------------------------------------------- prefill_attn
@@ -453,7 +502,7 @@ static void check_rows(const Tensor& x, const Tensor& w) {
   check_bf16_contig(w, "w");
   TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && w.size(1) == x.size(1),
               "x/W K mismatch");
-  TORCH_CHECK(x.size(0) >= 1 && x.size(0) <= 64, "1 to 64 rows, got ",
+  TORCH_CHECK(x.size(0) >= 1 && x.size(0) <= 128, "1 to 128 rows, got ",
               x.size(0));
   TORCH_CHECK(x.size(1) % 64 == 0 && x.size(1) > 0 && w.size(0) % 4 == 0 &&
                   w.size(0) > 0,
@@ -496,7 +545,8 @@ Tensor rows_linear(const Tensor& x, const Tensor& w) {
 Tensor rows_linear_silu(const Tensor& x, const Tensor& w) {
   check_rows(x, w);
   const int inter = int(w.size(0)) / 2;
-  TORCH_CHECK(w.size(0) % 8 == 0, "gate and up rows are multiples of 4");
+  TORCH_CHECK(w.size(0) % 16 == 0, "gate and up rows are multiples of 8");
+  if (!rlli::rows_gemm_silu_ok(inter)) return silu_mul(rows_linear(x, w));
   c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
   Tensor out = at::empty({x.size(0), inter}, x.options());
   rlli::launch_rows_gemm_silu(bf16_ptr(x), bf16_ptr(w), bf16_ptr(out),
@@ -587,6 +637,7 @@ Tensor sample(const Tensor& logits, const Tensor& temperatures,
 TORCH_LIBRARY(rlli, m) {
   m.def("rmsnorm(Tensor x, Tensor w, float eps) -> Tensor");
   m.def("rmsnorm_residual_(Tensor x, Tensor(a!) residual, Tensor w, float eps) -> Tensor");
+  m.def("rmsnorm_residual_parts_(Tensor parts, Tensor(a!) residual, Tensor w, float eps) -> Tensor");
   m.def("silu_mul(Tensor gate_up) -> Tensor");
   m.def("rmsnorm_fp8(Tensor x, Tensor w, float eps) -> (Tensor, Tensor)");
   m.def("rmsnorm_residual_fp8(Tensor x, Tensor(a!) residual, Tensor w, float eps) -> (Tensor, Tensor)");
@@ -604,6 +655,12 @@ TORCH_LIBRARY(rlli, m) {
   m.def("decode_attn_rope_qkv(Tensor qkv, Tensor positions, Tensor cos_sin, "
         "Tensor(a!) k_cache, Tensor(b!) v_cache, Tensor slot_mapping, "
         "Tensor block_table, Tensor seq_lens, float scale, int n_q) -> Tensor");
+  m.def("kv_append_qkv_(Tensor(a!) qkv, Tensor positions, Tensor cos_sin, "
+        "Tensor(b!) k_cache, Tensor(c!) v_cache, Tensor slot_mapping, "
+        "int n_q) -> ()");
+  m.def("decode_attn_q_rope(Tensor qkv, Tensor positions, Tensor cos_sin, "
+        "Tensor k_cache, Tensor v_cache, Tensor block_table, "
+        "Tensor seq_lens, float scale, int n_q) -> Tensor");
   m.def("prefill_attn_qkv(Tensor qkv, Tensor cu_seqlens, float scale, "
         "int n_q, int n_kv, int head_dim) -> Tensor");
   m.def("prefill_attn(Tensor q, Tensor k, Tensor v, Tensor cu_seqlens, "
@@ -625,6 +682,7 @@ TORCH_LIBRARY(rlli, m) {
 TORCH_LIBRARY_IMPL(rlli, CUDA, m) {
   m.impl("rmsnorm", &rmsnorm);
   m.impl("rmsnorm_residual_", &rmsnorm_residual_);
+  m.impl("rmsnorm_residual_parts_", &rmsnorm_residual_parts_);
   m.impl("silu_mul", &silu_mul);
   m.impl("rmsnorm_fp8", &rmsnorm_fp8);
   m.impl("rmsnorm_residual_fp8", &rmsnorm_residual_fp8);
@@ -634,6 +692,8 @@ TORCH_LIBRARY_IMPL(rlli, CUDA, m) {
   m.impl("rope_kv_append_qkv_", &rope_kv_append_qkv_);
   m.impl("decode_attn_qkv", &decode_attn_qkv);
   m.impl("decode_attn_rope_qkv", &decode_attn_rope_qkv);
+  m.impl("kv_append_qkv_", &kv_append_qkv_);
+  m.impl("decode_attn_q_rope", &decode_attn_q_rope);
   m.impl("prefill_attn_qkv", &prefill_attn_qkv);
   m.impl("prefill_attn", &prefill_attn);
   m.impl("sample", &sample);

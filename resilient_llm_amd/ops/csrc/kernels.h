@@ -14,6 +14,11 @@ void launch_rmsnorm(const uint16_t* x, uint16_t* residual, const uint16_t* w,
                     uint16_t* y, int rows, int dim, float eps,
                     hipStream_t stream);
 
+// The same with x = the sum of n f32 parts [n, rows, dim]; dim <= 8192.
+void launch_rmsnorm_parts(const float* parts, int n, uint16_t* residual,
+                          const uint16_t* w, uint16_t* y, int rows, int dim,
+                          float eps, hipStream_t stream);
+
 // out[t, i] = silu(gu[t, i]) * gu[t, I + i]   for packed gate|up rows
 void launch_silu_mul(const uint16_t* gate_up, uint16_t* out, int rows,
                      int inter, hipStream_t stream);
@@ -43,35 +48,25 @@ void launch_rope_kv_append(
     int block_size, int q_stride, int kv_stride, bool cache_fp8,
     hipStream_t stream);
 
-// Split-K factor for decode attention (flash-decode): >1 when
-// batch*n_kv_heads workgroups cannot fill 256 CUs.  The caller sizes
-// the f32 scratch as [batch*n_kv*n_split*group*head_dim] (part_out)
-// and [batch*n_kv*n_split*group*2] (part_ml) and passes both; n_split=1
-// (or null scratch) is the classic single-workgroup-per-(seq,head) path.
-int decode_attn_n_split(int batch, int n_kv_heads);
-
-// Paged GQA decode attention: one new q token per sequence.
+// Paged GQA decode attention, one new query per sequence.  Fused form
+// (positions given): q | k | v rows, or their f32 parts, are rotated and
+// appended as well (no slot_mapping: queries are rotated, nothing appended).  decode_attn_shares: equal shares of all sequences'
+// tokens that workgroups take per key/value head, 0: a workgroup takes a
+// whole sequence.  Then part_out [n_kv, shares + batch, group, head_dim]
+// and part_ml [.., group, 2] are needed.
+int decode_attn_shares(int batch, int n_kv_heads, int max_tokens);
 void launch_decode_attn(
-    const uint16_t* q,                 // [batch, n_q_heads, head_dim]
-    const void* k_cache,               // [blocks, n_kv, block_size, head_dim]
-    const void* v_cache,
+    const uint16_t* q,                 // [batch, q_stride], or null:
+    const float* parts, int n_parts,   // [n_parts, batch, q_stride]
+    void* k_cache,                     // [blocks, n_kv, block_size, head_dim]
+    void* v_cache,
     const int32_t* block_table,        // [batch, max_blocks]
     const int32_t* seq_lens,           // [batch]
+    const int32_t* positions,          // [batch] or null
+    const float* cos_sin, const int32_t* slot_mapping,    // or null
     uint16_t* out,                     // [batch, n_q_heads, head_dim]
-    int batch, int n_q_heads, int n_kv_heads, int head_dim,
-    int block_size, int max_blocks, float scale, int q_stride,
-    int n_split, float* part_out, float* part_ml, bool cache_fp8,
-    hipStream_t stream);
-
-// Fused decode: rope(q,k) + cache append + paged attention in ONE
-// kernel (decode path; qkv is the raw fused GEMM output).
-void launch_decode_attn_fused(
-    const uint16_t* qkv, void* k_cache, void* v_cache,
-    const int32_t* block_table, const int32_t* seq_lens,
-    const int32_t* positions, const float* cos_sin,
-    const int32_t* slot_mapping, uint16_t* out, int batch, int n_q_heads,
-    int n_kv_heads, int head_dim, int block_size, int max_blocks,
-    float scale, int qkv_stride, int n_split, float* part_out,
+    int batch, int n_q_heads, int n_kv_heads, int head_dim, int block_size,
+    int max_blocks, float scale, int q_stride, int shares, float* part_out,
     float* part_ml, bool cache_fp8, hipStream_t stream);
 
 // Varlen causal prefill attention over in-batch q/k/v.
@@ -102,7 +97,7 @@ void launch_prefill_paged(const uint16_t* qkv, const void* k_cache,
                           int block_size, float scale, bool cache_fp8,
                           hipStream_t stream);
 
-// Products of at most 64 rows, y[M, N] = x[M, K] w[N, K]^T (rows_gemm.hip).
+// Products of at most 128 rows, y[M, N] = x[M, K] w[N, K]^T (rows_gemm.hip).
 // With parts given, f32 [splits, M, N] whose sum is y; otherwise out.
 // N % 4 == 0, K % 64 == 0, 16-byte aligned rows.
 int rows_gemm_splits(int N, int K);

@@ -14,7 +14,9 @@
 // weights are the second product's operand as they are, keys in the order
 // 0-3, 8-11 | 4-7, 12-15 of sixteen.  Its other operand, values by channel,
 // is read from the row-major tile with the transposing LDS read in just that
-// order, so nothing transposes values on the way in.
+// order, so nothing transposes values on the way in.  A query's accumulators
+// are scaled again only when its maximum has grown by 2^8 since they last
+// were; until then weights are up to 2^8, with the same relative rounding.
 //
 // Bounds: for long prompts the products (32 MFMA of 32 cycles a tile and
 // wave) beside about as many cycles of exponentials and conversions and of
@@ -301,7 +303,7 @@ void prefill_flash_kernel(Src src, uint16_t* __restrict__ out, int n_tiles,
     mx = fmaxf(mx, __shfl_xor(mx, 32, kWave));
     // each query by itself, so that a row's result does not depend on the
     // rows it shares a tile with
-    const bool grown = mx > m;
+    const bool grown = (mx - m) * c2 > 8.f;
     if (__any(grown)) {
       const float mn = grown ? mx : m;
       const float corr = __builtin_amdgcn_exp2f((m - mn) * c2);

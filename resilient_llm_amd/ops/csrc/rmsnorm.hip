@@ -88,6 +88,54 @@ __global__ void rmsnorm_one_vec(const uint16_t* __restrict__ x,
   }
 }
 
+// The residual form where x is a product in f32 parts (rows_gemm.hip): they
+// are summed here, in order, and rounded once with the residual.  Latency of
+// one row's loads bounds it; a launch and a pass of their own for the sum
+// cost 2 to 4 us.
+__global__ void rmsnorm_parts_kernel(const float* __restrict__ parts, int n,
+                                     uint16_t* __restrict__ residual,
+                                     const uint16_t* __restrict__ w,
+                                     uint16_t* __restrict__ y, int dim,
+                                     float eps) {
+  __shared__ float lds[16];
+  const int64_t base = int64_t(blockIdx.x) * dim;
+  const int64_t step = int64_t(gridDim.x) * dim;
+  const int d = threadIdx.x * 8;
+  const bool active = d < dim;
+  float vals[8] = {};
+  bf16x8 wv, out;
+  if (active) {
+    bf16x8 rv;
+    rv.u = *reinterpret_cast<const uint4*>(residual + base + d);
+    wv.u = *reinterpret_cast<const uint4*>(w + d);
+    const float* p = parts + base + d;
+#pragma unroll 4
+    for (int s = 0; s < n; ++s) {
+      const float4 a = *reinterpret_cast<const float4*>(p + s * step);
+      const float4 b = *reinterpret_cast<const float4*>(p + s * step + 4);
+      vals[0] += a.x; vals[1] += a.y; vals[2] += a.z; vals[3] += a.w;
+      vals[4] += b.x; vals[5] += b.y; vals[6] += b.z; vals[7] += b.w;
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      out.s[i] = f32_to_bf16(vals[i] + bf16_to_f32(rv.s[i]));
+      vals[i] = bf16_to_f32(out.s[i]);      // y is of the stored residual
+    }
+    *reinterpret_cast<uint4*>(residual + base + d) = out.u;
+  }
+  float ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) ss += vals[i] * vals[i];
+  ss = block_sum<16>(ss, lds);
+  const float inv = rsqrtf(ss / dim + eps);
+  if (active) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      out.s[i] = f32_to_bf16(vals[i] * inv * bf16_to_f32(wv.s[i]));
+    *reinterpret_cast<uint4*>(y + base + d) = out.u;
+  }
+}
+
 // Large dims: pass 1 accumulates sumsq (and stores fused residual),
 // pass 2 re-reads (L2-hot) and writes.
 template <bool FUSE_RESIDUAL>
@@ -331,6 +379,15 @@ void launch_rmsnorm_fp8(const uint16_t* x, uint16_t* residual,
     hipLaunchKernelGGL((rmsnorm_one_vec_fp8<false>), dim3(rows),
                        dim3(threads), smem, stream, x, nullptr, w, y8,
                        scales, dim, eps);
+}
+
+void launch_rmsnorm_parts(const float* parts, int n, uint16_t* residual,
+                          const uint16_t* w, uint16_t* y, int rows, int dim,
+                          float eps, hipStream_t stream) {
+  if (rows == 0) return;
+  const int threads = ((dim / 8 + kWave - 1) / kWave) * kWave;
+  hipLaunchKernelGGL(rmsnorm_parts_kernel, dim3(rows), dim3(threads), 0,
+                     stream, parts, n, residual, w, y, dim, eps);
 }
 
 void launch_rmsnorm(const uint16_t* x, uint16_t* residual, const uint16_t* w,

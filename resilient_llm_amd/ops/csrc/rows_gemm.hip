@@ -1,5 +1,5 @@
 // Products of few rows with a weight matrix, as decoding has them:
-// y[M, N] = x[M, K] w[N, K]^T, M <= 64, bf16 with f32 sums.
+// y[M, N] = x[M, K] w[N, K]^T, M <= 128, bf16 with f32 sums.
 //
 // What there is to do is to read w once; everything else has to stay out of
 // its way.  A workgroup has 64 (or 128) rows of w over a range of K, four
@@ -239,13 +239,13 @@ void sum_parts_kernel(const float* __restrict__ parts,
       uint2{pack2(v[0], v[1]), pack2(v[2], v[3])};
 }
 
-// R32, R64: steps in the ring with 32 and with 64 rows of x
-template <int CT, int R32, int R64, int OUT>
+// R32, R64, R128: steps in the ring with as many rows of x
+template <int CT, int R32, int R64, int R128, int OUT>
 void go(const uint16_t* x, const uint16_t* w, void* out, int M, int N, int K,
         int panels, int splits, hipStream_t st) {
   auto run = [&](auto xr, auto mt) {
     constexpr int XR = decltype(xr)::value, MT = decltype(mt)::value;
-    constexpr int R = XR == 32 ? R32 : R64;
+    constexpr int R = XR == 32 ? R32 : XR == 64 ? R64 : R128;
     constexpr size_t smem = size_t(R) * (4 * CT * 16 + XR) * LINE * 2;
     auto* k = rows_gemm_kernel<CT, XR, MT, R, OUT>;
     if (smem > 65536)
@@ -260,11 +260,16 @@ void go(const uint16_t* x, const uint16_t* w, void* out, int M, int N, int K,
   using I3 = std::integral_constant<int, 3>;
   using I4 = std::integral_constant<int, 4>;
   using X32 = std::integral_constant<int, 32>;
+  using I6 = std::integral_constant<int, 6>;
+  using I8 = std::integral_constant<int, 8>;
   using X64 = std::integral_constant<int, 64>;
+  using X128 = std::integral_constant<int, 128>;
   if (M <= 16) run(X32{}, I1{});
   else if (M <= 32) run(X32{}, I2{});
   else if (M <= 48) run(X64{}, I3{});
-  else run(X64{}, I4{});
+  else if (M <= 64) run(X64{}, I4{});
+  else if (M <= 96) run(X128{}, I6{});
+  else run(X128{}, I8{});
 }
 
 }  // namespace
@@ -289,11 +294,11 @@ void launch_rows_gemm(const uint16_t* x, const uint16_t* w, float* parts,
                       hipStream_t st) {
   const int panels = (N + 63) / 64;
   if (parts)
-    go<1, 6, 5, OUT_PARTS>(x, w, parts, M, N, K, panels, splits, st);
+    go<1, 6, 5, 5, OUT_PARTS>(x, w, parts, M, N, K, panels, splits, st);
   else if (panels < 400)
-    go<1, 6, 5, OUT_BF16>(x, w, out, M, N, K, panels, 1, st);
+    go<1, 6, 5, 3, OUT_BF16>(x, w, out, M, N, K, panels, 1, st);
   else
-    go<2, 3, 3, OUT_BF16>(x, w, out, M, N, K, (N + 127) / 128, 1, st);
+    go<2, 3, 3, 4, OUT_BF16>(x, w, out, M, N, K, (N + 127) / 128, 1, st);
 }
 
 // Panels of 64 pairs where they cover the CUs, of 32 otherwise (14336 pairs
@@ -304,10 +309,10 @@ void launch_rows_gemm_silu(const uint16_t* x, const uint16_t* w,
                            uint16_t* out, int M, int inter, int K,
                            hipStream_t st) {
   if ((inter + 63) / 64 >= 200)
-    go<2, 5, 5, OUT_SILU>(x, w, out, M, 2 * inter, K, (inter + 63) / 64, 1,
+    go<2, 5, 5, 4, OUT_SILU>(x, w, out, M, 2 * inter, K, (inter + 63) / 64, 1,
                           st);
   else
-    go<1, 6, 5, OUT_SILU>(x, w, out, M, 2 * inter, K, (inter + 31) / 32, 1,
+    go<1, 6, 5, 3, OUT_SILU>(x, w, out, M, 2 * inter, K, (inter + 31) / 32, 1,
                           st);
 }
 

@@ -7,7 +7,6 @@ us/call and effective TB/s against the op's minimum HBM traffic.
 
 Env knobs (statics in the .so, so A/B variants need fresh processes):
   RLLI_WAVE_NORM=1    wave-per-row rmsnorm variant
-  RLLI_ATTN_SPLIT=N   force decode-attn split-K factor
 
 Usage: python scripts/bench_decode_ops.py [--batch 64] [--len 192]
 """
@@ -70,7 +69,7 @@ def main():
     dim, inter, vocab = 4096, 14336, 128256
     n_q, n_kv, D = 32, 8, 128
     bs = 16                                   # engine KV block size
-    env = {k: os.environ.get(k) for k in ("RLLI_WAVE_NORM", "RLLI_ATTN_SPLIT")}
+    env = {k: os.environ.get(k) for k in ("RLLI_WAVE_NORM",)}
     print(f"# batch={B} len={L} env={env}", flush=True)
 
     results = {}

@@ -1,0 +1,143 @@
+"""Decode attention where its units, parts and pages end: 32 tokens, 256
+tokens, lengths counted 64 sequences at a time, pages of any size; queries
+as rows and as the parts of a product."""
+
+import pytest
+import torch
+
+from resilient_llm_amd import ops
+from resilient_llm_amd.ops import ref
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+LENS = {
+    "whole": [1, 31, 32, 33, 64, 255, 256],
+    "parts": [257, 1, 1000, 33, 4097, 0, 512],
+    "many": [0, 0] + [40] * 66 + [700, 1],
+}
+
+
+def setup(lens, n_q, n_kv, D, bs, fp8, width=None):
+    gen = torch.Generator().manual_seed(D + bs + len(lens))
+    need = [-(-n // bs) for n in lens]
+    pages = sum(need) + 1
+    k, v = (torch.randn(pages, n_kv, bs, D, generator=gen) for _ in "kv")
+    dtype = torch.float8_e4m3fn if fp8 else torch.bfloat16
+    order = torch.randperm(pages, generator=gen).to(torch.int32)
+    tables = torch.zeros(len(lens), width or max(need), dtype=torch.int32)
+    at = 0
+    for i, n in enumerate(need):
+        tables[i, :n] = order[at:at + n]
+        at += n
+    qkv = torch.randn(len(lens), (n_q + 2 * n_kv) * D, generator=gen)
+    return (k.to(dtype), v.to(dtype), tables, torch.tensor(
+        lens, dtype=torch.int32), qkv.to(torch.bfloat16))
+
+
+def exact(q, k, v, tables, lens, scale):
+    """In 64 bits; sequences without tokens give zeros."""
+    out = torch.zeros(q.shape, dtype=torch.float64)
+    for b, n in enumerate(lens.tolist()):
+        if n:
+            keys, values = (
+                t[tables[b].long()].transpose(0, 1)
+                .reshape(t.shape[1], -1, t.shape[3])[:, :n].float().double()
+                .repeat_interleave(q.shape[1] // t.shape[1], 0)
+                for t in (k, v))
+            w = torch.softmax(torch.einsum("hd,hnd->hn", q[b].double(), keys)
+                              * scale, -1)
+            out[b] = torch.einsum("hn,hnd->hd", w, values)
+    return out
+
+
+def close(got, want):
+    # f32 throughout, rounded to bf16 once
+    torch.testing.assert_close(got.cpu().double(), want, rtol=2 ** -8,
+                               atol=2 ** -14)
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("lens", LENS)
+@pytest.mark.parametrize("n_q,n_kv,D,bs", [
+    (8, 2, 128, 16), (8, 1, 64, 16), (2, 2, 128, 16), (2, 1, 64, 8),
+    (4, 1, 128, 32)])
+def test_cached(n_q, n_kv, D, bs, lens, fp8):
+    k, v, tables, n, qkv = setup(LENS[lens], n_q, n_kv, D, bs, fp8)
+    q = qkv[:, :n_q * D].reshape(-1, n_q, D).contiguous()
+    # scores far apart as well
+    for scale in (D ** -0.5, 1.0):
+        got = ops.decode_attn(q.to(DEV), k.to(DEV), v.to(DEV),
+                              tables.to(DEV), n.to(DEV), scale)
+        close(got, exact(q, k, v, tables, n, scale))
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("lens", ["whole", "parts"])
+@pytest.mark.parametrize("n_q,n_kv,D,bs", [
+    (8, 2, 128, 16), (8, 1, 64, 16), (4, 1, 128, 8)])
+def test_fused(n_q, n_kv, D, bs, lens, fp8):
+    """Rotation, append and the new token; its slot held NaN."""
+    lens = [max(1, x) for x in LENS[lens]]
+    k, v, tables, n, qkv = setup(lens, n_q, n_kv, D, bs, fp8)
+    pos = n - 1
+    slots = tables.gather(1, (pos // bs).long()[:, None])[:, 0] * bs + pos % bs
+    cs = ref.build_cos_sin(max(lens), D)
+    args = [x.to(DEV) for x in (pos, cs)]
+    tail = [x.to(DEV) for x in (slots, tables, n)]
+
+    def run(rows):
+        kc, vc = k.clone(), v.clone()
+        for t in (kc, vc):
+            t.float()
+            raw = t.view(torch.uint8 if fp8 else torch.int16)
+            raw[(slots // bs).long(), :, (slots % bs).long()] = \
+                0x7f if fp8 else 0x7fc0
+        kc, vc = kc.to(DEV), vc.to(DEV)
+        out = ops.decode_attn_rope_qkv(rows, *args, kc, vc, *tail,
+                                       D ** -0.5, n_q)
+        return out, kc, vc
+    got, kc, vc = run(qkv.to(DEV))
+    kr, vr = k.clone(), v.clone()
+    q, key, value = (t.reshape(len(lens), -1, D) for t in torch.split(
+        qkv, [n_q * D, n_kv * D, n_kv * D], 1))
+    rot = ref._rotate(torch.cat([q, key], 1).float(), pos, cs)
+    at = (slots // bs).long(), slice(None), (slots % bs).long()
+    kr[at] = rot[:, n_q:].to(k.dtype)
+    vr[at] = value.to(v.dtype)
+    # a rotation's rounding may fall either way
+    torch.testing.assert_close(kc.cpu().float(), kr.float(), rtol=2 ** -3
+                               if fp8 else 2 ** -7, atol=2 ** -9)
+    assert torch.equal(vc.cpu().float(), vr.float())
+    close(got.view(-1, n_q, D), exact(rot[:, :n_q], kc.cpu(), vr, tables, n,
+                                      D ** -0.5))
+    # the same rows as a sum
+    rows = qkv.float().to(DEV)
+    part = torch.randn(rows.shape, device=DEV).to(torch.bfloat16).float() / 8
+    again, k2, v2 = run(torch.stack([rows - part, part]))
+    assert torch.equal(again, got)
+    assert torch.equal(k2.float(), kc.float())
+    assert torch.equal(v2.float(), vc.float())
+
+
+def test_rows_of_one_sequence():
+    """Rows appended first and attended like decoded tokens: the same bits,
+    whichever way they came."""
+    lens = [37, 38, 39, 300, 301]
+    k, v, tables, n, qkv = (t.to(DEV) for t in setup(
+        lens, 8, 2, 128, 16, False))
+    tables[1:3] = tables[0:1].clone()         # three tokens of one sequence
+    tables[4] = tables[3]
+    pos = n - 1
+    slots = tables.gather(1, (pos // 16).long()[:, None])[:, 0] * 16 \
+        + pos % 16
+    cs = ref.build_cos_sin(512, 128, device=DEV)
+    kc, vc = k.clone(), v.clone()
+    got = ops.decode_attn_rows_qkv(qkv.clone(), pos, cs, kc, vc, slots,
+                                   tables, n, 0.1, 8)
+    for order in ([0, 3], [1, 4], [2]):
+        at = torch.tensor(order, device=DEV)
+        want = ops.decode_attn_rope_qkv(
+            qkv[at], pos[at], cs, k, v, slots[at], tables[at], n[at], 0.1, 8)
+        assert torch.equal(got[at], want)
+    assert torch.equal(k, kc) and torch.equal(v, vc)

@@ -8,19 +8,19 @@ from resilient_llm_amd import ops
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
-ROWS = [1, 15, 16, 17, 32, 33, 48, 49, 64]
+ROWS = [1, 15, 16, 17, 32, 33, 48, 49, 64, 65, 96, 97]
 
 
 def operands(N, K, seed=0):
     gen = torch.Generator().manual_seed(seed)
-    x = torch.randn(64, K, generator=gen).to(torch.bfloat16).to(DEV)
+    x = torch.randn(128, K, generator=gen).to(torch.bfloat16).to(DEV)
     w = torch.randn(N, K, generator=gen).to(torch.bfloat16).to(DEV)
     return x, w
 
 
-def close(got, want, size):
+def close(got, want, size, rtol=2 ** -8):
     # half a step of bf16 for the result, K f32 roundings of sums of ``size``
-    torch.testing.assert_close(got.double(), want, rtol=2 ** -8,
+    torch.testing.assert_close(got.double(), want, rtol=rtol,
                                atol=float(size) * 2 ** -20)
 
 
@@ -41,24 +41,43 @@ def test_rows_linear(N, K):
         assert torch.equal(s.to(torch.bfloat16), whole)
 
 
-@pytest.mark.parametrize("inter,K", [(4, 64), (68, 128), (5152, 64),
-                                     (12740, 192), (12800, 448)])
+@pytest.mark.parametrize("inter,K", [(8, 64), (72, 128), (5152, 64),
+                                     (12744, 192), (12800, 448)])
 def test_rows_linear_silu(inter, K):
     x, w = operands(2 * inter, K, 1)
     w *= K ** -0.5
     whole = torch.ops.rlli.rows_linear_silu(x, w)
     g, u = (x.double() @ w.double().T).chunk(2, 1)
-    # a sum's f32 error times the other factor, both of size one
-    close(whole, torch.nn.functional.silu(g) * u, 8.0)
+    # a sum's f32 error times the other factor, both of size one; few pairs
+    # take the product in 16 bits, whose half steps grow with 1 + |gate|
+    close(whole, torch.nn.functional.silu(g) * u, 8.0,
+          2 ** -8 if inter > 5000 else 8 * 2 ** -8)
     for m in ROWS:
         assert torch.equal(
             torch.ops.rlli.rows_linear_silu(x[:m].contiguous(), w), whole[:m])
 
 
-@pytest.mark.parametrize("M,N,K", [(65, 64, 64), (1, 64, 96), (1, 6, 64)])
+@pytest.mark.parametrize("M,N,K", [(129, 64, 64), (1, 64, 96), (1, 6, 64)])
 def test_what_does_not_fit(M, N, K):
     x = torch.zeros(M, K, dtype=torch.bfloat16, device=DEV)
     w = torch.zeros(N, K, dtype=torch.bfloat16, device=DEV)
     assert not ops.rows_fit(x, w)
     with pytest.raises(RuntimeError):
         ops.rows_linear(x, w)
+
+
+@pytest.mark.parametrize("n,rows,dim", [(1, 1, 8), (2, 3, 520), (5, 64, 4096),
+                                        (8, 2, 8192)])
+def test_norm_of_parts(n, rows, dim):
+    gen = torch.Generator().manual_seed(dim)
+    parts = torch.randn(n, rows, dim, generator=gen).to(DEV)
+    res = torch.randn(rows, dim, generator=gen).to(torch.bfloat16).to(DEV)
+    w = torch.randn(dim, generator=gen).to(torch.bfloat16).to(DEV)
+    want = (parts.double().sum(0) + res.double())
+    got = ops.rmsnorm_residual_(parts, res, w, 1e-5)
+    # the f32 sum's rounding may move a result to the next bf16 number
+    torch.testing.assert_close(res.double(), want, rtol=2 ** -8,
+                               atol=n * 2 ** -20)
+    r = res.double()
+    y = r * torch.rsqrt(r.pow(2).mean(-1, keepdim=True) + 1e-5) * w.double()
+    torch.testing.assert_close(got.double(), y, rtol=2 ** -8, atol=2 ** -16)

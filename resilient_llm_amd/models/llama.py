@@ -51,6 +51,21 @@ def _linear(x, w):
     return F.linear(x, w)
 
 
+def _linear_silu(x, w):
+    """silu_mul of _linear."""
+    if (not _USE_SKINNY and not lt_autotune.enabled() and ops.rows_fit(x, w)
+            and w.shape[0] % 16 == 0):
+        return ops.rows_linear_silu(x, w)
+    return ops.silu_mul(_linear(x, w))
+
+
+def _linear_parts(x, w):
+    """_linear for a reader that sums parts (ops.rows_linear_parts)."""
+    if (not _USE_SKINNY and not lt_autotune.enabled() and ops.rows_fit(x, w)):
+        return ops.rows_linear_parts(x, w)
+    return _linear(x, w)
+
+
 @dataclasses.dataclass
 class LlamaConfig:
     name: str
@@ -345,20 +360,24 @@ class LlamaForCausalLM:
 
     def _layer(self, i: int, x: torch.Tensor, residual: Optional[torch.Tensor],
                positions: torch.Tensor, kv_cache, slot_mapping: torch.Tensor,
-               attn_fn) -> tuple[torch.Tensor, torch.Tensor]:
+               attn_fn, qkv_parts: bool) -> tuple[torch.Tensor, torch.Tensor]:
         p = self.params
         c = self.config
+        # what the next norm adds to the residual may come in parts, if
+        # nothing has to be done with their sum before
+        out = (_linear_parts if self.tp_world == 1 and self.quant is None
+               and c.hidden_size <= 8192 else _linear)
         if residual is None:
             residual = x.clone()
             h = ops.rmsnorm(x, p[f"l{i}.ln1"], c.rms_eps)
         else:
             h = ops.rmsnorm_residual_(x, residual, p[f"l{i}.ln1"], c.rms_eps)
-        qkv = _linear(h, p[f"l{i}.qkv"])
+        qkv = (_linear_parts if qkv_parts else _linear)(h, p[f"l{i}.qkv"])
         k_cache, v_cache = kv_cache.layer(i)
         # rope + cache append happen inside attn_fn (the decode path fuses
         # them into the attention kernel itself)
         attn_out = attn_fn(i, qkv, k_cache, v_cache)   # [T, q_size]
-        h = self._all_reduce(_linear(attn_out, p[f"l{i}.o"]))
+        h = self._all_reduce(out(attn_out, p[f"l{i}.o"]))
         if self.quant == "fp8":
             h2q, h2s = ops.rmsnorm_residual_fp8(h, residual, p[f"l{i}.ln2"],
                                                 c.rms_eps)
@@ -367,8 +386,8 @@ class LlamaForCausalLM:
             mlp = self._all_reduce(self._linear_fp8(dq, ds, f"l{i}.down"))
             return mlp, residual
         h2 = ops.rmsnorm_residual_(h, residual, p[f"l{i}.ln2"], c.rms_eps)
-        gu = _linear(h2, p[f"l{i}.gate_up"])
-        mlp = self._all_reduce(_linear(ops.silu_mul(gu), p[f"l{i}.down"]))
+        act = _linear_silu(h2, p[f"l{i}.gate_up"])
+        mlp = self._all_reduce(out(act, p[f"l{i}.down"]))
         return mlp, residual
 
     def forward_prefill(self, input_ids: torch.Tensor, positions: torch.Tensor,
@@ -393,6 +412,21 @@ class LlamaForCausalLM:
         """Mixed batch: rows [0, n_decode) are decode tokens, the rest
         are prefill-chunk tokens attending over the paged cache
         (chunked prefill).  Returns logits for ``sample_idx`` rows."""
+        if self._few_rows(input_ids.shape[0] - n_decode,
+                          chunk_row0.shape[0]):
+            tables = self._row_tables(
+                input_ids.shape[0], n_decode, block_tables_dec, chunk_row0,
+                chunk_nrows, chunk_btrow, block_tables_pre)
+            seq_lens = positions + 1
+
+            def attn_rows(i, qkv, k_cache, v_cache):
+                return ops.decode_attn_rows_qkv(
+                    qkv, positions, self.cos_sin, k_cache, v_cache,
+                    slot_mapping, tables, seq_lens, self.scale, self.n_heads)
+            return self._forward(input_ids, positions, kv_cache,
+                                 slot_mapping, attn_rows,
+                                 last_idx=sample_idx)
+
         def attn(i, qkv, k_cache, v_cache):
             ops.rope_kv_append_qkv_(qkv, positions, self.cos_sin, k_cache,
                                     v_cache, slot_mapping, self.n_heads)
@@ -408,6 +442,35 @@ class LlamaForCausalLM:
         return self._forward(input_ids, positions, kv_cache, slot_mapping,
                              attn, last_idx=sample_idx)
 
+    def _few_rows(self, rows: int, tiles: int) -> bool:
+        """Whether a step's prompt rows (speculated tokens, what a cached
+        prefix left) are so few that the decode kernel, which reads a
+        sequence once per row but over many workgroups, beats tiles of 32
+        rows that walk it one after another (8 key/value heads, us: 5 rows
+        behind 200 tokens 12.5 and 8.9, behind 4000 94 and 21; 3 x 8 rows
+        behind 1000 30 and 22, 16 behind 4000 97 and 31)."""
+        return (self.device.type == "cuda" and 0 < rows <= 16 * tiles
+                and rows * self.n_kv_heads <= 256)
+
+    @staticmethod
+    def _row_tables(rows, n_decode, tables_dec, row0, nrows, btrow,
+                    tables_pre) -> torch.Tensor:
+        """The block table of every row of a mixed step."""
+        n = rows - n_decode
+        n64 = nrows.long()
+        first = row0.long() - (n64.cumsum(0) - n64)
+        at = torch.repeat_interleave(first, n64, output_size=n) \
+            + torch.arange(n, device=row0.device)
+        wide = max([tables_pre.shape[1]] + ([tables_dec.shape[1]]
+                                            if n_decode else []))
+        out = torch.zeros((rows, wide), dtype=torch.int32,
+                          device=row0.device)
+        out[at, :tables_pre.shape[1]] = tables_pre[torch.repeat_interleave(
+            btrow.long(), n64, output_size=n)]
+        if n_decode:
+            out[:n_decode, :tables_dec.shape[1]] = tables_dec
+        return out
+
     def forward_decode(self, input_ids: torch.Tensor, positions: torch.Tensor,
                        kv_cache, slot_mapping: torch.Tensor,
                        block_tables: torch.Tensor,
@@ -418,16 +481,17 @@ class LlamaForCausalLM:
                 qkv, positions, self.cos_sin, k_cache, v_cache, slot_mapping,
                 block_tables, seq_lens, self.scale, self.n_heads)
         return self._forward(input_ids, positions, kv_cache, slot_mapping,
-                             attn, last_idx=None)
+                             attn, last_idx=None, qkv_parts=True)
 
     def _forward(self, input_ids, positions, kv_cache, slot_mapping, attn_fn,
-                 last_idx) -> torch.Tensor:
+                 last_idx, qkv_parts: bool = False) -> torch.Tensor:
+        """``qkv_parts``: attn_fn takes the product in parts."""
         p = self.params
         x = F.embedding(input_ids.long(), p["embed"])
         residual = None
         for i in range(self.config.n_layers):
             x, residual = self._layer(i, x, residual, positions, kv_cache,
-                                      slot_mapping, attn_fn)
+                                      slot_mapping, attn_fn, qkv_parts)
         if self.quant == "fp8":
             h8, hs = ops.rmsnorm_residual_fp8(x, residual, p["final_ln"],
                                               self.config.rms_eps)

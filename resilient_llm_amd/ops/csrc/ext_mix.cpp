@@ -173,7 +173,8 @@ Tensor moe_run(rlli::MoeArgs& a, const Tensor& h, Tensor& ids, Tensor& w) {
   auto io = h.options().dtype(at::kInt);
   ids = at::empty({a.rows, a.top}, io);
   w = at::empty({a.rows, a.top}, h.options().dtype(at::kFloat));
-  Tensor plan = at::empty({P + 3 * int64_t(a.max_tiles) + 2 * a.experts}, io);
+  Tensor plan =
+      at::empty({P + 3 * int64_t(a.max_tiles) + 2 * a.experts + 2}, io);
   Tensor act = at::empty({P, a.ffp}, h.options());
   Tensor y = at::empty({a.rows, a.top, a.width}, h.options());
   a.ids = ids.data_ptr<int32_t>();

@@ -44,7 +44,8 @@ struct MoeArgs {
   int32_t* tile_expert;    // [max_tiles]
   int32_t* tile_row0;      // [max_tiles]
   int32_t* tile_rows;      // [max_tiles]
-  int32_t* counters;       // [2 * experts + 1]
+  int32_t* counters;       // [2 * experts + 2]; the last two: tiles more than
+                           // half full, others
   void* act;               // [rows * top, ffp]
   void* y;                 // [rows, top, width]
   int rows, width, experts, top, ffp, tile_m, max_tiles;

@@ -67,6 +67,9 @@ void moe_route_kernel(MoeArgs a) {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int lr = lane & 15, g = lane >> 4;
   const int row0 = blockIdx.x * 16;
+  // the plan's counters, for the kernels after this one
+  if (blockIdx.x == 0 && a.counters)
+    for (int e = threadIdx.x; e < 2 * a.experts; e += 512) a.counters[e] = 0;
   const T* h = reinterpret_cast<const T*>(a.h) +
                int64_t(min(row0 + lr, a.rows - 1)) * a.width;
   const T* wr = reinterpret_cast<const T*>(a.router);
@@ -229,28 +232,42 @@ void moe_route_kernel(MoeArgs a) {
 // --------------------------------------------------------------- plan
 constexpr int MAXE = 256;
 
-// start of each expert's rows, and (thread 0 of the writer) the tile list
+// The tile list: tiles more than half full in expert order, then the other
+// ones, so that the cheap tiles run where the last full ones leave compute
+// units idle.  The counts of both follow the counters of the plan.
 DEV_INLINE void write_tiles(const MoeArgs& a, const int* count,
                             const int* start, int tid, int nthr) {
-  // tile index of expert e's first tile
-  __shared__ int tfirst[MAXE + 1];
+  // index of expert e's first full tile, of its last one if that is not
+  __shared__ int tfull[MAXE + 1], tpart[MAXE + 1];
+  const int half = a.tile_m > 16 ? a.tile_m / 2 : 0;
+  auto full = [&](int n) {
+    return n / a.tile_m + (n % a.tile_m > half ? 1 : 0);
+  };
+  auto all = [&](int n) { return (n + a.tile_m - 1) / a.tile_m; };
   if (tid == 0) {
-    int t = 0;
+    int f = 0, p = 0;
     for (int e = 0; e < a.experts; ++e) {
-      tfirst[e] = t;
-      t += (count[e] + a.tile_m - 1) / a.tile_m;
+      tfull[e] = f;
+      tpart[e] = p;
+      f += full(count[e]);
+      p += all(count[e]) - full(count[e]);
     }
-    tfirst[a.experts] = t;
+    tfull[a.experts] = f;
+    tpart[a.experts] = p;
+    a.counters[2 * a.experts] = f;
+    a.counters[2 * a.experts + 1] = p;
   }
   __syncthreads();
+  const int nfull = tfull[a.experts];
   for (int e = tid; e < a.experts; e += nthr)
-    for (int t = tfirst[e]; t < tfirst[e + 1]; ++t) {
-      const int r = (t - tfirst[e]) * a.tile_m;
+    for (int i = 0; i < all(count[e]); ++i) {
+      const int r = i * a.tile_m;
+      const int t = i < full(count[e]) ? tfull[e] + i : nfull + tpart[e];
       a.tile_expert[t] = e;
       a.tile_row0[t] = start[e] + r;
       a.tile_rows[t] = min(a.tile_m, count[e] - r);
     }
-  for (int t = tfirst[a.experts] + tid; t < a.max_tiles; t += nthr)
+  for (int t = nfull + tpart[a.experts] + tid; t < a.max_tiles; t += nthr)
     a.tile_rows[t] = 0;
 }
 
@@ -276,11 +293,6 @@ void moe_plan_one_kernel(MoeArgs a) {
   for (int p = tid; p < P; p += 256)
     if (a.ids[p] < a.experts) a.perm[atomicAdd(&cursor[a.ids[p]], 1)] = p;
   write_tiles(a, count, start, tid, 256);
-}
-
-__global__ void moe_zero_kernel(MoeArgs a) {
-  for (int e = threadIdx.x; e < 2 * a.experts; e += blockDim.x)
-    a.counters[e] = 0;
 }
 
 constexpr int PLAN_PAIRS = 2048;          // pairs per workgroup
@@ -445,13 +457,48 @@ void moe_small_kernel(MoeArgs a) {
 // the global address), which spreads the fragment reads of 16 rows over
 // all banks.  Two heights: 256 x 256 with eight waves of 128 x 64 each
 // (fewest LDS bytes per MFMA), and 128 x 128 with four of 64 x 64 for
-// experts with fewer rows.
+// experts with fewer rows.  What bounds the tall ones (6001 rows of 2048 in
+// 32 experts): with the products taken out 220 of 265 us remain, with the
+// loads taken out 190, so a step of 64 KB into LDS costs as much as its
+// products and they overlap in part only; a block's start and end are 10 of
+// its 68 us.  Four waves of 128 x 128 (a third less LDS traffic), other K
+// starts per XCD and lines asked for three or four steps ahead gave nothing.
 constexpr int BK = 64;
 
 DEV_INLINE void lds_load16(const void* g, void* l) {
   __builtin_amdgcn_global_load_lds(
       (const __attribute__((address_space(1))) void*)g,
       (__attribute__((address_space(3))) void*)l, 16, 0, 0);
+}
+
+// Consecutive workgroups go to different XCDs.  Each XCD gets an equal run of
+// the full tiles' blocks, then an equal run of the others', counted on the
+// device: the tiles there could be are up to one per expert more, and runs of
+// those left whole XCDs idle.  A run goes over four tiles' column blocks at a
+// time, so that what an XCD works on at once, about 32 blocks, shares eight
+// column blocks' weights and four tiles' rows in its L2 (hits 49 -> 78 % at
+// width 4096).  Whole calls, before -> now: 8192 rows of 4096, 16 experts of
+// 3584, two each: 1704 -> 1409 us; 2048 rows of them 788 -> 622; 6001 rows of
+// 2048, 32 experts of 1024, four each: 397 -> 385.
+DEV_INLINE bool tile_of(const MoeArgs& a, int block, int n_blocks, int& tile,
+                        int& nb) {
+  const int x = block & 7;
+  int s = block >> 3, n = a.counters[2 * a.experts], first = 0;
+  int per = (n * n_blocks + 7) / 8;
+  if (s >= per) {
+    s -= per;
+    first = n;
+    n = a.counters[2 * a.experts + 1];
+    per = (n * n_blocks + 7) / 8;
+    if (s >= per) return false;
+  }
+  const int i = x * per + s;
+  if (i >= n * n_blocks) return false;
+  const int group = i / (4 * n_blocks), j = i - group * 4 * n_blocks;
+  const int high = min(4, n - group * 4);
+  nb = j / high;
+  tile = first + group * 4 + j % high;
+  return true;
 }
 
 template <bool UP, int TT, bool GATED>
@@ -462,15 +509,9 @@ void moe_tile_kernel(MoeArgs a, int n_blocks) {
   constexpr int MI = TT == 256 ? 8 : 4;           // 16-row blocks per wave
   constexpr int PIECES = TT * 8 / NT;
   extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
-  // consecutive workgroups go to different XCDs; give each XCD whole
-  // runs of one tile's column blocks so its L2 holds the rows once
-  const int total = gridDim.x;
-  const int per = (total + 7) / 8;
-  const int wid = (blockIdx.x % 8) * per + blockIdx.x / 8;
-  if (wid >= n_blocks * a.max_tiles) return;
-  const int tile = wid / n_blocks, nb = wid % n_blocks;
+  int tile, nb;
+  if (!tile_of(a, blockIdx.x, n_blocks, tile, nb)) return;
   const int rows = a.tile_rows[tile];
-  if (rows == 0) return;
   const int e = a.tile_expert[tile];
   const int p0 = a.tile_row0[tile];
   const int K = UP ? a.width : a.ffp;
@@ -491,21 +532,20 @@ void moe_tile_kernel(MoeArgs a, int n_blocks) {
 
   // piece i of this thread: tile row i * NT/8 + tid / 8, 16-byte column
   // tid % 8, holding global column (tid % 8) ^ (row & 7)
-  const uint16_t* abase =
-      reinterpret_cast<const uint16_t*>(UP ? a.h : a.act);
-  const uint16_t* bbase =
-      reinterpret_cast<const uint16_t*>(UP ? a.w_up : a.w_down) +
-      int64_t(e) * N * K;
-  uint32_t ap[PIECES], bp[PIECES];        // element offsets
+  const char* abase = reinterpret_cast<const char*>(UP ? a.h : a.act);
+  const char* bbase =
+      reinterpret_cast<const char*>(UP ? a.w_up : a.w_down) +
+      int64_t(e) * N * K * 2;
+  uint32_t ap[PIECES], bp[PIECES];        // bytes, below 2^32
 #pragma unroll
   for (int i = 0; i < PIECES; ++i) {
     const int r = i * (NT / 8) + (tid >> 3);
     const int c = ((tid & 7) ^ (r & 7)) * 8;
     if constexpr (UP)
-      ap[i] = uint32_t(s_pair[r] / a.top) * K + c;
+      ap[i] = (uint32_t(s_pair[r] / a.top) * K + c) * 2;
     else
-      ap[i] = uint32_t(p0 + min(r, rows - 1)) * K + c;
-    bp[i] = uint32_t(min(n0 + r, N - 1)) * K + c;
+      ap[i] = (uint32_t(p0 + min(r, rows - 1)) * K + c) * 2;
+    bp[i] = (uint32_t(min(n0 + r, N - 1)) * K + c) * 2;
   }
   auto stage = [&](int buf, int k0) {
     uint16_t* la = lds + buf * 2 * TT * BK;
@@ -513,8 +553,9 @@ void moe_tile_kernel(MoeArgs a, int n_blocks) {
 #pragma unroll
     for (int i = 0; i < PIECES; ++i) {
       // wave-uniform LDS base; lane l lands at base + 16 l
-      lds_load16(abase + k0 + ap[i], la + (i * (NT / 8) + w * 8) * BK);
-      lds_load16(bbase + k0 + bp[i], lb + (i * (NT / 8) + w * 8) * BK);
+      if (i * (NT / 8) < rows)
+        lds_load16(abase + k0 * 2 + ap[i], la + (i * (NT / 8) + w * 8) * BK);
+      lds_load16(bbase + k0 * 2 + bp[i], lb + (i * (NT / 8) + w * 8) * BK);
     }
   };
 
@@ -525,6 +566,8 @@ void moe_tile_kernel(MoeArgs a, int n_blocks) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
+  // none of this wave's rows is one of the tile's: it only loads
+  const bool idle = wm >= rows;
   const int nk = K / BK;
   stage(0, 0);
   for (int kt = 0; kt < nk; ++kt) {
@@ -532,6 +575,7 @@ void moe_tile_kernel(MoeArgs a, int n_blocks) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     if (kt + 1 < nk) stage((kt + 1) & 1, (kt + 1) * BK);
+    if (idle) continue;
     const uint16_t* la = lds + (kt & 1) * 2 * TT * BK;
     const uint16_t* lb = la + TT * BK;
     auto frag = [&](const uint16_t* base, int row, int kk) {
@@ -645,12 +689,14 @@ template <bool UP, int TT, bool GATED>
 void tiled_one(const MoeArgs& a, hipStream_t st) {
   const size_t smem = size_t(4) * TT * BK * 2;
   const int nb = ((UP ? (GATED ? 2 : 1) * a.ffp : a.width) + TT - 1) / TT;
+  // two runs per XCD, each up to one block longer than its part
+  const int blocks = (nb * a.max_tiles + 7) / 8 * 8 + 8;
   auto* k = moe_tile_kernel<UP, TT, GATED>;
   if (smem > 65536)
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(k),
                               hipFuncAttributeMaxDynamicSharedMemorySize,
                               int(smem));
-  hipLaunchKernelGGL(k, dim3((nb * a.max_tiles + 7) / 8 * 8),
+  hipLaunchKernelGGL(k, dim3(blocks),
                      dim3(TT == 256 ? 512 : 256), smem, st, a, nb);
 }
 
@@ -677,7 +723,6 @@ void launch_moe_plan(const MoeArgs& a, hipStream_t st) {
     return;
   }
   const dim3 grid((P + PLAN_PAIRS - 1) / PLAN_PAIRS);
-  hipLaunchKernelGGL(moe_zero_kernel, dim3(1), dim3(256), 0, st, a);
   hipLaunchKernelGGL(moe_count_kernel, grid, dim3(256), 0, st, a);
   hipLaunchKernelGGL(moe_scatter_kernel, grid, dim3(256), 0, st, a);
 }

@@ -361,7 +361,8 @@ class NesizenForCausalLM(MixedModel):
     def _feed_forward(self, i: int, h: torch.Tensor) -> torch.Tensor:
         P, f, p = self.params, self.config.layers[i].mlp, f"l{i}."
         if isinstance(f, DenseSpec):
-            return _linear(ops.relu2(_linear(h, P[p + "up"])), P[p + "down"])
+            return _linear(ops.linear_relu2(h, P[p + "up"], _linear),
+                           P[p + "down"])
         return ops.moe_experts(h, P[p + "router"], P[p + "w_up"],
                                P[p + "w_down"], f.top, f.limit)
 

@@ -298,6 +298,16 @@ def rows_linear_silu(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     return silu_mul(torch.nn.functional.linear(x, w))
 
 
+def linear_relu2(x: torch.Tensor, w: torch.Tensor, linear) -> torch.Tensor:
+    """relu2 of ``linear(x, w)``; for few rows and a w that is not large in
+    one kernel, which squares the f32 sums."""
+    if rows_fit(x, w):
+        _gpu()
+        if torch.ops.rlli.rows_relu2_ok(x.shape[0], *w.shape):
+            return torch.ops.rlli.rows_linear_relu2(x, w)
+    return relu2(linear(x, w))
+
+
 def skinny_linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """rows_linear for K % 256 == 0 and N % 64 == 0."""
     if x.is_cuda:

@@ -531,7 +531,24 @@ Tensor rows_linear_parts(const Tensor& x, const Tensor& w) {
   return out;
 }
 
+// whole products of at most 64 rows by workgroups that divide K themselves,
+// with or without the squared positive part; undefined where those are not
+// the faster ones
+Tensor rows_short(const Tensor& x, const Tensor& w, bool relu2) {
+  check_rows(x, w);
+  const int M = int(x.size(0)), N = int(w.size(0)), K = int(x.size(1));
+  if (M > 64 || rlli::rows_short_tiles(N, K) == 0) return Tensor();
+  c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
+  Tensor out = at::empty({M, N}, x.options());
+  rlli::launch_rows_short(bf16_ptr(x), bf16_ptr(w), bf16_ptr(out), M, N, K,
+                          relu2, current_stream(x));
+  check_launch("rows_short");
+  return out;
+}
+
 Tensor rows_linear(const Tensor& x, const Tensor& w) {
+  Tensor whole = rows_short(x, w, false);
+  if (whole.defined()) return whole;
   Tensor parts = rows_linear_parts(x, w);
   if (parts.dim() == 2) return parts;
   c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
@@ -540,6 +557,18 @@ Tensor rows_linear(const Tensor& x, const Tensor& w) {
                          int(parts.size(0)), out.numel(), current_stream(x));
   check_launch("sum_parts");
   return out;
+}
+
+// the squared positive part of x w^T, of the f32 sums
+Tensor rows_linear_relu2(const Tensor& x, const Tensor& w) {
+  Tensor whole = rows_short(x, w, true);
+  TORCH_CHECK(whole.defined(), "rows_relu2_ok says which products these are");
+  return whole;
+}
+
+bool rows_relu2_ok(int64_t M, int64_t N, int64_t K) {
+  return M <= 64 && N <= 8192 && K <= 8192 &&
+         rlli::rows_short_tiles(int(N), int(K)) > 0;
 }
 
 Tensor rows_linear_silu(const Tensor& x, const Tensor& w) {
@@ -669,6 +698,8 @@ TORCH_LIBRARY(rlli, m) {
   m.def("rows_linear_parts(Tensor x, Tensor w) -> Tensor");
   m.def("rows_linear(Tensor x, Tensor w) -> Tensor");
   m.def("rows_linear_silu(Tensor x, Tensor w) -> Tensor");
+  m.def("rows_linear_relu2(Tensor x, Tensor w) -> Tensor");
+  m.def("rows_relu2_ok(int m, int n, int k) -> bool", &rows_relu2_ok);
   m.def("skinny_linear(Tensor x, Tensor w) -> Tensor");
   m.def("skinny2_linear(Tensor x, Tensor w, int splitk) -> Tensor");
   m.def("skinny2_silu_linear(Tensor gu, Tensor w, int splitk) -> Tensor");
@@ -700,6 +731,7 @@ TORCH_LIBRARY_IMPL(rlli, CUDA, m) {
   m.impl("rows_linear_parts", &rows_linear_parts);
   m.impl("rows_linear", &rows_linear);
   m.impl("rows_linear_silu", &rows_linear_silu);
+  m.impl("rows_linear_relu2", &rows_linear_relu2);
   m.impl("skinny_linear", &skinny_linear);
   m.impl("skinny2_linear", &skinny2_linear);
   m.impl("skinny2_silu_linear", &skinny2_silu_linear);

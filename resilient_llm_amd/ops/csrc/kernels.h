@@ -110,6 +110,10 @@ bool rows_gemm_silu_ok(int inter);
 void launch_rows_gemm_silu(const uint16_t* x, const uint16_t* w,
                            uint16_t* out, int M, int inter, int K,
                            hipStream_t stream);
+// M <= 64 where rows_short_tiles is not 0; ``relu2``: squared positive part
+int rows_short_tiles(int N, int K);
+void launch_rows_short(const uint16_t* x, const uint16_t* w, uint16_t* out,
+                       int M, int N, int K, bool relu2, hipStream_t stream);
 void launch_sum_parts(const float* parts, uint16_t* out, int splits,
                       int64_t n, hipStream_t stream);
 

@@ -18,7 +18,8 @@
 // Where 64-row panels are fewer than the CUs, K is divided as well, and the
 // parts are written in f32, [splits, M, N], for whoever reads the product to
 // sum; in order, so a result does not depend on when workgroups run.  Nor
-// does it depend on M: the order of sums follows from N and K alone.
+// does it depend on M, up to 64 rows and from there on: the order of sums
+// follows from N and K alone.
 
 #include "common.h"
 
@@ -227,6 +228,129 @@ void rows_gemm_kernel(const uint16_t* __restrict__ x,
   }
 }
 
+// The same product by workgroups that divide K among their four waves, for
+// shapes whose 64-row panels leave CUs idle: 16 PT rows of w per workgroup, no
+// parts in memory and no launch to sum them.  A wave has a ring of its own for
+// the steps it takes (every fourth, so that the four together read 512 bytes of
+// a row at a time): its loads, waits and reads concern nobody else, and there
+// is no barrier before the sums meet at the end.  What bounds it is the time
+// from the launch to the first data and, past 4096 in K, that it reads x once
+// per 16 or 32 rows of w.
+template <int PT, int XR, int MT, int R, bool RELU2>
+__global__ __launch_bounds__(256)
+void rows_short_kernel(const uint16_t* __restrict__ x,
+                       const uint16_t* __restrict__ w,
+                       uint16_t* __restrict__ out, int M, int N, int K) {
+  constexpr int WPART = PT * 16 * LINE;              // elements of a step
+  constexpr int STEP = WPART + XR * LINE;
+  constexpr int LX = XR / 8, L = PT * 2 + LX;        // loads of a wave
+  extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
+  const int lane = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int n0 = blockIdx.x * PT * 16;
+  // this wave's steps: wv, wv + 4, ...
+  const int n = (K / KS - wv + 3) / 4;
+  const int rot = n > 0 ? int(blockIdx.x / 8 % unsigned(n)) : 0;
+  uint16_t* ring = lds + wv * R * STEP;
+
+  const int lr = lane >> 3;
+  const uint16_t *wp[PT * 2], *xp[LX];
+#pragma unroll
+  for (int j = 0; j < PT * 2; ++j) {
+    const int r = (j & 1) * 8 + lr;
+    // rows past the end repeat the last one; nobody stores them
+    const int row = min(n0 + (j >> 1) * 16 + r, N - 1);
+    wp[j] = w + int64_t(row) * K + wv * KS + ((lane & 7) ^ ((r >> 1) & 7)) * 8;
+  }
+#pragma unroll
+  for (int j = 0; j < LX; ++j) {
+    const int r = j * 8 + lr;
+    xp[j] = x + int64_t(min(r, M - 1)) * K + wv * KS +
+            ((lane & 7) ^ ((r >> 1) & 7)) * 8;
+  }
+  auto issue = [&](int s, int slot) {
+    uint16_t* at = ring + slot * STEP;
+    s += rot;
+    if (s >= n) s -= n;
+#pragma unroll
+    for (int j = 0; j < PT * 2; ++j)
+      lds_load16<2>(wp[j] + s * 4 * KS, at + j * 8 * LINE);
+#pragma unroll
+    for (int j = 0; j < LX; ++j)
+      lds_load16<0>(xp[j] + s * 4 * KS, at + WPART + j * 8 * LINE);
+  };
+
+  f32x4 acc[PT][MT];
+#pragma unroll
+  for (int t = 0; t < PT; ++t)
+#pragma unroll
+    for (int m = 0; m < MT; ++m) acc[t][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int tr = lane & 15, oct = lane >> 4;
+  const int sw = tr >> 1;
+#pragma unroll
+  for (int s = 0; s < R - 1; ++s)
+    if (s < n) issue(s, s);
+  int slot = 0;
+  for (int s = 0; s < n; ++s) {
+    wait_steps<L, R - 2>(n - 1 - s);
+    const uint16_t* at = ring + slot * STEP;
+    const uint16_t* wt = at + tr * LINE;
+    const uint16_t* xt = at + WPART + tr * LINE;
+    s16x8 a[2][PT], b[2][MT];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      const int piece = ((k * 4 + oct) ^ sw) * 8;
+#pragma unroll
+      for (int t = 0; t < PT; ++t)
+        a[k][t] = *reinterpret_cast<const s16x8*>(wt + t * 16 * LINE + piece);
+#pragma unroll
+      for (int m = 0; m < MT; ++m)
+        b[k][m] = *reinterpret_cast<const s16x8*>(xt + m * 16 * LINE + piece);
+    }
+    // the slot before this one was read a step ago
+    if (s + R - 1 < n) issue(s + R - 1, slot == 0 ? R - 1 : slot - 1);
+    slot = slot == R - 1 ? 0 : slot + 1;
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+#pragma unroll
+      for (int t = 0; t < PT; ++t)
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+          acc[t][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              a[k][t], b[k][m], acc[t][m], 0, 0, 0);
+  }
+
+  // the waves' sums meet, in order
+  __syncthreads();
+  f32x4* side = reinterpret_cast<f32x4*>(lds);
+#pragma unroll
+  for (int t = 0; t < PT; ++t)
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+      side[(wv * PT * MT + t * MT + m) * 64 + lane] = acc[t][m];
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < (PT * MT + 3) / 4; ++i) {
+    const int e = i * 4 + wv;
+    if (e >= PT * MT) break;
+    f32x4 v = side[e * 64 + lane];
+#pragma unroll
+    for (int o = 1; o < 4; ++o) v += side[(o * PT * MT + e) * 64 + lane];
+    if constexpr (RELU2) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        v[r] = fmaxf(v[r], 0.f);
+        v[r] *= v[r];
+      }
+    }
+    const int row = e % MT * 16 + tr;
+    const int c = n0 + e / MT * 16 + oct * 4;
+    if (row < M && c < N)
+      *reinterpret_cast<uint2*>(out + int64_t(row) * N + c) =
+          uint2{pack2(v[0], v[1]), pack2(v[2], v[3])};
+  }
+}
+
 __global__ __launch_bounds__(256)
 void sum_parts_kernel(const float* __restrict__ parts,
                       uint16_t* __restrict__ out, int splits, int64_t n) {
@@ -272,6 +396,26 @@ void go(const uint16_t* x, const uint16_t* w, void* out, int M, int N, int K,
   else run(X128{}, I8{});
 }
 
+template <int PT, int R16, int R32, int R64, bool RELU2>
+void go_short(const uint16_t* x, const uint16_t* w, uint16_t* out, int M,
+              int N, int K, hipStream_t st) {
+  auto run = [&](auto xr) {
+    constexpr int XR = decltype(xr)::value, MT = XR / 16;
+    constexpr int R = XR == 16 ? R16 : XR == 32 ? R32 : R64;
+    constexpr size_t smem = size_t(4) * R * (PT * 16 + XR) * LINE * 2;
+    auto* k = rows_short_kernel<PT, XR, MT, R, RELU2>;
+    if (smem > 65536)
+      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(k),
+                                hipFuncAttributeMaxDynamicSharedMemorySize,
+                                int(smem));
+    hipLaunchKernelGGL(k, dim3((N + PT * 16 - 1) / (PT * 16)), dim3(256), smem,
+                       st, x, w, out, M, N, K);
+  };
+  if (M <= 16) run(std::integral_constant<int, 16>{});
+  else if (M <= 32) run(std::integral_constant<int, 32>{});
+  else run(std::integral_constant<int, 64>{});
+}
+
 }  // namespace
 
 // As many parts as 64-row panels leave CUs for: with more workgroups than
@@ -314,6 +458,32 @@ void launch_rows_gemm_silu(const uint16_t* x, const uint16_t* w,
   else
     go<1, 6, 5, 3, OUT_SILU>(x, w, out, M, 2 * inter, K, (inter + 31) / 32, 1,
                           st);
+}
+
+// Tiles of 16 rows per workgroup of the products that rows_short_kernel takes,
+// 0 for others; by N and K alone, like all orders of sums here.  With 32 rows
+// per workgroup where 16 make more workgroups than CUs.  (1, 16, 64 rows of x,
+// us, parts and their sum first: 2048 x 2048 6.5 and 4.2, 7.7 and 5.0, 9.3 and
+// 7.1; 8192 x 2048 10.7 and 7.6, 11.5 and 7.8, 13.7 and 11.2; 6144 x 4096 13.6
+// and 10.3, 14.5 and 11.1, 18.3 and 17.0; 256 x 8192 18.7 and 7.8, 22.3 and
+// 10.1, 20.7 and 19.6; but 4096 x 4096 9.7 and 7.8, 10.3 and 8.9, 13.1 and
+// 13.4; 2048 x 8192 10.5 and 9.8, 11.6 and 12.4, 13.7 and 20.4; 5120 x 5120
+// 12.5 and 11.8, 13.4 and 15.9, 18.3 and 21.9.)
+int rows_short_tiles(int N, int K) {
+  if (N > 8192 || K > (N > 4096 ? 4096 : N > 512 ? 3072 : 8192)) return 0;
+  return N > 4096 ? 2 : 1;
+}
+
+void launch_rows_short(const uint16_t* x, const uint16_t* w, uint16_t* out,
+                       int M, int N, int K, bool relu2, hipStream_t st) {
+  const bool one = rows_short_tiles(N, K) == 1;
+  if (relu2) {
+    if (one) go_short<1, 9, 6, 3, true>(x, w, out, M, N, K, st);
+    else go_short<2, 6, 4, 3, true>(x, w, out, M, N, K, st);
+  } else {
+    if (one) go_short<1, 9, 6, 3, false>(x, w, out, M, N, K, st);
+    else go_short<2, 6, 4, 3, false>(x, w, out, M, N, K, st);
+  }
 }
 
 void launch_sum_parts(const float* parts, uint16_t* out, int splits,

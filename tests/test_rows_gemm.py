@@ -1,5 +1,6 @@
 """Products of few rows: edges of row tiles, weight panels, the ring of K
-steps and the division of K; a row's result is the same in any batch."""
+steps and the division of K; a row's result is the same in any batch of up to
+64 rows, and in any larger one."""
 
 import pytest
 import torch
@@ -26,13 +27,26 @@ def close(got, want, size, rtol=2 ** -8):
 
 @pytest.mark.parametrize("N,K", [
     (4, 64), (60, 64), (64, 128), (68, 192), (6160, 320), (8196, 448),
-    (16448, 64), (25540, 192), (25664, 704), (1536, 4096)])
+    (16448, 64), (25540, 192), (25664, 704), (1536, 4096),
+    # panels of 16 and of 32 rows with K divided among a workgroup's waves:
+    # fewer steps than waves, some waves one step more, around the lines
+    # between the kernels
+    (4096, 192), (4100, 320), (8188, 704), (4092, 3072), (2048, 3136),
+    (508, 8192), (516, 8192), (4112, 4096), (4100, 4160)])
 def test_rows_linear(N, K):
     x, w = operands(N, K)
     whole = ops.rows_linear(x, w)
     close(whole, x.double() @ w.double().T, K ** 0.5)
+    few = ops.rows_linear(x[:64].contiguous(), w)
+    close(few, x[:64].double() @ w.double().T, K ** 0.5)
     for m in ROWS:
-        assert torch.equal(ops.rows_linear(x[:m].contiguous(), w), whole[:m])
+        assert torch.equal(ops.rows_linear(x[:m].contiguous(), w),
+                           (few if m <= 64 else whole)[:m])
+    if torch.ops.rlli.rows_relu2_ok(64, N, K):
+        got = torch.ops.rlli.rows_linear_relu2(x[:64].contiguous(), w)
+        y = x[:64].double() @ w.double().T
+        # the square doubles a sum's relative error and scales it by the sum
+        close(got, y.clamp(min=0) ** 2, 8 * K)
     parts = torch.ops.rlli.rows_linear_parts(x, w)
     if parts.dim() == 3:
         s = parts[0].clone()

@@ -63,8 +63,10 @@ DEV_INLINE float log_rwkv(float z) {
 }
 
 // ------------------------------------------------------------- decode
-template <typename T, int KIND>
-__global__ __launch_bounds__(256)
+// One workgroup per sequence and head; what there is to do is to read and
+// write the state, of which NT threads have eight rows each in flight.
+template <typename T, int KIND, int NT>
+__global__ __launch_bounds__(NT)
 void gla_decode_kernel(GlaArgs a) {
   constexpr bool FG = KIND == kHgrn2, BONUS = KIND == kRwkv;
   extern __shared__ __attribute__((aligned(16))) float sm[];
@@ -78,7 +80,7 @@ void gla_decode_kernel(GlaArgs a) {
   float* red = a1 + (a.rank + 3) / 4 * 4;   // [rows][vpad] then sums
   const T* row = reinterpret_cast<const T*>(a.proj) + int64_t(seq) * a.stride;
   if constexpr (FG) {
-    for (int d = tid; d < a.dim; d += 256) {
+    for (int d = tid; d < a.dim; d += NT) {
       const int hc = h * a.dim + d;
       qs[d] = silu<T>(act_load(row + hc));
       ks[d] = forget_key<T>(act_load(row + a.off_k + hc) + a.a2_bias[hc],
@@ -87,17 +89,17 @@ void gla_decode_kernel(GlaArgs a) {
   } else {
     const T* low =
         reinterpret_cast<const T*>(a.a1) + int64_t(seq) * a.a1_stride;
-    for (int r = tid; r < a.rank; r += 256)
+    for (int r = tid; r < a.rank; r += NT)
       a1[r] = BONUS ? gtanh<T>(act_load(low + r)) : act_load(low + r);
     const float qscale = BONUS ? 1.f : 1.f / sqrtf(float(a.dim));
-    for (int d = tid; d < a.dim; d += 256) {
+    for (int d = tid; d < a.dim; d += NT) {
       qs[d] = act_load(row + h * a.dim + d) * qscale;
       ks[d] = act_load(row + a.off_k + h * a.dim + d);
       if constexpr (BONUS) uk[d] = a.bonus[h * a.dim + d] * ks[d];
     }
   }
   const int v4n = a.vpad / 4;
-  const int n_rows = 256 / v4n;
+  const int n_rows = NT / v4n;
   const int vr = tid / v4n, vc = tid % v4n;
   const bool live = vr < n_rows;
   f32x4_t v = f32x4_t{0.f, 0.f, 0.f, 0.f};
@@ -109,7 +111,7 @@ void gla_decode_kernel(GlaArgs a) {
   }
   __syncthreads();
   if constexpr (!FG) {
-    for (int d = tid; d < a.dim; d += 256) {
+    for (int d = tid; d < a.dim; d += NT) {
       const T* w = reinterpret_cast<const T*>(a.a2) +
                    int64_t(h * a.dim + d) * a.rank;
       float z = a.a2_bias[h * a.dim + d];
@@ -152,21 +154,23 @@ void gla_decode_kernel(GlaArgs a) {
   }
   __syncthreads();
   float ss = 0.f;
-  for (int e = tid; e < a.vdim; e += 256) {
+  for (int e = tid; e < a.vdim; e += NT) {
     float t = 0.f;
     for (int r = 0; r < n_rows; ++r) t += red[r * a.vpad + e];
     red[e] = t;                         // column e is this thread's alone
     ss += t * t;
   }
-  __shared__ float ws[4];
+  __shared__ float ws[NT / 64];
   ss = wave_sum(ss);
   if ((tid & 63) == 0) ws[tid >> 6] = ss;
   __syncthreads();
-  const float inv =
-      1.f / sqrtf((ws[0] + ws[1] + ws[2] + ws[3]) / a.vdim + a.eps);
+  ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < NT / 64; ++i) ss += ws[i];
+  const float inv = 1.f / sqrtf(ss / a.vdim + a.eps);
   T* out = reinterpret_cast<T*>(a.out) + int64_t(seq) * a.out_stride +
            h * a.vdim;
-  for (int e = tid; e < a.vdim; e += 256) {
+  for (int e = tid; e < a.vdim; e += NT) {
     float o2 = red[e] * inv * a.norm[h * a.norm_stride + e];
     if constexpr (!FG)
       o2 *= silu<T>(act_load(row + a.off_g + h * a.vdim + e));
@@ -546,13 +550,26 @@ void by_kind(const GlaArgs& a, F f) {
 
 void launch_gla_decode(const GlaArgs& a, hipStream_t st) {
   if (a.rows == 0) return;
-  const int n_rows = 256 / (a.vpad / 4);
+  // 1024 threads for states of 128 KB and more where each can have a CU of its
+  // own (us with 256 threads and with 1024, heads of 128 x 256: 8 of them 8.6
+  // and 6.8, 128 of them 10.7 and 9.0, 512 of them 24.1 and 26.5; of 128 x
+  // 128: 6.2 and 5.8, 7.2 and 6.9, 12.0 and 15.9; 256 of these 8.4 and 8.4)
+  const bool wide = int64_t(a.dim) * a.vpad >= 128 * 256 &&
+                    int64_t(a.rows) * a.heads <= 256;
+  const int n_rows = (wide ? 1024 : 256) / (a.vpad / 4);
   const size_t smem =
       size_t((a.kind == kRwkv ? 4 : 3) * a.dpad + (a.rank + 3) / 4 * 4 +
              n_rows * a.vpad) * sizeof(float);
   by_kind(a, [&](auto t, auto kind) {
-    hipLaunchKernelGGL((gla_decode_kernel<decltype(t), decltype(kind)::value>),
-                       dim3(a.rows, a.heads), dim3(256), smem, st, a);
+    using T = decltype(t);
+    constexpr int KIND = decltype(kind)::value;
+    const dim3 grid(a.rows, a.heads);
+    if (wide)
+      hipLaunchKernelGGL((gla_decode_kernel<T, KIND, 1024>), grid, dim3(1024),
+                         smem, st, a);
+    else
+      hipLaunchKernelGGL((gla_decode_kernel<T, KIND, 256>), grid, dim3(256),
+                         smem, st, a);
   });
 }
 

@@ -66,6 +66,14 @@ def _linear_parts(x, w):
     return _linear(x, w)
 
 
+def _linear_relu2(x, w):
+    """relu2 of _linear."""
+    if (not _USE_SKINNY and not lt_autotune.enabled() and ops.rows_fit(x, w)
+            and ops.rows_whole(x, w)):
+        return ops.rows_linear_relu2(x, w)
+    return ops.relu2(_linear(x, w))
+
+
 @dataclasses.dataclass
 class LlamaConfig:
     name: str

@@ -26,7 +26,7 @@ import torch.nn.functional as F
 
 from .. import ops
 from ..engine.kv_cache import KVLayer, StateLayer
-from .llama import _linear
+from .llama import _linear, _linear_parts, _linear_relu2
 from .mixed import DenseSpec, LayerSpec, MixedConfig, MixedModel
 
 
@@ -358,11 +358,17 @@ class NesizenForCausalLM(MixedModel):
             dist.all_reduce(y, group=self.tp_group)
         return y
 
+    def _last(self, x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+        """A sublayer's output; f32 parts where the kernel divides K and
+        hyper_step is the one to read them."""
+        if self.tp_world > 1 or (ops.rows_fit(x, w) and ops.rows_whole(x, w)):
+            return _linear(x, w)
+        return _linear_parts(x, w)
+
     def _feed_forward(self, i: int, h: torch.Tensor) -> torch.Tensor:
         P, f, p = self.params, self.config.layers[i].mlp, f"l{i}."
         if isinstance(f, DenseSpec):
-            return _linear(ops.linear_relu2(h, P[p + "up"], _linear),
-                           P[p + "down"])
+            return self._last(_linear_relu2(h, P[p + "up"]), P[p + "down"])
         return ops.moe_experts(h, P[p + "router"], P[p + "w_up"],
                                P[p + "w_down"], f.top, f.limit)
 
@@ -378,18 +384,21 @@ class NesizenForCausalLM(MixedModel):
         for n, (i, q) in enumerate(subs):
             p = f"l{i}."
             if q == 1:
-                y = _linear(mixer(i, _linear(h, P[p + "proj"])), P[p + "o"])
+                y = self._last(mixer(i, _linear(h, P[p + "proj"])),
+                               P[p + "o"])
             else:
                 y = self._feed_forward(i, h)
             y = self._reduce(y)
             mix, out = P[f"{p}hc{q}.mix"], P[f"{p}hc{q}.out"]
+            split = y.dtype == torch.float32 != self.dtype
             if n + 1 < len(subs):
                 j, r = subs[n + 1]
                 h = ops.hyper_step(x, y, mix, out, P[f"l{j}.hc{r}.in"],
-                                   P[f"l{j}.norm{r}"], c.rms_eps)
+                                   P[f"l{j}.norm{r}"], c.rms_eps, split=split)
             else:
                 h = ops.hyper_step(x, y, mix, out, None, P["final.norm"],
-                                   c.rms_eps, sample_idx, keep=False)
+                                   c.rms_eps, sample_idx, keep=False,
+                                   split=split)
         return _linear(h, P["head"])
 
     def _attn_args(self, i: int, m: AttentionSpec):

@@ -298,14 +298,17 @@ def rows_linear_silu(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     return silu_mul(torch.nn.functional.linear(x, w))
 
 
-def linear_relu2(x: torch.Tensor, w: torch.Tensor, linear) -> torch.Tensor:
-    """relu2 of ``linear(x, w)``; for few rows and a w that is not large in
-    one kernel, which squares the f32 sums."""
-    if rows_fit(x, w):
-        _gpu()
-        if torch.ops.rlli.rows_relu2_ok(x.shape[0], *w.shape):
-            return torch.ops.rlli.rows_linear_relu2(x, w)
-    return relu2(linear(x, w))
+def rows_whole(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """For x and w that rows_fit: whether rows_linear takes them without
+    dividing K over workgroups; rows_linear_relu2 is for these."""
+    _gpu()
+    return torch.ops.rlli.rows_whole_ok(x.shape[0], *w.shape)
+
+
+def rows_linear_relu2(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """relu2(x w^T), of the f32 sums."""
+    _gpu()
+    return torch.ops.rlli.rows_linear_relu2(x, w)
 
 
 def skinny_linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
@@ -377,10 +380,13 @@ def hyper_embed(ids, table, w_embed, x, in_w, gain, eps: float):
 
 
 def hyper_step(x, y, mix, out_w, in_w, gain, eps: float, rows=None,
-               keep: bool = True):
+               keep: bool = True, split: bool = False):
     """Write one sublayer's output into the streams and return the normed
     input of the next (``in_w`` None: the plain stream sum).  ``y`` may be
     [T, parts, W]; ``rows`` restricts the result (then keep=False)."""
+    if split:
+        return torch.ops.rlli_mix.hyper_step(x, y, mix, out_w, in_w, gain, eps,
+                                             rows, keep, True)
     return _mix(y).hyper_step(x, y, mix, out_w, in_w, gain, eps, rows, keep)
 
 

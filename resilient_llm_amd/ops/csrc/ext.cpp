@@ -562,11 +562,11 @@ Tensor rows_linear(const Tensor& x, const Tensor& w) {
 // the squared positive part of x w^T, of the f32 sums
 Tensor rows_linear_relu2(const Tensor& x, const Tensor& w) {
   Tensor whole = rows_short(x, w, true);
-  TORCH_CHECK(whole.defined(), "rows_relu2_ok says which products these are");
+  TORCH_CHECK(whole.defined(), "rows_whole_ok says which products these are");
   return whole;
 }
 
-bool rows_relu2_ok(int64_t M, int64_t N, int64_t K) {
+bool rows_whole_ok(int64_t M, int64_t N, int64_t K) {
   return M <= 64 && N <= 8192 && K <= 8192 &&
          rlli::rows_short_tiles(int(N), int(K)) > 0;
 }
@@ -699,7 +699,7 @@ TORCH_LIBRARY(rlli, m) {
   m.def("rows_linear(Tensor x, Tensor w) -> Tensor");
   m.def("rows_linear_silu(Tensor x, Tensor w) -> Tensor");
   m.def("rows_linear_relu2(Tensor x, Tensor w) -> Tensor");
-  m.def("rows_relu2_ok(int m, int n, int k) -> bool", &rows_relu2_ok);
+  m.def("rows_whole_ok(int m, int n, int k) -> bool", &rows_whole_ok);
   m.def("skinny_linear(Tensor x, Tensor w) -> Tensor");
   m.def("skinny2_linear(Tensor x, Tensor w, int splitk) -> Tensor");
   m.def("skinny2_silu_linear(Tensor gu, Tensor w, int splitk) -> Tensor");

@@ -46,20 +46,29 @@ Tensor hyper_embed(const Tensor& ids, const Tensor& table,
 }
 
 // in_w absent: the plain sum of the streams; rows: final subset, streams
-// are then left as they are
+// are then left as they are; split: y is the f32 parts [n, T, W] of a product
+// and h bf16
 Tensor hyper_step(Tensor x, const Tensor& y, const Tensor& mix,
                   const Tensor& out_w, const OptTensor& in_w,
                   const Tensor& gain, double eps, const OptTensor& rows,
-                  bool keep) {
+                  bool keep, bool split) {
   rlli::HyperArgs a{};
   check_streams(x);
-  a.f32 = act_f32(y, "y");
+  a.f32 = act_f32(y, "y") && !split;
   a.streams = int(x.size(1));
   a.width = int(x.size(2));
   const int64_t T = x.size(0);
-  TORCH_CHECK(y.numel() % (T * a.width ? T * a.width : 1) == 0 &&
-              y.size(0) == T && y.size(-1) == a.width, "y/streams mismatch");
-  a.parts = T ? int(y.numel() / (T * a.width)) : 1;
+  if (split) {
+    TORCH_CHECK(y.dim() == 3 && y.scalar_type() == at::kFloat &&
+                y.size(0) >= 1 && y.size(1) == T && y.size(2) == a.width,
+                "parts of y are f32 [n, rows, width]");
+    a.parts = int(y.size(0));
+    a.y_rows = int(T);
+  } else {
+    TORCH_CHECK(y.numel() % (T * a.width ? T * a.width : 1) == 0 &&
+                y.size(0) == T && y.size(-1) == a.width, "y/streams mismatch");
+    a.parts = T ? int(y.numel() / (T * a.width)) : 1;
+  }
   a.x = x.data_ptr<float>();
   a.y = y.data_ptr();
   a.mix = f32_vec(mix, int64_t(a.streams) * a.streams, "mix");
@@ -75,7 +84,8 @@ Tensor hyper_step(Tensor x, const Tensor& y, const Tensor& mix,
     a.rows = rows->data_ptr<int64_t>();
     a.n = int(rows->numel());
   }
-  Tensor h = at::empty({a.n, a.width}, y.options());
+  Tensor h = at::empty({a.n, a.width},
+                       split ? y.options().dtype(at::kBFloat16) : y.options());
   a.h = h.data_ptr();
   c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
   rlli::launch_hyper_step(a, stream_of(x));
@@ -277,8 +287,8 @@ TORCH_LIBRARY(rlli_mix, m) {
   m.def("hyper_embed(Tensor ids, Tensor table, Tensor w_embed, "
         "Tensor(a!) x, Tensor in_w, Tensor gain, float eps) -> Tensor");
   m.def("hyper_step(Tensor(a!) x, Tensor y, Tensor mix, Tensor out_w, "
-        "Tensor? in_w, Tensor gain, float eps, Tensor? rows, bool keep) "
-        "-> Tensor");
+        "Tensor? in_w, Tensor gain, float eps, Tensor? rows, bool keep, "
+        "bool split=False) -> Tensor");
   m.def("relu2(Tensor x) -> Tensor");
   m.def("window_tile_rows(int group) -> int", &window_tile_rows);
   m.def("window_tiled(Tensor qkv, Tensor k_cache, Tensor v_cache, "

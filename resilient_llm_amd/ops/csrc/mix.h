@@ -13,7 +13,8 @@ struct HyperArgs {
   const int32_t* ids;      // token ids (embed launch)
   const float* w_embed;    // embedding norm gain (embed launch)
   float* x;                // [rows, streams, width] residual streams
-  const void* y;           // [rows, parts, width] sublayer output
+  const void* y;           // [rows, parts, width] sublayer output, or f32
+                           // [parts, y_rows, width]
   const float* mix;        // [streams, streams] (from, to)
   const float* out_w;      // [streams]
   const float* in_w;       // [streams] of the next sublayer
@@ -21,6 +22,7 @@ struct HyperArgs {
   const int64_t* rows;     // row subset (final norm) or null
   void* h;                 // [n, width] normed input of the next sublayer
   int n, streams, width, parts;
+  int y_rows;              // rows of a part of y; 0: parts are a row's
   float eps;
   bool keep;               // write the streams back
   bool f32;

@@ -42,7 +42,7 @@ def test_rows_linear(N, K):
     for m in ROWS:
         assert torch.equal(ops.rows_linear(x[:m].contiguous(), w),
                            (few if m <= 64 else whole)[:m])
-    if torch.ops.rlli.rows_relu2_ok(64, N, K):
+    if torch.ops.rlli.rows_whole_ok(64, N, K):
         got = torch.ops.rlli.rows_linear_relu2(x[:64].contiguous(), w)
         y = x[:64].double() @ w.double().T
         # the square doubles a sum's relative error and scales it by the sum

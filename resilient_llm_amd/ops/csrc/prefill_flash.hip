@@ -1,70 +1,14 @@
-// Causal prompt attention on the matrix cores (bf16 products, f32 softmax):
-// over the rows of a batch of whole prompts, or over the pages of a cache
-// that holds a sequence's earlier tokens as well.
-//
-// A workgroup takes 32 rows of a sequence and up to four query heads of one
-// key/value head, a wave a head each, so that keys and values of a 64-key
-// tile are staged once for 128 (row, head) queries.  Tiles are double-
-// buffered in LDS; 16-bit ones arrive by direct global -> LDS loads that are
-// in flight under the products of the tile before, 8-bit ones pass through
-// registers, where they are widened.
-//
-// Scores are computed transposed (keys down, queries across): a lane holds
-// 32 scores of one query, the maximum needs one cross-lane step, and the
-// weights are the second product's operand as they are, keys in the order
-// 0-3, 8-11 | 4-7, 12-15 of sixteen.  Its other operand, values by channel,
-// is read from the row-major tile with the transposing LDS read in just that
-// order, so nothing transposes values on the way in.  A query's accumulators
-// are scaled again only when its maximum has grown by 2^8 since they last
-// were; until then weights are up to 2^8, with the same relative rounding.
-//
-// Bounds: for long prompts the products (32 MFMA of 32 cycles a tile and
-// wave) beside about as many cycles of exponentials and conversions and of
-// LDS reads; two workgroups share a CU so that one computes while the other
-// does the rest.  Against 16x16 tiles of 32 rows with weights through LDS and
-// values transposed on the way in, 32/8 heads of 128: a prompt of 7901 rows
-// 3850 -> 663 us (133 -> 771 TF), 64 prompts of 128 rows 140 -> 52 us, 512
-// rows behind 1500 cached tokens 236 -> 58 us.
+// Launches of prompt attention over batch rows and over pages; the kernel is
+// in prefill_flash.h.
 
-#include "common.h"
-
-#include <type_traits>
+#include "prefill_flash.h"
 
 namespace rlli {
 
 namespace {
 
-typedef short s16x8 __attribute__((ext_vector_type(8)));
-typedef short s16x4 __attribute__((ext_vector_type(4)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-typedef float f32x2 __attribute__((ext_vector_type(2)));
-typedef __bf16 b16x2 __attribute__((ext_vector_type(2)));
-
-constexpr float kHidden = -3e38f;
-constexpr int QR = 32;            // rows of a tile
-constexpr int KT = 64;            // keys of a tile
-
-DEV_INLINE uint32_t pack2(float a, float b) {
-  const b16x2 v = __builtin_convertvector((f32x2{a, b}), b16x2);
-  return __builtin_bit_cast(uint32_t, v);
-}
-
-DEV_INLINE void lds_load16(const void* g, void* l) {
-  __builtin_amdgcn_global_load_lds(
-      (const __attribute__((address_space(1))) void*)g,
-      (__attribute__((address_space(3))) void*)l, 16, 0, 0);
-}
-
-// four keys of this lane's channel; see prefill_flash_kernel for addresses
-DEV_INLINE s16x4 read_tr(const uint16_t* p) {
-  return __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-      (__attribute__((address_space(3))) s16x4*)p);
-}
-
-// Where a workgroup's keys are.  find(): which rows are this tile's;
-// false: none.
 struct BatchRows {                // k and v are columns of the batch's rows
-  static constexpr bool kPaged = false;
+  static constexpr bool kPaged = false, kWindow = false;
   using KC = CacheBF16;
   const uint16_t* qkv;
   const int32_t* cu;              // [n_seqs + 1]
@@ -106,7 +50,7 @@ struct BatchRows {                // k and v are columns of the batch's rows
 
 template <typename C>
 struct Pages {                    // [blocks, n_kv, block, D]
-  static constexpr bool kPaged = true;
+  static constexpr bool kPaged = true, kWindow = false;
   using KC = C;
   const uint16_t* qkv;
   const typename C::elem *k, *v;
@@ -122,273 +66,6 @@ struct Pages {                    // [blocks, n_kv, block, D]
     return nrows > 0;
   }
 };
-
-// D: head width; W: waves, each with a head of its own; BS: block size of
-// the cache where it is known
-template <int D, int W, int BS, typename Src>
-__global__ __launch_bounds__(64 * W, W == 4 ? 2 : 1)
-void prefill_flash_kernel(Src src, uint16_t* __restrict__ out, int n_tiles,
-                          int n_kv, int group, int stride, float scale) {
-  using KC = typename Src::KC;
-  constexpr bool kDirect = std::is_same<KC, CacheBF16>::value;
-  constexpr int NT = 64 * W;
-  constexpr int CH = D / 8;                  // 16-byte pieces of a row
-  constexpr int NP = KT * CH / NT;           // pieces a thread stages
-  constexpr int DC = D / 16;                 // steps of a score's product
-  constexpr int VT = D / 32;                 // channel tiles
-  constexpr int HALF = KT * D;
-  __shared__ __attribute__((aligned(16))) uint16_t lds[2 * 2 * HALF];
-
-  // the tiles of a key/value head stay on an XCD (workgroups go to XCDs in
-  // turn), those with the longest context first
-  const int per_head = n_tiles * (group / W);
-  int kvh, i;
-  if (n_kv % 8 == 0) {
-    i = blockIdx.x / 8;
-    kvh = i / per_head * 8 + blockIdx.x % 8;
-  } else {
-    i = blockIdx.x;
-    kvh = i / per_head;
-  }
-  i %= per_head;
-  const int tile = n_tiles - 1 - i / (group / W);
-  int row0, nrows, first, pos0;
-  if (!src.find(tile, row0, nrows, first, pos0)) return;
-
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int qi = lane & 31, hi = lane >> 5;
-  const int n_q = n_kv * group;
-  const int head = kvh * group + i % (group / W) * W + w;
-  const int qpos = pos0 + min(qi, nrows - 1);
-  const int len = pos0 + nrows;              // keys that the last row sees
-
-  // queries; a negative scale goes into their signs
-  s16x8 qf[DC];
-  {
-    const uint16_t* q = src.qkv + int64_t(row0 + min(qi, nrows - 1)) * stride +
-                        head * D + hi * 8;
-    const uint32_t flip = scale < 0.f ? 0x80008000u : 0u;
-#pragma unroll
-    for (int c = 0; c < DC; ++c) {
-      uint4 raw = *reinterpret_cast<const uint4*>(q + c * 16);
-      raw.x ^= flip; raw.y ^= flip; raw.z ^= flip; raw.w ^= flip;
-      qf[c] = __builtin_bit_cast(s16x8, raw);
-    }
-  }
-  const float c2 = fmaxf(fabsf(scale), 1e-30f) * 1.4426950408889634f;
-
-  // ---- staging.  Piece n of this thread goes to 16-byte slot n NT + tid
-  // of the tile; within a row the slots of keys are swizzled by the row so
-  // that sixteen rows' pieces of one column are in sixteen banks of 16
-  // bytes, those of values by 64 bytes so that four rows' 64-byte columns
-  // are in four.
-  auto row_of = [&](int n) { return (n * NT + tid) / CH; };
-  auto k_piece = [&](int n) {
-    const int r = row_of(n);
-    return (tid % CH) ^ (D == 128 ? r & 15 : (r >> 1) & 7);
-  };
-  auto v_piece = [&](int n) {
-    const int r = row_of(n);
-    return (tid % CH) ^ (D == 128 ? (r & 3) << 2 : ((r >> 1) & 1) << 2);
-  };
-  int page[NP];                              // of the tile to come
-  auto look_up = [&](int kv0) {
-    if constexpr (Src::kPaged) {
-#pragma unroll
-      for (int n = 0; n < NP; ++n) {
-        const int p = min(kv0 + row_of(n), len - 1);
-        const int bs = BS ? BS : src.block_size;
-        page[n] = src.tables[int64_t(first) * src.max_blocks + p / bs];
-      }
-    }
-  };
-  // rows past the last key repeat it: they are hidden, but have to be finite
-  auto k_at = [&](int n, int kv0) {
-    const int p = min(kv0 + row_of(n), len - 1);
-    if constexpr (Src::kPaged) {
-      const int bs = BS ? BS : src.block_size;
-      return src.k + ((int64_t(page[n]) * n_kv + kvh) * bs + p % bs) * D +
-             k_piece(n) * 8;
-    } else {
-      return src.qkv + int64_t(first + p) * stride + (n_q + kvh) * D +
-             k_piece(n) * 8;
-    }
-  };
-  auto v_at = [&](int n, int kv0) {
-    const int p = min(kv0 + row_of(n), len - 1);
-    if constexpr (Src::kPaged) {
-      const int bs = BS ? BS : src.block_size;
-      return src.v + ((int64_t(page[n]) * n_kv + kvh) * bs + p % bs) * D +
-             v_piece(n) * 8;
-    } else {
-      return src.qkv + int64_t(first + p) * stride + (n_q + n_kv + kvh) * D +
-             v_piece(n) * 8;
-    }
-  };
-  typename KC::vec8 kr[kDirect ? 1 : NP], vr[kDirect ? 1 : NP];
-  auto fetch = [&](uint16_t* buf, int kv0) {
-#pragma unroll
-    for (int n = 0; n < NP; ++n) {
-      if constexpr (kDirect) {
-        // wave-uniform LDS base; lane l lands at base + 16 l
-        uint16_t* l = buf + (n * NT + w * 64) * 8;
-        lds_load16(k_at(n, kv0), l);
-        lds_load16(v_at(n, kv0), l + HALF);
-      } else {
-        kr[n] = *reinterpret_cast<const typename KC::vec8*>(k_at(n, kv0));
-        vr[n] = *reinterpret_cast<const typename KC::vec8*>(v_at(n, kv0));
-      }
-    }
-  };
-  auto land = [&](uint16_t* buf) {           // 8-bit rows, widened
-    if constexpr (!kDirect) {
-#pragma unroll
-      for (int n = 0; n < NP; ++n) {
-        float f[8];
-        uint4 o;
-        KC::to_f32(kr[n], f);
-        o = {pack2(f[0], f[1]), pack2(f[2], f[3]), pack2(f[4], f[5]),
-             pack2(f[6], f[7])};
-        *reinterpret_cast<uint4*>(buf + (n * NT + tid) * 8) = o;
-        KC::to_f32(vr[n], f);
-        o = {pack2(f[0], f[1]), pack2(f[2], f[3]), pack2(f[4], f[5]),
-             pack2(f[6], f[7])};
-        *reinterpret_cast<uint4*>(buf + HALF + (n * NT + tid) * 8) = o;
-      }
-    }
-  };
-
-  f32x16 o[VT];
-#pragma unroll
-  for (int v = 0; v < VT; ++v)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) o[v][r] = 0.f;
-  float m = kHidden, l = 0.f;                // maximum in unscaled units
-
-  // A transposing read gives lane i of sixteen column i of a tile of four
-  // rows by sixteen; lane i names row i / 4, columns 4 (i % 4) ..
-  const int tr = (lane & 15) >> 2;
-  const int v_row = (tr + hi * 4) * D + ((lane >> 4) & 1) * 16 + (lane & 3) * 4;
-  const int v_sw = D == 128 ? tr : tr >> 1;
-  const int k_sw = D == 128 ? qi & 15 : (qi >> 1) & 7;
-
-  auto products = [&](const uint16_t* ks, int kv0) {
-    const uint16_t* vs = ks + HALF;
-    f32x16 s[2];
-#pragma unroll
-    for (int kt = 0; kt < 2; ++kt) {
-#pragma unroll
-      for (int r = 0; r < 16; ++r) s[kt][r] = 0.f;
-#pragma unroll
-      for (int c = 0; c < DC; ++c) {
-        const s16x8 kf = *reinterpret_cast<const s16x8*>(
-            ks + (kt * 32 + qi) * D + (((c * 2 + hi) ^ k_sw) * 8));
-        s[kt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[c], s[kt], 0,
-                                                        0, 0);
-      }
-    }
-    if (kv0 + KT - 1 > pos0) {               // some row does not see all
-#pragma unroll
-      for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int key = kv0 + kt * 32 + (r >> 2) * 8 + hi * 4 + (r & 3);
-          if (key > qpos) s[kt][r] = kHidden;
-        }
-    }
-    float mx = fmaxf(s[0][0], s[1][0]);
-#pragma unroll
-    for (int r = 1; r < 16; ++r) mx = fmaxf(fmaxf(mx, s[0][r]), s[1][r]);
-    mx = fmaxf(mx, __shfl_xor(mx, 32, kWave));
-    // each query by itself, so that a row's result does not depend on the
-    // rows it shares a tile with
-    const bool grown = (mx - m) * c2 > 8.f;
-    if (__any(grown)) {
-      const float mn = grown ? mx : m;
-      const float corr = __builtin_amdgcn_exp2f((m - mn) * c2);
-      l *= corr;
-#pragma unroll
-      for (int v = 0; v < VT; ++v)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) o[v][r] *= corr;
-      m = mn;
-    }
-    const float mc = m * c2;
-    float sum = 0.f;
-#pragma unroll
-    for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        s[kt][r] = __builtin_amdgcn_exp2f(fmaf(s[kt][r], c2, -mc));
-        sum += s[kt][r];
-      }
-    l += sum;                                // this half's keys
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      const f32x16& p = s[t >> 1];
-      const int r = (t & 1) * 8;
-      const uint4 raw = {pack2(p[r], p[r + 1]), pack2(p[r + 2], p[r + 3]),
-                         pack2(p[r + 4], p[r + 5]), pack2(p[r + 6], p[r + 7])};
-      const s16x8 pf = __builtin_bit_cast(s16x8, raw);
-#pragma unroll
-      for (int v = 0; v < VT; ++v) {
-        const uint16_t* at = vs + v_row + t * 16 * D + (v ^ v_sw) * 32;
-        const s16x4 a = read_tr(at), b = read_tr(at + 8 * D);
-        const s16x8 vf = __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7);
-        o[v] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, pf, o[v], 0, 0, 0);
-      }
-    }
-  };
-
-  look_up(0);
-  fetch(lds, 0);
-  land(lds);
-  look_up(KT);
-  int cur = 0;
-  for (int kv0 = 0; kv0 < len; kv0 += KT) {
-    // this wave's part of the tile has landed, then everybody's; and nobody
-    // reads the tile before any more
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    uint16_t* next = lds + (cur ^ 1) * 2 * HALF;
-    const bool more = kv0 + KT < len;
-    if (more) {
-      fetch(next, kv0 + KT);
-      look_up(kv0 + 2 * KT);
-    }
-    products(lds + cur * 2 * HALF, kv0);
-    if (more) land(next);
-    cur ^= 1;
-  }
-
-  if (qi >= nrows) return;
-  l += __shfl_xor(l, 32, kWave);
-  const float inv = 1.f / l;
-  uint16_t* to = out + int64_t(row0 + qi) * n_q * D + head * D;
-#pragma unroll
-  for (int v = 0; v < VT; ++v)
-#pragma unroll
-    for (int r = 0; r < 16; r += 4)
-      *reinterpret_cast<uint2*>(to + v * 32 + (r >> 2) * 8 + hi * 4) =
-          uint2{pack2(o[v][r] * inv, o[v][r + 1] * inv),
-                pack2(o[v][r + 2] * inv, o[v][r + 3] * inv)};
-}
-
-template <int D, int BS, typename Src>
-void by_group(const Src& src, uint16_t* out, int n_tiles, int n_kv, int group,
-              int stride, float scale, hipStream_t st) {
-  auto go = [&](auto tag) {
-    constexpr int W = decltype(tag)::value;
-    hipLaunchKernelGGL((prefill_flash_kernel<D, W, BS, Src>),
-                       dim3(n_tiles * n_kv * (group / W)), dim3(64 * W), 0,
-                       st, src, out, n_tiles, n_kv, group, stride, scale);
-  };
-  if (n_tiles == 0) return;
-  if (group == 1) go(std::integral_constant<int, 1>{});
-  else if (group == 2) go(std::integral_constant<int, 2>{});
-  else go(std::integral_constant<int, 4>{});
-}
 
 }  // namespace
 

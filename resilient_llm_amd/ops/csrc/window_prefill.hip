@@ -7,9 +7,11 @@
 // 64-token K/V tiles that the window or the kept first tokens reach are
 // walked.  Rows were rotated and cached by window_rope_append before.
 // P is the larger of the key and value widths, rounded up; the unused
-// columns are zeros.
+// columns are zeros.  Heads of 64 and of 128 are with the transposed scores
+// of prefill_flash.h.
 
 #include "attn.h"
+#include "prefill_flash.h"
 
 #include <type_traits>
 
@@ -249,6 +251,53 @@ void by_cache(const WindowAttnArgs& a, hipStream_t st) {
   else go<P, CacheBF16>(a, st);
 }
 
+// ``sub`` tiles of 32 rows per tile of the table
+template <typename C>
+struct WindowPages {
+  static constexpr bool kPaged = true, kWindow = true;
+  using KC = C;
+  const uint16_t* qkv;
+  const typename C::elem *k, *v;
+  const int32_t *rows, *tables;   // [4, n] as WindowAttnArgs::tiles
+  const float* sink;
+  int n, sub, max_blocks, block_size, window, keep;
+
+  DEV_INLINE bool find(int tile, int& row0, int& nrows, int& first,
+                       int& pos0) const {
+    const int t = tile / sub, off = tile % sub * QR;
+    row0 = rows[t] + off;
+    pos0 = rows[n + t] + off;
+    nrows = min(QR, rows[2 * n + t] - off);
+    first = rows[3 * n + t];
+    return nrows > 0;
+  }
+};
+
+template <typename KC>
+void flash(const WindowAttnArgs& a, hipStream_t st) {
+  const int group = a.n_q / a.n_kv, sub = window_prefill_sub_tiles(group);
+  const WindowPages<KC> src{
+      static_cast<const uint16_t*>(a.qkv),
+      static_cast<const typename KC::elem*>(a.k_cache),
+      static_cast<const typename KC::elem*>(a.v_cache), a.tiles,
+      a.block_tables, a.sink, a.n_tiles, sub, a.max_blocks, a.block_size,
+      a.window, a.keep_first};
+  auto go = [&](auto d, auto bs) {
+    by_group<decltype(d)::value, decltype(bs)::value>(
+        src, static_cast<uint16_t*>(a.out), a.n_tiles * sub, a.n_kv, group,
+        a.stride, a.scale, st);
+  };
+  using I16 = std::integral_constant<int, 16>;
+  using I0 = std::integral_constant<int, 0>;
+  using D128 = std::integral_constant<int, 128>;
+  using D64 = std::integral_constant<int, 64>;
+  if (a.dim == 128) {
+    if (a.block_size == 16) go(D128{}, I16{}); else go(D128{}, I0{});
+  } else {
+    if (a.block_size == 16) go(D64{}, I16{}); else go(D64{}, I0{});
+  }
+}
+
 }  // namespace
 
 // 32-row sub-tiles per tile: fills up to eight waves with (head, rows)
@@ -258,6 +307,20 @@ int window_prefill_sub_tiles(int group) {
 
 void launch_window_prefill(const WindowAttnArgs& a, hipStream_t st) {
   if (a.n_tiles == 0) return;
+  const int group = a.n_q / a.n_kv;
+  // heads that prefill_flash.h is made for, in whole pieces as its direct
+  // loads take them (16/4 heads of 128, four prompts of up to 2048 rows,
+  // window 1024: 93 us against 285)
+  auto whole = [](const void* p) {
+    return reinterpret_cast<uintptr_t>(p) % 16 == 0;
+  };
+  if (a.dim == a.vdim && (a.dim == 128 || a.dim == 64) &&
+      (group <= 2 || group % 4 == 0) && whole(a.qkv) && whole(a.k_cache) &&
+      whole(a.v_cache)) {
+    if (a.cache == kCacheFP8) flash<CacheFP8>(a, st);
+    else flash<CacheBF16>(a, st);
+    return;
+  }
   const int d = a.dim > a.vdim ? a.dim : a.vdim;
   if (d <= 32) by_cache<32>(a, st);
   else if (d <= 64) by_cache<64>(a, st);

@@ -28,7 +28,7 @@
 // lane groups with one accumulator each, 32/8 heads of 128, us: 64 sequences
 // of 134-192 tokens 19.6 -> 13.2 (3.2 TB/s); 16 of 1.7k-4.1k 59 -> 48
 // (4 TB/s, 5 but for what a launch, the lengths and the second kernel take);
-// 37 of 1k-2k with an 8-bit cache 59 -> 40; one of 8000 33 -> 16.
+// 37 of 1k-2k with an 8-bit cache 59 -> 36; one of 8000 33 -> 16.
 //
 // Fused form: rotation of q and k, the append to the cache and the new
 // token's own term are part of it; that token's key and value come from LDS,
@@ -155,7 +155,9 @@ DEV_INLINE uint32_t bf16_pair(float a, float b) {
                             __builtin_convertvector((f32x2{a, b}), b16x2));
 }
 
-// cache elements as bf16 (8-bit ones are exact in it), two per dword
+// cache elements as bf16 (8-bit ones are exact in it), two per dword; by one
+// conversion a pair (through 32-bit floats, and with keys loaded 8 bytes a
+// lane, 37 sequences of 1k-2k took 40 us)
 template <typename KC, int N, typename R>
 DEV_INLINE void widen(const R& raw, uint32_t (&out)[N]) {
   if constexpr (std::is_same<KC, CacheBF16>::value) {
@@ -164,11 +166,11 @@ DEV_INLINE void widen(const R& raw, uint32_t (&out)[N]) {
   } else {
 #pragma unroll
     for (int i = 0; i < N; i += 2) {
-      const int w = int(word(raw, i / 2));
-      const f32x2_cvt a = __builtin_amdgcn_cvt_pk_f32_fp8(w, false);
-      const f32x2_cvt b = __builtin_amdgcn_cvt_pk_f32_fp8(w, true);
-      out[i] = bf16_pair(a.x, a.y);
-      out[i + 1] = bf16_pair(b.x, b.y);
+      const uint32_t w = word(raw, i / 2);
+      out[i] = __builtin_bit_cast(
+          uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, 1.f, false));
+      out[i + 1] = __builtin_bit_cast(
+          uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, 1.f, true));
     }
   }
 }
@@ -181,7 +183,10 @@ void decode_attn_kernel(DecodeArgs a) {
   using vec8 = typename KC::vec8;
   constexpr int KSTEPS = D / 32;
   constexpr int VT = D / 16;               // channel tiles
-  using kraw = typename Words<sizeof(elem) * 8>::type;
+  // A lane's 16 bytes of a key are the channels of KPL steps of the scores'
+  // product: step k has of lane group ``oct`` those from k_chan(k).
+  constexpr int KPL = 2 / sizeof(elem), KLOADS = KSTEPS / KPL;
+  using kraw = typename Words<16>::type;
   using vraw = typename Words<sizeof(elem) * VT>::type;
   constexpr int QROW = D + 8;
   __shared__ __attribute__((aligned(16))) float raw[(GROUP + 2) * D];
@@ -200,6 +205,9 @@ void decode_attn_kernel(DecodeArgs a) {
   const elem* vc = static_cast<const elem*>(a.v_cache);
   const int n_q = a.n_kv * GROUP;
   const float c2 = a.scale * 1.4426950408889634f;
+  auto k_chan = [&](int k) {
+    return k / KPL * 32 * KPL + (oct * KPL + k % KPL) * 8;
+  };
 
   int kvh, seq, part = 0, u0 = 0, u1, n_parts = 1;
   if constexpr (SHARES) {
@@ -256,16 +264,16 @@ void decode_attn_kernel(DecodeArgs a) {
     else
       return (int64_t(page[t * 5 + i]) * a.n_kv + kvh) * bs + tok % bs;
   };
-  kraw kr[2][KSTEPS];
+  kraw kr[2][KLOADS];
   vraw vr[2][4];
   auto load_keys = [&](int u) {
     if (u >= u1) return;
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
-      const elem* p = kc + row_of(u, t, 0, key_tok(u, t)) * D + oct * 8;
+      const elem* p = kc + row_of(u, t, 0, key_tok(u, t)) * D + k_chan(0);
 #pragma unroll
-      for (int k = 0; k < KSTEPS; ++k)
-        kr[t][k] = *reinterpret_cast<const kraw*>(p + k * 32);
+      for (int k = 0; k < KLOADS; ++k)
+        kr[t][k] = *reinterpret_cast<const kraw*>(p + k * 32 * KPL);
     }
   };
   auto load_values = [&](int u) {
@@ -358,8 +366,7 @@ void decode_attn_kernel(DecodeArgs a) {
   for (int k = 0; k < KSTEPS; ++k) {
     uint4 w{0, 0, 0, 0};
     if (head < GROUP)
-      w = *reinterpret_cast<const uint4*>(qs + col * QROW + k * 32 +
-                                          oct * 8);
+      w = *reinterpret_cast<const uint4*>(qs + col * QROW + k_chan(k));
     qf[k] = __builtin_bit_cast(s16x8, w);
   }
 
@@ -376,9 +383,9 @@ void decode_attn_kernel(DecodeArgs a) {
       for (int t = 0; t < 2; ++t) {
         const bool own = key_tok(u, t) == last;
 #pragma unroll
-        for (int k = 0; k < KSTEPS; ++k) {
+        for (int k = 0; k < KLOADS; ++k) {
           const kraw w =
-              *reinterpret_cast<const kraw*>(self + k * 32 + oct * 8);
+              *reinterpret_cast<const kraw*>(self + k_chan(k * KPL));
           kr[t][k] = own ? w : kr[t][k];
         }
       }
@@ -394,12 +401,15 @@ void decode_attn_kernel(DecodeArgs a) {
     for (int t = 0; t < 2; ++t) {
       s[t] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int k = 0; k < KSTEPS; ++k) {
-        uint32_t w[4];
+      for (int k = 0; k < KLOADS; ++k) {
+        uint32_t w[4 * KPL];
         widen<KC>(kr[t][k], w);
-        s[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-            __builtin_bit_cast(s16x8, (uint4{w[0], w[1], w[2], w[3]})),
-            qf[k], s[t], 0, 0, 0);
+#pragma unroll
+        for (int j = 0; j < KPL; ++j)
+          s[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              __builtin_bit_cast(s16x8, (uint4{w[j * 4], w[j * 4 + 1],
+                                               w[j * 4 + 2], w[j * 4 + 3]})),
+              qf[k * KPL + j], s[t], 0, 0, 0);
       }
     }
     load_keys(u + 4);

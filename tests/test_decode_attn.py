@@ -141,3 +141,22 @@ def test_rows_of_one_sequence():
             qkv[at], pos[at], cs, k, v, slots[at], tables[at], n[at], 0.1, 8)
         assert torch.equal(got[at], want)
     assert torch.equal(k, kc) and torch.equal(v, vc)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+def test_8_bit_codes_come_out_as_they_are(D):
+    codes = torch.arange(256).to(torch.uint8).view(torch.float8_e4m3fn)
+    # (the two NaNs as zeros)
+    codes = torch.where(codes.float().isnan(), torch.zeros(256),
+                        codes.float()).to(torch.float8_e4m3fn)
+    rows = codes.view(256 // D, 1, 1, D)
+    k = torch.zeros(256 // D, 1, 16, D).to(torch.float8_e4m3fn)
+    v = k.clone()
+    k[:, :, :1], v[:, :, :1] = rows, rows
+    n = torch.ones(256 // D, dtype=torch.int32)
+    q = torch.ones(256 // D, 2, D, dtype=torch.bfloat16)
+    got = ops.decode_attn(q.to(DEV), k.to(DEV), v.to(DEV),
+                          torch.arange(256 // D, dtype=torch.int32)[:, None]
+                          .contiguous().to(DEV), n.to(DEV), 0.01)
+    want = rows.float().view(-1, 1, D).expand(-1, 2, -1)
+    assert torch.equal(got.cpu().float(), want)

@@ -28,7 +28,7 @@
 // does the rest.  Against 16x16 tiles of 32 rows with weights through LDS and
 // values transposed on the way in, 32/8 heads of 128: a prompt of 7901 rows
 // 3850 -> 623 us (133 -> 820 TF), 64 prompts of 128 rows 140 -> 50 us, 512
-// rows behind 1500 cached tokens 236 -> 58 us.
+// rows behind 1500 cached tokens 236 -> 45 us.
 
 #pragma once
 
@@ -78,21 +78,27 @@ DEV_INLINE s16x4 read_tr(const uint16_t* p) {
 // are this tile's; false: none.  A windowed one also says which keys a row
 // sees (``window`` of them and the first ``keep``) and a head's sink.
 
-// D: head width; W: waves, each with a head of its own; BS: block size of
-// the cache where it is known
-template <int D, int W, int BS, typename Src>
-__global__ __launch_bounds__(64 * W, W == 4 ? 2 : 1)
+// D: head width; W: heads, a wave each; BS: block size of the cache where it
+// is known; KS: waves per head, each with every KS-th tile of keys, for
+// launches that leave CUs idle.  Their sums meet in LDS.
+template <int D, int W, int BS, int KS, typename Src>
+__global__ __launch_bounds__(64 * W * KS, W == 4 ? 2 : 1)
 void prefill_flash_kernel(Src src, uint16_t* __restrict__ out, int n_tiles,
                           int n_kv, int group, int stride, float scale) {
   using KC = typename Src::KC;
   constexpr bool kDirect = std::is_same<KC, CacheBF16>::value;
-  constexpr int NT = 64 * W;
+  static_assert(KS == 1 || !Src::kWindow, "windows skip single tiles");
+  constexpr int NT = 64 * W * KS;
   constexpr int CH = D / 8;                  // 16-byte pieces of a row
-  constexpr int NP = KT * CH / NT;           // pieces a thread stages
+  constexpr int NP = KS * KT * CH / NT;      // pieces a thread stages
   constexpr int DC = D / 16;                 // steps of a score's product
   constexpr int VT = D / 32;                 // channel tiles
   constexpr int HALF = KT * D;
-  __shared__ __attribute__((aligned(16))) uint16_t lds[2 * 2 * HALF];
+  constexpr int STAGE = KS * 2 * HALF;       // keys | values, of KS tiles
+  __shared__ __attribute__((aligned(16))) uint16_t
+      lds_static[KS == 1 ? 2 * STAGE : 8];
+  extern __shared__ __attribute__((aligned(16))) uint16_t lds_dynamic[];
+  uint16_t* lds = KS == 1 ? lds_static : lds_dynamic;
 
   // the tiles of a key/value head stay on an XCD (workgroups go to XCDs in
   // turn), those with the longest context first
@@ -111,7 +117,8 @@ void prefill_flash_kernel(Src src, uint16_t* __restrict__ out, int n_tiles,
   if (!src.find(tile, row0, nrows, first, pos0)) return;
 
   const int tid = threadIdx.x, lane = tid & 63;
-  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int w = wave % W, ks = wave / W;
   const int qi = lane & 31, hi = lane >> 5;
   const int n_q = n_kv * group;
   const int head = kvh * group + i % (group / W) * W + w;
@@ -126,7 +133,7 @@ void prefill_flash_kernel(Src src, uint16_t* __restrict__ out, int n_tiles,
     win0 = max(0, pos0 - window + 1) / KT * KT;
   }
   auto after = [&](int kv0) {
-    const int n = kv0 + KT;
+    const int n = kv0 + KS * KT;
     return Src::kWindow && n >= keep && n < win0 ? win0 : n;
   };
 
@@ -151,6 +158,9 @@ void prefill_flash_kernel(Src src, uint16_t* __restrict__ out, int n_tiles,
   // bytes, those of values by 64 bytes so that four rows' 64-byte columns
   // are in four.
   auto row_of = [&](int n) { return (n * NT + tid) / CH; };
+  auto slot_of = [&](int s) {                // slot of KS tiles -> elements
+    return (KS == 1 ? s : s / (KT * CH) * 2 * KT * CH + s % (KT * CH)) * 8;
+  };
   auto k_piece = [&](int n) {
     const int r = row_of(n);
     return (tid % CH) ^ (D == 128 ? r & 15 : (r >> 1) & 7);
@@ -199,7 +209,7 @@ void prefill_flash_kernel(Src src, uint16_t* __restrict__ out, int n_tiles,
     for (int n = 0; n < NP; ++n) {
       if constexpr (kDirect) {
         // wave-uniform LDS base; lane l lands at base + 16 l
-        uint16_t* l = buf + (n * NT + w * 64) * 8;
+        uint16_t* l = buf + slot_of(n * NT + wave * 64);
         lds_load16(k_at(n, kv0), l);
         lds_load16(v_at(n, kv0), l + HALF);
       } else {
@@ -217,11 +227,11 @@ void prefill_flash_kernel(Src src, uint16_t* __restrict__ out, int n_tiles,
         KC::to_f32(kr[n], f);
         o = {pack2(f[0], f[1]), pack2(f[2], f[3]), pack2(f[4], f[5]),
              pack2(f[6], f[7])};
-        *reinterpret_cast<uint4*>(buf + (n * NT + tid) * 8) = o;
+        *reinterpret_cast<uint4*>(buf + slot_of(n * NT + tid)) = o;
         KC::to_f32(vr[n], f);
         o = {pack2(f[0], f[1]), pack2(f[2], f[3]), pack2(f[4], f[5]),
              pack2(f[6], f[7])};
-        *reinterpret_cast<uint4*>(buf + HALF + (n * NT + tid) * 8) = o;
+        *reinterpret_cast<uint4*>(buf + HALF + slot_of(n * NT + tid)) = o;
       }
     }
   };
@@ -293,7 +303,8 @@ void prefill_flash_kernel(Src src, uint16_t* __restrict__ out, int n_tiles,
       m = mn;
     }
     // a row that has seen nothing yet: weights of what is hidden are nothing
-    const float mc = Src::kWindow && m == kHidden ? 0.f : m * c2;
+    const float mc =
+        (Src::kWindow || KS > 1) && m == kHidden ? 0.f : m * c2;
 #pragma unroll
     for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
@@ -332,19 +343,46 @@ void prefill_flash_kernel(Src src, uint16_t* __restrict__ out, int n_tiles,
     // reads the tile before any more
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    uint16_t* next = lds + (cur ^ 1) * 2 * HALF;
+    uint16_t* next = lds + (cur ^ 1) * STAGE;
     const bool more = ahead < len;
     if (more) {
       fetch(next, ahead);
       look_up(after(ahead));
     }
-    products(lds + cur * 2 * HALF, kv0);
+    if (KS == 1 || kv0 + ks * KT < len)
+      products(lds + cur * STAGE + ks * 2 * HALF, kv0 + ks * KT);
     if (more) land(next);
     cur ^= 1;
     kv0 = ahead;
     ahead = after(kv0);
   }
 
+  if constexpr (KS > 1) {
+    static_assert(KS == 2, "two waves of a head meet");
+    constexpr int ROW = VT * 16 + 2;
+    float* side = reinterpret_cast<float*>(lds) + w * ROW * 64 + lane;
+    __syncthreads();
+    if (ks == 1) {
+#pragma unroll
+      for (int v = 0; v < VT; ++v)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) side[(v * 16 + r) * 64] = o[v][r];
+      side[VT * 16 * 64] = m;
+      side[(VT * 16 + 1) * 64] = l;
+    }
+    __syncthreads();
+    if (ks == 1) return;
+    // this wave has the first tile, of which every row sees a key
+    const float m1 = side[VT * 16 * 64], top = fmaxf(m, m1);
+    const float c0 = __builtin_amdgcn_exp2f((m - top) * c2);
+    const float c1 = __builtin_amdgcn_exp2f((m1 - top) * c2);
+    l = l * c0 + side[(VT * 16 + 1) * 64] * c1;
+#pragma unroll
+    for (int v = 0; v < VT; ++v)
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        o[v][r] = o[v][r] * c0 + side[(v * 16 + r) * 64] * c1;
+  }
   if (qi >= nrows) return;
   l += __shfl_xor(l, 32, kWave);
   float inv = 1.f / l;
@@ -366,19 +404,37 @@ void prefill_flash_kernel(Src src, uint16_t* __restrict__ out, int n_tiles,
                 pack2(o[v][r + 2] * inv, o[v][r + 3] * inv)};
 }
 
+// ``keys``: as many as a sequence may have.
 template <int D, int BS, typename Src>
 void by_group(const Src& src, uint16_t* out, int n_tiles, int n_kv, int group,
-              int stride, float scale, hipStream_t st) {
-  auto go = [&](auto tag) {
-    constexpr int W = decltype(tag)::value;
-    hipLaunchKernelGGL((prefill_flash_kernel<D, W, BS, Src>),
-                       dim3(n_tiles * n_kv * (group / W)), dim3(64 * W), 0,
-                       st, src, out, n_tiles, n_kv, group, stride, scale);
+              int stride, float scale, int keys, hipStream_t st) {
+  auto go = [&](auto tag, auto waves) {
+    constexpr int W = decltype(tag)::value, KS = decltype(waves)::value;
+    constexpr size_t smem = KS == 1 ? 0 : size_t(KS) * 2 * 2 * KT * D * 2;
+    auto* k = prefill_flash_kernel<D, W, BS, KS, Src>;
+    if (smem > 65536)
+      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(k),
+                                hipFuncAttributeMaxDynamicSharedMemorySize,
+                                int(smem));
+    hipLaunchKernelGGL(k, dim3(n_tiles * n_kv * (group / W)),
+                       dim3(64 * W * KS), smem, st, src, out, n_tiles, n_kv,
+                       group, stride, scale);
   };
+  using I1 = std::integral_constant<int, 1>;
+  using I2 = std::integral_constant<int, 2>;
+  using I4 = std::integral_constant<int, 4>;
   if (n_tiles == 0) return;
-  if (group == 1) go(std::integral_constant<int, 1>{});
-  else if (group == 2) go(std::integral_constant<int, 2>{});
-  else go(std::integral_constant<int, 4>{});
+  if (group == 1) go(I1{}, I1{});
+  else if (group == 2) go(I2{}, I1{});
+  else if constexpr (Src::kWindow) go(I4{}, I1{});
+  // up to a workgroup and a half per CU, and more than a few tiles of keys (us
+  // with one wave per head and with two, 32/8 heads of 128: 512 rows behind
+  // 1500 tokens 56.5 and 45.0, 1536 behind 1500 93 and 88; a prompt of 1000
+  // 31.0 and 27.6, 1536 44.7 and 36.7, 384 15.4 and 15.0, 128 9.7 and 10.7;
+  // 4 of 512 28.0 and 31.1)
+  else if (n_tiles * n_kv * (group / 4) <= 400 && keys >= 384)
+    go(I4{}, I2{});
+  else go(I4{}, I1{});
 }
 
 }  // namespace

@@ -79,10 +79,10 @@ void launch_prefill_rows(const uint16_t* qkv, const int32_t* cu_seqlens,
   if (rows == 0) return;
   if (head_dim == 128)
     by_group<128, 0>(src, out, n_tiles, n_kv_heads, group, qkv_stride, scale,
-                     st);
+                     rows / n_seqs, st);
   else
     by_group<64, 0>(src, out, n_tiles, n_kv_heads, group, qkv_stride, scale,
-                    st);
+                    rows / n_seqs, st);
 }
 
 void launch_prefill_paged(const uint16_t* qkv, const void* k_cache,
@@ -103,7 +103,8 @@ void launch_prefill_paged(const uint16_t* qkv, const void* k_cache,
                         chunk_row0, chunk_pos0, chunk_nrows, chunk_btrow,
                         block_tables, max_blocks, block_size};
     by_group<decltype(d)::value, decltype(bs)::value>(
-        src, out, n_chunks, n_kv_heads, group, qkv_stride, scale, st);
+        src, out, n_chunks, n_kv_heads, group, qkv_stride, scale,
+        max_blocks * block_size, st);
   };
   auto by_dim = [&](auto kc) {
     using I16 = std::integral_constant<int, 16>;

@@ -285,7 +285,7 @@ void flash(const WindowAttnArgs& a, hipStream_t st) {
   auto go = [&](auto d, auto bs) {
     by_group<decltype(d)::value, decltype(bs)::value>(
         src, static_cast<uint16_t*>(a.out), a.n_tiles * sub, a.n_kv, group,
-        a.stride, a.scale, st);
+        a.stride, a.scale, 0, st);
   };
   using I16 = std::integral_constant<int, 16>;
   using I0 = std::integral_constant<int, 0>;

@@ -67,3 +67,37 @@ def test_pages(n_q, n_kv, D, bs, fp8):
         D ** -0.5, n_q)
     k, v = (x.float().to(torch.bfloat16) for x in (k, v))
     close(got, ref.prefill_paged_attn(qkv, k, v, *t, tables, D ** -0.5, n_q))
+
+
+@pytest.mark.parametrize("n_q,n_kv,D", [(4, 1, 128), (8, 1, 64)])
+@pytest.mark.parametrize("lens", [[385], [448, 449], [384, 1, 800]], ids=str)
+def test_two_waves_per_head(n_q, n_kv, D, lens):
+    """Few workgroups: tiles of keys go to two waves in turn; odd and even
+    counts of tiles, rows that the second wave has nothing for."""
+    test_batch_rows(n_q, n_kv, D, lens)
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("D,bs", [(128, 16), (64, 16), (128, 8)])
+def test_two_waves_per_head_over_pages(D, bs, fp8):
+    n_q, n_kv = 8, 2
+    gen = torch.Generator().manual_seed(bs)
+    seqs = [(0, 33), (63, 1), (447, 66), (512, 31), (0, 400)]
+    width = -(-544 // bs)
+    k, v = (torch.randn(len(seqs) * width, n_kv, bs, D, generator=gen)
+            .to(torch.float8_e4m3fn if fp8 else torch.bfloat16) for _ in "kv")
+    tables = torch.randperm(len(seqs) * width, generator=gen) \
+        .to(torch.int32).view(len(seqs), width)
+    qkv = torch.randn(sum(n for _, n in seqs), (n_q + 2 * n_kv) * D,
+                      generator=gen).to(torch.bfloat16)
+    tiles, row = [], 0
+    for b, (start, n) in enumerate(seqs):
+        tiles += [(row + o, start + o, min(32, n - o), b)
+                  for o in range(0, n, 32)]
+        row += n
+    t = torch.tensor(tiles, dtype=torch.int32).t().contiguous()
+    got = ops.prefill_paged_attn(
+        qkv.to(DEV), k.to(DEV), v.to(DEV), *t.to(DEV), tables.to(DEV),
+        D ** -0.5, n_q)
+    k, v = (x.float().to(torch.bfloat16) for x in (k, v))
+    close(got, ref.prefill_paged_attn(qkv, k, v, *t, tables, D ** -0.5, n_q))

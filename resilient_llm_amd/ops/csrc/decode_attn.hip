@@ -26,9 +26,9 @@
 //                    sequence together
 // Against as many parts for each sequence as the batch had of sequences, in
 // lane groups with one accumulator each, 32/8 heads of 128, us: 64 sequences
-// of 134-192 tokens 19.6 -> 13.2 (3.2 TB/s); 16 of 1.7k-4.1k 59 -> 48
-// (4 TB/s, 5 but for what a launch, the lengths and the second kernel take);
-// 37 of 1k-2k with an 8-bit cache 59 -> 36; one of 8000 33 -> 16.
+// of 134-192 tokens 19.6 -> 12.8 (3.3 TB/s); 16 of 1.7k-4.1k 59 -> 46
+// (4.3 TB/s, 5 but for what a launch, the lengths and the second kernel
+// take); 37 of 1k-2k with an 8-bit cache 59 -> 34; one of 8000 33 -> 16.
 //
 // Fused form: rotation of q and k, the append to the cache and the new
 // token's own term are part of it; that token's key and value come from LDS,
@@ -276,14 +276,17 @@ void decode_attn_kernel(DecodeArgs a) {
         kr[t][k] = *reinterpret_cast<const kraw*>(p + k * 32 * KPL);
     }
   };
+  // Whole lines that nobody reads again pass the caches by (16 sequences of
+  // 1.7k-4.1k: 49.0 -> 46.0 us); an instruction takes halves of lines of the
+  // keys, which come slower so (47.2).
   auto load_values = [&](int u) {
     if (u >= u1) return;
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
       for (int i = 0; i < 4; ++i)
-        vr[t][i] = *reinterpret_cast<const vraw*>(
-            vc + row_of(u, t, 1 + i, value_tok(u, t, i)) * D + col * VT);
+        vr[t][i] = __builtin_nontemporal_load(reinterpret_cast<const vraw*>(
+            vc + row_of(u, t, 1 + i, value_tok(u, t, i)) * D + col * VT));
   };
   look_up(u0 + wave);
   load_keys(u0 + wave);

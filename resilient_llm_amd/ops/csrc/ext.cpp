@@ -439,7 +439,7 @@ Tensor prefill_attn_qkv(const Tensor& qkv, const Tensor& cu_seqlens,
                         int64_t head_dim) {
   check_bf16_contig(qkv, "qkv");
   TORCH_CHECK(cu_seqlens.scalar_type() == at::kInt &&
-              cu_seqlens.is_contiguous() && cu_seqlens.numel() >= 1);
+              cu_seqlens.is_contiguous());
   const int T = int(qkv.size(0));
   const int D = int(head_dim);
   const int stride = int(qkv.size(1));
@@ -448,10 +448,14 @@ Tensor prefill_attn_qkv(const Tensor& qkv, const Tensor& cu_seqlens,
   TORCH_CHECK(group == 1 || group == 2 || group == 4 || group == 8);
   TORCH_CHECK(D == 64 || D == 128);
   const int n_seqs = int(cu_seqlens.numel()) - 1;
+  TORCH_CHECK(T == 0 || n_seqs >= 1, "rows without a sequence: cu_seqlens has ",
+              cu_seqlens.numel(), " entries");
   Tensor out = at::empty({T, n_q * D}, qkv.options());
   c10::hip::HIPGuardMasqueradingAsCUDA guard(qkv.device());
+  // on the host it may be too
+  const Tensor cu = cu_seqlens.to(qkv.device());
   rlli::launch_prefill_rows(
-      bf16_ptr(qkv), cu_seqlens.data_ptr<int32_t>(), bf16_ptr(out), n_seqs, T,
+      bf16_ptr(qkv), cu.data_ptr<int32_t>(), bf16_ptr(out), n_seqs, T,
       int(n_kv), group, D, stride, float(scale), current_stream(qkv));
   check_launch("prefill_attn_qkv");
   return out;

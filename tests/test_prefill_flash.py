@@ -101,3 +101,17 @@ def test_two_waves_per_head_over_pages(D, bs, fp8):
         D ** -0.5, n_q)
     k, v = (x.float().to(torch.bfloat16) for x in (k, v))
     close(got, ref.prefill_paged_attn(qkv, k, v, *t, tables, D ** -0.5, n_q))
+
+
+def test_row_offsets_of_any_device_and_count():
+    gen = torch.Generator().manual_seed(1)
+    qkv = torch.randn(45, 6 * 64, generator=gen).to(torch.bfloat16).to(DEV)
+    cu = torch.tensor([0, 13, 45], dtype=torch.int32)
+    args = 0.125, 4, 1, 64
+    assert torch.equal(ops.prefill_attn_qkv(qkv, cu, *args),
+                       ops.prefill_attn_qkv(qkv, cu.to(DEV), *args))
+    for none in (cu[:1], cu[:0]):
+        for t in (none, none.to(DEV)):
+            with pytest.raises(RuntimeError, match="without a sequence"):
+                ops.prefill_attn_qkv(qkv, t, *args)
+            assert ops.prefill_attn_qkv(qkv[:0], t, *args).shape == (0, 256)

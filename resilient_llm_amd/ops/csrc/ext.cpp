@@ -44,6 +44,12 @@ void check_bf16_contig(const Tensor& t, const char* name) {
 }
 
 
+// ``t`` from a multiple of 16 bytes on, copied if it is elsewhere: what direct
+// global -> LDS loads of 16 bytes are made for
+Tensor aligned(const Tensor& t) {
+  return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 ? t.clone() : t;
+}
+
 // cache tensors: bf16 or fp8-e4m3 (common.h codecs); returns the fp8
 // flag after validating dtype/contiguity/device
 bool check_cache(const Tensor& k_cache, const Tensor& v_cache) {
@@ -454,8 +460,9 @@ Tensor prefill_attn_qkv(const Tensor& qkv, const Tensor& cu_seqlens,
   c10::hip::HIPGuardMasqueradingAsCUDA guard(qkv.device());
   // on the host it may be too
   const Tensor cu = cu_seqlens.to(qkv.device());
+  const Tensor rows = aligned(qkv);
   rlli::launch_prefill_rows(
-      bf16_ptr(qkv), cu.data_ptr<int32_t>(), bf16_ptr(out), n_seqs, T,
+      bf16_ptr(rows), cu.data_ptr<int32_t>(), bf16_ptr(out), n_seqs, T,
       int(n_kv), group, D, stride, float(scale), current_stream(qkv));
   check_launch("prefill_attn_qkv");
   return out;
@@ -489,8 +496,9 @@ Tensor prefill_paged_attn(const Tensor& qkv, const Tensor& k_cache,
   const int max_blocks = int(block_tables.size(1));
   Tensor out = at::empty({T, n_q * D}, qkv.options());
   c10::hip::HIPGuardMasqueradingAsCUDA guard(qkv.device());
+  const Tensor k = aligned(k_cache), v = aligned(v_cache);
   rlli::launch_prefill_paged(
-      bf16_ptr(qkv), k_cache.data_ptr(), v_cache.data_ptr(),
+      bf16_ptr(qkv), k.data_ptr(), v.data_ptr(),
       chunk_row0.data_ptr<int32_t>(), chunk_pos0.data_ptr<int32_t>(),
       chunk_nrows.data_ptr<int32_t>(), chunk_btrow.data_ptr<int32_t>(),
       block_tables.data_ptr<int32_t>(), bf16_ptr(out), n_chunks, n_kv,
@@ -604,12 +612,12 @@ static void check_skinny(const char* op, const Tensor& x, const Tensor& w,
 
 Tensor skinny_linear(const Tensor& x, const Tensor& w) {
   check_skinny("skinny_linear", x, w, x.size(1));
-  return rows_linear(x, w);
+  return rows_linear(aligned(x), aligned(w));
 }
 
 Tensor skinny2_linear(const Tensor& x, const Tensor& w, int64_t /*splitk*/) {
   check_skinny("skinny2_linear", x, w, x.size(1));
-  return rows_linear(x, w);
+  return rows_linear(aligned(x), aligned(w));
 }
 
 // down-proj behind SwiGLU: (silu(gu[:, :K]) * gu[:, K:]) @ w^T, gu [M, 2K]
@@ -617,7 +625,7 @@ Tensor skinny2_silu_linear(const Tensor& gu, const Tensor& w,
                            int64_t /*splitk*/) {
   TORCH_CHECK(gu.size(1) % 2 == 0, "gu must be [M, 2K]");
   check_skinny("skinny2_silu", gu, w, gu.size(1) / 2);
-  return rows_linear(silu_mul(gu), w);
+  return rows_linear(silu_mul(gu), aligned(w));
 }
 
 Tensor stream_probe(const Tensor& w, int64_t splitk) {

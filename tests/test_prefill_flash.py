@@ -115,3 +115,30 @@ def test_row_offsets_of_any_device_and_count():
             with pytest.raises(RuntimeError, match="without a sequence"):
                 ops.prefill_attn_qkv(qkv, t, *args)
             assert ops.prefill_attn_qkv(qkv[:0], t, *args).shape == (0, 256)
+
+
+def off_by(t, n):
+    """``t`` from ``n`` elements behind an aligned address on."""
+    flat = torch.empty(t.numel() + n, dtype=t.dtype, device=DEV)
+    flat[n:] = t.to(DEV).flatten()
+    return flat[n:].view(t.shape)
+
+
+def test_operands_of_any_alignment():
+    gen = torch.Generator().manual_seed(2)
+    qkv = torch.randn(45, 6 * 64, generator=gen).to(torch.bfloat16)
+    cu = torch.tensor([0, 13, 45], dtype=torch.int32).to(DEV)
+    args = 0.125, 4, 1, 64
+    want = ops.prefill_attn_qkv(qkv.to(DEV), cu, *args)
+    assert torch.equal(ops.prefill_attn_qkv(off_by(qkv, 4), cu, *args), want)
+    k, v = (torch.randn(4, 1, 16, 64, generator=gen).to(torch.bfloat16)
+            for _ in "kv")
+    tiles = torch.tensor([[0, 0, 32, 0], [32, 32, 13, 0]],
+                         dtype=torch.int32).t().contiguous().to(DEV)
+    table = torch.tensor([[2, 0, 3, 1]], dtype=torch.int32).to(DEV)
+
+    def paged(k, v):
+        return ops.prefill_paged_attn(qkv.to(DEV), k, v, *tiles, table, 0.125,
+                                      4)
+    assert torch.equal(paged(off_by(k, 4), off_by(v, 4)),
+                       paged(k.to(DEV), v.to(DEV)))

@@ -95,3 +95,26 @@ def test_norm_of_parts(n, rows, dim):
     r = res.double()
     y = r * torch.rsqrt(r.pow(2).mean(-1, keepdim=True) + 1e-5) * w.double()
     torch.testing.assert_close(got.double(), y, rtol=2 ** -8, atol=2 ** -16)
+
+
+def off_by(t, n):
+    """``t`` from ``n`` elements behind an aligned address on."""
+    flat = torch.empty(t.numel() + n, dtype=t.dtype, device=DEV)
+    flat[n:] = t.flatten()
+    return flat[n:].view(t.shape)
+
+
+def test_skinny_forms_take_any_alignment():
+    x, w = (t.contiguous() for t in operands(64, 512))
+    x = x[:5].contiguous()
+    want = ops.rows_linear(x[:, :256].contiguous(), w[:, :256].contiguous())
+    a = off_by(x[:, :256], 4)
+    b = off_by(w[:, :256], 4)
+    assert not ops.rows_fit(a, b)
+    for got in (ops.skinny_linear(a, b), ops.skinny2_linear(a, b),
+                ops.linear_auto(a, b)):
+        assert torch.equal(got, want)
+    gu = torch.cat([x[:, :256], x[:, 256:]], 1)
+    assert torch.equal(
+        ops.skinny2_silu_linear(gu, b),
+        ops.skinny2_silu_linear(gu, w[:, :256].contiguous()))

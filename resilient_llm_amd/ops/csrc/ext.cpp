@@ -124,7 +124,7 @@ Tensor rmsnorm_residual_parts_(const Tensor& parts, Tensor residual,
   const int64_t dim = residual.size(-1);
   TORCH_CHECK(parts.scalar_type() == at::kFloat && parts.is_cuda() &&
                   parts.is_contiguous() && parts.dim() == 3 &&
-                  parts.size(2) == dim &&
+                  parts.size(0) >= 1 && parts.size(2) == dim &&
                   parts.size(1) * dim == residual.numel() &&
                   w.numel() == dim,
               "parts must be contiguous f32 [n, rows, dim]");
@@ -295,7 +295,8 @@ static Tensor decode_attn_any(const Tensor& q, int64_t n_q,
                               const Tensor* slot_mapping) {
   const bool parts = q.scalar_type() == at::kFloat;
   if (parts) {
-    TORCH_CHECK(q.is_cuda() && q.is_contiguous() && q.dim() == 3,
+    TORCH_CHECK(q.is_cuda() && q.is_contiguous() && q.dim() == 3 &&
+                    q.size(0) >= 1,
                 "parts must be contiguous f32 [n, batch, width]");
   } else {
     check_bf16_contig(q, "q");
@@ -316,8 +317,11 @@ static Tensor decode_attn_any(const Tensor& q, int64_t n_q,
                                   group == 8),
               "GQA group must be 1/2/4/8, got ", group);
   TORCH_CHECK(D == 64 || D == 128, "head_dim must be 64 or 128, got ", D);
-  TORCH_CHECK(block_size > 0 && v_cache.sizes() == k_cache.sizes());
-  TORCH_CHECK(block_table.size(0) == batch && seq_lens.numel() == batch);
+  TORCH_CHECK(block_size > 0 &&
+              v_cache.sizes().slice(1) == k_cache.sizes().slice(1));
+  // (longer ones, as a batch's buffers are, end in what nobody reads)
+  TORCH_CHECK(block_table.size(0) >= batch && seq_lens.numel() >= batch,
+              "tables and lengths of ", batch, " sequences are needed");
   Tensor out = at::empty({batch, n_q * D},
                          q.options().dtype(at::kBFloat16));
   if (batch == 0) return out;
@@ -353,7 +357,10 @@ Tensor decode_attn(const Tensor& q, const Tensor& k_cache,
                    const Tensor& v_cache, const Tensor& block_table,
                    const Tensor& seq_lens, double scale) {
   check_bf16_contig(q, "q");
-  TORCH_CHECK(q.dim() == 3 && q.size(2) == k_cache.size(3));
+  TORCH_CHECK(q.dim() == 3 && q.size(2) == k_cache.size(3) &&
+              v_cache.sizes() == k_cache.sizes());
+  TORCH_CHECK(block_table.size(0) == q.size(0) &&
+              seq_lens.numel() == q.size(0));
   const int gpw = 64 / (int(q.size(2)) / 8);
   TORCH_CHECK(k_cache.size(2) % gpw == 0, "block_size must be a multiple of ",
               gpw);
@@ -364,7 +371,9 @@ Tensor decode_attn(const Tensor& q, const Tensor& k_cache,
 
 static void check_qkv_width(const Tensor& qkv, const Tensor& k_cache,
                             int64_t n_q) {
-  TORCH_CHECK(qkv.size(-1) == (n_q + 2 * k_cache.size(1)) * k_cache.size(3),
+  TORCH_CHECK(qkv.dim() == (qkv.scalar_type() == at::kFloat ? 3 : 2) &&
+                  qkv.size(-1) ==
+                      (n_q + 2 * k_cache.size(1)) * k_cache.size(3),
               "qkv width mismatch");
 }
 
@@ -389,9 +398,10 @@ Tensor decode_attn_rope_qkv(const Tensor& qkv, const Tensor& positions,
   TORCH_CHECK(slot_mapping.scalar_type() == at::kInt && slot_mapping.is_contiguous());
   TORCH_CHECK(cos_sin.scalar_type() == at::kFloat && cos_sin.is_contiguous());
   TORCH_CHECK(cos_sin.size(1) == k_cache.size(3));
-  const int64_t batch = qkv.size(qkv.dim() == 3 ? 1 : 0);
-  TORCH_CHECK(positions.numel() == batch && slot_mapping.numel() == batch);
   check_qkv_width(qkv, k_cache, n_q);
+  const int64_t batch = qkv.size(qkv.dim() == 3 ? 1 : 0);
+  TORCH_CHECK(positions.numel() >= batch && slot_mapping.numel() >= batch,
+              "positions and slots of ", batch, " sequences are needed");
   return decode_attn_any(qkv, n_q, k_cache, v_cache, block_table, seq_lens,
                          scale, &positions, &cos_sin, &slot_mapping);
 }

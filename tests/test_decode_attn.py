@@ -160,3 +160,55 @@ def test_8_bit_codes_come_out_as_they_are(D):
                           .contiguous().to(DEV), n.to(DEV), 0.01)
     want = rows.float().view(-1, 1, D).expand(-1, 2, -1)
     assert torch.equal(got.cpu().float(), want)
+
+
+def fused_args(lens, n_q=8, n_kv=2, D=128):
+    k, v, tables, n, qkv = (t.to(DEV) for t in setup(lens, n_q, n_kv, D, 16,
+                                                     False))
+    pos = n - 1
+    slots = tables.gather(1, (pos // 16).long()[:, None])[:, 0] * 16 \
+        + pos % 16
+    return qkv, pos, ref.build_cos_sin(max(lens), D, device=DEV), k, v, \
+        slots, tables, n
+
+
+def test_buffers_longer_than_the_batch():
+    qkv, pos, cs, k, v, slots, tables, n = fused_args([37, 300, 5, 64])
+    want = ops.decode_attn_rope_qkv(qkv[:3], pos[:3], cs, k.clone(), v.clone(),
+                                    slots[:3], tables[:3], n[:3], 0.1, 8)
+    got = ops.decode_attn_rope_qkv(qkv[:3], pos, cs, k.clone(), v.clone(),
+                                   slots, tables, n, 0.1, 8)
+    assert torch.equal(got, want)
+    want = ops.decode_attn_qkv(qkv[:3], k, v, tables[:3], n[:3], 0.1, 8)
+    assert torch.equal(ops.decode_attn_qkv(qkv[:3], k, v, tables, n, 0.1, 8),
+                       want)
+    # a values' cache of more pages
+    more = torch.cat([v, v[:1]])
+    assert torch.equal(ops.decode_attn_qkv(qkv[:3], k, more, tables, n, 0.1,
+                                           8), want)
+
+
+@pytest.mark.parametrize("short", range(4))
+def test_buffers_shorter_than_the_batch(short):
+    qkv, pos, cs, k, v, slots, tables, n = fused_args([37, 300, 5])
+    bufs = [pos, slots, tables, n]
+    bufs[short] = bufs[short][:2]
+    pos, slots, tables, n = bufs
+    with pytest.raises(RuntimeError):
+        ops.decode_attn_rope_qkv(qkv, pos, cs, k, v, slots, tables, n, 0.1, 8)
+
+
+def test_rows_of_other_ranks_are_refused():
+    qkv, pos, cs, k, v, slots, tables, n = fused_args([37, 300, 5])
+    # one row per sequence in between, no parts, f32 that is not parts
+    for rows, n_pos in ((qkv[:, None], 1), (qkv.float()[None][:0], 3),
+                        (qkv.float(), 3)):
+        with pytest.raises(RuntimeError):
+            ops.decode_attn_rope_qkv(rows, pos[:n_pos], cs, k, v,
+                                     slots[:n_pos], tables, n, 0.1, 8)
+    with pytest.raises(RuntimeError):
+        ops.decode_attn_qkv(qkv[:, None], k, v, tables, n, 0.1, 8)
+    res = torch.zeros(3, 64, dtype=torch.bfloat16, device=DEV)
+    with pytest.raises(RuntimeError):
+        ops.rmsnorm_residual_(torch.zeros(0, 3, 64, device=DEV), res,
+                              res[0].clone())

@@ -422,10 +422,10 @@ class LlamaForCausalLM:
         (chunked prefill).  Returns logits for ``sample_idx`` rows."""
         if self._few_rows(input_ids.shape[0] - n_decode,
                           chunk_row0.shape[0]):
-            tables = self._row_tables(
-                input_ids.shape[0], n_decode, block_tables_dec, chunk_row0,
-                chunk_nrows, chunk_btrow, block_tables_pre)
-            seq_lens = positions + 1
+            tables, seq_lens = ops.mixed_row_tables(
+                input_ids.shape[0], n_decode, block_tables_dec, seq_lens_dec,
+                chunk_row0, chunk_pos0, chunk_nrows, chunk_btrow,
+                block_tables_pre)
 
             def attn_rows(i, qkv, k_cache, v_cache):
                 return ops.decode_attn_rows_qkv(
@@ -459,25 +459,6 @@ class LlamaForCausalLM:
         behind 1000 30 and 22, 16 behind 4000 97 and 31)."""
         return (self.device.type == "cuda" and 0 < rows <= 16 * tiles
                 and rows * self.n_kv_heads <= 256)
-
-    @staticmethod
-    def _row_tables(rows, n_decode, tables_dec, row0, nrows, btrow,
-                    tables_pre) -> torch.Tensor:
-        """The block table of every row of a mixed step."""
-        n = rows - n_decode
-        n64 = nrows.long()
-        first = row0.long() - (n64.cumsum(0) - n64)
-        at = torch.repeat_interleave(first, n64, output_size=n) \
-            + torch.arange(n, device=row0.device)
-        wide = max([tables_pre.shape[1]] + ([tables_dec.shape[1]]
-                                            if n_decode else []))
-        out = torch.zeros((rows, wide), dtype=torch.int32,
-                          device=row0.device)
-        out[at, :tables_pre.shape[1]] = tables_pre[torch.repeat_interleave(
-            btrow.long(), n64, output_size=n)]
-        if n_decode:
-            out[:n_decode, :tables_dec.shape[1]] = tables_dec
-        return out
 
     def forward_decode(self, input_ids: torch.Tensor, positions: torch.Tensor,
                        kv_cache, slot_mapping: torch.Tensor,

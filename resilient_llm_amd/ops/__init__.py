@@ -199,6 +199,21 @@ def decode_attn_rows_qkv(qkv, positions, cos_sin, k_cache, v_cache,
                            scale, n_q)
 
 
+def mixed_row_tables(rows: int, n_decode: int, tables_dec, lens_dec,
+                     chunk_row0, chunk_pos0, chunk_nrows, chunk_btrow,
+                     tables_pre) -> tuple[torch.Tensor, torch.Tensor]:
+    """Block table and length of every row of a mixed step, for
+    decode_attn_rows_qkv; rows of no tile see nothing."""
+    if tables_pre.is_cuda:
+        _gpu()
+        return torch.ops.rlli.mixed_row_tables(
+            rows, n_decode, tables_dec, lens_dec, chunk_row0, chunk_pos0,
+            chunk_nrows, chunk_btrow, tables_pre)
+    return ref.mixed_row_tables(rows, n_decode, tables_dec, lens_dec,
+                                chunk_row0, chunk_pos0, chunk_nrows,
+                                chunk_btrow, tables_pre)
+
+
 def prefill_attn_qkv(qkv: torch.Tensor, cu_seqlens: torch.Tensor,
                      scale: float, n_q: int, n_kv: int,
                      head_dim: int) -> torch.Tensor:

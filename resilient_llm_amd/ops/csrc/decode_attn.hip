@@ -35,6 +35,7 @@
 // so nothing waits for the append.  Without slots it rotates queries only.
 
 #include "common.h"
+#include "kernels.h"
 
 #include <algorithm>
 #include <cstdlib>
@@ -596,6 +597,41 @@ void decode_combine_kernel(DecodeArgs a) {
       f32_to_bf16(y > 0.f ? x / y : 0.f);
 }
 
+// A workgroup per row of a mixed step: the row's table and length, from the
+// decoding sequences or from the tile of prompt rows that has it.  Rows of no
+// tile see nothing.  (One launch instead of the ten or so that tensor ops
+// take, which small models' steps, waiting for the host, would feel.)
+__global__ __launch_bounds__(256)
+void row_tables_kernel(RowTables a, int32_t* __restrict__ tables,
+                       int32_t* __restrict__ lens, int wide) {
+  __shared__ int tile;
+  const int row = blockIdx.x;
+  const bool decoding = row < a.n_decode;
+  if (threadIdx.x == 0) tile = -1;
+  __syncthreads();
+  if (!decoding)
+    for (int t = threadIdx.x; t < a.n_tiles; t += 256) {
+      const int at = row - a.row0[t];
+      if (at >= 0 && at < min(a.nrows[t], 32)) atomicMax(&tile, t);
+    }
+  __syncthreads();
+  const int t = tile;
+  const int32_t* src = nullptr;
+  int width = 0, len = 0;
+  if (decoding) {
+    src = a.tables_dec + int64_t(row) * a.dec_width;
+    width = a.dec_width;
+    len = a.lens_dec[row];
+  } else if (t >= 0) {
+    src = a.tables_pre + int64_t(a.btrow[t]) * a.pre_width;
+    width = a.pre_width;
+    len = a.pos0[t] + row - a.row0[t] + 1;
+  }
+  for (int c = threadIdx.x; c < wide; c += 256)
+    tables[int64_t(row) * wide + c] = c < width ? src[c] : 0;
+  if (threadIdx.x == 0) lens[row] = len;
+}
+
 template <int D, int GROUP, typename KC, bool FUSED>
 void run(const DecodeArgs& a, hipStream_t st) {
   auto go = [&](auto bs) {
@@ -641,6 +677,13 @@ int decode_attn_shares(int batch, int n_kv_heads, int max_tokens) {
   if (batch * n_kv_heads >= 384 && max_tokens <= 1024) return 0;
   if (max_tokens <= MIN_UNITS * UNIT) return 0;      // never cut
   return std::max(1, 512 / n_kv_heads);
+}
+
+void launch_row_tables(const RowTables& a, int32_t* tables, int32_t* lens,
+                       int rows, int wide, hipStream_t stream) {
+  if (rows == 0) return;
+  hipLaunchKernelGGL(row_tables_kernel, dim3(rows), dim3(256), 0, stream, a,
+                     tables, lens, wide);
 }
 
 void launch_decode_attn(

@@ -421,6 +421,54 @@ Tensor decode_attn_q_rope(const Tensor& qkv, const Tensor& positions,
                          scale, &positions, &cos_sin, nullptr);
 }
 
+// Block table [rows, width] and length [rows] of every row of a mixed step;
+// tables and lengths of the decoding sequences may be absent if there are none.
+std::tuple<Tensor, Tensor> mixed_row_tables(
+    int64_t rows, int64_t n_decode, const c10::optional<Tensor>& tables_dec,
+    const c10::optional<Tensor>& lens_dec, const Tensor& row0,
+    const Tensor& pos0, const Tensor& nrows, const Tensor& btrow,
+    const Tensor& tables_pre) {
+  auto check = [&](const Tensor& t) {
+    TORCH_CHECK(t.scalar_type() == at::kInt && t.is_contiguous() &&
+                t.device() == tables_pre.device(),
+                "tables, lengths and tiles must be contiguous int32 on one "
+                "GPU");
+  };
+  rlli::RowTables a{};
+  for (const Tensor* t : {&row0, &pos0, &nrows, &btrow, &tables_pre})
+    check(*t);
+  a.n_tiles = int(row0.numel());
+  TORCH_CHECK(tables_pre.dim() == 2 && pos0.numel() == a.n_tiles &&
+              nrows.numel() == a.n_tiles && btrow.numel() == a.n_tiles);
+  TORCH_CHECK(n_decode >= 0 && n_decode <= rows);
+  a.n_decode = int(n_decode);
+  a.pre_width = int(tables_pre.size(1));
+  if (n_decode > 0) {
+    TORCH_CHECK(tables_dec && lens_dec);
+    check(*tables_dec);
+    check(*lens_dec);
+    TORCH_CHECK(tables_dec->dim() == 2 && tables_dec->size(0) >= n_decode &&
+                lens_dec->numel() >= n_decode);
+    a.tables_dec = tables_dec->data_ptr<int32_t>();
+    a.lens_dec = lens_dec->data_ptr<int32_t>();
+    a.dec_width = int(tables_dec->size(1));
+  }
+  a.row0 = row0.data_ptr<int32_t>();
+  a.pos0 = pos0.data_ptr<int32_t>();
+  a.nrows = nrows.data_ptr<int32_t>();
+  a.btrow = btrow.data_ptr<int32_t>();
+  a.tables_pre = tables_pre.data_ptr<int32_t>();
+  const int wide = std::max(a.pre_width, a.dec_width);
+  c10::hip::HIPGuardMasqueradingAsCUDA guard(tables_pre.device());
+  Tensor tables = at::empty({rows, wide}, tables_pre.options());
+  Tensor lens = at::empty({rows}, tables_pre.options());
+  rlli::launch_row_tables(a, tables.data_ptr<int32_t>(),
+                          lens.data_ptr<int32_t>(), int(rows), wide,
+                          current_stream(tables_pre));
+  check_launch("mixed_row_tables");
+  return {tables, lens};
+}
+
 // --------------------------------------------------------- prefill_attn
 Tensor prefill_attn(const Tensor& q, const Tensor& k, const Tensor& v,
                     const Tensor& cu_seqlens, double scale) {
@@ -712,6 +760,9 @@ TORCH_LIBRARY(rlli, m) {
   m.def("decode_attn_q_rope(Tensor qkv, Tensor positions, Tensor cos_sin, "
         "Tensor k_cache, Tensor v_cache, Tensor block_table, "
         "Tensor seq_lens, float scale, int n_q) -> Tensor");
+  m.def("mixed_row_tables(int rows, int n_decode, Tensor? tables_dec, "
+        "Tensor? lens_dec, Tensor row0, Tensor pos0, Tensor nrows, "
+        "Tensor btrow, Tensor tables_pre) -> (Tensor, Tensor)");
   m.def("prefill_attn_qkv(Tensor qkv, Tensor cu_seqlens, float scale, "
         "int n_q, int n_kv, int head_dim) -> Tensor");
   m.def("prefill_attn(Tensor q, Tensor k, Tensor v, Tensor cu_seqlens, "
@@ -747,6 +798,7 @@ TORCH_LIBRARY_IMPL(rlli, CUDA, m) {
   m.impl("decode_attn_rope_qkv", &decode_attn_rope_qkv);
   m.impl("kv_append_qkv_", &kv_append_qkv_);
   m.impl("decode_attn_q_rope", &decode_attn_q_rope);
+  m.impl("mixed_row_tables", &mixed_row_tables);
   m.impl("prefill_attn_qkv", &prefill_attn_qkv);
   m.impl("prefill_attn", &prefill_attn);
   m.impl("sample", &sample);

@@ -69,6 +69,18 @@ void launch_decode_attn(
     int max_blocks, float scale, int q_stride, int shares, float* part_out,
     float* part_ml, bool cache_fp8, hipStream_t stream);
 
+// What says which pages the rows of a mixed step see: decoding sequences
+// first, then tiles of at most 32 prompt rows.
+struct RowTables {
+  const int32_t *tables_dec, *lens_dec;       // [n_decode, dec_width], [..]
+  const int32_t *row0, *pos0, *nrows, *btrow; // [n_tiles]
+  const int32_t* tables_pre;                  // [.., pre_width]
+  int n_decode, dec_width, n_tiles, pre_width;
+};
+// tables [rows, wide], lens [rows]
+void launch_row_tables(const RowTables& a, int32_t* tables, int32_t* lens,
+                       int rows, int wide, hipStream_t stream);
+
 // Varlen causal prefill attention over in-batch q/k/v.
 void launch_prefill_attn(
     const uint16_t* q, const uint16_t* k, const uint16_t* v,

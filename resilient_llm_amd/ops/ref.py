@@ -174,6 +174,23 @@ def prefill_paged_attn(qkv: torch.Tensor, k_cache: torch.Tensor,
     return out
 
 
+def mixed_row_tables(rows, n_decode, tables_dec, lens_dec, row0, pos0, nrows,
+                     btrow, tables_pre):
+    wide = max(tables_pre.shape[1],
+               tables_dec.shape[1] if n_decode else 0)
+    tables = torch.zeros(rows, wide, dtype=torch.int32)
+    lens = torch.zeros(rows, dtype=torch.int32)
+    if n_decode:
+        tables[:n_decode, :tables_dec.shape[1]] = tables_dec[:n_decode]
+        lens[:n_decode] = lens_dec[:n_decode]
+    for r0, p0, n, b in zip(*(t.tolist() for t in (row0, pos0, nrows,
+                                                   btrow))):
+        for r in range(min(n, 32)):
+            tables[r0 + r, :tables_pre.shape[1]] = tables_pre[b]
+            lens[r0 + r] = p0 + r + 1
+    return tables, lens
+
+
 def sample(logits: torch.Tensor, temperatures: torch.Tensor,
            seeds: torch.Tensor, step: int = 0) -> torch.Tensor:
     """Greedy rows match the kernel exactly; stochastic rows use torch

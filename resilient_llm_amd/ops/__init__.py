@@ -398,11 +398,11 @@ def hyper_step(x, y, mix, out_w, in_w, gain, eps: float, rows=None,
                keep: bool = True, split: bool = False):
     """Write one sublayer's output into the streams and return the normed
     input of the next (``in_w`` None: the plain stream sum).  ``y`` may be
-    [T, parts, W]; ``rows`` restricts the result (then keep=False)."""
-    if split:
-        return torch.ops.rlli_mix.hyper_step(x, y, mix, out_w, in_w, gain, eps,
-                                             rows, keep, True)
-    return _mix(y).hyper_step(x, y, mix, out_w, in_w, gain, eps, rows, keep)
+    [T, parts, W], or with ``split`` the f32 parts [parts, T, W] of
+    rows_linear_parts, the result then bf16; ``rows`` restricts the result
+    (then keep=False)."""
+    return _mix(y).hyper_step(x, y, mix, out_w, in_w, gain, eps, rows, keep,
+                              split)
 
 
 def relu2(x):

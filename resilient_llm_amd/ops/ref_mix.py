@@ -17,11 +17,11 @@ def hyper_embed(ids, table, w_embed, x, in_w, gain, eps):
         .to(table.dtype)
 
 
-def hyper_step(x, y, mix, out_w, in_w, gain, eps, rows, keep):
-    dtype = y.dtype
+def hyper_step(x, y, mix, out_w, in_w, gain, eps, rows, keep, split=False):
+    dtype = torch.bfloat16 if split else y.dtype
     y = y.float()
     if y.dim() == 3:
-        y = y.sum(1)
+        y = y.sum(0 if split else 1)
     new = torch.einsum("st,nsw->ntw", mix, x) \
         + out_w[None, :, None] * y[:, None]
     if keep:

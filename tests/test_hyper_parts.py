@@ -2,12 +2,29 @@
 step over their sum: widths of every launch shape, odd counts of parts, a
 subset of rows."""
 
+import subprocess
+import sys
+
 import pytest
 import torch
 
 import resilient_llm_amd.ops as ops
 from nesizen_util import F32
 from test_mix_ops import rel, rnd
+
+
+def test_the_op_is_there_on_first_use():
+    """In a process of its own: the library may be loaded here already."""
+    code = (
+        "import torch, resilient_llm_amd.ops as ops\n"
+        "d = 'cuda:0' if torch.cuda.is_available() else 'cpu'\n"
+        "x, y = torch.ones(3, 2, 8, device=d), torch.ones(4, 3, 8, device=d)\n"
+        "one = torch.ones(8, device=d)\n"
+        "h = ops.hyper_step(x, y, one[:4].view(2, 2).clone(), one[:2].clone(),"
+        " None, one, 0.0, split=True)\n"
+        "assert h.dtype == torch.bfloat16 and bool((h == 1).all()), h\n"
+        "assert bool((x == 6).all()), x\n")
+    subprocess.run([sys.executable, "-c", code], check=True, timeout=300)
 
 
 @pytest.mark.gpu

@@ -271,16 +271,48 @@ def prefill_paged_attn(qkv, k_cache, v_cache, chunk_row0, chunk_pos0,
                                   block_tables, scale, n_q)
 
 
+def _rows_faster(M: int, N: int, K: int) -> bool:
+    """Where rows_linear beats the library, with weights that no cache holds.
+    Timed at 1 to 128 rows of 300 shapes from 16 to 128256 by 256 to 28672; by
+    more than 7 % it is slower at K 8192 alone, for which the library is at its
+    best (1 row, N 4096: 17.0 and 19.1 us)."""
+    if M > 64:
+        # rows of x cost too, and panels that leave CUs idle more so (128 rows,
+        # us, the library first: 4096 x 4096 25.1 and 19.1, 4096 x 14336 77.5
+        # and 40.9, 28672 x 4096 60.6 and 57.6, 16384 x 2048 with silu 26.6 and
+        # 21.8; but 8192 x 2048 16.6 and 19.0, 12288 x 4096 34.3 and 37.0,
+        # 20480 x 4096 47.9 and 61.4, 57344 x 5120 125 and 144)
+        if N * K < 1 << 24:
+            return False
+        if N < 25600:
+            return K >= 4096 if N <= 8192 else (12288 < N <= 16384
+                                                and K <= 4096)
+        return N <= 32768 or N >= 65536 or K >= 8192
+    if N < 1024:
+        # few panels: many parts to sum, or waves with long runs of K (256 x
+        # 8192: 1 row 11.3 and 7.8, 64 rows 11.0 and 19.5; 64 x 14336, 1 row
+        # 12.4 and 51; 512 x 14336, 64 rows 19.1 and 15.6)
+        return K <= 4096 or (M <= 8 if K <= 8192 else N >= 512)
+    if 16384 < N < 25600:
+        # 64-row panels for more than one workgroup per CU and fewer than two
+        # (20480 x 3072, 16 rows 58 and 30, 64 rows 33.9 and 38.6; 20480 x
+        # 8192, 1 row 73.7 and 83.6)
+        return K <= 1024 or K < 8192 and (M <= 16 or M <= 32 and K <= 4096)
+    if 8192 < N <= 11520 and K <= 2048:
+        # parts that cost as much as what they divide (10240 x 256, 16 rows
+        # 6.3 and 6.2, 64 rows 6.7 and 10.2)
+        return M <= 16
+    return True
+
+
 def rows_fit(x: torch.Tensor, w: torch.Tensor) -> bool:
-    """Whether rows_linear takes x w^T: as many rows as leave reading w what
-    costs.  That is 64, or 128 where w is large (128 rows, us, the library's
-    time first: 4096 x 4096 24.4 and 18.6, 4096 x 14336 75.5 and 41.2, but
-    6144 x 2048 15.4 and 17.1, and for 129 rows 21.8 and 26.8)."""
+    """Whether rows_linear takes x w^T and is the faster way: as many rows as
+    leave reading w what costs."""
     return (x.is_cuda and x.dim() == 2 and 1 <= x.shape[0] <= 128
-            and (x.shape[0] <= 64 or w.numel() >= 1 << 24)
             and x.dtype == w.dtype == torch.bfloat16
             and x.shape[1] % 64 == 0 and x.shape[1] > 0
             and w.shape[0] % 4 == 0 and w.shape[0] > 0
+            and _rows_faster(x.shape[0], w.shape[0], x.shape[1])
             and x.is_contiguous() and w.is_contiguous()
             and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
             and not (x.requires_grad or w.requires_grad))

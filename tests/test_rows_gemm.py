@@ -118,3 +118,21 @@ def test_skinny_forms_take_any_alignment():
     assert torch.equal(
         ops.skinny2_silu_linear(gu, b),
         ops.skinny2_silu_linear(gu, w[:, :256].contiguous()))
+
+
+@pytest.mark.parametrize("M,N,K,fits", [
+    # as timed beside the library
+    (1, 4096, 14336, True), (64, 28672, 4096, True), (1, 256, 8192, True),
+    (64, 256, 8192, False), (1, 64, 14336, False), (64, 512, 14336, True),
+    (16, 20480, 3072, True), (64, 20480, 3072, False),
+    (1, 20480, 8192, False), (64, 24576, 1024, True),
+    (64, 10240, 256, False), (64, 10240, 4096, True),
+    (128, 4096, 4096, True), (128, 16384, 2048, True),
+    (128, 8192, 2048, False), (128, 12288, 4096, False),
+    (128, 20480, 4096, False), (128, 57344, 5120, False),
+    (128, 128256, 4096, True), (65, 2048, 2048, False)])
+def test_rows_that_fit_are_the_faster_ones(M, N, K, fits):
+    assert ops._rows_faster(M, N, K) == fits
+    x = torch.empty(M, K, dtype=torch.bfloat16, device=DEV)
+    assert ops.rows_fit(x, torch.empty(N, K, dtype=torch.bfloat16,
+                                       device=DEV)) == fits

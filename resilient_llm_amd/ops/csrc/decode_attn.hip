@@ -3,15 +3,20 @@
 // What it costs is to read every key and value once, so the work is laid out
 // by tokens: a wave takes units of 32 of them for the query heads of one
 // key/value head, asks for all their keys and values at once (16 KB), and
-// needs few registers beyond, so that four waves per SIMD keep several times
-// what memory's latency asks for under way.
+// needs few registers beyond, so that three waves per SIMD (five with heads of
+// 64) keep several times what memory's latency asks for under way.
 //
 // Both products run on the matrix cores, 16 tokens by 16 columns.  A query
-// and a weight are 32-bit numbers: each is cut into two 16-bit ones whose
-// sum has 16 bits of it, and the two are two columns of the same product
-// (columns 0-7 the heads' upper parts, 8-15 the lower), which costs nothing
-// as no more than eight heads share a key/value head.  Scores come out as the
-// second product wants its weights: a lane holds four tokens of a column.
+// and a weight are 32-bit numbers: each is cut into three 16-bit ones that
+// add up to it, all 24 bits, and for up to four heads the three are columns
+// of one product (0-3 the heads' first parts, 4-7 the second, 8-11 the
+// third), which costs nothing.  Eight heads take two products into the same
+// sums: columns 0-7 have half of the first part in both, 8-15 the second part
+// in one and the third in the other.  (With two parts, 16 bits, 0.36 % of the
+// outputs were not the bf16 number nearest to the 64-bit result; so 0.029 %,
+// with f32 products 0.028 %.  It takes 0.2 us more of 12.1 and 0.5 of 33.1.)
+// Scores come out as the second product wants its weights: a lane holds four
+// tokens of a column.
 // The second product is transposed; row n of its tile t is channel VT n + t,
 // so a lane loads VT neighbouring channels of each of its tokens, in whole
 // rows, and makes the operands of all tiles from them.
@@ -132,8 +137,13 @@ DEV_INLINE void lds_barrier() {
   asm volatile("" ::: "memory");
 }
 
-// the column eight away has the other part
-DEV_INLINE float other_part(float v) { return dpp_mov_f32<0x128>(v); }
+// the sum of the parts in a head's columns, HS apart; the same bits in each
+template <int HS>
+DEV_INLINE float sum_parts(float v) {
+  v += dpp_mov_f32<0x128>(v);              // the column eight away
+  if constexpr (HS == 4) v += dpp_mov_f32<0x124>(v);
+  return v;
+}
 
 // N bytes of cache elements, in registers
 template <int N>
@@ -149,11 +159,20 @@ DEV_INLINE uint32_t word(uint32_t w, int) { return w; }
 template <typename V>
 DEV_INLINE uint32_t word(const V& w, int i) { return w[i]; }
 
-DEV_INLINE uint32_t bf16_pair(float a, float b) {
-  typedef float f32x2 __attribute__((ext_vector_type(2)));
-  typedef __bf16 b16x2 __attribute__((ext_vector_type(2)));
-  return __builtin_bit_cast(uint32_t,
-                            __builtin_convertvector((f32x2{a, b}), b16x2));
+// The upper half of a 32-bit float is a bf16 number, its first eight bits; what
+// is left has sixteen, of which its upper half has eight, and the rest fits a
+// bf16 number.
+constexpr uint32_t kUpper = 0xffff0000u;
+
+DEV_INLINE float masked(float v, uint32_t mask) {
+  return __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, v) & mask);
+}
+DEV_INLINE uint16_t upper_half(float v) {
+  return uint16_t(__builtin_bit_cast(uint32_t, v) >> 16);
+}
+DEV_INLINE uint32_t upper_halves(float a, float b) {
+  return __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, b),
+                               __builtin_bit_cast(uint32_t, a), 0x07060302u);
 }
 
 // cache elements as bf16 (8-bit ones are exact in it), two per dword; by one
@@ -190,8 +209,9 @@ void decode_attn_kernel(DecodeArgs a) {
   using kraw = typename Words<16>::type;
   using vraw = typename Words<sizeof(elem) * VT>::type;
   constexpr int QROW = D + 8;
+  constexpr int HS = GROUP <= 4 ? 4 : 8;   // columns of a part
   __shared__ __attribute__((aligned(16))) float raw[(GROUP + 2) * D];
-  __shared__ __attribute__((aligned(16))) uint16_t qs[16 * QROW];
+  __shared__ __attribute__((aligned(16))) uint16_t qs[3 * HS * QROW];
   __shared__ __attribute__((aligned(16))) elem self[2 * D];       // k | v
   __shared__ __attribute__((aligned(16))) float accs[4 * GROUP * D];
   __shared__ float ml[4 * GROUP * 2];
@@ -199,8 +219,8 @@ void decode_attn_kernel(DecodeArgs a) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int col = lane & 15, oct = lane >> 4;
-  const int head = col & 7;
-  const bool lower = col >= 8;
+  const int cpart = col / HS;              // of its head's query or weight
+  const uint32_t mask1 = cpart > 0 ? kUpper : 0, mask2 = cpart > 1 ? kUpper : 0;
   const int bs = BS ? BS : a.block_size;
   const elem* kc = static_cast<const elem*>(a.k_cache);
   const elem* vc = static_cast<const elem*>(a.v_cache);
@@ -328,9 +348,10 @@ void decode_attn_kernel(DecodeArgs a) {
     const float* cs =
         FUSED ? a.cos_sin + int64_t(a.positions[seq]) * D : nullptr;
     auto store = [&](int h, int d, float v) {
-      const uint16_t up = f32_to_bf16(v);
-      qs[h * QROW + d] = up;
-      qs[(8 + h) * QROW + d] = f32_to_bf16(v - bf16_to_f32(up));
+      const float r0 = v - masked(v, kUpper), r1 = r0 - masked(r0, kUpper);
+      qs[h * QROW + d] = upper_half(HS == 4 ? v : 0.5f * v);
+      qs[(HS + h) * QROW + d] = upper_half(r0);
+      qs[(2 * HS + h) * QROW + d] = upper_half(r1);
     };
     for (int e = tid; e < (GROUP + (newest ? 1 : 0)) * HALF; e += 256) {
       const int h = e / HALF, j = e % HALF;
@@ -369,7 +390,7 @@ void decode_attn_kernel(DecodeArgs a) {
 #pragma unroll
   for (int k = 0; k < KSTEPS; ++k) {
     uint4 w{0, 0, 0, 0};
-    if (head < GROUP)
+    if (col < 3 * HS && col % HS < GROUP)
       w = *reinterpret_cast<const uint4*>(qs + col * QROW + k_chan(k));
     qf[k] = __builtin_bit_cast(s16x8, w);
   }
@@ -401,6 +422,9 @@ void decode_attn_kernel(DecodeArgs a) {
           vr[t][i] = value_tok(u, t, i) == last ? w : vr[t][i];
     }
     f32x4 s[2];
+    // (read again for each unit: registers are short)
+    if constexpr (HS == 8) asm volatile("" ::: "memory");
+    const uint16_t* third = qs + (col < 8 ? col : col + 8) * QROW;
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
       s[t] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -409,11 +433,18 @@ void decode_attn_kernel(DecodeArgs a) {
         uint32_t w[4 * KPL];
         widen<KC>(kr[t][k], w);
 #pragma unroll
-        for (int j = 0; j < KPL; ++j)
-          s[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+        for (int j = 0; j < KPL; ++j) {
+          const s16x8 kf =
               __builtin_bit_cast(s16x8, (uint4{w[j * 4], w[j * 4 + 1],
-                                               w[j * 4 + 2], w[j * 4 + 3]})),
-              qf[k * KPL + j], s[t], 0, 0, 0);
+                                               w[j * 4 + 2], w[j * 4 + 3]}));
+          s[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              kf, qf[k * KPL + j], s[t], 0, 0, 0);
+          if constexpr (HS == 8)
+            s[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                kf,
+                *reinterpret_cast<const s16x8*>(third + k_chan(k * KPL + j)),
+                s[t], 0, 0, 0);
+        }
       }
     }
     load_keys(u + 4);
@@ -423,7 +454,7 @@ void decode_attn_kernel(DecodeArgs a) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int tok = tok0 + t * 16 + oct * 4 + r;
-        const float v = (s[t][r] + other_part(s[t][r])) * c2;
+        const float v = sum_parts<HS>(s[t][r]) * c2;
         s[t][r] = tok <= last ? v : kNegInf;
         mx = fmaxf(mx, s[t][r]);
       }
@@ -437,27 +468,27 @@ void decode_attn_kernel(DecodeArgs a) {
       for (int t = 0; t < VT; ++t) o[t] *= corr;
       m = mn;
     }
-    uint32_t pw[4];
+    // this column's part of the weights: what is left of them when the parts
+    // before are taken off, its upper half
+    uint32_t pw[2][4];
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      float p[4];
+    for (int i = 0; i < 4; ++i) {
+      float x[2], y[2];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        p[r] = __builtin_amdgcn_exp2f(s[t][r] - m);
-        l += p[r];
+      for (int r = 0; r < 2; ++r) {
+        const float p = __builtin_amdgcn_exp2f(s[i / 2][i % 2 * 2 + r] - m);
+        l += p;
+        x[r] = fmaf(p, HS == 4 || cpart ? 1.f : 0.5f, -masked(p, mask1));
+        y[r] = x[r] - masked(x[r], HS == 4 ? mask2 : mask1);
       }
-      const uint32_t u01 = bf16_pair(p[0], p[1]), u23 = bf16_pair(p[2], p[3]);
-      const uint32_t l01 =
-          bf16_pair(p[0] - __builtin_bit_cast(float, u01 << 16),
-                    p[1] - __builtin_bit_cast(float, u01 & 0xffff0000u));
-      const uint32_t l23 =
-          bf16_pair(p[2] - __builtin_bit_cast(float, u23 << 16),
-                    p[3] - __builtin_bit_cast(float, u23 & 0xffff0000u));
-      pw[t * 2] = lower ? l01 : u01;
-      pw[t * 2 + 1] = lower ? l23 : u23;
+      if constexpr (HS == 8) pw[1][i] = upper_halves(x[0], x[1]);
+      pw[0][i] = upper_halves(y[0], y[1]);
     }
-    const s16x8 pf =
-        __builtin_bit_cast(s16x8, (uint4{pw[0], pw[1], pw[2], pw[3]}));
+    s16x8 pf[2];
+#pragma unroll
+    for (int i = 0; i < HS / 4; ++i)
+      pf[i] = __builtin_bit_cast(
+          s16x8, (uint4{pw[i][0], pw[i][1], pw[i][2], pw[i][3]}));
     uint32_t vw[2][4][VT / 2];
 #pragma unroll
     for (int t = 0; t < 2; ++t)
@@ -472,8 +503,10 @@ void decode_attn_kernel(DecodeArgs a) {
           __builtin_amdgcn_perm(vw[0][3][d], vw[0][2][d], sel),
           __builtin_amdgcn_perm(vw[1][1][d], vw[1][0][d], sel),
           __builtin_amdgcn_perm(vw[1][3][d], vw[1][2][d], sel)};
-      o[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-          __builtin_bit_cast(s16x8, w), pf, o[t], 0, 0, 0);
+#pragma unroll
+      for (int i = 0; i < HS / 4; ++i)
+        o[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+            __builtin_bit_cast(s16x8, w), pf[i], o[t], 0, 0, 0);
     }
     load_values(u + 4);
     look_up(u + 8);
@@ -485,7 +518,13 @@ void decode_attn_kernel(DecodeArgs a) {
 #pragma unroll
   for (int t = 0; t < VT; ++t)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) o[t][r] += other_part(o[t][r]);
+    for (int r = 0; r < 4; ++r) {
+      // to the first part's column; of four heads the last four columns have
+      // the third part once more
+      const float v = o[t][r];
+      o[t][r] = HS == 4 ? v + (dpp_mov_f32<0x12c>(v) + dpp_mov_f32<0x128>(v))
+                        : sum_parts<HS>(v);
+    }
   if (col < GROUP) {
     float* to = accs + (wave * GROUP + col) * D + oct * 4 * VT;
 #pragma unroll

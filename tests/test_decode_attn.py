@@ -212,3 +212,26 @@ def test_rows_of_other_ranks_are_refused():
     with pytest.raises(RuntimeError):
         ops.rmsnorm_residual_(torch.zeros(0, 3, 64, device=DEV), res,
                               res[0].clone())
+
+
+@pytest.mark.parametrize("n_q,n_kv,D,L", [
+    (32, 8, 128, 1000), (32, 4, 128, 70), (32, 4, 64, 1000), (16, 8, 64, 40),
+    (8, 8, 128, 300)])
+def test_queries_and_weights_keep_32_bits(n_q, n_kv, D, L):
+    """Of outputs with a relative error e, 2 e / 2^-8 are not the bf16 number
+    nearest to the exact one: 2^-12 for f32 sums with e = 2^-21, 2^-8 if
+    queries and weights had 16 bits."""
+    k, v, tables, n, qkv = setup([L] * 32, n_q, n_kv, D, 16, False)
+    q = qkv[:, :n_q * D].reshape(32, n_q, D)
+    cs = ref.build_cos_sin(L, D)
+    slots = tables[:, (L - 1) // 16] * 16 + (L - 1) % 16
+    kc, vc = k.to(DEV), v.to(DEV)
+    got = ops.decode_attn_rope_qkv(
+        qkv.to(DEV), (n - 1).to(DEV), cs.to(DEV), kc, vc, slots.to(DEV),
+        tables.to(DEV), n.to(DEV), D ** -0.5, n_q)
+    c, s = cs[L - 1].double().chunk(2)
+    a, b = q.double().chunk(2, -1)
+    want = exact(torch.cat([a * c - b * s, b * c + a * s], -1), kc.cpu(),
+                 vc.cpu(), tables, n, D ** -0.5)
+    off = got.cpu().view_as(q) != want.to(torch.bfloat16)
+    assert off.double().mean() < 2 ** -10

@@ -14,7 +14,9 @@
 // sums: columns 0-7 have half of the first part in both, 8-15 the second part
 // in one and the third in the other.  (With two parts, 16 bits, 0.36 % of the
 // outputs were not the bf16 number nearest to the 64-bit result; so 0.029 %,
-// with f32 products 0.028 %.  It takes 0.2 us more of 12.1 and 0.5 of 33.1.)
+// with f32 products 0.028 %.  That, and infinite keys and values as they are,
+// took the first three calls below from 12.1 to 12.6, from 45.1 to 45.6 and
+// from 33.0 to 33.7 us.)
 // Scores come out as the second product wants its weights: a lane holds four
 // tokens of a column.
 // The second product is transposed; row n of its tile t is channel VT n + t,
@@ -454,7 +456,14 @@ void decode_attn_kernel(DecodeArgs a) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int tok = tok0 + t * 16 + oct * 4 + r;
-        const float v = sum_parts<HS>(s[t][r]) * c2;
+        // An infinite key makes its score's first part infinite; the others,
+        // which may be NaN then, as a query's parts may be zero, or of the
+        // other sign, stay finite.  (8-bit keys are.)
+        const float w =
+            std::is_same<KC, CacheFP8>::value || cpart == 0
+                ? s[t][r]
+                : __builtin_amdgcn_fmed3f(s[t][r], -1e38f, 1e38f);
+        const float v = sum_parts<HS>(w) * c2;
         s[t][r] = tok <= last ? v : kNegInf;
         mx = fmaxf(mx, s[t][r]);
       }
@@ -522,8 +531,10 @@ void decode_attn_kernel(DecodeArgs a) {
       // to the first part's column; of four heads the last four columns have
       // the third part once more
       const float v = o[t][r];
-      o[t][r] = HS == 4 ? v + (dpp_mov_f32<0x12c>(v) + dpp_mov_f32<0x128>(v))
-                        : sum_parts<HS>(v);
+      const float sum =
+          HS == 4 ? v + (dpp_mov_f32<0x12c>(v) + dpp_mov_f32<0x128>(v))
+                  : sum_parts<HS>(v);
+      o[t][r] = __builtin_isinf(v) ? v : sum;    // of infinite values
     }
   if (col < GROUP) {
     float* to = accs + (wave * GROUP + col) * D + oct * 4 * VT;
@@ -597,6 +608,7 @@ void decode_combine_kernel(DecodeArgs a) {
       const bool ok = g + i * NG < n;
       const int64_t at = int64_t(ok ? g + i * NG : g) * GROUP;
       v[i] = *reinterpret_cast<const f32x4*>(po + at * D);
+      if (!ok) v[i] = f32x4{0.f, 0.f, 0.f, 0.f};     // not 0 * inf
       mm[i] = ok ? pm[at * 2] : kNegInf;
       ll[i] = ok ? pm[at * 2 + 1] : 0.f;
     }

@@ -235,3 +235,23 @@ def test_queries_and_weights_keep_32_bits(n_q, n_kv, D, L):
                  vc.cpu(), tables, n, D ** -0.5)
     off = got.cpu().view_as(q) != want.to(torch.bfloat16)
     assert off.double().mean() < 2 ** -10
+
+
+@pytest.mark.parametrize("n_q,n_kv,D,L", [(8, 2, 128, 70), (8, 1, 64, 600),
+                                          (2, 2, 64, 40)])
+def test_infinite_keys_and_values(n_q, n_kv, D, L):
+    """A key that is -inf where queries are positive takes no weight; values
+    that are infinite make their channel so.  Queries have 8 bits here, so
+    that all parts but the first are zero."""
+    k, v, tables, n, qkv = setup([L] * 3, n_q, n_kv, D, 16, False)
+    q = qkv[:, :n_q * D].reshape(3, n_q, D).contiguous()
+    q[..., 5] = q[..., 5].abs() + 0.5
+    page, at = tables[:, 1].long(), 3
+    k[page, :, at, 5] = -torch.inf
+    v[page, :, at + 1, 7] = torch.inf
+    v[page, :, at + 2, 9] = -torch.inf
+    got = ops.decode_attn(q.to(DEV), k.to(DEV), v.to(DEV), tables.to(DEV),
+                          n.to(DEV), D ** -0.5)
+    want = exact(q, k, v, tables, n, D ** -0.5)
+    assert want[..., 7].isinf().all() and want[..., :5].isfinite().all()
+    close(got, want)

@@ -122,7 +122,8 @@ def test_fused(n_q, n_kv, D, bs, lens, fp8):
 
 def test_rows_of_one_sequence():
     """Rows appended first and attended like decoded tokens: the same bits,
-    whichever way they came."""
+    whichever way they came, as no sequence of this batch is cut into other
+    parts than in a smaller one."""
     lens = [37, 38, 39, 300, 301]
     k, v, tables, n, qkv = (t.to(DEV) for t in setup(
         lens, 8, 2, 128, 16, False))
@@ -255,3 +256,20 @@ def test_infinite_keys_and_values(n_q, n_kv, D, L):
     want = exact(q, k, v, tables, n, D ** -0.5)
     assert want[..., 7].isinf().all() and want[..., :5].isfinite().all()
     close(got, want)
+
+
+def test_parts_follow_from_the_batch():
+    """Together the sequences have parts of ten units, alone of eight: the
+    sums' order differs, and with it the last bit of some outputs."""
+    lens = [4097, 4000, 4097, 4096, 3000, 700]
+    qkv, pos, cs, k, v, slots, tables, n = fused_args(lens, 8, 8, 64)
+    got = ops.decode_attn_rope_qkv(qkv, pos, cs, k.clone(), v.clone(), slots,
+                                   tables, n, 0.1, 8)
+    for b in range(len(lens)):
+        at = slice(b, b + 1)
+        want = ops.decode_attn_rope_qkv(
+            qkv[at], pos[at], cs, k.clone(), v.clone(), slots[at], tables[at],
+            n[at], 0.1, 8)
+        # each rounded to bf16 once, of sums that agree to about 2^-20
+        torch.testing.assert_close(got[at].float(), want.float(),
+                                   rtol=2 ** -7, atol=2 ** -14)

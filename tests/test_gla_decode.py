@@ -1,12 +1,15 @@
-"""Steps of gated linear attention by workgroups of 1024 and of 256 threads:
-states around the line between them, columns that do not divide the threads."""
+"""Steps of gated linear attention, HGRN2 and RWKV by workgroups of 1024 and of
+256 threads: states around the line between them, columns that do not divide
+the threads."""
 
 import pytest
 import torch
 
 import resilient_llm_amd.ops as ops
 from nesizen_util import BF16, F32
+from test_lat_ops import hgrn2_case
 from test_mix_ops import gla_case, rel, tol
+from test_rec_ops import Rwkv
 
 
 @pytest.mark.gpu
@@ -29,3 +32,35 @@ def test_steps(dim, vdim, rank, dtype):
     # the bounds of the longer runs over the same steps
     assert rel(got, want) < tol(dtype)
     assert rel(st[1, :, :, :vdim], S) < 1e-5
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [F32, BF16])
+@pytest.mark.parametrize("dim,vdim", [(128, 256), (127, 256), (164, 200),
+                                      (256, 256), (252, 130)])
+def test_hgrn2_steps(dim, vdim, dtype):
+    T, H = 9, 2
+    *inputs, eps, want, S = hgrn2_case(T, H, dim, vdim, 1.0, 0.8, dim, dtype)
+    proj, b, lower, norm = (t.cuda() for t in inputs)
+    st = torch.full((3, H, dim, -(-vdim // 4) * 4), float("nan"),
+                    device="cuda")
+    slot = torch.tensor([1], dtype=torch.int32, device="cuda")
+    got = torch.cat([
+        ops.hgrn2_decode(proj[p:p + 1].contiguous(), b, lower, norm, st, slot,
+                         torch.tensor([p], dtype=torch.int32, device="cuda"),
+                         vdim, eps) for p in range(T)])
+    assert rel(got, want) < tol(dtype)
+    assert rel(st[1, :, :, :vdim], S) < 3e-5
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [F32, BF16])
+@pytest.mark.parametrize("dim", [180, 184, 255, 256])
+def test_rwkv_steps(dim, dtype):
+    T = 9
+    a = Rwkv(T, 2, dim, 16, "cuda", dtype, seed=dim)
+    want, S = a.want()
+    got = torch.cat([a.call(p, 1, 1) for p in range(T)])
+    # the bounds of the longer runs
+    assert rel(got, want) < (1e-5 if dtype == F32 else 8e-3)
+    assert rel(a.state[1, :, :, :a.dim].cpu(), S) < 2e-5

@@ -9,7 +9,7 @@
 // Both products run on the matrix cores, 16 tokens by 16 columns.  A query
 // and a weight are 32-bit numbers: each is cut into three 16-bit ones that
 // add up to it, all 24 bits, and for up to four heads the three are columns
-// of one product (0-3 the heads' first parts, 4-7 the second, 8-11 the
+// of one product (0-3 the heads' first parts, 4-7 the second, 12-15 the
 // third), which costs nothing.  Eight heads take two products into the same
 // sums: columns 0-7 have half of the first part in both, 8-15 the second part
 // in one and the third in the other.  (With two parts, 16 bits, 0.36 % of the
@@ -139,10 +139,12 @@ DEV_INLINE void lds_barrier() {
   asm volatile("" ::: "memory");
 }
 
-// the sum of the parts in a head's columns, HS apart; the same bits in each
+// the sum of the parts in a head's columns, HS apart; the same bits in each.
+// (Of up to four heads, second and third part first: they are eight columns
+// apart, and so are the first and a column of zeros.)
 template <int HS>
 DEV_INLINE float sum_parts(float v) {
-  v += dpp_mov_f32<0x128>(v);              // the column eight away
+  v += dpp_mov_f32<0x128>(v);
   if constexpr (HS == 4) v += dpp_mov_f32<0x124>(v);
   return v;
 }
@@ -392,8 +394,9 @@ void decode_attn_kernel(DecodeArgs a) {
 #pragma unroll
   for (int k = 0; k < KSTEPS; ++k) {
     uint4 w{0, 0, 0, 0};
-    if (col < 3 * HS && col % HS < GROUP)
-      w = *reinterpret_cast<const uint4*>(qs + col * QROW + k_chan(k));
+    if (col % HS < GROUP && (HS == 8 || cpart != 2))
+      w = *reinterpret_cast<const uint4*>(
+          qs + (cpart == 3 ? col - HS : col) * QROW + k_chan(k));
     qf[k] = __builtin_bit_cast(s16x8, w);
   }
 
@@ -528,11 +531,11 @@ void decode_attn_kernel(DecodeArgs a) {
   for (int t = 0; t < VT; ++t)
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      // to the first part's column; of four heads the last four columns have
-      // the third part once more
+      // to the first part's column; of four heads the idle columns have the
+      // third part once more
       const float v = o[t][r];
       const float sum =
-          HS == 4 ? v + (dpp_mov_f32<0x12c>(v) + dpp_mov_f32<0x128>(v))
+          HS == 4 ? v + (dpp_mov_f32<0x12c>(v) + dpp_mov_f32<0x124>(v))
                   : sum_parts<HS>(v);
       o[t][r] = __builtin_isinf(v) ? v : sum;    // of infinite values
     }

@@ -307,14 +307,16 @@ def _rows_faster(M: int, N: int, K: int) -> bool:
 
 def rows_fit(x: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether rows_linear takes x w^T and is the faster way: as many rows as
-    leave reading w what costs."""
-    return (x.is_cuda and x.dim() == 2 and 1 <= x.shape[0] <= 128
+    leave reading w what costs.  (Sizes first: short prompts wait for the host,
+    and what does not fit, as most of their products, is to cost it little.)"""
+    if x.dim() != 2 or not x.is_cuda:
+        return False
+    (M, K), N = x.shape, w.shape[0]
+    return (1 <= M <= 128 and K % 64 == 0 and K > 0 and N % 4 == 0 and N > 0
+            and _rows_faster(M, N, K)
             and x.dtype == w.dtype == torch.bfloat16
-            and x.shape[1] % 64 == 0 and x.shape[1] > 0
-            and w.shape[0] % 4 == 0 and w.shape[0] > 0
-            and _rows_faster(x.shape[0], w.shape[0], x.shape[1])
             and x.is_contiguous() and w.is_contiguous()
-            and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+            and (x.data_ptr() | w.data_ptr()) % 16 == 0
             and not (x.requires_grad or w.requires_grad))
 
 

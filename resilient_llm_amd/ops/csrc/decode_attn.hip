@@ -167,6 +167,7 @@ DEV_INLINE uint32_t word(const V& w, int i) { return w[i]; }
 // is left has sixteen, of which its upper half has eight, and the rest fits a
 // bf16 number.
 constexpr uint32_t kUpper = 0xffff0000u;
+constexpr float kLeast = 0x1p-120f;
 
 DEV_INLINE float masked(float v, uint32_t mask) {
   return __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, v) & mask);
@@ -215,7 +216,7 @@ void decode_attn_kernel(DecodeArgs a) {
   constexpr int QROW = D + 8;
   constexpr int HS = GROUP <= 4 ? 4 : 8;   // columns of a part
   __shared__ __attribute__((aligned(16))) float raw[(GROUP + 2) * D];
-  __shared__ __attribute__((aligned(16))) uint16_t qs[3 * HS * QROW];
+  __shared__ __attribute__((aligned(16))) uint16_t qs[(HS == 4 ? 16 : 24) * QROW];
   __shared__ __attribute__((aligned(16))) elem self[2 * D];       // k | v
   __shared__ __attribute__((aligned(16))) float accs[4 * GROUP * D];
   __shared__ float ml[4 * GROUP * 2];
@@ -352,10 +353,15 @@ void decode_attn_kernel(DecodeArgs a) {
     const float* cs =
         FUSED ? a.cos_sin + int64_t(a.positions[seq]) * D : nullptr;
     auto store = [&](int h, int d, float v) {
-      const float r0 = v - masked(v, kUpper), r1 = r0 - masked(r0, kUpper);
+      // All parts have the sign of the first, and none is zero, so that an
+      // infinite key makes all of a score's parts infinite alike and not NaN.
+      const float least = copysignf(kLeast, v);
+      const float r0 = v - masked(v, kUpper) + least;
+      const float r1 = r0 - masked(r0, kUpper) + least;
       qs[h * QROW + d] = upper_half(HS == 4 ? v : 0.5f * v);
       qs[(HS + h) * QROW + d] = upper_half(r0);
-      qs[(2 * HS + h) * QROW + d] = upper_half(r1);
+      qs[(2 * HS + h) * QROW + d] = upper_half(HS == 4 ? least : r1);
+      if (HS == 4) qs[(3 * HS + h) * QROW + d] = upper_half(r1);
     };
     for (int e = tid; e < (GROUP + (newest ? 1 : 0)) * HALF; e += 256) {
       const int h = e / HALF, j = e % HALF;
@@ -394,9 +400,8 @@ void decode_attn_kernel(DecodeArgs a) {
 #pragma unroll
   for (int k = 0; k < KSTEPS; ++k) {
     uint4 w{0, 0, 0, 0};
-    if (col % HS < GROUP && (HS == 8 || cpart != 2))
-      w = *reinterpret_cast<const uint4*>(
-          qs + (cpart == 3 ? col - HS : col) * QROW + k_chan(k));
+    if (col % HS < GROUP)
+      w = *reinterpret_cast<const uint4*>(qs + col * QROW + k_chan(k));
     qf[k] = __builtin_bit_cast(s16x8, w);
   }
 
@@ -459,14 +464,7 @@ void decode_attn_kernel(DecodeArgs a) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int tok = tok0 + t * 16 + oct * 4 + r;
-        // An infinite key makes its score's first part infinite; the others,
-        // which may be NaN then, as a query's parts may be zero, or of the
-        // other sign, stay finite.  (8-bit keys are.)
-        const float w =
-            std::is_same<KC, CacheFP8>::value || cpart == 0
-                ? s[t][r]
-                : __builtin_amdgcn_fmed3f(s[t][r], -1e38f, 1e38f);
-        const float v = sum_parts<HS>(w) * c2;
+        const float v = sum_parts<HS>(s[t][r]) * c2;
         s[t][r] = tok <= last ? v : kNegInf;
         mx = fmaxf(mx, s[t][r]);
       }

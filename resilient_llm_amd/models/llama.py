@@ -29,7 +29,9 @@ import torch.nn.functional as F
 from .. import ops
 from ..ops import autotune as lt_autotune
 
-# Opt-in: the kernel for few rows ahead of everything else (A/B lever)
+# Opt-in (A/B lever): ops.linear_auto for all products, that is the kernel for
+# few rows where the library would be the faster one too, and without silu,
+# squares and sums in its epilogues and readers
 _USE_SKINNY = os.environ.get("RLLI_SKINNY") == "1"
 
 
@@ -456,7 +458,9 @@ class LlamaForCausalLM:
         sequence once per row but over many workgroups, beats tiles of 32
         rows that walk it one after another (8 key/value heads, us: 5 rows
         behind 200 tokens 12.5 and 8.9, behind 4000 94 and 21; 3 x 8 rows
-        behind 1000 30 and 22, 16 behind 4000 97 and 31)."""
+        behind 1000 30 and 22, 16 behind 4000 97 and 31; whole steps of the 1B
+        model, 1 x 16 rows behind 200 866 and 864, behind 4000 1466 and 1072,
+        but 4 x 5 behind 300 873 and 930)."""
         return (self.device.type == "cuda" and 0 < rows <= 16 * tiles
                 and rows * self.n_kv_heads <= 256)
 

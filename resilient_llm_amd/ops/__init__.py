@@ -369,7 +369,8 @@ def skinny_linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 
 
 def linear_auto(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
-    """rows_linear when the shape qualifies, else hipBLASLt via F.linear."""
+    """rows_linear for up to 64 rows, K % 256 == 0 and N % 64 == 0, whether it
+    is the faster one or not; else hipBLASLt via F.linear."""
     if (x.is_cuda and x.dim() == 2 and 1 <= x.shape[0] <= 64
             and x.shape[1] % 256 == 0 and w.shape[0] % 64 == 0):
         _gpu()

@@ -553,7 +553,9 @@ void launch_gla_decode(const GlaArgs& a, hipStream_t st) {
   // 1024 threads for states of 128 KB and more where each can have a CU of its
   // own (us with 256 threads and with 1024, heads of 128 x 256: 8 of them 8.6
   // and 6.8, 128 of them 10.7 and 9.0, 512 of them 24.1 and 26.5; of 128 x
-  // 128: 6.2 and 5.8, 7.2 and 6.9, 12.0 and 15.9; 256 of these 8.4 and 8.4)
+  // 128: 6.2 and 5.8, 7.2 and 6.9, 12.0 and 15.9; 256 of these 8.4 and 8.4).
+  // The readout sums rows in another order with them, so that its last bits
+  // depend on the batch.
   const bool wide = int64_t(a.dim) * a.vpad >= 128 * 256 &&
                     int64_t(a.rows) * a.heads <= 256;
   const int n_rows = (wide ? 1024 : 256) / (a.vpad / 4);

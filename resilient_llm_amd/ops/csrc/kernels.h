@@ -50,10 +50,11 @@ void launch_rope_kv_append(
 
 // Paged GQA decode attention, one new query per sequence.  Fused form
 // (positions given): q | k | v rows, or their f32 parts, are rotated and
-// appended as well (no slot_mapping: queries are rotated, nothing appended).  decode_attn_shares: equal shares of all sequences'
-// tokens that workgroups take per key/value head, 0: a workgroup takes a
-// whole sequence.  Then part_out [n_kv, shares + batch, group, head_dim]
-// and part_ml [.., group, 2] are needed.
+// appended as well (no slot_mapping: queries are rotated, nothing appended).
+// decode_attn_shares: equal shares of all sequences' tokens that workgroups
+// take per key/value head, for which part_out [n_kv, shares + batch, group,
+// head_dim] and part_ml [.., group, 2] are needed; 0: a workgroup takes a
+// whole sequence.
 int decode_attn_shares(int batch, int n_kv_heads, int max_tokens);
 void launch_decode_attn(
     const uint16_t* q,                 // [batch, q_stride], or null:
@@ -129,7 +130,7 @@ void launch_rows_short(const uint16_t* x, const uint16_t* w, uint16_t* out,
 void launch_sum_parts(const float* parts, uint16_t* out, int splits,
                       int64_t n, hipStream_t stream);
 
-// Diagnostic: pure nt-stream of W at skinny_gemm geometry.
+// Diagnostic: W streamed past the caches, 64 rows by a part of K per workgroup.
 void launch_stream_probe(const uint16_t* w, float* sink, int N, int K,
                          int splitk, hipStream_t stream);
 

@@ -476,10 +476,11 @@ DEV_INLINE void lds_load16(const void* g, void* l) {
 // device: the tiles there could be are up to one per expert more, and runs of
 // those left whole XCDs idle.  A run goes over four tiles' column blocks at a
 // time, so that what an XCD works on at once, about 32 blocks, shares eight
-// column blocks' weights and four tiles' rows in its L2 (hits 49 -> 78 % at
-// width 4096).  Whole calls, before -> now: 8192 rows of 4096, 16 experts of
-// 3584, two each: 1704 -> 1409 us; 2048 rows of them 788 -> 622; 6001 rows of
-// 2048, 32 experts of 1024, four each: 397 -> 385.
+// column blocks' weights and four tiles' rows in its L2 (hits at width 4096: 49
+// -> 77 % up, 62 -> 77 % down).  Whole calls, before -> now, us, three runs
+// each: 8192 rows of 4096, 16 experts of 3584, two each: 1658-1669 ->
+// 1389-1398; 2048 rows of them 753-783 -> 604-635; 6001 rows of 2048, 32
+// experts of 1024, four each: 397-407 -> 375-381 (on another card 404 -> 396).
 DEV_INLINE bool tile_of(const MoeArgs& a, int block, int n_blocks, int& tile,
                         int& nb) {
   const int x = block & 7;

@@ -290,7 +290,7 @@ void prefill_flash_kernel(Src src, uint16_t* __restrict__ out, int n_tiles,
     for (int r = 1; r < 16; ++r) mx = fmaxf(fmaxf(mx, s[0][r]), s[1][r]);
     mx = fmaxf(mx, __shfl_xor(mx, 32, kWave));
     // each query by itself, so that a row's result does not depend on the
-    // rows it shares a tile with
+    // rows it shares a tile with (only on the waves per head, see by_group)
     const bool grown = mx > m;
     if (__any(grown)) {
       const float mn = grown ? mx : m;
@@ -404,7 +404,9 @@ void prefill_flash_kernel(Src src, uint16_t* __restrict__ out, int n_tiles,
                 pack2(o[v][r + 2] * inv, o[v][r + 3] * inv)};
 }
 
-// ``keys``: as many as a sequence may have.
+// ``keys``: about how many a sequence has, as far as the host knows without
+// waiting for the device: the mean of a batch of prompts, the width of the
+// block table for pages.
 template <int D, int BS, typename Src>
 void by_group(const Src& src, uint16_t* out, int n_tiles, int n_kv, int group,
               int stride, float scale, int keys, hipStream_t st) {
@@ -431,7 +433,12 @@ void by_group(const Src& src, uint16_t* out, int n_tiles, int n_kv, int group,
   // with one wave per head and with two, 32/8 heads of 128: 512 rows behind
   // 1500 tokens 56.5 and 45.0, 1536 behind 1500 93 and 88; a prompt of 1000
   // 31.0 and 27.6, 1536 44.7 and 36.7, 384 15.4 and 15.0, 128 9.7 and 10.7;
-  // 4 of 512 28.0 and 31.1)
+  // 4 of 512 28.0 and 31.1).  Neither count is that of a ragged batch's longest
+  // sequence: 1000 rows and 4 of 100, mean 280, take one wave, 28.1, and would
+  // 24.2 with two, but 4000 rows and 20 of 30, mean 219, 160 and 174; 128 rows
+  // of pages in a table for 8192 take two, 9.1, and would 8.3 with one.  The
+  // two forms sum keys in different order, so that the last bits of a row's
+  // result depend on the batch.
   else if (n_tiles * n_kv * (group / 4) <= 400 && keys >= 384)
     go(I4{}, I2{});
   else go(I4{}, I1{});

@@ -429,8 +429,10 @@ int rows_gemm_splits(int N, int K) {
   return std::min(n, K / KS);
 }
 
-// Rings of about 72 KB (whole 64-row steps of x) to 80 KB: one workgroup per
-// CU keeps enough under way, two fit where there are more.  Panels of 128
+// Rings with up to 32, 64 and 128 rows of x: parts 72, 80 and 120 KB, whole
+// panels of 64 (and 32 pairs with silu) 72, 80 and 72, of 128 60, 72 and 128, of
+// 64 pairs 100, 120 and 128.  One workgroup per CU keeps enough under way; two
+// share its 160 KB where rings are of 80 or less.  Panels of 128
 // halve what x costs and are taken where they still cover the CUs (128256
 // rows of 4096: 155 us against 158 for one row, 177 against 207 for 64).
 void launch_rows_gemm(const uint16_t* x, const uint16_t* w, float* parts,

@@ -1,8 +1,8 @@
 // Microbench kernel: pure nontemporal streaming read of an [N, K] bf16
-// weight matrix with the EXACT grid/wave geometry of skinny_gemm
-// (BN=64 panels x splitk, 4 waves, B-fragment addressing) — establishes
-// the per-shape streaming ceiling the GEMM could reach if compute and
-// staging were free.  Diagnostic only; not part of the serving path.
+// weight matrix (64-row panels x splitk, 4 waves, each lane in the rows
+// that a matrix operand takes) — what a product that reads its operands
+// straight into registers could reach per shape if compute were free.
+// Diagnostic only; not part of the serving path.
 #include "common.h"
 
 namespace rlli {

@@ -1,5 +1,5 @@
 #!/usr/bin/env python3
-"""Within-process A/B: skinny_linear vs hipBLASLt on the decode shapes."""
+"""Within-process A/B: rows_linear vs hipBLASLt on the decode shapes."""
 import sys, os, time
 sys.path.insert(0, os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
 import torch
@@ -21,7 +21,7 @@ def timeit(fn, iters=50):
 
 def probe():
     ops.load_extension(required=True)
-    print("— pure nt-stream ceiling at skinny geometry —")
+    print("— pure nt-stream of the weights —")
     for name, M, N, K in SHAPES:
         w = torch.randn(N, K, dtype=torch.bfloat16, device="cuda")
         gb = N * K * 2 / 1e9
@@ -40,11 +40,11 @@ def main():
         w = torch.randn(N, K, dtype=torch.bfloat16, device="cuda")
         gb = N * K * 2 / 1e9
         t_b = timeit(lambda: torch.nn.functional.linear(x, w))
-        t_s = timeit(lambda: ops.skinny_linear(x, w))
+        t_s = timeit(lambda: ops.rows_linear(x, w))
         tot_s += t_s; tot_b += t_b
         print(f"{name:8s} M{M} N{N} K{K}: blaslt {t_b:7.1f} us ({gb/t_b*1e6/1e3:5.2f} TB/s)"
-              f"  skinny {t_s:7.1f} us ({gb/t_s*1e6/1e3:5.2f} TB/s)  x{t_b/t_s:.2f}")
-    print(f"TOTAL: blaslt {tot_b:.0f} us, skinny {tot_s:.0f} us, x{tot_b/tot_s:.2f}")
+              f"  rows {t_s:7.1f} us ({gb/t_s*1e6/1e3:5.2f} TB/s)  x{t_b/t_s:.2f}")
+    print(f"TOTAL: blaslt {tot_b:.0f} us, rows {tot_s:.0f} us, x{tot_b/tot_s:.2f}")
 
 if __name__ == "__main__":
     main()

@@ -1,11 +1,11 @@
 #!/usr/bin/env python3
-"""A/B the v2 skinny GEMM against hipBLASLt (F.linear) and the r01 kernel
-on the Llama-3-8B decode shapes, plus the fused-SiLU down-proj against
-silu_mul + F.linear.  Correctness-checks every config against fp32
-matmul first; timing is 200 reps between cuda events, L2-cold by
-construction (weights >> 32 MB L2 stream every reps).
+"""A/B the products of few rows, whole and in parts for a reader that sums,
+against hipBLASLt (F.linear) on the Llama-3-8B decode shapes, plus gate and up
+with silu in the epilogue against F.linear + silu_mul.  Correctness-checks
+every form against fp32 matmul first; timing is 200 reps between cuda events,
+L2-cold by construction (weights >> 32 MB L2 stream every reps).
 
-Usage (GPU box):  python scripts/bench_skinny2.py [--m 64] [--sk 1 2 4 8]
+Usage:  python scripts/bench_skinny2.py [--m 64] [--copies 8]
 """
 
 import argparse
@@ -50,14 +50,13 @@ def check(a, b, tag, tol=2e-2):
 def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--m", type=int, nargs="*", default=[64])
-    ap.add_argument("--sk", type=int, nargs="*", default=[1, 2, 4, 8])
     ap.add_argument("--reps", type=int, default=200)
     ap.add_argument("--copies", type=int, default=1,
                     help="cycle this many weight copies per shape: >1 "
                          "defeats the 256 MB LLC, reproducing the REAL "
-                         "decode regime (r02 finding: isolated timings "
-                         "are L3-warm — hipBLASLt measured 20 us isolated "
-                         "vs 48 us in the decode stream)")
+                         "decode regime (isolated timings are L3-warm — "
+                         "hipBLASLt measured 20 us isolated vs 48 us in "
+                         "the decode stream)")
     args = ap.parse_args()
     ops.load_extension(required=True)
     dev = "cuda:0"
@@ -85,47 +84,35 @@ def main():
                           args.reps)
             row = [f"{name:8s} lt={t_lt:7.1f}us"]
             best = (t_lt, "lt")
-            for sk in args.sk:
-                if sk > K // 256:
-                    continue
-                out = ops.skinny2_linear(x, w, sk)
-                check(out, ref, f"{name} sk{sk}")
-                t = timeit(lambda: ops.skinny2_linear(x, next_w(), sk),
-                           args.reps)
-                row.append(f"sk{sk}={t:7.1f}")
+            for form, fn in (("whole", ops.rows_linear),
+                             ("parts", ops.rows_linear_parts)):
+                out = fn(x, w)
+                check(out.sum(0) if out.dim() == 3 else out, ref,
+                      f"{name} {form}")
+                t = timeit(lambda: fn(x, next_w()), args.reps)
+                row.append(f"{form}={t:7.1f}")
                 if t < best[0]:
-                    best = (t, f"sk{sk}")
+                    best = (t, form)
             print(" ".join(row) + f"   best={best[1]} "
                   f"({t_lt / best[0]:.2f}x vs lt)", flush=True)
 
-        # fused SwiGLU down-proj: vs silu_mul + F.linear
-        I = 14336
-        gu = torch.randn(M, 2 * I, device=dev, dtype=torch.bfloat16) * 0.3
-        next_wd = cycler(lambda: torch.randn(
-            4096, I, device=dev, dtype=torch.bfloat16) * 0.02)
-        wd = next_wd()
-        gf, uf = gu.float().chunk(2, -1)
-        ref = (torch.nn.functional.silu(gf) * uf) @ wd.float().t()
+        # gate and up with silu in the epilogue: vs F.linear + silu_mul
+        N, K = SHAPES[2][1:]
+        x = torch.randn(M, K, device=dev, dtype=torch.bfloat16) * 0.3
+        next_w = cycler(lambda: torch.randn(
+            N, K, device=dev, dtype=torch.bfloat16) * 0.02)
+        w = next_w()
+        g, u = (x.float() @ w.float().t()).chunk(2, -1)
+        ref = torch.nn.functional.silu(g) * u
 
-        def eager():
-            return torch.nn.functional.linear(ops.silu_mul(gu), next_wd())
-        check(torch.nn.functional.linear(ops.silu_mul(gu), wd), ref,
-              "down eager", tol=3e-2)
-        t_e = timeit(eager, args.reps)
-        row = [f"down+silu eager={t_e:7.1f}us"]
-        best = (t_e, "eager")
-        for sk in args.sk:
-            if sk > I // 256:
-                continue
-            out = ops.skinny2_silu_linear(gu, wd, sk)
-            check(out, ref, f"down fused sk{sk}", tol=3e-2)
-            t = timeit(lambda: ops.skinny2_silu_linear(gu, next_wd(), sk),
-                       args.reps)
-            row.append(f"fused-sk{sk}={t:7.1f}")
-            if t < best[0]:
-                best = (t, f"fused-sk{sk}")
-        print(" ".join(row) + f"   best={best[1]} "
-              f"({t_e / best[0]:.2f}x vs eager)", flush=True)
+        def eager(w):
+            return ops.silu_mul(torch.nn.functional.linear(x, w))
+        check(eager(w), ref, "gate_up eager", tol=3e-2)
+        check(ops.rows_linear_silu(x, w), ref, "gate_up fused", tol=3e-2)
+        t_e = timeit(lambda: eager(next_w()), args.reps)
+        t = timeit(lambda: ops.rows_linear_silu(x, next_w()), args.reps)
+        print(f"gate_up+silu eager={t_e:7.1f}us fused={t:7.1f}   "
+              f"({t_e / t:.2f}x vs eager)", flush=True)
 
 
 if __name__ == "__main__":

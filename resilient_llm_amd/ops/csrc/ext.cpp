@@ -570,6 +570,7 @@ Tensor prefill_paged_attn(const Tensor& qkv, const Tensor& k_cache,
 static void check_rows(const Tensor& x, const Tensor& w) {
   check_bf16_contig(x, "x");
   check_bf16_contig(w, "w");
+  TORCH_CHECK(x.device() == w.device(), "x and W on one GPU");
   TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && w.size(1) == x.size(1),
               "x/W K mismatch");
   TORCH_CHECK(x.size(0) >= 1 && x.size(0) <= 128, "1 to 128 rows, got ",

@@ -136,3 +136,9 @@ def test_rows_that_fit_are_the_faster_ones(M, N, K, fits):
     x = torch.empty(M, K, dtype=torch.bfloat16, device=DEV)
     assert ops.rows_fit(x, torch.empty(N, K, dtype=torch.bfloat16,
                                        device=DEV)) == fits
+
+
+def test_weights_elsewhere_are_refused():
+    x, w = operands(64, 128)
+    with pytest.raises(RuntimeError):
+        ops.rows_linear(x, w.cpu())

@@ -141,7 +141,8 @@ DEV_INLINE void lds_barrier() {
 
 // the sum of the parts in a head's columns, HS apart; the same bits in each.
 // (Of up to four heads, second and third part first: they are eight columns
-// apart, and so are the first and a column of zeros.)
+// apart, and so are the first and the idle column, where a query's part is the
+// least number.)
 template <int HS>
 DEV_INLINE float sum_parts(float v) {
   v += dpp_mov_f32<0x128>(v);
@@ -216,7 +217,10 @@ void decode_attn_kernel(DecodeArgs a) {
   constexpr int QROW = D + 8;
   constexpr int HS = GROUP <= 4 ? 4 : 8;   // columns of a part
   __shared__ __attribute__((aligned(16))) float raw[(GROUP + 2) * D];
-  __shared__ __attribute__((aligned(16))) uint16_t qs[(HS == 4 ? 16 : 24) * QROW];
+  // queries by part and head: of up to four heads as the columns have them,
+  // of eight first (halved), second, third part
+  constexpr int QROWS = HS == 4 ? 16 : 24;
+  __shared__ __attribute__((aligned(16))) uint16_t qs[QROWS * QROW];
   __shared__ __attribute__((aligned(16))) elem self[2 * D];       // k | v
   __shared__ __attribute__((aligned(16))) float accs[4 * GROUP * D];
   __shared__ float ml[4 * GROUP * 2];
@@ -690,7 +694,8 @@ void run(const DecodeArgs& a, hipStream_t st) {
     constexpr int BS = decltype(bs)::value;
     if (a.shares > 0) {
       hipLaunchKernelGGL((decode_attn_kernel<D, GROUP, KC, BS, FUSED, true>),
-                         dim3((a.shares + a.batch) * a.n_kv), dim3(256), 0, st, a);
+                         dim3((a.shares + a.batch) * a.n_kv), dim3(256), 0, st,
+                         a);
       hipLaunchKernelGGL((decode_combine_kernel<D, GROUP>),
                          dim3(a.batch * a.n_kv * GROUP), dim3(256), 0, st, a);
     } else {

@@ -76,6 +76,17 @@ def _linear_relu2(x, w):
     return ops.relu2(_linear(x, w))
 
 
+def _norm_linear(x, residual, gain, eps, w, linear):
+    """x + residual, normed, through ``linear`` with w: the result and the new
+    residual.  Of one row the norm is made inside the product."""
+    silu = linear is _linear_silu
+    if ((silu and w.shape[0] % 16 == 0 or linear is _linear_parts)
+            and not _USE_SKINNY and not lt_autotune.enabled()
+            and ops.rows_norm_fit(x, residual, w, silu)):
+        return ops.rows_norm_linear(x, residual, gain, eps, w, silu)
+    return linear(ops.rmsnorm_residual_(x, residual, gain, eps), w), residual
+
+
 @dataclasses.dataclass
 class LlamaConfig:
     name: str
@@ -377,12 +388,14 @@ class LlamaForCausalLM:
         # nothing has to be done with their sum before
         out = (_linear_parts if self.tp_world == 1 and self.quant is None
                and c.hidden_size <= 8192 else _linear)
+        to_qkv = _linear_parts if qkv_parts else _linear
         if residual is None:
             residual = x.clone()
             h = ops.rmsnorm(x, p[f"l{i}.ln1"], c.rms_eps)
+            qkv = to_qkv(h, p[f"l{i}.qkv"])
         else:
-            h = ops.rmsnorm_residual_(x, residual, p[f"l{i}.ln1"], c.rms_eps)
-        qkv = (_linear_parts if qkv_parts else _linear)(h, p[f"l{i}.qkv"])
+            qkv, residual = _norm_linear(x, residual, p[f"l{i}.ln1"],
+                                         c.rms_eps, p[f"l{i}.qkv"], to_qkv)
         k_cache, v_cache = kv_cache.layer(i)
         # rope + cache append happen inside attn_fn (the decode path fuses
         # them into the attention kernel itself)
@@ -395,8 +408,8 @@ class LlamaForCausalLM:
             dq, ds = ops.silu_mul_fp8(gu)
             mlp = self._all_reduce(self._linear_fp8(dq, ds, f"l{i}.down"))
             return mlp, residual
-        h2 = ops.rmsnorm_residual_(h, residual, p[f"l{i}.ln2"], c.rms_eps)
-        act = _linear_silu(h2, p[f"l{i}.gate_up"])
+        act, residual = _norm_linear(h, residual, p[f"l{i}.ln2"], c.rms_eps,
+                                     p[f"l{i}.gate_up"], _linear_silu)
         mlp = self._all_reduce(out(act, p[f"l{i}.down"]))
         return mlp, residual
 

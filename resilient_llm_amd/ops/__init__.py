@@ -347,6 +347,26 @@ def rows_linear_silu(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     return silu_mul(torch.nn.functional.linear(x, w))
 
 
+def rows_norm_fit(parts: torch.Tensor, residual: torch.Tensor,
+                  w: torch.Tensor, silu: bool) -> bool:
+    """Whether rows_norm_linear takes these."""
+    if parts.dim() != 3 or parts.dtype != torch.float32 \
+            or parts.shape[1] != 1 or not rows_fit(residual, w):
+        return False
+    _gpu()
+    return torch.ops.rlli.rows_norm_ok(*w.shape, silu)
+
+
+def rows_norm_linear(parts: torch.Tensor, residual: torch.Tensor,
+                     gain: torch.Tensor, eps: float, w: torch.Tensor,
+                     silu: bool) -> tuple[torch.Tensor, torch.Tensor]:
+    """Of one row: rmsnorm_residual_ of rows_linear_parts's result and
+    rows_linear_parts or rows_linear_silu of that, in one launch; the product
+    and the new residual (``residual`` stays as it is)."""
+    _gpu()
+    return torch.ops.rlli.rows_norm_linear(parts, residual, gain, eps, w, silu)
+
+
 def rows_whole(x: torch.Tensor, w: torch.Tensor) -> bool:
     """For x and w that rows_fit: whether rows_linear takes them without
     dividing K over workgroups; rows_linear_relu2 is for these."""

@@ -656,6 +656,54 @@ Tensor rows_linear_silu(const Tensor& x, const Tensor& w) {
   return out;
 }
 
+bool rows_norm_ok(int64_t N, int64_t K, bool silu) {
+  return N <= 1 << 20 && K <= 8192 &&
+         rlli::rows_norm_ok(int(N), int(K), silu);
+}
+
+// Of one row: rows_linear_parts or (silu) rows_linear_silu of the rmsnorm of
+// residual + the sum of parts [n, 1, K], in one launch; and the new residual.
+std::tuple<Tensor, Tensor> rows_norm_linear(const Tensor& parts,
+                                            const Tensor& residual,
+                                            const Tensor& gain, double eps,
+                                            const Tensor& w, bool silu) {
+  check_rows(residual, w);
+  check_bf16_contig(gain, "gain");
+  const int K = int(residual.size(1)), N = int(w.size(0));
+  TORCH_CHECK(residual.size(0) == 1 && rows_norm_ok(N, K, silu) &&
+                  (!silu || N % 16 == 0),
+              "one row; rows_norm_ok says which products these are");
+  TORCH_CHECK(parts.scalar_type() == at::kFloat && parts.is_contiguous() &&
+                  parts.device() == residual.device() && parts.dim() == 3 &&
+                  parts.size(0) >= 1 && parts.size(1) == 1 &&
+                  parts.size(2) == K,
+              "parts: f32 [n, 1, K]");
+  TORCH_CHECK(gain.numel() == K && gain.device() == residual.device(),
+              "a gain of K");
+  for (const Tensor* t : {&parts, &gain})
+    TORCH_CHECK(reinterpret_cast<uintptr_t>(t->data_ptr()) % 16 == 0,
+                "parts and gain start at multiples of 16 bytes");
+  c10::hip::HIPGuardMasqueradingAsCUDA guard(residual.device());
+  const hipStream_t st = current_stream(residual);
+  Tensor after = at::empty_like(residual);
+  const rlli::RowsNorm norm{parts.data_ptr<float>(), bf16_ptr(residual),
+                            bf16_ptr(after), bf16_ptr(gain),
+                            int(parts.size(0)), float(eps)};
+  Tensor out;
+  if (silu) {
+    out = at::empty({1, N / 2}, residual.options());
+    rlli::launch_rows_norm_silu(norm, bf16_ptr(w), bf16_ptr(out), N / 2, K,
+                                st);
+  } else {
+    const int splits = rlli::rows_gemm_splits(N, K);
+    out = at::empty({splits, 1, N}, parts.options());
+    rlli::launch_rows_norm(norm, bf16_ptr(w), out.data_ptr<float>(), N, K,
+                           splits, st);
+  }
+  check_launch("rows_norm_linear");
+  return {out, after};
+}
+
 // The same under the names and limits of earlier kernels; ``splitk`` has no
 // effect any more.
 static void check_skinny(const char* op, const Tensor& x, const Tensor& w,
@@ -774,6 +822,10 @@ TORCH_LIBRARY(rlli, m) {
   m.def("rows_linear_silu(Tensor x, Tensor w) -> Tensor");
   m.def("rows_linear_relu2(Tensor x, Tensor w) -> Tensor");
   m.def("rows_whole_ok(int m, int n, int k) -> bool", &rows_whole_ok);
+  m.def("rows_norm_ok(int n, int k, bool silu) -> bool",
+        &rows_norm_ok);
+  m.def("rows_norm_linear(Tensor parts, Tensor residual, Tensor gain, "
+        "float eps, Tensor w, bool silu) -> (Tensor, Tensor)");
   m.def("skinny_linear(Tensor x, Tensor w) -> Tensor");
   m.def("skinny2_linear(Tensor x, Tensor w, int splitk) -> Tensor");
   m.def("skinny2_silu_linear(Tensor gu, Tensor w, int splitk) -> Tensor");
@@ -807,6 +859,7 @@ TORCH_LIBRARY_IMPL(rlli, CUDA, m) {
   m.impl("rows_linear", &rows_linear);
   m.impl("rows_linear_silu", &rows_linear_silu);
   m.impl("rows_linear_relu2", &rows_linear_relu2);
+  m.impl("rows_norm_linear", &rows_norm_linear);
   m.impl("skinny_linear", &skinny_linear);
   m.impl("skinny2_linear", &skinny2_linear);
   m.impl("skinny2_silu_linear", &skinny2_silu_linear);

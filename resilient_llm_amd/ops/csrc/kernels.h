@@ -123,6 +123,22 @@ bool rows_gemm_silu_ok(int inter);
 void launch_rows_gemm_silu(const uint16_t* x, const uint16_t* w,
                            uint16_t* out, int M, int inter, int K,
                            hipStream_t stream);
+// The same two for one row, the norm of residual + the sum of n parts [n, K],
+// which goes to residual_out, where rows_norm_ok.
+struct RowsNorm {
+  const float* parts;
+  const uint16_t* residual;
+  uint16_t* residual_out;
+  const uint16_t* gain;
+  int n;
+  float eps;
+};
+bool rows_norm_ok(int N, int K, bool silu);
+void launch_rows_norm(const RowsNorm& norm, const uint16_t* w, float* parts,
+                      int N, int K, int splits, hipStream_t stream);
+void launch_rows_norm_silu(const RowsNorm& norm, const uint16_t* w,
+                           uint16_t* out, int inter, int K,
+                           hipStream_t stream);
 // M <= 64 where rows_short_tiles is not 0; ``relu2``: squared positive part
 int rows_short_tiles(int N, int K);
 void launch_rows_short(const uint16_t* x, const uint16_t* w, uint16_t* out,

@@ -22,6 +22,7 @@
 // follows from N and K alone.
 
 #include "common.h"
+#include "kernels.h"
 
 #include <algorithm>
 #include <type_traits>
@@ -68,14 +69,124 @@ DEV_INLINE void wait_steps(int left) {
   }
 }
 
+// ---- the norm ahead of a product ----------------------------------------
+// Of a single row, what a norm reads is so little that every workgroup of the
+// product behind it can make x for itself: the residual plus the sum of an
+// earlier product's f32 parts, normed, in LDS, by four more waves while the
+// others' first steps of w are under way.  What bounds it is the time to that
+// read's data.  us, norm and product apart and in one: 6144 x 4096 parts 4.5 +
+// 9.6 and 11.6, 28672 x 4096 with silu 4.5 + 35.8 and 37.1, 3072 x 2048 4.5 +
+// 4.8 and 6.0, 16384 x 2048 with silu 4.5 + 12.4 and 13.7.  (Two rows read
+// twice as much: 2 us slower than apart.  Rows made once and handed to the
+// other workgroups through memory: 2 us slower as well, five trips to memory
+// while it is busy with weights.)
+struct NormArgs {
+  const float* parts;          // [n, K]
+  const uint16_t* residual;    // [K]
+  uint16_t* residual_out;      // residual + sum of the parts
+  const uint16_t* gain;        // [K]
+  int n;
+  float eps;
+};
+
+// loads into LDS stay under way
+DEV_INLINE void lds_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+// The row by 256 threads, NCH pieces of 8 elements each.  All of the
+// workgroup's waves pass two barriers: behind the first, what is read here has
+// been asked for, ahead of the weights, behind which it would wait for 1 to 3
+// us more.
+template <int NCH>
+DEV_INLINE void norm_row(const NormArgs& a, int K, int t, float* sums,
+                         uint16_t* xs) {
+  constexpr int B = 8 / NCH;              // parts whose loads are one batch
+  uint4 r[NCH], gain[NCH];
+  float4 first[B][NCH][2];
+  float v[NCH][8];
+  int at[NCH];
+#pragma unroll
+  for (int c = 0; c < NCH; ++c) at[c] = min((c * 256 + t) * 8, K - 8);
+#pragma unroll
+  for (int s = 0; s < B; ++s)
+    if (s < a.n)
+#pragma unroll
+      for (int c = 0; c < NCH; ++c)
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+          first[s][c][i] = *reinterpret_cast<const float4*>(
+              a.parts + int64_t(s) * K + at[c] + i * 4);
+#pragma unroll
+  for (int c = 0; c < NCH; ++c) {
+    r[c] = *reinterpret_cast<const uint4*>(a.residual + at[c]);
+    gain[c] = *reinterpret_cast<const uint4*>(a.gain + at[c]);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[c][i] = 0.f;
+  }
+  lds_barrier();
+  auto add = [&](int c, const float4& x, const float4& y) {
+    v[c][0] += x.x; v[c][1] += x.y; v[c][2] += x.z; v[c][3] += x.w;
+    v[c][4] += y.x; v[c][5] += y.y; v[c][6] += y.z; v[c][7] += y.w;
+  };
+#pragma unroll
+  for (int s = 0; s < B; ++s)
+    if (s < a.n)
+#pragma unroll
+      for (int c = 0; c < NCH; ++c) add(c, first[s][c][0], first[s][c][1]);
+#pragma unroll(B)
+  for (int s = B; s < a.n; ++s)
+#pragma unroll
+    for (int c = 0; c < NCH; ++c) {
+      const float* q = a.parts + int64_t(s) * K + at[c];
+      add(c, *reinterpret_cast<const float4*>(q),
+          *reinterpret_cast<const float4*>(q + 4));
+    }
+  float ss = 0.f;
+#pragma unroll
+  for (int c = 0; c < NCH; ++c) {
+    bf16x8 o;
+    o.u = r[c];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      o.s[i] = f32_to_bf16(v[c][i] + bf16_to_f32(o.s[i]));
+      const float f = bf16_to_f32(o.s[i]);    // x is of the stored residual
+      if ((c * 256 + t) * 8 < K) ss += f * f;
+    }
+    r[c] = o.u;
+  }
+  ss = wave_sum(ss);
+  if ((t & 63) == 0) sums[t >> 6] = ss;
+  lds_barrier();
+  ss = sums[0] + sums[1] + sums[2] + sums[3];
+  const float inv = rsqrtf(ss / K + a.eps);
+#pragma unroll
+  for (int c = 0; c < NCH; ++c) {
+    const int d = (c * 256 + t) * 8;
+    if (d >= K) continue;
+    if (blockIdx.x == 0)
+      *reinterpret_cast<uint4*>(a.residual_out + d) = r[c];
+    bf16x8 o, g;
+    o.u = r[c];
+    g.u = gain[c];
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      o.s[i] = f32_to_bf16(bf16_to_f32(o.s[i]) * inv * bf16_to_f32(g.s[i]));
+    *reinterpret_cast<uint4*>(xs + d) = o.u;
+  }
+}
+
 // CT: 16-row tiles of w per wave; XR: rows of x that are staged; MT: 16-row
 // tiles of x; R: steps in the ring.  OUT_SILU: a wave's first tile is of the
 // gate's rows, the second the same rows of the upper half of w.
-template <int CT, int XR, int MT, int R, int OUT>
-__global__ __launch_bounds__(256)
+// NORM: of one row x, made here (XR 0); all of it stays in LDS, behind the ring.
+template <int CT, int XR, int MT, int R, int OUT, bool NORM = false>
+__global__ __launch_bounds__(NORM ? 512 : 256)
 void rows_gemm_kernel(const uint16_t* __restrict__ x,
                       const uint16_t* __restrict__ w, void* __restrict__ out,
-                      int M, int N, int K, int splits) {
+                      int M, int N, int K, int splits, NormArgs norm) {
   constexpr int WPART = 4 * CT * 16 * LINE;          // elements of a step
   constexpr int STEP = WPART + XR * LINE;
   constexpr int L = CT * 2 + XR / 32;                // loads of a wave
@@ -88,6 +199,19 @@ void rows_gemm_kernel(const uint16_t* __restrict__ x,
   const int lane = threadIdx.x & 63;
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int half = N / 2;
+  uint16_t* xs = lds + R * STEP;
+  if constexpr (NORM) {
+    if (wv >= 4) {
+      // (the ring's last step is not asked for before the second barrier)
+      float* sums = reinterpret_cast<float*>(lds + (R - 1) * STEP);
+      const int t = threadIdx.x - 256;
+      if (K <= 2048) norm_row<1>(norm, K, t, sums, xs);
+      else if (K <= 4096) norm_row<2>(norm, K, t, sums, xs);
+      else norm_row<4>(norm, K, t, sums, xs);
+      lds_barrier();
+      return;
+    }
+  }
   // where this workgroup starts within its steps
   const int rot = int(blockIdx.x / 8 % unsigned(n));
 
@@ -101,7 +225,7 @@ void rows_gemm_kernel(const uint16_t* __restrict__ x,
   // a load takes 8 rows, a lane the piece of row lane / 8 that belongs in
   // slot lane % 8
   const int lr = lane >> 3;
-  const uint16_t *wp[CT * 2], *xp[XR / 32];
+  const uint16_t *wp[CT * 2], *xp[XR / 32 + 1];
 #pragma unroll
   for (int j = 0; j < CT * 2; ++j) {
     const int r = (j & 1) * 8 + lr;
@@ -140,9 +264,15 @@ void rows_gemm_kernel(const uint16_t* __restrict__ x,
 
   const int tr = lane & 15, oct = lane >> 4;
   const int sw = tr >> 1;
+  if constexpr (NORM) lds_barrier();
 #pragma unroll
   for (int s = 0; s < R - 1; ++s)
     if (s < n) issue(s, s);
+  if constexpr (NORM) {
+    lds_barrier();
+    lds_barrier();
+  }
+  const uint16_t* own = xs + int64_t(s0) * KS + oct * 8;
   int slot = 0;
   for (int s = 0; s < n; ++s) {
     // this wave's loads of the step have landed, then everybody's; nobody
@@ -155,6 +285,7 @@ void rows_gemm_kernel(const uint16_t* __restrict__ x,
     slot = slot == R - 1 ? 0 : slot + 1;
     const uint16_t* wt = at + wv * CT * 16 * LINE + tr * LINE;
     const uint16_t* xt = at + WPART + tr * LINE;
+    const uint16_t* xo = own + (s + rot < n ? s + rot : s + rot - n) * KS;
     s16x8 a[2][CT], b[2][MT];
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
@@ -164,7 +295,8 @@ void rows_gemm_kernel(const uint16_t* __restrict__ x,
         a[k][t] = *reinterpret_cast<const s16x8*>(wt + t * 16 * LINE + piece);
 #pragma unroll
       for (int m = 0; m < MT; ++m)
-        b[k][m] = *reinterpret_cast<const s16x8*>(xt + m * 16 * LINE + piece);
+        b[k][m] = *reinterpret_cast<const s16x8*>(
+            NORM ? xo + k * 32 : xt + m * 16 * LINE + piece);
     }
 #pragma unroll
     for (int k = 0; k < 2; ++k)
@@ -377,7 +509,7 @@ void go(const uint16_t* x, const uint16_t* w, void* out, int M, int N, int K,
                                 hipFuncAttributeMaxDynamicSharedMemorySize,
                                 int(smem));
     hipLaunchKernelGGL(k, dim3(panels * splits), dim3(256), smem, st, x, w,
-                       out, M, N, K, splits);
+                       out, M, N, K, splits, NormArgs{});
   };
   using I1 = std::integral_constant<int, 1>;
   using I2 = std::integral_constant<int, 2>;
@@ -394,6 +526,21 @@ void go(const uint16_t* x, const uint16_t* w, void* out, int M, int N, int K,
   else if (M <= 64) run(X64{}, I4{});
   else if (M <= 96) run(X128{}, I6{});
   else run(X128{}, I8{});
+}
+
+template <int CT, int R, int OUT>
+void go_norm(const RowsNorm& norm, const uint16_t* w, void* out, int N, int K,
+             int panels, int splits, hipStream_t st) {
+  const size_t smem = (size_t(R) * 4 * CT * 16 * LINE + size_t(K)) * 2;
+  auto* k = rows_gemm_kernel<CT, 0, 1, R, OUT, true>;
+  if (smem > 65536)
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(k),
+                              hipFuncAttributeMaxDynamicSharedMemorySize,
+                              int(smem));
+  hipLaunchKernelGGL(k, dim3(panels * splits), dim3(512), smem, st, nullptr, w,
+                     out, 1, N, K, splits,
+                     NormArgs{norm.parts, norm.residual, norm.residual_out,
+                              norm.gain, norm.n, norm.eps});
 }
 
 template <int PT, int R16, int R32, int R64, bool RELU2>
@@ -460,6 +607,30 @@ void launch_rows_gemm_silu(const uint16_t* x, const uint16_t* w,
   else
     go<1, 6, 5, 3, OUT_SILU>(x, w, out, M, 2 * inter, K, (inter + 31) / 32, 1,
                           st);
+}
+
+// Whether a product of one row makes it from a residual by itself: with no more
+// workgroups than CUs, as each makes all of it.
+bool rows_norm_ok(int N, int K, bool silu) {
+  if (K > 8192) return false;
+  if (silu) return rows_gemm_silu_ok(N / 2) && (N / 2 + 63) / 64 <= 256;
+  return (N + 63) / 64 <= 256 && rows_gemm_splits(N, K) > 1;
+}
+
+// Rings of 80 KB and up to 16 KB of x.
+void launch_rows_norm(const RowsNorm& norm, const uint16_t* w, float* parts,
+                      int N, int K, int splits, hipStream_t st) {
+  go_norm<1, 10, OUT_PARTS>(norm, w, parts, N, K, (N + 63) / 64, splits, st);
+}
+
+void launch_rows_norm_silu(const RowsNorm& norm, const uint16_t* w,
+                           uint16_t* out, int inter, int K, hipStream_t st) {
+  if ((inter + 63) / 64 >= 200)
+    go_norm<2, 5, OUT_SILU>(norm, w, out, 2 * inter, K, (inter + 63) / 64, 1,
+                            st);
+  else
+    go_norm<1, 10, OUT_SILU>(norm, w, out, 2 * inter, K, (inter + 31) / 32, 1,
+                             st);
 }
 
 // Tiles of 16 rows per workgroup of the products that rows_short_kernel takes,

@@ -55,16 +55,21 @@ def _linear(x, w):
 
 def _linear_silu(x, w):
     """silu_mul of _linear."""
-    if (not _USE_SKINNY and not lt_autotune.enabled() and ops.rows_fit(x, w)
-            and w.shape[0] % 16 == 0):
-        return ops.rows_linear_silu(x, w)
+    if not _USE_SKINNY and not lt_autotune.enabled():
+        if w.shape[0] % 16 == 0 and ops.rows_fit(x, w):
+            return ops.rows_linear_silu(x, w)
+        if ops.tile_silu_fit(x, w):
+            return ops.tile_linear_silu(x, w)
     return ops.silu_mul(_linear(x, w))
 
 
 def _linear_parts(x, w):
     """_linear for a reader that sums parts (ops.rows_linear_parts)."""
-    if (not _USE_SKINNY and not lt_autotune.enabled() and ops.rows_fit(x, w)):
-        return ops.rows_linear_parts(x, w)
+    if not _USE_SKINNY and not lt_autotune.enabled():
+        if ops.tile_parts_fit(x, w):
+            return ops.tile_linear_parts(x, w)
+        if ops.rows_fit(x, w):
+            return ops.rows_linear_parts(x, w)
     return _linear(x, w)
 
 

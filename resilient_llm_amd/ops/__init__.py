@@ -380,6 +380,56 @@ def rows_linear_relu2(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     return torch.ops.rlli.rows_linear_relu2(x, w)
 
 
+def _tiles_take(x: torch.Tensor, w: torch.Tensor) -> bool:
+    return (x.dtype == w.dtype == torch.bfloat16 and x.shape[1] % 64 == 0
+            and w.shape[0] % 16 == 0
+            and x.is_contiguous() and w.is_contiguous()
+            and x.numel() < 1 << 31 and w.numel() < 1 << 31
+            and (x.data_ptr() | w.data_ptr()) % 16 == 0
+            and not (x.requires_grad or w.requires_grad))
+
+
+def tile_parts_fit(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether tile_linear_parts takes x w^T and is the faster way, the pass
+    that sums the parts included.  Divided, K keeps all CUs busy where the
+    library leaves some idle; parts cost the more the shorter K is.  (us with
+    the norm behind it, the other way first, the library from 129 rows on: 4096
+    x 14336, 65 rows 36 and 31, 160 89 and 41, 536 118 and 72, 1000 145 and
+    109, 2048 233 and 209, but 3072 297 and 299; 2048 x 8192, 128 rows 20 and
+    17, 536 43 and 32, 1300 61 and 55, 1536 60 and 62; 4096 x 4096, 65 rows 17
+    and 15.5, 128 21 and 19, but 256 23 and 25, 700 36 and 40; 2048 x 2048, 128
+    rows 12 and 14.)"""
+    if x.dim() != 2 or not x.is_cuda:
+        return False
+    (M, K), N = x.shape, w.shape[0]
+    return (64 < M <= (2048 if K >= 12288 else 1280 if K >= 6144 else 128)
+            and K >= 4096 and 1024 <= N <= 8192 and _tiles_take(x, w))
+
+
+def tile_linear_parts(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """rows_linear_parts for more rows."""
+    _gpu()
+    return torch.ops.rlli.tile_linear_parts(x, w)
+
+
+def tile_silu_fit(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether tile_linear_silu takes x w^T and is faster than the library and
+    silu_mul.  (us, those first: 28672 x 4096, 160 rows 64 and 68, 192 66 and
+    62, 536 147 and 113, 1024 222 and 190, 2048 416 and 383, 8000 1410 and
+    1406; 16384 x 2048, 160 rows 32 and 25, 536 49 and 43, 3072 200 and 167,
+    8000 489 and 452; 12288 x 2048, 65 rows 20 and 17.)"""
+    return (x.dim() == 2 and x.is_cuda
+            and x.shape[0] >= (65 if w.shape[0] <= 16384 else 192)
+            and x.shape[1] >= 1024 and w.shape[0] >= 4096
+            and _tiles_take(x, w))
+
+
+def tile_linear_silu(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """rows_linear_silu for more rows."""
+    _gpu()
+    return torch.ops.rlli.tile_linear_silu(x, w)
+
+
 def skinny_linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """rows_linear for K % 256 == 0 and N % 64 == 0."""
     if x.is_cuda:

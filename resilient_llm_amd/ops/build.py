@@ -46,6 +46,7 @@ LIBRARIES = {
         "prefill_flash.hip",
         "sampling.hip",
         "rows_gemm.hip",
+        "tile_gemm.hip",
         "streamprobe.hip",
     ],
     "rlli_attn": [

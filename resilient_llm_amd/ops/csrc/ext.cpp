@@ -704,6 +704,54 @@ std::tuple<Tensor, Tensor> rows_norm_linear(const Tensor& parts,
   return {out, after};
 }
 
+static void check_tiles(const Tensor& x, const Tensor& w, int multiple) {
+  check_bf16_contig(x, "x");
+  check_bf16_contig(w, "w");
+  TORCH_CHECK(x.device() == w.device(), "x and W on one GPU");
+  TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && w.size(1) == x.size(1),
+              "x/W K mismatch");
+  TORCH_CHECK(x.size(0) >= 1 && x.size(1) % 64 == 0 && x.size(1) > 0 &&
+                  w.size(0) % multiple == 0 && w.size(0) > 0,
+              "K % 64 == 0 and N % ", multiple, " == 0, got K=", x.size(1),
+              " N=", w.size(0));
+  TORCH_CHECK(x.numel() < int64_t(1) << 31 && w.numel() < int64_t(1) << 31,
+              "x and W below 4 GiB");
+  TORCH_CHECK(reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0 &&
+                  reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0,
+              "x and W start at multiples of 16 bytes");
+}
+
+// x w^T in f32 parts [splits, M, N], or in bf16 [M, N] where K is not divided
+Tensor tile_linear_parts(const Tensor& x, const Tensor& w) {
+  check_tiles(x, w, 8);
+  const int M = int(x.size(0)), N = int(w.size(0)), K = int(x.size(1));
+  c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
+  const rlli::TilePlan plan = rlli::tile_gemm_plan(M, N, K, false);
+  const bool parts = plan.splits > 1;
+  Tensor out = parts ? at::empty({plan.splits, M, N},
+                                 x.options().dtype(at::kFloat))
+                     : at::empty({M, N}, x.options());
+  rlli::launch_tile_gemm(bf16_ptr(x), bf16_ptr(w),
+                         parts ? out.data_ptr<float>() : nullptr,
+                         parts ? nullptr : bf16_ptr(out), M, N, K, false, plan,
+                         current_stream(x));
+  check_launch("tile_linear_parts");
+  return out;
+}
+
+// silu(x w[:I]^T) * (x w[I:]^T) for w [2 I, K]
+Tensor tile_linear_silu(const Tensor& x, const Tensor& w) {
+  check_tiles(x, w, 16);
+  const int M = int(x.size(0)), N = int(w.size(0)), K = int(x.size(1));
+  c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
+  Tensor out = at::empty({M, N / 2}, x.options());
+  rlli::launch_tile_gemm(bf16_ptr(x), bf16_ptr(w), nullptr, bf16_ptr(out), M,
+                         N, K, true, rlli::tile_gemm_plan(M, N, K, true),
+                         current_stream(x));
+  check_launch("tile_linear_silu");
+  return out;
+}
+
 // The same under the names and limits of earlier kernels; ``splitk`` has no
 // effect any more.
 static void check_skinny(const char* op, const Tensor& x, const Tensor& w,
@@ -826,6 +874,8 @@ TORCH_LIBRARY(rlli, m) {
         &rows_norm_ok);
   m.def("rows_norm_linear(Tensor parts, Tensor residual, Tensor gain, "
         "float eps, Tensor w, bool silu) -> (Tensor, Tensor)");
+  m.def("tile_linear_parts(Tensor x, Tensor w) -> Tensor");
+  m.def("tile_linear_silu(Tensor x, Tensor w) -> Tensor");
   m.def("skinny_linear(Tensor x, Tensor w) -> Tensor");
   m.def("skinny2_linear(Tensor x, Tensor w, int splitk) -> Tensor");
   m.def("skinny2_silu_linear(Tensor gu, Tensor w, int splitk) -> Tensor");
@@ -860,6 +910,8 @@ TORCH_LIBRARY_IMPL(rlli, CUDA, m) {
   m.impl("rows_linear_silu", &rows_linear_silu);
   m.impl("rows_linear_relu2", &rows_linear_relu2);
   m.impl("rows_norm_linear", &rows_norm_linear);
+  m.impl("tile_linear_parts", &tile_linear_parts);
+  m.impl("tile_linear_silu", &tile_linear_silu);
   m.impl("skinny_linear", &skinny_linear);
   m.impl("skinny2_linear", &skinny2_linear);
   m.impl("skinny2_silu_linear", &skinny2_silu_linear);

@@ -416,10 +416,10 @@ def tile_silu_fit(x: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether tile_linear_silu takes x w^T and is faster than the library and
     silu_mul.  (us, those first: 28672 x 4096, 160 rows 64 and 68, 192 66 and
     62, 536 147 and 113, 1024 222 and 190, 2048 416 and 383, 8000 1410 and
-    1406; 16384 x 2048, 160 rows 32 and 25, 536 49 and 43, 3072 200 and 167,
+    1406, but 8192 1412 and 1467; 16384 x 2048, 160 rows 32 and 25, 536 49 and 43, 3072 200 and 167,
     8000 489 and 452; 12288 x 2048, 65 rows 20 and 17.)"""
     return (x.dim() == 2 and x.is_cuda
-            and x.shape[0] >= (65 if w.shape[0] <= 16384 else 192)
+            and (65 if w.shape[0] <= 16384 else 192) <= x.shape[0] <= 8000
             and x.shape[1] >= 1024 and w.shape[0] >= 4096
             and _tiles_take(x, w))
 

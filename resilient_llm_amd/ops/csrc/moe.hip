@@ -22,6 +22,7 @@
 // split over the waves; large ones run 128 x 128 tiles through LDS.
 
 #include "mix.h"
+#include "tile_product.h"
 
 namespace rlli {
 namespace {
@@ -451,26 +452,8 @@ void moe_small_kernel(MoeArgs a) {
 }
 
 // ------------------------------------------- large row counts: LDS tiles
-// (32 WM) x (16 WN) MFMA blocks per wave pair grid, K step 64, double-
-// buffered through direct global->LDS loads.  A row's eight 16-byte
-// pieces land XOR-swizzled by the row number (the swizzle is applied to
-// the global address), which spreads the fragment reads of 16 rows over
-// all banks.  Two heights: 256 x 256 with eight waves of 128 x 64 each
-// (fewest LDS bytes per MFMA), and 128 x 128 with four of 64 x 64 for
-// experts with fewer rows.  What bounds the tall ones (6001 rows of 2048 in
-// 32 experts): with the products taken out 220 of 265 us remain, with the
-// loads taken out 190, so a step of 64 KB into LDS costs as much as its
-// products and they overlap in part only; a block's start and end are 10 of
-// its 68 us.  Four waves of 128 x 128 (a third less LDS traffic), other K
-// starts per XCD and lines asked for three or four steps ahead gave nothing.
-constexpr int BK = 64;
-
-DEV_INLINE void lds_load16(const void* g, void* l) {
-  __builtin_amdgcn_global_load_lds(
-      (const __attribute__((address_space(1))) void*)g,
-      (__attribute__((address_space(3))) void*)l, 16, 0, 0);
-}
-
+// A workgroup has a tile of 256 x 256, or 128 rows by 256 for experts with
+// fewer rows (tile_product.h).
 // Consecutive workgroups go to different XCDs.  Each XCD gets an equal run of
 // the full tiles' blocks, then an equal run of the others', counted on the
 // device: the tiles there could be are up to one per expert more, and runs of
@@ -502,13 +485,12 @@ DEV_INLINE bool tile_of(const MoeArgs& a, int block, int n_blocks, int& tile,
   return true;
 }
 
-template <bool UP, int TT, bool GATED>
-__global__ __launch_bounds__(TT == 256 ? 512 : 256, 2)
+template <bool UP, int MH, int NH, bool GATED>
+__global__ __launch_bounds__(512, 2)
 void moe_tile_kernel(MoeArgs a, int n_blocks) {
-  constexpr int NT = TT == 256 ? 512 : 256;       // threads
-  constexpr int NCOL = TT == 256 ? 4 : 2;         // waves along columns
-  constexpr int MI = TT == 256 ? 8 : 4;           // 16-row blocks per wave
-  constexpr int PIECES = TT * 8 / NT;
+  using P = tile::Product<MH, NH>;
+  constexpr int TM = P::TM, TN = P::TN;
+  static_assert(!GATED || NH % 2 == 0);
   extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
   int tile, nb;
   if (!tile_of(a, blockIdx.x, n_blocks, tile, nb)) return;
@@ -517,139 +499,73 @@ void moe_tile_kernel(MoeArgs a, int n_blocks) {
   const int p0 = a.tile_row0[tile];
   const int K = UP ? a.width : a.ffp;
   const int N = UP ? (GATED ? 2 : 1) * a.ffp : a.width;
-  const int n0 = nb * TT;
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int lr = lane & 15, g = lane >> 4;
+  const int n0 = nb * TN;
 
   // the rows' pairs and weights, for the gather and the epilogue
-  __shared__ int s_pair[TT];
-  __shared__ float s_weight[TT];
-  for (int r = tid; r < TT; r += NT) {
+  __shared__ int s_pair[TM];
+  __shared__ float s_weight[TM];
+  for (int r = threadIdx.x; r < TM; r += 512) {
     const int pair = a.perm[p0 + min(r, rows - 1)];
     s_pair[r] = pair;
     if constexpr (UP) s_weight[r] = a.weights[pair];
   }
   __syncthreads();
 
-  // piece i of this thread: tile row i * NT/8 + tid / 8, 16-byte column
-  // tid % 8, holding global column (tid % 8) ^ (row & 7)
-  const char* abase = reinterpret_cast<const char*>(UP ? a.h : a.act);
-  const char* bbase =
-      reinterpret_cast<const char*>(UP ? a.w_up : a.w_down) +
-      int64_t(e) * N * K * 2;
-  uint32_t ap[PIECES], bp[PIECES];        // bytes, below 2^32
-#pragma unroll
-  for (int i = 0; i < PIECES; ++i) {
-    const int r = i * (NT / 8) + (tid >> 3);
-    const int c = ((tid & 7) ^ (r & 7)) * 8;
-    if constexpr (UP)
-      ap[i] = (uint32_t(s_pair[r] / a.top) * K + c) * 2;
-    else
-      ap[i] = (uint32_t(p0 + min(r, rows - 1)) * K + c) * 2;
-    bp[i] = (uint32_t(min(n0 + r, N - 1)) * K + c) * 2;
-  }
-  auto stage = [&](int buf, int k0) {
-    uint16_t* la = lds + buf * 2 * TT * BK;
-    uint16_t* lb = la + TT * BK;
-#pragma unroll
-    for (int i = 0; i < PIECES; ++i) {
-      // wave-uniform LDS base; lane l lands at base + 16 l
-      if (i * (NT / 8) < rows)
-        lds_load16(abase + k0 * 2 + ap[i], la + (i * (NT / 8) + w * 8) * BK);
-      lds_load16(bbase + k0 * 2 + bp[i], lb + (i * (NT / 8) + w * 8) * BK);
-    }
-  };
+  P p;
+  p.rows(
+      [&](int r) {
+        return uint32_t(UP ? s_pair[r] / a.top : p0 + min(r, rows - 1)) * K *
+               2;
+      },
+      [&](int r) { return uint32_t(min(n0 + r, N - 1)) * K * 2; });
+  p.run(static_cast<const char*>(UP ? a.h : a.act),
+        static_cast<const char*>(UP ? a.w_up : a.w_down) +
+            int64_t(e) * N * K * 2,
+        K / tile::KS, lds);
 
-  const int wm = (w / NCOL) * MI * 16, wn = (w % NCOL) * 64;
-  f32x4_t acc[MI][4];
+  // a lane has four columns of a row
 #pragma unroll
-  for (int i = 0; i < MI; ++i)
+  for (int half = 0; half < 2; ++half)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-
-  // none of this wave's rows is one of the tile's: it only loads
-  const bool idle = wm >= rows;
-  const int nk = K / BK;
-  stage(0, 0);
-  for (int kt = 0; kt < nk; ++kt) {
-    // this wave's pieces of stage kt have landed, then everybody's
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    if (kt + 1 < nk) stage((kt + 1) & 1, (kt + 1) * BK);
-    if (idle) continue;
-    const uint16_t* la = lds + (kt & 1) * 2 * TT * BK;
-    const uint16_t* lb = la + TT * BK;
-    auto frag = [&](const uint16_t* base, int row, int kk) {
-      return *reinterpret_cast<const s16x8_t*>(
-          base + row * BK + (((kk * 4 + g) ^ (row & 7)) * 8));
-    };
-    // all of the first half's fragments, then the second half's one by
-    // one under the first half's MFMAs
-    s16x8_t fa[2][MI], fb[2][4];
-#pragma unroll
-    for (int kk = 0; kk < 2; ++kk) {
-#pragma unroll
-      for (int j = 0; j < 4; ++j) fb[kk][j] = frag(lb, wn + j * 16 + lr, kk);
-#pragma unroll
-      for (int i = 0; i < MI; ++i) fa[kk][i] = frag(la, wm + i * 16 + lr, kk);
-    }
-#pragma unroll
-    for (int kk = 0; kk < 2; ++kk)
-#pragma unroll
-      for (int i = 0; i < MI; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-              fa[kk][i], fb[kk][j], acc[i][j], 0, 0, 0);
-    constexpr int MFMA = 0x8, DS_READ = 0x100;
-    __builtin_amdgcn_sched_group_barrier(DS_READ, 4 + MI, 0);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      __builtin_amdgcn_sched_group_barrier(MFMA, 4, 0);
-      __builtin_amdgcn_sched_group_barrier(DS_READ, 2, 0);
-    }
-#pragma unroll
-    for (int i = 4; i < MI; ++i) {
-      __builtin_amdgcn_sched_group_barrier(MFMA, 4, 0);
-      __builtin_amdgcn_sched_group_barrier(DS_READ, 1, 0);
-    }
-    __builtin_amdgcn_sched_group_barrier(MFMA, 4 * MI, 0);
-  }
-
-#pragma unroll
-  for (int i = 0; i < MI; ++i)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int tr = wm + i * 16 + g * 4 + r;
+    for (int i = 0; i < MH; ++i) {
+      const int tr = P::row_of(half, i);
       if (tr >= rows) continue;
       const int pair = s_pair[tr];
-      if constexpr (UP) {
-        const float wt = s_weight[tr];
-        uint16_t* o = reinterpret_cast<uint16_t*>(a.act) +
-                      int64_t(p0 + tr) * a.ffp;
-        if constexpr (GATED) {
+      const float wt = UP ? s_weight[tr] : 0.f;
 #pragma unroll
-          for (int j = 0; j < 4; j += 2) {
-            const int f = (n0 + wn + j * 16) / 2 + lr;
+      for (int b = 0; b < 2; ++b) {
+        const auto& acc = p.acc[half][b][i];
+        if constexpr (UP && GATED) {
+          // blocks of 16 gate rows and their 16 up rows by turns
+#pragma unroll
+          for (int j = 0; j < NH; j += 2) {
+            const int n = n0 + P::col_of(b, j);
+            const int f = n / 32 * 16 + n % 16;
+            f32x4_t v;
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+              v[r] = expert_gate<uint16_t>(acc[j][r] * wt, acc[j + 1][r] * wt,
+                                           a.limit);
             if (f < a.ffp)
-              o[f] = f32_to_bf16(expert_gate<uint16_t>(
-                  acc[i][j][r] * wt, acc[i][j + 1][r] * wt, a.limit));
+              act_store4(static_cast<uint16_t*>(a.act) +
+                             int64_t(p0 + tr) * a.ffp + f, v);
           }
         } else {
 #pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            const int f = n0 + wn + j * 16 + lr;
-            if (f < a.ffp)
-              o[f] = f32_to_bf16(relu_squared(acc[i][j][r]) * wt);
-          }
-        }
-      } else {
-        uint16_t* o = reinterpret_cast<uint16_t*>(a.y) +
-                      int64_t(pair) * a.width;
+          for (int j = 0; j < NH; ++j) {
+            const int c = n0 + P::col_of(b, j);
+            if (c >= N) continue;
+            if constexpr (UP) {
+              f32x4_t v;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int c = n0 + wn + j * 16 + lr;
-          if (c < N) o[c] = f32_to_bf16(acc[i][j][r]);
+              for (int r = 0; r < 4; ++r) v[r] = relu_squared(acc[j][r]) * wt;
+              act_store4(static_cast<uint16_t*>(a.act) +
+                             int64_t(p0 + tr) * a.ffp + c, v);
+            } else {
+              act_store4(static_cast<uint16_t*>(a.y) +
+                             int64_t(pair) * a.width + c, acc[j]);
+            }
+          }
         }
       }
     }
@@ -686,26 +602,26 @@ void small(const MoeArgs& a, hipStream_t st) {
                      a);
 }
 
-template <bool UP, int TT, bool GATED>
+template <bool UP, int MH, int NH, bool GATED>
 void tiled_one(const MoeArgs& a, hipStream_t st) {
-  const size_t smem = size_t(4) * TT * BK * 2;
-  const int nb = ((UP ? (GATED ? 2 : 1) * a.ffp : a.width) + TT - 1) / TT;
+  using P = tile::Product<MH, NH>;
+  const int nb =
+      ((UP ? (GATED ? 2 : 1) * a.ffp : a.width) + P::TN - 1) / P::TN;
   // two runs per XCD, each up to one block longer than its part
   const int blocks = (nb * a.max_tiles + 7) / 8 * 8 + 8;
-  auto* k = moe_tile_kernel<UP, TT, GATED>;
-  if (smem > 65536)
+  auto* k = moe_tile_kernel<UP, MH, NH, GATED>;
+  if (P::LDS > 65536)
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(k),
                               hipFuncAttributeMaxDynamicSharedMemorySize,
-                              int(smem));
-  hipLaunchKernelGGL(k, dim3(blocks),
-                     dim3(TT == 256 ? 512 : 256), smem, st, a, nb);
+                              int(P::LDS));
+  hipLaunchKernelGGL(k, dim3(blocks), dim3(512), P::LDS, st, a, nb);
 }
 
-template <int TT>
+template <int MH>
 void tiled(const MoeArgs& a, hipStream_t st) {
-  if (a.gated) tiled_one<true, TT, true>(a, st);
-  else tiled_one<true, TT, false>(a, st);
-  tiled_one<false, TT, false>(a, st);
+  if (a.gated) tiled_one<true, MH, 2, true>(a, st);
+  else tiled_one<true, MH, 2, false>(a, st);
+  tiled_one<false, MH, 2, false>(a, st);
 }
 
 }  // namespace
@@ -735,8 +651,8 @@ void launch_moe_experts(const MoeArgs& a, hipStream_t st) {
   } else if (a.tile_m == 16) {
     small<uint16_t>(a, st);
   } else {
-    if (a.tile_m == 256) tiled<256>(a, st);
-    else tiled<128>(a, st);
+    if (a.tile_m == 256) tiled<4>(a, st);
+    else tiled<2>(a, st);
   }
 }
 

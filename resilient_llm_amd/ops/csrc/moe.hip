@@ -486,17 +486,11 @@ DEV_INLINE bool tile_of(const MoeArgs& a, int block, int n_blocks, int& tile,
 }
 
 template <bool UP, int MH, int NH, bool GATED>
-__global__ __launch_bounds__(512, 2)
-void moe_tile_kernel(MoeArgs a, int n_blocks) {
+DEV_INLINE void moe_tile(const MoeArgs& a, int rows, int e, int p0, int nb) {
   using P = tile::Product<MH, NH>;
   constexpr int TM = P::TM, TN = P::TN;
   static_assert(!GATED || NH % 2 == 0);
   extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
-  int tile, nb;
-  if (!tile_of(a, blockIdx.x, n_blocks, tile, nb)) return;
-  const int rows = a.tile_rows[tile];
-  const int e = a.tile_expert[tile];
-  const int p0 = a.tile_row0[tile];
   const int K = UP ? a.width : a.ffp;
   const int N = UP ? (GATED ? 2 : 1) * a.ffp : a.width;
   const int n0 = nb * TN;
@@ -569,6 +563,20 @@ void moe_tile_kernel(MoeArgs a, int n_blocks) {
         }
       }
     }
+}
+
+// Tiles that are up to half full take half the height (6001 rows of 2048 in 32
+// experts of 1024, four each: 1.075 -> 1.130 times as fast as before both).
+template <bool UP, int MH, int NH, bool GATED>
+__global__ __launch_bounds__(512, 2)
+void moe_tile_kernel(MoeArgs a, int n_blocks) {
+  int tile, nb;
+  if (!tile_of(a, blockIdx.x, n_blocks, tile, nb)) return;
+  const int rows = a.tile_rows[tile];
+  const int e = a.tile_expert[tile];
+  const int p0 = a.tile_row0[tile];
+  if (MH == 4 && rows <= 128) moe_tile<UP, 2, NH, GATED>(a, rows, e, p0, nb);
+  else moe_tile<UP, MH, NH, GATED>(a, rows, e, p0, nb);
 }
 
 template <typename T>

@@ -462,10 +462,9 @@ class LlamaForCausalLM:
                 qkv, k_cache, v_cache, chunk_row0, chunk_pos0, chunk_nrows,
                 chunk_btrow, block_tables_pre, self.scale, self.n_heads)
             if n_decode:
-                out_d = ops.decode_attn_qkv(
+                ops.decode_attn_qkv_out(
                     qkv[:n_decode], k_cache, v_cache, block_tables_dec,
-                    seq_lens_dec, self.scale, self.n_heads)
-                out[:n_decode] = out_d
+                    seq_lens_dec, self.scale, self.n_heads, out)
             return out
         return self._forward(input_ids, positions, kv_cache, slot_mapping,
                              attn, last_idx=sample_idx)

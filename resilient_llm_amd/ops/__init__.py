@@ -164,6 +164,18 @@ def decode_attn_qkv(qkv: torch.Tensor, k_cache: torch.Tensor,
     return out.reshape(B, n_q * D)
 
 
+def decode_attn_qkv_out(qkv, k_cache, v_cache, block_table, seq_lens,
+                        scale: float, n_q: int, out: torch.Tensor) -> None:
+    """decode_attn_qkv to the first rows of ``out``."""
+    if qkv.is_cuda:
+        _gpu()
+        torch.ops.rlli.decode_attn_qkv_out(qkv, k_cache, v_cache, block_table,
+                                           seq_lens, scale, n_q, out)
+        return
+    out[:qkv.shape[0]] = decode_attn_qkv(qkv, k_cache, v_cache, block_table,
+                                         seq_lens, scale, n_q)
+
+
 def decode_attn_rope_qkv(qkv, positions, cos_sin, k_cache, v_cache,
                          slot_mapping, block_table, seq_lens, scale: float,
                          n_q: int) -> torch.Tensor:

@@ -292,7 +292,8 @@ static Tensor decode_attn_any(const Tensor& q, int64_t n_q,
                               const Tensor& block_table,
                               const Tensor& seq_lens, double scale,
                               const Tensor* positions, const Tensor* cos_sin,
-                              const Tensor* slot_mapping) {
+                              const Tensor* slot_mapping,
+                              const Tensor* into = nullptr) {
   const bool parts = q.scalar_type() == at::kFloat;
   if (parts) {
     TORCH_CHECK(q.is_cuda() && q.is_contiguous() && q.dim() == 3 &&
@@ -322,8 +323,17 @@ static Tensor decode_attn_any(const Tensor& q, int64_t n_q,
   // (longer ones, as a batch's buffers are, end in what nobody reads)
   TORCH_CHECK(block_table.size(0) >= batch && seq_lens.numel() >= batch,
               "tables and lengths of ", batch, " sequences are needed");
-  Tensor out = at::empty({batch, n_q * D},
-                         q.options().dtype(at::kBFloat16));
+  if (into) {
+    check_bf16_contig(*into, "out");
+    TORCH_CHECK(into->dim() == 2 && into->size(0) >= batch &&
+                    into->size(1) == n_q * D &&
+                    into->device() == q.device() &&
+                    reinterpret_cast<uintptr_t>(into->data_ptr()) % 16 == 0,
+                "out: rows of the queries' width");
+  }
+  Tensor out = into ? *into
+                    : at::empty({batch, n_q * D},
+                                q.options().dtype(at::kBFloat16));
   if (batch == 0) return out;
   c10::hip::HIPGuardMasqueradingAsCUDA guard(q.device());
   // scratch of sequences that several workgroups share; allocated here, so
@@ -385,6 +395,17 @@ Tensor decode_attn_qkv(const Tensor& qkv, const Tensor& k_cache,
   check_qkv_width(qkv, k_cache, n_q);
   return decode_attn_any(qkv, n_q, k_cache, v_cache, block_table, seq_lens,
                          scale, nullptr, nullptr, nullptr);
+}
+
+// The same to the first rows of ``out``.
+void decode_attn_qkv_out(const Tensor& qkv, const Tensor& k_cache,
+                         const Tensor& v_cache, const Tensor& block_table,
+                         const Tensor& seq_lens, double scale, int64_t n_q,
+                         Tensor out) {
+  check_bf16_contig(qkv, "qkv");
+  check_qkv_width(qkv, k_cache, n_q);
+  decode_attn_any(qkv, n_q, k_cache, v_cache, block_table, seq_lens, scale,
+                  nullptr, nullptr, nullptr, &out);
 }
 
 // Fused decode: rope + append + attention in one kernel.  qkv: bf16 rows, or
@@ -555,12 +576,24 @@ Tensor prefill_paged_attn(const Tensor& qkv, const Tensor& k_cache,
   Tensor out = at::empty({T, n_q * D}, qkv.options());
   c10::hip::HIPGuardMasqueradingAsCUDA guard(qkv.device());
   const Tensor k = aligned(k_cache), v = aligned(v_cache);
+  rlli::PrefillParts parts{nullptr, nullptr,
+                           rlli::prefill_splits(n_chunks, n_kv, group,
+                                                max_blocks * block_size),
+                           T};
+  Tensor part, ml;
+  if (parts.splits > 1) {
+    const auto f32 = qkv.options().dtype(at::kFloat);
+    part = at::empty({parts.splits, T, n_q * D}, f32);
+    ml = at::empty({parts.splits, T, n_q, 2}, f32);
+    parts.o = part.data_ptr<float>();
+    parts.ml = ml.data_ptr<float>();
+  }
   rlli::launch_prefill_paged(
       bf16_ptr(qkv), k.data_ptr(), v.data_ptr(),
       chunk_row0.data_ptr<int32_t>(), chunk_pos0.data_ptr<int32_t>(),
       chunk_nrows.data_ptr<int32_t>(), chunk_btrow.data_ptr<int32_t>(),
       block_tables.data_ptr<int32_t>(), bf16_ptr(out), n_chunks, n_kv,
-      group, D, stride, max_blocks, block_size, float(scale), cache_fp8,
+      group, D, stride, max_blocks, block_size, float(scale), cache_fp8, parts,
       current_stream(qkv));
   check_launch("prefill_paged_attn");
   return out;
@@ -848,6 +881,9 @@ TORCH_LIBRARY(rlli, m) {
         "int n_q) -> ()");
   m.def("decode_attn_qkv(Tensor qkv, Tensor k_cache, Tensor v_cache, "
         "Tensor block_table, Tensor seq_lens, float scale, int n_q) -> Tensor");
+  m.def("decode_attn_qkv_out(Tensor qkv, Tensor k_cache, Tensor v_cache, "
+        "Tensor block_table, Tensor seq_lens, float scale, int n_q, "
+        "Tensor(a!) out) -> ()");
   m.def("decode_attn_rope_qkv(Tensor qkv, Tensor positions, Tensor cos_sin, "
         "Tensor(a!) k_cache, Tensor(b!) v_cache, Tensor slot_mapping, "
         "Tensor block_table, Tensor seq_lens, float scale, int n_q) -> Tensor");
@@ -898,6 +934,7 @@ TORCH_LIBRARY_IMPL(rlli, CUDA, m) {
   m.impl("decode_attn", &decode_attn);
   m.impl("rope_kv_append_qkv_", &rope_kv_append_qkv_);
   m.impl("decode_attn_qkv", &decode_attn_qkv);
+  m.impl("decode_attn_qkv_out", &decode_attn_qkv_out);
   m.impl("decode_attn_rope_qkv", &decode_attn_rope_qkv);
   m.impl("kv_append_qkv_", &kv_append_qkv_);
   m.impl("decode_attn_q_rope", &decode_attn_q_rope);

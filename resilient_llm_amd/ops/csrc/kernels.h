@@ -6,6 +6,8 @@
 #include <hip/hip_runtime.h>
 #include <cstdint>
 
+#include "prefill_parts.h"
+
 namespace rlli {
 
 // y = rmsnorm(x) * w           (residual == nullptr)
@@ -108,7 +110,7 @@ void launch_prefill_paged(const uint16_t* qkv, const void* k_cache,
                           int n_chunks, int n_kv_heads, int group,
                           int head_dim, int qkv_stride, int max_blocks,
                           int block_size, float scale, bool cache_fp8,
-                          hipStream_t stream);
+                          const PrefillParts& parts, hipStream_t stream);
 
 // Products of at most 128 rows, y[M, N] = x[M, K] w[N, K]^T (rows_gemm.hip).
 // With parts given, f32 [splits, M, N] whose sum is y; otherwise out.

@@ -33,6 +33,7 @@
 #pragma once
 
 #include "common.h"
+#include "prefill_parts.h"
 
 #include <type_traits>
 
@@ -78,13 +79,19 @@ DEV_INLINE s16x4 read_tr(const uint16_t* p) {
 // are this tile's; false: none.  A windowed one also says which keys a row
 // sees (``window`` of them and the first ``keep``) and a head's sink.
 
+// How many parts a tile's steps of KS tiles of keys are divided into.
+DEV_INLINE int parts_of(int steps, int splits) {
+  return min(splits, max(steps / 4, 1));
+}
+
 // D: head width; W: heads, a wave each; BS: block size of the cache where it
 // is known; KS: waves per head, each with every KS-th tile of keys, for
 // launches that leave CUs idle.  Their sums meet in LDS.
 template <int D, int W, int BS, int KS, typename Src>
 __global__ __launch_bounds__(64 * W * KS, W == 4 ? 2 : 1)
 void prefill_flash_kernel(Src src, uint16_t* __restrict__ out, int n_tiles,
-                          int n_kv, int group, int stride, float scale) {
+                          int n_kv, int group, int stride, float scale,
+                          PrefillParts parts) {
   using KC = typename Src::KC;
   constexpr bool kDirect = std::is_same<KC, CacheBF16>::value;
   static_assert(KS == 1 || !Src::kWindow, "windows skip single tiles");
@@ -102,7 +109,8 @@ void prefill_flash_kernel(Src src, uint16_t* __restrict__ out, int n_tiles,
 
   // the tiles of a key/value head stay on an XCD (workgroups go to XCDs in
   // turn), those with the longest context first
-  const int per_head = n_tiles * (group / W);
+  const int splits = KS > 1 ? parts.splits : 1;
+  const int per_head = n_tiles * (group / W) * splits;
   int kvh, i;
   if (n_kv % 8 == 0) {
     i = blockIdx.x / 8;
@@ -112,6 +120,8 @@ void prefill_flash_kernel(Src src, uint16_t* __restrict__ out, int n_tiles,
     kvh = i / per_head;
   }
   i %= per_head;
+  const int part = i % splits;
+  i /= splits;
   const int tile = n_tiles - 1 - i / (group / W);
   int row0, nrows, first, pos0;
   if (!src.find(tile, row0, nrows, first, pos0)) return;
@@ -124,6 +134,11 @@ void prefill_flash_kernel(Src src, uint16_t* __restrict__ out, int n_tiles,
   const int head = kvh * group + i % (group / W) * W + w;
   const int qpos = pos0 + min(qi, nrows - 1), qpos_last = pos0 + nrows - 1;
   const int len = pos0 + nrows;              // keys that the last row sees
+  const int steps = (len + KS * KT - 1) / (KS * KT);
+  const int n_parts = parts_of(steps, splits);
+  if (part >= n_parts) return;
+  const int begin = steps * part / n_parts * (KS * KT);
+  const int end = min(len, steps * (part + 1) / n_parts * (KS * KT));
   // tiles of keys between the kept ones and the first row's window are
   // passed over
   int window = 0, keep = 0, win0 = 0;
@@ -332,19 +347,19 @@ void prefill_flash_kernel(Src src, uint16_t* __restrict__ out, int n_tiles,
     }
   };
 
-  int kv0 = keep > 0 ? 0 : win0, ahead = after(kv0);
+  int kv0 = Src::kWindow ? (keep > 0 ? 0 : win0) : begin, ahead = after(kv0);
   look_up(kv0);
   fetch(lds, kv0);
   land(lds);
   look_up(ahead);
   int cur = 0;
-  while (kv0 < len) {
+  while (kv0 < end) {
     // this wave's part of the tile has landed, then everybody's; and nobody
     // reads the tile before any more
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     uint16_t* next = lds + (cur ^ 1) * STAGE;
-    const bool more = ahead < len;
+    const bool more = ahead < end;
     if (more) {
       fetch(next, ahead);
       look_up(after(ahead));
@@ -372,7 +387,7 @@ void prefill_flash_kernel(Src src, uint16_t* __restrict__ out, int n_tiles,
     }
     __syncthreads();
     if (ks == 1) return;
-    // this wave has the first tile, of which every row sees a key
+    // (of a later part, either wave's tiles may be hidden from a row)
     const float m1 = side[VT * 16 * 64], top = fmaxf(m, m1);
     const float c0 = __builtin_amdgcn_exp2f((m - top) * c2);
     const float c1 = __builtin_amdgcn_exp2f((m1 - top) * c2);
@@ -382,9 +397,25 @@ void prefill_flash_kernel(Src src, uint16_t* __restrict__ out, int n_tiles,
 #pragma unroll
       for (int r = 0; r < 16; ++r)
         o[v][r] = o[v][r] * c0 + side[(v * 16 + r) * 64] * c1;
+    m = top;
   }
   if (qi >= nrows) return;
   l += __shfl_xor(l, 32, kWave);
+  if (KS > 1 && n_parts > 1) {
+    const int64_t at = (int64_t(part) * parts.rows + row0 + qi) * n_q + head;
+    if (hi == 0) {
+      parts.ml[at * 2] = m;
+      parts.ml[at * 2 + 1] = l;
+    }
+#pragma unroll
+    for (int v = 0; v < VT; ++v)
+#pragma unroll
+      for (int r = 0; r < 16; r += 4)
+        *reinterpret_cast<float4*>(parts.o + at * D + v * 32 + (r >> 2) * 8 +
+                                   hi * 4) =
+            float4{o[v][r], o[v][r + 1], o[v][r + 2], o[v][r + 3]};
+    return;
+  }
   float inv = 1.f / l;
   if constexpr (Src::kWindow) {
     if (src.sink) {                          // it takes its share, no value
@@ -404,12 +435,53 @@ void prefill_flash_kernel(Src src, uint16_t* __restrict__ out, int n_tiles,
                 pack2(o[v][r + 2] * inv, o[v][r + 3] * inv)};
 }
 
+// The parts of a tile's rows together: a workgroup per (tile, query head).
+template <int D, typename Src>
+__global__ __launch_bounds__(256)
+void prefill_combine_kernel(Src src, uint16_t* __restrict__ out, int n_q,
+                            float scale, PrefillParts parts) {
+  const int tile = blockIdx.x / n_q, head = blockIdx.x % n_q;
+  int row0, nrows, first, pos0;
+  if (!src.find(tile, row0, nrows, first, pos0)) return;
+  const int n =
+      parts_of((pos0 + nrows + 2 * KT - 1) / (2 * KT), parts.splits);
+  if (n == 1) return;
+  const float c2 = fmaxf(fabsf(scale), 1e-30f) * 1.4426950408889634f;
+  for (int e = threadIdx.x; e < nrows * (D / 4); e += 256) {
+    const int64_t row = int64_t(row0 + e / (D / 4)) * n_q + head;
+    const int d = e % (D / 4) * 4;
+    const int64_t step = int64_t(parts.rows) * n_q;
+    float top = kHidden;
+    for (int p = 0; p < n; ++p)
+      top = fmaxf(top, parts.ml[(p * step + row) * 2]);
+    float4 num = {0.f, 0.f, 0.f, 0.f};
+    float den = 0.f;
+#pragma unroll 4
+    for (int p = 0; p < n; ++p) {
+      const float2 ml = *reinterpret_cast<const float2*>(
+          parts.ml + (p * step + row) * 2);
+      const float4 o = *reinterpret_cast<const float4*>(
+          parts.o + (p * step + row) * D + d);
+      const float c = __builtin_amdgcn_exp2f((ml.x - top) * c2);
+      num.x += c * o.x;
+      num.y += c * o.y;
+      num.z += c * o.z;
+      num.w += c * o.w;
+      den += c * ml.y;
+    }
+    const float inv = 1.f / den;
+    *reinterpret_cast<uint2*>(out + row * D + d) =
+        uint2{pack2(num.x * inv, num.y * inv), pack2(num.z * inv, num.w * inv)};
+  }
+}
+
 // ``keys``: about how many a sequence has, as far as the host knows without
 // waiting for the device: the mean of a batch of prompts, the width of the
 // block table for pages.
 template <int D, int BS, typename Src>
 void by_group(const Src& src, uint16_t* out, int n_tiles, int n_kv, int group,
-              int stride, float scale, int keys, hipStream_t st) {
+              int stride, float scale, int keys, hipStream_t st,
+              const PrefillParts& parts = {nullptr, nullptr, 1, 0}) {
   auto go = [&](auto tag, auto waves) {
     constexpr int W = decltype(tag)::value, KS = decltype(waves)::value;
     constexpr size_t smem = KS == 1 ? 0 : size_t(KS) * 2 * 2 * KT * D * 2;
@@ -418,9 +490,15 @@ void by_group(const Src& src, uint16_t* out, int n_tiles, int n_kv, int group,
       (void)hipFuncSetAttribute(reinterpret_cast<const void*>(k),
                                 hipFuncAttributeMaxDynamicSharedMemorySize,
                                 int(smem));
-    hipLaunchKernelGGL(k, dim3(n_tiles * n_kv * (group / W)),
+    const int splits = KS > 1 ? parts.splits : 1;
+    hipLaunchKernelGGL(k, dim3(n_tiles * n_kv * (group / W) * splits),
                        dim3(64 * W * KS), smem, st, src, out, n_tiles, n_kv,
-                       group, stride, scale);
+                       group, stride, scale, parts);
+    if constexpr (KS > 1)
+      if (splits > 1)
+        hipLaunchKernelGGL((prefill_combine_kernel<D, Src>),
+                           dim3(n_tiles * n_kv * group), dim3(256), 0, st, src,
+                           out, n_kv * group, scale, parts);
   };
   using I1 = std::integral_constant<int, 1>;
   using I2 = std::integral_constant<int, 2>;
@@ -439,7 +517,7 @@ void by_group(const Src& src, uint16_t* out, int n_tiles, int n_kv, int group,
   // of pages in a table for 8192 take two, 9.1, and would 8.3 with one.  The
   // two forms sum keys in different order, so that the last bits of a row's
   // result depend on the batch.
-  else if (n_tiles * n_kv * (group / 4) <= 400 && keys >= 384)
+  else if (two_waves(n_tiles, n_kv, group, keys))
     go(I4{}, I2{});
   else go(I4{}, I1{});
 }

@@ -1,6 +1,7 @@
 // Launches of prompt attention over batch rows and over pages; the kernel is
 // in prefill_flash.h.
 
+#include "kernels.h"
 #include "prefill_flash.h"
 
 namespace rlli {
@@ -94,7 +95,7 @@ void launch_prefill_paged(const uint16_t* qkv, const void* k_cache,
                           int n_chunks, int n_kv_heads, int group,
                           int head_dim, int qkv_stride, int max_blocks,
                           int block_size, float scale, bool cache_fp8,
-                          hipStream_t st) {
+                          const PrefillParts& parts, hipStream_t st) {
   auto go = [&](auto kc, auto d, auto bs) {
     using KC = decltype(kc);
     const Pages<KC> src{qkv,
@@ -104,7 +105,7 @@ void launch_prefill_paged(const uint16_t* qkv, const void* k_cache,
                         block_tables, max_blocks, block_size};
     by_group<decltype(d)::value, decltype(bs)::value>(
         src, out, n_chunks, n_kv_heads, group, qkv_stride, scale,
-        max_blocks * block_size, st);
+        max_blocks * block_size, st, parts);
   };
   auto by_dim = [&](auto kc) {
     using I16 = std::integral_constant<int, 16>;

@@ -103,6 +103,39 @@ def test_two_waves_per_head_over_pages(D, bs, fp8):
     close(got, ref.prefill_paged_attn(qkv, k, v, *t, tables, D ** -0.5, n_q))
 
 
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("n_q,n_kv,D,bs", [(4, 1, 128, 16), (8, 2, 64, 16),
+                                           (8, 1, 128, 8)])
+@pytest.mark.parametrize("seqs", [
+    [(2000, 40)], [(2047, 1)], [(0, 65), (1023, 2), (255, 31), (8100, 33)]],
+    ids=str)
+def test_keys_in_parts(n_q, n_kv, D, bs, fp8, seqs):
+    """Workgroups that share a tile's keys: up to sixteen parts, sequences too
+    short for them, rows that see nothing of a part's last keys."""
+    gen = torch.Generator().manual_seed(bs)
+    width = -(-max(s + n for s, n in seqs) // bs)
+    k, v = (torch.randn(len(seqs) * width, n_kv, bs, D, generator=gen)
+            .to(torch.float8_e4m3fn if fp8 else torch.bfloat16) for _ in "kv")
+    tables = torch.randperm(len(seqs) * width, generator=gen) \
+        .to(torch.int32).view(len(seqs), width)
+    # a row in front and one behind that are nobody's
+    T = sum(n for _, n in seqs) + 2
+    qkv = torch.randn(T, (n_q + 2 * n_kv) * D, generator=gen) \
+        .to(torch.bfloat16)
+    tiles, row = [], 1
+    for b, (start, n) in enumerate(seqs):
+        tiles += [(row + o, start + o, min(32, n - o), b)
+                  for o in range(0, n, 32)]
+        row += n
+    t = torch.tensor(tiles, dtype=torch.int32).t().contiguous()
+    got = ops.prefill_paged_attn(
+        qkv.to(DEV), k.to(DEV), v.to(DEV), *t.to(DEV), tables.to(DEV),
+        D ** -0.5, n_q)
+    k, v = (x.float().to(torch.bfloat16) for x in (k, v))
+    want = ref.prefill_paged_attn(qkv, k, v, *t, tables, D ** -0.5, n_q)
+    close(got[1:-1], want[1:-1])
+
+
 def test_row_offsets_of_any_device_and_count():
     gen = torch.Generator().manual_seed(1)
     qkv = torch.randn(45, 6 * 64, generator=gen).to(torch.bfloat16).to(DEV)

@@ -517,52 +517,44 @@ DEV_INLINE void moe_tile(const MoeArgs& a, int rows, int e, int p0, int nb) {
             int64_t(e) * N * K * 2,
         K / tile::KS, lds);
 
-  // a lane has four columns of a row
+  constexpr bool PAIRS = UP && GATED;
 #pragma unroll
-  for (int half = 0; half < 2; ++half)
+  for (int i = 0; i < MH; ++i) {
+    float wt[2];
 #pragma unroll
-    for (int i = 0; i < MH; ++i) {
-      const int tr = P::row_of(half, i);
-      if (tr >= rows) continue;
-      const int pair = s_pair[tr];
-      const float wt = UP ? s_weight[tr] : 0.f;
+    for (int half = 0; half < 2; ++half)
+      wt[half] = UP ? s_weight[half * TM / 2 + P::row_of(i)] : 0.f;
+    const int tr = P::half_of() * TM / 2 + P::row_of(i);
+    uint16_t* to = UP ? static_cast<uint16_t*>(a.act) + int64_t(p0 + tr) * a.ffp
+                      : static_cast<uint16_t*>(a.y) +
+                            int64_t(s_pair[tr]) * a.width;
 #pragma unroll
-      for (int b = 0; b < 2; ++b) {
-        const auto& acc = p.acc[half][b][i];
-        if constexpr (UP && GATED) {
-          // blocks of 16 gate rows and their 16 up rows by turns
+    for (int b = 0; b < 2; ++b)
 #pragma unroll
-          for (int j = 0; j < NH; j += 2) {
-            const int n = n0 + P::col_of(b, j);
-            const int f = n / 32 * 16 + n % 16;
-            f32x4_t v;
+      for (int j = 0; j < NH; j += PAIRS ? 2 : 1) {
+        uint2 v[2];
 #pragma unroll
-            for (int r = 0; r < 4; ++r)
-              v[r] = expert_gate<uint16_t>(acc[j][r] * wt, acc[j + 1][r] * wt,
-                                           a.limit);
-            if (f < a.ffp)
-              act_store4(static_cast<uint16_t*>(a.act) +
-                             int64_t(p0 + tr) * a.ffp + f, v);
+        for (int half = 0; half < 2; ++half) {
+          f32x4_t f = p.acc[half][b][i][j];
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            // blocks of 16 gate rows and their 16 up rows by turns
+            if constexpr (PAIRS)
+              f[r] = expert_gate<uint16_t>(
+                  f[r] * wt[half], p.acc[half][b][i][j + 1][r] * wt[half],
+                  a.limit);
+            else if constexpr (UP)
+              f[r] = relu_squared(f[r]) * wt[half];
           }
-        } else {
-#pragma unroll
-          for (int j = 0; j < NH; ++j) {
-            const int c = n0 + P::col_of(b, j);
-            if (c >= N) continue;
-            if constexpr (UP) {
-              f32x4_t v;
-#pragma unroll
-              for (int r = 0; r < 4; ++r) v[r] = relu_squared(acc[j][r]) * wt;
-              act_store4(static_cast<uint16_t*>(a.act) +
-                             int64_t(p0 + tr) * a.ffp + c, v);
-            } else {
-              act_store4(static_cast<uint16_t*>(a.y) +
-                             int64_t(pair) * a.width + c, acc[j]);
-            }
-          }
+          act_store4(reinterpret_cast<uint16_t*>(&v[half]), f);
         }
+        const uint4 eight = P::eight(v[0], v[1]);
+        const int c = n0 + P::eight_of(b, j);
+        const int col = PAIRS ? c / 32 * 16 + c % 16 : c;
+        if (tr < rows && col < (UP ? a.ffp : a.width))
+          *reinterpret_cast<uint4*>(to + col) = eight;
       }
-    }
+  }
 }
 
 // Tiles that are up to half full take half the height (6001 rows of 2048 in 32

@@ -63,45 +63,53 @@ void tile_gemm_kernel(const uint16_t* __restrict__ x,
   p.run(reinterpret_cast<const char*>(x + int64_t(s0) * tile::KS),
         reinterpret_cast<const char*>(w + int64_t(s0) * tile::KS), nk, lds);
 
-  // a lane has four columns of y of one row
+  if constexpr (OUT == OUT_PARTS) {
+    float* y = static_cast<float*>(out) + int64_t(split) * M * N;
 #pragma unroll
-  for (int a = 0; a < 2; ++a)
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+      for (int i = 0; i < MH; ++i) {
+        const int row = m0 + a * TM / 2 + P::row_of(i);
+        if (row >= M) continue;
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+          for (int j = 0; j < NH; ++j) {
+            const int col = n0 + P::col_of(b, j);
+            if (col < N)
+              *reinterpret_cast<tile::f32x4*>(y + int64_t(row) * N + col) =
+                  p.acc[a][b][i][j];
+          }
+      }
+  } else {
+    constexpr bool SILU = OUT == OUT_SILU;
+    const int wide = SILU ? half : N;
 #pragma unroll
     for (int i = 0; i < MH; ++i) {
-      const int row = m0 + P::row_of(a, i);
-      if (row >= M) continue;
+      const int row = m0 + P::half_of() * TM / 2 + P::row_of(i);
 #pragma unroll
-      for (int j = 0; j < NH; ++j) {
-        if constexpr (OUT == OUT_SILU) {
-          const int col = panel * TN / 2 + P::col_of(0, j);
-          if (col >= half) continue;
-          float v[4];
+      for (int b = 0; b < (SILU ? 1 : 2); ++b)
 #pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const float g = p.acc[a][0][i][j][r];
-            v[r] = g / (1.f + __expf(-g)) * p.acc[a][1][i][j][r];
+        for (int j = 0; j < NH; ++j) {
+          uint2 v[2];
+#pragma unroll
+          for (int a = 0; a < 2; ++a) {
+            tile::f32x4 f = p.acc[a][b][i][j];
+            if constexpr (SILU) {
+#pragma unroll
+              for (int r = 0; r < 4; ++r)
+                f[r] = f[r] / (1.f + __expf(-f[r])) * p.acc[a][1][i][j][r];
+            }
+            v[a] = uint2{pack2(f[0], f[1]), pack2(f[2], f[3])};
           }
-          *reinterpret_cast<uint2*>(static_cast<uint16_t*>(out) +
-                                    int64_t(row) * half + col) =
-              uint2{pack2(v[0], v[1]), pack2(v[2], v[3])};
-        } else {
-#pragma unroll
-          for (int b = 0; b < 2; ++b) {
-            const int col = n0 + P::col_of(b, j);
-            if (col >= N) continue;
-            const tile::f32x4 v = p.acc[a][b][i][j];
-            if constexpr (OUT == OUT_PARTS)
-              *reinterpret_cast<tile::f32x4*>(
-                  static_cast<float*>(out) +
-                  (int64_t(split) * M + row) * N + col) = v;
-            else
-              *reinterpret_cast<uint2*>(static_cast<uint16_t*>(out) +
-                                        int64_t(row) * N + col) =
-                  uint2{pack2(v[0], v[1]), pack2(v[2], v[3])};
-          }
+          const uint4 eight = P::eight(v[0], v[1]);
+          const int col = panel * (SILU ? TN / 2 : TN) + P::eight_of(b, j);
+          if (row < M && col < wide)
+            *reinterpret_cast<uint4*>(static_cast<uint16_t*>(out) +
+                                      int64_t(row) * wide + col) = eight;
         }
-      }
     }
+  }
 }
 
 template <int MH, int NH, int OUT>

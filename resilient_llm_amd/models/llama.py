@@ -75,9 +75,11 @@ def _linear_parts(x, w):
 
 def _linear_relu2(x, w):
     """relu2 of _linear."""
-    if (not _USE_SKINNY and not lt_autotune.enabled() and ops.rows_fit(x, w)
-            and ops.rows_whole(x, w)):
-        return ops.rows_linear_relu2(x, w)
+    if not _USE_SKINNY and not lt_autotune.enabled():
+        if ops.tile_relu2_fit(x, w):
+            return ops.tile_linear_relu2(x, w)
+        if ops.rows_fit(x, w) and ops.rows_whole(x, w):
+            return ops.rows_linear_relu2(x, w)
     return ops.relu2(_linear(x, w))
 
 

@@ -442,6 +442,23 @@ def tile_linear_silu(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     return torch.ops.rlli.tile_linear_silu(x, w)
 
 
+def tile_relu2_fit(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether tile_linear_relu2 takes x w^T and is faster than the library and
+    relu2.  (us, those first: 6144 x 2048, 128 rows 16 and 17, 192 21 and 18,
+    600 26 and 20, 2048 53 and 41, 7613 170 and 149; 4096 x 2048, 192 rows 19
+    and 16.5, 1024 26 and 20; 12288 x 4096, 192 rows 45 and 39, 2048 174 and
+    164, 8000 613 and 608; 8192 x 4096, 160 rows 33 and 36.)"""
+    return (x.dim() == 2 and x.is_cuda and 192 <= x.shape[0] <= 8000
+            and x.shape[1] >= 1024 and w.shape[0] >= 4096
+            and _tiles_take(x, w))
+
+
+def tile_linear_relu2(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """rows_linear_relu2 for more rows."""
+    _gpu()
+    return torch.ops.rlli.tile_linear_relu2(x, w)
+
+
 def skinny_linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """rows_linear for K % 256 == 0 and N % 64 == 0."""
     if x.is_cuda:

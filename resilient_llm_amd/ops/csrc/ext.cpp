@@ -766,23 +766,34 @@ Tensor tile_linear_parts(const Tensor& x, const Tensor& w) {
                      : at::empty({M, N}, x.options());
   rlli::launch_tile_gemm(bf16_ptr(x), bf16_ptr(w),
                          parts ? out.data_ptr<float>() : nullptr,
-                         parts ? nullptr : bf16_ptr(out), M, N, K, false, plan,
-                         current_stream(x));
+                         parts ? nullptr : bf16_ptr(out), M, N, K,
+                         rlli::TileAct::none, plan, current_stream(x));
   check_launch("tile_linear_parts");
+  return out;
+}
+
+static Tensor tile_linear_act(const Tensor& x, const Tensor& w,
+                              rlli::TileAct act) {
+  const bool silu = act == rlli::TileAct::silu;
+  check_tiles(x, w, silu ? 16 : 8);
+  const int M = int(x.size(0)), N = int(w.size(0)), K = int(x.size(1));
+  c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
+  Tensor out = at::empty({M, silu ? N / 2 : N}, x.options());
+  rlli::launch_tile_gemm(bf16_ptr(x), bf16_ptr(w), nullptr, bf16_ptr(out), M,
+                         N, K, act, rlli::tile_gemm_plan(M, N, K, true),
+                         current_stream(x));
+  check_launch("tile_linear");
   return out;
 }
 
 // silu(x w[:I]^T) * (x w[I:]^T) for w [2 I, K]
 Tensor tile_linear_silu(const Tensor& x, const Tensor& w) {
-  check_tiles(x, w, 16);
-  const int M = int(x.size(0)), N = int(w.size(0)), K = int(x.size(1));
-  c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
-  Tensor out = at::empty({M, N / 2}, x.options());
-  rlli::launch_tile_gemm(bf16_ptr(x), bf16_ptr(w), nullptr, bf16_ptr(out), M,
-                         N, K, true, rlli::tile_gemm_plan(M, N, K, true),
-                         current_stream(x));
-  check_launch("tile_linear_silu");
-  return out;
+  return tile_linear_act(x, w, rlli::TileAct::silu);
+}
+
+// the squared positive part of x w^T, of the f32 sums
+Tensor tile_linear_relu2(const Tensor& x, const Tensor& w) {
+  return tile_linear_act(x, w, rlli::TileAct::relu2);
 }
 
 // The same under the names and limits of earlier kernels; ``splitk`` has no
@@ -912,6 +923,7 @@ TORCH_LIBRARY(rlli, m) {
         "float eps, Tensor w, bool silu) -> (Tensor, Tensor)");
   m.def("tile_linear_parts(Tensor x, Tensor w) -> Tensor");
   m.def("tile_linear_silu(Tensor x, Tensor w) -> Tensor");
+  m.def("tile_linear_relu2(Tensor x, Tensor w) -> Tensor");
   m.def("skinny_linear(Tensor x, Tensor w) -> Tensor");
   m.def("skinny2_linear(Tensor x, Tensor w, int splitk) -> Tensor");
   m.def("skinny2_silu_linear(Tensor gu, Tensor w, int splitk) -> Tensor");
@@ -949,6 +961,7 @@ TORCH_LIBRARY_IMPL(rlli, CUDA, m) {
   m.impl("rows_norm_linear", &rows_norm_linear);
   m.impl("tile_linear_parts", &tile_linear_parts);
   m.impl("tile_linear_silu", &tile_linear_silu);
+  m.impl("tile_linear_relu2", &tile_linear_relu2);
   m.impl("skinny_linear", &skinny_linear);
   m.impl("skinny2_linear", &skinny2_linear);
   m.impl("skinny2_silu_linear", &skinny2_silu_linear);

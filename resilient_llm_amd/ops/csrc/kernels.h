@@ -149,15 +149,17 @@ void launch_sum_parts(const float* parts, uint16_t* out, int splits,
                       int64_t n, hipStream_t stream);
 
 // The same product of more rows (tile_gemm.hip): f32 parts [splits, M, N] or, if
-// the plan does not divide K, out [M, N]; with ``silu`` out [M, N / 2] of w's
-// gate and up rows.  K % 64 == 0, N % 8 == 0 (16 with silu), 16-byte aligned
-// rows, operands below 2^32 bytes.
+// the plan does not divide K, out [M, N]; with an activation, which wants the
+// product ``whole``, out [M, N / 2] of w's gate and up rows or its squared
+// positive part.  K % 64 == 0, N % 8 == 0 (16 with silu), 16-byte aligned rows,
+// operands below 2^32 bytes.
 struct TilePlan {
   int mh, nh, splits;
 };
-TilePlan tile_gemm_plan(int M, int N, int K, bool silu);
+enum class TileAct { none, silu, relu2 };
+TilePlan tile_gemm_plan(int M, int N, int K, bool whole);
 void launch_tile_gemm(const uint16_t* x, const uint16_t* w, float* parts,
-                      uint16_t* out, int M, int N, int K, bool silu,
+                      uint16_t* out, int M, int N, int K, TileAct act,
                       const TilePlan& plan, hipStream_t stream);
 
 // Diagnostic: W streamed past the caches, 64 rows by a part of K per workgroup.

@@ -21,7 +21,7 @@ namespace {
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 b16x2 __attribute__((ext_vector_type(2)));
 
-enum { OUT_PARTS = 0, OUT_BF16 = 1, OUT_SILU = 2 };
+enum { OUT_PARTS = 0, OUT_BF16 = 1, OUT_SILU = 2, OUT_RELU2 = 3 };
 
 DEV_INLINE uint32_t pack2(float a, float b) {
   const b16x2 v = __builtin_convertvector((f32x2{a, b}), b16x2);
@@ -100,6 +100,13 @@ void tile_gemm_kernel(const uint16_t* __restrict__ x,
               for (int r = 0; r < 4; ++r)
                 f[r] = f[r] / (1.f + __expf(-f[r])) * p.acc[a][1][i][j][r];
             }
+            if constexpr (OUT == OUT_RELU2) {
+#pragma unroll
+              for (int r = 0; r < 4; ++r) {
+                f[r] = fmaxf(f[r], 0.f);
+                f[r] *= f[r];
+              }
+            }
             v[a] = uint2{pack2(f[0], f[1]), pack2(f[2], f[3])};
           }
           const uint4 eight = P::eight(v[0], v[1]);
@@ -146,14 +153,14 @@ constexpr int MOST_SPLITS = 8;
 // workgroups, each with its steps, and 0.6 us for each megabyte of parts that
 // is written and read again.  (Over seven shapes at 14 numbers of rows from 132
 // to 2048 what it chose took 2 % more than the best did.)
-TilePlan tile_gemm_plan(int M, int N, int K, bool silu) {
+TilePlan tile_gemm_plan(int M, int N, int K, bool whole) {
   TilePlan best{};
   float least = 0.f;
   const int steps = K / tile::KS;
   for (const Tile& t : TILES) {
     const int rows = (M + 64 * t.mh - 1) / (64 * t.mh);
     const int tiles = rows * ((N + 128 * t.nh - 1) / (128 * t.nh));
-    for (int s = 1; s <= (silu ? 1 : std::min(MOST_SPLITS, steps)); ++s) {
+    for (int s = 1; s <= (whole ? 1 : std::min(MOST_SPLITS, steps)); ++s) {
       const int rounds = (tiles * s + 255) / 256;
       const float parts = s > 1 ? float(s) * M * N * 4e-6f : 0.f;
       const float us =
@@ -168,12 +175,14 @@ TilePlan tile_gemm_plan(int M, int N, int K, bool silu) {
 }
 
 void launch_tile_gemm(const uint16_t* x, const uint16_t* w, float* parts,
-                      uint16_t* out, int M, int N, int K, bool silu,
+                      uint16_t* out, int M, int N, int K, TileAct act,
                       const TilePlan& plan, hipStream_t st) {
   auto run = [&](auto m, auto n) {
     constexpr int MH = decltype(m)::value, NH = decltype(n)::value;
-    if (silu)
+    if (act == TileAct::silu)
       go<MH, NH, OUT_SILU>(x, w, out, M, N, K, 1, st);
+    else if (act == TileAct::relu2)
+      go<MH, NH, OUT_RELU2>(x, w, out, M, N, K, 1, st);
     else if (parts)
       go<MH, NH, OUT_PARTS>(x, w, parts, M, N, K, plan.splits, st);
     else

@@ -57,6 +57,16 @@ def test_tile_linear_silu(M, N, K):
                                atol=2 ** -16)
 
 
+@pytest.mark.parametrize("M,N,K", SIZES)
+def test_tile_linear_relu2(M, N, K):
+    x, w = operands(M, N, K, 3)
+    got = torch.ops.rlli.tile_linear_relu2(x, w)
+    want = (x.double() @ w.double().T).clamp(min=0) ** 2
+    # the square doubles a sum's error and scales it by the sum, five or so
+    torch.testing.assert_close(got.double(), want, rtol=2 ** -8,
+                               atol=2 ** -14)
+
+
 def test_same_bits_in_every_pass():
     x, w = operands(536, 4096, 4096, 2)
     first = torch.ops.rlli.tile_linear_parts(x, w)

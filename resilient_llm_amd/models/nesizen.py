@@ -359,9 +359,10 @@ class NesizenForCausalLM(MixedModel):
         return y
 
     def _last(self, x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
-        """A sublayer's output; f32 parts where the kernel divides K and
-        hyper_step is the one to read them."""
-        if self.tp_world > 1 or (ops.rows_fit(x, w) and ops.rows_whole(x, w)):
+        """A sublayer's output; of few rows f32 parts where the kernel divides
+        K and hyper_step is the one to read them."""
+        if (self.tp_world > 1 or not ops.rows_fit(x, w)
+                or ops.rows_whole(x, w)):
             return _linear(x, w)
         return _linear_parts(x, w)
 

@@ -454,7 +454,7 @@ def tile_relu2_fit(x: torch.Tensor, w: torch.Tensor) -> bool:
 
 
 def tile_linear_relu2(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
-    """rows_linear_relu2 for more rows."""
+    """relu2(x w^T), of the 16-bit product."""
     _gpu()
     return torch.ops.rlli.tile_linear_relu2(x, w)
 

@@ -791,7 +791,7 @@ Tensor tile_linear_silu(const Tensor& x, const Tensor& w) {
   return tile_linear_act(x, w, rlli::TileAct::silu);
 }
 
-// the squared positive part of x w^T, of the f32 sums
+// the squared positive part of the 16-bit x w^T
 Tensor tile_linear_relu2(const Tensor& x, const Tensor& w) {
   return tile_linear_act(x, w, rlli::TileAct::relu2);
 }

@@ -101,9 +101,11 @@ void tile_gemm_kernel(const uint16_t* __restrict__ x,
                 f[r] = f[r] / (1.f + __expf(-f[r])) * p.acc[a][1][i][j][r];
             }
             if constexpr (OUT == OUT_RELU2) {
+              // of the 16-bit product: a prompt's first tokens can turn any
+              // difference to the product and relu2 apart into large ones
 #pragma unroll
               for (int r = 0; r < 4; ++r) {
-                f[r] = fmaxf(f[r], 0.f);
+                f[r] = fmaxf(bf16_to_f32(f32_to_bf16(f[r])), 0.f);
                 f[r] *= f[r];
               }
             }

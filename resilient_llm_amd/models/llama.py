@@ -431,8 +431,30 @@ class LlamaForCausalLM:
             return ops.prefill_attn_qkv(qkv, cu_seqlens, self.scale,
                                         self.n_heads, self.n_kv_heads,
                                         self.config.head_dim)
+
+        def layer(i, x, residual):
+            p = self.params
+            names = ("ln1", "qkv", "o", "ln2", "gate_up", "down")
+            return ops.prompt_rows_layer(
+                x, residual, *(p[f"l{i}.{n}"] for n in names), positions,
+                self.cos_sin, *kv_cache.layer(i), slot_mapping, cu_seqlens,
+                self.config.rms_eps, self.scale, self.n_heads)
         return self._forward(input_ids, positions, kv_cache, slot_mapping,
-                             attn, last_idx=cu_seqlens[1:].long() - 1)
+                             attn, last_idx=cu_seqlens[1:].long() - 1,
+                             layer=layer if self._prompt_rows(
+                                 input_ids.shape[0]) else None)
+
+    def _prompt_rows(self, rows: int) -> bool:
+        """Whether ops.prompt_rows_layer launches what _layer would."""
+        c = self.config
+        return (self.device.type == "cuda" and self.dtype == torch.bfloat16
+                and 0 < rows <= 64 and self.tp_world == 1
+                and self.quant is None and c.hidden_size <= 8192
+                and not _USE_SKINNY and not lt_autotune.enabled()
+                and not any(w.requires_grad for w in self.params.values())
+                and ops.rows_faster(rows, *(
+                    self.params[f"l0.{n}"].shape
+                    for n in ("qkv", "o", "gate_up", "down"))))
 
     def forward_mixed(self, input_ids: torch.Tensor, positions: torch.Tensor,
                       kv_cache, slot_mapping: torch.Tensor, n_decode: int,
@@ -496,12 +518,17 @@ class LlamaForCausalLM:
                              attn, last_idx=None, qkv_parts=True)
 
     def _forward(self, input_ids, positions, kv_cache, slot_mapping, attn_fn,
-                 last_idx, qkv_parts: bool = False) -> torch.Tensor:
-        """``qkv_parts``: attn_fn takes the product in parts."""
+                 last_idx, qkv_parts: bool = False,
+                 layer=None) -> torch.Tensor:
+        """``qkv_parts``: attn_fn takes the product in parts.  ``layer``: all of
+        a layer but the first at once."""
         p = self.params
         x = F.embedding(input_ids.long(), p["embed"])
         residual = None
         for i in range(self.config.n_layers):
+            if layer is not None and i > 0:
+                x = layer(i, x, residual)
+                continue
             x, residual = self._layer(i, x, residual, positions, kv_cache,
                                       slot_mapping, attn_fn, qkv_parts)
         if self.quant == "fp8":

@@ -226,6 +226,26 @@ def mixed_row_tables(rows: int, n_decode: int, tables_dec, lens_dec,
                                 chunk_btrow, tables_pre)
 
 
+def rows_faster(M: int, *shapes) -> bool:
+    """Whether M rows' products with weights of these shapes are rows_linear's,
+    as far as the shapes go."""
+    return all(K % 64 == 0 and N % 16 == 0 and _rows_faster(M, N, K)
+               for N, K in shapes)
+
+
+def prompt_rows_layer(x, residual, ln1, w_qkv, w_o, ln2, w_gate_up, w_down,
+                      positions, cos_sin, k_cache, v_cache, slot_mapping,
+                      cu_seqlens, eps: float, scale: float,
+                      n_q: int) -> torch.Tensor:
+    """A Llama layer behind the first for few rows of whole prompts on the GPU:
+    x + residual, normed, ... the last product, which may come in parts;
+    residual is updated.  The launches are those of the ops one by one."""
+    _gpu()
+    return torch.ops.rlli.prompt_rows_layer(
+        x, residual, ln1, w_qkv, w_o, ln2, w_gate_up, w_down, positions,
+        cos_sin, k_cache, v_cache, slot_mapping, cu_seqlens, eps, scale, n_q)
+
+
 def prefill_attn_qkv(qkv: torch.Tensor, cu_seqlens: torch.Tensor,
                      scale: float, n_q: int, n_kv: int,
                      head_dim: int) -> torch.Tensor:

@@ -1,0 +1,54 @@
+"""Short prompts' layers launched at once: the same bits as op by op, weights
+that the kernels for few rows do not take included."""
+
+import pytest
+import torch
+
+from resilient_llm_amd.engine import LLMEngine, PagedKVCache
+from resilient_llm_amd.models import LlamaForCausalLM, get_config
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def feed(model, prompts, at_once, kv_dtype):
+    kv = PagedKVCache.for_model(model.config, 16, device=DEV,
+                                kv_dtype=kv_dtype)
+    kv.k.zero_()
+    kv.v.zero_()
+    engine = LLMEngine(model, kv, max_batch_size=4)
+    model._prompt_rows, kept = at_once, model._prompt_rows
+    try:
+        logits = engine.feed([(str(i), p, [len(p) - 1])
+                              for i, p in enumerate(prompts)])
+    finally:
+        model._prompt_rows = kept
+    return [logits] + [t.view(torch.uint8) for t in (kv.k, kv.v)]
+
+
+@pytest.mark.parametrize("kv_dtype", [torch.bfloat16, torch.float8_e4m3fn])
+@pytest.mark.parametrize("name", ["tiny", "tiny-128"])
+@pytest.mark.parametrize("lens", [[1], [33], [20, 1, 43]], ids=str)
+@pytest.mark.parametrize("shifted", [None, "qkv", "o", "gate_up", "down"])
+def test_same_bits(name, lens, shifted, kv_dtype):
+    model = LlamaForCausalLM(get_config(name), device=DEV,
+                             dtype=torch.bfloat16, seed=1)
+    assert model._prompt_rows(sum(lens))
+    if shifted:
+        w = model.params[f"l1.{shifted}"]
+        buf = torch.empty(w.numel() + 1, dtype=w.dtype, device=DEV)
+        model.params[f"l1.{shifted}"] = buf[1:].view(w.shape).copy_(w)
+    prompts = [[(7 * i + n) % 500 + 5 for i in range(n)] for n in lens]
+    one, apart = (feed(model, prompts, lambda rows: x, kv_dtype)
+                  for x in (True, False))
+    for a, b in zip(one, apart):
+        assert torch.equal(a, b)
+
+
+def test_which_prompts():
+    model = LlamaForCausalLM(get_config("tiny"), device=DEV,
+                             dtype=torch.bfloat16)
+    assert model._prompt_rows(64) and not model._prompt_rows(65)
+    assert not model._prompt_rows(0)
+    model.params["l1.o"].requires_grad_()
+    assert not model._prompt_rows(8)

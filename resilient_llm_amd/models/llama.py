@@ -48,6 +48,8 @@ def _linear(x, w):
     if (lt_autotune.enabled() and x.is_cuda and x.dim() == 2
             and x.shape[0] in _LT_ROWS):
         return lt_autotune.tuned_linear(x, w)
+    if ops.tile_linear_fit(x, w):
+        return ops.tile_linear(x, w)
     if ops.rows_fit(x, w):
         return ops.rows_linear(x, w)
     return F.linear(x, w)

@@ -444,6 +444,27 @@ def tile_linear_parts(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     return torch.ops.rlli.tile_linear_parts(x, w)
 
 
+def tile_linear_fit(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether tile_linear takes x w^T and is the faster way.  (us, the other
+    way first, rows_linear up to 128 rows and the library from there: 6144 x
+    4096, 65 rows 20 and 17, 129 39 and 23, 160 25 and 24, but 200 23 and 25;
+    4096 x 4096, 128 rows 19 and 15.5, 160 23 and 17; 10240 x 8192, 65 rows 77
+    and 40, 129 57 and 49, 256 88 and 56, 257 64 and 64; 5120 x 5120, 65 rows
+    20 and 18, 250 32 and 28, 288 30 and 30; 12288 x 4096, 128 rows 32 and 35;
+    3072 x 2048, 128 rows 12 and 14.)"""
+    if x.dim() != 2 or not x.is_cuda:
+        return False
+    (M, K), N = x.shape, w.shape[0]
+    return (64 < M <= (256 if K > 4096 else 160) and K >= 4096
+            and 4096 <= N <= 10240 and _tiles_take(x, w))
+
+
+def tile_linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """rows_linear for more rows."""
+    _gpu()
+    return torch.ops.rlli.tile_linear(x, w)
+
+
 def tile_silu_fit(x: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether tile_linear_silu takes x w^T and is faster than the library and
     silu_mul.  (us, those first: 28672 x 4096, 160 rows 64 and 68, 192 66 and

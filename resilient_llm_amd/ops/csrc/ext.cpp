@@ -772,6 +772,18 @@ Tensor tile_linear_parts(const Tensor& x, const Tensor& w) {
   return out;
 }
 
+// the whole product in bf16
+Tensor tile_linear(const Tensor& x, const Tensor& w) {
+  const Tensor parts = tile_linear_parts(x, w);
+  if (parts.dim() == 2) return parts;
+  c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
+  Tensor out = at::empty({x.size(0), w.size(0)}, x.options());
+  rlli::launch_sum_parts(parts.data_ptr<float>(), bf16_ptr(out),
+                         int(parts.size(0)), out.numel(), current_stream(x));
+  check_launch("sum_parts");
+  return out;
+}
+
 static Tensor tile_linear_act(const Tensor& x, const Tensor& w,
                               rlli::TileAct act) {
   const bool silu = act == rlli::TileAct::silu;
@@ -971,6 +983,7 @@ TORCH_LIBRARY(rlli, m) {
   m.def("rows_norm_linear(Tensor parts, Tensor residual, Tensor gain, "
         "float eps, Tensor w, bool silu) -> (Tensor, Tensor)");
   m.def("tile_linear_parts(Tensor x, Tensor w) -> Tensor");
+  m.def("tile_linear(Tensor x, Tensor w) -> Tensor");
   m.def("tile_linear_silu(Tensor x, Tensor w) -> Tensor");
   m.def("tile_linear_relu2(Tensor x, Tensor w) -> Tensor");
   m.def("skinny_linear(Tensor x, Tensor w) -> Tensor");
@@ -1010,6 +1023,7 @@ TORCH_LIBRARY_IMPL(rlli, CUDA, m) {
   m.impl("rows_linear_relu2", &rows_linear_relu2);
   m.impl("rows_norm_linear", &rows_norm_linear);
   m.impl("tile_linear_parts", &tile_linear_parts);
+  m.impl("tile_linear", &tile_linear);
   m.impl("tile_linear_silu", &tile_linear_silu);
   m.impl("tile_linear_relu2", &tile_linear_relu2);
   m.impl("skinny_linear", &skinny_linear);

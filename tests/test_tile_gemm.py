@@ -47,6 +47,19 @@ def test_tile_linear_parts(M, N, K):
 
 
 @pytest.mark.parametrize("M,N,K", SIZES)
+def test_tile_linear(M, N, K):
+    x, w = operands(M, N, K, 4)
+    got = torch.ops.rlli.tile_linear(x, w)
+    parts = torch.ops.rlli.tile_linear_parts(x, w)
+    if parts.dim() == 3:
+        want = parts[0].clone()
+        for p in parts[1:]:
+            want += p
+        parts = want.to(torch.bfloat16)
+    assert torch.equal(got, parts)
+
+
+@pytest.mark.parametrize("M,N,K", SIZES)
 def test_tile_linear_silu(M, N, K):
     x, w = operands(M, N - N % 16, K, 1)
     got = torch.ops.rlli.tile_linear_silu(x, w)

@@ -390,7 +390,8 @@ class LlamaForCausalLM:
 
     def _layer(self, i: int, x: torch.Tensor, residual: Optional[torch.Tensor],
                positions: torch.Tensor, kv_cache, slot_mapping: torch.Tensor,
-               attn_fn, qkv_parts: bool) -> tuple[torch.Tensor, torch.Tensor]:
+               attn_fn, qkv_parts: bool,
+               attn_out_fn=None) -> tuple[torch.Tensor, torch.Tensor]:
         p = self.params
         c = self.config
         # what the next norm adds to the residual may come in parts, if
@@ -408,8 +409,11 @@ class LlamaForCausalLM:
         k_cache, v_cache = kv_cache.layer(i)
         # rope + cache append happen inside attn_fn (the decode path fuses
         # them into the attention kernel itself)
-        attn_out = attn_fn(i, qkv, k_cache, v_cache)   # [T, q_size]
-        h = self._all_reduce(out(attn_out, p[f"l{i}.o"]))
+        if attn_out_fn is not None:
+            h = attn_out_fn(i, qkv, k_cache, v_cache)
+        else:
+            attn_out = attn_fn(i, qkv, k_cache, v_cache)   # [T, q_size]
+            h = self._all_reduce(out(attn_out, p[f"l{i}.o"]))
         if self.quant == "fp8":
             h2q, h2s = ops.rmsnorm_residual_fp8(h, residual, p[f"l{i}.ln2"],
                                                 c.rms_eps)
@@ -447,7 +451,8 @@ class LlamaForCausalLM:
                                  input_ids.shape[0]) else None)
 
     def _prompt_rows(self, rows: int) -> bool:
-        """Whether ops.prompt_rows_layer launches what _layer would."""
+        """Whether ops.prompt_rows_layer (and decode_attn_rope_linear) launches
+        what _layer would."""
         c = self.config
         return (self.device.type == "cuda" and self.dtype == torch.bfloat16
                 and 0 < rows <= 64 and self.tp_world == 1
@@ -516,14 +521,23 @@ class LlamaForCausalLM:
             return ops.decode_attn_rope_qkv(
                 qkv, positions, self.cos_sin, k_cache, v_cache, slot_mapping,
                 block_tables, seq_lens, self.scale, self.n_heads)
+
+        def attn_out(i, qkv, k_cache, v_cache):
+            return ops.decode_attn_rope_linear(
+                qkv, positions, self.cos_sin, k_cache, v_cache, slot_mapping,
+                block_tables, seq_lens, self.scale, self.n_heads,
+                self.params[f"l{i}.o"])
         return self._forward(input_ids, positions, kv_cache, slot_mapping,
-                             attn, last_idx=None, qkv_parts=True)
+                             attn, last_idx=None, qkv_parts=True,
+                             attn_out_fn=attn_out if input_ids.shape[0] == 1
+                             and self._prompt_rows(1) else None)
 
     def _forward(self, input_ids, positions, kv_cache, slot_mapping, attn_fn,
-                 last_idx, qkv_parts: bool = False,
-                 layer=None) -> torch.Tensor:
+                 last_idx, qkv_parts: bool = False, layer=None,
+                 attn_out_fn=None) -> torch.Tensor:
         """``qkv_parts``: attn_fn takes the product in parts.  ``layer``: all of
-        a layer but the first at once."""
+        a layer but the first at once.  ``attn_out_fn``: attention and the
+        product behind it."""
         p = self.params
         x = F.embedding(input_ids.long(), p["embed"])
         residual = None
@@ -532,7 +546,8 @@ class LlamaForCausalLM:
                 x = layer(i, x, residual)
                 continue
             x, residual = self._layer(i, x, residual, positions, kv_cache,
-                                      slot_mapping, attn_fn, qkv_parts)
+                                      slot_mapping, attn_fn, qkv_parts,
+                                      attn_out_fn)
         if self.quant == "fp8":
             h8, hs = ops.rmsnorm_residual_fp8(x, residual, p["final_ln"],
                                               self.config.rms_eps)

@@ -193,6 +193,17 @@ def decode_attn_rope_qkv(qkv, positions, cos_sin, k_cache, v_cache,
                            scale, n_q)
 
 
+def decode_attn_rope_linear(qkv, positions, cos_sin, k_cache, v_cache,
+                            slot_mapping, block_table, seq_lens, scale: float,
+                            n_q: int, w: torch.Tensor) -> torch.Tensor:
+    """rows_linear_parts of decode_attn_rope_qkv's result with w.  Of one long
+    sequence the product puts its parts together, without a launch for it."""
+    _gpu()
+    return torch.ops.rlli.decode_attn_rope_linear(
+        qkv, positions, cos_sin, k_cache, v_cache, slot_mapping, block_table,
+        seq_lens, scale, n_q, w)
+
+
 def decode_attn_rows_qkv(qkv, positions, cos_sin, k_cache, v_cache,
                          slot_mapping, block_table, seq_lens, scale: float,
                          n_q: int) -> torch.Tensor:

@@ -42,6 +42,7 @@
 // so nothing waits for the append.  Without slots it rotates queries only.
 
 #include "common.h"
+#include "decode_parts.h"
 #include "kernels.h"
 
 #include <algorithm>
@@ -55,9 +56,7 @@ namespace {
 typedef short s16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-constexpr float kNegInf = -1e30f;
-constexpr int UNIT = 32;          // tokens
-constexpr int MIN_UNITS = 8;      // of a part: two per wave
+using namespace decode;
 
 struct DecodeArgs {
   const uint16_t* q;       // rows q_stride apart: q heads (| k | v: fused)
@@ -74,9 +73,8 @@ struct DecodeArgs {
   float* part_ml;          //         [.., GROUP, 2]
   int batch, n_kv, block_size, max_blocks, q_stride, n_parts, shares;
   float scale;
+  bool apart;              // whoever reads the parts puts them together
 };
-
-DEV_INLINE int units_of(int len) { return (len + UNIT - 1) / UNIT; }
 
 // How many units a part may have, so that ``shares`` parts cover all
 // sequences (each ends in one that is not full).
@@ -86,12 +84,7 @@ DEV_INLINE int part_size(const DecodeArgs& a) {
     t += units_of(a.seq_lens[s]);
 #pragma unroll
   for (int d = 1; d < 64; d <<= 1) t += __shfl_xor(t, d, kWave);
-  return max((__builtin_amdgcn_readfirstlane(t) + a.shares - 1) / a.shares,
-             MIN_UNITS);
-}
-
-DEV_INLINE int parts_of(int len, int size) {
-  return (units_of(len) + size - 1) / size;
+  return part_size_of(__builtin_amdgcn_readfirstlane(t), a.shares);
 }
 
 // Parts of the sequences ahead of ``seq``.
@@ -696,6 +689,7 @@ void run(const DecodeArgs& a, hipStream_t st) {
       hipLaunchKernelGGL((decode_attn_kernel<D, GROUP, KC, BS, FUSED, true>),
                          dim3((a.shares + a.batch) * a.n_kv), dim3(256), 0, st,
                          a);
+      if (a.apart) return;
       hipLaunchKernelGGL((decode_combine_kernel<D, GROUP>),
                          dim3(a.batch * a.n_kv * GROUP), dim3(256), 0, st, a);
     } else {
@@ -750,11 +744,11 @@ void launch_decode_attn(
     const int32_t* slot_mapping, uint16_t* out, int batch, int n_q_heads,
     int n_kv_heads, int head_dim, int block_size, int max_blocks, float scale,
     int q_stride, int shares, float* part_out, float* part_ml, bool cache_fp8,
-    hipStream_t stream) {
+    bool apart, hipStream_t stream) {
   const DecodeArgs a{q, parts, k_cache, v_cache, k_cache, v_cache,
                      block_table, seq_lens, positions, cos_sin, slot_mapping,
                      out, part_out, part_ml, batch, n_kv_heads, block_size,
-                     max_blocks, q_stride, n_parts, shares, scale};
+                     max_blocks, q_stride, n_parts, shares, scale, apart};
   const int group = n_q_heads / n_kv_heads;
   if (positions) dispatch<true>(a, group, head_dim, cache_fp8, stream);
   else dispatch<false>(a, group, head_dim, cache_fp8, stream);

@@ -283,6 +283,17 @@ void kv_append_qkv_(Tensor qkv, const Tensor& positions,
 }
 
 // ---------------------------------------------------------- decode_attn
+Tensor rows_linear_parts(const Tensor& x, const Tensor& w);
+
+// whether rows_linear takes x w^T
+static bool rows_take(const Tensor& x, const Tensor& w) {
+  return w.scalar_type() == at::kBFloat16 && w.is_contiguous() &&
+         x.is_contiguous() && w.device() == x.device() &&
+         x.size(1) % 64 == 0 && w.size(0) % 16 == 0 &&
+         (reinterpret_cast<uintptr_t>(x.data_ptr()) |
+          reinterpret_cast<uintptr_t>(w.data_ptr())) % 16 == 0;
+}
+
 // One launch for all forms.  q: bf16 rows that start with the query heads
 // ([batch, .., stride]), or f32 parts [n, batch, stride] whose sum they are.
 // With ``positions`` queries are rotated here; with ``slot_mapping`` as well
@@ -293,7 +304,8 @@ static Tensor decode_attn_any(const Tensor& q, int64_t n_q,
                               const Tensor& seq_lens, double scale,
                               const Tensor* positions, const Tensor* cos_sin,
                               const Tensor* slot_mapping,
-                              const Tensor* into = nullptr) {
+                              const Tensor* into = nullptr,
+                              const Tensor* w_next = nullptr) {
   const bool parts = q.scalar_type() == at::kFloat;
   if (parts) {
     TORCH_CHECK(q.is_cuda() && q.is_contiguous() && q.dim() == 3 &&
@@ -347,6 +359,11 @@ static Tensor decode_attn_any(const Tensor& q, int64_t n_q,
     part = at::empty({slots, D}, opt);
     ml = at::empty({slots, 2}, opt);
   }
+  // of one row, the product behind it puts the shares together
+  const int K = int(n_q) * D, N = w_next ? int(w_next->size(0)) : 0;
+  const bool apart = w_next && shares > 0 && batch == 1 &&
+                     rows_take(out, *w_next) && w_next->size(1) == K &&
+                     rlli::rows_norm_ok(N, K, false);
   rlli::launch_decode_attn(
       parts ? nullptr : bf16_ptr(q), parts ? q.data_ptr<float>() : nullptr,
       parts ? int(q.size(0)) : 0, k_cache.data_ptr(), v_cache.data_ptr(),
@@ -357,10 +374,22 @@ static Tensor decode_attn_any(const Tensor& q, int64_t n_q,
       bf16_ptr(out), batch, int(n_q), n_kv, D, block_size, max_blocks,
       float(scale), stride, shares,
       shares > 0 ? part.data_ptr<float>() : nullptr,
-      shares > 0 ? ml.data_ptr<float>() : nullptr, cache_fp8,
+      shares > 0 ? ml.data_ptr<float>() : nullptr, cache_fp8, apart,
       current_stream(q));
   check_launch("decode_attn");
-  return out;
+  if (!w_next) return out;
+  if (!apart)
+    return rows_take(out, *w_next) ? rows_linear_parts(out, *w_next)
+                                   : at::linear(out, *w_next);
+  const int splits = rlli::rows_gemm_splits(N, K);
+  Tensor y = at::empty({splits, 1, N}, out.options().dtype(at::kFloat));
+  rlli::launch_rows_combine(
+      rlli::RowsCombine{part.data_ptr<float>(), ml.data_ptr<float>(),
+                        bf16_ptr(out), seq_lens.data_ptr<int32_t>(), shares,
+                        group, D},
+      bf16_ptr(*w_next), y.data_ptr<float>(), N, K, splits, current_stream(q));
+  check_launch("rows_combine");
+  return y;
 }
 
 Tensor decode_attn(const Tensor& q, const Tensor& k_cache,
@@ -408,13 +437,9 @@ void decode_attn_qkv_out(const Tensor& qkv, const Tensor& k_cache,
                   nullptr, nullptr, nullptr, &out);
 }
 
-// Fused decode: rope + append + attention in one kernel.  qkv: bf16 rows, or
-// the f32 parts of rows_linear_parts.
-Tensor decode_attn_rope_qkv(const Tensor& qkv, const Tensor& positions,
-                            const Tensor& cos_sin, Tensor k_cache,
-                            Tensor v_cache, const Tensor& slot_mapping,
-                            const Tensor& block_table, const Tensor& seq_lens,
-                            double scale, int64_t n_q) {
+static void check_rope_qkv(const Tensor& qkv, const Tensor& positions,
+                           const Tensor& cos_sin, const Tensor& k_cache,
+                           const Tensor& slot_mapping, int64_t n_q) {
   TORCH_CHECK(positions.scalar_type() == at::kInt && positions.is_contiguous());
   TORCH_CHECK(slot_mapping.scalar_type() == at::kInt && slot_mapping.is_contiguous());
   TORCH_CHECK(cos_sin.scalar_type() == at::kFloat && cos_sin.is_contiguous());
@@ -423,8 +448,32 @@ Tensor decode_attn_rope_qkv(const Tensor& qkv, const Tensor& positions,
   const int64_t batch = qkv.size(qkv.dim() == 3 ? 1 : 0);
   TORCH_CHECK(positions.numel() >= batch && slot_mapping.numel() >= batch,
               "positions and slots of ", batch, " sequences are needed");
+}
+
+// Fused decode: rope + append + attention in one kernel.  qkv: bf16 rows, or
+// the f32 parts of rows_linear_parts.
+Tensor decode_attn_rope_qkv(const Tensor& qkv, const Tensor& positions,
+                            const Tensor& cos_sin, Tensor k_cache,
+                            Tensor v_cache, const Tensor& slot_mapping,
+                            const Tensor& block_table, const Tensor& seq_lens,
+                            double scale, int64_t n_q) {
+  check_rope_qkv(qkv, positions, cos_sin, k_cache, slot_mapping, n_q);
   return decode_attn_any(qkv, n_q, k_cache, v_cache, block_table, seq_lens,
                          scale, &positions, &cos_sin, &slot_mapping);
+}
+
+// The product with w of decode_attn_rope_qkv's result, as rows_linear_parts has
+// it.
+Tensor decode_attn_rope_linear(const Tensor& qkv, const Tensor& positions,
+                               const Tensor& cos_sin, Tensor k_cache,
+                               Tensor v_cache, const Tensor& slot_mapping,
+                               const Tensor& block_table,
+                               const Tensor& seq_lens, double scale,
+                               int64_t n_q, const Tensor& w) {
+  check_rope_qkv(qkv, positions, cos_sin, k_cache, slot_mapping, n_q);
+  return decode_attn_any(qkv, n_q, k_cache, v_cache, block_table, seq_lens,
+                         scale, &positions, &cos_sin, &slot_mapping, nullptr,
+                         &w);
 }
 
 // Queries rotated here, everything they see already in the cache.
@@ -892,14 +941,6 @@ static Tensor norm_any(const Tensor& x, const Tensor& residual,
              : rmsnorm_residual_(x, residual, gain, eps);
 }
 
-static bool rows_take(const Tensor& x, const Tensor& w) {
-  return w.scalar_type() == at::kBFloat16 && w.is_contiguous() &&
-         x.is_contiguous() && w.device() == x.device() &&
-         x.size(1) % 64 == 0 && w.size(0) % 16 == 0 &&
-         (reinterpret_cast<uintptr_t>(x.data_ptr()) |
-          reinterpret_cast<uintptr_t>(w.data_ptr())) % 16 == 0;
-}
-
 // All of a Llama layer but the first for the rows of a few short prompts, whose
 // step waits for the host: the ops in their order, launched from here.
 // (A prompt of 45 tokens through 16 layers of 2048: 8 us a launch from Python, 5
@@ -954,6 +995,10 @@ TORCH_LIBRARY(rlli, m) {
   m.def("decode_attn_rope_qkv(Tensor qkv, Tensor positions, Tensor cos_sin, "
         "Tensor(a!) k_cache, Tensor(b!) v_cache, Tensor slot_mapping, "
         "Tensor block_table, Tensor seq_lens, float scale, int n_q) -> Tensor");
+  m.def("decode_attn_rope_linear(Tensor qkv, Tensor positions, "
+        "Tensor cos_sin, Tensor(a!) k_cache, Tensor(b!) v_cache, "
+        "Tensor slot_mapping, Tensor block_table, Tensor seq_lens, "
+        "float scale, int n_q, Tensor w) -> Tensor");
   m.def("kv_append_qkv_(Tensor(a!) qkv, Tensor positions, Tensor cos_sin, "
         "Tensor(b!) k_cache, Tensor(c!) v_cache, Tensor slot_mapping, "
         "int n_q) -> ()");
@@ -1010,6 +1055,7 @@ TORCH_LIBRARY_IMPL(rlli, CUDA, m) {
   m.impl("decode_attn_qkv", &decode_attn_qkv);
   m.impl("decode_attn_qkv_out", &decode_attn_qkv_out);
   m.impl("decode_attn_rope_qkv", &decode_attn_rope_qkv);
+  m.impl("decode_attn_rope_linear", &decode_attn_rope_linear);
   m.impl("kv_append_qkv_", &kv_append_qkv_);
   m.impl("decode_attn_q_rope", &decode_attn_q_rope);
   m.impl("mixed_row_tables", &mixed_row_tables);

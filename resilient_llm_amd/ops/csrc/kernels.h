@@ -56,7 +56,7 @@ void launch_rope_kv_append(
 // decode_attn_shares: equal shares of all sequences' tokens that workgroups
 // take per key/value head, for which part_out [n_kv, shares + batch, group,
 // head_dim] and part_ml [.., group, 2] are needed; 0: a workgroup takes a
-// whole sequence.
+// whole sequence.  ``apart``: sequences that were cut are left in their parts.
 int decode_attn_shares(int batch, int n_kv_heads, int max_tokens);
 void launch_decode_attn(
     const uint16_t* q,                 // [batch, q_stride], or null:
@@ -70,7 +70,7 @@ void launch_decode_attn(
     uint16_t* out,                     // [batch, n_q_heads, head_dim]
     int batch, int n_q_heads, int n_kv_heads, int head_dim, int block_size,
     int max_blocks, float scale, int q_stride, int shares, float* part_out,
-    float* part_ml, bool cache_fp8, hipStream_t stream);
+    float* part_ml, bool cache_fp8, bool apart, hipStream_t stream);
 
 // What says which pages the rows of a mixed step see: decoding sequences
 // first, then tiles of at most 32 prompt rows.
@@ -135,6 +135,17 @@ struct RowsNorm {
   int n;
   float eps;
 };
+// Of one sequence's attention in parts, which launch_decode_attn left apart:
+// its output, at ``whole`` if it was not cut, times w.
+struct RowsCombine {
+  const float *o, *ml;         // as launch_decode_attn has them
+  const uint16_t* whole;       // [K]
+  const int32_t* len;
+  int shares, group, head_dim;
+};
+void launch_rows_combine(const RowsCombine& attn, const uint16_t* w,
+                         float* parts, int N, int K, int splits,
+                         hipStream_t stream);
 bool rows_norm_ok(int N, int K, bool silu);
 void launch_rows_norm(const RowsNorm& norm, const uint16_t* w, float* parts,
                       int N, int K, int splits, hipStream_t stream);

@@ -22,6 +22,7 @@
 // follows from N and K alone.
 
 #include "common.h"
+#include "decode_parts.h"
 #include "kernels.h"
 
 #include <algorithm>
@@ -178,15 +179,91 @@ DEV_INLINE void norm_row(const NormArgs& a, int K, int t, float* sums,
   }
 }
 
+// The same for a decoded row's attention that comes in parts (decode_attn.hip):
+// channels from c0 to c1 of it, put together by whom they are multiplied by
+// anyway.  4096 x 4096 behind 1000 tokens, us: the launch that put them together
+// and the product 4.7 + 7.6, in one 8.6.
+DEV_INLINE void combine_row(const RowsCombine& a, int c0, int c1, int t,
+                            uint16_t* xs) {
+  using namespace decode;
+  constexpr int B = 8;                    // parts whose loads are one batch
+  const int D = a.head_dim, G = a.group;
+  int c = c0 + t * 4;
+  // (parts that there are not are somebody's scratch: read, not used)
+  auto head_of = [&](int ch) { return ch / D; };
+  auto slot = [&](int ch, int p) {
+    const int h = head_of(ch);
+    return (int64_t(h / G) * (a.shares + 1) + p) * G + h % G;
+  };
+  f32x4 v[B];
+  f32x2 ml[B];
+  auto ask = [&](int ch, int p0, int top) {
+#pragma unroll
+    for (int i = 0; i < B; ++i) {
+      const int64_t at = slot(ch, min(p0 + i, top));
+      v[i] = *reinterpret_cast<const f32x4*>(a.o + at * D + ch % D);
+      ml[i] = *reinterpret_cast<const f32x2*>(a.ml + at * 2);
+    }
+  };
+  const int len = *a.len;
+  uint2 raw{0, 0};
+  if (c < c1) {
+    ask(c, 0, a.shares);
+    raw = *reinterpret_cast<const uint2*>(a.whole + c);
+  }
+  lds_barrier();
+  const int n = parts_of(len, part_size_of(units_of(len), a.shares));
+  for (; c < c1; c += 1024) {
+    if (c >= c0 + 1024) {
+      ask(c, 0, a.shares);
+      raw = *reinterpret_cast<const uint2*>(a.whole + c);
+    }
+    if (n != 1) {
+      float M = kNegInf, den = 0.f;
+      f32x4 num = {0.f, 0.f, 0.f, 0.f};
+      for (int p0 = 0; p0 < n; p0 += B) {
+        if (p0 > 0) ask(c, p0, n - 1);
+        float top = M;
+#pragma unroll
+        for (int i = 0; i < B; ++i)
+          if (p0 + i < n) top = fmaxf(top, ml[i][0]);
+        const float corr = __builtin_amdgcn_exp2f(M - top);
+        num *= corr;
+        den *= corr;
+        M = top;
+#pragma unroll
+        for (int i = 0; i < B; ++i)
+          if (p0 + i < n) {
+            const float w = __builtin_amdgcn_exp2f(ml[i][0] - top);
+            num += w * v[i];
+            den += w * ml[i][1];
+          }
+      }
+      float x[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) x[i] = den > 0.f ? num[i] / den : 0.f;
+      raw = uint2{uint32_t(f32_to_bf16(x[0])) |
+                      uint32_t(f32_to_bf16(x[1])) << 16,
+                  uint32_t(f32_to_bf16(x[2])) |
+                      uint32_t(f32_to_bf16(x[3])) << 16};
+    }
+    *reinterpret_cast<uint2*>(xs + c) = raw;
+  }
+  lds_barrier();
+}
+
+enum { NO_PRE = 0, PRE_NORM = 1, PRE_COMBINE = 2 };
+
 // CT: 16-row tiles of w per wave; XR: rows of x that are staged; MT: 16-row
 // tiles of x; R: steps in the ring.  OUT_SILU: a wave's first tile is of the
 // gate's rows, the second the same rows of the upper half of w.
-// NORM: of one row x, made here (XR 0); all of it stays in LDS, behind the ring.
-template <int CT, int XR, int MT, int R, int OUT, bool NORM = false>
-__global__ __launch_bounds__(NORM ? 512 : 256)
+// PRE: of one row x, made here (XR 0); it stays in LDS, behind the ring.
+template <int CT, int XR, int MT, int R, int OUT, int PRE = NO_PRE>
+__global__ __launch_bounds__(PRE ? 512 : 256)
 void rows_gemm_kernel(const uint16_t* __restrict__ x,
                       const uint16_t* __restrict__ w, void* __restrict__ out,
-                      int M, int N, int K, int splits, NormArgs norm) {
+                      int M, int N, int K, int splits, NormArgs norm,
+                      RowsCombine attn) {
   constexpr int WPART = 4 * CT * 16 * LINE;          // elements of a step
   constexpr int STEP = WPART + XR * LINE;
   constexpr int L = CT * 2 + XR / 32;                // loads of a wave
@@ -200,7 +277,14 @@ void rows_gemm_kernel(const uint16_t* __restrict__ x,
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int half = N / 2;
   uint16_t* xs = lds + R * STEP;
-  if constexpr (NORM) {
+  if constexpr (PRE == PRE_COMBINE) {
+    if (wv >= 4) {
+      combine_row(attn, s0 * KS, (s0 + n) * KS, threadIdx.x - 256, xs);
+      lds_barrier();
+      return;
+    }
+  }
+  if constexpr (PRE == PRE_NORM) {
     if (wv >= 4) {
       // (the ring's last step is not asked for before the second barrier)
       float* sums = reinterpret_cast<float*>(lds + (R - 1) * STEP);
@@ -264,11 +348,11 @@ void rows_gemm_kernel(const uint16_t* __restrict__ x,
 
   const int tr = lane & 15, oct = lane >> 4;
   const int sw = tr >> 1;
-  if constexpr (NORM) lds_barrier();
+  if constexpr (PRE) lds_barrier();
 #pragma unroll
   for (int s = 0; s < R - 1; ++s)
     if (s < n) issue(s, s);
-  if constexpr (NORM) {
+  if constexpr (PRE) {
     lds_barrier();
     lds_barrier();
   }
@@ -296,7 +380,7 @@ void rows_gemm_kernel(const uint16_t* __restrict__ x,
 #pragma unroll
       for (int m = 0; m < MT; ++m)
         b[k][m] = *reinterpret_cast<const s16x8*>(
-            NORM ? xo + k * 32 : xt + m * 16 * LINE + piece);
+            PRE ? xo + k * 32 : xt + m * 16 * LINE + piece);
     }
 #pragma unroll
     for (int k = 0; k < 2; ++k)
@@ -509,7 +593,7 @@ void go(const uint16_t* x, const uint16_t* w, void* out, int M, int N, int K,
                                 hipFuncAttributeMaxDynamicSharedMemorySize,
                                 int(smem));
     hipLaunchKernelGGL(k, dim3(panels * splits), dim3(256), smem, st, x, w,
-                       out, M, N, K, splits, NormArgs{});
+                       out, M, N, K, splits, NormArgs{}, RowsCombine{});
   };
   using I1 = std::integral_constant<int, 1>;
   using I2 = std::integral_constant<int, 2>;
@@ -532,7 +616,7 @@ template <int CT, int R, int OUT>
 void go_norm(const RowsNorm& norm, const uint16_t* w, void* out, int N, int K,
              int panels, int splits, hipStream_t st) {
   const size_t smem = (size_t(R) * 4 * CT * 16 * LINE + size_t(K)) * 2;
-  auto* k = rows_gemm_kernel<CT, 0, 1, R, OUT, true>;
+  auto* k = rows_gemm_kernel<CT, 0, 1, R, OUT, PRE_NORM>;
   if (smem > 65536)
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(k),
                               hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -540,7 +624,8 @@ void go_norm(const RowsNorm& norm, const uint16_t* w, void* out, int N, int K,
   hipLaunchKernelGGL(k, dim3(panels * splits), dim3(512), smem, st, nullptr, w,
                      out, 1, N, K, splits,
                      NormArgs{norm.parts, norm.residual, norm.residual_out,
-                              norm.gain, norm.n, norm.eps});
+                              norm.gain, norm.n, norm.eps},
+                     RowsCombine{});
 }
 
 template <int PT, int R16, int R32, int R64, bool RELU2>
@@ -622,6 +707,20 @@ bool rows_norm_ok(int N, int K, bool silu) {
 void launch_rows_norm(const RowsNorm& norm, const uint16_t* w, float* parts,
                       int N, int K, int splits, hipStream_t st) {
   go_norm<1, 6, OUT_PARTS>(norm, w, parts, N, K, (N + 63) / 64, splits, st);
+}
+
+void launch_rows_combine(const RowsCombine& attn, const uint16_t* w,
+                         float* parts, int N, int K, int splits,
+                         hipStream_t st) {
+  constexpr int R = 6;
+  const size_t smem = (size_t(R) * 64 * LINE + size_t(K)) * 2;
+  auto* k = rows_gemm_kernel<1, 0, 1, R, OUT_PARTS, PRE_COMBINE>;
+  if (smem > 65536)
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(k),
+                              hipFuncAttributeMaxDynamicSharedMemorySize,
+                              int(smem));
+  hipLaunchKernelGGL(k, dim3((N + 63) / 64 * splits), dim3(512), smem, st,
+                     nullptr, w, parts, 1, N, K, splits, NormArgs{}, attn);
 }
 
 void launch_rows_norm_silu(const RowsNorm& norm, const uint16_t* w,

@@ -84,7 +84,7 @@ DEV_INLINE int part_size(const DecodeArgs& a) {
     t += units_of(a.seq_lens[s]);
 #pragma unroll
   for (int d = 1; d < 64; d <<= 1) t += __shfl_xor(t, d, kWave);
-  return part_size_of(__builtin_amdgcn_readfirstlane(t), a.shares);
+  return part_size_of(__builtin_amdgcn_readfirstlane(t), a.shares, a.batch);
 }
 
 // Parts of the sequences ahead of ``seq``.

@@ -212,7 +212,7 @@ DEV_INLINE void combine_row(const RowsCombine& a, int c0, int c1, int t,
     raw = *reinterpret_cast<const uint2*>(a.whole + c);
   }
   lds_barrier();
-  const int n = parts_of(len, part_size_of(units_of(len), a.shares));
+  const int n = parts_of(len, part_size_of(units_of(len), a.shares, 1));
   for (; c < c1; c += 1024) {
     if (c >= c0 + 1024) {
       ask(c, 0, a.shares);

@@ -19,7 +19,8 @@
 //                 [token, choice]; the sum over choices happens in the
 //                 residual kernel that reads it anyway.
 // Small row counts stream the weights straight into MFMA fragments, K
-// split over the waves; large ones run 128 x 128 tiles through LDS.
+// split over the waves; large ones run tiles of 128 or 256 rows by 256
+// columns through LDS (tile_product.h).
 
 #include "mix.h"
 #include "tile_product.h"

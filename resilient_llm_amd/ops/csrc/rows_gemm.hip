@@ -76,8 +76,8 @@ DEV_INLINE void wait_steps(int left) {
 // earlier product's f32 parts, normed, in LDS, by four more waves while the
 // others' first steps of w are under way.  What bounds it is the time to that
 // read's data.  us, norm and product apart and in one: 6144 x 4096 parts 4.5 +
-// 9.6 and 11.6, 28672 x 4096 with silu 4.5 + 35.8 and 37.1, 3072 x 2048 4.5 +
-// 4.8 and 6.0, 16384 x 2048 with silu 4.5 + 12.4 and 13.7.  (Two rows read
+// 9.6 and 11.3, 28672 x 4096 with silu 4.5 + 35.8 and 37.3, 3072 x 2048 4.5 +
+// 4.8 and 5.6, 16384 x 2048 with silu 4.5 + 12.4 and 13.5.  (Two rows read
 // twice as much: 2 us slower than apart.  Rows made once and handed to the
 // other workgroups through memory: 2 us slower as well, five trips to memory
 // while it is busy with weights.)

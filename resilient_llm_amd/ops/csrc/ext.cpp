@@ -762,14 +762,14 @@ std::tuple<Tensor, Tensor> rows_norm_linear(const Tensor& parts,
               "parts: f32 [n, 1, K]");
   TORCH_CHECK(gain.numel() == K && gain.device() == residual.device(),
               "a gain of K");
-  for (const Tensor* t : {&parts, &gain})
-    TORCH_CHECK(reinterpret_cast<uintptr_t>(t->data_ptr()) % 16 == 0,
-                "parts and gain start at multiples of 16 bytes");
+  TORCH_CHECK(reinterpret_cast<uintptr_t>(parts.data_ptr()) % 16 == 0,
+              "parts start at multiples of 16 bytes");
   c10::hip::HIPGuardMasqueradingAsCUDA guard(residual.device());
   const hipStream_t st = current_stream(residual);
+  const Tensor whole_gain = aligned(gain);
   Tensor after = at::empty_like(residual);
   const rlli::RowsNorm norm{parts.data_ptr<float>(), bf16_ptr(residual),
-                            bf16_ptr(after), bf16_ptr(gain),
+                            bf16_ptr(after), bf16_ptr(whole_gain),
                             int(parts.size(0)), float(eps)};
   Tensor out;
   if (silu) {

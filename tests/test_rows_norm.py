@@ -70,3 +70,13 @@ def test_operands_are_checked():
                 gain), (parts, residual, gain.cpu()), (parts, two, gain)):
         with pytest.raises(RuntimeError):
             ops.rows_norm_linear(*bad, 1e-5, w, False)
+
+
+def test_gain_of_any_alignment():
+    parts, residual, gain, w = inputs(4, 64, 128)
+    odd = torch.cat([gain[:1], gain])[1:]
+    assert odd.data_ptr() % 16
+    for got, want in zip(
+            ops.rows_norm_linear(parts, residual, odd, 1e-5, w, False),
+            ops.rows_norm_linear(parts, residual, gain, 1e-5, w, False)):
+        assert torch.equal(got, want)

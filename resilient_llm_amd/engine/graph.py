@@ -85,21 +85,17 @@ class DecodeGraphRunner:
 
     # ---- the captured step ----
     def _steady_body(self, b: int) -> torch.Tensor:
-        bsz = self.kv.block_size
         pos = self.positions[:b]
-        bi = torch.clamp((pos // bsz).long(), max=self.bt_width - 1)
-        slots = (self.block_tables[:b].gather(1, bi.unsqueeze(1)).squeeze(1)
-                 * bsz + pos % bsz)
-        seq_lens = pos + 1
+        slots, seq_lens = ops.decode_begin(pos, self.block_tables[:b],
+                                           self.kv.block_size)
         extra = ({"state_slots": self.state_slots[:b]}
                  if getattr(self.model, "mixed_layers", False) else {})
         logits = self.model.forward_decode(self.in_ids[:b], pos, self.kv,
                                            slots, self.block_tables[:b],
                                            seq_lens, **extra)
         toks = ops.sample(logits, self.temps[:b], self.seeds[:b], 0)
-        self.in_ids[:b].copy_(toks)
-        self.positions[:b].add_(1)
-        self.seeds[:b].add_(GOLDEN_SIGNED)
+        ops.decode_advance_(self.in_ids[:b], pos, self.seeds[:b], toks,
+                            GOLDEN_SIGNED)
         return logits, toks
 
     def _capture_all(self) -> None:
@@ -165,24 +161,12 @@ class DecodeGraphRunner:
         when the batch composition changed — a steady batch replays with
         zero host->device traffic."""
         B = input_ids.shape[0]
-        W = block_tables.shape[1]
         nb = self._bucket(B)
-        self.in_ids[:B].copy_(input_ids)
-        self.positions[:B].copy_(positions)
-        self.block_tables[:B, :W].copy_(block_tables)
-        self.temps[:B].copy_(temps)
-        self.seeds[:B].copy_(seeds)
-        if state_slots is not None:
-            self.state_slots[:B].copy_(state_slots)
-        if W < self.bt_width:          # stale tail from an earlier batch
-            self.block_tables[:B, W:].fill_(self.scratch_block)
-        if nb > B:                     # neutralize padded lanes
-            self.in_ids[B:nb].zero_()
-            self.positions[B:nb].zero_()
-            self.block_tables[B:nb].fill_(self.scratch_block)
-            self.temps[B:nb].zero_()
-            self.seeds[B:nb].zero_()
-            self.state_slots[B:nb].fill_(self.scratch_slot)
+        ops.decode_load(
+            (self.in_ids, self.positions, self.block_tables, self.temps,
+             self.seeds, self.state_slots),
+            (input_ids, positions, block_tables, temps, seeds, state_slots),
+            nb, self.scratch_block, self.scratch_slot)
         self._nb = nb
         self._live = B
 

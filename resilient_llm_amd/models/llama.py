@@ -400,7 +400,7 @@ class LlamaForCausalLM:
                and c.hidden_size <= 8192 else _linear)
         to_qkv = _linear_parts if qkv_parts else _linear
         if residual is None:
-            residual = x.clone()
+            residual = x        # the embedding's rows, nobody else's
             h = ops.rmsnorm(x, p[f"l{i}.ln1"], c.rms_eps)
             qkv = to_qkv(h, p[f"l{i}.qkv"])
         else:
@@ -539,7 +539,10 @@ class LlamaForCausalLM:
         a layer but the first at once.  ``attn_out_fn``: attention and the
         product behind it."""
         p = self.params
-        x = F.embedding(input_ids.long(), p["embed"])
+        ids = input_ids
+        if ids.dtype not in (torch.int32, torch.int64):
+            ids = ids.long()
+        x = F.embedding(ids, p["embed"])
         residual = None
         for i in range(self.config.n_layers):
             if layer is not None and i > 0:

@@ -301,6 +301,63 @@ def sample(logits: torch.Tensor, temperatures: torch.Tensor,
     return ref.sample(logits, temperatures, seeds, step)
 
 
+def decode_load(state, batch, bucket: int, scratch_block: int,
+                scratch_slot: int) -> None:
+    """The first ``bucket`` rows of a decode step's buffers ``state`` (ids,
+    positions, tables, temperatures, seeds, state slots) from those of
+    ``batch``, whose slots may be None; rows and pages that it does not have
+    are the scratch block's and slot's.  One launch for tensors of the
+    buffers' types on their GPU, a copy each for others."""
+    ids, tables = batch[0], batch[2]
+    B, W = ids.shape[0], tables.shape[1]
+    if (B <= bucket and W <= state[2].shape[1] and state[0].is_cuda
+            and all(t is None or (t.device == to.device and t.dtype == to.dtype
+                                  and t.is_contiguous()
+                                  and t.shape == ((B, W) if t is tables
+                                                  else (B,)))
+                    for t, to in zip(batch, state))):
+        _gpu()
+        torch.ops.rlli.decode_load(*state, *batch, bucket, scratch_block,
+                                   scratch_slot)
+        return
+    for t, to in zip(batch, state):
+        if t is tables:
+            to[:B, :W].copy_(t)
+            if W < to.shape[1]:          # stale tail from an earlier batch
+                to[:B, W:].fill_(scratch_block)
+        elif t is not None:
+            to[:B].copy_(t)
+    for to, fill in zip(state, (0, 0, scratch_block, 0, 0, scratch_slot)):
+        to[B:bucket].fill_(fill)         # neutralize padded lanes
+
+
+def decode_begin(positions: torch.Tensor, tables: torch.Tensor,
+                 block_size: int) -> tuple[torch.Tensor, torch.Tensor]:
+    """Of rows at ``positions``: the slots of their keys and values (in the
+    table's last block beyond its end), and the tokens they see."""
+    if positions.is_cuda:
+        _gpu()
+        return torch.ops.rlli.decode_begin(positions, tables, block_size)
+    block = torch.clamp((positions // block_size).long(),
+                        max=tables.shape[1] - 1)
+    return (tables.gather(1, block.unsqueeze(1)).squeeze(1) * block_size
+            + positions % block_size, positions + 1)
+
+
+def decode_advance_(ids: torch.Tensor, positions: torch.Tensor,
+                    seeds: torch.Tensor, tokens: torch.Tensor,
+                    seed_step: int) -> None:
+    """The next step's ids, positions and (mod 2^64) seeds."""
+    if ids.is_cuda:
+        _gpu()
+        torch.ops.rlli.decode_advance_(ids, positions, seeds, tokens,
+                                       seed_step)
+        return
+    ids.copy_(tokens)
+    positions.add_(1)
+    seeds.add_(seed_step)
+
+
 def prefill_paged_attn(qkv, k_cache, v_cache, chunk_row0, chunk_pos0,
                        chunk_nrows, chunk_btrow, block_tables,
                        scale: float, n_q: int) -> torch.Tensor:

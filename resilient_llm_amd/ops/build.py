@@ -47,6 +47,7 @@ LIBRARIES = {
         "sampling.hip",
         "rows_gemm.hip",
         "tile_gemm.hip",
+        "decode_state.hip",
         "streamprobe.hip",
     ],
     "rlli_attn": [

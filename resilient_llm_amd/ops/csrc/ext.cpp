@@ -933,6 +933,105 @@ Tensor sample(const Tensor& logits, const Tensor& temperatures,
   return out;
 }
 
+// ------------------------------------------------- a captured step's state
+static void check_rows_of(const Tensor& t, at::ScalarType type, int64_t rows,
+                          int64_t width, const Tensor& like, const char* name) {
+  TORCH_CHECK(t.is_cuda() && t.device() == like.device() &&
+                  t.scalar_type() == type && t.is_contiguous() &&
+                  t.dim() == (width < 0 ? 1 : 2) && t.size(0) == rows &&
+                  (width < 0 || t.size(1) == width),
+              name, ": ", rows, " rows of the step's type on its GPU");
+}
+
+// The first ``bucket`` rows of a step's buffers from a batch; those that it
+// does not fill have nothing but the scratch block and slot.
+void decode_load(Tensor ids_to, Tensor positions_to, Tensor tables_to,
+                 Tensor temps_to, Tensor seeds_to, Tensor slots_to,
+                 const Tensor& ids, const Tensor& positions,
+                 const Tensor& tables, const Tensor& temps,
+                 const Tensor& seeds, const std::optional<Tensor>& slots,
+                 int64_t bucket, int64_t scratch_block, int64_t scratch_slot) {
+  TORCH_CHECK(ids_to.dim() == 1 && tables_to.dim() == 2 && ids.dim() == 1 &&
+                  tables.dim() == 2,
+              "rows of ids and of tables");
+  const int64_t rows = ids_to.size(0), width = tables_to.size(1);
+  const int64_t batch = ids.size(0), wide = tables.size(1);
+  TORCH_CHECK(batch <= bucket && bucket >= 1 && bucket <= rows &&
+                  wide <= width,
+              "a batch of ", batch, " by ", wide, " in ", bucket, " of ", rows,
+              " rows by ", width);
+  const Tensor& at = ids_to;
+  check_rows_of(ids_to, at::kInt, rows, -1, at, "ids_to");
+  check_rows_of(positions_to, at::kInt, rows, -1, at, "positions_to");
+  check_rows_of(tables_to, at::kInt, rows, width, at, "tables_to");
+  check_rows_of(temps_to, at::kFloat, rows, -1, at, "temps_to");
+  check_rows_of(seeds_to, at::kLong, rows, -1, at, "seeds_to");
+  check_rows_of(slots_to, at::kInt, rows, -1, at, "slots_to");
+  check_rows_of(ids, at::kInt, batch, -1, at, "ids");
+  check_rows_of(positions, at::kInt, batch, -1, at, "positions");
+  check_rows_of(tables, at::kInt, batch, wide, at, "tables");
+  check_rows_of(temps, at::kFloat, batch, -1, at, "temps");
+  check_rows_of(seeds, at::kLong, batch, -1, at, "seeds");
+  if (slots) check_rows_of(*slots, at::kInt, batch, -1, at, "slots");
+  c10::hip::HIPGuardMasqueradingAsCUDA guard(at.device());
+  auto state = [](const Tensor& i, const Tensor& p, const Tensor& t,
+                  const Tensor& f, const Tensor& s, const Tensor* slot) {
+    return rlli::DecodeState{
+        i.data_ptr<int32_t>(), p.data_ptr<int32_t>(), t.data_ptr<int32_t>(),
+        f.data_ptr<float>(),   s.data_ptr<int64_t>(),
+        slot ? slot->data_ptr<int32_t>() : nullptr, int(t.size(1))};
+  };
+  rlli::launch_decode_load(
+      state(ids_to, positions_to, tables_to, temps_to, seeds_to, &slots_to),
+      state(ids, positions, tables, temps, seeds, slots ? &*slots : nullptr),
+      int(bucket), int(batch), int(wide), int(scratch_block),
+      int(scratch_slot), current_stream(at));
+  check_launch("decode_load");
+}
+
+// Rows of decoding sequences at ``positions``: where their keys and values go,
+// and how many tokens they see.
+std::tuple<Tensor, Tensor> decode_begin(const Tensor& positions,
+                                        const Tensor& tables,
+                                        int64_t block_size) {
+  TORCH_CHECK(positions.dim() == 1 && tables.dim() == 2 &&
+                  tables.size(1) >= 1 && block_size >= 1,
+              "positions, their tables and a block's size");
+  const int64_t batch = positions.size(0);
+  check_rows_of(positions, at::kInt, batch, -1, positions, "positions");
+  check_rows_of(tables, at::kInt, batch, tables.size(1), positions, "tables");
+  Tensor slots = at::empty_like(positions), lens = at::empty_like(positions);
+  if (batch == 0) return {slots, lens};
+  c10::hip::HIPGuardMasqueradingAsCUDA guard(positions.device());
+  rlli::launch_decode_begin(positions.data_ptr<int32_t>(),
+                            tables.data_ptr<int32_t>(),
+                            slots.data_ptr<int32_t>(),
+                            lens.data_ptr<int32_t>(), int(batch),
+                            int(tables.size(1)), int(block_size),
+                            current_stream(positions));
+  check_launch("decode_begin");
+  return {slots, lens};
+}
+
+// One token on: the sampled tokens are the next ids.
+void decode_advance_(Tensor ids, Tensor positions, Tensor seeds,
+                     const Tensor& tokens, int64_t seed_step) {
+  TORCH_CHECK(ids.dim() == 1, "rows of ids");
+  const int64_t batch = ids.size(0);
+  check_rows_of(ids, at::kInt, batch, -1, ids, "ids");
+  check_rows_of(positions, at::kInt, batch, -1, ids, "positions");
+  check_rows_of(seeds, at::kLong, batch, -1, ids, "seeds");
+  check_rows_of(tokens, at::kInt, batch, -1, ids, "tokens");
+  if (batch == 0) return;
+  c10::hip::HIPGuardMasqueradingAsCUDA guard(ids.device());
+  rlli::launch_decode_advance(ids.data_ptr<int32_t>(),
+                              positions.data_ptr<int32_t>(),
+                              seeds.data_ptr<int64_t>(),
+                              tokens.data_ptr<int32_t>(), int(batch),
+                              seed_step, current_stream(ids));
+  check_launch("decode_advance_");
+}
+
 // ------------------------------------------------------- a prompt's layer
 static Tensor norm_any(const Tensor& x, const Tensor& residual,
                        const Tensor& gain, double eps) {
@@ -1017,6 +1116,15 @@ TORCH_LIBRARY(rlli, m) {
         "Tensor cu_seqlens, float eps, float scale, int n_q) -> Tensor");
   m.def("prefill_attn(Tensor q, Tensor k, Tensor v, Tensor cu_seqlens, "
         "float scale) -> Tensor");
+  m.def("decode_load(Tensor(a!) ids_to, Tensor(b!) positions_to, "
+        "Tensor(c!) tables_to, Tensor(d!) temps_to, Tensor(e!) seeds_to, "
+        "Tensor(f!) slots_to, Tensor ids, Tensor positions, Tensor tables, "
+        "Tensor temps, Tensor seeds, Tensor? slots, int bucket, "
+        "int scratch_block, int scratch_slot) -> ()");
+  m.def("decode_begin(Tensor positions, Tensor tables, int block_size) -> "
+        "(Tensor, Tensor)");
+  m.def("decode_advance_(Tensor(a!) ids, Tensor(b!) positions, "
+        "Tensor(c!) seeds, Tensor tokens, int seed_step) -> ()");
   m.def("sample(Tensor logits, Tensor temperatures, Tensor seeds, int step) -> Tensor");
   m.def("rows_linear_parts(Tensor x, Tensor w) -> Tensor");
   m.def("rows_linear(Tensor x, Tensor w) -> Tensor");
@@ -1062,6 +1170,9 @@ TORCH_LIBRARY_IMPL(rlli, CUDA, m) {
   m.impl("prefill_attn_qkv", &prefill_attn_qkv);
   m.impl("prompt_rows_layer", &prompt_rows_layer);
   m.impl("prefill_attn", &prefill_attn);
+  m.impl("decode_load", &decode_load);
+  m.impl("decode_begin", &decode_begin);
+  m.impl("decode_advance_", &decode_advance_);
   m.impl("sample", &sample);
   m.impl("rows_linear_parts", &rows_linear_parts);
   m.impl("rows_linear", &rows_linear);

@@ -173,6 +173,27 @@ void launch_tile_gemm(const uint16_t* x, const uint16_t* w, float* parts,
                       uint16_t* out, int M, int N, int K, TileAct act,
                       const TilePlan& plan, hipStream_t stream);
 
+// A decode step's buffers, rows of a batch (decode_state.hip).
+struct DecodeState {
+  int32_t *ids, *positions;
+  int32_t* tables;             // [.., width]
+  float* temps;
+  int64_t* seeds;
+  int32_t* slots;              // of what is loaded: or null
+  int width;
+};
+// The first ``bucket`` rows, of which ``batch`` come from a batch with tables
+// [batch, wide].
+void launch_decode_load(const DecodeState& to, const DecodeState& from,
+                        int bucket, int batch, int wide, int scratch_block,
+                        int scratch_slot, hipStream_t stream);
+void launch_decode_begin(const int32_t* positions, const int32_t* tables,
+                         int32_t* slots, int32_t* lens, int batch, int width,
+                         int block_size, hipStream_t stream);
+void launch_decode_advance(int32_t* ids, int32_t* positions, int64_t* seeds,
+                           const int32_t* tokens, int batch,
+                           int64_t seed_step, hipStream_t stream);
+
 // Diagnostic: W streamed past the caches, 64 rows by a part of K per workgroup.
 void launch_stream_probe(const uint16_t* w, float* sink, int N, int K,
                          int splitk, hipStream_t stream);

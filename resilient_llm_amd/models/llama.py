@@ -489,14 +489,15 @@ class LlamaForCausalLM:
         def attn(i, qkv, k_cache, v_cache):
             ops.rope_kv_append_qkv_(qkv, positions, self.cos_sin, k_cache,
                                     v_cache, slot_mapping, self.n_heads)
-            out = ops.prefill_paged_attn(
+            if n_decode:
+                return ops.mixed_attn_qkv(
+                    qkv, k_cache, v_cache, chunk_row0, chunk_pos0,
+                    chunk_nrows, chunk_btrow, block_tables_pre,
+                    block_tables_dec, seq_lens_dec, n_decode, self.scale,
+                    self.n_heads)
+            return ops.prefill_paged_attn(
                 qkv, k_cache, v_cache, chunk_row0, chunk_pos0, chunk_nrows,
                 chunk_btrow, block_tables_pre, self.scale, self.n_heads)
-            if n_decode:
-                ops.decode_attn_qkv_out(
-                    qkv[:n_decode], k_cache, v_cache, block_tables_dec,
-                    seq_lens_dec, self.scale, self.n_heads, out)
-            return out
         return self._forward(input_ids, positions, kv_cache, slot_mapping,
                              attn, last_idx=sample_idx)
 

@@ -372,6 +372,25 @@ def prefill_paged_attn(qkv, k_cache, v_cache, chunk_row0, chunk_pos0,
                                   block_tables, scale, n_q)
 
 
+def mixed_attn_qkv(qkv, k_cache, v_cache, chunk_row0, chunk_pos0, chunk_nrows,
+                   chunk_btrow, tables_pre, tables_dec, lens_dec,
+                   n_decode: int, scale: float, n_q: int) -> torch.Tensor:
+    """Attention of a mixed step whose keys and values are in the cache:
+    decode_attn_qkv for rows [0, n_decode), n_decode > 0, prefill_paged_attn for
+    the tiles', at the same time where that is the faster way."""
+    if qkv.is_cuda:
+        _gpu()
+        return torch.ops.rlli.mixed_attn_qkv(
+            qkv, k_cache, v_cache, chunk_row0, chunk_pos0, chunk_nrows,
+            chunk_btrow, tables_pre, tables_dec, lens_dec, n_decode, scale,
+            n_q)
+    out = prefill_paged_attn(qkv, k_cache, v_cache, chunk_row0, chunk_pos0,
+                             chunk_nrows, chunk_btrow, tables_pre, scale, n_q)
+    decode_attn_qkv_out(qkv[:n_decode], k_cache, v_cache, tables_dec,
+                        lens_dec, scale, n_q, out)
+    return out
+
+
 def _rows_faster(M: int, N: int, K: int) -> bool:
     """Where rows_linear beats the library, with weights that no cache holds.
     Timed at 1 to 128 rows of 300 shapes from 16 to 128256 by 256 to 28672; by

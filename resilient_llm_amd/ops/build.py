@@ -44,6 +44,7 @@ LIBRARIES = {
         "decode_attn.hip",
         "prefill_attn.hip",
         "prefill_flash.hip",
+        "mixed_attn.hip",
         "sampling.hip",
         "rows_gemm.hip",
         "tile_gemm.hip",
@@ -80,9 +81,9 @@ LIBRARIES = {
 }
 _ACT = ["common.h", "act.h", "ext_common.h"]
 _ATTN = _ACT + ["attn.h", "attn_rows.h", "ext_window.h"]
-HEADERS = {"rlli_hip": ["common.h", "decode_parts.h", "kernels.h",
-                        "prefill_flash.h",
-                        "prefill_parts.h", "tile_product.h"],
+HEADERS = {"rlli_hip": ["common.h", "decode_attn.h", "decode_parts.h",
+                        "kernels.h", "prefill_flash.h", "prefill_parts.h",
+                        "tile_product.h"],
            "rlli_attn": _ATTN,
            "rlli_mix": _ATTN + ["mix.h", "prefill_flash.h", "prefill_parts.h",
                                 "tile_product.h"],

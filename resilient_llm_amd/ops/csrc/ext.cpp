@@ -649,6 +649,91 @@ Tensor prefill_paged_attn(const Tensor& qkv, const Tensor& k_cache,
   return out;
 }
 
+// Attention of a mixed step: rows [0, n_decode) are decoding sequences', the
+// others the tiles'.  In one launch where mixed_attn_plan takes the sizes (with
+// the parts and shares of ``given`` if there are any), one after the other
+// elsewhere.
+Tensor mixed_attn_qkv(const Tensor& qkv, const Tensor& k_cache,
+                      const Tensor& v_cache, const Tensor& chunk_row0,
+                      const Tensor& chunk_pos0, const Tensor& chunk_nrows,
+                      const Tensor& chunk_btrow, const Tensor& tables_pre,
+                      const Tensor& tables_dec, const Tensor& lens_dec,
+                      int64_t n_decode, double scale, int64_t n_q,
+                      at::IntArrayRef given) {
+  check_bf16_contig(qkv, "qkv");
+  check_qkv_width(qkv, k_cache, n_q);
+  const bool cache_fp8 = check_cache(k_cache, v_cache);
+  TORCH_CHECK(n_decode >= 0 && n_decode <= qkv.size(0), "decoding rows: ",
+              n_decode, " of ", qkv.size(0));
+  const int T = int(qkv.size(0)), batch = int(n_decode);
+  const int n_kv = int(k_cache.size(1)), block_size = int(k_cache.size(2));
+  const int D = int(k_cache.size(3)), group = int(n_q) / n_kv;
+  const int n_tiles = int(chunk_row0.numel());
+  auto table = [&](const Tensor& t) {
+    return t.scalar_type() == at::kInt && t.is_contiguous() &&
+           t.device() == qkv.device();
+  };
+  rlli::MixedPlan plan{0, 0};
+  if (n_tiles > 0 && batch > 0 && n_q % n_kv == 0 && (D == 64 || D == 128) &&
+      table(chunk_row0) && table(chunk_pos0) && table(chunk_nrows) &&
+      table(chunk_btrow) && table(tables_pre) && table(tables_dec) &&
+      table(lens_dec) && tables_pre.dim() == 2 && tables_dec.dim() == 2 &&
+      chunk_pos0.numel() == n_tiles && chunk_nrows.numel() == n_tiles &&
+      chunk_btrow.numel() == n_tiles && tables_dec.size(0) >= batch &&
+      lens_dec.numel() >= batch && v_cache.sizes() == k_cache.sizes() &&
+      k_cache.device() == qkv.device() && v_cache.device() == qkv.device() &&
+      (reinterpret_cast<uintptr_t>(qkv.data_ptr()) |
+       reinterpret_cast<uintptr_t>(k_cache.data_ptr()) |
+       reinterpret_cast<uintptr_t>(v_cache.data_ptr())) % 16 == 0)
+    plan = rlli::mixed_attn_plan(
+        n_tiles, batch, n_kv, group, D, int(tables_pre.size(1)) * block_size,
+        int(tables_dec.size(1)) * block_size, int(k_cache.element_size()),
+        block_size);
+  if (!given.empty()) {
+    TORCH_CHECK(plan.splits > 0 && given.size() == 2 && given[0] >= 1 &&
+                    given[0] <= 16 && given[1] >= 0 && given[1] <= 512,
+                "no such division for these sizes");
+    plan = {int(given[0]), int(given[1])};
+  }
+  if (plan.splits == 0) {
+    Tensor out = prefill_paged_attn(qkv, k_cache, v_cache, chunk_row0,
+                                    chunk_pos0, chunk_nrows, chunk_btrow,
+                                    tables_pre, scale, n_q);
+    if (batch > 0)
+      decode_attn_qkv_out(qkv.narrow(0, 0, batch), k_cache, v_cache,
+                          tables_dec, lens_dec, scale, n_q, out);
+    return out;
+  }
+  Tensor out = at::empty({T, n_q * D}, qkv.options());
+  c10::hip::HIPGuardMasqueradingAsCUDA guard(qkv.device());
+  const auto f32 = qkv.options().dtype(at::kFloat);
+  rlli::PrefillParts parts{nullptr, nullptr, plan.splits, T};
+  Tensor tile_part, tile_ml, part, ml;
+  if (plan.splits > 1) {
+    tile_part = at::empty({plan.splits, T, n_q * D}, f32);
+    tile_ml = at::empty({plan.splits, T, n_q, 2}, f32);
+    parts.o = tile_part.data_ptr<float>();
+    parts.ml = tile_ml.data_ptr<float>();
+  }
+  if (plan.shares > 0) {
+    const int64_t slots = int64_t(n_kv) * (plan.shares + batch) * group;
+    part = at::empty({slots, D}, f32);
+    ml = at::empty({slots, 2}, f32);
+  }
+  rlli::launch_mixed_attn(
+      bf16_ptr(qkv), k_cache.data_ptr(), v_cache.data_ptr(),
+      chunk_row0.data_ptr<int32_t>(), chunk_pos0.data_ptr<int32_t>(),
+      chunk_nrows.data_ptr<int32_t>(), chunk_btrow.data_ptr<int32_t>(),
+      tables_pre.data_ptr<int32_t>(), int(tables_pre.size(1)),
+      tables_dec.data_ptr<int32_t>(), lens_dec.data_ptr<int32_t>(),
+      int(tables_dec.size(1)), bf16_ptr(out), n_tiles, batch, n_kv, group, D,
+      int(qkv.size(1)), float(scale), cache_fp8, parts, plan.shares,
+      plan.shares > 0 ? part.data_ptr<float>() : nullptr,
+      plan.shares > 0 ? ml.data_ptr<float>() : nullptr, current_stream(qkv));
+  check_launch("mixed_attn_qkv");
+  return out;
+}
+
 // ------------------------------------------------------------ rows_gemm
 static void check_rows(const Tensor& x, const Tensor& w) {
   check_bf16_contig(x, "x");
@@ -1176,6 +1261,11 @@ TORCH_LIBRARY(rlli, m) {
         "Tensor chunk_row0, Tensor chunk_pos0, Tensor chunk_nrows, "
         "Tensor chunk_btrow, Tensor block_tables, float scale, int n_q) "
         "-> Tensor");
+  m.def("mixed_attn_qkv(Tensor qkv, Tensor k_cache, Tensor v_cache, "
+        "Tensor chunk_row0, Tensor chunk_pos0, Tensor chunk_nrows, "
+        "Tensor chunk_btrow, Tensor tables_pre, Tensor tables_dec, "
+        "Tensor lens_dec, int n_decode, float scale, int n_q, int[] plan=[]) "
+        "-> Tensor");
 }
 
 TORCH_LIBRARY_IMPL(rlli, CUDA, m) {
@@ -1217,4 +1307,5 @@ TORCH_LIBRARY_IMPL(rlli, CUDA, m) {
   m.impl("skinny2_silu_linear", &skinny2_silu_linear);
   m.impl("stream_probe", &stream_probe);
   m.impl("prefill_paged_attn", &prefill_paged_attn);
+  m.impl("mixed_attn_qkv", &mixed_attn_qkv);
 }

@@ -112,6 +112,26 @@ void launch_prefill_paged(const uint16_t* qkv, const void* k_cache,
                           int block_size, float scale, bool cache_fp8,
                           const PrefillParts& parts, hipStream_t stream);
 
+// Prompt rows and decoding sequences of a mixed step at once (mixed_attn.hip).
+// What the tiles' keys are divided into and the sequences' shares; splits 0:
+// not for these sizes.  ``keys``, ``max_tokens``: what the tables have room for.
+struct MixedPlan {
+  int splits, shares;
+};
+MixedPlan mixed_attn_plan(int n_tiles, int batch, int n_kv, int group,
+                          int head_dim, int keys, int max_tokens, int elem,
+                          int block_size);
+void launch_mixed_attn(const uint16_t* qkv, void* k_cache, void* v_cache,
+                       const int32_t* chunk_row0, const int32_t* chunk_pos0,
+                       const int32_t* chunk_nrows, const int32_t* chunk_btrow,
+                       const int32_t* tables_pre, int pre_blocks,
+                       const int32_t* tables_dec, const int32_t* lens_dec,
+                       int dec_blocks, uint16_t* out, int n_tiles, int batch,
+                       int n_kv, int group, int head_dim, int stride,
+                       float scale, bool cache_fp8, const PrefillParts& parts,
+                       int shares, float* part_out, float* part_ml,
+                       hipStream_t stream);
+
 // Products of at most 128 rows, y[M, N] = x[M, K] w[N, K]^T (rows_gemm.hip).
 // With parts given, f32 [splits, M, N] whose sum is y; otherwise out.
 // N % 4 == 0, K % 64 == 0, 16-byte aligned rows.

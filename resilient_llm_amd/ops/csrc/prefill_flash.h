@@ -79,6 +79,25 @@ DEV_INLINE s16x4 read_tr(const uint16_t* p) {
 // are this tile's; false: none.  A windowed one also says which keys a row
 // sees (``window`` of them and the first ``keep``) and a head's sink.
 
+template <typename C>
+struct Pages {                    // [blocks, n_kv, block, D]
+  static constexpr bool kPaged = true, kWindow = false;
+  using KC = C;
+  const uint16_t* qkv;
+  const typename C::elem *k, *v;
+  const int32_t *row0s, *pos0s, *nrowss, *btrows, *tables;
+  int max_blocks, block_size;
+
+  DEV_INLINE bool find(int tile, int& row0, int& nrows, int& first,
+                       int& pos0) const {
+    row0 = row0s[tile];
+    pos0 = pos0s[tile];
+    nrows = nrowss[tile];
+    first = btrows[tile];
+    return nrows > 0;
+  }
+};
+
 // How many parts a tile's steps of KS tiles of keys are divided into.
 DEV_INLINE int parts_of(int steps, int splits) {
   return min(splits, max(steps / 4, 1));
@@ -87,11 +106,15 @@ DEV_INLINE int parts_of(int steps, int splits) {
 // D: head width; W: heads, a wave each; BS: block size of the cache where it
 // is known; KS: waves per head, each with every KS-th tile of keys, for
 // launches that leave CUs idle.  Their sums meet in LDS.
+// ``lds`` holds two stages, FLASH_LDS bytes.
+template <int D, int KS>
+constexpr size_t FLASH_LDS = size_t(2) * KS * 2 * KT * D * 2;
+
 template <int D, int W, int BS, int KS, typename Src>
-__global__ __launch_bounds__(64 * W * KS, W == 4 ? 2 : 1)
-void prefill_flash_kernel(Src src, uint16_t* __restrict__ out, int n_tiles,
-                          int n_kv, int group, int stride, float scale,
-                          PrefillParts parts) {
+DEV_INLINE void flash_tile(const Src& src, uint16_t* __restrict__ out,
+                           int block, int n_tiles, int n_kv, int group,
+                           int stride, float scale, const PrefillParts& parts,
+                           uint16_t* lds) {
   using KC = typename Src::KC;
   constexpr bool kDirect = std::is_same<KC, CacheBF16>::value;
   static_assert(KS == 1 || !Src::kWindow, "windows skip single tiles");
@@ -102,10 +125,6 @@ void prefill_flash_kernel(Src src, uint16_t* __restrict__ out, int n_tiles,
   constexpr int VT = D / 32;                 // channel tiles
   constexpr int HALF = KT * D;
   constexpr int STAGE = KS * 2 * HALF;       // keys | values, of KS tiles
-  __shared__ __attribute__((aligned(16))) uint16_t
-      lds_static[KS == 1 ? 2 * STAGE : 8];
-  extern __shared__ __attribute__((aligned(16))) uint16_t lds_dynamic[];
-  uint16_t* lds = KS == 1 ? lds_static : lds_dynamic;
 
   // the tiles of a key/value head stay on an XCD (workgroups go to XCDs in
   // turn), those with the longest context first
@@ -113,10 +132,10 @@ void prefill_flash_kernel(Src src, uint16_t* __restrict__ out, int n_tiles,
   const int per_head = n_tiles * (group / W) * splits;
   int kvh, i;
   if (n_kv % 8 == 0) {
-    i = blockIdx.x / 8;
-    kvh = i / per_head * 8 + blockIdx.x % 8;
+    i = block / 8;
+    kvh = i / per_head * 8 + block % 8;
   } else {
-    i = blockIdx.x;
+    i = block;
     kvh = i / per_head;
   }
   i %= per_head;
@@ -435,12 +454,25 @@ void prefill_flash_kernel(Src src, uint16_t* __restrict__ out, int n_tiles,
                 pack2(o[v][r + 2] * inv, o[v][r + 3] * inv)};
 }
 
-// The parts of a tile's rows together: a workgroup per (tile, query head).
+template <int D, int W, int BS, int KS, typename Src>
+__global__ __launch_bounds__(64 * W * KS, W == 4 ? 2 : 1)
+void prefill_flash_kernel(Src src, uint16_t* __restrict__ out, int n_tiles,
+                          int n_kv, int group, int stride, float scale,
+                          PrefillParts parts) {
+  __shared__ __attribute__((aligned(16))) uint16_t
+      lds_static[KS == 1 ? FLASH_LDS<D, KS> / 2 : 8];
+  extern __shared__ __attribute__((aligned(16))) uint16_t lds_dynamic[];
+  flash_tile<D, W, BS, KS>(src, out, blockIdx.x, n_tiles, n_kv, group, stride,
+                           scale, parts, KS == 1 ? lds_static : lds_dynamic);
+}
+
+// The parts of a tile's rows together: a workgroup of 256 threads per (tile,
+// query head).
 template <int D, typename Src>
-__global__ __launch_bounds__(256)
-void prefill_combine_kernel(Src src, uint16_t* __restrict__ out, int n_q,
-                            float scale, PrefillParts parts) {
-  const int tile = blockIdx.x / n_q, head = blockIdx.x % n_q;
+DEV_INLINE void flash_combine(const Src& src, uint16_t* __restrict__ out,
+                              int block, int n_q, float scale,
+                              const PrefillParts& parts) {
+  const int tile = block / n_q, head = block % n_q;
   int row0, nrows, first, pos0;
   if (!src.find(tile, row0, nrows, first, pos0)) return;
   const int n =
@@ -475,6 +507,13 @@ void prefill_combine_kernel(Src src, uint16_t* __restrict__ out, int n_q,
   }
 }
 
+template <int D, typename Src>
+__global__ __launch_bounds__(256)
+void prefill_combine_kernel(Src src, uint16_t* __restrict__ out, int n_q,
+                            float scale, PrefillParts parts) {
+  flash_combine<D>(src, out, blockIdx.x, n_q, scale, parts);
+}
+
 // ``keys``: about how many a sequence has, as far as the host knows without
 // waiting for the device: the mean of a batch of prompts, the width of the
 // block table for pages.
@@ -484,7 +523,7 @@ void by_group(const Src& src, uint16_t* out, int n_tiles, int n_kv, int group,
               const PrefillParts& parts = {nullptr, nullptr, 1, 0}) {
   auto go = [&](auto tag, auto waves) {
     constexpr int W = decltype(tag)::value, KS = decltype(waves)::value;
-    constexpr size_t smem = KS == 1 ? 0 : size_t(KS) * 2 * 2 * KT * D * 2;
+    constexpr size_t smem = KS == 1 ? 0 : FLASH_LDS<D, KS>;
     auto* k = prefill_flash_kernel<D, W, BS, KS, Src>;
     if (smem > 65536)
       (void)hipFuncSetAttribute(reinterpret_cast<const void*>(k),

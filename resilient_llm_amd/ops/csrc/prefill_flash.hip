@@ -49,25 +49,6 @@ struct BatchRows {                // k and v are columns of the batch's rows
   }
 };
 
-template <typename C>
-struct Pages {                    // [blocks, n_kv, block, D]
-  static constexpr bool kPaged = true, kWindow = false;
-  using KC = C;
-  const uint16_t* qkv;
-  const typename C::elem *k, *v;
-  const int32_t *row0s, *pos0s, *nrowss, *btrows, *tables;
-  int max_blocks, block_size;
-
-  DEV_INLINE bool find(int tile, int& row0, int& nrows, int& first,
-                       int& pos0) const {
-    row0 = row0s[tile];
-    pos0 = pos0s[tile];
-    nrows = nrowss[tile];
-    first = btrows[tile];
-    return nrows > 0;
-  }
-};
-
 }  // namespace
 
 void launch_prefill_rows(const uint16_t* qkv, const int32_t* cu_seqlens,

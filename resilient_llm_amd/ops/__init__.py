@@ -250,8 +250,9 @@ def prompt_rows_layer(x, residual, ln1, w_qkv, w_o, ln2, w_gate_up, w_down,
                       n_q: int) -> tuple[torch.Tensor, torch.Tensor]:
     """A Llama layer behind the first for few rows of whole prompts on the GPU:
     x + residual, normed, ... the last product, which may come in parts, and
-    the new residual (``residual`` is updated on the way).  The launches are
-    those of the ops one by one."""
+    the new residual (``residual`` is updated on the way).  The results are
+    those of the ops one by one; of up to 64 rows attention rotates and appends
+    in its own launch."""
     _gpu()
     return torch.ops.rlli.prompt_rows_layer(
         x, residual, ln1, w_qkv, w_o, ln2, w_gate_up, w_down, positions,

@@ -86,6 +86,15 @@ struct CacheFP8 {
   }
 };
 
+// A rotated pair (x1, x2); which product is rounded by itself is written out, so
+// that all who rotate have the same bits.
+DEV_INLINE float rope_lower(float x1, float x2, float c, float s) {
+  return fmaf(x1, c, -(x2 * s));
+}
+DEV_INLINE float rope_upper(float x1, float x2, float c, float s) {
+  return fmaf(x1, s, x2 * c);
+}
+
 // Wave-wide reductions (64 lanes).
 DEV_INLINE float wave_sum(float v) {
 #pragma unroll

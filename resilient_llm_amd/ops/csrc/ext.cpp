@@ -597,6 +597,44 @@ Tensor prefill_attn_qkv(const Tensor& qkv, const Tensor& cu_seqlens,
   return out;
 }
 
+// rope_kv_append_qkv_ and prefill_attn_qkv: of up to 64 rows in one launch, which
+// leaves qkv as it is.
+static Tensor prompt_rows_attn(Tensor qkv, const Tensor& positions,
+                               const Tensor& cos_sin, Tensor k_cache,
+                               Tensor v_cache, const Tensor& slot_mapping,
+                               const Tensor& cu_seqlens, double scale,
+                               int64_t n_q) {
+  const int64_t T = qkv.size(0), n_kv = k_cache.size(1), D = k_cache.size(3);
+  if (T > 64 || (D != 64 && D != 128) || n_q % n_kv != 0) {
+    rope_kv_append_qkv_(qkv, positions, cos_sin, k_cache, v_cache,
+                        slot_mapping, n_q);
+    return prefill_attn_qkv(qkv, cu_seqlens, scale, n_q, n_kv, D);
+  }
+  check_bf16_contig(qkv, "qkv");
+  const bool cache_fp8 = check_cache(k_cache, v_cache);
+  TORCH_CHECK(qkv.size(1) == (n_q + 2 * n_kv) * D, "qkv width mismatch");
+  TORCH_CHECK(positions.numel() == T && slot_mapping.numel() == T);
+  TORCH_CHECK(cos_sin.size(1) == D);
+  TORCH_CHECK(cu_seqlens.scalar_type() == at::kInt &&
+              cu_seqlens.is_contiguous());
+  const int group = int(n_q / n_kv), n_seqs = int(cu_seqlens.numel()) - 1;
+  TORCH_CHECK(group == 1 || group == 2 || group == 4 || group == 8);
+  TORCH_CHECK(T == 0 || n_seqs >= 1, "rows without a sequence: cu_seqlens has ",
+              cu_seqlens.numel(), " entries");
+  Tensor out = at::empty({T, n_q * D}, qkv.options());
+  c10::hip::HIPGuardMasqueradingAsCUDA guard(qkv.device());
+  const Tensor cu = cu_seqlens.to(qkv.device());
+  const Tensor rows = aligned(qkv);
+  rlli::launch_prompt_rows_attn(
+      bf16_ptr(rows), cu.data_ptr<int32_t>(), positions.data_ptr<int32_t>(),
+      cos_sin.data_ptr<float>(), k_cache.data_ptr(), v_cache.data_ptr(),
+      slot_mapping.data_ptr<int32_t>(), bf16_ptr(out), n_seqs, int(T),
+      int(n_kv), group, int(D), int(k_cache.size(2)), int(qkv.size(1)),
+      float(scale), cache_fp8, current_stream(qkv));
+  check_launch("prompt_rows_attn");
+  return out;
+}
+
 // ------------------------------------------------------ prefill (paged)
 Tensor prefill_paged_attn(const Tensor& qkv, const Tensor& k_cache,
                           const Tensor& v_cache, const Tensor& chunk_row0,
@@ -1145,8 +1183,8 @@ static Tensor norm_any(const Tensor& x, const Tensor& residual,
 }
 
 // All of a Llama layer but the first for the rows of a few short prompts, whose
-// step waits for the host: the ops in their order, launched from here; the last
-// product and the new residual, which is ``residual`` itself unless the one row's
+// step waits for the host: the ops in their order, rotation, append and attention
+// as one, launched from here; the last product and the new residual, which is ``residual`` itself unless the one row's
 // norm is made inside gate and up.
 // (A prompt of 45 tokens through 16 layers of 2048: 8 us a launch from Python, 5
 // from here; 1150 -> 1040 us.)
@@ -1156,13 +1194,12 @@ std::tuple<Tensor, Tensor> prompt_rows_layer(
     const Tensor& w_down, const Tensor& positions, const Tensor& cos_sin,
     Tensor k_cache, Tensor v_cache, const Tensor& slot_mapping,
     const Tensor& cu_seqlens, double eps, double scale, int64_t n_q) {
-  const int64_t n_kv = k_cache.size(1), D = k_cache.size(3);
   const Tensor h = norm_any(x, residual, ln1, eps);
   Tensor qkv = rows_take(h, w_qkv) ? rows_linear(h, w_qkv)
                                    : at::linear(h, w_qkv);
-  rope_kv_append_qkv_(qkv, positions, cos_sin, k_cache, v_cache, slot_mapping,
-                      n_q);
-  const Tensor seen = prefill_attn_qkv(qkv, cu_seqlens, scale, n_q, n_kv, D);
+  const Tensor seen =
+      prompt_rows_attn(qkv, positions, cos_sin, k_cache, v_cache, slot_mapping,
+                       cu_seqlens, scale, n_q);
   const Tensor mixed = rows_take(seen, w_o) ? rows_linear_parts(seen, w_o)
                                             : at::linear(seen, w_o);
   Tensor act, after = residual;

@@ -100,6 +100,16 @@ void launch_prefill_rows(const uint16_t* qkv, const int32_t* cu_seqlens,
                          int group, int head_dim, int qkv_stride, float scale,
                          hipStream_t stream);
 
+// The same of sequences of up to 64 rows with the rotation of queries and keys
+// and the append to the cache; qkv stays as it is.
+void launch_prompt_rows_attn(const uint16_t* qkv, const int32_t* cu_seqlens,
+                             const int32_t* positions, const float* cos_sin,
+                             void* k_cache, void* v_cache,
+                             const int32_t* slot_mapping, uint16_t* out,
+                             int n_seqs, int rows, int n_kv_heads, int group,
+                             int head_dim, int block_size, int qkv_stride,
+                             float scale, bool cache_fp8, hipStream_t stream);
+
 // The same over the paged cache (chunks and mixed batches).
 void launch_prefill_paged(const uint16_t* qkv, const void* k_cache,
                           const void* v_cache, const int32_t* chunk_row0,

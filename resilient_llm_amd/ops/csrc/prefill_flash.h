@@ -75,13 +75,43 @@ DEV_INLINE s16x4 read_tr(const uint16_t* p) {
       (__attribute__((address_space(3))) s16x4*)p);
 }
 
+// Eight channels of a rotated row, of its lower or upper half, from those and
+// their partners; ``cs``: the cosines, ``half`` before the sines.
+DEV_INLINE void rotate8(bool lower, const uint4& own, const uint4& other,
+                        const float* cs, int half, float* out) {
+  bf16x8 a, b;
+  a.u = lower ? own : other;
+  b.u = lower ? other : own;
+  float c[8], s[8];
+#pragma unroll
+  for (int i = 0; i < 8; i += 4) {
+    *reinterpret_cast<float4*>(c + i) =
+        *reinterpret_cast<const float4*>(cs + i);
+    *reinterpret_cast<float4*>(s + i) =
+        *reinterpret_cast<const float4*>(cs + half + i);
+  }
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const float x = bf16_to_f32(a.s[i]), y = bf16_to_f32(b.s[i]);
+    // rope_lower and rope_upper
+    out[i] = fmaf(x, lower ? c[i] : s[i], y * (lower ? -s[i] : c[i]));
+  }
+}
+
+DEV_INLINE uint4 flipped(const uint4& v, const uint4& f) {
+  return uint4{v.x ^ f.x, v.y ^ f.y, v.z ^ f.z, v.w ^ f.w};
+}
+
 // A source says where a workgroup's rows and keys are.  find(): which rows
 // are this tile's; false: none.  A windowed one also says which keys a row
-// sees (``window`` of them and the first ``keep``) and a head's sink.
+// sees (``window`` of them and the first ``keep``) and a head's sink.  Of kRope
+// the rows are as the product left them, one tile of keys a sequence at most:
+// queries and keys are rotated on their way in, and a tile of rows writes their
+// keys and values to the cache.
 
 template <typename C>
 struct Pages {                    // [blocks, n_kv, block, D]
-  static constexpr bool kPaged = true, kWindow = false;
+  static constexpr bool kPaged = true, kWindow = false, kRope = false;
   using KC = C;
   const uint16_t* qkv;
   const typename C::elem *k, *v;
@@ -116,7 +146,8 @@ DEV_INLINE void flash_tile(const Src& src, uint16_t* __restrict__ out,
                            int stride, float scale, const PrefillParts& parts,
                            uint16_t* lds) {
   using KC = typename Src::KC;
-  constexpr bool kDirect = std::is_same<KC, CacheBF16>::value;
+  constexpr bool kRope = Src::kRope;
+  constexpr bool kDirect = std::is_same<KC, CacheBF16>::value && !kRope;
   static_assert(KS == 1 || !Src::kWindow, "windows skip single tiles");
   constexpr int NT = 64 * W * KS;
   constexpr int CH = D / 8;                  // 16-byte pieces of a row
@@ -143,6 +174,13 @@ DEV_INLINE void flash_tile(const Src& src, uint16_t* __restrict__ out,
   i /= splits;
   const int tile = n_tiles - 1 - i / (group / W);
   int row0, nrows, first, pos0;
+  // (of kRope, a lane's row's: asked for beside what find() reads)
+  int place = 0, slot = 0;
+  if constexpr (Src::kRope) {
+    const int r = min(int(threadIdx.x) & 63, src.rows - 1);
+    place = src.positions[r];
+    slot = src.slots[r];
+  }
   if (!src.find(tile, row0, nrows, first, pos0)) return;
 
   const int tid = threadIdx.x, lane = tid & 63;
@@ -180,8 +218,26 @@ DEV_INLINE void flash_tile(const Src& src, uint16_t* __restrict__ out,
 #pragma unroll
     for (int c = 0; c < DC; ++c) {
       uint4 raw = *reinterpret_cast<const uint4*>(q + c * 16);
-      raw.x ^= flip; raw.y ^= flip; raw.z ^= flip; raw.w ^= flip;
+      if constexpr (!kRope) {
+        raw.x ^= flip; raw.y ^= flip; raw.z ^= flip; raw.w ^= flip;
+      }
       qf[c] = __builtin_bit_cast(s16x8, raw);
+    }
+    if constexpr (kRope) {
+      const int at = __shfl(place, row0 + min(qi, nrows - 1), kWave);
+      const float* cs = src.cos_sin + int64_t(at) * D;
+#pragma unroll
+      for (int c = 0; c < DC / 2; ++c) {
+        const uint4 a = __builtin_bit_cast(uint4, qf[c]);
+        const uint4 b = __builtin_bit_cast(uint4, qf[c + DC / 2]);
+        float x[8], y[8];
+        rotate8(true, a, b, cs + c * 16 + hi * 8, D / 2, x);
+        rotate8(false, b, a, cs + c * 16 + hi * 8, D / 2, y);
+        const uint4 f{flip, flip, flip, flip};
+        qf[c] = __builtin_bit_cast(s16x8, flipped(CacheBF16::from_f32(x), f));
+        qf[c + DC / 2] =
+            __builtin_bit_cast(s16x8, flipped(CacheBF16::from_f32(y), f));
+      }
     }
   }
   const float c2 = fmaxf(fabsf(scale), 1e-30f) * 1.4426950408889634f;
@@ -238,10 +294,16 @@ DEV_INLINE void flash_tile(const Src& src, uint16_t* __restrict__ out,
     }
   };
   typename KC::vec8 kr[kDirect ? 1 : NP], vr[kDirect ? 1 : NP];
+  typename KC::vec8 kr2[kRope ? NP : 1];     // the other halves' channels
   auto fetch = [&](uint16_t* buf, int kv0) {
 #pragma unroll
     for (int n = 0; n < NP; ++n) {
-      if constexpr (kDirect) {
+      if constexpr (kRope) {
+        const int other = ((k_piece(n) ^ (CH / 2)) - k_piece(n)) * 8;
+        kr[n] = *reinterpret_cast<const uint4*>(k_at(n, kv0));
+        kr2[n] = *reinterpret_cast<const uint4*>(k_at(n, kv0) + other);
+        vr[n] = *reinterpret_cast<const uint4*>(v_at(n, kv0));
+      } else if constexpr (kDirect) {
         // wave-uniform LDS base; lane l lands at base + 16 l
         uint16_t* l = buf + slot_of(n * NT + wave * 64);
         lds_load16(k_at(n, kv0), l);
@@ -253,7 +315,24 @@ DEV_INLINE void flash_tile(const Src& src, uint16_t* __restrict__ out,
     }
   };
   auto land = [&](uint16_t* buf) {           // 8-bit rows, widened
-    if constexpr (!kDirect) {
+    if constexpr (kRope) {
+#pragma unroll
+      for (int n = 0; n < NP; ++n) {
+        const int p = row_of(n), row = first + min(p, len - 1);
+        const float* cs = src.cos_sin + int64_t(__shfl(place, row, kWave)) * D +
+                          k_piece(n) % (CH / 2) * 8;
+        float f[8], g[8];
+        rotate8(k_piece(n) < CH / 2, kr[n], kr2[n], cs, D / 2, f);
+        *reinterpret_cast<uint4*>(buf + slot_of(n * NT + tid)) =
+            CacheBF16::from_f32(f);
+        *reinterpret_cast<uint4*>(buf + HALF + slot_of(n * NT + tid)) = vr[n];
+        // a row's key and value by the tile and head that have it
+        const int to = __shfl(slot, row, kWave);
+        if (p < pos0 || p >= len || i % (group / W) != 0) continue;
+        CacheBF16::to_f32(vr[n], g);
+        src.keep(to, kvh, n_kv, D, k_piece(n) * 8, f, v_piece(n) * 8, g);
+      }
+    } else if constexpr (!kDirect) {
 #pragma unroll
       for (int n = 0; n < NP; ++n) {
         float f[8];
@@ -378,7 +457,7 @@ DEV_INLINE void flash_tile(const Src& src, uint16_t* __restrict__ out,
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     uint16_t* next = lds + (cur ^ 1) * STAGE;
-    const bool more = ahead < end;
+    const bool more = !kRope && ahead < end;
     if (more) {
       fetch(next, ahead);
       look_up(after(ahead));
@@ -545,7 +624,7 @@ void by_group(const Src& src, uint16_t* out, int n_tiles, int n_kv, int group,
   if (n_tiles == 0) return;
   if (group == 1) go(I1{}, I1{});
   else if (group == 2) go(I2{}, I1{});
-  else if constexpr (Src::kWindow) go(I4{}, I1{});
+  else if constexpr (Src::kWindow || Src::kRope) go(I4{}, I1{});
   // up to a workgroup and a half per CU, and more than a few tiles of keys (us
   // with one wave per head and with two, 32/8 heads of 128: 512 rows behind
   // 1500 tokens 56.5 and 45.0, 1536 behind 1500 93 and 88; a prompt of 1000

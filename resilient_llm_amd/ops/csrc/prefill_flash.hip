@@ -9,7 +9,7 @@ namespace rlli {
 namespace {
 
 struct BatchRows {                // k and v are columns of the batch's rows
-  static constexpr bool kPaged = false, kWindow = false;
+  static constexpr bool kPaged = false, kWindow = false, kRope = false;
   using KC = CacheBF16;
   const uint16_t* qkv;
   const int32_t* cu;              // [n_seqs + 1]
@@ -49,7 +49,61 @@ struct BatchRows {                // k and v are columns of the batch's rows
   }
 };
 
+// Up to 64 rows, whose queries and keys are not rotated yet, and the cache for
+// what comes of them.
+template <typename C>
+struct RopedRows : BatchRows {
+  static constexpr bool kRope = true;
+  const int32_t* positions;
+  const float* cos_sin;
+  const int32_t* slots;
+  typename C::elem *k, *v;        // [blocks, n_kv, block, D]
+  int block_size, rows;
+
+  // eight channels of a row's key, from ``kd`` on, and of its value
+  DEV_INLINE void keep(int slot, int kvh, int n_kv, int D, int kd,
+                       const float* k8, int vd, const float* v8) const {
+    if (slot < 0) return;
+    const int64_t at = ((int64_t(slot / block_size) * n_kv + kvh) * block_size +
+                        slot % block_size) * D;
+    *reinterpret_cast<typename C::vec8*>(k + at + kd) = C::from_f32(k8);
+    *reinterpret_cast<typename C::vec8*>(v + at + vd) = C::from_f32(v8);
+  }
+};
+
 }  // namespace
+
+// Rotation and append inside, us in a layer of 45 rows, 32/8 heads of 64: launches
+// of their own 3.1 and 5.7 and a gap, in one 7.5; a prompt of the 1B model 899 and
+// 885.  What bounds it is latency: two rounds of loads, sixteen workgroups.
+void launch_prompt_rows_attn(const uint16_t* qkv, const int32_t* cu_seqlens,
+                             const int32_t* positions, const float* cos_sin,
+                             void* k_cache, void* v_cache,
+                             const int32_t* slot_mapping, uint16_t* out,
+                             int n_seqs, int rows, int n_kv_heads, int group,
+                             int head_dim, int block_size, int qkv_stride,
+                             float scale, bool cache_fp8, hipStream_t st) {
+  if (rows == 0) return;
+  auto go = [&](auto kc, auto d) {
+    using C = decltype(kc);
+    const RopedRows<C> src{{qkv, cu_seqlens, n_seqs}, positions, cos_sin,
+                           slot_mapping,
+                           static_cast<typename C::elem*>(k_cache),
+                           static_cast<typename C::elem*>(v_cache),
+                           block_size, rows};
+    // (of so few keys always by one wave a head)
+    by_group<decltype(d)::value, 0>(src, out, rows / QR + n_seqs, n_kv_heads,
+                                    group, qkv_stride, scale, rows / n_seqs,
+                                    st);
+  };
+  using D128 = std::integral_constant<int, 128>;
+  using D64 = std::integral_constant<int, 64>;
+  if (cache_fp8) {
+    if (head_dim == 128) go(CacheFP8{}, D128{}); else go(CacheFP8{}, D64{});
+  } else {
+    if (head_dim == 128) go(CacheBF16{}, D128{}); else go(CacheBF16{}, D64{});
+  }
+}
 
 void launch_prefill_rows(const uint16_t* qkv, const int32_t* cu_seqlens,
                          uint16_t* out, int n_seqs, int rows, int n_kv_heads,

@@ -65,8 +65,8 @@ __global__ void rope_kv_kernel(uint16_t* __restrict__ q,
     for (int i = 0; i < 8; ++i) {
       const float x1 = bf16_to_f32(lo.s[i]);
       const float x2 = bf16_to_f32(hi.s[i]);
-      rlo[i] = x1 * cv[i] - x2 * sv[i];
-      rhi[i] = x2 * cv[i] + x1 * sv[i];
+      rlo[i] = rope_lower(x1, x2, cv[i], sv[i]);
+      rhi[i] = rope_upper(x1, x2, cv[i], sv[i]);
       olo.s[i] = f32_to_bf16(rlo[i]);
       ohi.s[i] = f32_to_bf16(rhi[i]);
     }

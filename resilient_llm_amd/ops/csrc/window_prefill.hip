@@ -254,7 +254,7 @@ void by_cache(const WindowAttnArgs& a, hipStream_t st) {
 // ``sub`` tiles of 32 rows per tile of the table
 template <typename C>
 struct WindowPages {
-  static constexpr bool kPaged = true, kWindow = true;
+  static constexpr bool kPaged = true, kWindow = true, kRope = false;
   using KC = C;
   const uint16_t* qkv;
   const typename C::elem *k, *v;

@@ -14,11 +14,11 @@ DEV = "cuda:0"
 
 
 def feed(model, prompts, at_once, kv_dtype):
-    kv = PagedKVCache.for_model(model.config, 16, device=DEV,
+    kv = PagedKVCache.for_model(model.config, 40, device=DEV,
                                 kv_dtype=kv_dtype)
     kv.k.zero_()
     kv.v.zero_()
-    engine = LLMEngine(model, kv, max_batch_size=4)
+    engine = LLMEngine(model, kv, max_batch_size=32)
     model._prompt_rows, kept = at_once, model._prompt_rows
     try:
         logits = engine.feed([(str(i), p, [len(p) - 1])
@@ -42,6 +42,23 @@ def test_same_bits(name, lens, shifted, kv_dtype):
         model.params[f"l1.{shifted}"] = buf[1:].view(w.shape).copy_(w)
     prompts = [[(7 * i + n) % 500 + 5 for i in range(n)] for n in lens]
     one, apart = (feed(model, prompts, lambda rows: x, kv_dtype)
+                  for x in (True, False))
+    for a, b in zip(one, apart):
+        assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("name", ["tiny", "tiny-128"])
+@pytest.mark.parametrize("heads", [(4, 4), (4, 2), (8, 1)], ids=str)
+@pytest.mark.parametrize("lens", [[64], [32, 32], [31, 33], [2] * 32],
+                         ids=lambda lens: f"{len(lens)}x{lens[0]}")
+def test_rotation_inside(name, heads, lens):
+    """Tiles of rows that end where keys' do, heads in groups of any size."""
+    config = dataclasses.replace(get_config(name), n_heads=heads[0],
+                                 n_kv_heads=heads[1])
+    model = LlamaForCausalLM(config, device=DEV, dtype=torch.bfloat16, seed=1)
+    assert model._prompt_rows(64)
+    prompts = [[(7 * i + n) % 500 + 5 for i in range(n)] for n in lens]
+    one, apart = (feed(model, prompts, lambda rows: x, torch.bfloat16)
                   for x in (True, False))
     for a, b in zip(one, apart):
         assert torch.equal(a, b)

@@ -174,26 +174,43 @@ Tensor moe_run(rlli::MoeArgs& a, const Tensor& h, Tensor& ids, Tensor& w) {
               (a.gated ? 2 : 1) * int64_t(a.ffp) * a.width <
                   (int64_t(1) << 31),
               "too many rows or too wide an expert for one call");
-  // Tall tiles once experts have enough rows each to fill them.  Both lines are
-  // those of earlier, slower tiles and could lie lower.  (us for all of it, 32
-  // experts of 1024 by 2048, four each: 47 rows each by 16 245, 48 by 128 120;
-  // 375 by 128 252, 384 by 256 213.  16 of 3584 by 4096, two each: 754 and 279,
-  // 715 and 626.)
+  // Weights are streamed for few rows of an expert; tiles beyond, whose height
+  // costs nothing while reading weights is what takes long, but for few blocks of
+  // more rows than a low tile has.  (us for all of it by 16, 128 and 256 rows, 32
+  // experts of 1024 by 2048, four each: 12 rows an expert 97, 112 and 112, 18 126,
+  // 113 and 113, 38 202, 117 and 116, 150 641, 192 and 134, 300 1229, 222 and 222;
+  // 16 of 3584 by 4096, two each: 8 rows 273, 265 and 266, 38 636, 269 and 269; 8
+  // of 2048 by 1024, two each: 8 rows 34, 44 and 43, 16 43, 44 and 44, 150 -, 62
+  // and 80, 300 -, 76 and 84, 400 -, 87 and 87.)
   const int64_t each = P / a.routes;
-  a.tile_m = (a.f32 || a.width % 64 != 0 || each < 48) ? 16
-             : each < 384                              ? 128
-                                                       : 256;
+  const int64_t blocks =
+      a.experts * (((a.gated ? 2 : 1) * int64_t(a.ffp) + 255) / 256);
+  a.tile_m = (a.f32 || a.width % 64 != 0 || each < (a.width >= 4096 ? 8 : 16))
+                 ? 16
+             : blocks < 192 && each > 112 && each < 384 ? 128
+                                                        : 256;
+  // An expert's low tile right behind its full ones, so that its weights are
+  // still in the caches, where most experts have one.  (us, last and there, as
+  // above: 300 rows an expert 222 and 182, 375 214 and 186, 625 292 and 277, 875
+  // 375 and 357; but 250 168 and 189, 500 230 and 263, 750 319 and 351, 1024 408
+  // and 435, whose few low tiles fill the last round.)
+  a.together = a.tile_m == 256 && each >= 256 && each % 256 >= 24 &&
+               each % 256 <= 144;
   a.max_tiles = int(P / a.tile_m + std::min<int64_t>(a.experts, P));
   auto io = h.options().dtype(at::kInt);
   ids = at::empty({a.rows, a.top}, io);
   w = at::empty({a.rows, a.top}, h.options().dtype(at::kFloat));
+  // (the router's counts first: they are read eight bytes at a time)
+  const int64_t chosen =
+      (int64_t(a.rows) + 15) / 16 * rlli::chosen_stride(a.experts) / 2;
   Tensor plan =
-      at::empty({P + 3 * int64_t(a.max_tiles) + 2 * a.experts + 2}, io);
+      at::empty({chosen + P + 3 * int64_t(a.max_tiles) + 2}, io);
   Tensor act = at::empty({P, a.ffp}, h.options());
   Tensor y = at::empty({a.rows, a.top, a.width}, h.options());
   a.ids = ids.data_ptr<int32_t>();
   a.weights = w.data_ptr<float>();
-  a.perm = plan.data_ptr<int32_t>();
+  a.chosen = reinterpret_cast<uint16_t*>(plan.data_ptr<int32_t>());
+  a.perm = plan.data_ptr<int32_t>() + chosen;
   a.tile_expert = a.perm + P;
   a.tile_row0 = a.tile_expert + a.max_tiles;
   a.tile_rows = a.tile_row0 + a.max_tiles;

@@ -33,6 +33,11 @@ void launch_relu2(const void* x, void* out, int64_t n, bool f32,
                   hipStream_t stream);
 
 // ---- moe.hip -----------------------------------------------------------
+// experts in whole groups of four
+__host__ __device__ inline int chosen_stride(int experts) {
+  return (experts + 3) / 4 * 4;
+}
+
 struct MoeArgs {
   const void* h;           // [rows, width]
   const void* router;      // [routes, width]
@@ -46,8 +51,9 @@ struct MoeArgs {
   int32_t* tile_expert;    // [max_tiles]
   int32_t* tile_row0;      // [max_tiles]
   int32_t* tile_rows;      // [max_tiles]
-  int32_t* counters;       // [2 * experts + 2]; the last two: tiles more than
-                           // half full, others
+  int32_t* counters;       // [2]: tiles more than half full (or all), others
+  uint16_t* chosen;        // [(rows + 15) / 16, chosen_stride]: pairs of each
+                           // expert by 16 rows, 8-byte aligned; null: not kept
   void* act;               // [rows * top, ffp]
   void* y;                 // [rows, top, width]
   int rows, width, experts, top, ffp, tile_m, max_tiles;
@@ -59,6 +65,7 @@ struct MoeArgs {
   bool gated;              // gated experts, weight on the input; else relu
                            // squared, weight on the output
   float limit;
+  bool together;           // an expert's tiles follow each other
   bool f32;
 };
 void launch_moe_route(const MoeArgs& a, hipStream_t stream);

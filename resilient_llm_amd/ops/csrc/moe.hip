@@ -8,9 +8,8 @@
 //
 //   moe_route     router logits (f32 accumulation over the activation's
 //                 own values), scores, top-k
-//   moe_plan      (token, choice) pairs in expert order + row tiles; one
-//                 workgroup for decode-sized batches, three small grids
-//                 for prompts; no host round trip, so it is capturable
+//   moe_plan      (token, choice) pairs in expert order + row tiles, from the
+//                 router's counts; no host round trip, so it is capturable
 //   moe_experts   two grouped GEMMs.  Up: w * (W h) is scaled in the
 //                 accumulator, gated in registers (gate and up rows are
 //                 packed in alternating blocks of 16) and leaves as one
@@ -25,53 +24,58 @@
 #include "mix.h"
 #include "tile_product.h"
 
+#include <algorithm>
+
 namespace rlli {
 namespace {
 
 // ------------------------------------------------------------- router
-// Wave-wide reductions on the VALU, the result in every lane: rows of 16,
-// then across rows, then out of the last lane.
+// Reductions over either half of a wave on the VALU, the result in all of its
+// lanes: rows of 16, then across the two, then out of the half's last lane.
 template <int CTRL>
 DEV_INLINE float dpp_or_own(float v) {
   const int b = __builtin_bit_cast(int, v);
   return __builtin_bit_cast(
       float, __builtin_amdgcn_update_dpp(b, b, CTRL, 0xf, 0xf, false));
 }
-DEV_INLINE float last_lane(float v) {
-  return __builtin_bit_cast(
-      float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63));
+// of each half, what it has in its lane at0 or at1
+DEV_INLINE float of_lane(float v, int at0, int at1) {
+  const int b = __builtin_bit_cast(int, v);
+  const int x = __builtin_amdgcn_readlane(b, at0);
+  const int y = __builtin_amdgcn_readlane(b, 32 + at1);
+  return __builtin_bit_cast(float, threadIdx.x & 32 ? y : x);
 }
-DEV_INLINE float wave_sum_dpp(float v) {
+DEV_INLINE float half_sum_dpp(float v) {
   v = group_sum_dpp<16>(v);
-  // rows 0 + 1 | 2 + 3, then all four, in the last lane
+  // rows 0 + 1 | 2 + 3
   v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(
            0, __builtin_bit_cast(int, v), 0x142, 0xa, 0xf, false));
-  v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(
-           0, __builtin_bit_cast(int, v), 0x143, 0xc, 0xf, false));
-  return last_lane(v);
+  return of_lane(v, 31, 31);
 }
-DEV_INLINE float wave_max_dpp(float v) {
+DEV_INLINE float half_max_dpp(float v) {
   v = fmaxf(v, dpp_or_own<0x111>(v));     // row_shr 1, 2, 4, 8
   v = fmaxf(v, dpp_or_own<0x112>(v));
   v = fmaxf(v, dpp_or_own<0x114>(v));
   v = fmaxf(v, dpp_or_own<0x118>(v));
-  v = fmaxf(v, dpp_or_own<0x142>(v));     // row_bcast 15, 31
-  v = fmaxf(v, dpp_or_own<0x143>(v));
-  return last_lane(v);
+  v = fmaxf(v, dpp_or_own<0x142>(v));     // row_bcast 15
+  return of_lane(v, 31, 31);
 }
 
-// 16 rows per workgroup, K split over eight waves
+// 16 rows per workgroup, K split over eight waves, whose halves then rank a row
+// each.  What bounds it is latency: a round of loads where they fit the
+// registers (32 routes of 2048: all of them), sums through LDS, and a choice
+// after the other.  It leaves how often its rows chose each expert behind, so
+// that the plan needs no pass of its own over the choices.
 template <typename T, int ET>
 __global__ __launch_bounds__(512)
 void moe_route_kernel(MoeArgs a) {
   constexpr int E16 = ET * 16, NW = 8;
   __shared__ float part[NW][16][E16 + 1];
+  __shared__ int chosen[E16];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int lr = lane & 15, g = lane >> 4;
   const int row0 = blockIdx.x * 16;
-  // the plan's counters, for the kernels after this one
-  if (blockIdx.x == 0 && a.counters)
-    for (int e = threadIdx.x; e < 2 * a.experts; e += 512) a.counters[e] = 0;
+  if (threadIdx.x < E16) chosen[threadIdx.x] = 0;
   const T* h = reinterpret_cast<const T*>(a.h) +
                int64_t(min(row0 + lr, a.rows - 1)) * a.width;
   const T* wr = reinterpret_cast<const T*>(a.router);
@@ -119,229 +123,243 @@ void moe_route_kernel(MoeArgs a) {
     for (int r = 0; r < 4; ++r)
       part[w][g * 4 + r][e * 16 + lr] = acc[e][r];
   __syncthreads();
-  // each wave ranks two rows, lane l holding routes l, l + 64, ...
-  constexpr int EL = (E16 + 63) / 64;
+  // a half ranks a row, its lane l holding routes l, l + 32, ...
+  constexpr int EL = (E16 + 31) / 32;
   constexpr float kNone = -INFINITY;      // cannot be chosen
   auto wave_fence = [] {
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
   };
-  for (int t = w * 2; t < w * 2 + 2; ++t) {
-    const int row = row0 + t;
-    if (row >= a.rows) break;
-    float s[EL], choice[EL];
+  const int hl = lane & 31;
+  const int t = w * 2 + (lane >> 5);
+  const int row = row0 + t;               // (past the last: nobody's)
+  float s[EL], choice[EL];
+#pragma unroll
+  for (int i = 0; i < EL; ++i) {
+    const int e = i * 32 + hl;
+    s[i] = kNone;
+    if (e < a.routes) {
+      s[i] = 0.f;
+#pragma unroll
+      for (int p = 0; p < NW; ++p) s[i] += part[p][t][e];
+    }
+  }
+  if (a.softmax) {
+    float mx = kNone, sum = 0.f;
+#pragma unroll
+    for (int i = 0; i < EL; ++i) mx = fmaxf(mx, s[i]);
+    mx = half_max_dpp(mx);
 #pragma unroll
     for (int i = 0; i < EL; ++i) {
-      const int e = i * 64 + lane;
-      s[i] = kNone;
-      if (e < a.routes) {
-        s[i] = 0.f;
-#pragma unroll
-        for (int p = 0; p < NW; ++p) s[i] += part[p][t][e];
-      }
+      s[i] = expf(s[i] - mx);             // 0 past the last route
+      sum += s[i];
     }
-    if (a.softmax) {
-      float mx = kNone, sum = 0.f;
+    sum = half_sum_dpp(sum);
 #pragma unroll
-      for (int i = 0; i < EL; ++i) mx = fmaxf(mx, s[i]);
-      mx = wave_max_dpp(mx);
+    for (int i = 0; i < EL; ++i) s[i] /= sum;
+  } else {
 #pragma unroll
-      for (int i = 0; i < EL; ++i) {
-        s[i] = expf(s[i] - mx);           // 0 past the last route
-        sum += s[i];
-      }
-      sum = wave_sum_dpp(sum);
+    for (int i = 0; i < EL; ++i) s[i] = 1.f / (1.f + expf(-s[i]));
+  }
 #pragma unroll
-      for (int i = 0; i < EL; ++i) s[i] /= sum;
-    } else {
-#pragma unroll
-      for (int i = 0; i < EL; ++i) s[i] = 1.f / (1.f + expf(-s[i]));
-    }
-#pragma unroll
-    for (int i = 0; i < EL; ++i) {
-      const int e = i * 64 + lane;
-      choice[i] = kNone;
-      if (e < a.routes)
-        choice[i] = s[i] + (a.correction ? a.correction[e] : 0.f);
-    }
-    if (a.keep < a.groups) {
-      // this row's part sums are read; their place holds the choice scores,
-      // the groups' best ones, and which groups stay
-      float *cs = part[0][t], *best = part[1][t], *stays = part[2][t];
-      const int size = a.routes / a.groups;
-      wave_fence();
-#pragma unroll
-      for (int i = 0; i < EL; ++i)
-        if (i * 64 + lane < a.routes) cs[i * 64 + lane] = choice[i];
-      wave_fence();
-      for (int g = lane; g < a.groups; g += 64) {
-        float b = kNone;
-        for (int e = g * size; e < (g + 1) * size; ++e) b = fmaxf(b, cs[e]);
-        best[g] = b;
-      }
-      wave_fence();
-      for (int g = lane; g < a.groups; g += 64) {
-        int ahead = 0;
-        for (int o = 0; o < a.groups; ++o)
-          ahead += best[o] > best[g] || (best[o] == best[g] && o < g);
-        stays[g] = ahead < a.keep ? 1.f : 0.f;
-      }
-      wave_fence();
-#pragma unroll
-      for (int i = 0; i < EL; ++i) {
-        const int e = i * 64 + lane;
-        if (e < a.routes && stays[e / size] == 0.f) choice[i] = kNone;
-      }
-    }
-    float won[EL], total = 0.f;           // lane c & 63 keeps weight c
-    for (int c = 0; c < a.top; ++c) {
-      // the best score left, and the first route that has it
-      float bv = choice[0];
-#pragma unroll
-      for (int i = 1; i < EL; ++i) bv = fmaxf(bv, choice[i]);
-      bv = wave_max_dpp(bv);
-      int bi = 0x7fffffff;
-#pragma unroll
-      for (int i = EL - 1; i >= 0; --i) {
-        const uint64_t has = __ballot(choice[i] == bv);
-        if (has) bi = i * 64 + __builtin_ctzll(has);
-      }
-#pragma unroll
-      for (int i = 0; i < EL; ++i)
-        if (i * 64 + lane == bi) choice[i] = kNone;
-      bi = min(bi, a.routes - 1);       // a NaN row still names a route
-      float mine = s[0];
-#pragma unroll
-      for (int i = 1; i < EL; ++i)
-        if (bi >> 6 == i) mine = s[i];
-      mine = __builtin_bit_cast(
-          float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, mine),
-                                           bi & 63));
-      total += mine;
-#pragma unroll
-      for (int i = 0; i < EL; ++i)
-        if (c == i * 64 + lane) won[i] = mine;
-      if (lane == 0) a.ids[int64_t(row) * a.top + c] = bi;
-    }
-    const float scale = a.softmax ? 1.f / (total + 1e-20f) : 1.f;
+  for (int i = 0; i < EL; ++i) {
+    const int e = i * 32 + hl;
+    choice[i] = kNone;
+    if (e < a.routes)
+      choice[i] = s[i] + (a.correction ? a.correction[e] : 0.f);
+  }
+  if (a.keep < a.groups) {
+    // this row's part sums are read; their place holds the choice scores,
+    // the groups' best ones, and which groups stay
+    float *cs = part[0][t], *best = part[1][t], *stays = part[2][t];
+    const int size = a.routes / a.groups;
+    wave_fence();
 #pragma unroll
     for (int i = 0; i < EL; ++i)
-      if (i * 64 + lane < a.top)
-        a.weights[int64_t(row) * a.top + i * 64 + lane] = won[i] * scale;
+      if (i * 32 + hl < a.routes) cs[i * 32 + hl] = choice[i];
+    wave_fence();
+    for (int g = hl; g < a.groups; g += 32) {
+      float b = kNone;
+      for (int e = g * size; e < (g + 1) * size; ++e) b = fmaxf(b, cs[e]);
+      best[g] = b;
+    }
+    wave_fence();
+    for (int g = hl; g < a.groups; g += 32) {
+      int ahead = 0;
+      for (int o = 0; o < a.groups; ++o)
+        ahead += best[o] > best[g] || (best[o] == best[g] && o < g);
+      stays[g] = ahead < a.keep ? 1.f : 0.f;
+    }
+    wave_fence();
+#pragma unroll
+    for (int i = 0; i < EL; ++i) {
+      const int e = i * 32 + hl;
+      if (e < a.routes && stays[e / size] == 0.f) choice[i] = kNone;
+    }
   }
+  float won[EL], total = 0.f;             // lane c & 31 keeps weight c
+  for (int c = 0; c < a.top; ++c) {
+    // the best score left, and the first route that has it, of either half
+    float bv = choice[0];
+#pragma unroll
+    for (int i = 1; i < EL; ++i) bv = fmaxf(bv, choice[i]);
+    bv = half_max_dpp(bv);
+    int b0 = 0x7fffffff, b1 = b0;
+#pragma unroll
+    for (int i = EL - 1; i >= 0; --i) {
+      const uint64_t has = __ballot(choice[i] == bv);
+      if (uint32_t(has)) b0 = i * 32 + __builtin_ctz(uint32_t(has));
+      if (has >> 32) b1 = i * 32 + __builtin_ctz(uint32_t(has >> 32));
+    }
+    int bi = lane & 32 ? b1 : b0;
+#pragma unroll
+    for (int i = 0; i < EL; ++i)
+      if (i * 32 + hl == bi) choice[i] = kNone;
+    bi = min(bi, a.routes - 1);           // a NaN row still names a route
+    b0 = min(b0, a.routes - 1);
+    b1 = min(b1, a.routes - 1);
+    float mine = s[0];
+#pragma unroll
+    for (int i = 1; i < EL; ++i)
+      if (bi >> 5 == i) mine = s[i];
+    mine = of_lane(mine, b0 & 31, b1 & 31);
+    total += mine;
+#pragma unroll
+    for (int i = 0; i < EL; ++i)
+      if (c == i * 32 + hl) won[i] = mine;
+    if (hl == 0 && row < a.rows) {
+      a.ids[int64_t(row) * a.top + c] = bi;
+      atomicAdd(&chosen[bi], 1);
+    }
+  }
+  const float scale = a.softmax ? 1.f / (total + 1e-20f) : 1.f;
+#pragma unroll
+  for (int i = 0; i < EL; ++i)
+    if (i * 32 + hl < a.top && row < a.rows)
+      a.weights[int64_t(row) * a.top + i * 32 + hl] = won[i] * scale;
+  if (!a.chosen) return;
+  __syncthreads();
+  // (a row of NaN may choose one route ``top`` times: 4096 at most)
+  if (threadIdx.x < chosen_stride(a.experts))
+    a.chosen[int64_t(blockIdx.x) * chosen_stride(a.experts) + threadIdx.x] =
+        threadIdx.x < a.experts ? uint16_t(chosen[threadIdx.x]) : 0;
 }
 
 // --------------------------------------------------------------- plan
 constexpr int MAXE = 256;
 
-// The tile list: tiles more than half full in expert order, then the other
-// ones, so that the cheap tiles run where the last full ones leave compute
-// units idle.  The counts of both follow the counters of the plan.
-DEV_INLINE void write_tiles(const MoeArgs& a, const int* count,
-                            const int* start, int tid, int nthr) {
-  // index of expert e's first full tile, of its last one if that is not
-  __shared__ int tfull[MAXE + 1], tpart[MAXE + 1];
+// Pairs to places in expert order, from how often each workgroup of the router
+// chose each expert: a workgroup sums all of that and what belongs to rows ahead
+// of its own, PLAN_ROWS or more, and places its pairs.  What bounds it is latency:
+// 8.4 us for 6001 rows and 32 experts, four each, 4.8 for 64 rows.  (Two passes
+// over the choices with counts by atomics between them 14.8 and a gap, one
+// workgroup for 64 rows 6.0.)
+constexpr int PLAN_ROWS = 512, PLAN_MOST = 64;    // rows, workgroups
+
+__global__ __launch_bounds__(256)
+void moe_plan_kernel(MoeArgs a, int rows_each) {
+  __shared__ int part[2][4 * 256];        // by four experts: threads' sums
+  __shared__ int cursor[MAXE], wave_total[4][3];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int blocks = (a.rows + 15) / 16, own = blockIdx.x * rows_each / 16;
+  const int cols = chosen_stride(a.experts) / 4;
+  const int sums = min(256 / cols, min(blocks, 32));
+  // its pairs' choices, the first eight of a thread asked for at once
+  const int p0 = blockIdx.x * rows_each * a.top;
+  const int p1 = min(a.rows * a.top, p0 + rows_each * a.top);
+  constexpr int EARLY = 8;
+  int early[EARLY];
+#pragma unroll
+  for (int i = 0; i < EARLY; ++i)
+    early[i] = a.ids[min(p0 + i * 256 + tid, p1 - 1)];
+  {
+    // four experts' counts at a time: all, and of the router's workgroups
+    // ahead of this one's rows
+    const int c = tid % cols, p = tid / cols;
+    int all[4] = {0, 0, 0, 0}, ahead[4] = {0, 0, 0, 0};
+    if (p < sums) {
+      const uint2* from = reinterpret_cast<const uint2*>(a.chosen) + c;
+#pragma unroll 8
+      for (int b = p; b < blocks; b += sums) {
+        const uint2 v = from[int64_t(b) * cols];
+        const int n[4] = {int(v.x & 0xffff), int(v.x >> 16),
+                          int(v.y & 0xffff), int(v.y >> 16)};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          all[i] += n[i];
+          ahead[i] += b < own ? n[i] : 0;
+        }
+      }
+      // [p][4 c + i], as wide as the experts' columns
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        part[0][p * cols * 4 + c * 4 + i] = all[i];
+        part[1][p * cols * 4 + c * 4 + i] = ahead[i];
+      }
+    }
+  }
+  __syncthreads();
+  int n = 0, before = 0;
+  if (tid < a.experts)
+    for (int p = 0; p < sums; ++p) {
+      n += part[0][p * cols * 4 + tid];
+      before += part[1][p * cols * 4 + tid];
+    }
   const int half = a.tile_m > 16 ? a.tile_m / 2 : 0;
-  auto full = [&](int n) {
-    return n / a.tile_m + (n % a.tile_m > half ? 1 : 0);
+  const int tiles = (n + a.tile_m - 1) / a.tile_m;
+  const int full = a.together ? tiles
+                              : n / a.tile_m + (n % a.tile_m > half ? 1 : 0);
+  // pairs, full tiles and others of the experts up to each: sums over lanes,
+  // then over waves
+  int upto[3] = {n, full, tiles - full};
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1)
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      const int v = __shfl_up(upto[i], d, kWave);
+      if (lane >= d) upto[i] += v;
+    }
+  if (lane == 63)
+#pragma unroll
+    for (int i = 0; i < 3; ++i) wave_total[tid >> 6][i] = upto[i];
+  __syncthreads();
+  for (int w = 0; w < tid >> 6; ++w)
+#pragma unroll
+    for (int i = 0; i < 3; ++i) upto[i] += wave_total[w][i];
+  const int start = upto[0] - n;
+  if (tid < a.experts) cursor[tid] = start + before;
+  __syncthreads();
+  auto place = [&](int p, int e) {
+    if (p < p1 && e < a.experts) a.perm[atomicAdd(&cursor[e], 1)] = p;
   };
-  auto all = [&](int n) { return (n + a.tile_m - 1) / a.tile_m; };
-  if (tid == 0) {
-    int f = 0, p = 0;
-    for (int e = 0; e < a.experts; ++e) {
-      tfull[e] = f;
-      tpart[e] = p;
-      f += full(count[e]);
-      p += all(count[e]) - full(count[e]);
-    }
-    tfull[a.experts] = f;
-    tpart[a.experts] = p;
-    a.counters[2 * a.experts] = f;
-    a.counters[2 * a.experts + 1] = p;
+#pragma unroll
+  for (int i = 0; i < EARLY; ++i) place(p0 + i * 256 + tid, early[i]);
+  for (int p = p0 + EARLY * 256 + tid; p < p1; p += 256) place(p, a.ids[p]);
+  if (blockIdx.x != 0) return;
+
+  // The tile list: tiles more than half full in expert order, then the other
+  // ones, so that the cheap tiles run where the last full ones leave compute
+  // units idle; or all in expert order (a.together), where an expert's weights
+  // would be read twice for its two tiles.
+  int all_full = 0, others = 0;
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    all_full += wave_total[w][1];
+    others += wave_total[w][2];
   }
-  __syncthreads();
-  const int nfull = tfull[a.experts];
-  for (int e = tid; e < a.experts; e += nthr)
-    for (int i = 0; i < all(count[e]); ++i) {
-      const int r = i * a.tile_m;
-      const int t = i < full(count[e]) ? tfull[e] + i : nfull + tpart[e];
-      a.tile_expert[t] = e;
-      a.tile_row0[t] = start[e] + r;
-      a.tile_rows[t] = min(a.tile_m, count[e] - r);
-    }
-  for (int t = nfull + tpart[a.experts] + tid; t < a.max_tiles; t += nthr)
+  for (int i = 0; i < tiles; ++i) {
+    const int t = i < full ? upto[1] - full + i
+                           : all_full + upto[2] - (tiles - full);
+    a.tile_expert[t] = tid;
+    a.tile_row0[t] = start + i * a.tile_m;
+    a.tile_rows[t] = min(a.tile_m, n - i * a.tile_m);
+  }
+  for (int t = all_full + others + tid; t < a.max_tiles; t += 256)
     a.tile_rows[t] = 0;
-}
-
-__global__ __launch_bounds__(256)
-void moe_plan_one_kernel(MoeArgs a) {
-  __shared__ int count[MAXE], start[MAXE], cursor[MAXE];
-  const int tid = threadIdx.x;
-  const int P = a.rows * a.top;
-  for (int e = tid; e < a.experts; e += 256) count[e] = 0;
-  __syncthreads();
-  for (int p = tid; p < P; p += 256)
-    if (a.ids[p] < a.experts) atomicAdd(&count[a.ids[p]], 1);
-  __syncthreads();
   if (tid == 0) {
-    int s = 0;
-    for (int e = 0; e < a.experts; ++e) {
-      start[e] = s;
-      cursor[e] = s;
-      s += count[e];
-    }
+    a.counters[0] = all_full;
+    a.counters[1] = others;
   }
-  __syncthreads();
-  for (int p = tid; p < P; p += 256)
-    if (a.ids[p] < a.experts) a.perm[atomicAdd(&cursor[a.ids[p]], 1)] = p;
-  write_tiles(a, count, start, tid, 256);
-}
-
-constexpr int PLAN_PAIRS = 2048;          // pairs per workgroup
-
-__global__ __launch_bounds__(256)
-void moe_count_kernel(MoeArgs a) {
-  __shared__ int count[MAXE];
-  const int tid = threadIdx.x;
-  const int P = a.rows * a.top;
-  const int p0 = blockIdx.x * PLAN_PAIRS;
-  for (int e = tid; e < a.experts; e += 256) count[e] = 0;
-  __syncthreads();
-  for (int p = p0 + tid; p < min(P, p0 + PLAN_PAIRS); p += 256)
-    if (a.ids[p] < a.experts) atomicAdd(&count[a.ids[p]], 1);
-  __syncthreads();
-  for (int e = tid; e < a.experts; e += 256)
-    if (count[e]) atomicAdd(&a.counters[e], count[e]);
-}
-
-__global__ __launch_bounds__(256)
-void moe_scatter_kernel(MoeArgs a) {
-  __shared__ int count[MAXE], start[MAXE], total[MAXE], base[MAXE];
-  const int tid = threadIdx.x;
-  const int P = a.rows * a.top;
-  const int p0 = blockIdx.x * PLAN_PAIRS;
-  for (int e = tid; e < a.experts; e += 256) {
-    total[e] = a.counters[e];
-    count[e] = 0;
-  }
-  __syncthreads();
-  if (tid == 0) {
-    int s = 0;
-    for (int e = 0; e < a.experts; ++e) {
-      start[e] = s;
-      s += total[e];
-    }
-  }
-  for (int p = p0 + tid; p < min(P, p0 + PLAN_PAIRS); p += 256)
-    if (a.ids[p] < a.experts) atomicAdd(&count[a.ids[p]], 1);
-  __syncthreads();
-  for (int e = tid; e < a.experts; e += 256)
-    base[e] = start[e] +
-              (count[e] ? atomicAdd(&a.counters[a.experts + e], count[e]) : 0);
-  __syncthreads();
-  for (int p = p0 + tid; p < min(P, p0 + PLAN_PAIRS); p += 256)
-    if (a.ids[p] < a.experts) a.perm[atomicAdd(&base[a.ids[p]], 1)] = p;
-  if (blockIdx.x == 0) write_tiles(a, total, start, tid, 256);
 }
 
 template <typename T>
@@ -465,15 +483,22 @@ void moe_small_kernel(MoeArgs a) {
 // each: 8192 rows of 4096, 16 experts of 3584, two each: 1658-1669 ->
 // 1389-1398; 2048 rows of them 753-783 -> 604-635; 6001 rows of 2048, 32
 // experts of 1024, four each: 397-407 -> 375-381 (on another card 404 -> 396).
+enum TileKind { FULL, LOW, NARROW };
+
 DEV_INLINE bool tile_of(const MoeArgs& a, int block, int n_blocks, int& tile,
-                        int& nb) {
+                        int& nb, TileKind& kind) {
   const int x = block & 7;
-  int s = block >> 3, n = a.counters[2 * a.experts], first = 0;
+  int s = block >> 3, n = a.counters[0], first = 0;
   int per = (n * n_blocks + 7) / 8;
+  kind = FULL;
   if (s >= per) {
     s -= per;
+    // CUs that the full tiles' last round leaves idle
+    const int idle = 255 - (n * n_blocks + 255) % 256;
     first = n;
-    n = a.counters[2 * a.experts + 1];
+    n = a.counters[1];
+    kind = n * n_blocks > 2 * idle && n * n_blocks <= 128 ? NARROW : LOW;
+    if (kind == NARROW) n_blocks *= 2;
     per = (n * n_blocks + 7) / 8;
     if (s >= per) return false;
   }
@@ -490,11 +515,13 @@ template <bool UP, int MH, int NH, bool GATED>
 DEV_INLINE void moe_tile(const MoeArgs& a, int rows, int e, int p0, int nb) {
   using P = tile::Product<MH, NH>;
   constexpr int TM = P::TM, TN = P::TN;
-  static_assert(!GATED || NH % 2 == 0);
   extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
   const int K = UP ? a.width : a.ffp;
   const int N = UP ? (GATED ? 2 : 1) * a.ffp : a.width;
-  const int n0 = nb * TN;
+  // gate rows in one half of the tile, the same channels' up rows in the other
+  constexpr bool PAIRS = UP && GATED;
+  constexpr int CHANNELS = PAIRS ? TN / 2 : TN;
+  const int n0 = nb * CHANNELS, n1 = UP ? a.ffp : a.width;
 
   // the rows' pairs and weights, for the gather and the epilogue
   __shared__ int s_pair[TM];
@@ -512,13 +539,16 @@ DEV_INLINE void moe_tile(const MoeArgs& a, int rows, int e, int p0, int nb) {
         return uint32_t(UP ? s_pair[r] / a.top : p0 + min(r, rows - 1)) * K *
                2;
       },
-      [&](int r) { return uint32_t(min(n0 + r, N - 1)) * K * 2; });
+      [&](int r) {
+        const int c = min(n0 + r % CHANNELS, n1 - 1);
+        return uint32_t(PAIRS ? c / 16 * 32 + c % 16 + r / CHANNELS * 16 : c) *
+               K * 2;
+      });
   p.run(static_cast<const char*>(UP ? a.h : a.act),
         static_cast<const char*>(UP ? a.w_up : a.w_down) +
             int64_t(e) * N * K * 2,
         K / tile::KS, lds);
 
-  constexpr bool PAIRS = UP && GATED;
 #pragma unroll
   for (int i = 0; i < MH; ++i) {
     float wt[2];
@@ -530,45 +560,49 @@ DEV_INLINE void moe_tile(const MoeArgs& a, int rows, int e, int p0, int nb) {
                       : static_cast<uint16_t*>(a.y) +
                             int64_t(s_pair[tr]) * a.width;
 #pragma unroll
-    for (int b = 0; b < 2; ++b)
+    for (int b = 0; b < (PAIRS ? 1 : 2); ++b)
 #pragma unroll
-      for (int j = 0; j < NH; j += PAIRS ? 2 : 1) {
+      for (int j = 0; j < NH; ++j) {
         uint2 v[2];
 #pragma unroll
         for (int half = 0; half < 2; ++half) {
           f32x4_t f = p.acc[half][b][i][j];
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
-            // blocks of 16 gate rows and their 16 up rows by turns
             if constexpr (PAIRS)
-              f[r] = expert_gate<uint16_t>(
-                  f[r] * wt[half], p.acc[half][b][i][j + 1][r] * wt[half],
-                  a.limit);
+              f[r] = expert_gate<uint16_t>(f[r] * wt[half],
+                                           p.acc[half][1][i][j][r] * wt[half],
+                                           a.limit);
             else if constexpr (UP)
               f[r] = relu_squared(f[r]) * wt[half];
           }
           act_store4(reinterpret_cast<uint16_t*>(&v[half]), f);
         }
         const uint4 eight = P::eight(v[0], v[1]);
-        const int c = n0 + P::eight_of(b, j);
-        const int col = PAIRS ? c / 32 * 16 + c % 16 : c;
-        if (tr < rows && col < (UP ? a.ffp : a.width))
-          *reinterpret_cast<uint4*>(to + col) = eight;
+        const int col = n0 + P::eight_of(b, j);
+        if (tr < rows && col < n1) *reinterpret_cast<uint4*>(to + col) = eight;
       }
   }
 }
 
-// Tiles that are up to half full take half the height (6001 rows of 2048 in 32
-// experts of 1024, four each: 1.05 times as fast, 336 to 345 us for all of it).
+// Tiles that are up to half full take half the height.  They come last; where
+// they are few and the CUs that full ones leave idle are not for most of them,
+// they are half as wide as well, shared out over the chip.  (6001 rows of 2048 in
+// 32 experts of 1024, four each, us for all of it: full ones only 345, half the
+// height 336, and half the width 326.  8192 rows, 116 full tiles and 12 others,
+// with half the width 434 and without 417: they run beside the last full ones.)
 template <bool UP, int MH, int NH, bool GATED>
 __global__ __launch_bounds__(512, 2)
 void moe_tile_kernel(MoeArgs a, int n_blocks) {
   int tile, nb;
-  if (!tile_of(a, blockIdx.x, n_blocks, tile, nb)) return;
+  TileKind kind;
+  if (!tile_of(a, blockIdx.x, n_blocks, tile, nb, kind)) return;
   const int rows = a.tile_rows[tile];
   const int e = a.tile_expert[tile];
   const int p0 = a.tile_row0[tile];
-  if (MH == 4 && rows <= 128) moe_tile<UP, 2, NH, GATED>(a, rows, e, p0, nb);
+  if (MH == 4 && kind == FULL && rows <= 128) kind = LOW;     // a.together
+  if (kind == NARROW) moe_tile<UP, 2, NH / 2, GATED>(a, rows, e, p0, nb);
+  else if (kind == LOW) moe_tile<UP, 2, NH, GATED>(a, rows, e, p0, nb);
   else moe_tile<UP, MH, NH, GATED>(a, rows, e, p0, nb);
 }
 
@@ -608,8 +642,10 @@ void tiled_one(const MoeArgs& a, hipStream_t st) {
   using P = tile::Product<MH, NH>;
   const int nb =
       ((UP ? (GATED ? 2 : 1) * a.ffp : a.width) + P::TN - 1) / P::TN;
-  // two runs per XCD, each up to one block longer than its part
-  const int blocks = (nb * a.max_tiles + 7) / 8 * 8 + 8;
+  // Two runs per XCD, each up to one block longer than its part, and of narrow
+  // blocks two for one.
+  const int blocks =
+      (nb * a.max_tiles + 128 + 7) / 8 * 8 + 8;
   auto* k = moe_tile_kernel<UP, MH, NH, GATED>;
   if (P::LDS > 65536)
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(k),
@@ -634,15 +670,12 @@ void launch_moe_route(const MoeArgs& a, hipStream_t st) {
 }
 
 void launch_moe_plan(const MoeArgs& a, hipStream_t st) {
-  const int P = a.rows * a.top;
-  if (P == 0) return;
-  if (P <= 2 * PLAN_PAIRS) {
-    hipLaunchKernelGGL(moe_plan_one_kernel, dim3(1), dim3(256), 0, st, a);
-    return;
-  }
-  const dim3 grid((P + PLAN_PAIRS - 1) / PLAN_PAIRS);
-  hipLaunchKernelGGL(moe_count_kernel, grid, dim3(256), 0, st, a);
-  hipLaunchKernelGGL(moe_scatter_kernel, grid, dim3(256), 0, st, a);
+  if (a.rows == 0) return;
+  // whole workgroups of the router's
+  const int each = std::max(PLAN_ROWS,
+                            ((a.rows + PLAN_MOST - 1) / PLAN_MOST + 15) / 16 * 16);
+  hipLaunchKernelGGL(moe_plan_kernel, dim3((a.rows + each - 1) / each),
+                     dim3(256), 0, st, a, each);
 }
 
 void launch_moe_experts(const MoeArgs& a, hipStream_t st) {

@@ -419,6 +419,17 @@ def test_experts(T, W, E, top, ff, skew, device, dtype):
     assert rel(got.double().sum(1), want) < tol(dtype)
 
 
+@GPU
+@pytest.mark.parametrize("T,E,top,ff", [
+    # rows an expert: below and above the line to tiles, low tiles alone, tiles of
+    # 128 rows, low ones behind full ones and last
+    (63, 4, 1, 64), (64, 4, 1, 64), (100, 4, 1, 1100), (449, 4, 1, 64),
+    (452, 4, 1, 64), (300, 1, 1, 2000), (560, 2, 1, 64), (1280, 3, 1, 130),
+    (700, 2, 2, 200)])
+def test_heights_of_tiles(T, E, top, ff):
+    test_experts(T, 64, E, top, ff, 0, "cuda:0", BF16)
+
+
 @pytest.mark.parametrize("device", DEVICES)
 def test_router_ties_go_to_the_lower_expert(device):
     h = torch.ones(3, 64)

@@ -26,7 +26,9 @@ import torch.nn.functional as F
 
 from .. import ops
 from ..engine.kv_cache import KVLayer, StateLayer
-from .llama import _linear, _linear_parts, _linear_relu2
+from .llama import (
+    _USE_SKINNY, _linear, _linear_parts, _linear_relu2, lt_autotune,
+)
 from .mixed import DenseSpec, LayerSpec, MixedConfig, MixedModel
 
 
@@ -366,8 +368,12 @@ class NesizenForCausalLM(MixedModel):
             return _linear(x, w)
         return _linear_parts(x, w)
 
-    def _feed_forward(self, i: int, h: torch.Tensor) -> torch.Tensor:
+    def _feed_forward(self, i: int, h: torch.Tensor,
+                      squares: Optional[torch.Tensor]) -> torch.Tensor:
         P, f, p = self.params, self.config.layers[i].mlp, f"l{i}."
+        if squares is not None:
+            return self._last(ops.rows_linear_scaled_relu2(
+                h, squares, self.config.rms_eps, P[p + "up"]), P[p + "down"])
         if isinstance(f, DenseSpec):
             return self._last(_linear_relu2(h, P[p + "up"]), P[p + "down"])
         return ops.moe_experts(h, P[p + "router"], P[p + "w_up"],
@@ -382,15 +388,26 @@ class NesizenForCausalLM(MixedModel):
                 for q in ((1, 2) if s.mlp is not None else (1,))]
         h = ops.hyper_embed(input_ids, P["embed"], P["embed.norm"], x,
                             P["l0.hc1.in"], P["l0.norm1"], c.rms_eps)
+        squares = None          # of a norm that the feed-forward has to finish
         for n, (i, q) in enumerate(subs):
             p = f"l{i}."
-            if q == 1:
-                y = self._last(mixer(i, _linear(h, P[p + "proj"])),
-                               P[p + "o"])
-            else:
-                y = self._feed_forward(i, h)
-            y = self._reduce(y)
             mix, out = P[f"{p}hc{q}.mix"], P[f"{p}hc{q}.out"]
+            if q == 1:
+                y = mixer(i, _linear(h, P[p + "proj"]))
+                if (isinstance(c.layers[i].mlp, DenseSpec)
+                        and self.tp_world == 1 and not _USE_SKINNY
+                        and not lt_autotune.enabled()
+                        and ops.rows_streams_fit(
+                            y, P[p + "o"], x, P[p + "up"])):
+                    h, squares = ops.rows_linear_streams_(
+                        y, P[p + "o"], x, mix, out, P[p + "hc2.in"],
+                        P[p + "norm2"])
+                    continue
+                y = self._last(y, P[p + "o"])
+            else:
+                y = self._feed_forward(i, h, squares)
+                squares = None
+            y = self._reduce(y)
             split = y.dtype == torch.float32 != self.dtype
             if n + 1 < len(subs):
                 j, r = subs[n + 1]

@@ -501,6 +501,37 @@ def rows_linear_relu2(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     return torch.ops.rlli.rows_linear_relu2(x, w)
 
 
+def rows_streams_fit(x: torch.Tensor, w: torch.Tensor, streams: torch.Tensor,
+                     w_next: torch.Tensor) -> bool:
+    """Whether rows_linear_streams_ and then rows_linear_scaled_relu2 take x, w and
+    w_next."""
+    if not rows_fit(x, w) or x.shape[0] > 32 \
+            or not (w_next.dim() == 2 and w_next.shape[1] == w.shape[0]
+                    and w_next.dtype == torch.bfloat16
+                    and w_next.device == w.device and w_next.is_contiguous()
+                    and w_next.data_ptr() % 16 == 0
+                    and not w_next.requires_grad):
+        return False
+    _gpu()
+    return torch.ops.rlli.rows_streams_ok(x.shape[0], *w.shape,
+                                          streams.shape[1], w_next.shape[0])
+
+
+def rows_linear_streams_(x, w, streams, mix, out_w, in_w, gain):
+    """hyper_step of rows_linear, but for the norm's factor of a row: the next
+    sublayer's input without it, and sums of squares for
+    rows_linear_scaled_relu2."""
+    _gpu()
+    return torch.ops.rlli.rows_linear_streams_(x, w, streams, mix, out_w, in_w,
+                                               gain)
+
+
+def rows_linear_scaled_relu2(h, ss, eps: float, w):
+    """rows_linear_relu2 of what rows_linear_streams_ left, normed."""
+    _gpu()
+    return torch.ops.rlli.rows_linear_scaled_relu2(h, ss, eps, w)
+
+
 def _tiles_take(x: torch.Tensor, w: torch.Tensor, faster) -> bool:
     """Whether the kernel of tiles takes x w^T and ``faster`` (rows, N, K)."""
     return (x.dim() == w.dim() == 2 and x.is_cuda

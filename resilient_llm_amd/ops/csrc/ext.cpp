@@ -910,6 +910,76 @@ std::tuple<Tensor, Tensor> rows_norm_linear(const Tensor& parts,
   return {out, after};
 }
 
+// Of up to 32 rows, the first of two products that share a norm: x w^T into the
+// streams, what is normed of them times the gains, and sums of squares
+// [N / 16, 16 or 32].
+std::tuple<Tensor, Tensor> rows_linear_streams_(
+    const Tensor& x, const Tensor& w, Tensor streams, const Tensor& mix,
+    const Tensor& out_w, const Tensor& in_w, const Tensor& gain) {
+  check_rows(x, w);
+  auto f32 = [&](const Tensor& t, int64_t n, const char* name) {
+    TORCH_CHECK(t.scalar_type() == at::kFloat && t.is_contiguous() &&
+                    t.numel() == n && t.device() == x.device(),
+                name, " must be ", n, " contiguous f32 beside x");
+  };
+  const int M = int(x.size(0)), N = int(w.size(0)), K = int(x.size(1));
+  TORCH_CHECK(streams.dim() == 3 && streams.size(0) == M &&
+                  streams.size(2) == N, "streams of the product's rows");
+  const int S = int(streams.size(1));
+  TORCH_CHECK(rlli::rows_adds_ok(M, N, K, S), "not for these sizes: ", M,
+              " rows, ", N, " x ", K, ", ", S, " streams");
+  f32(streams, streams.numel(), "streams");
+  f32(mix, S * S, "mix");
+  f32(out_w, S, "out_w");
+  f32(in_w, S, "in_w");
+  f32(gain, N, "gain");
+  TORCH_CHECK((reinterpret_cast<uintptr_t>(streams.data_ptr()) |
+               reinterpret_cast<uintptr_t>(gain.data_ptr())) % 16 == 0,
+              "streams and gains start at multiples of 16 bytes");
+  Tensor h = at::empty({M, N}, x.options());
+  Tensor ss = at::empty({N / 16, M <= 16 ? 16 : 32},
+                        x.options().dtype(at::kFloat));
+  c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
+  rlli::launch_rows_adds(
+      bf16_ptr(x), bf16_ptr(w), bf16_ptr(h), M, N, K, S,
+      rlli::RowsAdds{streams.data_ptr<float>(), mix.data_ptr<float>(),
+                     out_w.data_ptr<float>(), in_w.data_ptr<float>(),
+                     gain.data_ptr<float>(), ss.data_ptr<float>()},
+      current_stream(x));
+  check_launch("rows_linear_streams_");
+  return {h, ss};
+}
+
+// Whether the two take m rows, weights [n, k] and then [next, n].
+bool rows_streams_ok(int64_t m, int64_t n, int64_t k, int64_t streams,
+                     int64_t next) {
+  return rlli::rows_adds_ok(int(m), int(n), int(k), int(streams)) &&
+         rlli::rows_scaled_ok(int(m), int(next), int(n));
+}
+
+// The second of them, the squared positive part of its result.
+Tensor rows_linear_scaled_relu2(const Tensor& h, const Tensor& ss, double eps,
+                                const Tensor& w) {
+  check_rows(h, w);
+  const int M = int(h.size(0)), N = int(w.size(0)), K = int(h.size(1));
+  TORCH_CHECK(rlli::rows_scaled_ok(M, N, K), "not for these sizes: ", M,
+              " rows, ", N, " x ", K);
+  TORCH_CHECK(ss.scalar_type() == at::kFloat && ss.is_contiguous() &&
+                  ss.dim() == 2 && ss.size(0) * 16 == K && ss.size(0) <= 256 &&
+                  ss.size(1) == (M <= 16 ? 16 : 32) &&
+                  ss.device() == h.device() &&
+                  reinterpret_cast<uintptr_t>(ss.data_ptr()) % 16 == 0,
+              "sums of squares of the rows by sixteen columns");
+  Tensor out = at::empty({M, N}, h.options());
+  c10::hip::HIPGuardMasqueradingAsCUDA guard(h.device());
+  rlli::launch_rows_scaled_relu2(
+      bf16_ptr(h), bf16_ptr(w), bf16_ptr(out), M, N, K,
+      rlli::RowsScale{ss.data_ptr<float>(), int(ss.size(0)), K, float(eps)},
+      current_stream(h));
+  check_launch("rows_linear_scaled_relu2");
+  return out;
+}
+
 static void check_tiles(const Tensor& x, const Tensor& w, int multiple) {
   check_bf16_contig(x, "x");
   check_bf16_contig(w, "w");
@@ -1286,6 +1356,13 @@ TORCH_LIBRARY(rlli, m) {
         &rows_norm_ok);
   m.def("rows_norm_linear(Tensor parts, Tensor residual, Tensor gain, "
         "float eps, Tensor w, bool silu) -> (Tensor, Tensor)");
+  m.def("rows_streams_ok(int m, int n, int k, int streams, int next) -> bool",
+        &rows_streams_ok);
+  m.def("rows_linear_streams_(Tensor x, Tensor w, Tensor(a!) streams, "
+        "Tensor mix, Tensor out_w, Tensor in_w, Tensor gain) -> "
+        "(Tensor, Tensor)");
+  m.def("rows_linear_scaled_relu2(Tensor h, Tensor ss, float eps, Tensor w) "
+        "-> Tensor");
   m.def("tile_linear_parts(Tensor x, Tensor w, int[] plan=[]) -> Tensor");
   m.def("tile_linear(Tensor x, Tensor w, int[] plan=[]) -> Tensor");
   m.def("tile_linear_silu(Tensor x, Tensor w, int[] plan=[]) -> Tensor");
@@ -1335,6 +1412,8 @@ TORCH_LIBRARY_IMPL(rlli, CUDA, m) {
   m.impl("rows_linear_silu", &rows_linear_silu);
   m.impl("rows_linear_relu2", &rows_linear_relu2);
   m.impl("rows_norm_linear", &rows_norm_linear);
+  m.impl("rows_linear_streams_", &rows_linear_streams_);
+  m.impl("rows_linear_scaled_relu2", &rows_linear_scaled_relu2);
   m.impl("tile_linear_parts", &tile_linear_parts);
   m.impl("tile_linear", &tile_linear);
   m.impl("tile_linear_silu", &tile_linear_silu);

@@ -184,6 +184,28 @@ void launch_rows_norm(const RowsNorm& norm, const uint16_t* w, float* parts,
 void launch_rows_norm_silu(const RowsNorm& norm, const uint16_t* w,
                            uint16_t* out, int inter, int K,
                            hipStream_t stream);
+// A norm that two products share, of up to 32 rows.  The first adds its result to
+// the streams [M, S, N] (each takes out_w of it and mix [from, to] of all, and in_w
+// of each is what is normed) and writes rows times gains and sums of squares
+// [N / 16, 16 or 32]; the second takes both, for its squared positive part.
+struct RowsAdds {
+  float* streams;
+  const float *mix, *out_w, *in_w, *gain;
+  float* ss;
+};
+struct RowsScale {
+  const float* ss;
+  int panels, width;           // N / 16 and N of the first product
+  float eps;
+};
+bool rows_adds_ok(int M, int N, int K, int streams);
+void launch_rows_adds(const uint16_t* x, const uint16_t* w, uint16_t* out,
+                      int M, int N, int K, int streams, const RowsAdds& adds,
+                      hipStream_t stream);
+bool rows_scaled_ok(int M, int N, int K);
+void launch_rows_scaled_relu2(const uint16_t* x, const uint16_t* w,
+                              uint16_t* out, int M, int N, int K,
+                              const RowsScale& scale, hipStream_t stream);
 // M <= 64 where rows_short_tiles is not 0; ``relu2``: squared positive part
 int rows_short_tiles(int N, int K);
 void launch_rows_short(const uint16_t* x, const uint16_t* w, uint16_t* out,

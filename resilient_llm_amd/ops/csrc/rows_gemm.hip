@@ -258,6 +258,51 @@ DEV_INLINE void combine_row(const RowsCombine& a, int c0, int c1, int t,
 
 enum { NO_PRE = 0, PRE_NORM = 1, PRE_COMBINE = 2 };
 
+// ---- a norm shared between two products ---------------------------------
+// The product ahead of a norm, where it is whole, adds its result to the
+// streams and leaves rows times gains and, by sixteen columns, their sums of
+// squares behind (ADDS of rows_short_kernel); the product behind it multiplies
+// its sums by what the norm would have multiplied the rows by.  The norm's launch
+// is gone; rows are rounded to 16 bits once, as before.  us, apart and so, two
+// streams of 2048 behind 2048 x 2048 and ahead of 6144 x 2048 with the squared
+// positive part: 1 row 12.9 and 11.5, 16 14.9 and 12.7, 32 17.2 and 14.8.  (Not
+// where the first product is faster in parts: 2048 x 6144, 16 rows 16.7 and 17.8.
+// With one 16-bit residual, 4096 x 4096 and 28672 x 4096 with silu: 16 rows 46.1
+// and 44.9, 32 47.7 and 47.6, which is not worth another order of roundings.)
+template <int MT>
+struct Scale {
+  static constexpr int Q = MT * 4;        // four rows each
+  f32x4 v[Q];
+  // ``part``: [4][16 MT], for a workgroup of 256
+  DEV_INLINE void ask(const RowsScale& a) {
+    const int q = threadIdx.x % Q, p0 = threadIdx.x / Q;
+#pragma unroll
+    for (int i = 0; i < Q; ++i)
+      v[i] = *reinterpret_cast<const f32x4*>(
+          a.ss + (min(p0 + i * (256 / Q), a.panels - 1) * Q + q) * 4);
+  }
+  DEV_INLINE void land(const RowsScale& a, float* part) {
+    const int q = threadIdx.x % Q, p0 = threadIdx.x / Q;
+    f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < Q; ++i)
+      if (p0 + i * (256 / Q) < a.panels) sum += v[i];
+#pragma unroll
+    for (int d = Q; d < 64; d <<= 1)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) sum[r] += __shfl_xor(sum[r], d, kWave);
+    if ((threadIdx.x & 63) < Q)
+      *reinterpret_cast<f32x4*>(part + (threadIdx.x >> 6) * 16 * MT + q * 4) =
+          sum;
+  }
+  static DEV_INLINE float of(const RowsScale& a, const float* part, int row) {
+    float ss = 0.f;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) ss += part[w * 16 * MT + row];
+    return rsqrtf(ss / a.width + a.eps);
+  }
+};
+
 // CT: 16-row tiles of w per wave; XR: rows of x that are staged; MT: 16-row
 // tiles of x; R: steps in the ring.  OUT_SILU: a wave's first tile is of the
 // gate's rows, the second the same rows of the upper half of w.
@@ -456,11 +501,16 @@ void rows_gemm_kernel(const uint16_t* __restrict__ x,
 // is no barrier before the sums meet at the end.  What bounds it is the time
 // from the launch to the first data and, past 4096 in K, that it reads x once
 // per 16 or 32 rows of w.
-template <int PT, int XR, int MT, int R, bool RELU2>
+// END: the result, its squared positive part, or (ADDS; PT 1) S streams with it.
+enum End { WHOLE, RELU2, ADDS };
+
+template <int PT, int XR, int MT, int R, End END, int S = 0,
+          bool SCALED = false>
 __global__ __launch_bounds__(256)
 void rows_short_kernel(const uint16_t* __restrict__ x,
                        const uint16_t* __restrict__ w,
-                       uint16_t* __restrict__ out, int M, int N, int K) {
+                       uint16_t* __restrict__ out, int M, int N, int K,
+                       RowsScale scale, RowsAdds adds) {
   constexpr int WPART = PT * 16 * LINE;              // elements of a step
   constexpr int STEP = WPART + XR * LINE;
   constexpr int LX = XR / 8, L = PT * 2 + LX;        // loads of a wave
@@ -507,9 +557,31 @@ void rows_short_kernel(const uint16_t* __restrict__ x,
     for (int m = 0; m < MT; ++m) acc[t][m] = f32x4{0.f, 0.f, 0.f, 0.f};
   const int tr = lane & 15, oct = lane >> 4;
   const int sw = tr >> 1;
+  __shared__ __attribute__((aligned(16))) float part[SCALED ? 64 * MT : 4];
+  Scale<SCALED ? MT : 1> sc;
+  if constexpr (SCALED) sc.ask(scale);
+  // what a lane of wave m < MT adds to: four columns of row 16 m + tr
+  const int arow = min(wv * 16 + tr, M - 1), acol = n0 + oct * 4;
+  f32x4 had[S > 0 ? S : 1], gain;
+  float mix[S > 0 ? S : 1][S > 0 ? S : 1], outw[S > 0 ? S : 1],
+      inw[S > 0 ? S : 1];
+  if constexpr (END == ADDS) {
+    static_assert(PT == 1 && MT <= 4, "");
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+      had[s] = *reinterpret_cast<const f32x4*>(
+          adds.streams + (int64_t(arow) * S + s) * N + acol);
+      outw[s] = adds.out_w[s];
+      inw[s] = adds.in_w[s];
+#pragma unroll
+      for (int t = 0; t < S; ++t) mix[s][t] = adds.mix[s * S + t];
+    }
+    gain = *reinterpret_cast<const f32x4*>(adds.gain + acol);
+  }
 #pragma unroll
   for (int s = 0; s < R - 1; ++s)
     if (s < n) issue(s, s);
+  if constexpr (SCALED) sc.land(scale, part);
   int slot = 0;
   for (int s = 0; s < n; ++s) {
     wait_steps<L, R - 2>(n - 1 - s);
@@ -556,15 +628,42 @@ void rows_short_kernel(const uint16_t* __restrict__ x,
     f32x4 v = side[e * 64 + lane];
 #pragma unroll
     for (int o = 1; o < 4; ++o) v += side[(o * PT * MT + e) * 64 + lane];
-    if constexpr (RELU2) {
+    const int row = e % MT * 16 + tr;
+    const int c = n0 + e / MT * 16 + oct * 4;
+    if constexpr (SCALED) v *= Scale<SCALED ? MT : 1>::of(scale, part, row);
+    if constexpr (END == RELU2) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         v[r] = fmaxf(v[r], 0.f);
         v[r] *= v[r];
       }
     }
-    const int row = e % MT * 16 + tr;
-    const int c = n0 + e / MT * 16 + oct * 4;
+    if constexpr (END == ADDS) {
+      // (of one tile a wave, e is wv)
+      f32x4 u = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int t = 0; t < S; ++t) {
+        f32x4 to;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          float sum = outw[t] * v[r];
+#pragma unroll
+          for (int s = 0; s < S; ++s) sum += mix[s][t] * had[s][r];
+          to[r] = sum;
+          u[r] += inw[t] * sum;
+        }
+        if (row < M)
+          *reinterpret_cast<f32x4*>(adds.streams +
+                                    (int64_t(row) * S + t) * N + c) = to;
+      }
+      float ss = 0.f;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) ss += u[r] * u[r];
+      ss += __shfl_xor(ss, 16, kWave);
+      ss += __shfl_xor(ss, 32, kWave);
+      if (oct == 0) adds.ss[int64_t(blockIdx.x) * 16 * MT + row] = ss;
+      v = u * gain;
+    }
     if (row < M && c < N)
       *reinterpret_cast<uint2*>(out + int64_t(row) * N + c) =
           uint2{pack2(v[0], v[1]), pack2(v[2], v[3])};
@@ -632,24 +731,45 @@ void go_norm(const RowsNorm& norm, const uint16_t* w, void* out, int N, int K,
                      RowsCombine{});
 }
 
-template <int PT, int R16, int R32, int R64, bool RELU2>
+template <int PT, int R16, int R32, int R64, End END>
 void go_short(const uint16_t* x, const uint16_t* w, uint16_t* out, int M,
               int N, int K, hipStream_t st) {
   auto run = [&](auto xr) {
     constexpr int XR = decltype(xr)::value, MT = XR / 16;
     constexpr int R = XR == 16 ? R16 : XR == 32 ? R32 : R64;
     constexpr size_t smem = size_t(4) * R * (PT * 16 + XR) * LINE * 2;
-    auto* k = rows_short_kernel<PT, XR, MT, R, RELU2>;
+    auto* k = rows_short_kernel<PT, XR, MT, R, END>;
     if (smem > 65536)
       (void)hipFuncSetAttribute(reinterpret_cast<const void*>(k),
                                 hipFuncAttributeMaxDynamicSharedMemorySize,
                                 int(smem));
     hipLaunchKernelGGL(k, dim3((N + PT * 16 - 1) / (PT * 16)), dim3(256), smem,
-                       st, x, w, out, M, N, K);
+                       st, x, w, out, M, N, K, RowsScale{}, RowsAdds{});
   };
   if (M <= 16) run(std::integral_constant<int, 16>{});
   else if (M <= 32) run(std::integral_constant<int, 32>{});
   else run(std::integral_constant<int, 64>{});
+}
+
+// with a norm that is shared, up to 32 rows
+template <int PT, int R16, int R32, End END, int S, bool SCALED>
+void go_shared(const uint16_t* x, const uint16_t* w, uint16_t* out, int M,
+               int N, int K, const RowsScale& scale, const RowsAdds& adds,
+               hipStream_t st) {
+  auto run = [&](auto xr) {
+    constexpr int XR = decltype(xr)::value, MT = XR / 16;
+    constexpr int R = XR == 16 ? R16 : R32;
+    constexpr size_t smem = size_t(4) * R * (PT * 16 + XR) * LINE * 2;
+    auto* k = rows_short_kernel<PT, XR, MT, R, END, S, SCALED>;
+    if (smem > 65536)
+      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(k),
+                                hipFuncAttributeMaxDynamicSharedMemorySize,
+                                int(smem));
+    hipLaunchKernelGGL(k, dim3((N + PT * 16 - 1) / (PT * 16)), dim3(256), smem,
+                       st, x, w, out, M, N, K, scale, adds);
+  };
+  if (M <= 16) run(std::integral_constant<int, 16>{});
+  else run(std::integral_constant<int, 32>{});
 }
 
 }  // namespace
@@ -765,12 +885,48 @@ void launch_rows_short(const uint16_t* x, const uint16_t* w, uint16_t* out,
                        int M, int N, int K, bool relu2, hipStream_t st) {
   const bool one = rows_short_tiles(N, K) == 1;
   if (relu2) {
-    if (one) go_short<1, 9, 6, 3, true>(x, w, out, M, N, K, st);
-    else go_short<2, 6, 4, 3, true>(x, w, out, M, N, K, st);
+    if (one) go_short<1, 9, 6, 3, RELU2>(x, w, out, M, N, K, st);
+    else go_short<2, 6, 4, 3, RELU2>(x, w, out, M, N, K, st);
   } else {
-    if (one) go_short<1, 9, 6, 3, false>(x, w, out, M, N, K, st);
-    else go_short<2, 6, 4, 3, false>(x, w, out, M, N, K, st);
+    if (one) go_short<1, 9, 6, 3, WHOLE>(x, w, out, M, N, K, st);
+    else go_short<2, 6, 4, 3, WHOLE>(x, w, out, M, N, K, st);
   }
+}
+
+bool rows_adds_ok(int M, int N, int K, int streams) {
+  return M >= 1 && M <= 32 && N % 16 == 0 && N <= 4096 && K % 64 == 0 &&
+         rows_short_tiles(N, K) == 1 && streams >= 1 && streams <= 4;
+}
+
+void launch_rows_adds(const uint16_t* x, const uint16_t* w, uint16_t* out,
+                      int M, int N, int K, int streams, const RowsAdds& adds,
+                      hipStream_t st) {
+  auto run = [&](auto s) {
+    go_shared<1, 9, 6, ADDS, decltype(s)::value, false>(
+        x, w, out, M, N, K, RowsScale{}, adds, st);
+  };
+  switch (streams) {
+    case 1: return run(std::integral_constant<int, 1>{});
+    case 2: return run(std::integral_constant<int, 2>{});
+    case 3: return run(std::integral_constant<int, 3>{});
+    default: return run(std::integral_constant<int, 4>{});
+  }
+}
+
+bool rows_scaled_ok(int M, int N, int K) {
+  return M >= 1 && M <= 32 && N % 4 == 0 && K % 64 == 0 &&
+         rows_short_tiles(N, K) > 0;
+}
+
+void launch_rows_scaled_relu2(const uint16_t* x, const uint16_t* w,
+                              uint16_t* out, int M, int N, int K,
+                              const RowsScale& scale, hipStream_t st) {
+  if (rows_short_tiles(N, K) == 1)
+    go_shared<1, 9, 6, RELU2, 0, true>(x, w, out, M, N, K, scale, RowsAdds{},
+                                       st);
+  else
+    go_shared<2, 6, 4, RELU2, 0, true>(x, w, out, M, N, K, scale, RowsAdds{},
+                                       st);
 }
 
 void launch_sum_parts(const float* parts, uint16_t* out, int splits,

@@ -54,6 +54,7 @@ LIBRARIES = {
     "rlli_attn": [
         "ext_attn.cpp",
         "window_attn.hip",
+        "window_units.hip",
         "diff_attn.hip",
         "expanded_attn.hip",
     ],
@@ -84,7 +85,7 @@ _ATTN = _ACT + ["attn.h", "attn_rows.h", "ext_window.h"]
 HEADERS = {"rlli_hip": ["common.h", "decode_attn.h", "decode_parts.h",
                         "kernels.h", "prefill_flash.h", "prefill_parts.h",
                         "tile_product.h"],
-           "rlli_attn": _ATTN,
+           "rlli_attn": _ATTN + ["decode_attn.h", "decode_parts.h"],
            "rlli_mix": _ATTN + ["mix.h", "prefill_flash.h", "prefill_parts.h",
                                 "tile_product.h"],
            "rlli_blk": _ACT + ["blk.h"],

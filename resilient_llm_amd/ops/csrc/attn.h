@@ -67,6 +67,11 @@ bool diff_fast_ok(const WindowAttnArgs& a);
 int diff_head_blocks(int group);     // workgroups per kv head, sequence, split
 void launch_window_rope_append(const WindowAttnArgs& a, hipStream_t stream);
 void launch_window_decode(const WindowAttnArgs& a, hipStream_t stream);
+void launch_window_combine(const WindowAttnArgs& a, hipStream_t st);
+// The same by units of 32 tokens on the matrix cores, where window_units_ok.
+bool window_units_ok(const WindowAttnArgs& a);
+int window_units_splits(const WindowAttnArgs& a, int units);
+void launch_window_units(const WindowAttnArgs& a, hipStream_t st);
 void launch_window_rows(const WindowAttnArgs& a, bool decode,
                         hipStream_t stream);
 void launch_window_prefill(const WindowAttnArgs& a, hipStream_t stream);

@@ -51,9 +51,19 @@ void window_append(const Tensor& qkv, const Tensor& k_cache,
   check_launch("window_append");
 }
 
-// splits of a decode step that fill the chip, and room for their results;
-// ``visible``: the most tokens that a query sees
-// ``head_blocks``: workgroups per sequence, kv head and split
+// room for the results of a decode step's splits
+void decode_parts(rlli::WindowAttnArgs& a, const Tensor& qkv, Tensor& pa,
+                  Tensor& pm) {
+  if (a.n_split == 1) return;
+  auto fo = qkv.options().dtype(at::kFloat);
+  pa = at::empty({a.rows, a.n_q, a.maps, a.n_split, a.vdim}, fo);
+  pm = at::empty({a.rows, a.n_q, a.maps, a.n_split, 2}, fo);
+  a.part_acc = pa.data_ptr<float>();
+  a.part_ml = pm.data_ptr<float>();
+}
+
+// splits of a decode step that fill the chip; ``visible``: the most tokens that a
+// query sees, ``head_blocks``: workgroups per sequence, kv head and split
 void decode_splits(rlli::WindowAttnArgs& a, const Tensor& qkv,
                    int head_blocks, int64_t visible, Tensor& pa, Tensor& pm) {
   const int64_t wgs =
@@ -64,12 +74,7 @@ void decode_splits(rlli::WindowAttnArgs& a, const Tensor& qkv,
   const int64_t useful = std::max<int64_t>(1, reach / 64);
   a.n_split = int(std::min<int64_t>(
       {16, useful, std::max<int64_t>(1, (512 + wgs - 1) / wgs)}));
-  if (a.n_split == 1) return;
-  auto fo = qkv.options().dtype(at::kFloat);
-  pa = at::empty({a.rows, a.n_q, a.maps, a.n_split, a.vdim}, fo);
-  pm = at::empty({a.rows, a.n_q, a.maps, a.n_split, 2}, fo);
-  a.part_acc = pa.data_ptr<float>();
-  a.part_ml = pm.data_ptr<float>();
+  decode_parts(a, qkv, pa, pm);
 }
 
 // prompt rows, one wave each, at any sizes
@@ -128,9 +133,18 @@ Tensor window_decode(const Tensor& qkv, const Tensor& k_cache,
   }
   const int group = a.n_q / a.n_kv;
   const int hb = rlli::window_decode_heads_per_wg(group);
+  const int64_t visible = int64_t(a.window) + a.keep_first + 32;
   Tensor pa, pm;
-  decode_splits(a, qkv, (group + hb - 1) / hb,
-                int64_t(a.window) + a.keep_first + 32, pa, pm);
+  if (rlli::window_units_ok(a)) {
+    const int64_t reach = std::min<int64_t>(
+        int64_t(a.max_blocks) * a.block_size, visible + 32);
+    a.n_split = rlli::window_units_splits(a, int((reach + 31) / 32));
+    decode_parts(a, qkv, pa, pm);
+    rlli::launch_window_units(a, st);
+    check_launch("window_decode");
+    return out;
+  }
+  decode_splits(a, qkv, (group + hb - 1) / hb, visible, pa, pm);
   rlli::launch_window_decode(a, st);
   check_launch("window_decode");
   return out;

@@ -13,6 +13,7 @@
 //   window_rope_append  rotate q in place, rotate and cache k, cache v
 //   window_decode       one new token per sequence, split over the
 //                       visible cache blocks; rotation and append fused
+// window_units.hip has decode on the matrix cores, for the sizes it takes;
 // attn_rows.h has window_rows, any sizes and dtypes: the 32-bit path and
 // the shapes that the tiled kernels do not take.
 // The tiled prefill kernel is window_prefill.hip.
@@ -480,10 +481,12 @@ void launch_window_decode(const WindowAttnArgs& a, hipStream_t st) {
   else if (d <= 64) by_heads(std::integral_constant<int, 8>{});
   else if (d <= 128) by_heads(std::integral_constant<int, 16>{});
   else by_heads(std::integral_constant<int, 32>{});
-  if (a.n_split > 1)
-    hipLaunchKernelGGL(window_combine_kernel, dim3(a.rows * a.n_q),
-                       dim3(std::min(256, (a.vdim + 63) / 64 * 64)), 0, st,
-                       a);
+  if (a.n_split > 1) launch_window_combine(a, st);
+}
+
+void launch_window_combine(const WindowAttnArgs& a, hipStream_t st) {
+  hipLaunchKernelGGL(window_combine_kernel, dim3(a.rows * a.n_q),
+                     dim3(std::min(256, (a.vdim + 63) / 64 * 64)), 0, st, a);
 }
 
 }  // namespace rlli

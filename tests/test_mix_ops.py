@@ -252,6 +252,38 @@ def test_decode_batches_and_splits():
 
 
 @GPU
+@pytest.mark.parametrize("H,G,dim", [(8, 2, 128), (4, 2, 64), (2, 2, 128)])
+@pytest.mark.parametrize("window,keep", [(1000, 40), (64, 4), (33, 0)])
+def test_decode_units(H, G, dim, window, keep):
+    """Windows and kept tokens that begin and end where units of 32 tokens, waves
+    and parts of a sequence do; pages of 16 and of 48 tokens."""
+    T = 1345
+    a = Attn(T, H, G, dim, dim, 32, window, keep, "cuda:0", BF16)
+    a.run(0, T)
+    want = a.want()
+    at = [0, 1, 31, 32, 33, 63, 64, 383, 384, 999, 1000, 1031, 1063, 1064, 1343,
+          T - 1]
+    for i in at:
+        assert rel(a.run(i, 1, decode=True), want[i:i + 1]) < tol(BF16), i
+    # pages three times as long, all of the sequence in a row
+    n = -(-T // 48)
+    pages = [torch.full((n, G, 48, dim), float("nan"), dtype=BF16,
+                        device="cuda:0") for _ in "kv"]
+    for to, src in zip(pages, (a.kc, a.vc)):
+        flat = src[a.table[0].long()].transpose(0, 1).flatten(1, 2)
+        for b in range(n):
+            part = flat[:, b * 48:(b + 1) * 48]
+            to[b, :, :part.shape[1]] = part
+    table = torch.arange(n, dtype=torch.int32, device="cuda:0")[None]
+    for i in at:
+        pos = torch.tensor([i], dtype=torch.int32, device="cuda:0")
+        got = ops.window_decode(
+            a.qkv(i, 1), *pages, pos, a.cs, pos, table,
+            a.sink.to("cuda:0"), a.scale, H, window, keep, True)
+        assert rel(got, want[i:i + 1]) < tol(BF16), i
+
+
+@GPU
 def test_fp8_cache():
     a = Attn(120, 8, 2, 64, 64, 32, 50, 4, "cuda:0", BF16,
              cache_dtype=torch.float8_e4m3fn)

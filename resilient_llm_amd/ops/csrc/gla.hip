@@ -64,91 +64,151 @@ DEV_INLINE float log_rwkv(float z) {
 
 // ------------------------------------------------------------- decode
 // One workgroup per sequence and head; what there is to do is to read and
-// write the state, of which NT threads have eight rows each in flight.
-template <typename T, int KIND, int NT>
+// write the state, of which NT threads have U rows each in flight.  Few
+// sequences leave a chain of round trips, so everything is asked for at once,
+// what the decays are made from first and the state behind it, and nothing
+// that was loaded decides what to load but the state's slot.  16 sequences of
+// 8 heads of 128 x 256 with states in HBM: 13.9 us when the state was asked for
+// after the decays, which one thread a channel made, now 11.7; 1 sequence 7.7
+// and 6.8, 64 of them 34.3 and 31.3.
+template <typename T, int KIND, int NT, int U>
 __global__ __launch_bounds__(NT)
-void gla_decode_kernel(GlaArgs a) {
+void gla_decode_kernel(GlaArgs a, bool vec_a2) {
   constexpr bool FG = KIND == kHgrn2, BONUS = KIND == kRwkv;
   extern __shared__ __attribute__((aligned(16))) float sm[];
   const int seq = blockIdx.x, h = blockIdx.y;
   const int tid = threadIdx.x;
-  float* al = sm;                       // [dim]
-  float* ks = al + a.dpad;              // [dim]
-  float* qs = ks + a.dpad;              // [dim]
-  float* uk = qs + a.dpad;              // [dim] bonus times key (RWKV)
-  float* a1 = uk + (BONUS ? a.dpad : 0);    // [rank, padded to 4]
-  float* red = a1 + (a.rank + 3) / 4 * 4;   // [rows][vpad] then sums
+  // [dim] decay, key, query and (RWKV) bonus times key
+  f32x4_t* chan = reinterpret_cast<f32x4_t*>(sm);
+  float* red = sm + 4 * a.dpad;         // [rows][vpad] then sums
   const T* row = reinterpret_cast<const T*>(a.proj) + int64_t(seq) * a.stride;
-  if constexpr (FG) {
-    for (int d = tid; d < a.dim; d += NT) {
-      const int hc = h * a.dim + d;
-      qs[d] = silu<T>(act_load(row + hc));
-      ks[d] = forget_key<T>(act_load(row + a.off_k + hc) + a.a2_bias[hc],
-                            a.lower[hc], al + d);
-    }
-  } else {
-    const T* low =
-        reinterpret_cast<const T*>(a.a1) + int64_t(seq) * a.a1_stride;
-    for (int r = tid; r < a.rank; r += NT)
-      a1[r] = BONUS ? gtanh<T>(act_load(low + r)) : act_load(low + r);
-    const float qscale = BONUS ? 1.f : 1.f / sqrtf(float(a.dim));
-    for (int d = tid; d < a.dim; d += NT) {
-      qs[d] = act_load(row + h * a.dim + d) * qscale;
-      ks[d] = act_load(row + a.off_k + h * a.dim + d);
-      if constexpr (BONUS) uk[d] = a.bonus[h * a.dim + d] * ks[d];
-    }
-  }
   const int v4n = a.vpad / 4;
   const int n_rows = NT / v4n;
   const int vr = tid / v4n, vc = tid % v4n;
   const bool live = vr < n_rows;
-  f32x4_t v = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  if (live) {
-    const T* vp = row + a.off_v + h * a.vdim;
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      if (vc * 4 + j < a.vdim) v[j] = act_load(vp + vc * 4 + j);
-  }
-  __syncthreads();
-  if constexpr (!FG) {
-    for (int d = tid; d < a.dim; d += NT) {
-      const T* w = reinterpret_cast<const T*>(a.a2) +
-                   int64_t(h * a.dim + d) * a.rank;
-      float z = a.a2_bias[h * a.dim + d];
-      for (int r = 0; r < a.rank; ++r) z += act_load(w + r) * a1[r];
-      al[d] = BONUS ? expf(log_rwkv<T>(z))
-                    : expf(log_sigmoid<T>(z) / a.tau);
-    }
-    __syncthreads();
-  }
-
   const bool fresh = a.positions[seq] == 0;
-  float* S = a.state +
-             (int64_t(a.slots[seq]) * a.heads + h) * a.dim * a.vpad + vc * 4;
+  float* S =
+      a.state + (int64_t(a.slots[seq]) * a.heads + h) * a.dim * a.vpad;
+  const auto at = [&](int d) {            // (1 MB at most)
+    return reinterpret_cast<f32x4_t*>(S) + unsigned(d * v4n + vc);
+  };
+  const T* low = reinterpret_cast<const T*>(a.a1) + int64_t(seq) * a.a1_stride;
+  const float qscale = BONUS ? 1.f : 1.f / sqrtf(float(a.dim));
+  // 2^lg lanes a channel, as many as there are threads for, that take four
+  // neighbouring elements of the rank at a time
+  int lg = 0;
+  if constexpr (!FG)
+    while (lg < 4 && (a.dim << (lg + 1)) <= NT) ++lg;
+  const int part = tid & ((1 << lg) - 1);
+  struct Item {
+    float q, k, b, x;
+    f32x4_t w, l;
+  };
+  const auto load = [&](int i) {
+    const int d = i >> lg, hc = h * a.dim + d;
+    Item t;
+    t.q = act_load(row + hc);
+    t.k = act_load(row + a.off_k + hc);
+    t.b = a.a2_bias[hc];
+    if constexpr (FG) t.x = a.lower[hc];
+    if constexpr (BONUS) t.x = a.bonus[hc];
+    if constexpr (!FG) {
+      if (vec_a2) {
+        const int r = min(part * 4, a.rank - 4);
+        t.w = act_load4(reinterpret_cast<const T*>(a.a2) +
+                        int64_t(hc) * a.rank + r);
+        t.l = act_load4(low + r);
+      }
+    }
+    return t;
+  };
+  const auto finish = [&](int i, const Item& t) {
+    const int d = i >> lg, hc = h * a.dim + d;
+    if constexpr (FG) {
+      float alpha;
+      const float key = forget_key<T>(t.k + t.b, t.x, &alpha);
+      chan[d] = f32x4_t{alpha, key, silu<T>(t.q), 0.f};
+    } else {
+      const T* w = reinterpret_cast<const T*>(a.a2) + int64_t(hc) * a.rank;
+      const auto times = [](f32x4_t w4, f32x4_t l4) {
+        float z = 0.f;
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          z += w4[j] * (BONUS ? gtanh<T>(l4[j]) : l4[j]);
+        return z;
+      };
+      float z = 0.f;
+      int r = part * 4;
+      if (vec_a2) {
+        if (r < a.rank) z = times(t.w, t.l);
+        for (r += 4 << lg; r < a.rank; r += 4 << lg)
+          z += times(act_load4(w + r), act_load4(low + r));
+      } else {
+        for (; r < a.rank; r += 4 << lg)
+          for (int j = r; j < min(r + 4, a.rank); ++j)
+            z += act_load(w + j) *
+                 (BONUS ? gtanh<T>(act_load(low + j)) : act_load(low + j));
+      }
+      if (lg > 0) z += dpp_mov_f32<0xB1>(z);
+      if (lg > 1) z += dpp_mov_f32<0x4E>(z);
+      if (lg > 2) z += dpp_mov_f32<0x141>(z);
+      if (lg > 3) z += dpp_mov_f32<0x140>(z);
+      if (part == 0) {
+        z += t.b;
+        chan[d] = f32x4_t{
+            BONUS ? expf(log_rwkv<T>(z)) : expf(log_sigmoid<T>(z) / a.tau),
+            t.k, t.q * qscale, BONUS ? t.x * t.k : 0.f};
+      }
+    }
+  };
+  const Item first = load(min(tid, (a.dim << lg) - 1));
+  f32x4_t v;
+  const T* vp = row + a.off_v + h * a.vdim;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) v[j] = act_load(vp + min(vc * 4 + j, a.vdim - 1));
+  // the norm and the gate of the first columns
+  const int e0 = min(tid, a.vdim - 1);
+  float nw = a.norm[h * a.norm_stride + e0], gate = 0.f;
+  if constexpr (!FG) gate = act_load(row + a.off_g + h * a.vdim + e0);
+  f32x4_t s[U];
+  // (without a condition, so that none of the waits above is for these)
+  const auto ask = [&](int d0) {
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      s[u] = *at(min(d0 + u * n_rows, a.dim - 1));
+  };
+  ask(vr);
+  if (tid < a.dim << lg) finish(tid, first);
+  for (int i = tid + NT; i < a.dim << lg; i += NT) finish(i, load(i));
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    if (vc * 4 + j >= a.vdim) v[j] = 0.f;
+  __syncthreads();
   f32x4_t o = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  // ALL: none of the rows is behind the last one
+  const auto step = [&](int d0, auto all) {
+    constexpr bool ALL = decltype(all)::value;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const bool mine = ALL || d0 + u * n_rows < a.dim;
+      const int d = ALL ? d0 + u * n_rows : min(d0 + u * n_rows, a.dim - 1);
+      const f32x4_t c = chan[d];
+      if (fresh) s[u] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float before = s[u][j];
+        s[u][j] = c[0] * before + c[1] * v[j];
+        if (mine) o[j] += c[2] * (BONUS ? before + c[3] * v[j] : s[u][j]);
+      }
+      if (mine) *at(d) = s[u];
+    }
+  };
   if (live) {
-    constexpr int U = 8;
-    for (int d0 = vr; d0 < a.dim; d0 += U * n_rows) {
-      f32x4_t s[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int d = d0 + u * n_rows;
-        s[u] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-        if (d < a.dim && !fresh)
-          s[u] = *reinterpret_cast<const f32x4_t*>(S + int64_t(d) * a.vpad);
-      }
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int d = d0 + u * n_rows;
-        if (d >= a.dim) break;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          if constexpr (BONUS) o[j] += qs[d] * (s[u][j] + uk[d] * v[j]);
-          s[u][j] = al[d] * s[u][j] + ks[d] * v[j];
-          if constexpr (!BONUS) o[j] += qs[d] * s[u][j];
-        }
-        *reinterpret_cast<f32x4_t*>(S + int64_t(d) * a.vpad) = s[u];
-      }
+    for (int d0 = vr; d0 < a.dim;) {
+      if (d0 - vr + U * n_rows <= a.dim) step(d0, std::true_type{});
+      else step(d0, std::false_type{});
+      d0 += U * n_rows;
+      if (d0 < a.dim) ask(d0);
     }
     *reinterpret_cast<f32x4_t*>(red + vr * a.vpad + vc * 4) = o;
   }
@@ -171,9 +231,12 @@ void gla_decode_kernel(GlaArgs a) {
   T* out = reinterpret_cast<T*>(a.out) + int64_t(seq) * a.out_stride +
            h * a.vdim;
   for (int e = tid; e < a.vdim; e += NT) {
-    float o2 = red[e] * inv * a.norm[h * a.norm_stride + e];
-    if constexpr (!FG)
-      o2 *= silu<T>(act_load(row + a.off_g + h * a.vdim + e));
+    if (e != tid) {
+      nw = a.norm[h * a.norm_stride + e];
+      if constexpr (!FG) gate = act_load(row + a.off_g + h * a.vdim + e);
+    }
+    float o2 = red[e] * inv * nw;
+    if constexpr (!FG) o2 *= silu<T>(gate);
     act_store(out + e, o2);
   }
 }
@@ -550,28 +613,39 @@ void by_kind(const GlaArgs& a, F f) {
 
 void launch_gla_decode(const GlaArgs& a, hipStream_t st) {
   if (a.rows == 0) return;
-  // 1024 threads for states of 128 KB and more where each can have a CU of its
-  // own (us with 256 threads and with 1024, heads of 128 x 256: 8 of them 8.6
-  // and 6.8, 128 of them 10.7 and 9.0, 512 of them 24.1 and 26.5; of 128 x
-  // 128: 6.2 and 5.8, 7.2 and 6.9, 12.0 and 15.9; 256 of these 8.4 and 8.4).
-  // The readout sums rows in another order with them, so that its last bits
-  // depend on the batch.
-  const bool wide = int64_t(a.dim) * a.vpad >= 128 * 256 &&
+  // 512 threads for states of 64 KB and more where each can have a CU of its
+  // own (us with 256, 512 and 1024 threads, states in HBM; heads of 128 x 256:
+  // 8 of them 8.3, 6.8 and 7.0, 128 of them 13.6, 11.7 and 11.6, 512 of them
+  // 31.3, 30.5 and 33.1; of 128 x 128: 5.9, 5.3 and 6.9, 8.8, 7.9 and 9.3, 19.5,
+  // 19.4 and 23.0; of 64 x 128: 128 of them 5.7, 6.5 and 8.0).  The readout sums
+  // rows in another order with them, so that its last bits depend on the batch.
+  const bool wide = int64_t(a.dim) * a.vpad >= 128 * 128 &&
                     int64_t(a.rows) * a.heads <= 256;
-  const int n_rows = (wide ? 1024 : 256) / (a.vpad / 4);
+  const int n_rows = (wide ? 512 : 256) / (a.vpad / 4);
   const size_t smem =
-      size_t((a.kind == kRwkv ? 4 : 3) * a.dpad + (a.rank + 3) / 4 * 4 +
-             n_rows * a.vpad) * sizeof(float);
+      size_t(4 * a.dpad + n_rows * a.vpad) * sizeof(float);
   by_kind(a, [&](auto t, auto kind) {
     using T = decltype(t);
     constexpr int KIND = decltype(kind)::value;
+    // four elements of the rank at a time where all rows of both factors lie
+    // for it, otherwise one
+    const size_t four = 4 * sizeof(T);
+    const bool vec = a.rank >= 4 && a.rank % 4 == 0 && a.a1_stride % 4 == 0 &&
+                     reinterpret_cast<uintptr_t>(a.a1) % four == 0 &&
+                     reinterpret_cast<uintptr_t>(a.a2) % four == 0;
     const dim3 grid(a.rows, a.heads);
-    if (wide)
-      hipLaunchKernelGGL((gla_decode_kernel<T, KIND, 1024>), grid, dim3(1024),
-                         smem, st, a);
-    else
-      hipLaunchKernelGGL((gla_decode_kernel<T, KIND, 256>), grid, dim3(256),
-                         smem, st, a);
+    const auto run = [&](auto nt, auto u) {
+      constexpr int NT = decltype(nt)::value, U = decltype(u)::value;
+      hipLaunchKernelGGL((gla_decode_kernel<T, KIND, NT, U>), grid, dim3(NT),
+                         smem, st, a, vec);
+    };
+    using std::integral_constant;
+    // four rows a thread where that is all of them, so that none is asked for
+    // twice (1536 heads of 64 x 64: 18.3 us with eight, 15.6 with four)
+    if (wide) run(integral_constant<int, 512>{}, integral_constant<int, 8>{});
+    else if (a.dim <= 4 * n_rows)
+      run(integral_constant<int, 256>{}, integral_constant<int, 4>{});
+    else run(integral_constant<int, 256>{}, integral_constant<int, 8>{});
   });
 }
 

@@ -1,4 +1,4 @@
-"""Steps of gated linear attention, HGRN2 and RWKV by workgroups of 1024 and of
+"""Steps of gated linear attention, HGRN2 and RWKV by workgroups of 512 and of
 256 threads: states around the line between them, columns that do not divide
 the threads."""
 
@@ -64,3 +64,34 @@ def test_rwkv_steps(dim, dtype):
     # the bounds of the longer runs
     assert rel(got, want) < (1e-5 if dtype == F32 else 8e-3)
     assert rel(a.state[1, :, :, :a.dim].cpu(), S) < 2e-5
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [F32, BF16])
+@pytest.mark.parametrize("dim,vdim,rank", [
+    # 512 threads from 128 x 128 on
+    (128, 128, 16), (127, 128, 16), (256, 64, 4), (255, 64, 8),
+    # 256 threads with four rows each, where that is all rows, or eight
+    (64, 64, 16), (65, 64, 16), (16, 256, 68), (17, 256, 12), (1, 4, 4),
+    # one to sixteen lanes a channel; ranks that fours do not divide and rows
+    # that do not lie for them
+    (8, 30, 64), (16, 33, 64), (33, 20, 20), (120, 40, 3), (7, 12, 70),
+    (32, 7, 1), (200, 24, 130)])
+def test_lanes_and_rows(dim, vdim, rank, dtype):
+    T, H = 5, 3
+    *inputs, eps, want, S = gla_case(T, H, dim, vdim, rank, 8.0, 1.0,
+                                     dim + rank, dtype)
+    proj, a2, b, norm = (t.cuda() for t in inputs)
+    # rows of three sequences, whose other slots hold NaN
+    st = torch.full((5, H, dim, -(-vdim // 4) * 4), float("nan"),
+                    device="cuda")
+    slots = torch.tensor([4, 0, 2], dtype=torch.int32, device="cuda")
+    got = torch.stack([
+        ops.gla_decode(proj[p:p + 1].repeat(3, 1), a2, b, norm, st, slots,
+                       torch.full((3,), p, dtype=torch.int32, device="cuda"),
+                       vdim, 8.0, eps) for p in range(T)])
+    # the bounds of the longer runs over the same steps
+    for i, slot in enumerate((4, 0, 2)):
+        assert rel(got[:, i], want) < tol(dtype)
+        assert rel(st[slot, :, :, :vdim], S) < 1e-5
+    assert torch.isnan(st[[1, 3]]).all()

@@ -454,6 +454,8 @@ void gla_intra_kernel(GlaArgs a, bool vec, bool vec_a) {
   const int64_t ch = int64_t(tile) * a.heads + h;
   float* qd = a.qd + ch * C * DP;
   float* kd = a.kd + ch * DP * C;
+  // the lane whose operand this lane has once it is transposed
+  const int turned = (lr >> 2) * 16 + g * 4 + (lr & 3);
   f32x4_t diag = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int dt = 0; dt < NT; ++dt) {
@@ -463,7 +465,7 @@ void gla_intra_kernel(GlaArgs a, bool vec, bool vec_a) {
     f32x4_t eb = f32x4_t{1.f, 1.f, 1.f, 1.f}, ed = eb;
     if (w > 0) eb = *reinterpret_cast<const f32x4_t*>(EB + (w - 1) * DP + d);
     if (w < 3) ed = *reinterpret_cast<const f32x4_t*>(ED + w * DP + d);
-    f32x4_t kt = *reinterpret_cast<const f32x4_t*>(kl + trow * LR + d), qo;
+    f32x4_t kt = *reinterpret_cast<const f32x4_t*>(kl + trow * LR + d), qo, ko;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const float Lt = L[dt][j];
@@ -475,9 +477,11 @@ void gla_intra_kernel(GlaArgs a, bool vec, bool vec_a) {
       q[dt][j] *= gexp<T>(seen(Lt));
       qo[j] = q[dt][j] * eb[j];
       kt[j] *= gexp<T>(tw[j] - Lt);
-      kd[int64_t(d + j) * C + trow] = kt[j] * ed[j];
+      ko[j] = kt[j] * ed[j];
     }
-    *reinterpret_cast<f32x4_t*>(qd + trow * DP + d) = qo;
+    *reinterpret_cast<f32x4_t*>(qd + ((dt * 4 + w) * 64 + lane) * 4) = qo;
+    *reinterpret_cast<f32x4_t*>(kd + ((dt * 4 + w) * 64 + turned) * 4) =
+        quad_transposed(ko);
     *reinterpret_cast<f32x4_t*>(kl + trow * LR + d) = kt;
   }
   if (safe) {
@@ -518,12 +522,10 @@ void gla_intra_kernel(GlaArgs a, bool vec, bool vec_a) {
   for (int J = 0; J < 4; ++J) {
     if (J > w) break;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int t = g * 4 + r;
-      float v = acc[J][r];
-      if (J == w && lr > t) v = 0.f;
-      sc[(w * 16 + t) * C + J * 16 + lr] = v;
-    }
+    for (int r = 0; r < 4; ++r)
+      if (J == w && lr > g * 4 + r) acc[J][r] = 0.f;
+    *reinterpret_cast<f32x4_t*>(sc + ((w * 4 + J) * 64 + turned) * 4) =
+        quad_transposed(acc[J]);
   }
 }
 

@@ -26,10 +26,11 @@ enum ScanMode { kScanPlain = 0, kScanMax = 1, kScanDelta = 2 };
 struct ScanArgs {
   const void* v;           // value rows (plain, max), head h at h * vdim
   const void* q;           // query rows (max, delta), head h / group
-  const float* qd;         // [n_tiles, heads, 64, dpad] (plain)
+  const float* qd;         // [n_tiles, heads, 64, dpad] in tiles (plain)
   const void* kt;          // [n_tiles, heads / group, dpad, 64] keys down
-                           // the columns: f32 decayed (plain), or as they are
-  const float* sc;         // [n_tiles, heads, 64, 64] A
+                           // the columns: f32 decayed, in tiles (plain), or as
+                           // they are
+  const float* sc;         // [n_tiles, heads, 64, 64] A, in tiles (plain)
   const float* dec;        // [n_tiles, heads, dpad] (plain), [n_tiles, heads]
   const float* rows;       // [n_tiles, heads, 3, 64]: running log-decay F,
                            // a = i - F, running maximum of a (max); query
@@ -88,9 +89,11 @@ struct GlaArgs {
   const int32_t* positions;     // [rows] (decode)
   const int32_t* tiles;    // [4, n_tiles] chunks of kRecChunk rows
   const int32_t* seqs;     // [4, n_seqs]: first tile, tiles, pos0, slot
-  float* qd;               // [n_tiles, heads, 64, dpad] scratch
-  float* kd;               // [n_tiles, heads, dpad, 64]
-  float* sc;               // [n_tiles, heads, 64, 64]
+  // scratch in tiles of 16 x 16, a lane l's four elements of row l % 16 from
+  // column l / 16 * 4 on next to each other, tiles of
+  float* qd;               // [n_tiles, heads, 64, dpad] down the columns,
+  float* kd;               // [n_tiles, heads, dpad, 64] and
+  float* sc;               // [n_tiles, heads, 64, 64] along the rows
   float* dec;              // [n_tiles, heads, dpad]
   float* o;                // [rows + 64, heads * vdim]
   void* out;               // [rows, heads * vdim], rows out_stride apart

@@ -82,6 +82,25 @@ DEV_INLINE float wave_prefix_max(float v) {
   return v;
 }
 
+// 4 x 4 transposed within four neighbouring lanes: lane b gets element b of
+// each
+DEV_INLINE f32x4_t quad_transposed(f32x4_t v) {
+  const bool b0 = threadIdx.x & 1, b1 = threadIdx.x & 2;
+#pragma unroll
+  for (int i = 0; i < 4; i += 2) {
+    const float t = dpp_mov_f32<0xB1>(b0 ? v[i] : v[i + 1]);
+    v[i] = b0 ? t : v[i];
+    v[i + 1] = b0 ? v[i + 1] : t;
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const float t = dpp_mov_f32<0x4E>(b1 ? v[i] : v[i + 2]);
+    v[i] = b1 ? t : v[i];
+    v[i + 2] = b1 ? v[i + 2] : t;
+  }
+  return v;
+}
+
 DEV_INLINE f32x4_t mma4(float a, float b, f32x4_t c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }

@@ -11,6 +11,14 @@
 // goes to spare rows), since a branch around one makes later waits drain
 // everything in flight.
 //
+// kScanPlain's operands come in the order in which lanes take them, 1 KB a load:
+// read as rows are, neighbouring lanes have rows of their own, and the cache
+// looks up each lane's 16 bytes by themselves, which was what bounded it (4
+// sequences of 1.9k, 8 heads of 128 x 256: 179 us, of which 145 such lookups,
+// and 133 now, of which 67 products and 40 lookups; without loads and stores
+// 97).  (With outputs and state in waves of their own, a barrier a chunk and its
+// next but one asked for ahead: 126.)
+//
 // kScanMax: with F the chunk's running log-decay, a = i - F and the maximum
 // M_t = max(m, max_{s <= t} a_s), m what the chunk started with,
 //     m_t = F_t + M_t,   O_t = e^{m - M_t} q_t S + sum_s q_t k_s e^{a_s - M_t} v_s
@@ -106,10 +114,10 @@ void rec_scan_kernel(ScanArgs a, bool vec_q, bool vec_v) {
           qr[i] = raw_guard(q, i * 16 + g * 4, a.dim, ok, vec_q);
       }
     } else {
-      const float* qd = a.qd + chunk(t) * C * DP + trow * DP + g * 4;
+      const float* qd = a.qd + chunk(t) * C * DP + (w * 64 + lane) * 4;
 #pragma unroll
       for (int i = 0; i < NQ; ++i)
-        if (i < ndt) qr[i].load(qd + i * 16);
+        if (i < ndt) qr[i].load(qd + i * 1024);
     }
     if constexpr (DELTA) {
       const float* wp = a.w + chunk(t) * C * DP + trow * DP + g * 4;
@@ -119,10 +127,12 @@ void rec_scan_kernel(ScanArgs a, bool vec_q, bool vec_v) {
     }
   };
   auto load_a = [&](int t) {
-    const float* sc = a.sc + chunk(t) * C * C + trow * C + g * 4;
+    const float* sc = a.sc + chunk(t) * C * C +
+                      (RAW ? trow * C + g * 4 : (w * 256 + lane) * 4);
 #pragma unroll
     for (int J = 0; J < 4; ++J)            // (blocks behind w: not used)
-      ar[J] = *reinterpret_cast<const f32x4_t*>(sc + min(J, w) * 16);
+      ar[J] = *reinterpret_cast<const f32x4_t*>(sc + min(J, w) *
+                                                         (RAW ? 16 : 256));
   };
   auto load_v = [&](int t) {
     const float* rf = a.rows + chunk(t) * 3 * C;
@@ -173,7 +183,9 @@ void rec_scan_kernel(ScanArgs a, bool vec_q, bool vec_v) {
       if (FULL || i * 4 + w < ndt)
 #pragma unroll
         for (int s = 0; s < 4; ++s)
-          kr[i][s].load(kt + ((i * 4 + w) * 16 + lr) * C + s * 16 + g * 4);
+          kr[i][s].load(
+              kt + (RAW ? ((i * 4 + w) * 16 + lr) * C + s * 16 + g * 4
+                        : (((i * 4 + w) * 4 + s) * 64 + lane) * 4));
   };
   load_v(first);
   load_rows(first);

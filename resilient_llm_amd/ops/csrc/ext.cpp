@@ -814,7 +814,7 @@ Tensor rows_linear_parts(const Tensor& x, const Tensor& w) {
 Tensor rows_short(const Tensor& x, const Tensor& w, bool relu2) {
   check_rows(x, w);
   const int M = int(x.size(0)), N = int(w.size(0)), K = int(x.size(1));
-  if (M > 64 || rlli::rows_short_tiles(N, K) == 0) return Tensor();
+  if (M > 64 || !rlli::rows_short_ok(N, K)) return Tensor();
   c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
   Tensor out = at::empty({M, N}, x.options());
   rlli::launch_rows_short(bf16_ptr(x), bf16_ptr(w), bf16_ptr(out), M, N, K,
@@ -845,7 +845,7 @@ Tensor rows_linear_relu2(const Tensor& x, const Tensor& w) {
 
 bool rows_whole_ok(int64_t M, int64_t N, int64_t K) {
   return M <= 64 && N <= 8192 && K <= 8192 &&
-         rlli::rows_short_tiles(int(N), int(K)) > 0;
+         rlli::rows_short_ok(int(N), int(K));
 }
 
 Tensor rows_linear_silu(const Tensor& x, const Tensor& w) {

@@ -206,8 +206,8 @@ bool rows_scaled_ok(int M, int N, int K);
 void launch_rows_scaled_relu2(const uint16_t* x, const uint16_t* w,
                               uint16_t* out, int M, int N, int K,
                               const RowsScale& scale, hipStream_t stream);
-// M <= 64 where rows_short_tiles is not 0; ``relu2``: squared positive part
-int rows_short_tiles(int N, int K);
+// M <= 64 where rows_short_ok; ``relu2``: squared positive part
+bool rows_short_ok(int N, int K);
 void launch_rows_short(const uint16_t* x, const uint16_t* w, uint16_t* out,
                        int M, int N, int K, bool relu2, hipStream_t stream);
 void launch_sum_parts(const float* parts, uint16_t* out, int splits,

@@ -494,39 +494,40 @@ void rows_gemm_kernel(const uint16_t* __restrict__ x,
 }
 
 // The same product by workgroups that divide K among their four waves, for
-// shapes whose 64-row panels leave CUs idle: 16 PT rows of w per workgroup, no
+// shapes whose 64-row panels leave CUs idle: 8 HR rows of w per workgroup, no
 // parts in memory and no launch to sum them.  A wave has a ring of its own for
 // the steps it takes (every fourth, so that the four together read 512 bytes of
 // a row at a time): its loads, waits and reads concern nobody else, and there
 // is no barrier before the sums meet at the end.  What bounds it is the time
 // from the launch to the first data and, past 4096 in K, that it reads x once
-// per 16 or 32 rows of w.
-// END: the result, its squared positive part, or (ADDS; PT 1) S streams with it.
+// per 8 to 32 rows of w.
+// END: the result, its squared positive part, or (ADDS; HR 2) S streams with it.
 enum End { WHOLE, RELU2, ADDS };
 
-template <int PT, int XR, int MT, int R, End END, int S = 0,
+template <int HR, int XR, int MT, int R, End END, int S = 0,
           bool SCALED = false>
 __global__ __launch_bounds__(256)
 void rows_short_kernel(const uint16_t* __restrict__ x,
                        const uint16_t* __restrict__ w,
                        uint16_t* __restrict__ out, int M, int N, int K,
                        RowsScale scale, RowsAdds adds) {
-  constexpr int WPART = PT * 16 * LINE;              // elements of a step
+  constexpr int PT = (HR + 1) / 2;                   // tiles of w
+  constexpr int WPART = HR * 8 * LINE;               // elements of a step
   constexpr int STEP = WPART + XR * LINE;
-  constexpr int LX = XR / 8, L = PT * 2 + LX;        // loads of a wave
+  constexpr int LX = XR / 8, L = HR + LX;            // loads of a wave
   extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
   const int lane = threadIdx.x & 63;
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int n0 = blockIdx.x * PT * 16;
+  const int n0 = blockIdx.x * HR * 8;
   // this wave's steps: wv, wv + 4, ...
   const int n = (K / KS - wv + 3) / 4;
   const int rot = n > 0 ? int(blockIdx.x / 8 % unsigned(n)) : 0;
   uint16_t* ring = lds + wv * R * STEP;
 
   const int lr = lane >> 3;
-  const uint16_t *wp[PT * 2], *xp[LX];
+  const uint16_t *wp[HR], *xp[LX];
 #pragma unroll
-  for (int j = 0; j < PT * 2; ++j) {
+  for (int j = 0; j < HR; ++j) {
     const int r = (j & 1) * 8 + lr;
     // rows past the end repeat the last one; nobody stores them
     const int row = min(n0 + (j >> 1) * 16 + r, N - 1);
@@ -543,7 +544,7 @@ void rows_short_kernel(const uint16_t* __restrict__ x,
     s += rot;
     if (s >= n) s -= n;
 #pragma unroll
-    for (int j = 0; j < PT * 2; ++j)
+    for (int j = 0; j < HR; ++j)
       lds_load16<2>(wp[j] + s * 4 * KS, at + j * 8 * LINE);
 #pragma unroll
     for (int j = 0; j < LX; ++j)
@@ -566,7 +567,7 @@ void rows_short_kernel(const uint16_t* __restrict__ x,
   float mix[S > 0 ? S : 1][S > 0 ? S : 1], outw[S > 0 ? S : 1],
       inw[S > 0 ? S : 1];
   if constexpr (END == ADDS) {
-    static_assert(PT == 1 && MT <= 4, "");
+    static_assert(HR == 2 && MT <= 4, "");
 #pragma unroll
     for (int s = 0; s < S; ++s) {
       had[s] = *reinterpret_cast<const f32x4*>(
@@ -664,7 +665,8 @@ void rows_short_kernel(const uint16_t* __restrict__ x,
       if (oct == 0) adds.ss[int64_t(blockIdx.x) * 16 * MT + row] = ss;
       v = u * gain;
     }
-    if (row < M && c < N)
+    // (an odd last tile has only eight rows of w)
+    if (row < M && c < min(N, n0 + HR * 8))
       *reinterpret_cast<uint2*>(out + int64_t(row) * N + c) =
           uint2{pack2(v[0], v[1]), pack2(v[2], v[3])};
   }
@@ -731,19 +733,19 @@ void go_norm(const RowsNorm& norm, const uint16_t* w, void* out, int N, int K,
                      RowsCombine{});
 }
 
-template <int PT, int R16, int R32, int R64, End END>
+template <int HR, int R16, int R32, int R64, End END>
 void go_short(const uint16_t* x, const uint16_t* w, uint16_t* out, int M,
               int N, int K, hipStream_t st) {
   auto run = [&](auto xr) {
     constexpr int XR = decltype(xr)::value, MT = XR / 16;
     constexpr int R = XR == 16 ? R16 : XR == 32 ? R32 : R64;
-    constexpr size_t smem = size_t(4) * R * (PT * 16 + XR) * LINE * 2;
-    auto* k = rows_short_kernel<PT, XR, MT, R, END>;
+    constexpr size_t smem = size_t(4) * R * (HR * 8 + XR) * LINE * 2;
+    auto* k = rows_short_kernel<HR, XR, MT, R, END>;
     if (smem > 65536)
       (void)hipFuncSetAttribute(reinterpret_cast<const void*>(k),
                                 hipFuncAttributeMaxDynamicSharedMemorySize,
                                 int(smem));
-    hipLaunchKernelGGL(k, dim3((N + PT * 16 - 1) / (PT * 16)), dim3(256), smem,
+    hipLaunchKernelGGL(k, dim3((N + HR * 8 - 1) / (HR * 8)), dim3(256), smem,
                        st, x, w, out, M, N, K, RowsScale{}, RowsAdds{});
   };
   if (M <= 16) run(std::integral_constant<int, 16>{});
@@ -752,20 +754,20 @@ void go_short(const uint16_t* x, const uint16_t* w, uint16_t* out, int M,
 }
 
 // with a norm that is shared, up to 32 rows
-template <int PT, int R16, int R32, End END, int S, bool SCALED>
+template <int HR, int R16, int R32, End END, int S, bool SCALED>
 void go_shared(const uint16_t* x, const uint16_t* w, uint16_t* out, int M,
                int N, int K, const RowsScale& scale, const RowsAdds& adds,
                hipStream_t st) {
   auto run = [&](auto xr) {
     constexpr int XR = decltype(xr)::value, MT = XR / 16;
     constexpr int R = XR == 16 ? R16 : R32;
-    constexpr size_t smem = size_t(4) * R * (PT * 16 + XR) * LINE * 2;
-    auto* k = rows_short_kernel<PT, XR, MT, R, END, S, SCALED>;
+    constexpr size_t smem = size_t(4) * R * (HR * 8 + XR) * LINE * 2;
+    auto* k = rows_short_kernel<HR, XR, MT, R, END, S, SCALED>;
     if (smem > 65536)
       (void)hipFuncSetAttribute(reinterpret_cast<const void*>(k),
                                 hipFuncAttributeMaxDynamicSharedMemorySize,
                                 int(smem));
-    hipLaunchKernelGGL(k, dim3((N + PT * 16 - 1) / (PT * 16)), dim3(256), smem,
+    hipLaunchKernelGGL(k, dim3((N + HR * 8 - 1) / (HR * 8)), dim3(256), smem,
                        st, x, w, out, M, N, K, scale, adds);
   };
   if (M <= 16) run(std::integral_constant<int, 16>{});
@@ -867,42 +869,55 @@ void launch_rows_norm_silu(const RowsNorm& norm, const uint16_t* w,
                              st);
 }
 
-// Tiles of 16 rows per workgroup of the products that rows_short_kernel takes,
-// 0 for others; by N and K alone, like all orders of sums here.  With 32 rows
-// per workgroup where 16 make more workgroups than CUs.  (1, 16, 64 rows of x,
-// us, parts and their sum first: 2048 x 2048 6.5 and 4.2, 7.7 and 5.0, 9.3 and
-// 7.1; 8192 x 2048 10.7 and 7.6, 11.5 and 7.8, 13.7 and 11.2; 6144 x 4096 13.6
-// and 10.3, 14.5 and 11.1, 18.3 and 17.0; 256 x 8192 18.7 and 7.8, 22.3 and
-// 10.1, 20.7 and 19.6; but 4096 x 4096 9.7 and 7.8, 10.3 and 8.9, 13.1 and
-// 13.4; 2048 x 8192 10.5 and 9.8, 11.6 and 12.4, 13.7 and 20.4; 5120 x 5120
-// 12.5 and 11.8, 13.4 and 15.9, 18.3 and 21.9.)
-int rows_short_tiles(int N, int K) {
-  if (N > 8192 || K > (N > 4096 ? 4096 : N > 512 ? 3072 : 8192)) return 0;
-  return N > 4096 ? 2 : 1;
+// Whether rows_short_kernel takes a product; by N and K alone, like all orders of
+// sums here.  (1, 16, 64 rows of x, us, parts and their sum first: 2048 x 2048 6.5
+// and 3.9, 7.7 and 4.4, 9.3 and 7.0; 8192 x 2048 10.7 and 7.0, 11.5 and 7.2, 13.7
+// and 10.2; 6144 x 4096 13.6 and 9.3, 14.5 and 9.7, 18.3 and 14.7; 256 x 8192 18.7
+// and 7.0, 22.3 and 8.5, 20.7 and 17.3; but 4096 x 4096 9.7 and 7.8, 10.3 and 8.9,
+// 13.1 and 13.4; 2048 x 8192 10.5 and 9.8, 11.6 and 12.4, 13.7 and 20.4; 5120 x
+// 5120 12.5 and 11.8, 13.4 and 15.9, 18.3 and 21.9.)
+bool rows_short_ok(int N, int K) {
+  return N <= 8192 && K <= (N > 4096 ? 4096 : N > 512 ? 3072 : 8192);
 }
+
+namespace {
+
+// Rows of w of one of its workgroups, in eights: as few as make no more workgroups
+// than CUs, whose rings leave no room for a second one.  The order of sums does
+// not depend on it.  (1, 16, 64 rows of x, us, 8, 16, 24 and 32 rows of w: 2048 x
+// 2048 3.9 4.1 4.3 4.7, 4.4 4.8 5.1 5.6, 7.0 7.1 7.9 8.4; 4096 x 2048 6.8 4.9 4.7
+// 5.1, 7.7 5.1 5.6 6.0, 12.6 7.7 8.5 8.9; 6144 x 2048 9.6 7.8 5.7 5.8, 11.0 8.6 6.0
+// 6.4, 18.2 13.2 9.0 9.5; 6160 x 2048 11.5 7.7 8.1 5.8, 13.1 8.6 8.5 6.4, 22.2 13.0
+// 13.7 9.5.)
+int short_eights(int N) { return std::clamp((N + 2047) / 2048, 1, 4); }
+
+}  // namespace
 
 void launch_rows_short(const uint16_t* x, const uint16_t* w, uint16_t* out,
                        int M, int N, int K, bool relu2, hipStream_t st) {
-  const bool one = rows_short_tiles(N, K) == 1;
-  if (relu2) {
-    if (one) go_short<1, 9, 6, 3, RELU2>(x, w, out, M, N, K, st);
-    else go_short<2, 6, 4, 3, RELU2>(x, w, out, M, N, K, st);
-  } else {
-    if (one) go_short<1, 9, 6, 3, WHOLE>(x, w, out, M, N, K, st);
-    else go_short<2, 6, 4, 3, WHOLE>(x, w, out, M, N, K, st);
-  }
+  auto run = [&](auto end) {
+    constexpr End END = decltype(end)::value;
+    switch (short_eights(N)) {
+      case 1: return go_short<1, 12, 7, 4, END>(x, w, out, M, N, K, st);
+      case 2: return go_short<2, 9, 6, 3, END>(x, w, out, M, N, K, st);
+      case 3: return go_short<3, 7, 5, 3, END>(x, w, out, M, N, K, st);
+      default: return go_short<4, 6, 4, 3, END>(x, w, out, M, N, K, st);
+    }
+  };
+  if (relu2) run(std::integral_constant<End, RELU2>{});
+  else run(std::integral_constant<End, WHOLE>{});
 }
 
 bool rows_adds_ok(int M, int N, int K, int streams) {
   return M >= 1 && M <= 32 && N % 16 == 0 && N <= 4096 && K % 64 == 0 &&
-         rows_short_tiles(N, K) == 1 && streams >= 1 && streams <= 4;
+         rows_short_ok(N, K) && streams >= 1 && streams <= 4;
 }
 
 void launch_rows_adds(const uint16_t* x, const uint16_t* w, uint16_t* out,
                       int M, int N, int K, int streams, const RowsAdds& adds,
                       hipStream_t st) {
   auto run = [&](auto s) {
-    go_shared<1, 9, 6, ADDS, decltype(s)::value, false>(
+    go_shared<2, 9, 6, ADDS, decltype(s)::value, false>(
         x, w, out, M, N, K, RowsScale{}, adds, st);
   };
   switch (streams) {
@@ -915,18 +930,24 @@ void launch_rows_adds(const uint16_t* x, const uint16_t* w, uint16_t* out,
 
 bool rows_scaled_ok(int M, int N, int K) {
   return M >= 1 && M <= 32 && N % 4 == 0 && K % 64 == 0 &&
-         rows_short_tiles(N, K) > 0;
+         rows_short_ok(N, K);
 }
 
 void launch_rows_scaled_relu2(const uint16_t* x, const uint16_t* w,
                               uint16_t* out, int M, int N, int K,
                               const RowsScale& scale, hipStream_t st) {
-  if (rows_short_tiles(N, K) == 1)
-    go_shared<1, 9, 6, RELU2, 0, true>(x, w, out, M, N, K, scale, RowsAdds{},
-                                       st);
-  else
-    go_shared<2, 6, 4, RELU2, 0, true>(x, w, out, M, N, K, scale, RowsAdds{},
-                                       st);
+  switch (short_eights(N)) {
+    case 1:
+    case 2:
+      return go_shared<2, 9, 6, RELU2, 0, true>(x, w, out, M, N, K, scale,
+                                                RowsAdds{}, st);
+    case 3:
+      return go_shared<3, 7, 5, RELU2, 0, true>(x, w, out, M, N, K, scale,
+                                                RowsAdds{}, st);
+    default:
+      return go_shared<4, 6, 4, RELU2, 0, true>(x, w, out, M, N, K, scale,
+                                                RowsAdds{}, st);
+  }
 }
 
 void launch_sum_parts(const float* parts, uint16_t* out, int splits,

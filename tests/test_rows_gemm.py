@@ -28,7 +28,7 @@ def close(got, want, size, rtol=2 ** -8):
 @pytest.mark.parametrize("N,K", [
     (4, 64), (60, 64), (64, 128), (68, 192), (6160, 320), (8196, 448),
     (16448, 64), (25540, 192), (25664, 704), (1536, 4096),
-    # panels of 16 and of 32 rows with K divided among a workgroup's waves:
+    # panels of 8 to 32 rows with K divided among a workgroup's waves:
     # fewer steps than waves, some waves one step more, around the lines
     # between the kernels
     (4096, 192), (4100, 320), (8188, 704), (4092, 3072), (2048, 3136),
@@ -53,6 +53,19 @@ def test_rows_linear(N, K):
         for p in parts[1:]:
             s += p
         assert torch.equal(s.to(torch.bfloat16), whole)
+
+
+@pytest.mark.parametrize("N", [
+    # a workgroup's 8, 16, 24 or 32 rows of w: the lines between them, a last one
+    # with few rows, a half tile that is not there
+    4, 2044, 2048, 2052, 4092, 4096, 4104, 6120, 6132, 6144, 6148, 8184])
+def test_rows_of_a_workgroup(N):
+    x, w = operands(N, 576, N)
+    want = x[:64].double() @ w.double().T
+    few = ops.rows_linear(x[:64].contiguous(), w)
+    close(few, want, 24)
+    for m in (1, 16, 17, 32, 33):
+        assert torch.equal(ops.rows_linear(x[:m].contiguous(), w), few[:m])
 
 
 @pytest.mark.parametrize("inter,K", [(8, 64), (72, 128), (5152, 64),

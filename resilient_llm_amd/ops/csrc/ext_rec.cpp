@@ -145,14 +145,18 @@ void prefill(rlli::GlaArgs& a, const Tensor& proj, const Tensor& tiles,
   const int64_t C = rlli::kRecChunk;
   const int64_t nh = int64_t(a.n_tiles) * a.heads;
   auto fo = proj.options().dtype(at::kFloat);
-  Tensor qd = at::empty({nh, C, a.dpad}, fo);
-  Tensor kd = at::empty({nh, a.dpad, C}, fo);
-  Tensor sc = at::empty({nh, C, C}, fo);
+  // f32, or three 16-bit parts, of which columns of queries go in 32
+  const int64_t size = a.f32 ? 4 : 6;
+  const int64_t q_cols = a.f32 ? a.dpad : (a.dpad + 31) / 32 * 32;
+  auto bytes = proj.options().dtype(at::kByte);
+  Tensor qd = at::empty({nh * C * q_cols * size}, bytes);
+  Tensor kd = at::empty({nh * C * a.dpad * size}, bytes);
+  Tensor sc = at::empty({nh * C * C * size}, bytes);
   Tensor dec = at::empty({nh, a.dpad}, fo);
   Tensor o = at::empty({a.rows + C, int64_t(a.heads) * a.vdim}, fo);
-  a.qd = qd.data_ptr<float>();
-  a.kd = kd.data_ptr<float>();
-  a.sc = sc.data_ptr<float>();
+  a.qd = qd.data_ptr();
+  a.kd = kd.data_ptr();
+  a.sc = sc.data_ptr();
   a.dec = dec.data_ptr<float>();
   a.o = o.data_ptr<float>();
   c10::hip::HIPGuardMasqueradingAsCUDA guard(proj.device());

@@ -11,8 +11,8 @@
 //           present through a bonus u per channel
 //
 // Projections arrive as GEMM output rows; everything from z on is
-// 32-bit, matrix products included (the f32 MFMA forms), and so are the
-// states.
+// 32-bit, matrix products included (f32 MFMA, or three 16-bit parts of each
+// number in the scan), and so are the states.
 //
 // Decode is one fused kernel per layer: decay, state update, readout,
 // norm and gate; a state is read and written exactly once.
@@ -254,7 +254,7 @@ DEV_INLINE float seen_log(float L) {
 // columns of every 16; MD bounds the key tiles (dpad <= 64 * MD).  FULL: dim
 // is 64 MD, the rank a multiple of 16 and rows are aligned, so that no load
 // is conditional (rows behind the last one are loaded from it).
-template <typename T, int KIND, int MD, bool FULL>
+template <typename T, int KIND, int MD, bool FULL, bool PARTS>
 __global__ __launch_bounds__(256)
 void gla_intra_kernel(GlaArgs a, bool vec, bool vec_a) {
   constexpr bool FG = KIND == kHgrn2, BONUS = KIND == kRwkv;
@@ -452,8 +452,18 @@ void gla_intra_kernel(GlaArgs a, bool vec, bool vec_a) {
 
   // this wave's own rows: q e^{L}, k e^{tot - L} and the diagonal block
   const int64_t ch = int64_t(tile) * a.heads + h;
-  float* qd = a.qd + ch * C * DP;
-  float* kd = a.kd + ch * DP * C;
+  const int nks = (ndt + 1) / 2;
+  float* qd = static_cast<float*>(a.qd) + ch * C * DP;
+  float* kd = static_cast<float*>(a.kd) + ch * DP * C;
+  uint16_t* qp = static_cast<uint16_t*>(a.qd) + ch * nks * 6144;
+  uint16_t* kp = static_cast<uint16_t*>(a.kd) + ch * ndt * 3072;
+  uint2 qh[2][3];
+  auto put_q = [&](int ks) {
+#pragma unroll
+    for (int p = 0; p < 3; ++p)
+      *reinterpret_cast<uint4*>(qp + (((ks * 4 + w) * 3 + p) * 64 + lane) * 8) =
+          uint4{qh[0][p].x, qh[0][p].y, qh[1][p].x, qh[1][p].y};
+  };
   // the lane whose operand this lane has once it is transposed
   const int turned = (lr >> 2) * 16 + g * 4 + (lr & 3);
   f32x4_t diag = f32x4_t{0.f, 0.f, 0.f, 0.f};
@@ -479,10 +489,27 @@ void gla_intra_kernel(GlaArgs a, bool vec, bool vec_a) {
       kt[j] *= gexp<T>(tw[j] - Lt);
       ko[j] = kt[j] * ed[j];
     }
-    *reinterpret_cast<f32x4_t*>(qd + ((dt * 4 + w) * 64 + lane) * 4) = qo;
-    *reinterpret_cast<f32x4_t*>(kd + ((dt * 4 + w) * 64 + turned) * 4) =
-        quad_transposed(ko);
+    ko = quad_transposed(ko);
+    if constexpr (PARTS) {
+      three_parts(qo, qh[dt & 1]);
+      if (dt & 1) put_q(dt / 2);
+      uint2 kh[3];
+      three_parts(ko, kh);
+#pragma unroll
+      for (int p = 0; p < 3; ++p)
+        *reinterpret_cast<uint2*>(
+            kp + (((dt * 2 + w / 2) * 3 + p) * 64 + turned) * 8 + w % 2 * 4) =
+            kh[p];
+    } else {
+      *reinterpret_cast<f32x4_t*>(qd + ((dt * 4 + w) * 64 + lane) * 4) = qo;
+      *reinterpret_cast<f32x4_t*>(kd + ((dt * 4 + w) * 64 + turned) * 4) = ko;
+    }
     *reinterpret_cast<f32x4_t*>(kl + trow * LR + d) = kt;
+  }
+  if (PARTS && !FULL && ndt % 2) {
+#pragma unroll
+    for (int p = 0; p < 3; ++p) qh[1][p] = uint2{0, 0};
+    put_q(ndt / 2);
   }
   if (safe) {
     if constexpr (BONUS)
@@ -517,15 +544,26 @@ void gla_intra_kernel(GlaArgs a, bool vec, bool vec_a) {
       for (int j = 0; j < 4; ++j) acc[J] = mma4(qe[j], kt[j], acc[J]);
     }
   }
-  float* sc = a.sc + ch * C * C;
+  float* sc = static_cast<float*>(a.sc) + ch * C * C;
+  uint16_t* sp = static_cast<uint16_t*>(a.sc) + ch * 12288;
 #pragma unroll
   for (int J = 0; J < 4; ++J) {
-    if (J > w) break;
+    if (J > (PARTS ? w | 1 : w)) break;    // (a pair's second tile: zeros)
 #pragma unroll
     for (int r = 0; r < 4; ++r)
-      if (J == w && lr > g * 4 + r) acc[J][r] = 0.f;
-    *reinterpret_cast<f32x4_t*>(sc + ((w * 4 + J) * 64 + turned) * 4) =
-        quad_transposed(acc[J]);
+      if (J > w || (J == w && lr > g * 4 + r)) acc[J][r] = 0.f;
+    const f32x4_t v = quad_transposed(acc[J]);
+    if constexpr (PARTS) {
+      uint2 h[3];
+      three_parts(v, h);
+#pragma unroll
+      for (int p = 0; p < 3; ++p)
+        *reinterpret_cast<uint2*>(
+            sp + (((w * 2 + J / 2) * 3 + p) * 64 + turned) * 8 + J % 2 * 4) =
+            h[p];
+    } else {
+      *reinterpret_cast<f32x4_t*>(sc + ((w * 4 + J) * 64 + turned) * 4) = v;
+    }
   }
 }
 
@@ -545,20 +583,42 @@ void prefill(const GlaArgs& a, hipStream_t st) {
     hipLaunchKernelGGL(k, dim3(a.n_tiles, a.heads), dim3(256), smem, st, a,
                        vec, vec_a);
   };
+  // The scan's operands in parts where the activations are 16-bit ones; they are
+  // half as many bytes more, which cost more than they gain where many short heads
+  // fill the chip (heads of 64 x 64, whole prompts, us, f32 and parts: 32 of them
+  // 103 and 76, 128 245 and 242, 256 269 and 230, but 512 214 and 234).
+  const int64_t sh = int64_t(a.n_seqs) * a.heads;
+  const bool parts = sizeof(T) == 2 &&
+                     (a.dpad > 64 || sh * ((a.vdim + 63) / 64) < 512);
+  auto by_parts = [&](auto md, auto full) {
+    constexpr int MD = decltype(md)::value;
+    constexpr bool FULL = decltype(full)::value;
+    if constexpr (sizeof(T) == 4)
+      intra(gla_intra_kernel<T, KIND, MD, FULL, false>);
+    else if constexpr (MD > 1)
+      intra(gla_intra_kernel<T, KIND, MD, FULL, true>);
+    else if (parts)
+      intra(gla_intra_kernel<T, KIND, MD, FULL, true>);
+    else
+      intra(gla_intra_kernel<T, KIND, MD, FULL, false>);
+  };
+  using I1 = std::integral_constant<int, 1>;
+  using I2 = std::integral_constant<int, 2>;
+  using I4 = std::integral_constant<int, 4>;
   bool done = false;                      // (gains nothing for the others)
   if constexpr (sizeof(T) == 2 && KIND == kRwkv) {
     done = vec && vec_a && a.rank % 16 == 0 && (a.dim == 64 || a.dim == 128) &&
            reinterpret_cast<uintptr_t>(a.a2) % 8 == 0;
-    if (done && a.dim == 64) intra(gla_intra_kernel<T, KIND, 1, true>);
-    else if (done) intra(gla_intra_kernel<T, KIND, 2, true>);
+    if (done && a.dim == 64) by_parts(I1{}, std::true_type{});
+    else if (done) by_parts(I2{}, std::true_type{});
   }
   if (done) {
   } else if (a.dpad <= 64) {
-    intra(gla_intra_kernel<T, KIND, 1, false>);
+    by_parts(I1{}, std::false_type{});
   } else if (a.dpad <= 128) {
-    intra(gla_intra_kernel<T, KIND, 2, false>);
+    by_parts(I2{}, std::false_type{});
   } else {
-    intra(gla_intra_kernel<T, KIND, 4, false>);
+    by_parts(I4{}, std::false_type{});
   }
   ScanArgs sa{};
   sa.v = reinterpret_cast<const T*>(a.proj) + a.off_v;
@@ -582,6 +642,7 @@ void prefill(const GlaArgs& a, hipStream_t st) {
   sa.vpad = a.vpad;
   sa.mode = kScanPlain;
   sa.f32 = a.f32;
+  sa.parts = parts;
   launch_rec_scan(sa, st);
   RecGateArgs ga{};
   ga.o = a.o;

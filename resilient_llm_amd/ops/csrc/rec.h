@@ -26,11 +26,11 @@ enum ScanMode { kScanPlain = 0, kScanMax = 1, kScanDelta = 2 };
 struct ScanArgs {
   const void* v;           // value rows (plain, max), head h at h * vdim
   const void* q;           // query rows (max, delta), head h / group
-  const float* qd;         // [n_tiles, heads, 64, dpad] in tiles (plain)
+  const void* qd;          // [n_tiles, heads, 64, dpad] in tiles (plain)
   const void* kt;          // [n_tiles, heads / group, dpad, 64] keys down
                            // the columns: f32 decayed, in tiles (plain), or as
                            // they are
-  const float* sc;         // [n_tiles, heads, 64, 64] A, in tiles (plain)
+  const void* sc;          // [n_tiles, heads, 64, 64] A, in tiles (plain)
   const float* dec;        // [n_tiles, heads, dpad] (plain), [n_tiles, heads]
   const float* rows;       // [n_tiles, heads, 3, 64]: running log-decay F,
                            // a = i - F, running maximum of a (max); query
@@ -49,7 +49,7 @@ struct ScanArgs {
   int cols;                // value columns of state and o
   float qscale;            // (max)
   int mode;
-  bool f32;
+  bool f32, parts;         // parts: qd, kt and sc (plain)
 };
 void launch_rec_scan(const ScanArgs& a, hipStream_t stream);
 
@@ -91,9 +91,11 @@ struct GlaArgs {
   const int32_t* seqs;     // [4, n_seqs]: first tile, tiles, pos0, slot
   // scratch in tiles of 16 x 16, a lane l's four elements of row l % 16 from
   // column l / 16 * 4 on next to each other, tiles of
-  float* qd;               // [n_tiles, heads, 64, dpad] down the columns,
-  float* kd;               // [n_tiles, heads, dpad, 64] and
-  float* sc;               // [n_tiles, heads, 64, 64] along the rows
+  // (or in pairs of tiles as three 16-bit parts, 1 KB a part, a lane's fours of
+  // both next to each other; queries' columns are an even number of tiles then)
+  void* qd;                // [n_tiles, heads, 64, dpad] down the columns,
+  void* kd;                // [n_tiles, heads, dpad, 64] and
+  void* sc;                // [n_tiles, heads, 64, 64] along the rows
   float* dec;              // [n_tiles, heads, dpad]
   float* o;                // [rows + 64, heads * vdim]
   void* out;               // [rows, heads * vdim], rows out_stride apart

@@ -101,6 +101,22 @@ DEV_INLINE f32x4_t quad_transposed(f32x4_t v) {
   return v;
 }
 
+// Three 16-bit parts that add up to each of four 32-bit numbers: a float's upper
+// half is a bf16 number, its first eight bits, and so on for what is left.
+DEV_INLINE void three_parts(f32x4_t v, uint2 (&p)[3]) {
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    uint32_t u[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      u[j] = __float_as_uint(v[j]);
+      v[j] -= __uint_as_float(u[j] & 0xffff0000u);
+    }
+    p[i] = uint2{__builtin_amdgcn_perm(u[1], u[0], 0x07060302u),
+                 __builtin_amdgcn_perm(u[3], u[2], 0x07060302u)};
+  }
+}
+
 DEV_INLINE f32x4_t mma4(float a, float b, f32x4_t c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }

@@ -3,8 +3,8 @@
 // that follow.
 //
 // A workgroup owns one (sequence, head, slice of value columns); a wave the
-// 16 output rows of a sub-chunk and every fourth key tile of the state.  All
-// products are f32 MFMA.  A chunk's operands travel in registers, loaded
+// 16 output rows of a sub-chunk and every fourth key tile of the state.
+// Products are f32 MFMA (but see rec_scan_parts_kernel).  A chunk's operands travel in registers, loaded
 // while the chunk before it computes.  A sequence's chunks follow one
 // another and only the last is short, so no table is on the path of a load.
 // Loads and stores are unconditional where sizes allow (what has no place
@@ -15,9 +15,7 @@
 // read as rows are, neighbouring lanes have rows of their own, and the cache
 // looks up each lane's 16 bytes by themselves, which was what bounded it (4
 // sequences of 1.9k, 8 heads of 128 x 256: 179 us, of which 145 such lookups,
-// and 133 now, of which 67 products and 40 lookups; without loads and stores
-// 97).  (With outputs and state in waves of their own, a barrier a chunk and its
-// next but one asked for ahead: 126.)
+// and 133 so).
 //
 // kScanMax: with F the chunk's running log-decay, a = i - F and the maximum
 // M_t = max(m, max_{s <= t} a_s), m what the chunk started with,
@@ -114,7 +112,8 @@ void rec_scan_kernel(ScanArgs a, bool vec_q, bool vec_v) {
           qr[i] = raw_guard(q, i * 16 + g * 4, a.dim, ok, vec_q);
       }
     } else {
-      const float* qd = a.qd + chunk(t) * C * DP + (w * 64 + lane) * 4;
+      const float* qd = static_cast<const float*>(a.qd) + chunk(t) * C * DP +
+                        (w * 64 + lane) * 4;
 #pragma unroll
       for (int i = 0; i < NQ; ++i)
         if (i < ndt) qr[i].load(qd + i * 1024);
@@ -127,7 +126,7 @@ void rec_scan_kernel(ScanArgs a, bool vec_q, bool vec_v) {
     }
   };
   auto load_a = [&](int t) {
-    const float* sc = a.sc + chunk(t) * C * C +
+    const float* sc = static_cast<const float*>(a.sc) + chunk(t) * C * C +
                       (RAW ? trow * C + g * 4 : (w * 256 + lane) * 4);
 #pragma unroll
     for (int J = 0; J < 4; ++J)            // (blocks behind w: not used)
@@ -367,6 +366,280 @@ void rec_scan_kernel(ScanArgs a, bool vec_q, bool vec_v) {
       a.m_new[int64_t(seq) * a.heads + h] = m;
 }
 
+// kScanPlain in parts, of 16-bit activations.  The values are 16-bit numbers; queries, keys,
+// A and the state are 32-bit ones, each of three 16-bit parts that add up to it,
+// so that products run on the 16-bit matrix cores: three for each of the values',
+// six for queries and state (what is left out is 2^-24 of a product).  Four
+// waves carry the state from chunk to chunk (w every fourth of its key tiles),
+// four others have the outputs (w the rows of a sub-chunk) of the chunk that the
+// state is carried over, from its parts in LDS.  There are two copies by turns, and
+// of the values, so that a chunk takes one barrier.  What bounds it is a chunk's
+// chain of latencies, 2.4 us (asked for a chunk ahead of their turn, operands take
+// 3 us of 77 off and twice the registers).  4 sequences of 1.9k, 8 heads of 128 x
+// 256: 133 us with f32 products, of which these 67, and 77 now; the kernel that
+// makes the operands 49 and 54.  (Against 64 bits, 2048 tokens, the state is off by
+// 4.3e-7 and 2.6e-7, as it is rounded less often; 6e-4 and 4e-4 of the outputs are
+// not the nearest 16-bit number.)
+template <int VT, int MD, bool FULL>
+__global__ __launch_bounds__(512, 2)
+void rec_scan_parts_kernel(ScanArgs a, bool vec_v) {
+  using T = uint16_t;
+  constexpr int VS = VT * 16, NKS = 2 * MD;
+  extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
+  const int DP = FULL ? 64 * MD : a.dpad, ndt = DP / 16;
+  const int nks = FULL ? NKS : (ndt + 1) / 2;
+  // a copy: [nks][3][VT][64][8] state, [2][VT][64][8] values
+  const int copy = (nks * 3 + 2) * VT * 512;
+  const int seq = blockIdx.x / a.heads, h = blockIdx.x % a.heads;
+  const int v0 = blockIdx.y * VS;
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6 & 3);
+  const int lr = lane & 15, g = lane >> 4;
+  const int first = a.seqs[seq], count = a.seqs[a.n_seqs + seq];
+  if (count <= 0) return;
+  const int last = first + count - 1;
+  auto chunk = [&](int t) { return int64_t(t) * a.heads + h; };
+  auto frag = [&](const uint16_t* p) {
+    return *reinterpret_cast<const s16x8_t*>(p);
+  };
+  auto mma = [](const s16x8_t& x, const s16x8_t& y, const f32x4_t& c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, y, c, 0, 0, 0);
+  };
+  auto values = [&](int t, s16x8_t (&v)[2][VT]) {
+    const uint16_t* from =
+        lds + (t & 1) * copy + nks * 3 * VT * 512 + lane * 8;
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int nt = 0; nt < VT; ++nt)
+        v[ks][nt] = frag(from + (ks * VT + nt) * 512);
+  };
+
+  if (threadIdx.x < 256) {
+    const bool fresh = a.seqs[2 * a.n_seqs + seq] == 0;
+    float* state = a.state + (int64_t(a.seqs[3 * a.n_seqs + seq]) * a.heads +
+                              h) * a.dim * a.vpad;
+    f32x4_t S[MD][VT], dv[MD];
+    s16x8_t kr[MD][2][3];
+#pragma unroll
+    for (int i = 0; i < MD; ++i)
+#pragma unroll
+      for (int nt = 0; nt < VT; ++nt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int d = (i * 4 + w) * 16 + g * 4 + r;
+          const int c = v0 + nt * 16 + lr;
+          S[i][nt][r] = (!fresh && d < a.dim && c < a.cols)
+                            ? state[int64_t(d) * a.vpad + c] : 0.f;
+        }
+    auto load = [&](int t) {
+      const uint16_t* k = static_cast<const uint16_t*>(a.kt) +
+                          chunk(t) * ndt * 3072 + lane * 8;
+      const float* dec = a.dec + chunk(t) * DP;
+#pragma unroll
+      for (int i = 0; i < MD; ++i)
+        if (FULL || i * 4 + w < ndt) {
+#pragma unroll
+          for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+            for (int p = 0; p < 3; ++p)
+              kr[i][ks][p] =
+                  frag(k + (((i * 4 + w) * 2 + ks) * 3 + p) * 512);
+          dv[i] = *reinterpret_cast<const f32x4_t*>(
+              dec + (i * 4 + w) * 16 + g * 4);
+        }
+    };
+    auto put = [&](int t, int tile, int nt, const f32x4_t& v) {
+      uint2 part[3];
+      three_parts(v, part);
+      uint16_t* to = lds + (t & 1) * copy + lane * 8 + tile % 2 * 4;
+#pragma unroll
+      for (int p = 0; p < 3; ++p)
+        *reinterpret_cast<uint2*>(to + ((tile / 2 * 3 + p) * VT + nt) * 512) =
+            part[p];
+    };
+    load(first);
+    if (!FULL && ndt % 2 && w == ndt % 4)  // (the last pair's second tile)
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int nt = 0; nt < VT; ++nt)
+          put(t, ndt, nt, f32x4_t{0.f, 0.f, 0.f, 0.f});
+    for (int t = first; t <= last; ++t) {
+#pragma unroll
+      for (int i = 0; i < MD; ++i)
+        if (FULL || i * 4 + w < ndt)
+#pragma unroll
+          for (int nt = 0; nt < VT; ++nt) put(t, i * 4 + w, nt, S[i][nt]);
+      __syncthreads();
+      s16x8_t v[2][VT];
+      values(t, v);
+#pragma unroll
+      for (int i = 0; i < MD; ++i)
+#pragma unroll
+        for (int nt = 0; nt < VT; ++nt) S[i][nt] *= dv[i];
+#pragma unroll
+      for (int p = 2; p >= 0; --p)
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+          for (int i = 0; i < MD; ++i)
+            if (FULL || i * 4 + w < ndt)
+#pragma unroll
+              for (int nt = 0; nt < VT; ++nt)
+                S[i][nt] = mma(kr[i][ks][p], v[ks][nt], S[i][nt]);
+      load(min(t + 1, last));             // (no load is conditional)
+    }
+#pragma unroll
+    for (int i = 0; i < MD; ++i)
+#pragma unroll
+      for (int nt = 0; nt < VT; ++nt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int d = (i * 4 + w) * 16 + g * 4 + r;
+          const int c = v0 + nt * 16 + lr;
+          if (d < a.dim && c < a.cols)
+            state[int64_t(d) * a.vpad + c] = S[i][nt][r];
+        }
+    return;
+  }
+
+  constexpr int VQ = VS / 4;
+  const int tid = threadIdx.x - 256;
+  const int row_first = a.tiles[first];
+  const int n_last = a.tiles[2 * a.n_tiles + last];
+  s16x8_t qr[NKS][3], ar[2][3];
+  Raw4<T> vr[VT];                         // four columns of a row
+  const T* vb = static_cast<const T*>(a.v) + h * a.vdim;
+  auto row_of = [&](int t) { return row_first + (t - first) * C; };
+  auto rows_of = [&](int t) { return t == last ? n_last : C; };
+  auto load_q = [&](int t) {
+    const uint16_t* q = static_cast<const uint16_t*>(a.qd) +
+                        chunk(t) * nks * 6144 + (w * 192 + lane) * 8;
+#pragma unroll
+    for (int ks = 0; ks < NKS; ++ks)
+      if (FULL || ks < nks)
+#pragma unroll
+        for (int p = 0; p < 3; ++p) qr[ks][p] = frag(q + (ks * 12 + p) * 512);
+  };
+  auto load_a = [&](int t) {
+    const uint16_t* sc = static_cast<const uint16_t*>(a.sc) +
+                         chunk(t) * 12288 + (w * 384 + lane) * 8;
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)         // (a pair behind w: not used)
+#pragma unroll
+      for (int p = 0; p < 3; ++p)
+        ar[ks][p] = frag(sc + (min(ks, w / 2) * 3 + p) * 512);
+  };
+  auto load_v = [&](int t) {
+    const int row0 = row_of(t), n = rows_of(t);
+#pragma unroll
+    for (int i = 0; i < VT; ++i) {
+      const int e = i * 256 + tid;
+      const int r = e / VQ, c = v0 + e % VQ * 4;
+      if constexpr (FULL)
+        vr[i].load(vb + int64_t(row0 + min(r, n - 1)) * a.v_stride + c);
+      else
+        vr[i] = raw_guard(vb + int64_t(row0 + r) * a.v_stride, c, a.vdim,
+                          r < n, vec_v);
+    }
+  };
+  load_v(first);
+  load_q(first);
+  load_a(first);
+  for (int t = first; t <= last; ++t) {
+    const int next = min(t + 1, last);     // (no load is conditional)
+    const int row0 = row_of(t), n = rows_of(t);
+    const uint16_t* Sl = lds + (t & 1) * copy + lane * 8;
+    uint16_t* Vl = lds + (t & 1) * copy + nks * 3 * VT * 512;
+#pragma unroll
+    for (int i = 0; i < VT; ++i) {
+      const int e = i * 256 + tid;
+      const int r = e / VQ, c = e % VQ * 4;
+      const uint2 v = r < n ? vr[i].r : uint2{0, 0};
+      // down a column, as the products take it
+      uint16_t* to = Vl + (r / 32 * VT + c / 16) * 512 +
+                     ((r % 16 / 4) * 16 + c % 16) * 8 + r / 16 % 2 * 4 + r % 4;
+      to[0] = uint16_t(v.x);
+      to[8] = uint16_t(v.x >> 16);
+      to[16] = uint16_t(v.y);
+      to[24] = uint16_t(v.y >> 16);
+    }
+    load_v(next);
+    __syncthreads();
+    f32x4_t o[2][VT];
+#pragma unroll
+    for (int nt = 0; nt < VT; ++nt)
+      o[0][nt] = o[1][nt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int ks = 0; ks < NKS; ++ks) {
+      if (!FULL && ks >= nks) continue;
+      s16x8_t s[3][VT];
+#pragma unroll
+      for (int p = 0; p < 3; ++p)
+#pragma unroll
+        for (int nt = 0; nt < VT; ++nt)
+          s[p][nt] = frag(Sl + ((ks * 3 + p) * VT + nt) * 512);
+      auto both = [&](int acc, int x, int y) {
+#pragma unroll
+        for (int nt = 0; nt < VT; ++nt)
+          o[acc][nt] = mma(qr[ks][x], s[y][nt], o[acc][nt]);
+      };
+      both(0, 0, 2);
+      both(1, 2, 0);
+      both(0, 1, 1);
+      both(1, 1, 0);
+      both(0, 0, 0);
+      both(1, 0, 1);
+    }
+    load_q(next);
+    s16x8_t v[2][VT];
+    values(t, v);
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+      if (ks > w / 2) break;
+#pragma unroll
+      for (int p = 2; p >= 0; --p)
+#pragma unroll
+        for (int nt = 0; nt < VT; ++nt)
+          o[p > 0][nt] = mma(ar[ks][p], v[ks][nt], o[p > 0][nt]);
+    }
+    load_a(next);
+#pragma unroll
+    for (int nt = 0; nt < VT; ++nt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int tr = w * 16 + g * 4 + r, c = v0 + nt * 16 + lr;
+        const bool ok = tr < n && (FULL || c < a.cols);
+        a.o[(int64_t(ok ? row0 + tr : a.n_rows + tr) * a.heads + h) * a.opad +
+            (ok ? c : 0)] = o[0][nt][r] + o[1][nt][r];
+      }
+  }
+}
+
+template <int VT>
+void scan_parts(const ScanArgs& a, hipStream_t st) {
+  constexpr int VS = VT * 16;
+  const int nks = (a.dpad / 16 + 1) / 2;
+  const size_t smem = size_t(2) * (nks * 3 + 2) * VT * 1024;
+  const bool vec_v = a.v_stride % 4 == 0 && a.vdim % 4 == 0 &&
+                     reinterpret_cast<uintptr_t>(a.v) % 8 == 0;
+  auto run = [&](auto* k) {
+    if (smem > 65536)
+      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(k),
+                                hipFuncAttributeMaxDynamicSharedMemorySize,
+                                int(smem));
+    hipLaunchKernelGGL(k, dim3(a.n_seqs * a.heads, (a.cols + VS - 1) / VS),
+                       dim3(512), smem, st, a, vec_v);
+  };
+  const bool full = vec_v && a.vdim % VS == 0;
+  if (full && a.dim == 64) run(rec_scan_parts_kernel<VT, 1, true>);
+  else if (full && a.dim == 128) run(rec_scan_parts_kernel<VT, 2, true>);
+  else if (a.dpad <= 64) run(rec_scan_parts_kernel<VT, 1, false>);
+  else if (a.dpad <= 128) run(rec_scan_parts_kernel<VT, 2, false>);
+  else if constexpr (VT < 4) run(rec_scan_parts_kernel<VT, 4, false>);
+}
+
 template <typename T, int MODE, int VT>
 void scan_md(const ScanArgs& a, hipStream_t st) {
   constexpr int VS = VT * 16;
@@ -406,6 +679,20 @@ void scan(const ScanArgs& a, hipStream_t st) {
   // a scan step is latency-bound: narrow value slices, several
   // workgroups per CU, until there are plenty anyway
   const int64_t sh = int64_t(a.n_seqs) * a.heads;
+  if constexpr (MODE == kScanPlain && sizeof(T) == 2)
+    if (a.parts) {
+      // as wide slices as leave a workgroup for each CU (two copies of 256 rows
+      // by 64 columns do not fit LDS; whole prompts, us, slices of 16, 32 and 64
+      // columns: heads of 128 x 256, 8 of them 97 105 141, 16 113 119 151, 32 190
+      // 158 183, 64 195 163 141)
+      if (a.dpad <= 128 && sh * ((a.vdim + 63) / 64) >= 256)
+        scan_parts<4>(a, st);
+      else if (sh * ((a.vdim + 31) / 32) >= 256)
+        scan_parts<2>(a, st);
+      else
+        scan_parts<1>(a, st);
+      return;
+    }
   if (a.vdim > 32 && sh * ((a.vdim + 63) / 64) >= 512)
     scan_md<T, MODE, 4>(a, st);
   else if (a.vdim > 16 && sh * ((a.vdim + 31) / 32) >= 1024)

@@ -7,6 +7,7 @@ import torch
 
 import resilient_llm_amd.ops as ops
 from nesizen_util import BF16, F32
+from resilient_llm_amd.engine.batch import Portion, PromptRows
 from test_lat_ops import hgrn2_case
 from test_mix_ops import gla_case, rel, tol
 from test_rec_ops import Rwkv
@@ -95,3 +96,31 @@ def test_lanes_and_rows(dim, vdim, rank, dtype):
         assert rel(got[:, i], want) < tol(dtype)
         assert rel(st[slot, :, :, :vdim], S) < 1e-5
     assert torch.isnan(st[[1, 3]]).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("seqs,H,dim,vdim", [
+    # slices of 16, 32 and 64 columns, full and ragged ones; odd numbers of
+    # tiles down the columns
+    (2, 3, 128, 48), (2, 3, 40, 33), (2, 64, 40, 33), (2, 64, 64, 32),
+    (2, 64, 130, 40), (2, 64, 128, 128), (2, 64, 24, 97), (2, 64, 72, 70),
+    # short heads that fill the chip: f32 operands
+    (4, 128, 16, 20), (4, 128, 64, 64)])
+def test_prompts_by_slices(seqs, H, dim, vdim):
+    lens = [130, 65, 3, 64][:seqs]
+    *inputs, eps, want, S = gla_case(lens[0], H, dim, vdim, 8, 8.0, 1.0,
+                                     dim + vdim, BF16)
+    proj, a2, b, norm = (t.cuda() for t in inputs)
+    st = torch.full((seqs + 1, H, dim, -(-vdim // 4) * 4), float("nan"),
+                    device="cuda")
+    portions, at = [], 0
+    for i, n in enumerate(lens):
+        portions.append(Portion(at, 0, n, i, i))
+        at += n
+    got = ops.gla_prefill(torch.cat([proj[:n] for n in lens]), a2, b, norm,
+                          st, PromptRows(portions, "cuda"), vdim, 8.0, eps)
+    # the bounds of the longer runs over the same steps
+    for n, rows in zip(lens, got.split(lens)):
+        assert rel(rows, want[:n]) < tol(BF16)
+    assert rel(st[0, :, :, :vdim], S) < 1e-5
+    assert torch.isnan(st[seqs]).all()

@@ -64,14 +64,27 @@ DEV_INLINE float half_max_dpp(float v) {
 // 16 rows per workgroup, K split over eight waves, whose halves then rank a row
 // each.  What bounds it is latency: a round of loads where they fit the
 // registers (32 routes of 2048: all of them), sums through LDS, and a choice
-// after the other.  It leaves how often its rows chose each expert behind, so
+// after the other.  Loaded as the products take them, neighbouring lanes have rows
+// of their own and the cache looks up 16 bytes at a time; turned in LDS they come
+// by 64 (32 routes of 2048, us: 1 row 8.5 and 7.5, 64 9.7 and 8.1, 6001 17.8 and
+// 16.1).  It leaves how often its rows chose each expert behind, so
 // that the plan needs no pass of its own over the choices.
 template <typename T, int ET>
 __global__ __launch_bounds__(512)
 void moe_route_kernel(MoeArgs a) {
   constexpr int E16 = ET * 16, NW = 8;
-  __shared__ float part[NW][16][E16 + 1];
+  // (32-bit activations and many routes are too much for LDS)
+  constexpr bool LINES = sizeof(T) == 2 && ET <= 4;
+  __shared__ union {
+    s16x8_t turns[LINES ? NW * 64 * (ET + 1) : 1];
+    float part[NW][16][E16 + 1];          // behind them
+  } lds;
+  auto& part = lds.part;
   __shared__ int chosen[E16];
+  auto wave_fence = [] {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  };
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int lr = lane & 15, g = lane >> 4;
   const int row0 = blockIdx.x * 16;
@@ -89,6 +102,46 @@ void moe_route_kernel(MoeArgs a) {
   }
   constexpr int U = ET <= 4 ? 4 : 1;      // k steps with loads in flight
   int k0 = w * 32;
+  if constexpr (LINES) {
+    // four lanes to 64 bytes of a row, and to the lanes that multiply them
+    // through LDS, turned by the row so that reads meet no bank twice
+    s16x8_t* turn = lds.turns + w * 64 * (ET + 1);
+    const int rr = lane >> 2, piece = (lane & 3) ^ (rr >> 2);
+    const T* hp = reinterpret_cast<const T*>(a.h) +
+                  int64_t(min(row0 + rr, a.rows - 1)) * a.width + piece * 8;
+    const T* rp[ET];
+#pragma unroll
+    for (int e = 0; e < ET; ++e)
+      rp[e] = wr + int64_t(min(e * 16 + rr, a.routes - 1)) * a.width +
+              piece * 8;
+    const int mine = lr * 4 + (g ^ (lr >> 2));
+    for (; k0 + (U - 1) * NW * 32 + 32 <= a.width; k0 += U * NW * 32) {
+      s16x8_t raw[U][ET + 1];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int k = k0 + u * NW * 32;
+        raw[u][ET] = *reinterpret_cast<const s16x8_t*>(hp + k);
+#pragma unroll
+        for (int e = 0; e < ET; ++e)
+          raw[u][e] = *reinterpret_cast<const s16x8_t*>(rp[e] + k);
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+#pragma unroll
+        for (int i = 0; i <= ET; ++i) turn[i * 64 + lane] = raw[u][i];
+        wave_fence();
+        Frag8<T> fa, fb[ET];
+        fa.v = turn[ET * 64 + mine];
+#pragma unroll
+        for (int e = 0; e < ET; ++e)
+          fb[e].v = turn[e * 64 + mine];
+        wave_fence();
+#pragma unroll
+        for (int e = 0; e < ET; ++e)
+          acc[e] = Frag8<T>::mma(fa, fb[e], acc[e]);
+      }
+    }
+  }
   for (; k0 + (U - 1) * NW * 32 + 32 <= a.width; k0 += U * NW * 32) {
     Frag8<T> fa[U], fb[U][ET];
 #pragma unroll
@@ -117,6 +170,7 @@ void moe_route_kernel(MoeArgs a) {
       acc[e] = Frag8<T>::mma(fa, fb, acc[e]);
     }
   }
+  if constexpr (LINES) __syncthreads();
 #pragma unroll
   for (int e = 0; e < ET; ++e)
 #pragma unroll
@@ -126,10 +180,6 @@ void moe_route_kernel(MoeArgs a) {
   // a half ranks a row, its lane l holding routes l, l + 32, ...
   constexpr int EL = (E16 + 31) / 32;
   constexpr float kNone = -INFINITY;      // cannot be chosen
-  auto wave_fence = [] {
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-  };
   const int hl = lane & 31;
   const int t = w * 2 + (lane >> 5);
   const int row = row0 + t;               // (past the last: nobody's)

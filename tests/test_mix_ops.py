@@ -462,6 +462,16 @@ def test_heights_of_tiles(T, E, top, ff):
     test_experts(T, 64, E, top, ff, 0, "cuda:0", BF16)
 
 
+@GPU
+@pytest.mark.parametrize("T,W,E", [
+    # whole rounds of the router's loads, their rest, and neither; routes around
+    # the lines between its kernels
+    (1, 1024, 16), (17, 1032, 17), (15, 2048, 33), (16, 2056, 48),
+    (33, 1288, 49), (5, 3072, 64), (16, 1024, 65), (3, 1000, 31)])
+def test_rounds_of_the_router(T, W, E):
+    test_experts(T, W, E, 3, 32, 0, "cuda:0", BF16)
+
+
 @pytest.mark.parametrize("device", DEVICES)
 def test_router_ties_go_to_the_lower_expert(device):
     h = torch.ones(3, 64)

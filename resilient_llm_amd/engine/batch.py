@@ -14,6 +14,18 @@ import dataclasses
 import torch
 
 
+def sent(values, dtype, device) -> torch.Tensor:
+    """``values`` on ``device`` by a copy that the host does not wait for (and, on
+    the same stream, whoever reads them needs not either).  One from pageable
+    memory ends when the stream has come to it, and until the host has launched
+    anew the GPU is idle: five such copies in the first layers of the mixed
+    models' prompts cost 0.2 ms of a step."""
+    device = torch.device(device)
+    return torch.tensor(values, dtype=dtype,
+                        pin_memory=device.type == "cuda").to(
+        device, non_blocking=True)
+
+
 @dataclasses.dataclass(frozen=True)
 class Portion:
     row0: int
@@ -36,8 +48,7 @@ class PromptRows:
 
     def _table(self, rows: list) -> torch.Tensor:
         """Columns of ``rows`` as the rows of one int32 tensor."""
-        return torch.tensor(rows, dtype=torch.int32).t().contiguous() \
-            .to(self.device)
+        return sent(list(zip(*rows)), torch.int32, self.device)
 
     def tiles(self, height: int) -> torch.Tensor:
         """int32 [4, n]: first row, its position, rows, sequence."""
@@ -77,7 +88,7 @@ class PromptRows:
             pos = [0] * (1 + max(p.seq for p in self.portions))
             for p in self.portions:
                 pos[p.seq] = p.pos0
-            return torch.tensor(pos, dtype=torch.int32).to(self.device)
+            return sent(pos, torch.int32, self.device)
         return self._once(("pos0",), make)
 
     def gathered(self, height: int, chunk: int = 0) -> tuple:
@@ -99,5 +110,5 @@ class PromptRows:
                          for o in range(start, ctx, height)]
                 at += -(-(ctx - start) // height) * height
             return (self._table(rows),
-                    torch.tensor(off, dtype=torch.int32).to(self.device), at)
+                    sent(off, torch.int32, self.device), at)
         return self._once(("gathered", height, chunk), make)

@@ -23,7 +23,7 @@ from typing import Optional
 import torch
 
 from .. import ops
-from .batch import Portion, PromptRows
+from .batch import Portion, PromptRows, sent
 from .kv_cache import OutOfBlocks, PagedKVCache, block_hash_chain
 
 # roctx phase markers for rocprofv3 --marker-trace:
@@ -734,14 +734,11 @@ class LLMEngine:
             row += n
 
         def i32(x):
-            return torch.tensor(x, dtype=torch.int32, device=dev)
+            return sent(x, torch.int32, dev)
 
         def bt_tensor(rows):
             w = max((len(r) for r in rows), default=1)
-            t = torch.zeros((max(len(rows), 1), w), dtype=torch.int32)
-            for i, r in enumerate(rows):
-                t[i, :len(r)] = torch.tensor(r, dtype=torch.int32)
-            return t.to(dev)
+            return i32([r + [0] * (w - len(r)) for r in rows] or [[0] * w])
 
         state_slots = None if self.states is None else i32(
             [s.slot for s, _ in dec])
@@ -752,8 +749,7 @@ class LLMEngine:
                 i32(input_ids), i32(positions), self.kv, i32(slots),
                 bt_tensor([s.blocks for s, _ in dec]), i32(seq_lens_d),
                 **extra)
-            return logits[torch.tensor(sample_idx, dtype=torch.long,
-                                       device=dev)]
+            return logits[sent(sample_idx, torch.long, dev)]
         # fast path: no decode rows and every chunk is a whole prompt ->
         # classic batched varlen prefill over in-batch K/V (no paged
         # reads, no row-copy) — this is the bench/burst-arrival shape
@@ -783,7 +779,7 @@ class LLMEngine:
         args = (i32(input_ids), i32(positions), self.kv, i32(slots), B_d,
                 bt_tensor([s.blocks for s, _ in dec]) if B_d else None,
                 i32(seq_lens_d) if B_d else None)
-        sample_t = torch.tensor(sample_idx, dtype=torch.long, device=dev)
+        sample_t = sent(sample_idx, torch.long, dev)
         if mixed_layers:
             args += (bt_tensor(bt_rows), PromptRows(portions, dev), sample_t,
                      state_slots)

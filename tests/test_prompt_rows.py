@@ -7,6 +7,7 @@ import pytest
 import torch
 
 from resilient_llm_amd.engine import LLMEngine, PagedKVCache
+from resilient_llm_amd.engine.batch import Portion, PromptRows
 from resilient_llm_amd.models import LlamaForCausalLM, get_config
 
 pytestmark = pytest.mark.gpu
@@ -93,3 +94,21 @@ def test_one_token():
                                                 rows)
                           for i in range(5, 1005)])
     assert torch.equal(logits(True), logits(False))
+
+
+@pytest.mark.parametrize("n", [1, 64, 65, 700])
+def test_tables_behind_a_busy_stream(n):
+    """Tables are sent by copies that nobody waits for: made one after another
+    while the stream is busy, each has its own values."""
+    def tables(device, i):
+        rows = PromptRows([Portion(0, i, n, 0, 1), Portion(n, 0, i + 1, 1, i)],
+                          device)
+        return [rows.tiles(64), rows.seqs(64), rows.spans(32), rows.pos0(),
+                *rows.gathered(32)[:2], rows.vectors(16, 3)]
+    x = torch.randn(4096, 4096, device="cuda")
+    for _ in range(20):
+        x = torch.mm(x, x) * 1e-3
+    got = [tables("cuda", i) for i in range(30)]
+    for i, made in enumerate(got):
+        for g, want in zip(made, tables("cpu", i)):
+            assert g.dtype == want.dtype and torch.equal(g.cpu(), want)

@@ -1254,8 +1254,8 @@ static Tensor norm_any(const Tensor& x, const Tensor& residual,
 
 // All of a Llama layer but the first for the rows of a few short prompts, whose
 // step waits for the host: the ops in their order, rotation, append and attention
-// as one, launched from here; the last product and the new residual, which is ``residual`` itself unless the one row's
-// norm is made inside gate and up.
+// as one, launched from here; the last product and the new residual, which is
+// ``residual`` itself unless the one row's norm is made inside gate and up.
 // (A prompt of 45 tokens through 16 layers of 2048: 8 us a launch from Python, 5
 // from here; 1150 -> 1040 us.)
 std::tuple<Tensor, Tensor> prompt_rows_layer(

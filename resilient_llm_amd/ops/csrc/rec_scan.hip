@@ -4,9 +4,10 @@
 //
 // A workgroup owns one (sequence, head, slice of value columns); a wave the
 // 16 output rows of a sub-chunk and every fourth key tile of the state.
-// Products are f32 MFMA (but see rec_scan_parts_kernel).  A chunk's operands travel in registers, loaded
-// while the chunk before it computes.  A sequence's chunks follow one
-// another and only the last is short, so no table is on the path of a load.
+// Products are f32 MFMA (but see rec_scan_parts_kernel).  A chunk's operands
+// travel in registers, loaded while the chunk before it computes.  A
+// sequence's chunks follow one another and only the last is short, so no table
+// is on the path of a load.
 // Loads and stores are unconditional where sizes allow (what has no place
 // goes to spare rows), since a branch around one makes later waits drain
 // everything in flight.
@@ -366,11 +367,11 @@ void rec_scan_kernel(ScanArgs a, bool vec_q, bool vec_v) {
       a.m_new[int64_t(seq) * a.heads + h] = m;
 }
 
-// kScanPlain in parts, of 16-bit activations.  The values are 16-bit numbers; queries, keys,
-// A and the state are 32-bit ones, each of three 16-bit parts that add up to it,
-// so that products run on the 16-bit matrix cores: three for each of the values',
-// six for queries and state (what is left out is 2^-24 of a product).  Four
-// waves carry the state from chunk to chunk (w every fourth of its key tiles),
+// kScanPlain in parts, of 16-bit activations.  The values are 16-bit numbers;
+// queries, keys, A and the state are 32-bit ones, each of three 16-bit parts that
+// add up to it, so that products run on the 16-bit matrix cores: three for each of
+// the values', six for queries and state (what is left out is 2^-24 of a product).
+// Four waves carry the state from chunk to chunk (w every fourth of its key tiles),
 // four others have the outputs (w the rows of a sub-chunk) of the chunk that the
 // state is carried over, from its parts in LDS.  There are two copies by turns, and
 // of the values, so that a chunk takes one barrier.  What bounds it is a chunk's

@@ -2,8 +2,8 @@
 // other, up to four query heads of a key/value head, no distance bias.
 //
 // The work of a wave is decode_attn.h's: units of 32 tokens whose keys and
-// values are all asked for at once, 24 bits of every weight.  Units are those of the
-// kept tokens and then the window's, whose number is bounded, so that a workgroup
+// values are all asked for at once, 24 bits of every weight.  Units are those of
+// the kept tokens and then the window's, whose number is bounded, so that a workgroup
 // of twelve waves has all of a sequence's units or as many parts of them as make a
 // round each, where that leaves CUs idle.  What bounds it is latency: from the
 // launch to positions, pages and keys 3 us, 3.5 us a round.  us, in lane groups of

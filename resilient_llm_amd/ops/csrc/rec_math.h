@@ -102,15 +102,21 @@ DEV_INLINE f32x4_t quad_transposed(f32x4_t v) {
 }
 
 // Three 16-bit parts that add up to each of four 32-bit numbers: a float's upper
-// half is a bf16 number, its first eight bits, and so on for what is left.
+// half is a bf16 number, its first eight bits, and so on for what is left.  All
+// have the number's sign, the later ones are never zero and of an infinite number
+// least, so that products with infinite numbers are infinite alike and not NaN.
 DEV_INLINE void three_parts(f32x4_t v, uint2 (&p)[3]) {
+  float least[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) least[j] = copysignf(0x1p-120f, v[j]);
 #pragma unroll
   for (int i = 0; i < 3; ++i) {
     uint32_t u[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       u[j] = __float_as_uint(v[j]);
-      v[j] -= __uint_as_float(u[j] & 0xffff0000u);
+      const float left = v[j] - __uint_as_float(u[j] & 0xffff0000u);
+      v[j] = (i > 0 || u[j] & 0xffffu ? left : 0.f) + least[j];
     }
     p[i] = uint2{__builtin_amdgcn_perm(u[1], u[0], 0x07060302u),
                  __builtin_amdgcn_perm(u[3], u[2], 0x07060302u)};

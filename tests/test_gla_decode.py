@@ -124,3 +124,28 @@ def test_prompts_by_slices(seqs, H, dim, vdim):
         assert rel(rows, want[:n]) < tol(BF16)
     assert rel(st[0, :, :, :vdim], S) < 1e-5
     assert torch.isnan(st[seqs]).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [F32, BF16])
+def test_infinite_state(dtype):
+    """One infinite number of a state makes its column infinite, whatever its
+    sign and the queries, and the norm the head's other columns zero; no other
+    head sees it."""
+    T, H, dim, vdim, at = 70, 3, 64, 96, 37
+    *inputs, eps, want, S = gla_case(T, H, dim, vdim, 8, 8.0, 1.0, 5, dtype)
+    proj, a2, b, norm = (t.cuda() for t in inputs)
+    st = torch.zeros(1, H, dim, vdim, device="cuda")
+    clean = st.clone()
+    st[0, 1, 9, at] = float("-inf")
+    rows = PromptRows([Portion(0, 64, T, 0, 0)], "cuda")
+    got, ref = (ops.gla_prefill(proj, a2, b, norm, s, rows, vdim, 8.0,
+                                eps).view(T, H, vdim) for s in (st, clean))
+    assert torch.equal(got[:, 0], ref[:, 0])
+    assert torch.equal(got[:, 2], ref[:, 2])
+    rest = torch.arange(vdim, device="cuda") != at
+    assert not torch.isfinite(got[:, 1, at]).any()
+    assert (got[:, 1][:, rest] == 0).all()
+    assert torch.isinf(st[0, 1, 9, at])
+    st[0, 1, 9, at] = clean[0, 1, 9, at]
+    assert torch.equal(st, clean)

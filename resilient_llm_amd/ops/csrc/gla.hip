@@ -605,8 +605,10 @@ void prefill(const GlaArgs& a, hipStream_t st) {
   using I1 = std::integral_constant<int, 1>;
   using I2 = std::integral_constant<int, 2>;
   using I4 = std::integral_constant<int, 4>;
-  bool done = false;                      // (gains nothing for the others)
-  if constexpr (sizeof(T) == 2 && KIND == kRwkv) {
+  // without a conditional load where sizes allow (GLA, 4 sequences of 1.9k, 8 heads
+  // of 128 x 256: 57 and 50 us)
+  bool done = false;
+  if constexpr (sizeof(T) == 2 && KIND != kHgrn2) {
     done = vec && vec_a && a.rank % 16 == 0 && (a.dim == 64 || a.dim == 128) &&
            reinterpret_cast<uintptr_t>(a.a2) % 8 == 0;
     if (done && a.dim == 64) by_parts(I1{}, std::true_type{});

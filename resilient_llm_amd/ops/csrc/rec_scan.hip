@@ -378,9 +378,10 @@ void rec_scan_kernel(ScanArgs a, bool vec_q, bool vec_v) {
 // chain of latencies, 2.4 us (asked for a chunk ahead of their turn, operands take
 // 3 us of 80 off and twice the registers).  4 sequences of 1.9k, 8 heads of 128 x
 // 256: 133 us with f32 products, of which these 67, and 80 now; the kernel that
-// makes the operands 49 and 57 (77 and 54 if infinite numbers had NaN for parts).  (Against 64 bits, 2048 tokens, the state is off by
-// 4.3e-7 and 2.6e-7, as it is rounded less often; 6e-4 and 4e-4 of the outputs are
-// not the nearest 16-bit number.)
+// makes the operands 49 and 50 (with infinite numbers' parts NaN, 3 us less each).
+// Against 64 bits, 2048 tokens, the state is off by 4.3e-7 and 2.6e-7, as it is
+// rounded less often; 6e-4 and 4e-4 of the outputs are not the nearest 16-bit
+// number.
 template <int VT, int MD, bool FULL>
 __global__ __launch_bounds__(512, 2)
 void rec_scan_parts_kernel(ScanArgs a, bool vec_v) {

@@ -149,3 +149,24 @@ def test_infinite_state(dtype):
     assert torch.isinf(st[0, 1, 9, at])
     st[0, 1, 9, at] = clean[0, 1, 9, at]
     assert torch.equal(st, clean)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T", [1, 15, 63, 64, 65, 130])
+@pytest.mark.parametrize("dim,rank", [(64, 16), (128, 16), (128, 48), (64, 24)])
+def test_prompts_without_conditions(T, dim, rank):
+    """Heads of 64 and 128 whose rows and ranks come in whole loads, up to and
+    beyond a chunk's last row."""
+    H, vdim = 2, 48
+    *inputs, eps, want, S = gla_case(T, H, dim, vdim, rank, 8.0, 1.0, T + rank,
+                                     BF16)
+    # what lies behind the last row is not a row
+    proj, a2, b, norm = (t.cuda() for t in inputs)
+    proj = torch.cat([proj, torch.full_like(proj[:1], float("nan"))])[:T]
+    st = torch.full((2, H, dim, vdim), float("nan"), device="cuda")
+    got = ops.gla_prefill(proj, a2, b, norm, st,
+                          PromptRows([Portion(0, 0, T, 0, 1)], "cuda"), vdim,
+                          8.0, eps)
+    # the bounds of the longer runs over the same steps
+    assert rel(got, want) < tol(BF16)
+    assert rel(st[1], S) < 1e-5

@@ -235,13 +235,14 @@ void window_units_kernel(WindowAttnArgs a) {
         s[t][r] = seen(tok0 + t * 16 + oct * 4 + r) ? v : kNegInf;
         mx = fmaxf(mx, s[t][r]);
       }
-    // what is hidden may be anything
-    if (last - tok0 >= a.window)
+    // what is hidden may be anything, and what repeats the last value infinite,
+    // of which no weight makes zero
+    if (last - tok0 >= a.window || tok0 + UNIT - 1 > last)
 #pragma unroll
       for (int t = 0; t < 2; ++t)
 #pragma unroll
         for (int r = 0; r < 4; ++r)
-          if (!seen(min(tok0 + t * 16 + oct * 4 + r, last))) vr[t][r] = vraw{};
+          if (!seen(tok0 + t * 16 + oct * 4 + r)) vr[t][r] = vraw{};
     mx = fmaxf(mx, __shfl_xor(mx, 16, kWave));
     mx = fmaxf(mx, __shfl_xor(mx, 32, kWave));
     const float mn = fmaxf(m, mx);

@@ -284,6 +284,25 @@ def test_decode_units(H, G, dim, window, keep):
 
 
 @GPU
+@pytest.mark.parametrize("H,G,dim", [(8, 2, 128), (4, 2, 64), (2, 2, 128)])
+@pytest.mark.parametrize("window,keep", [(1000, 40), (33, 0)])
+def test_newest_value_infinite(H, G, dim, window, keep):
+    """An infinite value makes its channel so also as the newest token's, wherever
+    in a unit of 32 tokens that is."""
+    a = Attn(430, H, G, dim, dim, 32, window, keep, "cuda:0", BF16)
+    inf = float("inf")
+    rest = [d for d in range(dim) if d not in (7, dim - 1)]
+    for i in (0, 1, 14, 30, 31, 32, 45, 399, 429):
+        a.v[i, :, 7], a.v[i, :, -1] = inf, -inf
+        a.run(0, i + 1)
+        got, want = (t[-1].float().cpu().view(H, dim)
+                     for t in (a.run(i, 1, decode=True), a.want()[:i + 1]))
+        assert (got[:, 7] == inf).all() and (got[:, -1] == -inf).all(), i
+        assert rel(got[:, rest], want[:, rest]) < tol(BF16), i
+        a.v[i, :, 7] = a.v[i, :, -1] = 0
+
+
+@GPU
 def test_fp8_cache():
     a = Attn(120, 8, 2, 64, 64, 32, 50, 4, "cuda:0", BF16,
              cache_dtype=torch.float8_e4m3fn)

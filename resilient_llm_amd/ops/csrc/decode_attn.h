@@ -505,6 +505,13 @@ DEV_INLINE void attend(const DecodeArgs& a, int block,
     for (int i = 0; i < HS / 4; ++i)
       pf[i] = __builtin_bit_cast(
           s16x8, (uint4{pw[i][0], pw[i][1], pw[i][2], pw[i][3]}));
+    // what repeats the last value may be infinite, of which no weight makes zero
+    if (std::is_same<KC, CacheBF16>::value && tok0 + UNIT > len)
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (tok0 + t * 16 + oct * 4 + i > last) vr[t][i] = vraw{};
     uint32_t vw[2][4][VT / 2];
 #pragma unroll
     for (int t = 0; t < 2; ++t)

@@ -258,6 +258,33 @@ def test_infinite_keys_and_values(n_q, n_kv, D, L):
     close(got, want)
 
 
+@pytest.mark.parametrize("n_q,n_kv,D,bs", [(8, 2, 128, 16), (8, 1, 64, 16),
+                                           (2, 2, 64, 8)])
+def test_newest_value_infinite(n_q, n_kv, D, bs):
+    """An infinite value makes its channel so also as the newest token's, wherever
+    in a unit of 32 tokens that is."""
+    k, v, tables, n, qkv = setup([1, 31, 32, 33, 70, 257, 1000], n_q, n_kv, D,
+                                 bs, False)
+    new = qkv[:, (n_q + n_kv) * D:].view(len(n), n_kv, D)
+    new[..., 7], new[..., 9] = torch.inf, -torch.inf
+    pos = n - 1
+    slots = tables.gather(1, (pos // bs).long()[:, None])[:, 0] * bs + pos % bs
+    cs = ref.build_cos_sin(1000, D)
+    kc, vc = k.to(DEV), v.to(DEV)
+    got = ops.decode_attn_rope_qkv(
+        qkv.to(DEV), pos.to(DEV), cs.to(DEV), kc, vc, slots.to(DEV),
+        tables.to(DEV), n.to(DEV), D ** -0.5, n_q).view(-1, n_q, D)
+    q = qkv[:, :n_q * D].reshape(-1, n_q, D)
+    want = exact(ref._rotate(q.float(), pos, cs), kc.cpu(), vc.cpu(), tables, n,
+                 D ** -0.5)
+    assert (want[..., 7] == torch.inf).all() and want[..., :7].isfinite().all()
+    close(got, want)
+    # and where the cache has it
+    got = ops.decode_attn(q.to(DEV), kc, vc, tables.to(DEV), n.to(DEV),
+                          D ** -0.5)
+    close(got, exact(q, kc.cpu(), vc.cpu(), tables, n, D ** -0.5))
+
+
 def test_parts_follow_from_the_batch():
     """Together the sequences have parts of ten units, alone of eight: the
     sums' order differs, and with it the last bit of some outputs."""

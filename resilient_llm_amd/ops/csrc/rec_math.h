@@ -103,12 +103,14 @@ DEV_INLINE f32x4_t quad_transposed(f32x4_t v) {
 
 // Three 16-bit parts that add up to each of four 32-bit numbers: a float's upper
 // half is a bf16 number, its first eight bits, and so on for what is left.  All
-// have the number's sign, the later ones are never zero and of an infinite number
+// have the number's sign, the later ones are not zero and of an infinite number
 // least, so that products with infinite numbers are infinite alike and not NaN.
+// Zero has zeros only: a score that is masked takes nothing of a value.
 DEV_INLINE void three_parts(f32x4_t v, uint2 (&p)[3]) {
   float least[4];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) least[j] = copysignf(0x1p-120f, v[j]);
+  for (int j = 0; j < 4; ++j)
+    least[j] = __builtin_amdgcn_fmed3f(v[j], -0x1p-120f, 0x1p-120f);
 #pragma unroll
   for (int i = 0; i < 3; ++i) {
     uint32_t u[4];

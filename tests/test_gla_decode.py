@@ -152,6 +152,26 @@ def test_infinite_state(dtype):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [F32, BF16])
+@pytest.mark.parametrize("row", [1, 9, 17, 40, 63])
+def test_nothing_of_later_rows(row, dtype):
+    """Values as large as there are leave the bits of small rows ahead of them as
+    they are."""
+    T, H, dim, vdim = 64, 2, 64, 32
+    proj, a2, b, norm = (t.cuda() for t in gla_case(T, H, dim, vdim, 8, 8.0, 1.0,
+                                                    5, dtype)[:4])
+    proj[:row] *= 2.0 ** -20
+    loud = proj.clone()
+    loud[row:, 2 * H * dim:2 * H * dim + H * vdim] = 2.0 ** 126
+    got, want = (ops.gla_prefill(
+        p, a2, b, norm, torch.zeros(1, H, dim, vdim, device="cuda"),
+        PromptRows([Portion(0, 0, T, 0, 0)], "cuda"), vdim, 8.0, 1e-30)[:row]
+        for p in (loud, proj))
+    assert want.isfinite().all() and (want != 0).any()
+    assert torch.equal(got, want)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("T", [1, 15, 63, 64, 65, 130])
 @pytest.mark.parametrize("dim,rank", [(64, 16), (128, 16), (128, 48), (64, 24)])
 def test_prompts_without_conditions(T, dim, rank):

@@ -933,9 +933,6 @@ std::tuple<Tensor, Tensor> rows_linear_streams_(
   f32(out_w, S, "out_w");
   f32(in_w, S, "in_w");
   f32(gain, N, "gain");
-  TORCH_CHECK((reinterpret_cast<uintptr_t>(streams.data_ptr()) |
-               reinterpret_cast<uintptr_t>(gain.data_ptr())) % 16 == 0,
-              "streams and gains start at multiples of 16 bytes");
   Tensor h = at::empty({M, N}, x.options());
   Tensor ss = at::empty({N / 16, M <= 16 ? 16 : 32},
                         x.options().dtype(at::kFloat));

@@ -34,6 +34,8 @@ namespace {
 
 typedef short s16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+// streams and gains may start at any float
+typedef f32x4 f32x4_any __attribute__((aligned(4)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 b16x2 __attribute__((ext_vector_type(2)));
 
@@ -570,14 +572,14 @@ void rows_short_kernel(const uint16_t* __restrict__ x,
     static_assert(HR == 2 && MT <= 4, "");
 #pragma unroll
     for (int s = 0; s < S; ++s) {
-      had[s] = *reinterpret_cast<const f32x4*>(
+      had[s] = *reinterpret_cast<const f32x4_any*>(
           adds.streams + (int64_t(arow) * S + s) * N + acol);
       outw[s] = adds.out_w[s];
       inw[s] = adds.in_w[s];
 #pragma unroll
       for (int t = 0; t < S; ++t) mix[s][t] = adds.mix[s * S + t];
     }
-    gain = *reinterpret_cast<const f32x4*>(adds.gain + acol);
+    gain = *reinterpret_cast<const f32x4_any*>(adds.gain + acol);
   }
 #pragma unroll
   for (int s = 0; s < R - 1; ++s)
@@ -654,8 +656,8 @@ void rows_short_kernel(const uint16_t* __restrict__ x,
           u[r] += inw[t] * sum;
         }
         if (row < M)
-          *reinterpret_cast<f32x4*>(adds.streams +
-                                    (int64_t(row) * S + t) * N + c) = to;
+          *reinterpret_cast<f32x4_any*>(adds.streams +
+                                        (int64_t(row) * S + t) * N + c) = to;
       }
       float ss = 0.f;
 #pragma unroll

@@ -53,6 +53,20 @@ def test_shared_norm(M, N, K, nxt, S):
                                rtol=2 ** -10)
 
 
+def test_streams_and_gains_anywhere():
+    """They may start at any float, as those of a step by itself."""
+    args = [t.to(DEV) for t in operands(17, 256, 2048, 1024, 2)][:-1]
+    off = list(args)
+    for i in (2, 3, 4, 5, 6):
+        off[i] = torch.empty(args[i].numel() + 1, device=DEV)[1:] \
+            .view(args[i].shape).copy_(args[i])
+    want, got = (ops.rows_linear_streams_(*a) for a in (args, off))
+    # (sums of squares of rows that there are)
+    assert torch.equal(got[0], want[0])
+    assert torch.equal(got[1][:, :17], want[1][:, :17])
+    assert torch.equal(off[2], args[2])
+
+
 def test_what_does_not_fit():
     x, w, streams, mix, out_w, in_w, gain, w2 = (
         t.to(DEV) for t in operands(8, 256, 2048, 1024, 2))

@@ -38,10 +38,14 @@ class Portion:
 class PromptRows:
     def __init__(self, portions: list, device) -> None:
         self.portions = portions
-        self.device = device
+        self.device = torch.device(device)
         self._made: dict[tuple, object] = {}
 
     def _once(self, key: tuple, make):
+        """A table is there on the stream that it was sent on; another stream
+        gets one of its own."""
+        if self.device.type == "cuda":
+            key += (torch.cuda.current_stream(self.device).cuda_stream,)
         if key not in self._made:
             self._made[key] = make()
         return self._made[key]

@@ -112,3 +112,19 @@ def test_tables_behind_a_busy_stream(n):
     for i, made in enumerate(got):
         for g, want in zip(made, tables("cpu", i)):
             assert g.dtype == want.dtype and torch.equal(g.cpu(), want)
+
+
+def test_tables_on_another_stream():
+    """A table that a busy stream has not come to yet is none for others."""
+    portions = [Portion(0, i, 40 + i, 0, i) for i in range(9)]
+    rows, x = PromptRows(portions, "cuda"), torch.randn(4096, 4096,
+                                                        device="cuda")
+    torch.cuda.synchronize()
+    with torch.cuda.stream(torch.cuda.Stream()):
+        for _ in range(40):
+            x = torch.mm(x, x) * 1e-3
+        first = rows.tiles(16)
+    want = PromptRows(portions, "cpu").tiles(16)
+    assert torch.equal(rows.tiles(16).cpu(), want)
+    torch.cuda.synchronize()
+    assert torch.equal(first.cpu(), want)

@@ -146,8 +146,9 @@ void prefill(rlli::GlaArgs& a, const Tensor& proj, const Tensor& tiles,
   const int64_t nh = int64_t(a.n_tiles) * a.heads;
   auto fo = proj.options().dtype(at::kFloat);
   // f32, or three 16-bit parts, of which columns of queries go in 32
-  const int64_t size = a.f32 ? 4 : 6;
-  const int64_t q_cols = a.f32 ? a.dpad : (a.dpad + 31) / 32 * 32;
+  const bool parts = rlli::gla_parts(a);
+  const int64_t size = parts ? 6 : 4;
+  const int64_t q_cols = parts ? (a.dpad + 31) / 32 * 32 : a.dpad;
   auto bytes = proj.options().dtype(at::kByte);
   Tensor qd = at::empty({nh * C * q_cols * size}, bytes);
   Tensor kd = at::empty({nh * C * a.dpad * size}, bytes);

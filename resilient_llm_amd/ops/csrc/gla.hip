@@ -583,13 +583,7 @@ void prefill(const GlaArgs& a, hipStream_t st) {
     hipLaunchKernelGGL(k, dim3(a.n_tiles, a.heads), dim3(256), smem, st, a,
                        vec, vec_a);
   };
-  // The scan's operands in parts where the activations are 16-bit ones; they are
-  // half as many bytes more, which cost more than they gain where many short heads
-  // fill the chip (heads of 64 x 64, whole prompts, us, f32 and parts: 32 of them
-  // 103 and 76, 128 245 and 242, 256 269 and 230, but 512 214 and 234).
-  const int64_t sh = int64_t(a.n_seqs) * a.heads;
-  const bool parts = sizeof(T) == 2 &&
-                     (a.dpad > 64 || sh * ((a.vdim + 63) / 64) < 512);
+  const bool parts = gla_parts(a);
   auto by_parts = [&](auto md, auto full) {
     constexpr int MD = decltype(md)::value;
     constexpr bool FULL = decltype(full)::value;
@@ -675,6 +669,15 @@ void by_kind(const GlaArgs& a, F f) {
 }
 
 }  // namespace
+
+// The scan's operands in parts where the activations are 16-bit ones; they are
+// half as many bytes more, which cost more than they gain where many short heads
+// fill the chip (heads of 64 x 64, whole prompts, us, f32 and parts: 32 of them
+// 103 and 76, 128 245 and 242, 256 269 and 230, but 512 214 and 234).
+bool gla_parts(const GlaArgs& a) {
+  const int64_t sh = int64_t(a.n_seqs) * a.heads;
+  return !a.f32 && (a.dpad > 64 || sh * ((a.vdim + 63) / 64) < 512);
+}
 
 void launch_gla_decode(const GlaArgs& a, hipStream_t st) {
   if (a.rows == 0) return;

@@ -89,13 +89,13 @@ struct GlaArgs {
   const int32_t* positions;     // [rows] (decode)
   const int32_t* tiles;    // [4, n_tiles] chunks of kRecChunk rows
   const int32_t* seqs;     // [4, n_seqs]: first tile, tiles, pos0, slot
-  // scratch in tiles of 16 x 16, a lane l's four elements of row l % 16 from
-  // column l / 16 * 4 on next to each other, tiles of
-  // (or in pairs of tiles as three 16-bit parts, 1 KB a part, a lane's fours of
-  // both next to each other; queries' columns are an even number of tiles then)
-  void* qd;                // [n_tiles, heads, 64, dpad] down the columns,
+  // scratch, f32 in tiles of 16 x 16, a lane l's four elements of row l % 16 from
+  // column l / 16 * 4 on next to each other; or, of gla_parts, in pairs of tiles
+  // as three 16-bit parts, 1 KB a part, a lane's fours of both tiles next to each
+  // other (queries' columns are an even number of tiles then)
+  void* qd;                // [n_tiles, heads, 64, dpad], tiles down the columns
   void* kd;                // [n_tiles, heads, dpad, 64] and
-  void* sc;                // [n_tiles, heads, 64, 64] along the rows
+  void* sc;                // [n_tiles, heads, 64, 64], tiles along the rows
   float* dec;              // [n_tiles, heads, dpad]
   float* o;                // [rows + 64, heads * vdim]
   void* out;               // [rows, heads * vdim], rows out_stride apart
@@ -107,6 +107,7 @@ struct GlaArgs {
   int kind;                // GlaKind
   bool f32;
 };
+bool gla_parts(const GlaArgs& a);        // of a prompt's scratch
 void launch_gla_decode(const GlaArgs& a, hipStream_t stream);
 void launch_gla_prefill(const GlaArgs& a, hipStream_t stream);
 

@@ -190,3 +190,29 @@ def test_prompts_without_conditions(T, dim, rank):
     # the bounds of the longer runs over the same steps
     assert rel(got, want) < tol(BF16)
     assert rel(st[1], S) < 1e-5
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,seqs,dim,each", [
+    (BF16, 16, 64, 4), (BF16, 15, 64, 6), (BF16, 2, 128, 6), (F32, 2, 128, 4)])
+def test_scratch_of_prompts(dtype, seqs, dim, each):
+    """As many bytes as the scan's operands have: four a number where they are f32,
+    as of short heads that fill the chip, or three parts."""
+    H, vdim, T = 32, 64, 64
+    rows = PromptRows([Portion(i * T, 0, T, i, i) for i in range(seqs)], "cuda")
+    proj = torch.zeros(T * seqs, 2 * H * (dim + vdim) + 8, device="cuda",
+                       dtype=dtype)
+    a2 = torch.zeros(H * dim, 8, device="cuda", dtype=dtype)
+    st = torch.zeros(seqs, H, dim, vdim, device="cuda")
+    args = (proj, a2, torch.zeros(H * dim, device="cuda"),
+            torch.ones(vdim, device="cuda"), st, rows, vdim, 8.0, 1e-5)
+    ops.gla_prefill(*args)                # (makes the tables)
+    before = torch.cuda.memory_allocated()
+    torch.cuda.reset_peak_memory_stats()
+    out = ops.gla_prefill(*args)
+    took = torch.cuda.max_memory_allocated() - before
+    chunks = H * seqs
+    want = (chunks * (64 * dim * 2 + 64 * 64) * each + chunks * dim * 4
+            + (T * seqs + 64) * H * vdim * 4 + out.nbytes)
+    # (allocations are multiples of 512 bytes; larger ones may be split later)
+    assert took <= want + (1 << 20)

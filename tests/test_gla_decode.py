@@ -214,5 +214,6 @@ def test_scratch_of_prompts(dtype, seqs, dim, each):
     chunks = H * seqs
     want = (chunks * (64 * dim * 2 + 64 * 64) * each + chunks * dim * 4
             + (T * seqs + 64) * H * vdim * 4 + out.nbytes)
-    # (allocations are multiples of 512 bytes; larger ones may be split later)
-    assert took <= want + (1 << 20)
+    # (each of six allocations may have a block that is up to 1 MB larger; with six
+    # bytes for four the first case would take 12 MB more)
+    assert took <= want + (6 << 20)

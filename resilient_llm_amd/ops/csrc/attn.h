@@ -68,8 +68,10 @@ int diff_head_blocks(int group);     // workgroups per kv head, sequence, split
 void launch_window_rope_append(const WindowAttnArgs& a, hipStream_t stream);
 void launch_window_decode(const WindowAttnArgs& a, hipStream_t stream);
 void launch_window_combine(const WindowAttnArgs& a, hipStream_t st);
-// The same by units of 32 tokens on the matrix cores, where window_units_ok.
+// The same by units of 32 tokens on the matrix cores, where window_units_ok and, of
+// up to ``reach`` tokens a sequence, window_units_faster.
 bool window_units_ok(const WindowAttnArgs& a);
+bool window_units_faster(const WindowAttnArgs& a, int64_t reach);
 int window_units_splits(const WindowAttnArgs& a, int units);
 void launch_window_units(const WindowAttnArgs& a, hipStream_t st);
 void launch_window_rows(const WindowAttnArgs& a, bool decode,

@@ -135,10 +135,11 @@ Tensor window_decode(const Tensor& qkv, const Tensor& k_cache,
   const int hb = rlli::window_decode_heads_per_wg(group);
   const int64_t visible = int64_t(a.window) + a.keep_first + 32;
   Tensor pa, pm;
-  if (rlli::window_units_ok(a)) {
-    const int64_t reach = std::min<int64_t>(
-        int64_t(a.max_blocks) * a.block_size, visible + 32);
-    a.n_split = rlli::window_units_splits(a, int((reach + 31) / 32));
+  const int64_t room = int64_t(a.max_blocks) * a.block_size;
+  if (rlli::window_units_ok(a) &&
+      rlli::window_units_faster(a, std::min(room, visible))) {
+    a.n_split = rlli::window_units_splits(
+        a, int((std::min(room, visible + 32) + 31) / 32));
     decode_parts(a, qkv, pa, pm);
     rlli::launch_window_units(a, st);
     check_launch("window_decode");

@@ -1,5 +1,5 @@
 // Windowed decode attention on the matrix cores: keys and values as wide as each
-// other, up to four query heads of a key/value head, no distance bias.
+// other, four query heads of a key/value head, no distance bias.
 //
 // The work of a wave is decode_attn.h's: units of 32 tokens whose keys and
 // values are all asked for at once, 24 bits of every weight.  Units are those of
@@ -25,9 +25,9 @@ using decode::s16x8;
 
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr int NW = 12;            // waves of a workgroup
-constexpr int UNIT = decode::UNIT;
+constexpr int UNIT = decode::UNIT, GROUP = 4;
 
-template <int D, int GROUP, typename KC>
+template <int D, typename KC>
 __global__ __launch_bounds__(NW * 64, NW / 4)
 void window_units_kernel(WindowAttnArgs a) {
   using namespace decode;
@@ -175,9 +175,8 @@ void window_units_kernel(WindowAttnArgs a) {
   s16x8 qf[KSTEPS];
 #pragma unroll
   for (int k = 0; k < KSTEPS; ++k) {
-    uint4 w{0, 0, 0, 0};
-    if (col % HS < GROUP)
-      w = *reinterpret_cast<const uint4*>(qs + col * QROW + k_chan(k));
+    const uint4 w =
+        *reinterpret_cast<const uint4*>(qs + col * QROW + k_chan(k));
     qf[k] = __builtin_bit_cast(s16x8, w);
   }
 
@@ -348,10 +347,26 @@ void window_units_kernel(WindowAttnArgs a) {
 }  // namespace
 
 bool window_units_ok(const WindowAttnArgs& a) {
-  const int group = a.n_q / a.n_kv;
   return !a.f32 && a.dim == a.vdim && (a.dim == 64 || a.dim == 128) &&
-         (group == 1 || group == 2 || group == 4) && !a.r1 && !a.v_norm &&
-         a.rot % 2 == 0 && a.block_size % 16 == 0 && a.stride % 8 == 0;
+         a.n_q == GROUP * a.n_kv && !a.r1 && !a.v_norm && a.rot % 2 == 0 &&
+         a.block_size % 16 == 0 && a.stride % 8 == 0;
+}
+
+// Where it is the faster one whatever the sequences' lengths are, of which the host
+// knows the tables' room and the window (``reach``): no more pairs of a sequence and
+// a key/value head than CUs, or than those for which lane groups would go in parts as
+// well.  A workgroup is large; where more of them than that have short sequences in
+// wide tables, waves without work cost more than the others gain, and where one or
+// two heads share a read, far more.  (us, lane groups and so, tables of 4096 tokens,
+// window 1024: 16/4 heads of 128, 64 sequences of 20 tokens 13.7 and 7.0, 100 20.9 and
+// 11.7, 256 19.2 and 21.6; 16/8 heads, 64 of 20 7.9 and 11.5, of 300 19.0 and 22.4, of
+// 1000 51 and 45; 8/8 heads, 64 of 20 6.9 and 11.4, 8 of 300 11.9 and 13.5.)  512
+// pairs that may see much go so too, for what they gain on long sequences: 32/8 heads
+// of 128, 64 of 1000 60 and 46, of 20 10.7 and 11.5.
+bool window_units_faster(const WindowAttnArgs& a, int64_t reach) {
+  const int64_t pairs = int64_t(a.rows) * a.n_kv;
+  return pairs <= 256 || (pairs < 512 && reach >= 128) ||
+         (pairs == 512 && reach >= 512 && a.dim == 128);
 }
 
 // Parts of a sequence's ``units`` (as many as its window can have): rounds of
@@ -373,24 +388,17 @@ int window_units_splits(const WindowAttnArgs& a, int units) {
 
 void launch_window_units(const WindowAttnArgs& a, hipStream_t st) {
   if (a.rows == 0) return;
-  auto go = [&](auto d, auto g, auto kc) {
-    hipLaunchKernelGGL((window_units_kernel<decltype(d)::value,
-                                            decltype(g)::value, decltype(kc)>),
+  auto go = [&](auto d, auto kc) {
+    hipLaunchKernelGGL((window_units_kernel<decltype(d)::value, decltype(kc)>),
                        dim3(a.n_split, a.n_kv, a.rows), dim3(NW * 64), 0, st,
                        a);
   };
-  auto by_cache = [&](auto d, auto g) {
-    if (a.cache == kCacheFP8) go(d, g, CacheFP8{});
-    else go(d, g, CacheBF16{});
+  auto by_cache = [&](auto d) {
+    if (a.cache == kCacheFP8) go(d, CacheFP8{});
+    else go(d, CacheBF16{});
   };
-  auto by_group = [&](auto d) {
-    const int group = a.n_q / a.n_kv;
-    if (group == 4) by_cache(d, std::integral_constant<int, 4>{});
-    else if (group == 2) by_cache(d, std::integral_constant<int, 2>{});
-    else by_cache(d, std::integral_constant<int, 1>{});
-  };
-  if (a.dim == 128) by_group(std::integral_constant<int, 128>{});
-  else by_group(std::integral_constant<int, 64>{});
+  if (a.dim == 128) by_cache(std::integral_constant<int, 128>{});
+  else by_cache(std::integral_constant<int, 64>{});
   if (a.n_split > 1) launch_window_combine(a, st);
 }
 

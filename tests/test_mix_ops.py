@@ -284,6 +284,42 @@ def test_decode_units(H, G, dim, window, keep):
 
 
 @GPU
+@pytest.mark.parametrize("cache", [BF16, torch.float8_e4m3fn])
+@pytest.mark.parametrize("dim", [64, 128])
+@pytest.mark.parametrize("H,G", [(8, 2), (4, 2), (2, 2)])
+@pytest.mark.parametrize("copies", [1, 3, 9])
+def test_units_of_batches(H, G, dim, cache, copies):
+    """Sequences that end where units of 32 tokens, rounds of twelve and parts do,
+    in batches for which they or lane groups are the faster way; against attention
+    over what the cache holds."""
+    T, window, keep, n = 1345, 1000, 40, 85
+    a = Attn(T, H, G, dim, dim, 32, window, keep, "cuda:0", BF16,
+             cache_dtype=cache)
+    a.run(0, T)
+    pos = torch.tensor([0, 1, 31, 32, 63, 64, 383, 384, 767, 768, 999, 1000, 1063,
+                        1064, 1343, 1344] * copies, dtype=torch.int32)
+    B = len(pos)
+    kc, vc = (t[a.table[0].long()].repeat(B, 1, 1, 1) for t in (a.kc, a.vc))
+    table = torch.arange(B * n, dtype=torch.int32).view(B, n)
+    slots = table[torch.arange(B), pos.long() // 16] * 16 + pos % 16
+    got = ops.window_decode(
+        torch.cat([a.qkv(int(p), 1) for p in pos]), kc, vc, pos.cuda(), a.cs,
+        slots.cuda(), table.cuda(), a.sink.cuda(), a.scale, H, window, keep, True)
+    q = plain.rotate_interleaved(a.q.double(), torch.arange(T), 32, a.base)
+    k, v = (t.view(B, n, G, 16, dim).transpose(2, 3).flatten(1, 2).float().cpu()
+            .double() for t in (kc, vc))
+    at = torch.arange(T)
+    want = []
+    for b, p in enumerate(pos.tolist()):
+        seen = ((p - at < window) | (at < keep))[:p + 1]
+        keys, values = (t[b, :p + 1][seen].repeat_interleave(H // G, 1)
+                        for t in (k, v))
+        s = torch.cat([(keys * q[p]).sum(-1) * a.scale, a.sink.double()[None]])
+        want.append((torch.softmax(s, 0)[:-1, :, None] * values).sum(0).flatten())
+    assert rel(got, torch.stack(want)) < tol(BF16)
+
+
+@GPU
 @pytest.mark.parametrize("H,G,dim", [(8, 2, 128), (4, 2, 64), (2, 2, 128)])
 @pytest.mark.parametrize("window,keep", [(1000, 40), (33, 0)])
 def test_newest_value_infinite(H, G, dim, window, keep):

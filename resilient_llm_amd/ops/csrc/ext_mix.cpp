@@ -174,28 +174,33 @@ Tensor moe_run(rlli::MoeArgs& a, const Tensor& h, Tensor& ids, Tensor& w) {
               (a.gated ? 2 : 1) * int64_t(a.ffp) * a.width <
                   (int64_t(1) << 31),
               "too many rows or too wide an expert for one call");
-  // Weights are streamed for few rows of an expert; tiles beyond, whose height
-  // costs nothing while reading weights is what takes long, but for few blocks of
-  // more rows than a low tile has.  (us for all of it by 16, 128 and 256 rows, 32
-  // experts of 1024 by 2048, four each: 12 rows an expert 97, 112 and 112, 18 126,
-  // 113 and 113, 38 202, 117 and 116, 150 641, 192 and 134, 300 1229, 222 and 222;
-  // 16 of 3584 by 4096, two each: 8 rows 273, 265 and 266, 38 636, 269 and 269; 8
-  // of 2048 by 1024, two each: 8 rows 34, 44 and 43, 16 43, 44 and 44, 150 -, 62
-  // and 80, 300 -, 76 and 84, 400 -, 87 and 87.)
+  // Weights are streamed for few rows of an expert; tiles beyond.  (us for all of it
+  // by 16, 128 and 256 rows, 32 experts of 1024 by 2048, four each: 12 rows an expert
+  // 97, 112 and 112, 18 126, 113 and 113, 38 202, 117 and 116, 150 641, 192 and 134, 300
+  // 1229, 222 and 222; 16 of 3584 by 4096, two each: 8 rows 273, 265 and 266, 38 636,
+  // 269 and 269.)  Few blocks of w, for which tiles leave CUs idle, are streamed longer
+  // (4 experts of 512 by 1024, streamed and tiles: 16 rows 18 and 25, 47 22 and 25; of
+  // 2048 by 2048, 16 rows 41 and 43, 20 44 and 42; of 4096 by 4096, 8 rows 99 and 113)
+  // and have tiles of 128 rows, which routing that is not even leaves enough of (8 of
+  // 2048 by 1024, two each, 80 rows, 128 and 256: even 40 and 40, uneven 45 and 74).
   const int64_t each = P / a.routes;
   const int64_t blocks =
       a.experts * (((a.gated ? 2 : 1) * int64_t(a.ffp) + 255) / 256);
-  a.tile_m = (a.f32 || a.width % 64 != 0 || each < (a.width >= 4096 ? 8 : 16))
-                 ? 16
-             : blocks < 192 && each > 112 && each < 384 ? 128
-                                                        : 256;
-  // An expert's low tile right behind its full ones, so that its weights are
-  // still in the caches, where most experts have one.  (us, last and there, as
-  // above: 300 rows an expert 222 and 182, 375 214 and 186, 625 292 and 277, 875
-  // 375 and 357; but 250 168 and 189, 500 230 and 263, 750 319 and 351, 1024 408
-  // and 435, whose few low tiles fill the last round.)
-  a.together = a.tile_m == 256 && each >= 256 && each % 256 >= 24 &&
-               each % 256 <= 144;
+  const bool few = blocks < 192;
+  const int64_t least = blocks <= 32                 ? 48
+                        : blocks < 128               ? 20
+                        : !few && a.width >= 4096    ? 8
+                                                     : 16;
+  a.tile_m = (a.f32 || a.width % 64 != 0 || each < least) ? 16
+             : few && each < 384                          ? 128
+                                                          : 256;
+  // An expert's low tile right behind its full ones, so that its weights are still in
+  // the caches, where most experts have one that is clearly low, also if routing is
+  // not quite even.  (us, last and there, as above: 300 rows an expert 222 and 182,
+  // 375 214 and 186, 625 292 and 277, 875 375 and 357; but 250 168 and 189, 400 235 and
+  // 253, 540 158 and 175 for 16 experts, 640 310 and 339, 1024 408 and 435.)
+  a.together = a.tile_m == 256 && !few && each >= 256 && each % 256 >= 32 &&
+               each % 256 <= 120;
   a.max_tiles = int(P / a.tile_m + std::min<int64_t>(a.experts, P));
   auto io = h.options().dtype(at::kInt);
   ids = at::empty({a.rows, a.top}, io);

@@ -535,20 +535,26 @@ void moe_small_kernel(MoeArgs a) {
 // experts of 1024, four each: 397-407 -> 375-381 (on another card 404 -> 396).
 enum TileKind { FULL, LOW, NARROW };
 
+template <int MH>
 DEV_INLINE bool tile_of(const MoeArgs& a, int block, int n_blocks, int& tile,
                         int& nb, TileKind& kind) {
   const int x = block & 7;
   int s = block >> 3, n = a.counters[0], first = 0;
+  // of 128 rows, which are as high as low ones, all where CUs are left for them
+  const bool all = MH == 2 && (n + a.counters[1]) * n_blocks <= 128;
+  if (all) n_blocks *= 2;
   int per = (n * n_blocks + 7) / 8;
-  kind = FULL;
+  kind = all ? NARROW : FULL;
   if (s >= per) {
     s -= per;
     // CUs that the full tiles' last round leaves idle
     const int idle = 255 - (n * n_blocks + 255) % 256;
     first = n;
     n = a.counters[1];
-    kind = n * n_blocks > 2 * idle && n * n_blocks <= 128 ? NARROW : LOW;
-    if (kind == NARROW) n_blocks *= 2;
+    if (!all) {
+      kind = n * n_blocks > 2 * idle && n * n_blocks <= 128 ? NARROW : LOW;
+      if (kind == NARROW) n_blocks *= 2;
+    }
     per = (n * n_blocks + 7) / 8;
     if (s >= per) return false;
   }
@@ -641,12 +647,15 @@ DEV_INLINE void moe_tile(const MoeArgs& a, int rows, int e, int p0, int nb) {
 // 32 experts of 1024, four each, us for all of it: full ones only 345, half the
 // height 336, and half the width 326.  8192 rows, 116 full tiles and 12 others,
 // with half the width 434 and without 417: they run beside the last full ones.)
+// Of 128 rows, all are half as wide where that many blocks are no more than CUs (8
+// experts of 1024 by 2048, two each, 80 rows an expert 50 and 38; 4 of 512 by 1024 34
+// and 27).
 template <bool UP, int MH, int NH, bool GATED>
 __global__ __launch_bounds__(512, 2)
 void moe_tile_kernel(MoeArgs a, int n_blocks) {
   int tile, nb;
   TileKind kind;
-  if (!tile_of(a, blockIdx.x, n_blocks, tile, nb, kind)) return;
+  if (!tile_of<MH>(a, blockIdx.x, n_blocks, tile, nb, kind)) return;
   const int rows = a.tile_rows[tile];
   const int e = a.tile_expert[tile];
   const int p0 = a.tile_row0[tile];

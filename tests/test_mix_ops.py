@@ -518,6 +518,20 @@ def test_heights_of_tiles(T, E, top, ff):
 
 
 @GPU
+@pytest.mark.parametrize("T,E,top,ff,skew", [
+    # few blocks of w: rows an expert below and above the lines to tiles, of 128
+    # rows, all of them narrow or none, evenly and with one expert that has most
+    (191, 4, 1, 64, 0), (192, 4, 1, 64, 0), (192, 4, 1, 64, 9), (152, 16, 2, 250, 0),
+    (160, 16, 2, 250, 0), (320, 16, 2, 250, 9), (500, 8, 2, 1024, 0),
+    (1000, 8, 2, 1024, 9), (3000, 8, 1, 1024, 0),
+    # many: low tiles alone, behind full ones and last
+    (127, 64, 8, 384, 0), (128, 64, 8, 384, 0), (800, 64, 8, 384, 0),
+    (2400, 64, 8, 384, 0), (2400, 64, 8, 384, 9), (4000, 64, 8, 384, 0)])
+def test_tiles_by_blocks(T, E, top, ff, skew):
+    test_experts(T, 64, E, top, ff, skew, "cuda:0", BF16)
+
+
+@GPU
 @pytest.mark.parametrize("T,W,E", [
     # whole rounds of the router's loads, their rest, and neither; routes around
     # the lines between its kernels

@@ -209,7 +209,7 @@ enum Cut { WHOLE, SHARES, EITHER };      // EITHER: as a.shares says
 // Workgroup ``block``, of NW waves.  BS: block size of the cache where it is
 // known (0: any)
 template <int D, int GROUP, typename KC, int BS, bool FUSED, Cut CUT, int NW>
-DEV_INLINE void attend(const DecodeArgs& a, int block,
+DEV_INLINE void attend(const DecodeArgs& a, unsigned block,
                        Lds<D, GROUP, KC, NW>& lds) {
   using elem = typename KC::elem;
   using vec8 = typename KC::vec8;
@@ -596,7 +596,7 @@ DEV_INLINE void attend(const DecodeArgs& a, int block,
 // workgroup per (sequence, query head): D / 4 threads have a part's channels,
 // the others other parts.
 template <int D, int GROUP>
-DEV_INLINE void combine(const DecodeArgs& a, int block) {
+DEV_INLINE void combine(const DecodeArgs& a, unsigned block) {
   constexpr int TD = D / 4, NG = 256 / TD;
   const int n_q = a.n_kv * GROUP;
   const int seq = block / n_q, h = block % n_q;

@@ -711,7 +711,7 @@ Tensor mixed_attn_qkv(const Tensor& qkv, const Tensor& k_cache,
     return t.scalar_type() == at::kInt && t.is_contiguous() &&
            t.device() == qkv.device();
   };
-  rlli::MixedPlan plan{0, 0};
+  rlli::MixedPlan plan{0, 0, false};
   if (n_tiles > 0 && batch > 0 && n_q % n_kv == 0 && (D == 64 || D == 128) &&
       table(chunk_row0) && table(chunk_pos0) && table(chunk_nrows) &&
       table(chunk_btrow) && table(tables_pre) && table(tables_dec) &&
@@ -731,9 +731,9 @@ Tensor mixed_attn_qkv(const Tensor& qkv, const Tensor& k_cache,
     TORCH_CHECK(plan.splits > 0 && given.size() == 2 && given[0] >= 1 &&
                     given[0] <= 16 && given[1] >= 0 && given[1] <= 512,
                 "no such division for these sizes");
-    plan = {int(given[0]), int(given[1])};
+    plan = {int(given[0]), int(given[1]), true};
   }
-  if (plan.splits == 0) {
+  if (!plan.faster) {
     Tensor out = prefill_paged_attn(qkv, k_cache, v_cache, chunk_row0,
                                     chunk_pos0, chunk_nrows, chunk_btrow,
                                     tables_pre, scale, n_q);

@@ -124,9 +124,11 @@ void launch_prefill_paged(const uint16_t* qkv, const void* k_cache,
 
 // Prompt rows and decoding sequences of a mixed step at once (mixed_attn.hip).
 // What the tiles' keys are divided into and the sequences' shares; splits 0:
-// not for these sizes.  ``keys``, ``max_tokens``: what the tables have room for.
+// not for these sizes; faster: than one after the other.  ``keys``, ``max_tokens``:
+// what the tables have room for.
 struct MixedPlan {
   int splits, shares;
+  bool faster;
 };
 MixedPlan mixed_attn_plan(int n_tiles, int batch, int n_kv, int group,
                           int head_dim, int keys, int max_tokens, int elem,

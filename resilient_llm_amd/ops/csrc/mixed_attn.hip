@@ -66,28 +66,58 @@ void mixed_combine_kernel(Pages<KC> src, uint16_t* __restrict__ out,
 // 113; 16 of 4000 beside 128 behind 4000 79.9, 55 and 52; 37 with an 8-bit cache
 // beside 512 behind 1500 67.2, 49.3 and 47.9; 60 of 132 beside 52 behind 132, one
 // after the other still, 17.0.)
+//
+// And whether that is less than one after the other, with the rates that tell the
+// two apart at 2829 sizes: a step 2.6 (heads of 64 2.1, two workgroups a CU), 4.5
+// around a sequence.  Alone, tiles are divided by prefill_splits and take several
+// rounds where they are more than CUs; sequences have small workgroups that share a
+// CU, so that many short ones are little, and read at 3.1 TB/s with a launch for
+// their parts.  (64/8 heads of 128, 200 sequences of 16 tokens beside 512 rows 34
+// and here 45; 8/1, 2048 rows of an 8-bit cache, which two parts halve, 46 and 50.
+// Of those 2829, 1.17 times as fast in the mean, three below 0.95 by more than
+// two runs differ: 8 of 4000 beside 200 behind 4000, 64/8 heads, 88 and 100.)
 MixedPlan mixed_attn_plan(int n_tiles, int batch, int n_kv, int group,
                           int head_dim, int keys, int max_tokens, int elem,
                           int block_size) {
-  MixedPlan best{0, 0};
+  MixedPlan best{0, 0, false};
   if (n_tiles == 0 || batch == 0 || block_size != 16 ||
       (group != 4 && group != 8) || !two_waves(n_tiles, n_kv, group, keys))
     return best;
+  struct Rates {
+    float step, seq;
+    int places;                // workgroups that the chip holds
+  };
+  const Rates divide{2.1f, 5.f, 256};
+  const Rates decide =
+      head_dim == 128 ? Rates{2.6f, 4.5f, 256} : Rates{2.1f, 4.5f, 512};
   const int blocks = n_tiles * n_kv * (group / 4);
   const int steps = (keys + 2 * KT - 1) / (2 * KT);
-  const float reads =
-      1.2f * batch * max_tokens * n_kv * head_dim * elem / 5e6f;
+  const float bytes = float(batch) * max_tokens * n_kv * head_dim * elem;
   const float round = 1.2f + 2.f * head_dim * elem / 256;
   const bool never_cut = decode_attn_shares(batch, n_kv, max_tokens) == 0;
+  auto chain_of = [&](int n, const Rates& r) {
+    return (steps + n - 1) / n * r.step + (n > 1 ? 10.5f : 6.5f);
+  };
+  auto parts_of = [&](int n) {
+    const float of_one = 2.f * n_tiles * QR * n_kv * group * head_dim * 4;
+    return n > 1 ? 3.f + n * of_one / 5e6f : 0.f;
+  };
+  auto together = [&](int n, int shares, const Rates& r) {
+    const float chain = chain_of(n, r);
+    const float late = blocks * n >= r.places ? chain : 0.f;
+    const float all =
+        (blocks * n * chain + n_kv * (shares ? shares * 3.f : batch * r.seq)) /
+            r.places +
+        1.2f * bytes / 5e6f;
+    const float longest =
+        shares ? 0.f : late + 5.f + (max_tokens + 255) / 256 * round;
+    return std::max({chain, all, longest}) +
+           (n > 1 ? parts_of(n) : shares ? 3.f : 0.f);
+  };
   float least = 0.f;
   for (int n = 1; n <= std::max(1, std::min(16, 256 / blocks)); ++n) {
     if (n > 1 && (steps / n < 4 || (n_kv % 8 && n > 4 && n != 8 && n != 16)))
       continue;
-    const float chain = (steps + n - 1) / n * 2.1f + (n > 1 ? 10.5f : 6.5f);
-    const float together =
-        n > 1 ? 3.f + 2.f * n * n_tiles * QR * n_kv * group * head_dim * 4 / 5e6f
-              : 0.f;
-    const float late = blocks * n >= 256 ? chain : 0.f;
     for (const bool cut : {false, true}) {
       if (cut && never_cut) continue;
       const int left = 256 - blocks * n;
@@ -95,19 +125,24 @@ MixedPlan mixed_attn_plan(int n_tiles, int batch, int n_kv, int group,
       // its start.
       const int shares =
           cut ? std::max(1, 5 * (left >= 64 ? left : 256) / (4 * n_kv)) : 0;
-      const float all = (blocks * n * chain +
-                         n_kv * (cut ? shares * 3.f : batch * 5.f)) / 256 +
-                        reads;
-      const float longest =
-          cut ? 0.f : late + 5.f + (max_tokens + 255) / 256 * round;
-      const float us = std::max({chain, all, longest}) +
-                       (n > 1 ? together : cut ? 3.f : 0.f);
+      const float us = together(n, shares, divide);
       if (best.splits == 0 || us < least) {
-        best = MixedPlan{n, shares};
+        best = MixedPlan{n, shares, false};
         least = us;
       }
     }
   }
+  const int apart = prefill_splits(n_tiles, n_kv, group, keys);
+  const float tiles = (chain_of(apart, decide) + parts_of(apart)) *
+                      std::max(1.f, float(blocks * apart) / decide.places);
+  const float walk = never_cut ? (max_tokens + 127) / 128 * 1.2f : 0.f;
+  const float seqs = (never_cut ? 5.f : 9.f) +
+                     std::max({5.f + walk, 4.f + bytes / 3.1e6f,
+                               3.f + batch * n_kv * 0.65f / 256});
+  // (fewer parts of the tiles than they have alone have to be worth it)
+  best.faster = together(best.splits, best.shares, decide) *
+                    (apart > best.splits ? 1.09f : 0.97f) <=
+                tiles + seqs;
   return best;
 }
 

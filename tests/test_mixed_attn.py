@@ -79,6 +79,27 @@ def test_what_goes_apart():
         assert torch.equal(ops.mixed_attn_qkv(*gpu), want)
 
 
+@pytest.mark.parametrize("n_q,n_kv,D,lens,portions,apart", [
+    # many short sequences, tiles that have more parts alone; and not
+    (64, 8, 128, [16] * 200, [(0, 512)], True),
+    (8, 1, 128, [16] * 4, [(0, 2048)], True),
+    (32, 8, 128, [1500, 900, 1100], [(1500, 300)], False),
+    (32, 8, 64, [300] * 30, [(600, 64)], False)])
+def test_which_sizes_go_apart(n_q, n_kv, D, lens, portions, apart):
+    gpu = on_gpu(step(n_q, n_kv, D, lens, portions, n_kv == 1))
+    # (a step's tables of either kind have the pages of their longest)
+    gpu[8] = gpu[8][:, :-(-max(lens) // BS)].contiguous()
+    ops.load_extension(required=True)
+    torch.ops.rlli.mixed_attn_qkv(*gpu, [1, 0])      # sizes that it takes
+    torch.cuda.synchronize()
+    with torch.profiler.profile() as prof:
+        ops.mixed_attn_qkv(*gpu)
+        torch.cuda.synchronize()
+    names = [e.key for e in prof.key_averages()]
+    assert any("mixed_attn_kernel" in n for n in names) != apart
+    assert any("prefill_flash_kernel" in n for n in names) == apart
+
+
 def test_no_tokens():
     """Sequences without tokens come out as zero, cut or whole."""
     args = on_gpu(step(8, 2, 64, [0, 300, 0], [(400, 5)], False, room=40))

@@ -39,16 +39,20 @@ class PromptRows:
     def __init__(self, portions: list, device) -> None:
         self.portions = portions
         self.device = torch.device(device)
-        self._made: dict[tuple, object] = {}
+        self._made: dict[tuple, dict] = {}
 
     def _once(self, key: tuple, make):
         """A table is there on the stream that it was sent on; another stream
-        gets one of its own."""
-        if self.device.type == "cuda":
-            key += (torch.cuda.current_stream(self.device).cuda_stream,)
-        if key not in self._made:
-            self._made[key] = make()
-        return self._made[key]
+        gets one of its own, but a captured one what was sent before."""
+        made = self._made.setdefault(key, {})
+        stream = (torch.cuda.current_stream(self.device).cuda_stream
+                  if self.device.type == "cuda" else None)
+        if stream not in made:
+            if made and stream is not None \
+                    and torch.cuda.is_current_stream_capturing():
+                return next(iter(made.values()))
+            made[stream] = make()
+        return made[stream]
 
     def _table(self, rows: list) -> torch.Tensor:
         """Columns of ``rows`` as the rows of one int32 tensor."""

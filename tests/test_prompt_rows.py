@@ -128,3 +128,18 @@ def test_tables_on_another_stream():
     assert torch.equal(rows.tiles(16).cpu(), want)
     torch.cuda.synchronize()
     assert torch.equal(first.cpu(), want)
+
+
+def test_tables_in_a_capture():
+    """Tables that are there before a capture are taken as they are in it."""
+    rows = PromptRows([Portion(0, 0, 70, 0, 0)], "cuda")
+    want = rows.tiles(16), rows.seqs(64), rows.pos0()
+    graph, out = torch.cuda.CUDAGraph(), torch.zeros_like(want[0])
+    with torch.cuda.graph(graph):
+        got = rows.tiles(16), rows.seqs(64), rows.pos0()
+        out.copy_(got[0])
+    assert all(g is w for g, w in zip(got, want))
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        assert torch.equal(out, want[0])

@@ -589,8 +589,6 @@ void prefill(const GlaArgs& a, hipStream_t st) {
     constexpr bool FULL = decltype(full)::value;
     if constexpr (sizeof(T) == 4)
       intra(gla_intra_kernel<T, KIND, MD, FULL, false>);
-    else if constexpr (MD > 1)
-      intra(gla_intra_kernel<T, KIND, MD, FULL, true>);
     else if (parts)
       intra(gla_intra_kernel<T, KIND, MD, FULL, true>);
     else
@@ -670,13 +668,28 @@ void by_kind(const GlaArgs& a, F f) {
 
 }  // namespace
 
-// The scan's operands in parts where the activations are 16-bit ones; they are
-// half as many bytes more, which cost more than they gain where many short heads
-// fill the chip (heads of 64 x 64, whole prompts, us, f32 and parts: 32 of them
-// 103 and 76, 128 245 and 242, 256 269 and 230, but 512 214 and 234).
+// The scan's operands in parts where the activations are 16-bit ones: fewer steps
+// of each chunk's chain, and half as many bytes more, which cost more than they
+// give where the chip is full (`many` heads; up to 128 wide, of many rows as well)
+// or few blocks stream `much`. Whole prompts of plain decays, time in f32 over time in parts
+// (rows of a sequence, heads of all sequences times each):
+//   64 x 64     512 heads 0.92; 64, 8000 rows 0.87; 256, 64 rows 1.17
+//   128 x 64    64, 512 rows 1.00, 2048 rows 0.78; 128, 512 rows 0.99, 2048 0.93;
+//               256 1.05 to 1.38; 512, 16 rows 1.12, 256 rows 0.91
+//   128 x 128   16, 2048 rows 1.15, 8000 rows 0.82; 64, 8000 rows 1.01; 128, 2048
+//               1.10; 256, 256 rows 1.10, 1024 rows 0.88
+//   256 x 256   128 heads 1.05; 256 0.76 to 0.84, and 512 and more 0.72 to 0.81
+//   256 x 128   128 heads 1.17; 256 0.77 to 0.88
+//   256 x 64    64, 512 rows 1.03, 2048 rows 0.83; 256 heads 1.11; 512 0.80 to 0.86
 bool gla_parts(const GlaArgs& a) {
+  if (a.f32) return false;
   const int64_t sh = int64_t(a.n_seqs) * a.heads;
-  return !a.f32 && (a.dpad > 64 || sh * ((a.vdim + 63) / 64) < 512);
+  const int64_t blocks = sh * ((a.vdim + 63) / 64);
+  if (a.dpad <= 64 && blocks >= 512) return false;
+  const bool many = sh > 128 && blocks >= 512;
+  const bool much = int64_t(a.rows) * a.heads >= (sh < 512 ? 3 << 15 : 3 << 14);
+  if (a.dpad > 128) return !(many || (much && blocks <= 64));
+  return !(much && (many || blocks <= 128));
 }
 
 void launch_gla_decode(const GlaArgs& a, hipStream_t st) {

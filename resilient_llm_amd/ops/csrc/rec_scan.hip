@@ -664,24 +664,16 @@ void scan_md(const ScanArgs& a, hipStream_t st) {
   const bool full = (a.dim == 64 || a.dim == 128) && a.vdim % VS == 0 &&
                     (MODE == kScanPlain || vec_q) &&
                     (MODE == kScanDelta || vec_v);
-  // plain decays of 16-bit activations come here as short heads only (gla_parts)
-  constexpr bool SHORT = MODE == kScanPlain && sizeof(T) == 2;
-  if constexpr (SHORT) {
-    if (full) run(rec_scan_kernel<T, MODE, VT, 1, true>);
-    else run(rec_scan_kernel<T, MODE, VT, 1, false>);
-    return;
-  } else if constexpr (sizeof(T) == 2) {
+  if constexpr (sizeof(T) == 2) {
     if (full) {
       if (a.dim == 64) run(rec_scan_kernel<T, MODE, VT, 1, true>);
       else run(rec_scan_kernel<T, MODE, VT, 2, true>);
       return;
     }
   }
-  if constexpr (!SHORT) {
-    if (a.dpad <= 64) run(rec_scan_kernel<T, MODE, VT, 1, false>);
-    else if (a.dpad <= 128) run(rec_scan_kernel<T, MODE, VT, 2, false>);
-    else run(rec_scan_kernel<T, MODE, VT, 4, false>);
-  }
+  if (a.dpad <= 64) run(rec_scan_kernel<T, MODE, VT, 1, false>);
+  else if (a.dpad <= 128) run(rec_scan_kernel<T, MODE, VT, 2, false>);
+  else run(rec_scan_kernel<T, MODE, VT, 4, false>);
 }
 
 template <typename T, int MODE>

@@ -194,10 +194,11 @@ def test_prompts_without_conditions(T, dim, rank):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype,seqs,dim,each", [
-    (BF16, 16, 64, 4), (BF16, 15, 64, 6), (BF16, 2, 128, 6), (F32, 2, 128, 4)])
+    (BF16, 16, 64, 4), (BF16, 15, 64, 6), (BF16, 2, 128, 6), (F32, 2, 128, 4),
+    (BF16, 32, 128, 4), (BF16, 16, 256, 4), (BF16, 8, 256, 6)])
 def test_scratch_of_prompts(dtype, seqs, dim, each):
     """As many bytes as the scan's operands have: four a number where they are f32,
-    as of short heads that fill the chip, or three parts."""
+    as of heads that fill the chip, or three parts."""
     H, vdim, T = 32, 64, 64
     rows = PromptRows([Portion(i * T, 0, T, i, i) for i in range(seqs)], "cuda")
     proj = torch.zeros(T * seqs, 2 * H * (dim + vdim) + 8, device="cuda",
@@ -217,3 +218,47 @@ def test_scratch_of_prompts(dtype, seqs, dim, each):
     # (each of six allocations may have a block that is up to 1 MB larger; with six
     # bytes for four the first case would take 12 MB more)
     assert took <= want + (6 << 20)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["gla", "hgrn2", "rwkv"])
+@pytest.mark.parametrize("seqs,H,dim,vdim,T", [
+    # heads of more than 128: f32 operands where many fill the chip
+    (4, 64, 132, 72, 70), (2, 64, 132, 256, 66),
+    # of up to 128: from 48 Ki rows of all heads on where they fill it; 96 Ki
+    # elsewhere, also wide ones of few columns
+    (8, 64, 128, 40, 97), (8, 64, 100, 33, 95), (2, 16, 72, 20, 3100),
+    (1, 32, 132, 33, 3100)])
+def test_prompts_of_many_heads(seqs, H, dim, vdim, T, kind):
+    """Both sides of the lines where the scan's operands are f32 and not parts."""
+    rows = PromptRows([Portion(i * T, 0, T, i, i) for i in range(seqs)], "cuda")
+    cuda = lambda *ts: [t.cuda() for t in ts]
+    if kind == "rwkv":
+        vdim = dim
+        a = Rwkv(T, H, dim, 8, "cpu", BF16, seed=dim)
+        want, S = a.want()
+    elif kind == "gla":
+        *inputs, eps, want, S = gla_case(T, H, dim, vdim, 8, 8.0, 1.0,
+                                         dim + vdim, BF16)
+    else:
+        *inputs, eps, want, S = hgrn2_case(T, H, dim, vdim, 1.0, 0.8, dim, BF16)
+    st = torch.full((seqs + 1, H, dim, -(-vdim // 4) * 4), float("nan"),
+                    device="cuda")
+    if kind == "rwkv":
+        got = torch.full((seqs * T, H * dim), float("nan"), device="cuda",
+                         dtype=BF16)
+        ops.rwkv_prefill(
+            a.rkvg.repeat(1, seqs, 1).cuda(), a.low.repeat(seqs, 1).cuda(),
+            *cuda(a.w2, a.w0, a.u, a.norm), st, rows, a.eps, got)
+    else:
+        proj, *rest = cuda(*inputs)
+        proj = proj.repeat(seqs, 1)
+        got = ops.gla_prefill(proj, *rest, st, rows, vdim, 8.0, eps) \
+            if kind == "gla" else \
+            ops.hgrn2_prefill(proj, *rest, st, rows, vdim, eps)
+    # the bounds of the longer runs over the same steps
+    for i, of in enumerate(got.split(T)):
+        assert rel(of, want) < (8e-3 if kind == "rwkv" else tol(BF16))
+        assert rel(st[i, :, :, :vdim], S) < \
+            {"gla": 1e-5, "hgrn2": 3e-5, "rwkv": 2e-5}[kind]
+    assert torch.isnan(st[seqs]).all()

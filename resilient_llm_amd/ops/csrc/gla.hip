@@ -671,8 +671,8 @@ void by_kind(const GlaArgs& a, F f) {
 // The scan's operands in parts where the activations are 16-bit ones: fewer steps
 // of each chunk's chain, and half as many bytes more, which cost more than they
 // give where the chip is full (`many` heads; up to 128 wide, of many rows as well)
-// or few blocks stream `much`. Whole prompts of plain decays, time in f32 over time in parts
-// (rows of a sequence, heads of all sequences times each):
+// or few blocks stream `much`. Whole prompts, time in f32 over time in parts (heads
+// of all sequences and rows of each):
 //   64 x 64     512 heads 0.92; 64, 8000 rows 0.87; 256, 64 rows 1.17
 //   128 x 64    64, 512 rows 1.00, 2048 rows 0.78; 128, 512 rows 0.99, 2048 0.93;
 //               256 1.05 to 1.38; 512, 16 rows 1.12, 256 rows 0.91

@@ -87,7 +87,9 @@ struct CacheFP8 {
 };
 
 // A rotated pair (x1, x2); which product is rounded by itself is written out, so
-// that all who rotate have the same bits.
+// that the kernels of prompts, rope_kv.hip's and prefill_flash.h's rotate8, have the
+// same bits.  Those of decode leave it to the compiler: a key that they append may
+// differ from a prompt's in the last bit of the upper half before it is rounded.
 DEV_INLINE float rope_lower(float x1, float x2, float c, float s) {
   return fmaf(x1, c, -(x2 * s));
 }

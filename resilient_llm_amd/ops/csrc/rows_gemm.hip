@@ -884,13 +884,15 @@ bool rows_short_ok(int N, int K) {
 
 namespace {
 
-// Rows of w of one of its workgroups, in eights: as few as make no more workgroups
-// than CUs, whose rings leave no room for a second one.  The order of sums does
-// not depend on it.  (1, 16, 64 rows of x, us, 8, 16, 24 and 32 rows of w: 2048 x
-// 2048 3.9 4.1 4.3 4.7, 4.4 4.8 5.1 5.6, 7.0 7.1 7.9 8.4; 4096 x 2048 6.8 4.9 4.7
-// 5.1, 7.7 5.1 5.6 6.0, 12.6 7.7 8.5 8.9; 6144 x 2048 9.6 7.8 5.7 5.8, 11.0 8.6 6.0
-// 6.4, 18.2 13.2 9.0 9.5; 6160 x 2048 11.5 7.7 8.1 5.8, 13.1 8.6 8.5 6.4, 22.2 13.0
-// 13.7 9.5.)
+// Rows of w of one of its workgroups, in eights: as few as make no more
+// workgroups than CUs, whose rings leave no room for a second one.  The order of
+// sums follows it, as a workgroup begins its steps by its index: of one N it is
+// one order here, another in the products that share a norm, which take 16 rows
+// of w up to N of 4096.  (1, 16, 64 rows of x, us, 8, 16, 24 and 32 rows of w:
+// 2048 x 2048 3.9 4.1 4.3 4.7, 4.4 4.8 5.1 5.6, 7.0 7.1 7.9 8.4; 4096 x 2048 6.8
+// 4.9 4.7 5.1, 7.7 5.1 5.6 6.0, 12.6 7.7 8.5 8.9; 6144 x 2048 9.6 7.8 5.7 5.8,
+// 11.0 8.6 6.0 6.4, 18.2 13.2 9.0 9.5; 6160 x 2048 11.5 7.7 8.1 5.8, 13.1 8.6 8.5
+// 6.4, 22.2 13.0 13.7 9.5.)
 int short_eights(int N) { return std::clamp((N + 2047) / 2048, 1, 4); }
 
 }  // namespace

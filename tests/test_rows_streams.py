@@ -5,6 +5,7 @@ waves end."""
 import pytest
 import torch
 
+from nesizen_util import EVEN, check, expected, for_dtype, make_engine, tokens_of
 from resilient_llm_amd import ops
 
 pytestmark = pytest.mark.gpu
@@ -29,8 +30,7 @@ def operands(M, N, K, nxt, S):
 def test_shared_norm(M, N, K, nxt, S):
     x, w, streams, mix, out_w, in_w, gain, w2 = operands(M, N, K, nxt, S)
     dev = [t.to(DEV) for t in (x, w, streams, mix, out_w, in_w, gain)]
-    assert ops.rows_streams_fit(dev[0], dev[1], dev[2], w2.to(DEV)) \
-        or N * K < 1 << 20        # small ones are the library's
+    assert ops.rows_streams_fit(dev[0], dev[1], dev[2], w2.to(DEV))
     y = x.double() @ w.double().T
     want = torch.einsum("st,msn->mtn", mix.double(), streams.double()) \
         + out_w.double()[:, None] * y[:, None]
@@ -86,3 +86,22 @@ def test_what_does_not_fit():
     for bad in (ss[:-1], ss.double(), ss[:, :8]):
         with pytest.raises(RuntimeError):
             ops.rows_linear_scaled_relu2(h, bad, 1e-5, w2)
+
+
+def test_model_takes_it(monkeypatch):
+    """Of 32 rows the layers with a dense feed-forward share its norm, of 33 none."""
+    config = for_dtype(EVEN, BF16)
+    dense = sum(x["mlp"] is not None for x in config["layers"])
+    engine, w = make_engine(config, DEV, BF16)
+    rows, fused = [], ops.rows_linear_streams_
+
+    def counted(x, *rest):
+        rows.append(x.shape[0])
+        return fused(x, *rest)
+    monkeypatch.setattr(ops, "rows_linear_streams_", counted)
+    for n, calls in ((1, dense), (32, dense), (33, 0)):
+        rows.clear()
+        t = tokens_of(config, n, n)
+        got = engine.feed([(f"{n}", t, range(n))], [f"{n}"])
+        assert rows == [n] * calls
+        check(got, expected(config, w, t), BF16, f"{n} rows")

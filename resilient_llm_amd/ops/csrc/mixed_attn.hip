@@ -59,13 +59,14 @@ void mixed_combine_kernel(Pages<KC> src, uint16_t* __restrict__ out,
 // 256 tokens, 3.2 and 5 around them, 3 around a part; the tables' room, more
 // than half full, at 5 TB/s; another launch 3.  Workgroups of sequences start
 // with those of tiles or, where these fill the chip, behind them.  (One after
-// the other, so, and the best of 35 divisions, 32/8 heads of 128, 24 sequences of
-// 750 to 1500 tokens unless said otherwise: 512 rows behind 1500 67.3, 46.7 and
-// 45.8; 64 behind 1500 56.4, 36.8 and 32.9; 256 behind 700 53.9, 28.6 and 28.6;
-// 1500 behind 1500 125, 95 and 93; 8 of 7000 beside 512 behind 7000 137, 124 and
-// 113; 16 of 4000 beside 128 behind 4000 79.9, 55 and 52; 37 with an 8-bit cache
-// beside 512 behind 1500 67.2, 49.3 and 47.9; 60 of 132 beside 52 behind 132, one
-// after the other still, 17.0.)
+// the other, so, and the best of 35 divisions, kernels by themselves, 32/8
+// heads of 128, 24 sequences of 750 to 1500 tokens unless said otherwise: 512
+// rows behind 1500 67.3, 46.7 (in the step 52) and 45.8; 64 behind 1500 56.4,
+// 36.8 and 32.9; 256 behind 700 53.9, 28.6 and 28.6; 1500 behind 1500 125, 95
+// and 93; 8 of 7000 beside 512 behind 7000 137, 124 and 113; 16 of 4000 beside
+// 128 behind 4000 79.9, 55 and 52; 37 with an 8-bit cache beside 512 behind
+// 1500 67.2, 49.3 and 47.9; 60 of 132 beside 52 behind 132, one after the other
+// still, 17.0.)
 //
 // And whether that is less than one after the other, with the rates that tell the
 // two apart at 2829 sizes: a step 2.6 (heads of 64 2.1, two workgroups a CU), 4.5

@@ -370,18 +370,19 @@ void rec_scan_kernel(ScanArgs a, bool vec_q, bool vec_v) {
 // kScanPlain in parts, of 16-bit activations.  The values are 16-bit numbers;
 // queries, keys, A and the state are 32-bit ones, each of three 16-bit parts that
 // add up to it, so that products run on the 16-bit matrix cores: three for each of
-// the values', six for queries and state (what is left out is 2^-24 of a product).
-// Four waves carry the state from chunk to chunk (w every fourth of its key tiles),
-// four others have the outputs (w the rows of a sub-chunk) of the chunk that the
-// state is carried over, from its parts in LDS.  There are two copies by turns, and
-// of the values, so that a chunk takes one barrier.  What bounds it is a chunk's
-// chain of latencies, 2.4 us (asked for a chunk ahead of their turn, operands take
-// 3 us of 80 off and twice the registers).  4 sequences of 1.9k, 8 heads of 128 x
-// 256: 133 us with f32 products, of which these 67, and 80 now; the kernel that
-// makes the operands 49 and 50 (with infinite numbers' parts NaN, 3 us less each).
-// Against 64 bits, 2048 tokens, the state is off by 4.3e-7 and 2.6e-7, as it is
-// rounded less often; 6e-4 and 4e-4 of the outputs are not the nearest 16-bit
-// number.
+// the values', six for queries and state.  The three that are left out are up to
+// 2^-21 of a product, 2^-24 in the mean, always towards zero.  Four waves carry the
+// state from chunk to chunk (w every fourth of its key tiles), four others have the
+// outputs (w the rows of a sub-chunk) of the chunk that the state is carried over,
+// from its parts in LDS.  LDS has two copies of parts and values, written by turns,
+// so that a chunk takes one barrier.  What bounds it is a chunk's chain of
+// latencies, 2.4 us (asked for a chunk ahead of their turn, operands take 3 us of
+// 80 off and twice the registers).  4 sequences of 1.9k, 8 heads of 128 x 256: 133
+// us with f32 products, of which these 67, and 80 now, by itself (in a step's call
+// 110); the kernel that makes the operands 49 and 50 (with infinite numbers' parts
+// NaN, 3 us less each).  Against 64 bits, 2048 tokens, the state is off by 4.3e-7
+// and 2.6e-7, as it is rounded less often; 6e-4 and 4e-4 of the outputs are not the
+// nearest 16-bit number.
 template <int VT, int MD, bool FULL>
 __global__ __launch_bounds__(512, 2)
 void rec_scan_parts_kernel(ScanArgs a, bool vec_v) {

@@ -28,6 +28,7 @@ import torch.nn.functional as F
 
 from .. import ops
 from ..ops import autotune as lt_autotune
+from .mixed import narrow_to
 
 # Opt-in (A/B lever): ops.linear_auto for all products, that is the kernel for
 # few rows where the library would be the faster one too, and without silu,
@@ -390,8 +391,9 @@ class LlamaForCausalLM:
 
     def _layer(self, i: int, x: torch.Tensor, residual: Optional[torch.Tensor],
                positions: torch.Tensor, kv_cache, slot_mapping: torch.Tensor,
-               attn_fn, qkv_parts: bool,
-               attn_out_fn=None) -> tuple[torch.Tensor, torch.Tensor]:
+               attn_fn, qkv_parts: bool, attn_out_fn=None,
+               rows=None) -> tuple[torch.Tensor, torch.Tensor]:
+        """``rows``: those whose output is asked for (None: all)."""
         p = self.params
         c = self.config
         # what the next norm adds to the residual may come in parts, if
@@ -413,6 +415,8 @@ class LlamaForCausalLM:
             h = attn_out_fn(i, qkv, k_cache, v_cache)
         else:
             attn_out = attn_fn(i, qkv, k_cache, v_cache)   # [T, q_size]
+            if rows is not None:
+                attn_out, residual = attn_out[rows], residual[rows]
             h = self._all_reduce(out(attn_out, p[f"l{i}.o"]))
         if self.quant == "fp8":
             h2q, h2s = ops.rmsnorm_residual_fp8(h, residual, p[f"l{i}.ln2"],
@@ -545,13 +549,18 @@ class LlamaForCausalLM:
             ids = ids.long()
         x = F.embedding(ids, p["embed"])
         residual = None
+        last = self.config.n_layers - 1
+        narrow = layer is None and narrow_to(last_idx, ids.shape[0])
         for i in range(self.config.n_layers):
             if layer is not None and i > 0:
                 x, residual = layer(i, x, residual)
                 continue
             x, residual = self._layer(i, x, residual, positions, kv_cache,
                                       slot_mapping, attn_fn, qkv_parts,
-                                      attn_out_fn)
+                                      attn_out_fn, last_idx if narrow
+                                      and i == last else None)
+        if narrow:
+            last_idx = None
         if self.quant == "fp8":
             h8, hs = ops.rmsnorm_residual_fp8(x, residual, p["final_ln"],
                                               self.config.rms_eps)

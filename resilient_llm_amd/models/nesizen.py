@@ -29,7 +29,9 @@ from ..engine.kv_cache import KVLayer, StateLayer
 from .llama import (
     _USE_SKINNY, _linear, _linear_parts, _linear_relu2, lt_autotune,
 )
-from .mixed import DenseSpec, LayerSpec, MixedConfig, MixedModel
+from .mixed import (
+    DenseSpec, LayerSpec, MixedConfig, MixedModel, narrow_to,
+)
 
 
 @dataclasses.dataclass(frozen=True)
@@ -394,6 +396,8 @@ class NesizenForCausalLM(MixedModel):
             mix, out = P[f"{p}hc{q}.mix"], P[f"{p}hc{q}.out"]
             if q == 1:
                 y = mixer(i, _linear(h, P[p + "proj"]))
+                if i == c.n_layers - 1 and narrow_to(sample_idx, len(y)):
+                    x, y, sample_idx = x[sample_idx], y[sample_idx], None
                 if (isinstance(c.layers[i].mlp, DenseSpec)
                         and self.tp_world == 1 and not _USE_SKINNY
                         and not lt_autotune.enabled()

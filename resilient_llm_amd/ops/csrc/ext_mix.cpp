@@ -175,22 +175,24 @@ Tensor moe_run(rlli::MoeArgs& a, const Tensor& h, Tensor& ids, Tensor& w) {
                   (int64_t(1) << 31),
               "too many rows or too wide an expert for one call");
   // Weights are streamed for few rows of an expert; tiles beyond.  (us for all of it
-  // by 16, 128 and 256 rows, 32 experts of 1024 by 2048, four each: 12 rows an expert
-  // 97, 112 and 112, 18 126, 113 and 113, 38 202, 117 and 116, 150 641, 192 and 134, 300
-  // 1229, 222 and 222; 16 of 3584 by 4096, two each: 8 rows 273, 265 and 266, 38 636,
-  // 269 and 269.)  Few blocks of w, for which tiles leave CUs idle, are streamed longer
-  // (4 experts of 512 by 1024, streamed and tiles: 16 rows 18 and 25, 47 22 and 25; of
-  // 2048 by 2048, 16 rows 41 and 43, 20 44 and 42; of 4096 by 4096, 8 rows 99 and 113)
+  // by 16 rows and by tiles, 32 experts of 1024 by 2048, four each: 8 rows an expert
+  // 91 and 95, 10 93 and 94, 12 99 and 94, 16 118 and 94, 150 641 and 134; 16 of 3584
+  // by 4096, two each: 1 row 178 and 180, 2 247 and 239, 8 273 and 259; 8 of 2048 by
+  // 2048, two each: 12 rows 58 and 63, 16 71 and 63.)  Few blocks of w, for which
+  // tiles leave CUs idle, are streamed longer (4 experts of 512 by 1024: 16 rows 18
+  // and 25, 47 22 and 25; of 2048 by 2048, 20 rows 47 and 52, 32 58 and 53; 8 of 1024
+  // by 2048, 16 rows 42 and 45, 20 47 and 45; 4 of 4096 by 4096, 8 rows 99 and 113)
   // and have tiles of 128 rows, which routing that is not even leaves enough of (8 of
   // 2048 by 1024, two each, 80 rows, 128 and 256: even 40 and 40, uneven 45 and 74).
   const int64_t each = P / a.routes;
   const int64_t blocks =
       a.experts * (((a.gated ? 2 : 1) * int64_t(a.ffp) + 255) / 256);
   const bool few = blocks < 192;
-  const int64_t least = blocks <= 32                 ? 48
-                        : blocks < 128               ? 20
-                        : !few && a.width >= 4096    ? 8
-                                                     : 16;
+  const int64_t least = blocks <= 32      ? 48
+                        : blocks < 128    ? 20
+                        : few             ? 14
+                        : a.width >= 4096 ? 2
+                                          : 11;
   a.tile_m = (a.f32 || a.width % 64 != 0 || each < least) ? 16
              : few && each < 384                          ? 128
                                                           : 256;
@@ -201,6 +203,8 @@ Tensor moe_run(rlli::MoeArgs& a, const Tensor& h, Tensor& ids, Tensor& w) {
   // 253, 540 158 and 175 for 16 experts, 640 310 and 339, 1024 408 and 435.)
   a.together = a.tile_m == 256 && !few && each >= 256 && each % 256 >= 32 &&
                each % 256 <= 120;
+  // (beyond, an expert's weights are read by more than one row of tiles)
+  a.spread = each <= 256;
   a.max_tiles = int(P / a.tile_m + std::min<int64_t>(a.experts, P));
   auto io = h.options().dtype(at::kInt);
   ids = at::empty({a.rows, a.top}, io);

@@ -66,6 +66,7 @@ struct MoeArgs {
                            // squared, weight on the output
   float limit;
   bool together;           // an expert's tiles follow each other
+  bool spread;             // tiles begin K at steps of their own
   bool f32;
 };
 void launch_moe_route(const MoeArgs& a, hipStream_t stream);

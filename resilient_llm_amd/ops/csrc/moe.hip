@@ -578,6 +578,7 @@ DEV_INLINE void moe_tile(const MoeArgs& a, int rows, int e, int p0, int nb) {
   constexpr bool PAIRS = UP && GATED;
   constexpr int CHANNELS = PAIRS ? TN / 2 : TN;
   const int n0 = nb * CHANNELS, n1 = UP ? a.ffp : a.width;
+  const int panels = (n1 + CHANNELS - 1) / CHANNELS, nk = K / tile::KS;
 
   // the rows' pairs and weights, for the gather and the epilogue
   __shared__ int s_pair[TM];
@@ -589,6 +590,14 @@ DEV_INLINE void moe_tile(const MoeArgs& a, int rows, int e, int p0, int nb) {
   }
   __syncthreads();
 
+  // Where reading weights is what takes the time, column blocks start K at steps
+  // of their own, so that what is asked for at a time is spread over the memory
+  // channels (see rows_gemm.hip; the same block of an expert's other tiles starts
+  // where this one does and meets it in L2).  Of shorter rows it is slower.  (us
+  // without and with, for all of it: 32 experts of 1024 by 2048, four each, 400
+  // rows 116 and 97, 1000 127 and 113, 2000 167 and 154; 16 of 3584 by 4096, two
+  // each, 400 rows 287 and 270, 2000 468 and 440; but 64 of 1024 by 1024 102 and
+  // 108; more than a tile an expert, 32 of 1024 by 2048, 6001 rows 320 and 324.)
   P p;
   p.rows(
       [&](int r) {
@@ -603,7 +612,7 @@ DEV_INLINE void moe_tile(const MoeArgs& a, int rows, int e, int p0, int nb) {
   p.run(static_cast<const char*>(UP ? a.h : a.act),
         static_cast<const char*>(UP ? a.w_up : a.w_down) +
             int64_t(e) * N * K * 2,
-        K / tile::KS, lds);
+        nk, a.spread && nk >= 32 ? (e * panels + nb) % nk : 0, lds);
 
 #pragma unroll
   for (int i = 0; i < MH; ++i) {

@@ -62,7 +62,8 @@ void tile_gemm_kernel(const uint16_t* __restrict__ x,
         return uint32_t(h * half + min(at, half - 1)) * K * 2;
       });
   p.run(reinterpret_cast<const char*>(x + int64_t(s0) * tile::KS),
-        reinterpret_cast<const char*>(w + int64_t(s0) * tile::KS), nk, lds);
+        reinterpret_cast<const char*>(w + int64_t(s0) * tile::KS), nk, 0,
+        lds);
 
   if constexpr (OUT == OUT_PARTS) {
     float* y = static_cast<float*>(out) + int64_t(split) * M * N;

@@ -118,30 +118,38 @@ struct Product {
     return j * 8 + (MH == 3 && j ? wave() & 3 : wave());
   }
 
-  // nk steps of K from x and w on, nk > 0
-  DEV_INLINE void run(const char* xb, const char* wb, int nk, uint16_t* lds) {
+  // nk steps of K from x and w on, nk > 0, the first of them ``rot`` < nk
+  DEV_INLINE void run(const char* xb, const char* wb, int nk, int rot,
+                      uint16_t* lds) {
     const int lane = threadIdx.x & 63;
     const int wv = wave(), group = wv >> 2, wn = wv & 3;
+    // Where the next step's rows and those of the one after that begin; behind
+    // the last step, the last is asked for again: nobody reads it.
+    const uint32_t end = uint32_t(nk) * (KS * 2);
+    const uint32_t last = (rot ? uint32_t(rot) * (KS * 2) : end) - KS * 2;
+    uint32_t k1 = uint32_t(rot) * (KS * 2), k2 = k1;
+    auto advance = [&] {
+      k1 = k2;
+      if (k2 != last) k2 = k2 + KS * 2 == end ? 0 : k2 + KS * 2;
+    };
     // (offsets stay 32 bits wide beside a scalar address: kept as 64, they are
     // ten registers more, which the largest tile does not have)
-    auto ask_x = [&](int s, int h) {
+    auto ask_x = [&](int s, uint32_t k, int h) {
       uint16_t* to = lds + (s & 1) * STEP + h * TM / 2 * KS;
 #pragma unroll
       for (int j = 0; j < AL; ++j) {
         if (MH == 3 && j && h != group) continue;
         const int q = x_load(j);
         asm volatile("" : "+v"(ao[h][j]));
-        lds_load16(xb + int64_t(min(s, nk - 1)) * (KS * 2) + ao[h][j],
-                   to + q * 8 * KS);
+        lds_load16(xb + k + ao[h][j], to + q * 8 * KS);
       }
     };
-    auto ask_w = [&](int s, int h) {
+    auto ask_w = [&](int s, uint32_t k, int h) {
       uint16_t* to = lds + (s & 1) * STEP + (TM + h * TN / 2) * KS;
 #pragma unroll
       for (int j = 0; j < NH; ++j) {
         asm volatile("" : "+v"(bo[h][j]));
-        lds_load16(wb + int64_t(min(s, nk - 1)) * (KS * 2) + bo[h][j],
-                   to + (j * 8 + wv) * 8 * KS);
+        lds_load16(wb + k + bo[h][j], to + (j * 8 + wv) * 8 * KS);
       }
     };
     // All of this wave's loads but the newest have landed: X0 and X1 first and
@@ -213,38 +221,40 @@ struct Product {
     // A step.  The halves of w take turns in being the first (F), which was
     // read in the step before, so that a phase reads one half and needs no
     // registers beyond.  (The largest tile has none for two forms of the step:
-    // its first phase reads two halves.)  Behind the last step, the last is
-    // asked for again: nobody reads it.
+    // its first phase reads two halves.)
     constexpr bool TURNS = MH + NH < 6;
     auto step = [&](int s, auto first) {
       constexpr int F = decltype(first)::value;
       read_x(s, 0);
       if constexpr (!TURNS) read_w(s, F);
-      ask_x(s + 1, 1);
+      ask_x(s + 1, k1, 1);
       wait_but(I1{}, I2{}, I2{});
       multiply(0, F);
       read_w(s, 1 - F);
-      if constexpr (TURNS) ask_w(s + 2, F);
+      if constexpr (TURNS) ask_w(s + 2, k2, F);
       wait_but(I1{}, I1{}, std::integral_constant<int, TURNS ? 3 : 2>{});
       multiply(0, 1 - F);
       read_x(s, 1);
-      ask_x(s + 2, 0);
+      ask_x(s + 2, k2, 0);
       if constexpr (TURNS) wait_but(I2{}, I1{}, I2{});
-      else ask_w(s + 2, F);
+      else ask_w(s + 2, k2, F);
       multiply(1, 1 - F);
       if constexpr (TURNS) read_w(s + 1, 1 - F);
-      ask_w(s + 2, 1 - F);
+      ask_w(s + 2, k2, 1 - F);
       wait_but(I1{}, I1{}, I3{});
+      advance();
       multiply(1, F);
     };
 
-    ask_w(0, 0);
-    ask_x(0, 0);
-    ask_w(0, 1);
-    ask_x(0, 1);
-    ask_w(1, TURNS);
-    ask_x(1, 0);
-    ask_w(1, !TURNS);
+    ask_w(0, k1, 0);
+    ask_x(0, k1, 0);
+    ask_w(0, k1, 1);
+    ask_x(0, k1, 1);
+    advance();
+    ask_w(1, k2, TURNS);
+    ask_x(1, k2, 0);
+    ask_w(1, k2, !TURNS);
+    advance();
     wait_but(I1{}, I1{}, I3{});
     section();
     if constexpr (TURNS) read_w(0, 0);

@@ -21,7 +21,9 @@ COUNTS = [
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("W,ff", [(320, 192), (64, 1152)])
+# (from 2048 on, up to 256 rows an expert, blocks of w start K at their own steps)
+@pytest.mark.parametrize("W,ff", [(320, 192), (64, 1152), (2112, 192),
+                                  (64, 2112)])
 @pytest.mark.parametrize("counts", COUNTS, ids=str)
 def test_tiles_of_all_fills(counts, W, ff):
     E, limit = len(counts), 0.8

@@ -53,7 +53,7 @@ def _linear(x, w):
         return ops.tile_linear(x, w)
     if ops.rows_fit(x, w):
         return ops.rows_linear(x, w)
-    return F.linear(x, w)
+    return ops.library_linear(x, w)
 
 
 def _linear_silu(x, w):

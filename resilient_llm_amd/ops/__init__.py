@@ -599,6 +599,13 @@ def _tile_linear_faster(M: int, N: int, K: int) -> bool:
     rows 12 and 14.  Slower by more than 5 % of 541 points timed: 8192 x 8192,
     65 to 96 rows 38 and 41, 8192 x 4096, 129 and 144 rows 27 and 29, and 6144 x
     5120, 208 and 240 rows 33 and 37, all beside rows where they gain more.)"""
+    if K <= 2048 and N % 128 != 0:
+        # The library is slow where rows of the result end amid its tiles (as
+        # times as fast: 6160 x 2048, 1024 rows 1.20, 2048 1.20, 4000 1.05, 777
+        # 0.91, 7613 0.96; 3088 x 2048, 1024 1.20, 1300 0.89, 2048 1.19, 5000
+        # 1.13; 8208 x 2048, 1300 1.22, 3300 1.43; 6160 x 1024, 420 1.14, 1300
+        # 1.23, 5000 1.11; 2064 x 1024, 512 0.93, 1024 1.15, 5000 1.29).
+        return (1024 if K > 1024 else 600) <= M <= 6400 and 2048 <= N <= 10496
     return (64 < M <= (256 if K > 4096 else 160) and K >= 4096
             and 4096 <= N <= 10240 and (M > 128 or N * K > 1 << 24))
 
@@ -704,6 +711,19 @@ def tile_linear_relu2(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """relu2(x w^T), of the 16-bit product."""
     _gpu()
     return torch.ops.rlli.tile_linear_relu2(x, w)
+
+
+def library_linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """F.linear(x, w), on the GPU in 16 bits without the library's search for
+    its kernel at every call."""
+    if (x.is_cuda and x.dim() == w.dim() == 2
+            and x.dtype == w.dtype == torch.bfloat16
+            and x.device == w.device and x.shape[1] == w.shape[1]
+            and x.is_contiguous() and w.is_contiguous()
+            and not (x.requires_grad or w.requires_grad)):
+        _gpu()
+        return torch.ops.rlli.library_linear(x, w)
+    return torch.nn.functional.linear(x, w)
 
 
 def skinny_linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:

@@ -83,8 +83,8 @@ LIBRARIES = {
 _ACT = ["common.h", "act.h", "ext_common.h"]
 _ATTN = _ACT + ["attn.h", "attn_rows.h", "ext_window.h"]
 HEADERS = {"rlli_hip": ["common.h", "decode_attn.h", "decode_parts.h",
-                        "kernels.h", "prefill_flash.h", "prefill_parts.h",
-                        "tile_product.h"],
+                        "ext_common.h", "kernels.h", "prefill_flash.h",
+                        "prefill_parts.h", "tile_product.h"],
            "rlli_attn": _ATTN + ["decode_attn.h", "decode_parts.h"],
            "rlli_mix": _ATTN + ["mix.h", "prefill_flash.h", "prefill_parts.h",
                                 "tile_product.h"],

@@ -22,8 +22,19 @@
 #include <ATen/ATen.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
+#include <ATen/hip/HIPContextLight.h>
+#include <ATen/hip/tunable/Tunable.h>
 #include <hipblaslt/hipblaslt-ext.hpp>
+#include <hipblaslt/hipblaslt.h>
 
+#include "ext_common.h"
+#include "kernels.h"
+
+#include <algorithm>
+#include <array>
+#include <map>
+#include <memory>
+#include <mutex>
 #include <vector>
 
 namespace {
@@ -127,12 +138,124 @@ Tensor lt_heuristics(const Tensor& x, const Tensor& w, int64_t max_n) {
   return at::tensor(out, at::TensorOptions().dtype(at::kLong));
 }
 
+// ---- the library's own choice, without looking for it at every call ------
+// at::linear asks the library for its pick at each call: 18 us of the host,
+// of which 8 are spared by keeping what was found for a shape (a prompt of 165
+// rows through 16 layers of 2048 has 31 such products).
+struct LibraryPlan {
+  hipblasLtMatmulDesc_t product = nullptr;
+  hipblasLtMatrixLayout_t w = nullptr, x = nullptr, y = nullptr;
+  hipblasLtMatmulAlgo_t algo{};
+  size_t workspace = 0;
+  bool found = false;
+
+  LibraryPlan(int64_t M, int64_t N, int64_t K) {
+    const hipblasOperation_t t = HIPBLAS_OP_T, n = HIPBLAS_OP_N;
+    hipblasLtMatmulPreference_t pref = nullptr;
+    const size_t most = kWorkspaceBytes;
+    hipblasLtMatmulHeuristicResult_t result{};
+    int count = 0;
+    auto ok = [](hipblasStatus_t s) { return s == HIPBLAS_STATUS_SUCCESS; };
+    found =
+        ok(hipblasLtMatmulDescCreate(&product, HIPBLAS_COMPUTE_32F,
+                                     HIP_R_32F)) &&
+        ok(hipblasLtMatmulDescSetAttribute(
+            product, HIPBLASLT_MATMUL_DESC_TRANSA, &t, sizeof t)) &&
+        ok(hipblasLtMatmulDescSetAttribute(
+            product, HIPBLASLT_MATMUL_DESC_TRANSB, &n, sizeof n)) &&
+        ok(hipblasLtMatrixLayoutCreate(&w, HIP_R_16BF, K, N, K)) &&
+        ok(hipblasLtMatrixLayoutCreate(&x, HIP_R_16BF, K, M, K)) &&
+        ok(hipblasLtMatrixLayoutCreate(&y, HIP_R_16BF, N, M, N)) &&
+        ok(hipblasLtMatmulPreferenceCreate(&pref)) &&
+        ok(hipblasLtMatmulPreferenceSetAttribute(
+            pref, HIPBLASLT_MATMUL_PREF_MAX_WORKSPACE_BYTES, &most,
+            sizeof most)) &&
+        ok(hipblasLtMatmulAlgoGetHeuristic(
+            at::cuda::getCurrentCUDABlasLtHandle(), product, w, x, y, y, pref,
+            1, &result, &count)) &&
+        count == 1;
+    if (pref) hipblasLtMatmulPreferenceDestroy(pref);
+    algo = result.algo;
+    workspace = result.workspaceSize;
+  }
+  LibraryPlan(const LibraryPlan&) = delete;
+  ~LibraryPlan() {
+    for (auto layout : {w, x, y})
+      if (layout) hipblasLtMatrixLayoutDestroy(layout);
+    if (product) hipblasLtMatmulDescDestroy(product);
+  }
+};
+
+// by device and sizes, of any thread; a call keeps the plan that it uses
+std::shared_ptr<const LibraryPlan> library_plan(int device, int64_t M,
+                                                int64_t N, int64_t K) {
+  static std::mutex mutex;
+  static std::map<std::array<int64_t, 4>, std::shared_ptr<const LibraryPlan>>
+      plans;
+  constexpr size_t MOST = 1024;
+  const std::lock_guard<std::mutex> lock(mutex);
+  const std::array<int64_t, 4> key{device, M, N, K};
+  const auto at = plans.find(key);
+  if (at != plans.end()) return at->second;
+  if (plans.size() >= MOST) plans.clear();
+  return plans[key] = std::make_shared<const LibraryPlan>(M, N, K);
+}
+
+// x w^T as at::linear has it.  Of many rows, where the library's pick divides K
+// and sums in a workspace (beside tiles that do not come out even), tiles of our
+// own are faster (us, the library first: 4096 x 14336, 4300 rows 735 and 369,
+// 7613 979 and 665, 7000 644 and 615; 6160 x 2048, 7259 rows 188 and 160; 5120 x
+// 13824, 7400 rows 910 and 856; 8192 x 28672, 2100 rows 1470 and 729; where it
+// does not divide K the other way round, 7900 rows of the first 628 and 674).
+Tensor library_linear(const Tensor& x, const Tensor& w) {
+  check_linear_args(x, w);
+  TORCH_CHECK(x.device() == w.device(), "x and W on one GPU");
+  const int64_t M = x.size(0), N = w.size(0), K = x.size(1);
+  const auto start = reinterpret_cast<uintptr_t>(x.data_ptr()) |
+                     reinterpret_cast<uintptr_t>(w.data_ptr());
+  if (M == 0 || N == 0 || K == 0 || start % 16 != 0 ||
+      at::globalContext().blasPreferredBackend() != at::BlasBackend::Cublaslt ||
+      at::cuda::tunable::getTuningContext()->IsTunableOpEnabled())
+    return at::linear(x, w);
+  c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
+  const auto plan = library_plan(x.device().index(), M, N, K);
+  if (!plan->found) return at::linear(x, w);
+  Tensor y = at::empty({M, N}, x.options()), workspace;
+  const auto stream = at::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream();
+  if (plan->workspace && M > 1024 && K % 64 == 0 && N % 8 == 0 &&
+      std::max({x.numel(), w.numel(), y.numel()}) < int64_t(1) << 31) {
+    rlli::launch_tile_gemm(static_cast<const uint16_t*>(x.data_ptr()),
+                           static_cast<const uint16_t*>(w.data_ptr()), nullptr,
+                           static_cast<uint16_t*>(y.data_ptr()), int(M), int(N),
+                           int(K), rlli::TileAct::none,
+                           rlli::tile_gemm_plan(int(M), int(N), int(K), true),
+                           stream);
+    rlli_ext::check_launch("library_linear");
+    return y;
+  }
+  if (plan->workspace)
+    workspace = at::empty({int64_t(plan->workspace)},
+                          x.options().dtype(at::kByte));
+  const float one = 1.f, zero = 0.f;
+  const hipblasStatus_t status = hipblasLtMatmul(
+      at::cuda::getCurrentCUDABlasLtHandle(), plan->product, &one,
+      w.data_ptr(), plan->w, x.data_ptr(), plan->x, &zero, y.data_ptr(),
+      plan->y, y.data_ptr(), plan->y, &plan->algo,
+      workspace.defined() ? workspace.data_ptr() : nullptr, plan->workspace,
+      stream);
+  TORCH_CHECK(status == HIPBLAS_STATUS_SUCCESS, "library_linear: status ",
+              int(status), " for M=", M, " N=", N, " K=", K);
+  return y;
+}
+
 TORCH_LIBRARY_FRAGMENT(rlli, m) {
+  m.def("library_linear(Tensor x, Tensor w) -> Tensor");
   m.def("lt_linear(Tensor x, Tensor w, int algo_index) -> Tensor");
   m.def("lt_heuristics(Tensor x, Tensor w, int max_n) -> Tensor");
 }
 
 TORCH_LIBRARY_IMPL(rlli, CUDA, m) {
+  m.impl("library_linear", library_linear);
   m.impl("lt_linear", lt_linear);
   m.impl("lt_heuristics", lt_heuristics);
 }

@@ -49,6 +49,8 @@ def _linear(x, w):
     if (lt_autotune.enabled() and x.is_cuda and x.dim() == 2
             and x.shape[0] in _LT_ROWS):
         return lt_autotune.tuned_linear(x, w)
+    if ops.rows_tall_fit(x, w):
+        return ops.rows_tall(x, w)
     if ops.tile_linear_fit(x, w):
         return ops.tile_linear(x, w)
     if ops.rows_fit(x, w):
@@ -79,6 +81,8 @@ def _linear_parts(x, w):
 def _linear_relu2(x, w):
     """relu2 of _linear."""
     if not _USE_SKINNY and not lt_autotune.enabled():
+        if ops.rows_tall_fit(x, w):
+            return ops.rows_tall(x, w, relu2=True)
         if ops.tile_relu2_fit(x, w):
             return ops.tile_linear_relu2(x, w)
         if ops.rows_fit(x, w) and ops.rows_whole(x, w):

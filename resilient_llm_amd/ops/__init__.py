@@ -10,6 +10,7 @@ what the no-GPU plumbing tests and the gloo multi-process tests use.
 
 from __future__ import annotations
 
+import functools
 import os
 import torch
 
@@ -530,6 +531,44 @@ def rows_linear_scaled_relu2(h, ss, eps: float, w):
     """rows_linear_relu2 of what rows_linear_streams_ left, normed."""
     _gpu()
     return torch.ops.rlli.rows_linear_scaled_relu2(h, ss, eps, w)
+
+
+@functools.lru_cache(maxsize=4096)
+def _tall_faster(M: int, N: int, K: int) -> bool:
+    """Where rows_tall beats the other ways: rows_linear up to 128 rows, tiles and
+    the library.  (As many times as fast, with the rows of x and w that one of its
+    workgroups has where those decide: 2048 x 1024, 65 rows 1.90, 512 1.22; 1024 x
+    2048, 768 1.05; 2048 x 2048, 320 1.02, 512 rows (128) 0.98, 3072 x 2048, 320
+    rows (128) 0.93, but 4096 x 2048, 256 rows (128) 1.08; 256 x 2048, 96 rows
+    0.85; 3072 x 3072, 65 1.57, 320 1.07; 8192 x 3072, 112 1.02; 2048 x 3072, 80
+    1.00, 112 0.87; 2048 x 4096, 112 1.06, 448 1.09; 6144 x 4096, 65 1.09, 112
+    1.02; 8192 x 4096, 65 0.94; 1536 x 4096, 128 0.90; 4096 x 5120, 128 1.02, 160
+    0.82.)"""
+    if not 64 < M <= 768 or K > 4096 or K % 64 or N < 256:
+        return False
+    _gpu()
+    work = torch.ops.rlli.rows_tall_work(M, N)
+    if work == 0:
+        return False
+    if K <= 1024:
+        return True
+    if K <= 2048:
+        return N >= 512 and (work <= 112 or N >= 4096)
+    if K <= 3072:
+        return N >= 3072
+    return 2048 <= N <= 6144
+
+
+def rows_tall_fit(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether rows_tall takes x w^T and is the faster way."""
+    return _tiles_take(x, w, _tall_faster)
+
+
+def rows_tall(x: torch.Tensor, w: torch.Tensor,
+              relu2: bool = False) -> torch.Tensor:
+    """x w^T of some hundred rows, or relu2 of that."""
+    _gpu()
+    return torch.ops.rlli.rows_tall(x, w, relu2)
 
 
 def _tiles_take(x: torch.Tensor, w: torch.Tensor, faster) -> bool:

@@ -994,6 +994,30 @@ static void check_tiles(const Tensor& x, const Tensor& w, int multiple) {
               "x and W start at multiples of 16 bytes");
 }
 
+// Rows of x and w that a workgroup of rows_tall has; 0: it does not take M rows
+// by N columns.
+int64_t rows_tall_work(int64_t M, int64_t N) {
+  if (M < 1 || N < 1 || M > 1 << 20 || N > 1 << 20) return 0;
+  const rlli::TallPlan plan = rlli::rows_tall_plan(int(M), int(N));
+  return plan.rows + 8 * plan.eights;
+}
+
+// x w^T of some hundred rows, or the squared positive part of it in 16 bits, by
+// workgroups that divide K themselves
+Tensor rows_tall(const Tensor& x, const Tensor& w, bool relu2) {
+  check_tiles(x, w, 4);
+  TORCH_CHECK(rows_tall_work(x.size(0), w.size(0)) > 0,
+              "too many rows and columns to run at once");
+  const int M = int(x.size(0)), N = int(w.size(0)), K = int(x.size(1));
+  c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
+  Tensor out = at::empty({M, N}, x.options());
+  rlli::launch_rows_tall(bf16_ptr(x), bf16_ptr(w), bf16_ptr(out), M, N, K,
+                         relu2, rlli::rows_tall_plan(M, N),
+                         current_stream(x));
+  check_launch("rows_tall");
+  return out;
+}
+
 // The tile and the division of K that should take least, or those of ``plan``:
 // a tile's 64 rows and 128 columns, and parts.
 static rlli::TilePlan tile_plan(int M, int N, int K, bool whole,
@@ -1348,6 +1372,8 @@ TORCH_LIBRARY(rlli, m) {
   m.def("rows_linear(Tensor x, Tensor w) -> Tensor");
   m.def("rows_linear_silu(Tensor x, Tensor w) -> Tensor");
   m.def("rows_linear_relu2(Tensor x, Tensor w) -> Tensor");
+  m.def("rows_tall(Tensor x, Tensor w, bool relu2) -> Tensor");
+  m.def("rows_tall_work(int m, int n) -> int", &rows_tall_work);
   m.def("rows_whole_ok(int m, int n, int k) -> bool", &rows_whole_ok);
   m.def("rows_norm_ok(int n, int k, bool silu) -> bool",
         &rows_norm_ok);
@@ -1408,6 +1434,7 @@ TORCH_LIBRARY_IMPL(rlli, CUDA, m) {
   m.impl("rows_linear", &rows_linear);
   m.impl("rows_linear_silu", &rows_linear_silu);
   m.impl("rows_linear_relu2", &rows_linear_relu2);
+  m.impl("rows_tall", &rows_tall);
   m.impl("rows_norm_linear", &rows_norm_linear);
   m.impl("rows_linear_streams_", &rows_linear_streams_);
   m.impl("rows_linear_scaled_relu2", &rows_linear_scaled_relu2);

@@ -212,6 +212,15 @@ void launch_rows_scaled_relu2(const uint16_t* x, const uint16_t* w,
 bool rows_short_ok(int N, int K);
 void launch_rows_short(const uint16_t* x, const uint16_t* w, uint16_t* out,
                        int M, int N, int K, bool relu2, hipStream_t stream);
+// more rows: tiles of ``rows`` rows by 8 ``eights`` rows of w; ``relu2`` of the
+// 16-bit product
+struct TallPlan {
+  int rows, eights;
+};
+TallPlan rows_tall_plan(int M, int N);
+void launch_rows_tall(const uint16_t* x, const uint16_t* w, uint16_t* out,
+                      int M, int N, int K, bool relu2, const TallPlan& plan,
+                      hipStream_t stream);
 void launch_sum_parts(const float* parts, uint16_t* out, int splits,
                       int64_t n, hipStream_t stream);
 

@@ -503,16 +503,25 @@ void rows_gemm_kernel(const uint16_t* __restrict__ x,
 // is no barrier before the sums meet at the end.  What bounds it is the time
 // from the launch to the first data and, past 4096 in K, that it reads x once
 // per 8 to 32 rows of w.
+// More rows than 64 are tiles of 48 or 64 (TALL), as many as run at once.  What
+// bounds those is what a CU can ask for: it takes 58 bytes a ns while any of it
+// comes from HBM, whatever is under way, so that a workgroup's rows of x and w
+// together are what counts, and a tile that is nearly square is the best.  (us,
+// the other way first, 65, 128 and 256 rows: 2048 x 2048 8.7 and 6.1, 8.6 and
+// 7.3, 9.6 and 8.2; 6144 x 2048 14.0 and 10.8, 15.3 and 11.7; 4096 x 4096 14.9
+// and 14.8, 18.3 and 14.8, 22.6 and 20.7; 3072 x 1024 8.6 and 5.2, 9.4 and 6.1,
+// 8.9 and 7.4.)
 // END: the result, its squared positive part, or (ADDS; HR 2) S streams with it.
+// TALL: ``tiles`` of XR rows, which read the same rows of w on one XCD.
 enum End { WHOLE, RELU2, ADDS };
 
 template <int HR, int XR, int MT, int R, End END, int S = 0,
-          bool SCALED = false>
+          bool SCALED = false, bool TALL = false>
 __global__ __launch_bounds__(256)
 void rows_short_kernel(const uint16_t* __restrict__ x,
                        const uint16_t* __restrict__ w,
                        uint16_t* __restrict__ out, int M, int N, int K,
-                       RowsScale scale, RowsAdds adds) {
+                       RowsScale scale, RowsAdds adds, int tiles) {
   constexpr int PT = (HR + 1) / 2;                   // tiles of w
   constexpr int WPART = HR * 8 * LINE;               // elements of a step
   constexpr int STEP = WPART + XR * LINE;
@@ -520,10 +529,15 @@ void rows_short_kernel(const uint16_t* __restrict__ x,
   extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
   const int lane = threadIdx.x & 63;
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int n0 = blockIdx.x * HR * 8;
+  const int slot0 = blockIdx.x >> 3;
+  const int panel =
+      TALL ? slot0 / tiles * 8 + int(blockIdx.x & 7) : int(blockIdx.x);
+  const int m0 = TALL ? slot0 % tiles * XR : 0;
+  const int n0 = panel * HR * 8;
+  if (TALL && n0 >= N) return;
   // this wave's steps: wv, wv + 4, ...
   const int n = (K / KS - wv + 3) / 4;
-  const int rot = n > 0 ? int(blockIdx.x / 8 % unsigned(n)) : 0;
+  const int rot = n > 0 ? int(unsigned(panel) / 8 % unsigned(n)) : 0;
   uint16_t* ring = lds + wv * R * STEP;
 
   const int lr = lane >> 3;
@@ -538,7 +552,7 @@ void rows_short_kernel(const uint16_t* __restrict__ x,
 #pragma unroll
   for (int j = 0; j < LX; ++j) {
     const int r = j * 8 + lr;
-    xp[j] = x + int64_t(min(r, M - 1)) * K + wv * KS +
+    xp[j] = x + int64_t(min(m0 + r, M - 1)) * K + wv * KS +
             ((lane & 7) ^ ((r >> 1) & 7)) * 8;
   }
   auto issue = [&](int s, int slot) {
@@ -631,12 +645,14 @@ void rows_short_kernel(const uint16_t* __restrict__ x,
     f32x4 v = side[e * 64 + lane];
 #pragma unroll
     for (int o = 1; o < 4; ++o) v += side[(o * PT * MT + e) * 64 + lane];
-    const int row = e % MT * 16 + tr;
+    const int row = m0 + e % MT * 16 + tr;
     const int c = n0 + e / MT * 16 + oct * 4;
     if constexpr (SCALED) v *= Scale<SCALED ? MT : 1>::of(scale, part, row);
     if constexpr (END == RELU2) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
+        // (of more rows of the 16-bit product, as by tiles)
+        if constexpr (TALL) v[r] = bf16_to_f32(f32_to_bf16(v[r]));
         v[r] = fmaxf(v[r], 0.f);
         v[r] *= v[r];
       }
@@ -748,7 +764,7 @@ void go_short(const uint16_t* x, const uint16_t* w, uint16_t* out, int M,
                                 hipFuncAttributeMaxDynamicSharedMemorySize,
                                 int(smem));
     hipLaunchKernelGGL(k, dim3((N + HR * 8 - 1) / (HR * 8)), dim3(256), smem,
-                       st, x, w, out, M, N, K, RowsScale{}, RowsAdds{});
+                       st, x, w, out, M, N, K, RowsScale{}, RowsAdds{}, 1);
   };
   if (M <= 16) run(std::integral_constant<int, 16>{});
   else if (M <= 32) run(std::integral_constant<int, 32>{});
@@ -770,10 +786,26 @@ void go_shared(const uint16_t* x, const uint16_t* w, uint16_t* out, int M,
                                 hipFuncAttributeMaxDynamicSharedMemorySize,
                                 int(smem));
     hipLaunchKernelGGL(k, dim3((N + HR * 8 - 1) / (HR * 8)), dim3(256), smem,
-                       st, x, w, out, M, N, K, scale, adds);
+                       st, x, w, out, M, N, K, scale, adds, 1);
   };
   if (M <= 16) run(std::integral_constant<int, 16>{});
   else run(std::integral_constant<int, 32>{});
+}
+
+// of more rows than a tile has
+template <int HR, int XR, int R, End END>
+void go_tall(const uint16_t* x, const uint16_t* w, uint16_t* out, int M, int N,
+             int K, hipStream_t st) {
+  constexpr int MT = XR / 16;
+  constexpr size_t smem = size_t(4) * R * (HR * 8 + XR) * LINE * 2;
+  auto* k = rows_short_kernel<HR, XR, MT, R, END, 0, false, true>;
+  if (smem > 65536)
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(k),
+                              hipFuncAttributeMaxDynamicSharedMemorySize,
+                              int(smem));
+  const int tiles = (M + XR - 1) / XR, panels = (N + HR * 8 - 1) / (HR * 8);
+  hipLaunchKernelGGL(k, dim3((panels + 7) / 8 * 8 * tiles), dim3(256), smem, st,
+                     x, w, out, M, N, K, RowsScale{}, RowsAdds{}, tiles);
 }
 
 }  // namespace
@@ -906,6 +938,44 @@ void launch_rows_short(const uint16_t* x, const uint16_t* w, uint16_t* out,
       case 2: return go_short<2, 9, 6, 3, END>(x, w, out, M, N, K, st);
       case 3: return go_short<3, 7, 5, 3, END>(x, w, out, M, N, K, st);
       default: return go_short<4, 6, 4, 3, END>(x, w, out, M, N, K, st);
+    }
+  };
+  if (relu2) run(std::integral_constant<End, RELU2>{});
+  else run(std::integral_constant<End, WHOLE>{});
+}
+
+// The least rows of x and w a workgroup, where all workgroups of an XCD run at
+// once on its 32 CUs; none: rows 0.
+TallPlan rows_tall_plan(int M, int N) {
+  TallPlan best{0, 0};
+  for (int rows : {64, 48})
+    for (int eights : {2, 3, 4, 6, 8}) {
+      const int64_t tiles = (int64_t(M) + rows - 1) / rows;
+      const int64_t panels = (int64_t(N) + eights * 8 - 1) / (eights * 8);
+      if (tiles * ((panels + 7) / 8) <= 32 &&
+          (best.rows == 0 ||
+           rows + 8 * eights < best.rows + 8 * best.eights))
+        best = TallPlan{rows, eights};
+    }
+  return best;
+}
+
+void launch_rows_tall(const uint16_t* x, const uint16_t* w, uint16_t* out,
+                      int M, int N, int K, bool relu2, const TallPlan& plan,
+                      hipStream_t st) {
+  auto run = [&](auto end) {
+    constexpr End END = decltype(end)::value;
+    switch (plan.rows * 16 + plan.eights) {
+      case 48 * 16 + 2: return go_tall<2, 48, 4, END>(x, w, out, M, N, K, st);
+      case 48 * 16 + 3: return go_tall<3, 48, 4, END>(x, w, out, M, N, K, st);
+      case 48 * 16 + 4: return go_tall<4, 48, 3, END>(x, w, out, M, N, K, st);
+      case 48 * 16 + 6: return go_tall<6, 48, 3, END>(x, w, out, M, N, K, st);
+      case 48 * 16 + 8: return go_tall<8, 48, 2, END>(x, w, out, M, N, K, st);
+      case 64 * 16 + 2: return go_tall<2, 64, 3, END>(x, w, out, M, N, K, st);
+      case 64 * 16 + 3: return go_tall<3, 64, 3, END>(x, w, out, M, N, K, st);
+      case 64 * 16 + 4: return go_tall<4, 64, 3, END>(x, w, out, M, N, K, st);
+      case 64 * 16 + 6: return go_tall<6, 64, 2, END>(x, w, out, M, N, K, st);
+      default: return go_tall<8, 64, 2, END>(x, w, out, M, N, K, st);
     }
   };
   if (relu2) run(std::integral_constant<End, RELU2>{});

@@ -155,3 +155,58 @@ def test_weights_elsewhere_are_refused():
     x, w = operands(64, 128)
     with pytest.raises(RuntimeError):
         ops.rows_linear(x, w.cpu())
+
+
+# tiles of 48 and 64 rows by 16 to 64 rows of w: their edges, a last one with few
+# rows, one panel, fewer steps of K than waves, odd numbers of them
+TALL = [(65, 4, 64), (65, 2048, 192), (96, 2044, 320), (97, 2052, 64),
+        (128, 3076, 448), (129, 2048, 2048), (191, 2048, 128),
+        (192, 3072, 1088), (193, 3072, 256), (256, 4096, 320),
+        (257, 2040, 704), (96, 6160, 576), (128, 8192, 192), (768, 1024, 512),
+        (767, 260, 3136)]
+
+
+@pytest.mark.parametrize("M,N,K", TALL)
+def test_rows_tall(M, N, K):
+    gen = torch.Generator().manual_seed(M)
+    x = torch.randn(M, K, generator=gen).to(torch.bfloat16).to(DEV)
+    w = torch.randn(N, K, generator=gen).to(torch.bfloat16).to(DEV)
+    want = x.double() @ w.double().T
+    got = torch.ops.rlli.rows_tall(x, w, False)
+    close(got, want, K ** 0.5)
+    # of the 16-bit product, in f32 and rounded once more
+    relu2 = torch.ops.rlli.rows_tall(x, w, True)
+    assert torch.equal(relu2, got.float().clamp(min=0).square()
+                       .to(torch.bfloat16))
+
+
+@pytest.mark.parametrize("N", [16, 264, 1040, 2048, 2056, 4100, 6160, 8192])
+def test_every_tall_tile_is_in_one_round(N):
+    work = torch.ops.rlli.rows_tall_work
+    had = [work(M, N) for M in range(65, 800)]
+    # from some number of rows on there is none, and until there more rows are
+    # as much work or more
+    some = [v for v in had if v]
+    assert had == some + [0] * (len(had) - len(some))
+    assert all(64 <= v <= 128 for v in some)
+
+
+@pytest.mark.parametrize("M,N,K,fits", [
+    (65, 2048, 1024, True), (768, 1024, 1024, True), (769, 256, 1024, False),
+    (64, 2048, 2048, False), (320, 2048, 2048, True), (512, 2048, 2048, False),
+    (320, 3072, 2048, False), (256, 4096, 2048, True), (96, 256, 2048, False),
+    (128, 8192, 2048, True), (129, 8192, 2048, False), (80, 2048, 3072, False),
+    (65, 3072, 3072, True), (128, 6144, 4096, True), (65, 8192, 4096, False),
+    (129, 6144, 4096, False), (128, 1536, 4096, False), (65, 2048, 4160, False),
+    (65, 2048, 2080, False)])
+def test_tall_where_it_is_the_faster_one(M, N, K, fits):
+    assert ops._tall_faster(M, N, K) == fits
+
+
+def test_tall_refuses():
+    x, w = operands(64, 128)
+    for a, b in [(x, w.cpu()), (x.float(), w.float()), (x[:, :64], w[:, :64]),
+                 (x, w[:62]), (x[:0], w), (x.repeat(60, 1), w.repeat(60, 1)),
+                 (off_by(x, 4), w)]:
+        with pytest.raises(RuntimeError):
+            torch.ops.rlli.rows_tall(a, b, False)

@@ -543,8 +543,9 @@ def _tall_faster(M: int, N: int, K: int) -> bool:
     0.85; 3072 x 3072, 65 1.57, 320 1.07; 8192 x 3072, 112 1.02; 2048 x 3072, 80
     1.00, 112 0.87; 2048 x 4096, 112 1.06, 448 1.09; 6144 x 4096, 65 1.09, 112
     1.02; 8192 x 4096, 65 0.94; 1536 x 4096, 128 0.90; 4096 x 5120, 128 1.02, 160
-    0.82.)"""
-    if not 64 < M <= 768 or K > 4096 or K % 64 or N < 256:
+    0.82; 2048 x 6144, 65 1.06, 192 1.25, 320 1.07, 448 0.92; 1536 x 6144, 65
+    1.02, 384 1.20, 512 1.01.)"""
+    if not 64 < M <= 768 or K > 6144 or K % 64 or N < 256:
         return False
     _gpu()
     work = torch.ops.rlli.rows_tall_work(M, N)
@@ -556,7 +557,9 @@ def _tall_faster(M: int, N: int, K: int) -> bool:
         return N >= 512 and (work <= 112 or N >= 4096)
     if K <= 3072:
         return N >= 3072
-    return 2048 <= N <= 6144
+    if K <= 4096:
+        return 2048 <= N <= 6144
+    return 1536 <= N <= 2048 and M <= 384
 
 
 def rows_tall_fit(x: torch.Tensor, w: torch.Tensor) -> bool:

@@ -31,6 +31,7 @@
 
 #include "rec_math.h"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace rlli {
@@ -250,19 +251,23 @@ DEV_INLINE float seen_log(float L) {
   return L;
 }
 
-// Wave w owns sub-chunk w, lane l its row l & 15 and four neighbouring key
-// columns of every 16; MD bounds the key tiles (dpad <= 64 * MD).  FULL: dim
-// is 64 MD, the rank a multiple of 16 and rows are aligned, so that no load
-// is conditional (rows behind the last one are loaded from it).
-template <typename T, int KIND, int MD, bool FULL, bool PARTS>
-__global__ __launch_bounds__(256)
+// Waves w, w + 4, ... own sub-chunk w, NT 16-wide tiles of key columns each, lane
+// l its row l & 15 and four neighbouring columns of a tile; MD bounds the tiles
+// (dpad <= 64 * MD).  FULL: dim is 64 MD, the rank a multiple of 16 and rows are
+// aligned, so that no load is conditional (rows behind the last one are loaded
+// from it).  What bounds a workgroup is its waves' instructions, one after another
+// as no other waves are there to run between them: 128 columns in one wave are
+// some 10000 of them.
+template <typename T, int KIND, int MD, int NT, bool FULL, bool PARTS>
+__global__ __launch_bounds__(1024 * MD / NT)
 void gla_intra_kernel(GlaArgs a, bool vec, bool vec_a) {
   constexpr bool FG = KIND == kHgrn2, BONUS = KIND == kRwkv;
   extern __shared__ __attribute__((aligned(16))) float sm[];
-  constexpr int NT = 4 * MD;
+  constexpr int Q = 4 * MD / NT;
   const int tile = blockIdx.x, h = blockIdx.y;
   const int lane = threadIdx.x & 63;
-  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int w = wave & 3, part = wave >> 2, dt0 = part * NT;
   const int lr = lane & 15, g = lane >> 4;
   const int DP = FULL ? 64 * MD : a.dpad, LR = DP + 4, ndt = DP / 16;
   float* kl = sm;                        // [64][LR] keys, then decayed keys
@@ -295,17 +300,18 @@ void gla_intra_kernel(GlaArgs a, bool vec, bool vec_a) {
   float wmin = 0.f;
   // (raw keys wait in the registers of the log-decays)
 #pragma unroll
-  for (int dt = 0; dt < NT; ++dt) {
-    if (!FULL && dt >= ndt) continue;
-    const int d = dt * 16 + g * 4;
-    q[dt] = row4(qrow, d, a.dim, vec);
-    L[dt] = row4(krow, d, a.dim, vec);
+  for (int i = 0; i < NT; ++i) {
+    if (!FULL && dt0 + i >= ndt) continue;
+    const int d = (dt0 + i) * 16 + g * 4;
+    q[i] = row4(qrow, d, a.dim, vec);
+    L[i] = row4(krow, d, a.dim, vec);
   }
 #pragma unroll
-  for (int dt = 0; dt < NT; ++dt) {
+  for (int i = 0; i < NT; ++i) {
+    const int dt = dt0 + i;
     if (!FULL && dt >= ndt) continue;
     const int d = dt * 16 + g * 4;
-    f32x4_t k = L[dt];
+    f32x4_t k = L[i];
     if constexpr (FULL && !FG)
       if (!row_ok) k = f32x4_t{0.f, 0.f, 0.f, 0.f};
     const f32x4_t bv = vec4(bias, d);
@@ -317,8 +323,8 @@ void gla_intra_kernel(GlaArgs a, bool vec, bool vec_a) {
         float alpha;
         const float kk = forget_key<T>(k[j] + bv[j], lv[j], &alpha);
         k[j] = ok ? kk : 0.f;
-        L[dt][j] = ok ? log_forget<T>(alpha, kk) : 0.f;
-        q[dt][j] = silu<T>(q[dt][j]);
+        L[i][j] = ok ? log_forget<T>(alpha, kk) : 0.f;
+        q[i][j] = silu<T>(q[i][j]);
       }
     } else {
       // z transposed: columns down, rows across the lanes
@@ -343,18 +349,18 @@ void gla_intra_kernel(GlaArgs a, bool vec, bool vec_a) {
         const bool ok = row_ok && d + j < a.dim;
         const float lw = BONUS ? log_rwkv<T>(z[j] + bv[j])
                                : log_sigmoid<T>(z[j] + bv[j]) / a.tau;
-        L[dt][j] = ok ? lw : 0.f;
-        if constexpr (!BONUS) q[dt][j] *= qscale;
+        L[i][j] = ok ? lw : 0.f;
+        if constexpr (!BONUS) q[i][j] *= qscale;
       }
     }
     *reinterpret_cast<f32x4_t*>(kl + trow * LR + d) = k;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      L[dt][j] = row_prefix(L[dt][j]);
-      const float mid = __shfl(L[dt][j], g * 16 + 7, kWave);
+      L[i][j] = row_prefix(L[i][j]);
+      const float mid = __shfl(L[i][j], g * 16 + 7, kWave);
       if (lr == 15) {
-        tot[w * DP + d + j] = L[dt][j];
-        wmin = fminf(wmin, fminf(mid, L[dt][j] - mid));
+        tot[w * DP + d + j] = L[i][j];
+        wmin = fminf(wmin, fminf(mid, L[i][j] - mid));
       }
     }
   }
@@ -363,19 +369,19 @@ void gla_intra_kernel(GlaArgs a, bool vec, bool vec_a) {
   float own = 0.f;                       // this row's diagonal
   if constexpr (BONUS) {
 #pragma unroll
-    for (int dt = 0; dt < NT; ++dt) {
-      if (!FULL && dt >= ndt) continue;
-      const int d = dt * 16 + g * 4;
+    for (int i = 0; i < NT; ++i) {
+      if (!FULL && dt0 + i >= ndt) continue;
+      const int d = (dt0 + i) * 16 + g * 4;
       const f32x4_t kv = *reinterpret_cast<const f32x4_t*>(kl + trow * LR + d);
       const f32x4_t uv = vec4(a.bonus + h * a.dim, d);
 #pragma unroll
-      for (int j = 0; j < 4; ++j) own += q[dt][j] * uv[j] * kv[j];
+      for (int j = 0; j < 4; ++j) own += q[i][j] * uv[j] * kv[j];
     }
     own += __shfl_xor(own, 16, kWave);
     own += __shfl_xor(own, 32, kWave);
   }
   __syncthreads();
-  for (int d = threadIdx.x; d < DP; d += 256) {
+  for (int d = threadIdx.x; d < DP; d += blockDim.x) {
     float t[4], b = 0.f;
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
@@ -404,13 +410,13 @@ void gla_intra_kernel(GlaArgs a, bool vec, bool vec_a) {
     float near[4] = {0.f, 0.f, 0.f, 0.f};  // row lr and the row so far back
     f32x4_t far = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int dt = 0; dt < NT; ++dt) {
-      if (!FULL && dt >= ndt) continue;
+    for (int i = 0; i < NT; ++i) {
+      if (!FULL && dt0 + i >= ndt) continue;
       const f32x4_t k = *reinterpret_cast<const f32x4_t*>(
-          kl + trow * LR + dt * 16 + g * 4);
+          kl + trow * LR + (dt0 + i) * 16 + g * 4);
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const float Lt = L[dt][j], Lq = seen(Lt), qv = q[dt][j], kv = k[j];
+        const float Lt = L[i][j], Lq = seen(Lt), qv = q[i][j], kv = k[j];
         float ref[4];
 #pragma unroll
         for (int b = 1; b < 4; ++b)
@@ -468,7 +474,8 @@ void gla_intra_kernel(GlaArgs a, bool vec, bool vec_a) {
   const int turned = (lr >> 2) * 16 + g * 4 + (lr & 3);
   f32x4_t diag = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int dt = 0; dt < NT; ++dt) {
+  for (int i = 0; i < NT; ++i) {
+    const int dt = dt0 + i;
     if (!FULL && dt >= ndt) continue;
     const int d = dt * 16 + g * 4;
     const f32x4_t tw = *reinterpret_cast<const f32x4_t*>(tot + w * DP + d);
@@ -478,21 +485,21 @@ void gla_intra_kernel(GlaArgs a, bool vec, bool vec_a) {
     f32x4_t kt = *reinterpret_cast<const f32x4_t*>(kl + trow * LR + d), qo, ko;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      const float Lt = L[dt][j];
+      const float Lt = L[i][j];
       if (safe) {
         const float Lm = __shfl(Lt, g * 16 + 7, kWave);
-        diag = mma4(q[dt][j] * gexp<T>(seen(Lt) - Lm),
+        diag = mma4(q[i][j] * gexp<T>(seen(Lt) - Lm),
                     kt[j] * gexp<T>(Lm - Lt), diag);
       }
-      q[dt][j] *= gexp<T>(seen(Lt));
-      qo[j] = q[dt][j] * eb[j];
+      q[i][j] *= gexp<T>(seen(Lt));
+      qo[j] = q[i][j] * eb[j];
       kt[j] *= gexp<T>(tw[j] - Lt);
       ko[j] = kt[j] * ed[j];
     }
     ko = quad_transposed(ko);
     if constexpr (PARTS) {
-      three_parts(qo, qh[dt & 1]);
-      if (dt & 1) put_q(dt / 2);
+      three_parts(qo, qh[i & 1]);
+      if (i & 1) put_q(dt / 2);
       uint2 kh[3];
       three_parts(ko, kh);
 #pragma unroll
@@ -506,7 +513,7 @@ void gla_intra_kernel(GlaArgs a, bool vec, bool vec_a) {
     }
     *reinterpret_cast<f32x4_t*>(kl + trow * LR + d) = kt;
   }
-  if (PARTS && !FULL && ndt % 2) {
+  if (PARTS && !FULL && ndt % 2 && (ndt - 1) / NT == part) {
 #pragma unroll
     for (int p = 0; p < 3; ++p) qh[1][p] = uint2{0, 0};
     put_q(ndt / 2);
@@ -525,13 +532,14 @@ void gla_intra_kernel(GlaArgs a, bool vec, bool vec_a) {
   __syncthreads();
   // rows of the sub-chunks before
 #pragma unroll
-  for (int dt = 0; dt < NT; ++dt) {
+  for (int i = 0; i < NT; ++i) {
+    const int dt = dt0 + i;
     if (!FULL && dt >= ndt) continue;
     const int d = dt * 16 + g * 4;
 #pragma unroll
     for (int J = 0; J < 3; ++J) {
       if (J >= w) break;
-      f32x4_t qe = q[dt];
+      f32x4_t qe = q[i];
       if (J + 1 < w) {
         const f32x4_t e = *reinterpret_cast<const f32x4_t*>(
             EJ + (J == 1 ? 2 : w - 2) * DP + d);
@@ -544,15 +552,33 @@ void gla_intra_kernel(GlaArgs a, bool vec, bool vec_a) {
       for (int j = 0; j < 4; ++j) acc[J] = mma4(qe[j], kt[j], acc[J]);
     }
   }
+  // the waves' sums meet, in order; a wave finishes every Q-th tile
+  f32x4_t* sums = reinterpret_cast<f32x4_t*>(sm) + lane;
+  if constexpr (Q > 1) {
+    __syncthreads();
+#pragma unroll
+    for (int J = 0; J < 4; ++J)
+      if (J <= w) sums[(part * 10 + w * (w + 1) / 2 + J) * 64] = acc[J];
+    __syncthreads();
+  }
   float* sc = static_cast<float*>(a.sc) + ch * C * C;
   uint16_t* sp = static_cast<uint16_t*>(a.sc) + ch * 12288;
 #pragma unroll
   for (int J = 0; J < 4; ++J) {
     if (J > (PARTS ? w | 1 : w)) break;    // (a pair's second tile: zeros)
+    if (J % Q != part) continue;
+    f32x4_t v = acc[J];
+    if constexpr (Q > 1) {
+      v = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      if (J <= w)
+#pragma unroll
+        for (int i = 0; i < Q; ++i)
+          v += sums[(i * 10 + w * (w + 1) / 2 + J) * 64];
+    }
 #pragma unroll
     for (int r = 0; r < 4; ++r)
-      if (J > w || (J == w && lr > g * 4 + r)) acc[J][r] = 0.f;
-    const f32x4_t v = quad_transposed(acc[J]);
+      if (J > w || (J == w && lr > g * 4 + r)) v[r] = 0.f;
+    v = quad_transposed(v);
     if constexpr (PARTS) {
       uint2 h[3];
       three_parts(v, h);
@@ -573,26 +599,43 @@ void prefill(const GlaArgs& a, hipStream_t st) {
                    reinterpret_cast<uintptr_t>(a.proj) % (4 * sizeof(T)) == 0;
   const bool vec_a = a.rank % 4 == 0 && a.a1_stride % 4 == 0 &&
                      reinterpret_cast<uintptr_t>(a.a1) % (4 * sizeof(T)) == 0;
-  const size_t smem =
-      size_t(C * (a.dpad + 4) + 13 * a.dpad) * sizeof(float);
-  auto intra = [&](auto* k) {
+  auto intra = [&](auto* k, int waves) {
+    // keys and decays, then the waves' sums
+    const size_t smem =
+        std::max(size_t(C * (a.dpad + 4) + 13 * a.dpad) * sizeof(float),
+                 size_t(waves / 4) * 10 * 64 * sizeof(f32x4_t));
     if (smem > 65536)
       (void)hipFuncSetAttribute(reinterpret_cast<const void*>(k),
                                 hipFuncAttributeMaxDynamicSharedMemorySize,
                                 int(smem));
-    hipLaunchKernelGGL(k, dim3(a.n_tiles, a.heads), dim3(256), smem, st, a,
-                       vec, vec_a);
+    hipLaunchKernelGGL(k, dim3(a.n_tiles, a.heads), dim3(64 * waves), smem, st,
+                       a, vec, vec_a);
   };
   const bool parts = gla_parts(a);
   auto by_parts = [&](auto md, auto full) {
     constexpr int MD = decltype(md)::value;
     constexpr bool FULL = decltype(full)::value;
-    if constexpr (sizeof(T) == 4)
-      intra(gla_intra_kernel<T, KIND, MD, FULL, false>);
-    else if (parts)
-      intra(gla_intra_kernel<T, KIND, MD, FULL, true>);
+    auto by_tiles = [&](auto nt) {
+      constexpr int NT = decltype(nt)::value;
+      if constexpr (sizeof(T) == 4)
+        intra(gla_intra_kernel<T, KIND, MD, NT, FULL, false>, 16 * MD / NT);
+      else if (parts)
+        intra(gla_intra_kernel<T, KIND, MD, NT, FULL, true>, 16 * MD / NT);
+      else
+        intra(gla_intra_kernel<T, KIND, MD, NT, FULL, false>, 16 * MD / NT);
+    };
+    // Columns of a wave: 32 of heads of up to 128, 64 of wider ones, but of 128
+    // twice as many where workgroups are more than CUs.  (us by columns of a wave,
+    // all of them last, and workgroups: heads of 128, 32, 64 and 128 columns, 16:
+    // 14.4, 17.1 and 24.8, 256: 19.1, 20.7 and 27.4, 328: 31.0, 28.9 and 33.5, 960:
+    // 65.3, 59.8 and 63.5; of 64, 32: 11.2 and 15.0, 1920: 44.5 and 49.3; of 256,
+    // 64 columns, 16: 28 and 65, 960: 127 and 159.)
+    if constexpr (MD == 4)
+      by_tiles(std::integral_constant<int, 4>{});
+    else if (MD == 1 || a.n_tiles * a.heads <= 256)
+      by_tiles(std::integral_constant<int, 2>{});
     else
-      intra(gla_intra_kernel<T, KIND, MD, FULL, false>);
+      by_tiles(std::integral_constant<int, 2 * MD>{});
   };
   using I1 = std::integral_constant<int, 1>;
   using I2 = std::integral_constant<int, 2>;

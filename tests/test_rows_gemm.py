@@ -163,7 +163,7 @@ TALL = [(65, 4, 64), (65, 2048, 192), (96, 2044, 320), (97, 2052, 64),
         (128, 3076, 448), (129, 2048, 2048), (191, 2048, 128),
         (192, 3072, 1088), (193, 3072, 256), (256, 4096, 320),
         (257, 2040, 704), (96, 6160, 576), (128, 8192, 192), (768, 1024, 512),
-        (767, 260, 3136)]
+        (767, 260, 3136), (129, 2048, 6144)]
 
 
 @pytest.mark.parametrize("M,N,K", TALL)
@@ -197,8 +197,9 @@ def test_every_tall_tile_is_in_one_round(N):
     (320, 3072, 2048, False), (256, 4096, 2048, True), (96, 256, 2048, False),
     (128, 8192, 2048, True), (129, 8192, 2048, False), (80, 2048, 3072, False),
     (65, 3072, 3072, True), (128, 6144, 4096, True), (65, 8192, 4096, False),
-    (129, 6144, 4096, False), (128, 1536, 4096, False), (65, 2048, 4160, False),
-    (65, 2048, 2080, False)])
+    (129, 6144, 4096, False), (128, 1536, 4096, False), (65, 2048, 4160, True),
+    (384, 2048, 6144, True), (385, 2048, 6144, False), (65, 2048, 6208, False),
+    (128, 2112, 5120, False), (65, 2048, 2080, False)])
 def test_tall_where_it_is_the_faster_one(M, N, K, fits):
     assert ops._tall_faster(M, N, K) == fits
 

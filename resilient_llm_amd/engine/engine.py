@@ -15,6 +15,7 @@ from __future__ import annotations
 
 import collections
 import dataclasses
+import itertools
 import os
 import threading
 import time
@@ -707,6 +708,7 @@ class LLMEngine:
         t_prep = time.monotonic()
         mixed_layers = getattr(self.model, "mixed_layers", False)
         B_d = len(dec)
+        bs = self.block_size
         input_ids = [t for _, t in dec]
         positions = [s.n_cached for s, _ in dec]
         slots = [self._slot(s, s.n_cached) for s, _ in dec]
@@ -721,16 +723,20 @@ class LLMEngine:
             # pages that the portion sees: attention divides its keys by the
             # table's room
             bt_rows.append(seq.blocks if mixed_layers else
-                           seq.blocks[:-(-(start + n) // self.block_size)])
-            for q0 in range(0, n, 32):
-                c_row0.append(row + q0)
-                c_pos0.append(start + q0)
-                c_nrows.append(min(32, n - q0))
-                c_btrow.append(btr)
+                           seq.blocks[:-(-(start + n) // bs)])
+            if not mixed_layers:
+                c_row0.extend(range(row, row + n, 32))
+                c_pos0.extend(range(start, start + n, 32))
+                c_nrows.extend([32] * (n // 32) + [n % 32] * (n % 32 > 0))
+                c_btrow.extend([btr] * -(-n // 32))
             portions.append(Portion(row - B_d, start, n, btr, seq.slot or 0))
             input_ids.extend(toks)
             positions.extend(range(start, start + n))
-            slots.extend(self._slot(seq, p) for p in range(start, start + n))
+            # by pages: token by token 8000 of them took 1.4 ms
+            for p in range(start // bs, -(-(start + n) // bs)):
+                at = seq.blocks[p] * bs - p * bs
+                slots.extend(range(at + max(start, p * bs),
+                                   at + min(start + n, (p + 1) * bs)))
             row += n
 
         def i32(x):
@@ -764,11 +770,8 @@ class LLMEngine:
             # layers of 2048 took 1040 us with four that the host waits for,
             # takes 908)
             parts = (input_ids, positions, slots, [0] + ends)
-            packed = torch.tensor([v for part in parts for v in part],
-                                  dtype=torch.int32,
-                                  pin_memory=dev.type == "cuda")
-            ids_t, pos_t, slots_t, cu_t = packed.to(
-                dev, non_blocking=True).split([len(part) for part in parts])
+            ids_t, pos_t, slots_t, cu_t = i32(list(itertools.chain(
+                *parts))).split([len(part) for part in parts])
             self.stats["prefill_prep_time"] += time.monotonic() - t_prep
             t_fwd = time.monotonic()
             logits = self.model.forward_prefill(ids_t, pos_t, self.kv,

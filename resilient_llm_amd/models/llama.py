@@ -43,27 +43,34 @@ _USE_SKINNY = os.environ.get("RLLI_SKINNY") == "1"
 _LT_ROWS = frozenset({1, 2, 4, 8, 12, 16, 24, 32, 48, 64, 96, 128})
 
 
+def _way(form, x, w):
+    return ops.product_way(form, x.shape[0], *w.shape) \
+        if ops.product_operands(x, w) else None
+
+
 def _linear(x, w):
     if _USE_SKINNY:
         return ops.linear_auto(x, w)
     if (lt_autotune.enabled() and x.is_cuda and x.dim() == 2
             and x.shape[0] in _LT_ROWS):
         return lt_autotune.tuned_linear(x, w)
-    if ops.rows_tall_fit(x, w):
-        return ops.rows_tall(x, w)
-    if ops.tile_linear_fit(x, w):
-        return ops.tile_linear(x, w)
-    if ops.rows_fit(x, w):
+    way = _way("whole", x, w)
+    if way == "rows":
         return ops.rows_linear(x, w)
+    if way == "tall":
+        return ops.rows_tall(x, w)
+    if way == "tile":
+        return ops.tile_linear(x, w)
     return ops.library_linear(x, w)
 
 
 def _linear_silu(x, w):
     """silu_mul of _linear."""
     if not _USE_SKINNY and not lt_autotune.enabled():
-        if w.shape[0] % 16 == 0 and ops.rows_fit(x, w):
+        way = _way("silu", x, w)
+        if way == "rows":
             return ops.rows_linear_silu(x, w)
-        if ops.tile_silu_fit(x, w):
+        if way == "tile":
             return ops.tile_linear_silu(x, w)
     return ops.silu_mul(_linear(x, w))
 
@@ -71,9 +78,10 @@ def _linear_silu(x, w):
 def _linear_parts(x, w):
     """_linear for a reader that sums parts (ops.rows_linear_parts)."""
     if not _USE_SKINNY and not lt_autotune.enabled():
-        if ops.tile_parts_fit(x, w):
+        way = _way("parts", x, w)
+        if way == "tile":
             return ops.tile_linear_parts(x, w)
-        if ops.rows_fit(x, w):
+        if way == "rows":
             return ops.rows_linear_parts(x, w)
     return _linear(x, w)
 
@@ -81,12 +89,13 @@ def _linear_parts(x, w):
 def _linear_relu2(x, w):
     """relu2 of _linear."""
     if not _USE_SKINNY and not lt_autotune.enabled():
-        if ops.rows_tall_fit(x, w):
-            return ops.rows_tall(x, w, relu2=True)
-        if ops.tile_relu2_fit(x, w):
-            return ops.tile_linear_relu2(x, w)
-        if ops.rows_fit(x, w) and ops.rows_whole(x, w):
+        way = _way("relu2", x, w)
+        if way == "rows":
             return ops.rows_linear_relu2(x, w)
+        if way == "tall":
+            return ops.rows_tall(x, w, relu2=True)
+        if way == "tile":
+            return ops.tile_linear_relu2(x, w)
     return ops.relu2(_linear(x, w))
 
 

@@ -365,8 +365,8 @@ class NesizenForCausalLM(MixedModel):
     def _last(self, x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
         """A sublayer's output; of few rows f32 parts where the kernel divides
         K and hyper_step is the one to read them."""
-        if (self.tp_world > 1 or not ops.rows_fit(x, w)
-                or ops.rows_whole(x, w)):
+        if (self.tp_world > 1 or not ops.product_operands(x, w)
+                or not ops.product_way("divided", x.shape[0], *w.shape)):
             return _linear(x, w)
         return _linear_parts(x, w)
 

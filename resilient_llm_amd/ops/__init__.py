@@ -755,6 +755,56 @@ def tile_linear_relu2(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     return torch.ops.rlli.tile_linear_relu2(x, w)
 
 
+@functools.lru_cache(maxsize=8192)
+def product_way(form: str, M: int, N: int, K: int) -> str | None:
+    """Which kernel of ours takes M rows by w [N, K] for a reader of ``form``
+    the fastest, of operands that product_operands: "rows", "tall" or "tile";
+    None: none of them.  Forms: whole, parts, silu, relu2, and divided, which is
+    parts where the kernel of few rows divides K and nothing else.  (Asked of
+    the *_fit of one kernel after the other, a product cost the host 6 to 8 us
+    ahead of its launch, and prompts of 12 mixed layers have 48.)"""
+    if M < 1 or N < 1 or K < 1 or K % 64:
+        return None
+    rows = M <= 128 and N % 4 == 0 and _rows_faster(M, N, K)
+    tiles = N % 16 == 0 and max(M, N) * K < 1 << 31
+    if form == "whole":
+        if tiles and _tall_faster(M, N, K):
+            return "tall"
+        if tiles and _tile_linear_faster(M, N, K):
+            return "tile"
+        return "rows" if rows else None
+    if form == "parts":
+        if tiles and _tile_parts_faster(M, N, K):
+            return "tile"
+        return "rows" if rows else None
+    if form == "divided":
+        _gpu()
+        return product_way("parts", M, N, K) if rows and not \
+            torch.ops.rlli.rows_whole_ok(M, N, K) else None
+    if form == "silu":
+        if rows and N % 16 == 0:
+            return "rows"
+        return "tile" if tiles and _tile_silu_faster(M, N, K) else None
+    if tiles and _tall_faster(M, N, K):
+        return "tall"
+    if tiles and _tile_relu2_faster(M, N, K):
+        return "tile"
+    if rows:
+        _gpu()
+        if torch.ops.rlli.rows_whole_ok(M, N, K):
+            return "rows"
+    return None
+
+
+def product_operands(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether x w^T is one that the kernels of product_way take."""
+    return (x.is_cuda and x.dtype == w.dtype == torch.bfloat16
+            and x.dim() == w.dim() == 2
+            and x.is_contiguous() and w.is_contiguous()
+            and (x.data_ptr() | w.data_ptr()) % 16 == 0
+            and not (x.requires_grad or w.requires_grad))
+
+
 def library_linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """F.linear(x, w), on the GPU in 16 bits without the library's search for
     its kernel at every call."""
@@ -819,12 +869,18 @@ _CPU_FORMS = {"rlli_attn": ref_attn, "rlli_mix": ref_mix,
               "rlli_blk": ref_blk, "rlli_rec": ref_rec, "rlli_lat": ref_lat}
 
 
+_spaces: dict = {}       # of the libraries that are loaded
+
+
 def _ns(lib: str, t: torch.Tensor):
     """The op namespace of ``lib`` for ``t``'s device."""
-    if t.is_cuda:
+    if not t.is_cuda:
+        return _CPU_FORMS[lib]
+    space = _spaces.get(lib)
+    if space is None:
         load_libraries((lib,))
-        return getattr(torch.ops, lib)
-    return _CPU_FORMS[lib]
+        space = _spaces[lib] = getattr(torch.ops, lib)
+    return space
 
 
 def _mix(t: torch.Tensor):

@@ -713,17 +713,21 @@ void by_kind(const GlaArgs& a, F f) {
 
 // The scan's operands in parts where the activations are 16-bit ones: fewer steps
 // of each chunk's chain, and half as many bytes more, which cost more than they
-// give where the chip is full (`many` heads; up to 128 wide, of many rows as well)
-// or few blocks stream `much`. Whole prompts, time in f32 over time in parts (heads
-// of all sequences and rows of each):
-//   64 x 64     512 heads 0.92; 64, 8000 rows 0.87; 256, 64 rows 1.17
-//   128 x 64    64, 512 rows 1.00, 2048 rows 0.78; 128, 512 rows 0.99, 2048 0.93;
-//               256 1.05 to 1.38; 512, 16 rows 1.12, 256 rows 0.91
-//   128 x 128   16, 2048 rows 1.15, 8000 rows 0.82; 64, 8000 rows 1.01; 128, 2048
-//               1.10; 256, 256 rows 1.10, 1024 rows 0.88
-//   256 x 256   128 heads 1.05; 256 0.76 to 0.84, and 512 and more 0.72 to 0.81
-//   256 x 128   128 heads 1.17; 256 0.77 to 0.88
-//   256 x 64    64, 512 rows 1.03, 2048 rows 0.83; 256 heads 1.11; 512 0.80 to 0.86
+// give where the chip is full (`many` heads) or few narrow blocks stream `much`.
+// Whole prompts, time in f32 over time in parts (heads of all sequences and rows of
+// each):
+//   64 x 64     512 heads 0.89; 64, 2000 rows 0.88; 16, 8000 rows 1.04; 256, 500
+//               rows 1.09
+//   64 x 128    16, 8000 rows 1.11; 64, 2000 rows 1.00; 256, 500 rows 0.98
+//   64 x 256    64, 2000 rows 1.25; 256, 500 rows 0.97
+//   128 x 64    64, 512 rows 0.91, 2048 rows 0.88; 128, 2048 rows 0.95
+//   128 x 128   16, 2048 rows 1.11, 8000 rows 1.14; 64, 2000 rows 1.08; 128, 1000
+//               rows 1.16; 256, 512 rows 1.01; 480, 500 rows 0.98; 512 0.91
+//   128 x 256   16, 7000 rows 1.14; 32, 3500 rows 1.29, 7000 rows 1.37; 256, 400
+//               rows 1.13; 512, 250 rows 1.14, 400 rows 1.04
+//   256 x 256   16, 8000 rows 1.23; 64 1.62; 128 1.07; 256 0.74
+//   256 x 128   16, 8000 rows 1.24; 64 1.40; 128 1.14; 256 0.77
+//   256 x 64    64, 2048 rows 1.04; 256 heads 1.03; 512 0.80 to 0.86
 bool gla_parts(const GlaArgs& a) {
   if (a.f32) return false;
   const int64_t sh = int64_t(a.n_seqs) * a.heads;
@@ -731,8 +735,9 @@ bool gla_parts(const GlaArgs& a) {
   if (a.dpad <= 64 && blocks >= 512) return false;
   const bool many = sh > 128 && blocks >= 512;
   const bool much = int64_t(a.rows) * a.heads >= (sh < 512 ? 3 << 15 : 3 << 14);
-  if (a.dpad > 128) return !(many || (much && blocks <= 64));
-  return !(much && (many || blocks <= 128));
+  if (a.dpad > 128) return !many;
+  if (a.vdim <= 64) return !(much && (many || blocks <= 128));
+  return !(much && many && a.vdim <= 128);
 }
 
 void launch_gla_decode(const GlaArgs& a, hipStream_t st) {

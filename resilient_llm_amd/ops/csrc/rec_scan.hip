@@ -29,6 +29,7 @@
 
 #include "rec_math.h"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace rlli {
@@ -372,18 +373,24 @@ void rec_scan_kernel(ScanArgs a, bool vec_q, bool vec_v) {
 // add up to it, so that products run on the 16-bit matrix cores: three for each of
 // the values', six for queries and state.  The three that are left out are up to
 // 2^-21 of a product, 2^-24 in the mean, always towards zero.  Four waves carry the
-// state from chunk to chunk (w every fourth of its key tiles), four others have the
+// state from chunk to chunk (w MD of its key tiles), four others have the
 // outputs (w the rows of a sub-chunk) of the chunk that the state is carried over,
 // from its parts in LDS.  LDS has two copies of parts and values, written by turns,
-// so that a chunk takes one barrier.  What bounds it is a chunk's chain of
-// latencies, 2.4 us (asked for a chunk ahead of their turn, operands take 3 us of
-// 80 off and twice the registers).  4 sequences of 1.9k, 8 heads of 128 x 256: 133
-// us with f32 products, of which these 67, and 80 now, by itself (in a step's call
-// 110); the kernel that makes the operands 49 and 50 (with infinite numbers' parts
-// NaN, 3 us less each).  Against 64 bits, 2048 tokens, the state is off by 4.3e-7
-// and 2.6e-7, as it is rounded less often; 6e-4 and 4e-4 of the outputs are not the
-// nearest 16-bit number.
-template <int VT, int MD, bool FULL>
+// so that a chunk takes one barrier.  What bounds it is that each workgroup loads
+// 120 KB a chunk, which takes as long as its products and LDS: a fragment's next
+// load comes right behind its last product, so that loads go out between products
+// and not all at once with all waves waiting to issue them, and loads ahead of the
+// loop come in the loop's order, as the waits in it are for both.  Operands that no
+// cache holds any more come slower; TOUCH: each of the slices that read them asks
+// for its share of their lines a chunk ahead.  (In a step's call, 8 heads of 128 x
+// 256, us, loads together behind the products and now: 1 sequence of 2600 70 and
+// 57, 3 of 2000 105 and 73, 4 of 2000 111 and 80, 8 of 900 77 and 63, 16 of 500 92
+// and 83; asked for two chunks ahead 62, 76, 84, 64 and 93.)  4 sequences of 1.9k
+// with f32 products 133 us, of which these 67; the kernel that makes the operands 49
+// and 50 (with infinite numbers' parts NaN, 3 us less each).  Against 64 bits, 2048
+// tokens, the state is off by 4.3e-7 and 2.6e-7, as it is rounded less often; 6e-4
+// and 4e-4 of the outputs are not the nearest 16-bit number.
+template <int VT, int MD, bool FULL, bool TOUCH>
 __global__ __launch_bounds__(512, 2)
 void rec_scan_parts_kernel(ScanArgs a, bool vec_v) {
   using T = uint16_t;
@@ -430,68 +437,110 @@ void rec_scan_parts_kernel(ScanArgs a, bool vec_v) {
       for (int nt = 0; nt < VT; ++nt)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const int d = (i * 4 + w) * 16 + g * 4 + r;
+          const int d = (w * MD + i) * 16 + g * 4 + r;
           const int c = v0 + nt * 16 + lr;
           S[i][nt][r] = (!fresh && d < a.dim && c < a.cols)
                             ? state[int64_t(d) * a.vpad + c] : 0.f;
         }
-    auto load = [&](int t) {
+    // (tiles behind the last one have its operands, and nobody reads them)
+    auto tile_of = [&](int i) {
+      return FULL ? w * MD + i : min(w * MD + i, ndt - 1);
+    };
+    auto load_part = [&](int t, int ks, int p) {
       const uint16_t* k = static_cast<const uint16_t*>(a.kt) +
                           chunk(t) * ndt * 3072 + lane * 8;
+#pragma unroll
+      for (int i = 0; i < MD; ++i)
+        kr[i][ks][p] = frag(k + ((tile_of(i) * 2 + ks) * 3 + p) * 512);
+    };
+    auto load_dec = [&](int t) {
       const float* dec = a.dec + chunk(t) * DP;
 #pragma unroll
       for (int i = 0; i < MD; ++i)
-        if (FULL || i * 4 + w < ndt) {
+        dv[i] = *reinterpret_cast<const f32x4_t*>(dec + tile_of(i) * 16 +
+                                                  g * 4);
+    };
+    // two tiles are a fragment's two halves, an odd last one's second half zero
+    auto put = [&](int t) {
+      uint16_t* to = lds + (t & 1) * copy + lane * 8;
 #pragma unroll
-          for (int ks = 0; ks < 2; ++ks)
+      for (int i = 0; i < MD; i += 2) {
+        const int tile = w * MD + i;
+        if (!FULL && tile >= 2 * nks) break;
 #pragma unroll
-            for (int p = 0; p < 3; ++p)
-              kr[i][ks][p] =
-                  frag(k + (((i * 4 + w) * 2 + ks) * 3 + p) * 512);
-          dv[i] = *reinterpret_cast<const f32x4_t*>(
-              dec + (i * 4 + w) * 16 + g * 4);
+        for (int nt = 0; nt < VT; ++nt) {
+          uint2 part[2][3];
+          const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
+          three_parts(FULL || tile < ndt ? S[i][nt] : zero, part[0]);
+          if constexpr (MD > 1)
+            three_parts(FULL || tile + 1 < ndt ? S[i + 1][nt] : zero, part[1]);
+#pragma unroll
+          for (int p = 0; p < 3; ++p) {
+            uint16_t* at = to + ((tile / 2 * 3 + p) * VT + nt) * 512;
+            if constexpr (MD > 1)
+              *reinterpret_cast<uint4*>(at) =
+                  uint4{part[0][p].x, part[0][p].y, part[1][p].x,
+                        part[1][p].y};
+            else
+              *reinterpret_cast<uint2*>(at + tile % 2 * 4) = part[0][p];
+          }
         }
+      }
     };
-    auto put = [&](int t, int tile, int nt, const f32x4_t& v) {
-      uint2 part[3];
-      three_parts(v, part);
-      uint16_t* to = lds + (t & 1) * copy + lane * 8 + tile % 2 * 4;
-#pragma unroll
-      for (int p = 0; p < 3; ++p)
-        *reinterpret_cast<uint2*>(to + ((tile / 2 * 3 + p) * VT + nt) * 512) =
-            part[p];
+    // (TOUCH) a line of each chunk's operands
+    const char* line_at = nullptr;
+    int64_t line_step = 0;
+    uint32_t line = 0;
+    if constexpr (TOUCH) {
+      const int nk = ndt * 48, nq = nks * 96, all = nk + nq + 192;
+      const int i = min(int(blockIdx.y + gridDim.y * threadIdx.x), all - 1);
+      const void* p = i < nk ? a.kt : i < nk + nq ? a.qd : a.sc;
+      const int in = i < nk ? nk : i < nk + nq ? nq : 192;
+      const int at = i < nk ? i : i < nk + nq ? i - nk : i - nk - nq;
+      line_at = static_cast<const char*>(p) + (int64_t(h) * in + at) * 128;
+      line_step = int64_t(a.heads) * in * 128;
+    }
+    auto touch = [&](int t) {
+      if constexpr (!TOUCH) return;
+      asm volatile("" ::"v"(line));       // (it has landed)
+      line = *reinterpret_cast<const uint32_t*>(line_at + t * line_step);
     };
-    load(first);
-    if (!FULL && ndt % 2 && w == ndt % 4)  // (the last pair's second tile)
+    // (in the order that they come in in the loop, whose waits are for both)
+    touch(min(first + 1, last));
+    load_dec(first);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int t = 0; t < 2; ++t)
+    for (int p = 2; p >= 0; --p)
 #pragma unroll
-        for (int nt = 0; nt < VT; ++nt)
-          put(t, ndt, nt, f32x4_t{0.f, 0.f, 0.f, 0.f});
+      for (int ks = 0; ks < 2; ++ks) {
+        load_part(first, ks, p);
+        __builtin_amdgcn_sched_barrier(0);
+      }
     for (int t = first; t <= last; ++t) {
-#pragma unroll
-      for (int i = 0; i < MD; ++i)
-        if (FULL || i * 4 + w < ndt)
-#pragma unroll
-          for (int nt = 0; nt < VT; ++nt) put(t, i * 4 + w, nt, S[i][nt]);
+      put(t);
       __syncthreads();
       s16x8_t v[2][VT];
       values(t, v);
+      const int next = min(t + 1, last);  // (no load is conditional)
+      touch(min(t + 2, last));
 #pragma unroll
       for (int i = 0; i < MD; ++i)
 #pragma unroll
         for (int nt = 0; nt < VT; ++nt) S[i][nt] *= dv[i];
+      __builtin_amdgcn_sched_barrier(0);
+      load_dec(next);
 #pragma unroll
       for (int p = 2; p >= 0; --p)
 #pragma unroll
-        for (int ks = 0; ks < 2; ++ks)
+        for (int ks = 0; ks < 2; ++ks) {
 #pragma unroll
           for (int i = 0; i < MD; ++i)
-            if (FULL || i * 4 + w < ndt)
 #pragma unroll
-              for (int nt = 0; nt < VT; ++nt)
-                S[i][nt] = mma(kr[i][ks][p], v[ks][nt], S[i][nt]);
-      load(min(t + 1, last));             // (no load is conditional)
+            for (int nt = 0; nt < VT; ++nt)
+              S[i][nt] = mma(kr[i][ks][p], v[ks][nt], S[i][nt]);
+          __builtin_amdgcn_sched_barrier(0);
+          load_part(next, ks, p);
+        }
     }
 #pragma unroll
     for (int i = 0; i < MD; ++i)
@@ -499,7 +548,7 @@ void rec_scan_parts_kernel(ScanArgs a, bool vec_v) {
       for (int nt = 0; nt < VT; ++nt)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const int d = (i * 4 + w) * 16 + g * 4 + r;
+          const int d = (w * MD + i) * 16 + g * 4 + r;
           const int c = v0 + nt * 16 + lr;
           if (d < a.dim && c < a.cols)
             state[int64_t(d) * a.vpad + c] = S[i][nt][r];
@@ -507,67 +556,79 @@ void rec_scan_parts_kernel(ScanArgs a, bool vec_v) {
     return;
   }
 
-  constexpr int VQ = VS / 4;
   const int tid = threadIdx.x - 256;
   const int row_first = a.tiles[first];
   const int n_last = a.tiles[2 * a.n_tiles + last];
   s16x8_t qr[NKS][3], ar[2][3];
-  Raw4<T> vr[VT];                         // four columns of a row
+  // of the values, a lane stages four rows of VT columns
+  using VRow = std::conditional_t<
+      VT == 1, uint16_t, std::conditional_t<VT == 2, uint32_t, uint2>>;
+  VRow vr[4];
+  const int vrow = tid / 16 * 4, vcol = tid % 16 * VT;
   const T* vb = static_cast<const T*>(a.v) + h * a.vdim;
   auto row_of = [&](int t) { return row_first + (t - first) * C; };
   auto rows_of = [&](int t) { return t == last ? n_last : C; };
-  auto load_q = [&](int t) {
+  auto load_q = [&](int t, int ks) {
     const uint16_t* q = static_cast<const uint16_t*>(a.qd) +
-                        chunk(t) * nks * 6144 + (w * 192 + lane) * 8;
+                        chunk(t) * nks * 6144 + (w * 192 + lane) * 8 +
+                        (FULL ? ks : min(ks, nks - 1)) * 6144;
 #pragma unroll
-    for (int ks = 0; ks < NKS; ++ks)
-      if (FULL || ks < nks)
-#pragma unroll
-        for (int p = 0; p < 3; ++p) qr[ks][p] = frag(q + (ks * 12 + p) * 512);
+    for (int p = 0; p < 3; ++p) qr[ks][p] = frag(q + p * 512);
   };
-  auto load_a = [&](int t) {
+  auto load_a = [&](int t, int ks) {
     const uint16_t* sc = static_cast<const uint16_t*>(a.sc) +
                          chunk(t) * 12288 + (w * 384 + lane) * 8;
 #pragma unroll
-    for (int ks = 0; ks < 2; ++ks)         // (a pair behind w: not used)
-#pragma unroll
-      for (int p = 0; p < 3; ++p)
-        ar[ks][p] = frag(sc + (min(ks, w / 2) * 3 + p) * 512);
+    for (int p = 0; p < 3; ++p)            // (a pair behind w: not used)
+      ar[ks][p] = frag(sc + (min(ks, w / 2) * 3 + p) * 512);
   };
   auto load_v = [&](int t) {
-    const int row0 = row_of(t), n = rows_of(t);
+    const int row0 = row_of(t), n = rows_of(t), c = v0 + vcol;
 #pragma unroll
-    for (int i = 0; i < VT; ++i) {
-      const int e = i * 256 + tid;
-      const int r = e / VQ, c = v0 + e % VQ * 4;
-      if constexpr (FULL)
-        vr[i].load(vb + int64_t(row0 + min(r, n - 1)) * a.v_stride + c);
-      else
-        vr[i] = raw_guard(vb + int64_t(row0 + r) * a.v_stride, c, a.vdim,
-                          r < n, vec_v);
+    for (int i = 0; i < 4; ++i) {
+      const int r = min(vrow + i, n - 1);
+      const T* p = vb + int64_t(row0 + r) * a.v_stride + c;
+      if (FULL || (vec_v && c < a.vdim)) {
+        vr[i] = *reinterpret_cast<const VRow*>(p);
+      } else {
+        T v[VT];
+#pragma unroll
+        for (int k = 0; k < VT; ++k) v[k] = c + k < a.vdim ? p[k] : T(0);
+        __builtin_memcpy(&vr[i], v, sizeof v);
+      }
     }
   };
   load_v(first);
-  load_q(first);
-  load_a(first);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int ks = 0; ks < NKS; ++ks) {
+    load_q(first, ks);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+#pragma unroll
+  for (int ks = 0; ks < 2; ++ks) {
+    load_a(first, ks);
+    __builtin_amdgcn_sched_barrier(0);
+  }
   for (int t = first; t <= last; ++t) {
     const int next = min(t + 1, last);     // (no load is conditional)
     const int row0 = row_of(t), n = rows_of(t);
     const uint16_t* Sl = lds + (t & 1) * copy + lane * 8;
-    uint16_t* Vl = lds + (t & 1) * copy + nks * 3 * VT * 512;
+    // (down a column, as the products take it)
+    uint16_t* staged = lds + (t & 1) * copy + nks * 3 * VT * 512 +
+                       (vrow / 32 * VT + vcol / 16) * 512 +
+                       (vrow % 16 * 4 + vcol % 16) * 8 + vrow / 16 % 2 * 4;
+    T v[4][VT];
 #pragma unroll
-    for (int i = 0; i < VT; ++i) {
-      const int e = i * 256 + tid;
-      const int r = e / VQ, c = e % VQ * 4;
-      const uint2 v = r < n ? vr[i].r : uint2{0, 0};
-      // down a column, as the products take it
-      uint16_t* to = Vl + (r / 32 * VT + c / 16) * 512 +
-                     ((r % 16 / 4) * 16 + c % 16) * 8 + r / 16 % 2 * 4 + r % 4;
-      to[0] = uint16_t(v.x);
-      to[8] = uint16_t(v.x >> 16);
-      to[16] = uint16_t(v.y);
-      to[24] = uint16_t(v.y >> 16);
+    for (int i = 0; i < 4; ++i) {
+      const VRow row = vrow + i < n ? vr[i] : VRow{};
+      __builtin_memcpy(v[i], &row, sizeof row);
     }
+#pragma unroll
+    for (int k = 0; k < VT; ++k)
+      *reinterpret_cast<uint2*>(staged + k * 8) =
+          uint2{uint32_t(v[0][k]) | uint32_t(v[1][k]) << 16,
+                uint32_t(v[2][k]) | uint32_t(v[3][k]) << 16};
     load_v(next);
     __syncthreads();
     f32x4_t o[2][VT];
@@ -576,52 +637,64 @@ void rec_scan_parts_kernel(ScanArgs a, bool vec_v) {
       o[0][nt] = o[1][nt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int ks = 0; ks < NKS; ++ks) {
-      if (!FULL && ks >= nks) continue;
-      s16x8_t s[3][VT];
+      if (FULL || ks < nks) {
+        s16x8_t s[3][VT];
 #pragma unroll
-      for (int p = 0; p < 3; ++p)
+        for (int p = 0; p < 3; ++p)
 #pragma unroll
-        for (int nt = 0; nt < VT; ++nt)
-          s[p][nt] = frag(Sl + ((ks * 3 + p) * VT + nt) * 512);
-      auto both = [&](int acc, int x, int y) {
+          for (int nt = 0; nt < VT; ++nt)
+            s[p][nt] = frag(Sl + ((ks * 3 + p) * VT + nt) * 512);
+        auto both = [&](int acc, int i, int j) {
 #pragma unroll
-        for (int nt = 0; nt < VT; ++nt)
-          o[acc][nt] = mma(qr[ks][x], s[y][nt], o[acc][nt]);
-      };
-      both(0, 0, 2);
-      both(1, 2, 0);
-      both(0, 1, 1);
-      both(1, 1, 0);
-      both(0, 0, 0);
-      both(1, 0, 1);
+          for (int nt = 0; nt < VT; ++nt)
+            o[acc][nt] = mma(s[j][nt], qr[ks][i], o[acc][nt]);
+        };
+        both(0, 0, 2);
+        both(1, 2, 0);
+        both(0, 1, 1);
+        both(1, 1, 0);
+        both(0, 0, 0);
+        both(1, 0, 1);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      load_q(next, ks);
     }
-    load_q(next);
-    s16x8_t v[2][VT];
-    values(t, v);
+    s16x8_t vs[2][VT];
+    values(t, vs);
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) {
-      if (ks > w / 2) break;
+      if (ks <= w / 2)
 #pragma unroll
-      for (int p = 2; p >= 0; --p)
+        for (int p = 2; p >= 0; --p)
 #pragma unroll
-        for (int nt = 0; nt < VT; ++nt)
-          o[p > 0][nt] = mma(ar[ks][p], v[ks][nt], o[p > 0][nt]);
+          for (int nt = 0; nt < VT; ++nt)
+            o[p > 0][nt] = mma(vs[ks][nt], ar[ks][p], o[p > 0][nt]);
+      __builtin_amdgcn_sched_barrier(0);
+      load_a(next, ks);
     }
-    load_a(next);
+    // a lane has four columns of row lr of the sub-chunk
+    const int tr = w * 16 + lr;
+    auto out_row = [&](int row) {
+      return a.o + (int64_t(row) * a.heads + h) * a.opad;
+    };
+    float* to = out_row(tr < n ? row0 + tr : a.n_rows + tr) + v0 + g * 4;
 #pragma unroll
-    for (int nt = 0; nt < VT; ++nt)
+    for (int nt = 0; nt < VT; ++nt) {
+      const f32x4_t v = o[0][nt] + o[1][nt];
+      if constexpr (FULL)
+        *reinterpret_cast<f32x4_t*>(to + nt * 16) = v;
+      else
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int tr = w * 16 + g * 4 + r, c = v0 + nt * 16 + lr;
-        const bool ok = tr < n && (FULL || c < a.cols);
-        a.o[(int64_t(ok ? row0 + tr : a.n_rows + tr) * a.heads + h) * a.opad +
-            (ok ? c : 0)] = o[0][nt][r] + o[1][nt][r];
-      }
+        for (int r = 0; r < 4; ++r) {
+          const int c = v0 + nt * 16 + g * 4 + r;
+          *(c < a.cols ? to + nt * 16 + r : out_row(a.n_rows + tr)) = v[r];
+        }
+    }
   }
 }
 
 template <int VT>
-void scan_parts(const ScanArgs& a, hipStream_t st) {
+void scan_parts(const ScanArgs& a, bool touch, hipStream_t st) {
   constexpr int VS = VT * 16;
   const int nks = (a.dpad / 16 + 1) / 2;
   const size_t smem = size_t(2) * (nks * 3 + 2) * VT * 1024;
@@ -636,11 +709,18 @@ void scan_parts(const ScanArgs& a, hipStream_t st) {
                        dim3(512), smem, st, a, vec_v);
   };
   const bool full = vec_v && a.vdim % VS == 0;
-  if (full && a.dim == 64) run(rec_scan_parts_kernel<VT, 1, true>);
-  else if (full && a.dim == 128) run(rec_scan_parts_kernel<VT, 2, true>);
-  else if (a.dpad <= 64) run(rec_scan_parts_kernel<VT, 1, false>);
-  else if (a.dpad <= 128) run(rec_scan_parts_kernel<VT, 2, false>);
-  else if constexpr (VT < 4) run(rec_scan_parts_kernel<VT, 4, false>);
+  auto go = [&](auto md) {
+    constexpr int MD = decltype(md)::value;
+    if (!full || a.dim != MD * 64)
+      run(rec_scan_parts_kernel<VT, MD, false, false>);
+    else if (touch)
+      run(rec_scan_parts_kernel<VT, MD, true, true>);
+    else
+      run(rec_scan_parts_kernel<VT, MD, true, false>);
+  };
+  if (a.dpad <= 64) go(std::integral_constant<int, 1>{});
+  else if (a.dpad <= 128) go(std::integral_constant<int, 2>{});
+  else if constexpr (VT < 4) run(rec_scan_parts_kernel<VT, 4, false, false>);
 }
 
 template <typename T, int MODE, int VT>
@@ -684,16 +764,28 @@ void scan(const ScanArgs& a, hipStream_t st) {
   const int64_t sh = int64_t(a.n_seqs) * a.heads;
   if constexpr (MODE == kScanPlain && sizeof(T) == 2)
     if (a.parts) {
-      // as wide slices as leave a workgroup for each CU (two copies of 256 rows
-      // by 64 columns do not fit LDS; whole prompts, us, slices of 16, 32 and 64
-      // columns: heads of 128 x 256, 8 of them 97 105 141, 16 113 119 151, 32 190
-      // 158 183, 64 195 163 141)
-      if (a.dpad <= 128 && sh * ((a.vdim + 63) / 64) >= 256)
-        scan_parts<4>(a, st);
-      else if (sh * ((a.vdim + 31) / 32) >= 256)
-        scan_parts<2>(a, st);
-      else
-        scan_parts<1>(a, st);
+      // A CU has one workgroup, which takes the longer the wider its slice is.
+      // (us, slices of 16, 32 and 64 columns: heads of 128 x 256, 1000 tokens,
+      // 16 of them 34 38 50, 24 60 42 55, 32 67 46 59, 40 98 82 62, 64 of 900
+      // 134 88 64; of 64 x 64, 64 of them 33 40 41, 80 61 43 44.  Two copies of
+      // 256 rows by 64 columns do not fit LDS.)
+      auto groups = [&](int cols) { return sh * ((a.vdim + cols - 1) / cols); };
+      auto cost = [&](int cols, int each) {
+        return (groups(cols) + 255) / 256 * each;
+      };
+      const int64_t one = cost(16, 6), two = cost(32, 7);
+      const int cols = a.dpad <= 128 && cost(64, 9) < std::min(one, two) ? 64
+                       : two < one                                       ? 32
+                                                                         : 16;
+      // From some 60 MB of operands on, if all workgroups run at once (in a
+      // step's call, us without and with, heads of 128 x 256: 1 sequence of 2600
+      // 57 59, 2 of 2000 57 57, 3 80 73, 4 102 80, 8 of 900 65 63; 16 of 500,
+      // which take turns, 83 93).
+      const bool touch = int64_t(a.n_tiles) * a.heads * a.dpad >= 65536 &&
+                         groups(cols) <= 256;
+      if (cols == 64) scan_parts<4>(a, touch, st);
+      else if (cols == 32) scan_parts<2>(a, touch, st);
+      else scan_parts<1>(a, touch, st);
       return;
     }
   if (a.vdim > 32 && sh * ((a.vdim + 63) / 64) >= 512)

@@ -104,6 +104,11 @@ def test_lanes_and_rows(dim, vdim, rank, dtype):
     # tiles down the columns
     (2, 3, 128, 48), (2, 3, 40, 33), (2, 64, 40, 33), (2, 64, 64, 32),
     (2, 64, 130, 40), (2, 64, 128, 128), (2, 64, 24, 97), (2, 64, 72, 70),
+    # as many slices of 16, 32 and 64 columns as there are CUs, and one more head
+    (2, 8, 128, 256), (2, 9, 64, 256), (2, 16, 128, 256), (2, 17, 128, 250),
+    (2, 33, 64, 256), (1, 3, 256, 64), (2, 24, 256, 96), (2, 5, 144, 64),
+    # some 60 MB of operands and all slices at once; more slices than CUs
+    (2, 104, 128, 64), (4, 86, 96, 48), (4, 72, 128, 80),
     # short heads that fill the chip: f32 operands
     (4, 128, 16, 20), (4, 128, 64, 64)])
 def test_prompts_by_slices(seqs, H, dim, vdim):
@@ -124,6 +129,30 @@ def test_prompts_by_slices(seqs, H, dim, vdim):
         assert rel(rows, want[:n]) < tol(BF16)
     assert rel(st[0, :, :, :vdim], S) < 1e-5
     assert torch.isnan(st[seqs]).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("seqs,H,dim,vdim", [
+    (16, 2, 128, 128), (16, 2, 128, 256), (32, 2, 64, 64)])
+def test_prompts_of_many_operands(seqs, H, dim, vdim):
+    """Some 60 MB of a scan's operands, which each slice asks for its share of
+    ahead of time: chunk counts that are even, odd and one."""
+    lens = [1024] * seqs
+    lens[1], lens[2], lens[3] = 1023, 900, 1
+    lens[4:4] = [80] * 3
+    *inputs, eps, want, S = gla_case(1024, H, dim, vdim, 8, 8.0, 1.0, dim, BF16)
+    proj, a2, b, norm = (t.cuda() for t in inputs)
+    st = torch.full((len(lens), H, dim, vdim), float("nan"), device="cuda")
+    portions, at = [], 0
+    for i, n in enumerate(lens):
+        portions.append(Portion(at, 0, n, i, i))
+        at += n
+    got = ops.gla_prefill(torch.cat([proj[:n] for n in lens]), a2, b, norm,
+                          st, PromptRows(portions, "cuda"), vdim, 8.0, eps)
+    for i, (n, rows) in enumerate(zip(lens, got.split(lens))):
+        assert rel(rows, want[:n]) < tol(BF16)
+        if n == 1024:
+            assert rel(st[i], S) < 1e-5
 
 
 @pytest.mark.gpu

@@ -562,11 +562,6 @@ def _tall_faster(M: int, N: int, K: int) -> bool:
     return 1536 <= N <= 2048 and M <= 384
 
 
-def rows_tall_fit(x: torch.Tensor, w: torch.Tensor) -> bool:
-    """Whether rows_tall takes x w^T and is the faster way."""
-    return _tiles_take(x, w, _tall_faster)
-
-
 def rows_tall(x: torch.Tensor, w: torch.Tensor,
               relu2: bool = False) -> torch.Tensor:
     """x w^T of some hundred rows, or relu2 of that."""

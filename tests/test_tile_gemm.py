@@ -199,3 +199,28 @@ def test_unaligned_operands_are_refused():
     assert not ops.tile_parts_fit(x, w) and not ops.tile_silu_fit(x, w)
     with pytest.raises(RuntimeError, match="multiples of 16"):
         torch.ops.rlli.tile_linear_parts(x, w)
+
+
+@pytest.mark.parametrize("N,K", [(4096, 4096), (6144, 2048), (2048, 6144),
+                                 (28672, 4096), (8192, 2048), (260, 3136),
+                                 (4080, 1024), (4096, 96)])
+def test_the_way_is_that_of_the_rules(N, K):
+    w = torch.empty(N, K, dtype=torch.bfloat16, device=DEV)
+    for M in (1, 48, 64, 65, 96, 128, 129, 160, 256, 257, 600, 1024, 7000):
+        x = torch.empty(M, K, dtype=torch.bfloat16, device=DEV)
+        rows = ops.rows_fit(x, w)
+        tall = ops._tiles_take(x, w, ops._tall_faster)
+        whole, parts, silu, relu2 = (
+            ops.product_way(form, M, N, K)
+            for form in ("whole", "parts", "silu", "relu2"))
+        tile = ops.tile_linear_fit(x, w)
+        assert whole == ("tall" if tall else "tile" if tile
+                         else "rows" if rows else None)
+        assert parts == ("tile" if ops.tile_parts_fit(x, w)
+                         else "rows" if rows else None)
+        assert silu == ("rows" if rows and N % 16 == 0
+                        else "tile" if ops.tile_silu_fit(x, w) else None)
+        assert relu2 == ("tall" if tall
+                         else "tile" if ops.tile_relu2_fit(x, w)
+                         else "rows" if rows and ops.rows_whole(x, w)
+                         else None)

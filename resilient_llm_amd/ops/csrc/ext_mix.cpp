@@ -203,8 +203,10 @@ Tensor moe_run(rlli::MoeArgs& a, const Tensor& h, Tensor& ids, Tensor& w) {
   // 253, 540 158 and 175 for 16 experts, 640 310 and 339, 1024 408 and 435.)
   a.together = a.tile_m == 256 && !few && each >= 256 && each % 256 >= 32 &&
                each % 256 <= 120;
-  // (beyond, an expert's weights are read by more than one row of tiles)
-  a.spread = each <= 256;
+  // (beyond, an expert's weights are read by more than one row of tiles: as above,
+  // 258 rows an expert 180 and 168 us, 264 191 and 179, 275 204 and 189, 287 216 and
+  // 198, 312 192 and 192, 350 190 and 192)
+  a.spread = each <= 300;
   a.max_tiles = int(P / a.tile_m + std::min<int64_t>(a.experts, P));
   auto io = h.options().dtype(at::kInt);
   ids = at::empty({a.rows, a.top}, io);

@@ -597,7 +597,8 @@ DEV_INLINE void moe_tile(const MoeArgs& a, int rows, int e, int p0, int nb) {
   // without and with, for all of it: 32 experts of 1024 by 2048, four each, 400
   // rows 116 and 97, 1000 127 and 113, 2000 167 and 154; 16 of 3584 by 4096, two
   // each, 400 rows 287 and 270, 2000 468 and 440; but 64 of 1024 by 1024 102 and
-  // 108; more than a tile an expert, 32 of 1024 by 2048, 6001 rows 320 and 324.)
+  // 108; some more tiles than experts, 32 of 1024 by 2048, 2115 rows 191 and 179, but
+  // three times as many, 6001 rows, 320 and 324.)
   P p;
   p.rows(
       [&](int r) {

@@ -17,11 +17,12 @@ COUNTS = [
     # of 256 rows
     [128, 129, 127, 0, 1, 256, 257, 2600],
     [384, 385, 383, 640, 0, 1281, 900, 255],
+    [256, 257, 300, 290, 512, 1, 255, 529],
 ]
 
 
 @pytest.mark.gpu
-# (from 2048 on, up to 256 rows an expert, blocks of w start K at their own steps)
+# (from 2048 on, up to 300 rows an expert, blocks of w start K at their own steps)
 @pytest.mark.parametrize("W,ff", [(320, 192), (64, 1152), (2112, 192),
                                   (64, 2112)])
 @pytest.mark.parametrize("counts", COUNTS, ids=str)

@@ -72,15 +72,33 @@ struct DecodeArgs {
   bool apart;              // whoever reads the parts puts them together
 };
 
+// Sums of the lanes up to each; all lanes at once.  (On the VALU: fourteen steps
+// through LDS ahead of everything else were 0.5 us.)
+DEV_INLINE int sums_upto(int v) {
+  auto add = [&](auto ctrl, auto rows) {
+    v += __builtin_amdgcn_update_dpp(0, v, decltype(ctrl)::value,
+                                     decltype(rows)::value, 0xf, false);
+  };
+  using All = std::integral_constant<int, 0xf>;
+  add(std::integral_constant<int, 0x111>{}, All{});     // row_shr 1, 2, 4, 8
+  add(std::integral_constant<int, 0x112>{}, All{});
+  add(std::integral_constant<int, 0x114>{}, All{});
+  add(std::integral_constant<int, 0x118>{}, All{});
+  // the row before's last to rows 1 and 3, the lower half's to the upper
+  add(std::integral_constant<int, 0x142>{}, std::integral_constant<int, 0xa>{});
+  add(std::integral_constant<int, 0x143>{}, std::integral_constant<int, 0xc>{});
+  return v;
+}
+
 // How many units a part may have, so that ``shares`` parts cover all
 // sequences (each ends in one that is not full).
-DEV_INLINE int part_size(const DecodeArgs& a) {
-  int t = 0;
-  for (int s = threadIdx.x & 63; s < a.batch; s += 64)
+// (``own``: the length of the lane's sequence, of the first 64; or 0.)
+DEV_INLINE int part_size(const DecodeArgs& a, int own) {
+  int t = units_of(own);
+  for (int s = (threadIdx.x & 63) + 64; s < a.batch; s += 64)
     t += units_of(a.seq_lens[s]);
-#pragma unroll
-  for (int d = 1; d < 64; d <<= 1) t += __shfl_xor(t, d, kWave);
-  return part_size_of(__builtin_amdgcn_readfirstlane(t), a.shares, a.batch);
+  return part_size_of(__builtin_amdgcn_readlane(sums_upto(t), 63), a.shares,
+                      a.batch);
 }
 
 // Parts of the sequences ahead of ``seq``.
@@ -88,36 +106,30 @@ DEV_INLINE int parts_before(const DecodeArgs& a, int size, int seq) {
   int t = 0;
   for (int s = threadIdx.x & 63; s < seq; s += 64)
     t += parts_of(a.seq_lens[s], size);
-#pragma unroll
-  for (int d = 1; d < 64; d <<= 1) t += __shfl_xor(t, d, kWave);
-  return __builtin_amdgcn_readfirstlane(t);
+  return __builtin_amdgcn_readlane(sums_upto(t), 63);
 }
 
-// The sequence that part number ``part`` belongs to (a.batch: none) and
-// which of its parts it is.
-DEV_INLINE int find_part(const DecodeArgs& a, int size, int part, int& rel) {
+// The sequence that part number ``part`` belongs to (a.batch: none), its length
+// and which of its parts it is.
+DEV_INLINE int find_part(const DecodeArgs& a, int own, int size, int part,
+                         int& len, int& rel) {
   const int lane = threadIdx.x & 63;
   int before = 0;
   for (int s0 = 0; s0 < a.batch; s0 += 64) {
-    const int mine =
-        s0 + lane < a.batch ? parts_of(a.seq_lens[s0 + lane], size) : 0;
-    int upto = mine;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-      const int t = __shfl_up(upto, d, kWave);
-      if (lane >= d) upto += t;
-    }
+    if (s0 > 0) own = s0 + lane < a.batch ? a.seq_lens[s0 + lane] : 0;
+    const int mine = parts_of(own, size);
+    const int upto = sums_upto(mine);
     const int at = part - before;
     const uint64_t hit = __ballot(at < upto && at >= upto - mine);
     if (hit) {
-      const int src = __ffsll(static_cast<unsigned long long>(hit)) - 1;
-      rel = __builtin_amdgcn_readfirstlane(
-          at - __shfl(upto - mine, src, kWave));
-      return __builtin_amdgcn_readfirstlane(s0 + src);
+      const int src = __builtin_amdgcn_readfirstlane(__builtin_ctzll(hit));
+      rel = at - __builtin_amdgcn_readlane(upto - mine, src);
+      len = __builtin_amdgcn_readlane(own, src);
+      return s0 + src;
     }
-    before += __shfl(upto, 63, kWave);
+    before += __builtin_amdgcn_readlane(upto, 63);
   }
-  rel = 0;
+  len = rel = 0;
   return a.batch;
 }
 
@@ -242,25 +254,29 @@ DEV_INLINE void attend(const DecodeArgs& a, unsigned block,
     return k / KPL * 32 * KPL + (oct * KPL + k % KPL) * 8;
   };
 
-  int kvh, seq, part = 0, u0 = 0, u1, n_parts = 1;
+  int kvh, seq, len, part = 0, u0 = 0, u1, n_parts = 1;
   kvh = block % a.n_kv;
   if (cut) {
     part = block / a.n_kv;
-    const int size = part_size(a);
+    const int own = lane < a.batch ? a.seq_lens[lane] : 0;
+    const int size = part_size(a, own);
     int rel;
-    seq = find_part(a, size, part, rel);
+    seq = find_part(a, own, size, part, len, rel);
     if (seq >= a.batch) return;
-    const int all = units_of(a.seq_lens[seq]);
-    n_parts = parts_of(a.seq_lens[seq], size);
+    const int all = units_of(len);
+    n_parts = parts_of(len, size);
     u0 = all * rel / n_parts;
     u1 = all * (rel + 1) / n_parts;
   } else {
     seq = block / a.n_kv;
-    u1 = units_of(a.seq_lens[seq]);
+    len = a.seq_lens[seq];
+    u1 = units_of(len);
   }
-  const int len = a.seq_lens[seq];
   // whether this workgroup appends the new token
   const bool newest = FUSED && a.slot_mapping && u1 == units_of(len);
+  // what later loads and stores go by
+  const int position = FUSED ? a.positions[seq] : 0;
+  const int slot_at = newest ? a.slot_mapping[seq] : 0;
 
   const int32_t* table = a.block_table + int64_t(seq) * a.max_blocks;
   const int last = len - 1;
@@ -321,31 +337,65 @@ DEV_INLINE void attend(const DecodeArgs& a, unsigned block,
             vc + row_of(u, t, 1 + i, value_tok(u, t, i)) * D + col * VT));
   };
   look_up(u0 + wave);
-  load_keys(u0 + wave);
-  load_values(u0 + wave);
-  look_up(u0 + wave + NW);
-
   // ---- the heads' queries (and the new key and value) -----------------
+  // All that a lane takes of them is asked for at once, ahead of keys and values.
+  // (Part after part, then the position, the rotation and the slot are four to
+  // eight waits more, one behind the other.  us, with sums over lanes through LDS
+  // and now: one sequence of 101 tokens, 64-wide heads, five parts 5.7 and 4.9; of
+  // 1000, 128-wide, two parts 7.4 and 6.8; 64 of 192 10.7 and 10.3; 16 of 1.7k to
+  // 4.1k 30.7 and 30.1; 37 of 1k to 2k with an 8-bit cache 21.2 and 20.3.)
+  constexpr int EARLY = 8;                 // parts of the product
   const int n_in = (GROUP + (newest ? 2 : 0)) * D;
-  for (int e = tid * 4; e < n_in; e += NT * 4) {
+  auto place = [&](int e) {
     int at = kvh * GROUP * D + e;
     if (e >= GROUP * D) {
       const int r = e - GROUP * D;
       at = r < D ? (n_q + kvh) * D + r : (n_q + a.n_kv + kvh) * D + r - D;
     }
+    return int64_t(seq) * a.q_stride + at;
+  };
+  const int64_t part_step = int64_t(a.batch) * a.q_stride;
+  f32x4 early[EARLY];
+  uint2 early_q{0, 0};
+  auto ask = [&](int e) {
+    if (a.parts) {
+      const float* p = a.parts + place(e);
+#pragma unroll
+      for (int s = 0; s < EARLY; ++s)
+        if (s < a.n_parts)
+          early[s] = *reinterpret_cast<const f32x4*>(p + s * part_step);
+    } else {
+      early_q = *reinterpret_cast<const uint2*>(a.q + place(e));
+    }
+  };
+  if (tid * 4 < n_in) ask(tid * 4);
+  // (a thread's channel is the same of all heads)
+  float cosine = 1.f, sine = 0.f;
+  if constexpr (FUSED) {
+    const float* cs = a.cos_sin + int64_t(position) * D + tid % (D / 2);
+    cosine = cs[0];
+    sine = cs[D / 2];
+  }
+  load_keys(u0 + wave);
+  load_values(u0 + wave);
+  look_up(u0 + wave + NW);
+
+  for (int e = tid * 4; e < n_in; e += NT * 4) {
+    if (e != tid * 4) ask(e);
     f32x4 v;
     if (a.parts) {
-      const float* p = a.parts + int64_t(seq) * a.q_stride + at;
-      const int64_t step = int64_t(a.batch) * a.q_stride;
-      v = *reinterpret_cast<const f32x4*>(p);
-      for (int s = 1; s < a.n_parts; ++s)
-        v += *reinterpret_cast<const f32x4*>(p + s * step);
+      v = early[0];
+#pragma unroll
+      for (int s = 1; s < EARLY; ++s)
+        if (s < a.n_parts) v += early[s];
+      const float* p = a.parts + place(e);
+      for (int s = EARLY; s < a.n_parts; ++s)
+        v += *reinterpret_cast<const f32x4*>(p + s * part_step);
       // the product is a 16-bit one
 #pragma unroll
       for (int i = 0; i < 4; ++i) v[i] = bf16_to_f32(f32_to_bf16(v[i]));
     } else {
-      const uint2 w = *reinterpret_cast<const uint2*>(
-          a.q + int64_t(seq) * a.q_stride + at);
+      const uint2 w = early_q;
       v = f32x4{__builtin_bit_cast(float, w.x << 16),
                 __builtin_bit_cast(float, w.x & 0xffff0000u),
                 __builtin_bit_cast(float, w.y << 16),
@@ -356,8 +406,7 @@ DEV_INLINE void attend(const DecodeArgs& a, unsigned block,
   lds_barrier();
   {
     constexpr int HALF = D / 2;
-    const float* cs =
-        FUSED ? a.cos_sin + int64_t(a.positions[seq]) * D : nullptr;
+    static_assert(NT % HALF == 0, "");
     auto store = [&](int h, int d, float v) {
       // All parts have the sign of the first, and none is zero, so that an
       // infinite key makes all of a score's parts infinite alike and not NaN.
@@ -374,9 +423,8 @@ DEV_INLINE void attend(const DecodeArgs& a, unsigned block,
       const float u = raw[h * D + j], v = raw[h * D + HALF + j];
       float x = u, y = v;
       if constexpr (FUSED) {
-        const float c = cs[j], s = cs[HALF + j];
-        x = u * c - v * s;
-        y = v * c + u * s;
+        x = fmaf(u, cosine, -(v * sine));
+        y = fmaf(v, cosine, u * sine);
       }
       if (h < GROUP) {
         store(h, j, x);
@@ -393,7 +441,7 @@ DEV_INLINE void attend(const DecodeArgs& a, unsigned block,
     if (tid < 2 * D / 8) {
       const int e = tid * 8;
       const vec8 w = KC::from_f32(raw + GROUP * D + e);
-      const int slot = a.slot_mapping[seq];
+      const int slot = slot_at;
       elem* to = static_cast<elem*>(e < D ? a.k_cache_w : a.v_cache_w);
       *reinterpret_cast<vec8*>(
           to + ((int64_t(slot / bs) * a.n_kv + kvh) * bs + slot % bs) * D +
@@ -601,7 +649,8 @@ DEV_INLINE void combine(const DecodeArgs& a, unsigned block) {
   const int n_q = a.n_kv * GROUP;
   const int seq = block / n_q, h = block % n_q;
   const int kvh = h / GROUP;
-  const int size = part_size(a);
+  const int lane = threadIdx.x & 63;
+  const int size = part_size(a, lane < a.batch ? a.seq_lens[lane] : 0);
   const int n = parts_of(a.seq_lens[seq], size);
   if (n == 1) return;
   const int first = parts_before(a, size, seq);

@@ -13,6 +13,8 @@ from __future__ import annotations
 import functools
 import os
 import torch
+from torch._C._functorch import peek_interpreter_stack
+from torch.autograd import forward_ad
 
 from . import ref  # noqa: F401
 
@@ -791,13 +793,24 @@ def product_way(form: str, M: int, N: int, K: int) -> str | None:
     return None
 
 
+_STORED = frozenset((torch.Tensor, torch.nn.Parameter))
+
+
+def _plain(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether x and w are tensors with memory, which those of a trace and in
+    vmap are not, and neither gradients nor tangents of x w^T are asked for."""
+    return (type(x) in _STORED and type(w) in _STORED
+            and not (x.requires_grad or w.requires_grad)
+            and forward_ad._current_level < 0
+            and peek_interpreter_stack() is None)
+
+
 def product_operands(x: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether x w^T is one that the kernels of product_way take."""
     return (x.is_cuda and x.dtype == w.dtype == torch.bfloat16
-            and x.dim() == w.dim() == 2
+            and x.dim() == w.dim() == 2 and _plain(x, w)
             and x.is_contiguous() and w.is_contiguous()
-            and (x.data_ptr() | w.data_ptr()) % 16 == 0
-            and not (x.requires_grad or w.requires_grad))
+            and (x.data_ptr() | w.data_ptr()) % 16 == 0)
 
 
 def library_linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
@@ -805,9 +818,9 @@ def library_linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     its kernel at every call."""
     if (x.is_cuda and x.dim() == w.dim() == 2
             and x.dtype == w.dtype == torch.bfloat16
+            and _plain(x, w) and not torch.is_autocast_enabled()
             and x.device == w.device and x.shape[1] == w.shape[1]
-            and x.is_contiguous() and w.is_contiguous()
-            and not (x.requires_grad or w.requires_grad)):
+            and x.is_contiguous() and w.is_contiguous()):
         _gpu()
         return torch.ops.rlli.library_linear(x, w)
     return torch.nn.functional.linear(x, w)

@@ -7,8 +7,11 @@ import threading
 import pytest
 import torch
 import torch.nn.functional as F
+from torch._subclasses.fake_tensor import FakeTensorMode
+from torch.autograd import forward_ad
 
 from resilient_llm_amd import ops
+from resilient_llm_amd.models import llama
 
 DEV = "cuda:0"
 
@@ -86,3 +89,42 @@ def test_streams_and_threads():
     for t in threads:
         t.join()
     assert not wrong
+
+
+# rows that rows_tall, the library and (N not a multiple of 128) tiles take
+FORMS = [(200, 2048, 2048), (1000, 4096, 4096), (2048, 6160, 2048)]
+
+
+@pytest.mark.parametrize("M,N,K", FORMS)
+def test_sizes_of_a_trace(M, N, K):
+    """Tensors without memory, as of a trace and of vmap, go F.linear's way."""
+    with FakeTensorMode():
+        x = torch.empty(M, K, dtype=torch.bfloat16, device=DEV)
+        w = torch.empty(N, K, dtype=torch.bfloat16, device=DEV)
+        assert llama._linear(x, w).shape == (M, N)
+        many = torch.func.vmap(lambda a: llama._linear(a, w))(
+            x.expand(3, M, K))
+        assert many.shape == (3, M, N) and many.dtype == x.dtype
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", FORMS)
+def test_tangents(M, N, K):
+    x, w = operands(M, N, K)
+    t = torch.randn_like(x)
+    want = F.linear(t, w)
+    with forward_ad.dual_level():
+        y = llama._linear(forward_ad.make_dual(x, t), w)
+        tangent = forward_ad.unpack_dual(y).tangent
+    assert torch.equal(tangent, want)
+    y, tangent = torch.func.jvp(lambda a: llama._linear(a, w), (x,), (t,))
+    assert torch.equal(tangent, want)
+    close(y, x, w)
+
+
+@pytest.mark.gpu
+def test_autocast():
+    x, w = operands(130, 640, 1000)
+    with torch.autocast("cuda", torch.float16):
+        got, want = ops.library_linear(x, w), F.linear(x, w)
+    assert got.dtype == want.dtype and torch.equal(got, want)

@@ -32,6 +32,7 @@
 
 #include <algorithm>
 #include <array>
+#include <cstdlib>
 #include <map>
 #include <memory>
 #include <mutex>
@@ -141,7 +142,10 @@ Tensor lt_heuristics(const Tensor& x, const Tensor& w, int64_t max_n) {
 // ---- the library's own choice, without looking for it at every call ------
 // at::linear asks the library for its pick at each call: 18 us of the host,
 // of which 8 are spared by keeping what was found for a shape (a prompt of 165
-// rows through 16 layers of 2048 has 31 such products).
+// rows through 16 layers of 2048 has 31 such products).  The pick may have the
+// workspace that at::linear's may, and a process that sets that itself has no plans.
+// (One in which plans had up to 128 MiB and at::linear 64 KiB faulted the GPU at its
+// first product of either; the cause was not found.)
 struct LibraryPlan {
   hipblasLtMatmulDesc_t product = nullptr;
   hipblasLtMatrixLayout_t w = nullptr, x = nullptr, y = nullptr;
@@ -152,7 +156,7 @@ struct LibraryPlan {
   LibraryPlan(int64_t M, int64_t N, int64_t K) {
     const hipblasOperation_t t = HIPBLAS_OP_T, n = HIPBLAS_OP_N;
     hipblasLtMatmulPreference_t pref = nullptr;
-    const size_t most = kWorkspaceBytes;
+    const size_t most = at::cuda::getCUDABlasLtWorkspaceSize();
     hipblasLtMatmulHeuristicResult_t result{};
     int count = 0;
     auto ok = [](hipblasStatus_t s) { return s == HIPBLAS_STATUS_SUCCESS; };
@@ -186,19 +190,40 @@ struct LibraryPlan {
   }
 };
 
+// Whether the process sets the library's workspace itself
+bool own_workspace() {
+  static const bool own = std::getenv("HIPBLASLT_WORKSPACE_SIZE") ||
+                          std::getenv("CUBLASLT_WORKSPACE_SIZE");
+  return own;
+}
+
 // by device and sizes, of any thread; a call keeps the plan that it uses
+struct LibraryPlans {
+  std::mutex mutex;
+  std::map<std::array<int64_t, 4>, std::shared_ptr<const LibraryPlan>> plans;
+};
+
+LibraryPlans& library_plans() {
+  static LibraryPlans all;
+  return all;
+}
+
 std::shared_ptr<const LibraryPlan> library_plan(int device, int64_t M,
                                                 int64_t N, int64_t K) {
-  static std::mutex mutex;
-  static std::map<std::array<int64_t, 4>, std::shared_ptr<const LibraryPlan>>
-      plans;
   constexpr size_t MOST = 1024;
+  auto& [mutex, plans] = library_plans();
   const std::lock_guard<std::mutex> lock(mutex);
   const std::array<int64_t, 4> key{device, M, N, K};
   const auto at = plans.find(key);
   if (at != plans.end()) return at->second;
   if (plans.size() >= MOST) plans.clear();
   return plans[key] = std::make_shared<const LibraryPlan>(M, N, K);
+}
+
+int64_t library_plans_kept() {
+  auto& [mutex, plans] = library_plans();
+  const std::lock_guard<std::mutex> lock(mutex);
+  return int64_t(plans.size());
 }
 
 // x w^T as at::linear has it.  Of many rows, where the library's pick divides K
@@ -213,7 +238,7 @@ Tensor library_linear(const Tensor& x, const Tensor& w) {
   const int64_t M = x.size(0), N = w.size(0), K = x.size(1);
   const auto start = reinterpret_cast<uintptr_t>(x.data_ptr()) |
                      reinterpret_cast<uintptr_t>(w.data_ptr());
-  if (M == 0 || N == 0 || K == 0 || start % 16 != 0 ||
+  if (M == 0 || N == 0 || K == 0 || start % 16 != 0 || own_workspace() ||
       at::globalContext().blasPreferredBackend() != at::BlasBackend::Cublaslt ||
       at::cuda::tunable::getTuningContext()->IsTunableOpEnabled())
     return at::linear(x, w);
@@ -250,6 +275,7 @@ Tensor library_linear(const Tensor& x, const Tensor& w) {
 
 TORCH_LIBRARY_FRAGMENT(rlli, m) {
   m.def("library_linear(Tensor x, Tensor w) -> Tensor");
+  m.def("library_plans_kept() -> int", &library_plans_kept);
   m.def("lt_linear(Tensor x, Tensor w, int algo_index) -> Tensor");
   m.def("lt_heuristics(Tensor x, Tensor w, int max_n) -> Tensor");
 }

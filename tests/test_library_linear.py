@@ -2,6 +2,9 @@
 whatever the operands, streams and threads; tiles where that choice would sum
 parts in a workspace."""
 
+import os
+import subprocess
+import sys
 import threading
 
 import pytest
@@ -128,3 +131,28 @@ def test_autocast():
     with torch.autocast("cuda", torch.float16):
         got, want = ops.library_linear(x, w), F.linear(x, w)
     assert got.dtype == want.dtype and torch.equal(got, want)
+
+
+# in a process that sets the library's workspace itself (128 MiB), which has no
+# plan of ours then
+OWN_SPACE = """
+import torch
+import torch.nn.functional as F
+from resilient_llm_amd import ops
+x = torch.randn(130, 1000, device="cuda:0").bfloat16()
+w = torch.randn(640, 1000, device="cuda:0").bfloat16()
+assert torch.equal(ops.library_linear(x, w), F.linear(x, w))
+assert torch.ops.rlli.library_plans_kept() == 0
+"""
+
+
+@pytest.mark.gpu
+def test_workspace_of_the_process():
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    ran = subprocess.run(
+        [sys.executable, "-c", OWN_SPACE], cwd=root, timeout=100,
+        capture_output=True, text=True,
+        env={**os.environ, "HIPBLASLT_WORKSPACE_SIZE": str(128 << 10)})
+    assert ran.returncode == 0, ran.stderr[-2000:]
+    ops.library_linear(*operands(130, 640, 1000))
+    assert torch.ops.rlli.library_plans_kept() >= 1

@@ -33,6 +33,7 @@
 #include <algorithm>
 #include <array>
 #include <cstdlib>
+#include <list>
 #include <map>
 #include <memory>
 #include <mutex>
@@ -197,10 +198,40 @@ bool own_workspace() {
   return own;
 }
 
-// by device and sizes, of any thread; a call keeps the plan that it uses
-struct LibraryPlans {
-  std::mutex mutex;
-  std::map<std::array<int64_t, 4>, std::shared_ptr<const LibraryPlan>> plans;
+// Plans by device and sizes, of any thread: the 1024 that were asked for last.  A
+// call keeps the plan that it uses.
+class LibraryPlans {
+ public:
+  using Plan = std::shared_ptr<const LibraryPlan>;
+
+  Plan of(int device, int64_t M, int64_t N, int64_t K) {
+    const std::lock_guard<std::mutex> lock(mutex_);
+    const Key key{device, M, N, K};
+    const auto at = places_.find(key);
+    if (at != places_.end()) {
+      plans_.splice(plans_.begin(), plans_, at->second);
+      return plans_.front().second;
+    }
+    plans_.emplace_front(key, std::make_shared<const LibraryPlan>(M, N, K));
+    places_[key] = plans_.begin();
+    if (plans_.size() > MOST) {
+      places_.erase(plans_.back().first);
+      plans_.pop_back();
+    }
+    return plans_.front().second;
+  }
+
+  int64_t kept() {
+    const std::lock_guard<std::mutex> lock(mutex_);
+    return int64_t(plans_.size());
+  }
+
+ private:
+  using Key = std::array<int64_t, 4>;
+  static constexpr size_t MOST = 1024;
+  std::mutex mutex_;
+  std::list<std::pair<Key, Plan>> plans_;     // the last one first
+  std::map<Key, std::list<std::pair<Key, Plan>>::iterator> places_;
 };
 
 LibraryPlans& library_plans() {
@@ -208,23 +239,7 @@ LibraryPlans& library_plans() {
   return all;
 }
 
-std::shared_ptr<const LibraryPlan> library_plan(int device, int64_t M,
-                                                int64_t N, int64_t K) {
-  constexpr size_t MOST = 1024;
-  auto& [mutex, plans] = library_plans();
-  const std::lock_guard<std::mutex> lock(mutex);
-  const std::array<int64_t, 4> key{device, M, N, K};
-  const auto at = plans.find(key);
-  if (at != plans.end()) return at->second;
-  if (plans.size() >= MOST) plans.clear();
-  return plans[key] = std::make_shared<const LibraryPlan>(M, N, K);
-}
-
-int64_t library_plans_kept() {
-  auto& [mutex, plans] = library_plans();
-  const std::lock_guard<std::mutex> lock(mutex);
-  return int64_t(plans.size());
-}
+int64_t library_plans_kept() { return library_plans().kept(); }
 
 // x w^T as at::linear has it.  Of many rows, where the library's pick divides K
 // and sums in a workspace (beside tiles that do not come out even), tiles of our
@@ -243,7 +258,7 @@ Tensor library_linear(const Tensor& x, const Tensor& w) {
       at::cuda::tunable::getTuningContext()->IsTunableOpEnabled())
     return at::linear(x, w);
   c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
-  const auto plan = library_plan(x.device().index(), M, N, K);
+  const auto plan = library_plans().of(x.device().index(), M, N, K);
   if (!plan->found) return at::linear(x, w);
   Tensor y = at::empty({M, N}, x.options()), workspace;
   const auto stream = at::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream();

@@ -94,6 +94,18 @@ def test_streams_and_threads():
     assert not wrong
 
 
+@pytest.mark.gpu
+def test_plans_of_the_last_sizes():
+    """Of more shapes than are kept, the least recently used go, and those one by
+    one."""
+    kept = torch.ops.rlli.library_plans_kept
+    w = operands(1, 64, 64)[1]
+    x = operands(1200, 64, 64)[0]
+    for m in range(1, 1201):
+        ops.library_linear(x[:m], w)
+    assert kept() == 1024
+
+
 # rows that rows_tall, the library and (N not a multiple of 128) tiles take
 FORMS = [(200, 2048, 2048), (1000, 4096, 4096), (2048, 6160, 2048)]
 

@@ -5,7 +5,7 @@ parts in a workspace."""
 import os
 import subprocess
 import sys
-import threading
+from concurrent.futures import ThreadPoolExecutor
 
 import pytest
 import torch
@@ -75,7 +75,6 @@ def test_streams_and_threads():
     x = operands(1200, 64, 64)[0]
     want = F.linear(x, w)
     torch.cuda.synchronize()
-    wrong = []
 
     def run(n):
         s = torch.cuda.Stream()
@@ -84,14 +83,11 @@ def test_streams_and_threads():
                    for m in range(1 + n, 1200, 2)]
             s.synchronize()
         # (a row's sum may be in another order with another number of rows)
-        wrong.extend(m for m, y in got if not torch.allclose(
-            y.float(), want[:m].float(), rtol=2 ** -7, atol=2 ** -14))
-    threads = [threading.Thread(target=run, args=(i % 2,)) for i in range(4)]
-    for t in threads:
-        t.start()
-    for t in threads:
-        t.join()
-    assert not wrong
+        return len(got), [m for m, y in got if not torch.allclose(
+            y.float(), want[:m].float(), rtol=2 ** -7, atol=2 ** -14)]
+    with ThreadPoolExecutor(4) as pool:
+        ran = list(pool.map(run, [0, 1, 0, 1]))
+    assert ran == [(600, []), (599, [])] * 2
 
 
 @pytest.mark.gpu

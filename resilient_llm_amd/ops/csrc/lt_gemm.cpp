@@ -241,12 +241,34 @@ LibraryPlans& library_plans() {
 
 int64_t library_plans_kept() { return library_plans().kept(); }
 
+// The tiles of library_linear: K is divided where that takes less and the parts
+// have room in what the library may have.
+rlli::TilePlan tiles_for_library(int64_t M, int64_t N, int64_t K) {
+  const auto plan = rlli::tile_gemm_plan(int(M), int(N), int(K), false);
+  if (plan.splits == 1 ||
+      plan.splits * M * N * 4 <=
+          int64_t(at::cuda::getCUDABlasLtWorkspaceSize()))
+    return plan;
+  return rlli::tile_gemm_plan(int(M), int(N), int(K), true);
+}
+
+// its 64 rows and 128 columns of a tile, and parts
+std::vector<int64_t> tile_numbers(int64_t M, int64_t N, int64_t K) {
+  const rlli::TilePlan plan = tiles_for_library(M, N, K);
+  return {plan.mh, plan.nh, plan.splits};
+}
+
 // x w^T as at::linear has it.  Of many rows, where the library's pick divides K
 // and sums in a workspace (beside tiles that do not come out even), tiles of our
-// own are faster (us, the library first: 4096 x 14336, 4300 rows 735 and 369,
-// 7613 979 and 665, 7000 644 and 615; 6160 x 2048, 7259 rows 188 and 160; 5120 x
-// 13824, 7400 rows 910 and 856; 8192 x 28672, 2100 rows 1470 and 729; where it
-// does not divide K the other way round, 7900 rows of the first 628 and 674).
+// own are faster, which divide K themselves where they are few.  (us, the library,
+// tiles of all of K and these: 4096 x 14336, 4300 rows 735, 369 and 369, 7613 979,
+// 665 and 665; 6160 x 2048, 7259 rows 188 and 160; 8192 x 28672, 2100 rows 1470 and
+// 729; 1024 x 28672, 1900 rows 195, 250 and 99; 2048 x 28672, 3000 rows 283, 349 and
+// 273; 64 x 28672, 1100 rows 74, 227 and 38.  Of 410 such products the library was
+// faster by 5 % and more at 7, where its pick for one size is far better than for
+// those beside it: 576 x 28672, 8000 rows 246, 386 and 267, but 7900 403 and 256;
+// 3072 x 28672, 2048 rows 280, 360 and 297, but 1900 454 and 258; 14336 x 7168, 7000
+// rows 1005 and 1105, but 6500 1073 and 970.)
 Tensor library_linear(const Tensor& x, const Tensor& w) {
   check_linear_args(x, w);
   TORCH_CHECK(x.device() == w.device(), "x and W on one GPU");
@@ -264,13 +286,21 @@ Tensor library_linear(const Tensor& x, const Tensor& w) {
   const auto stream = at::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream();
   if (plan->workspace && M > 1024 && K % 64 == 0 && N % 8 == 0 &&
       std::max({x.numel(), w.numel(), y.numel()}) < int64_t(1) << 31) {
+    const rlli::TilePlan tiles = tiles_for_library(M, N, K);
+    auto* out = static_cast<uint16_t*>(y.data_ptr());
+    const bool divided = tiles.splits > 1;
+    if (divided)
+      workspace = at::empty({tiles.splits, M, N}, x.options().dtype(at::kFloat));
+    float* parts = divided ? workspace.data_ptr<float>() : nullptr;
     rlli::launch_tile_gemm(static_cast<const uint16_t*>(x.data_ptr()),
-                           static_cast<const uint16_t*>(w.data_ptr()), nullptr,
-                           static_cast<uint16_t*>(y.data_ptr()), int(M), int(N),
-                           int(K), rlli::TileAct::none,
-                           rlli::tile_gemm_plan(int(M), int(N), int(K), true),
-                           stream);
+                           static_cast<const uint16_t*>(w.data_ptr()), parts,
+                           divided ? nullptr : out, int(M), int(N), int(K),
+                           rlli::TileAct::none, tiles, stream);
     rlli_ext::check_launch("library_linear");
+    if (divided) {
+      rlli::launch_sum_parts(parts, out, tiles.splits, y.numel(), stream);
+      rlli_ext::check_launch("sum_parts");
+    }
     return y;
   }
   if (plan->workspace)
@@ -291,6 +321,7 @@ Tensor library_linear(const Tensor& x, const Tensor& w) {
 TORCH_LIBRARY_FRAGMENT(rlli, m) {
   m.def("library_linear(Tensor x, Tensor w) -> Tensor");
   m.def("library_plans_kept() -> int", &library_plans_kept);
+  m.def("tiles_for_library(int m, int n, int k) -> int[]", &tile_numbers);
   m.def("lt_linear(Tensor x, Tensor w, int algo_index) -> Tensor");
   m.def("lt_heuristics(Tensor x, Tensor w, int max_n) -> Tensor");
 }

@@ -48,6 +48,33 @@ def test_many_rows(M, N, K):
     close(ops.library_linear(x, w), x, w)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(1100, 64, 28672), (1900, 1024, 28672),
+                                   (2048, 256, 28672), (3000, 2048, 28672)])
+def test_few_tiles_divide_k(M, N, K):
+    """Whatever the library picks, tiles are not left to go through a long K where
+    a few of them are all."""
+    x, w = operands(M, N, K)
+    got = ops.library_linear(x, w)
+    close(got, x, w)
+    assert torch.equal(got, F.linear(x, w)) \
+        or torch.equal(got, torch.ops.rlli.tile_linear(x, w))
+
+
+@pytest.mark.parametrize("M,N,K,splits", [
+    (1100, 64, 28672, 8), (1900, 1024, 28672, 6), (4300, 4096, 14336, 1),
+    (6500, 5120, 2048, 1),
+    # parts of more than 76 MiB are not made
+    (2300, 4096, 28672, 1), (1025, 8192, 28672, 1), (2048, 2048, 28672, 4)])
+def test_parts_of_tiles(M, N, K, splits):
+    ops.load_extension(required=True)
+    mh, nh, n = torch.ops.rlli.tiles_for_library(M, N, K)
+    assert n == splits
+    if splits > 1:
+        tiles = -(-M // (64 * mh)) * -(-N // (128 * nh))
+        assert tiles * n > 64
+
+
 def test_other_operands_cpu():
     x, w = operands(5, 6, 7, torch.float32, "cpu")
     assert torch.equal(ops.library_linear(x, w), F.linear(x, w))

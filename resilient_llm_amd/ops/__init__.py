@@ -640,11 +640,21 @@ def _tile_linear_faster(M: int, N: int, K: int) -> bool:
     5120, 208 and 240 rows 33 and 37, all beside rows where they gain more.)"""
     if K <= 2048 and N % 128 != 0:
         # The library is slow where rows of the result end amid its tiles (as
-        # times as fast: 6160 x 2048, 1024 rows 1.20, 2048 1.20, 4000 1.05, 777
-        # 0.91, 7613 0.96; 3088 x 2048, 1024 1.20, 1300 0.89, 2048 1.19, 5000
-        # 1.13; 8208 x 2048, 1300 1.22, 3300 1.43; 6160 x 1024, 420 1.14, 1300
-        # 1.23, 5000 1.11; 2064 x 1024, 512 0.93, 1024 1.15, 5000 1.29).
-        return (1024 if K > 1024 else 600) <= M <= 6400 and 2048 <= N <= 10496
+        # times as fast: 6160 x 2048, 1024 rows 1.11, 2048 1.20, 4000 1.05, 777
+        # 0.91, 7613 0.96; 3088 x 2048, 1024 1.15, 2048 1.12, 5000 1.16; 8208 x
+        # 2048, 1300 1.18, 3300 1.40, 5000 1.03; 10256 x 2048, 1024 1.15, 5000
+        # 1.11; 6160 x 1024, 420 1.14, 1300 1.22, 5000 1.15; 2064 x 1024, 512
+        # 0.93, 1024 1.12, 5000 1.21).  With long K, somewhat more tiles of 128 x
+        # 128 than there are CUs take two rounds of them or of larger ones (3088 x
+        # 2048, 1200 rows 1.18, 1300 0.95, 1600 0.94, 1800 1.02; 2064 x 2048, 1800
+        # 1.14, 2048 0.93, 2300 0.92, 2600 1.00; 4112 x 2048, 1024 0.96, 1100 0.97,
+        # 1200 1.05; 3088 x 1536, 1300 1.06), and just more of 256 x 256 than four
+        # rounds have take a fifth (10256 x 2048, 6400 0.88; x 1536 0.92).
+        def tiles(side):
+            return -(-M // side) * -(-N // side)
+        return ((1024 if K > 1024 else 600) <= M <= 6400 and 2048 <= N <= 10496
+                and tiles(256) <= 1024
+                and not (K > 1536 and 256 < tiles(128) < 328))
     return (64 < M <= (256 if K > 4096 else 160) and K >= 4096
             and 4096 <= N <= 10240 and (M > 128 or N * K > 1 << 24))
 

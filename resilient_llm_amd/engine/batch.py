@@ -23,11 +23,8 @@ def sent(values, dtype, device) -> torch.Tensor:
     models' prompts cost 0.2 ms of a step."""
     device = torch.device(device)
     pin = device.type == "cuda"
-    code = _ARRAYS.get(dtype)
-    if pin and code and isinstance(values, list) and len(values) > 512 \
-            and isinstance(values[0], int):
-        # (7600 numbers by torch.tensor 480 us, so 140)
-        flat = torch.frombuffer(array.array(code, values), dtype=dtype)
+    flat = _numbers(values, dtype) if pin else None
+    if flat is not None:
         return torch.empty(len(values), dtype=dtype, pin_memory=True) \
             .copy_(flat).to(device, non_blocking=True)
     return torch.tensor(values, dtype=dtype, pin_memory=pin).to(
@@ -35,6 +32,19 @@ def sent(values, dtype, device) -> torch.Tensor:
 
 
 _ARRAYS = {torch.int32: "i", torch.long: "q"}
+
+
+def _numbers(values, dtype):
+    """A long list of whole numbers as a tensor (7600 of them by torch.tensor 480
+    us, so 140); None: for torch.tensor."""
+    code = _ARRAYS.get(dtype)
+    if not code or not isinstance(values, list) or len(values) <= 512 \
+            or not isinstance(values[0], int):
+        return None
+    try:
+        return torch.frombuffer(array.array(code, values), dtype=dtype)
+    except TypeError:                # a fraction among them, which is cut off
+        return None
 
 
 @dataclasses.dataclass(frozen=True)

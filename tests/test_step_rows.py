@@ -5,7 +5,7 @@ import pytest
 import torch
 
 from resilient_llm_amd.engine import LLMEngine, PagedKVCache
-from resilient_llm_amd.engine.batch import sent
+from resilient_llm_amd.engine.batch import _numbers, sent
 from resilient_llm_amd.models import build_model, get_config
 
 
@@ -67,3 +67,21 @@ def test_sent(n, dtype, device):
     pairs = list(zip(values, values[::-1]))
     if pairs:
         assert sent(pairs, dtype, device).tolist() == [list(p) for p in pairs]
+
+
+@pytest.mark.parametrize("device", ["cpu", pytest.param(
+    "cuda:0", marks=pytest.mark.gpu)])
+@pytest.mark.parametrize("dtype", [torch.int32, torch.long])
+def test_sent_with_a_fraction(dtype, device):
+    values = [1] * 600 + [2.7, -3.5]
+    got = sent(values, dtype, device)
+    assert got.dtype == dtype and got.tolist() == [1] * 600 + [2, -3]
+
+
+def test_long_lists_of_whole_numbers():
+    values = list(range(-300, 300))
+    for dtype in (torch.int32, torch.long):
+        assert _numbers(values, dtype).tolist() == values
+        assert _numbers(values[:512], dtype) is None
+        assert _numbers(values + [0.5], dtype) is None
+    assert _numbers(values, torch.float32) is None

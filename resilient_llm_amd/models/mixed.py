@@ -30,14 +30,15 @@ class LayerSpec:
 
 
 def narrow_to(rows: Optional[torch.Tensor], total: int) -> bool:
-    """Whether the last layer, behind its mixer, is for ``rows`` of a step's
-    ``total`` rows alone: nobody reads the others' output.  What it costs is
-    two gathers of those rows; up to 64 rows, products cost what reading their
-    weights does, whatever the rows.  (us, all rows first: 8B, 64 prompts of
+    """Whether the last layer, behind its mixer, is for ``rows`` (their numbers, in
+    a tensor) of a step's ``total`` rows alone: nobody reads the others' output.
+    What it costs is two gathers of those rows; up to 64 rows, products cost what
+    reading their weights does, whatever the rows.  (us, all rows first: 8B, 64 prompts of
     128 tokens 88700 and 86700, one of 7901 103600 and 101500, 24 decoding rows
     beside a chunk of 512 10530 and 10310; 12 mixed layers of 2048, four prompts
     of about 1900 9150 and 8770.)"""
-    return rows is not None and total > 64 and 0 < 2 * len(rows) <= total
+    return (total > 64 and isinstance(rows, torch.Tensor) and rows.dim() == 1
+            and rows.dtype != torch.bool and 0 < 2 * len(rows) <= total)
 
 
 class MixedConfig:

@@ -51,3 +51,12 @@ def test_which_rows():
     assert narrow_to(rows, 65) and narrow_to(rows[:1], 4096)
     assert not narrow_to(rows, 64) and not narrow_to(None, 4096)
     assert not narrow_to(rows[:0], 4096) and not narrow_to(torch.arange(33), 65)
+
+
+def test_other_indices():
+    """What the last norm's rows may be chosen by beside a list of them, they are
+    chosen by there."""
+    assert not narrow_to(torch.tensor(3), 4096)
+    assert not narrow_to(torch.zeros(2, 3, dtype=torch.long), 4096)
+    assert not narrow_to(torch.zeros(128, dtype=torch.bool), 4096)
+    assert not narrow_to(slice(0, 3), 4096) and not narrow_to([3, 5], 4096)

@@ -165,6 +165,30 @@ void prefill(rlli::GlaArgs& a, const Tensor& proj, const Tensor& tiles,
   check_launch("recurrent prefill");
 }
 
+// How a prompt of 16-bit activations goes through the scan: operands in parts or
+// not, and of those, columns of a workgroup and whether it asks for lines ahead
+std::vector<int64_t> gla_scan(int64_t rows, int64_t n_tiles, int64_t n_seqs,
+                              int64_t heads, int64_t dim, int64_t vdim) {
+  rlli::GlaArgs a{};
+  a.rows = int(rows);
+  a.n_tiles = int(n_tiles);
+  a.n_seqs = int(n_seqs);
+  a.heads = int(heads);
+  a.dim = int(dim);
+  a.dpad = (a.dim + 15) / 16 * 16;
+  a.vdim = int(vdim);
+  if (!rlli::gla_parts(a)) return {0, 0, 0};
+  rlli::ScanArgs s{};
+  s.n_tiles = a.n_tiles;
+  s.n_seqs = a.n_seqs;
+  s.heads = a.heads;
+  s.dim = a.dim;
+  s.dpad = a.dpad;
+  s.vdim = a.vdim;
+  const rlli::ScanSlices by = rlli::scan_slices(s);
+  return {1, by.cols, by.touch};
+}
+
 void gla_decode(const Tensor& proj, const Tensor& a2, const Tensor& a2_bias,
                 const Tensor& norm, Tensor state, const Tensor& slots,
                 const Tensor& positions, int64_t vdim, double tau,
@@ -391,6 +415,8 @@ TORCH_LIBRARY(rlli_rec, m) {
   m.def("gla_prefill(Tensor proj, Tensor a2, Tensor a2_bias, Tensor norm, "
         "Tensor(a!) state, Tensor tiles, Tensor seqs, int vdim, float tau, "
         "float eps, Tensor(b!) out) -> ()");
+  m.def("gla_scan(int rows, int n_tiles, int n_seqs, int heads, int dim, "
+        "int vdim) -> int[]", &gla_scan);
   m.def("hgrn2_decode(Tensor proj, Tensor bias, Tensor lower, Tensor norm, "
         "Tensor(a!) state, Tensor slots, Tensor positions, int vdim, "
         "float eps, Tensor(b!) out) -> ()");

@@ -51,6 +51,13 @@ struct ScanArgs {
   int mode;
   bool f32, parts;         // parts: qd, kt and sc (plain)
 };
+// Of operands in parts: columns of a workgroup, and whether each asks for lines of
+// the next chunk but one (of heads of 64 or 128 in whole slices).
+struct ScanSlices {
+  int cols;
+  bool touch;
+};
+ScanSlices scan_slices(const ScanArgs& a);
 void launch_rec_scan(const ScanArgs& a, hipStream_t stream);
 
 // o over its root mean square, times norm and gate

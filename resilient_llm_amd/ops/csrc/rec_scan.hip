@@ -382,7 +382,8 @@ void rec_scan_kernel(ScanArgs a, bool vec_q, bool vec_v) {
 // and not all at once with all waves waiting to issue them, and loads ahead of the
 // loop come in the loop's order, as the waits in it are for both.  Operands that no
 // cache holds any more come slower; TOUCH: each of the slices that read them asks
-// for its share of their lines a chunk ahead.  (In a step's call, 8 heads of 128 x
+// for 256 of their 576 or 960 lines a chunk ahead, so that three or four ask for
+// all.  (In a step's call, 8 heads of 128 x
 // 256, us, loads together behind the products and now: 1 sequence of 2600 70 and
 // 57, 3 of 2000 105 and 73, 4 of 2000 111 and 80, 8 of 900 77 and 63, 16 of 500 92
 // and 83; asked for two chunks ahead 62, 76, 84, 64 and 93.)  4 sequences of 1.9k
@@ -764,28 +765,10 @@ void scan(const ScanArgs& a, hipStream_t st) {
   const int64_t sh = int64_t(a.n_seqs) * a.heads;
   if constexpr (MODE == kScanPlain && sizeof(T) == 2)
     if (a.parts) {
-      // A CU has one workgroup, which takes the longer the wider its slice is.
-      // (us, slices of 16, 32 and 64 columns: heads of 128 x 256, 1000 tokens,
-      // 16 of them 34 38 50, 24 60 42 55, 32 67 46 59, 40 98 82 62, 64 of 900
-      // 134 88 64; of 64 x 64, 64 of them 33 40 41, 80 61 43 44.  Two copies of
-      // 256 rows by 64 columns do not fit LDS.)
-      auto groups = [&](int cols) { return sh * ((a.vdim + cols - 1) / cols); };
-      auto cost = [&](int cols, int each) {
-        return (groups(cols) + 255) / 256 * each;
-      };
-      const int64_t one = cost(16, 6), two = cost(32, 7);
-      const int cols = a.dpad <= 128 && cost(64, 9) < std::min(one, two) ? 64
-                       : two < one                                       ? 32
-                                                                         : 16;
-      // From some 60 MB of operands on, if all workgroups run at once (in a
-      // step's call, us without and with, heads of 128 x 256: 1 sequence of 2600
-      // 57 59, 2 of 2000 57 57, 3 80 73, 4 102 80, 8 of 900 65 63; 16 of 500,
-      // which take turns, 83 93).
-      const bool touch = int64_t(a.n_tiles) * a.heads * a.dpad >= 65536 &&
-                         groups(cols) <= 256;
-      if (cols == 64) scan_parts<4>(a, touch, st);
-      else if (cols == 32) scan_parts<2>(a, touch, st);
-      else scan_parts<1>(a, touch, st);
+      const ScanSlices by = scan_slices(a);
+      if (by.cols == 64) scan_parts<4>(a, by.touch, st);
+      else if (by.cols == 32) scan_parts<2>(a, by.touch, st);
+      else scan_parts<1>(a, by.touch, st);
       return;
     }
   if (a.vdim > 32 && sh * ((a.vdim + 63) / 64) >= 512)
@@ -891,6 +874,28 @@ void gate(const RecGateArgs& a, hipStream_t st) {
 }
 
 }  // namespace
+
+// A CU has one workgroup, which takes the longer the wider its slice is.  (us,
+// slices of 16, 32 and 64 columns: heads of 128 x 256, 1000 tokens, 16 of them 34 38
+// 50, 24 60 42 55, 32 67 46 59, 40 98 82 62, 64 of 900 134 88 64; of 64 x 64, 64 of
+// them 33 40 41, 80 61 43 44.  Two copies of 256 rows by 64 columns do not fit LDS.)
+ScanSlices scan_slices(const ScanArgs& a) {
+  const int64_t sh = int64_t(a.n_seqs) * a.heads;
+  auto groups = [&](int cols) { return sh * ((a.vdim + cols - 1) / cols); };
+  auto cost = [&](int cols, int each) {
+    return (groups(cols) + 255) / 256 * each;
+  };
+  const int64_t one = cost(16, 6), two = cost(32, 7);
+  const int cols = a.dpad <= 128 && cost(64, 9) < std::min(one, two) ? 64
+                   : two < one                                       ? 32
+                                                                     : 16;
+  // From some 60 MB of operands on, if all workgroups run at once (in a step's call,
+  // us without and with, heads of 128 x 256: 1 sequence of 2600 57 59, 2 of 2000 57
+  // 57, 3 80 73, 4 102 80, 8 of 900 65 63; 16 of 500, which take turns, 83 93).
+  return {cols, int64_t(a.n_tiles) * a.heads * a.dpad >= 65536 &&
+                    groups(cols) <= 256 && (a.dim == 64 || a.dim == 128) &&
+                    a.vdim % cols == 0};
+}
 
 void launch_rec_scan(const ScanArgs& a, hipStream_t st) {
   if (a.n_seqs == 0) return;

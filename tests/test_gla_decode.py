@@ -131,16 +131,28 @@ def test_prompts_by_slices(seqs, H, dim, vdim):
     assert torch.isnan(st[seqs]).all()
 
 
+def scan_of(lens, H, dim, vdim):
+    """Parts or f32, columns of a slice, and whether slices ask for lines ahead."""
+    ops.load_libraries(("rlli_rec",))
+    return torch.ops.rlli_rec.gla_scan(
+        sum(lens), sum(-(-n // 64) for n in lens), len(lens), H, dim, vdim)
+
+
 @pytest.mark.gpu
-@pytest.mark.parametrize("seqs,H,dim,vdim", [
-    (16, 2, 128, 128), (16, 2, 128, 256), (32, 2, 64, 64)])
-def test_prompts_of_many_operands(seqs, H, dim, vdim):
-    """Some 60 MB of a scan's operands, which each slice asks for its share of
-    ahead of time: chunk counts that are even, odd and one."""
-    lens = [1024] * seqs
-    lens[1], lens[2], lens[3] = 1023, 900, 1
-    lens[4:4] = [80] * 3
-    *inputs, eps, want, S = gla_case(1024, H, dim, vdim, 8, 8.0, 1.0, dim, BF16)
+@pytest.mark.parametrize("seqs,H,dim,vdim,T,cols", [
+    (8, 4, 128, 128, 1216, 16), (8, 4, 64, 128, 2400, 16),
+    (8, 4, 128, 256, 1216, 32), (8, 4, 64, 256, 2400, 32),
+    (11, 4, 128, 160, 900, 32), (11, 4, 64, 160, 1900, 32),
+    (16, 4, 128, 256, 600, 64), (16, 4, 64, 192, 1100, 64),
+    # one slice of a head
+    (20, 8, 128, 64, 280, 64), (24, 8, 64, 64, 460, 64)])
+def test_prompts_of_many_operands(seqs, H, dim, vdim, T, cols):
+    """Some 60 MB of a scan's operands, lines of which slices ask for ahead of
+    time: chunk counts that are even, odd and one."""
+    lens = [T] * seqs
+    lens[1], lens[2], lens[3] = T - 70, T - 1, 1
+    assert scan_of(lens, H, dim, vdim) == [1, cols, 1]
+    *inputs, eps, want, S = gla_case(T, H, dim, vdim, 8, 8.0, 1.0, dim, BF16)
     proj, a2, b, norm = (t.cuda() for t in inputs)
     st = torch.full((len(lens), H, dim, vdim), float("nan"), device="cuda")
     portions, at = [], 0
@@ -151,8 +163,23 @@ def test_prompts_of_many_operands(seqs, H, dim, vdim):
                           st, PromptRows(portions, "cuda"), vdim, 8.0, eps)
     for i, (n, rows) in enumerate(zip(lens, got.split(lens))):
         assert rel(rows, want[:n]) < tol(BF16)
-        if n == 1024:
+        if n == T:
             assert rel(st[i], S) < 1e-5
+
+
+@pytest.mark.parametrize("seqs,H,dim,vdim,T,form", [
+    # heads of more than 128: f32 operands where many fill the chip
+    (4, 64, 132, 72, 70, 0), (2, 64, 132, 256, 66, 1), (1, 32, 132, 33, 3100, 1),
+    # up to 64 columns: where they fill it and are 48 Ki rows of all heads, or 96 Ki
+    # on up to 128 workgroups
+    (8, 64, 128, 40, 97, 0), (8, 64, 100, 33, 95, 1), (2, 16, 72, 20, 3100, 0),
+    (2, 16, 72, 20, 3000, 1), (9, 16, 128, 64, 700, 1),
+    # more columns: where they fill it and up to 128
+    (2, 16, 72, 100, 3100, 1), (8, 64, 100, 128, 97, 0), (8, 64, 100, 130, 97, 1),
+    # short heads that fill it
+    (8, 64, 64, 64, 10, 0), (7, 64, 64, 64, 10, 1)])
+def test_form_of_the_scans_operands(seqs, H, dim, vdim, T, form):
+    assert scan_of([T] * seqs, H, dim, vdim)[0] == form
 
 
 @pytest.mark.gpu
@@ -255,9 +282,10 @@ def test_scratch_of_prompts(dtype, seqs, dim, each):
     # heads of more than 128: f32 operands where many fill the chip
     (4, 64, 132, 72, 70), (2, 64, 132, 256, 66),
     # of up to 128: from 48 Ki rows of all heads on where they fill it; 96 Ki
-    # elsewhere, also wide ones of few columns
+    # elsewhere, but not of more than 64 columns, nor wide ones
     (8, 64, 128, 40, 97), (8, 64, 100, 33, 95), (2, 16, 72, 20, 3100),
-    (1, 32, 132, 33, 3100)])
+    (1, 32, 132, 33, 3100), (2, 16, 72, 100, 3100), (8, 64, 100, 128, 97),
+    (8, 64, 100, 130, 97)])
 def test_prompts_of_many_heads(seqs, H, dim, vdim, T, kind):
     """Both sides of the lines where the scan's operands are f32 and not parts."""
     rows = PromptRows([Portion(i * T, 0, T, i, i) for i in range(seqs)], "cuda")

@@ -715,19 +715,27 @@ void by_kind(const GlaArgs& a, F f) {
 // of each chunk's chain, and half as many bytes more, which cost more than they
 // give where the chip is full (`many` heads) or few narrow blocks stream `much`.
 // Whole prompts, time in f32 over time in parts (heads of all sequences and rows of
-// each):
-//   64 x 64     512 heads 0.89; 64, 2000 rows 0.88; 16, 8000 rows 1.04; 256, 500
-//               rows 1.09
-//   64 x 128    16, 8000 rows 1.11; 64, 2000 rows 1.00; 256, 500 rows 0.98
-//   64 x 256    64, 2000 rows 1.25; 256, 500 rows 0.97
-//   128 x 64    64, 512 rows 0.91, 2048 rows 0.88; 128, 2048 rows 0.95
-//   128 x 128   16, 2048 rows 1.11, 8000 rows 1.14; 64, 2000 rows 1.08; 128, 1000
+// each; two boxes differ by up to 0.08):
+//   64 x 64     512 heads 0.89; 64, 2000 rows 0.90; 32, 4000 rows 1.01; 16, 4000
+//               rows 1.37, 8000 rows 1.04 to 1.14, left to f32; 256, 250 rows 1.11
+//   64 x 128    16, 8000 rows 1.15; 64, 2000 rows 1.00; 256, 500 rows 0.98
+//   64 x 256    32, 3200 rows 1.23; 64, 2000 rows 1.25; 256, 500 rows 0.97
+//   128 x 64    32, 500 rows 1.15; 64, 256 rows 1.09, 512 rows 0.91 to 0.99, 1000 rows
+//               0.99, 1600 rows 0.91; 128, 250 rows 1.06, 500 rows 0.99, 1000 rows
+//               0.93
+//   128 x 128   16, 2048 rows 1.11, 8000 rows 1.17; 64, 1600 rows 1.10; 128, 1000
 //               rows 1.16; 256, 512 rows 1.01; 480, 500 rows 0.98; 512 0.91
-//   128 x 256   16, 7000 rows 1.14; 32, 3500 rows 1.29, 7000 rows 1.37; 256, 400
-//               rows 1.13; 512, 250 rows 1.14, 400 rows 1.04
+//   128 x 256   8, 12500 rows 1.27; 16, 7000 rows 1.18; 32, 3500 rows 1.32; 256, 400
+//               rows 1.12; 512, 250 rows 1.14, 400 rows 1.04
 //   256 x 256   16, 8000 rows 1.23; 64 1.62; 128 1.07; 256 0.74
 //   256 x 128   16, 8000 rows 1.24; 64 1.40; 128 1.14; 256 0.77
-//   256 x 64    64, 2048 rows 1.04; 256 heads 1.03; 512 0.80 to 0.86
+//   256 x 64    32, 4000 rows 1.12; 64, 1600 rows 1.00; 256 heads 1.03; 512 0.80 to
+//               0.86
+// Parts are the closer ones on both sides of these lines: of 29 such prompts of GLA,
+// 10 of RWKV and 12 of HGRN2, of up to 12500 rows, the state's error against 64 bits
+// was 0.54 to 0.79, 0.59 to 0.63 and 0.98 to 1.00 of that of f32 products; of outputs
+// it was the same to five places, and 0.5 to 1.02 as many were not the nearest
+// 16-bit number.
 bool gla_parts(const GlaArgs& a) {
   if (a.f32) return false;
   const int64_t sh = int64_t(a.n_seqs) * a.heads;

@@ -191,11 +191,11 @@ struct LibraryPlan {
   }
 };
 
-// Whether the process sets the library's workspace itself
-bool own_workspace() {
-  static const bool own = std::getenv("HIPBLASLT_WORKSPACE_SIZE") ||
-                          std::getenv("CUBLASLT_WORKSPACE_SIZE");
-  return own;
+// Whether the process leaves the library's workspace as it is
+bool library_plans_on() {
+  static const bool on = !std::getenv("HIPBLASLT_WORKSPACE_SIZE") &&
+                         !std::getenv("CUBLASLT_WORKSPACE_SIZE");
+  return on;
 }
 
 // Plans by device and sizes, of any thread: the 1024 that were asked for last.  A
@@ -275,7 +275,7 @@ Tensor library_linear(const Tensor& x, const Tensor& w) {
   const int64_t M = x.size(0), N = w.size(0), K = x.size(1);
   const auto start = reinterpret_cast<uintptr_t>(x.data_ptr()) |
                      reinterpret_cast<uintptr_t>(w.data_ptr());
-  if (M == 0 || N == 0 || K == 0 || start % 16 != 0 || own_workspace() ||
+  if (M == 0 || N == 0 || K == 0 || start % 16 != 0 || !library_plans_on() ||
       at::globalContext().blasPreferredBackend() != at::BlasBackend::Cublaslt ||
       at::cuda::tunable::getTuningContext()->IsTunableOpEnabled())
     return at::linear(x, w);
@@ -320,6 +320,7 @@ Tensor library_linear(const Tensor& x, const Tensor& w) {
 
 TORCH_LIBRARY_FRAGMENT(rlli, m) {
   m.def("library_linear(Tensor x, Tensor w) -> Tensor");
+  m.def("library_plans_on() -> bool", &library_plans_on);
   m.def("library_plans_kept() -> int", &library_plans_kept);
   m.def("tiles_for_library(int m, int n, int k) -> int[]", &tile_numbers);
   m.def("lt_linear(Tensor x, Tensor w, int algo_index) -> Tensor");

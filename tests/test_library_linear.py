@@ -49,16 +49,17 @@ def test_many_rows(M, N, K):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,N,K", [(1100, 64, 28672), (1900, 1024, 28672),
-                                   (2048, 256, 28672), (3000, 2048, 28672)])
+@pytest.mark.parametrize("M,N,K", [(1700, 3072, 14336), (2600, 2560, 14336)])
 def test_few_tiles_divide_k(M, N, K):
     """Whatever the library picks, tiles are not left to go through a long K where
     a few of them are all."""
-    x, w = operands(M, N, K)
-    got = ops.library_linear(x, w)
-    close(got, x, w)
-    assert torch.equal(got, F.linear(x, w)) \
-        or torch.equal(got, torch.ops.rlli.tile_linear(x, w))
+    g = torch.Generator().manual_seed(M + N + K)
+    x = torch.randn(M, K, generator=g).bfloat16()
+    w = (torch.randn(N, K, generator=g) * K ** -0.5).bfloat16()
+    got = ops.library_linear(x.to(DEV), w.to(DEV)).cpu()
+    # (f32 here too: K roundings of sums of size one, then half a step of bf16)
+    torch.testing.assert_close(got.float(), x.float() @ w.float().T,
+                               rtol=2 ** -8, atol=2 ** -13)
 
 
 @pytest.mark.parametrize("M,N,K,splits", [
@@ -146,7 +147,8 @@ def test_sizes_of_a_trace(M, N, K):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,N,K", FORMS)
+@pytest.mark.parametrize("M,N,K", [(65, 256, 64), (130, 640, 1000),
+                                   (600, 2064, 64)])
 def test_tangents(M, N, K):
     x, w = operands(M, N, K)
     t = torch.randn_like(x)
@@ -168,26 +170,22 @@ def test_autocast():
     assert got.dtype == want.dtype and torch.equal(got, want)
 
 
-# in a process that sets the library's workspace itself (128 MiB), which has no
-# plan of ours then
 OWN_SPACE = """
 import torch
-import torch.nn.functional as F
 from resilient_llm_amd import ops
-x = torch.randn(130, 1000, device="cuda:0").bfloat16()
-w = torch.randn(640, 1000, device="cuda:0").bfloat16()
-assert torch.equal(ops.library_linear(x, w), F.linear(x, w))
-assert torch.ops.rlli.library_plans_kept() == 0
+ops.load_extension(required=True)
+print(torch.ops.rlli.library_plans_on())
 """
 
 
-@pytest.mark.gpu
-def test_workspace_of_the_process():
+@pytest.mark.parametrize("own", [None, "HIPBLASLT_WORKSPACE_SIZE",
+                                 "CUBLASLT_WORKSPACE_SIZE"])
+def test_workspace_of_the_process(own):
+    """One that sets the library's workspace itself has no plans of ours."""
+    env = {k: v for k, v in os.environ.items() if "WORKSPACE_SIZE" not in k}
+    if own:
+        env[own] = str(128 << 10)
     root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
-    ran = subprocess.run(
-        [sys.executable, "-c", OWN_SPACE], cwd=root, timeout=100,
-        capture_output=True, text=True,
-        env={**os.environ, "HIPBLASLT_WORKSPACE_SIZE": str(128 << 10)})
-    assert ran.returncode == 0, ran.stderr[-2000:]
-    ops.library_linear(*operands(130, 640, 1000))
-    assert torch.ops.rlli.library_plans_kept() >= 1
+    ran = subprocess.run([sys.executable, "-c", OWN_SPACE], cwd=root, env=env,
+                         timeout=100, capture_output=True, text=True)
+    assert ran.stdout.split() == [str(own is None)], ran.stderr[-2000:]

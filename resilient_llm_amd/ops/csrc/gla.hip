@@ -715,7 +715,7 @@ void by_kind(const GlaArgs& a, F f) {
 // of each chunk's chain, and half as many bytes more, which cost more than they
 // give where the chip is full (`many` heads) or few narrow blocks stream `much`.
 // Whole prompts, time in f32 over time in parts (heads of all sequences and rows of
-// each; two boxes differ by up to 0.08):
+// each; two MI355X differ by up to 0.08):
 //   64 x 64     512 heads 0.89; 64, 2000 rows 0.90; 32, 4000 rows 1.01; 16, 4000
 //               rows 1.37, 8000 rows 1.04 to 1.14, left to f32; 256, 250 rows 1.11
 //   64 x 128    16, 8000 rows 1.15; 64, 2000 rows 1.00; 256, 500 rows 0.98
